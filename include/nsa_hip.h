@@ -154,7 +154,10 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
                    const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                    int64_t delta_sh, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu,
                    int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
-/* same upstream site; dk/dv are stored (every key row has exactly one writer), bf16 or fp32 */
+/* same upstream site.  dkv_is_f32 0 / 1: dk/dv are stored (every key row has exactly one writer), bf16 / fp32; 2: added
+ * with fp32 atomics into the caller's initialised fp32 buffers, which lets the launch cut the queries of a key tile into
+ * nsa_swa_bwd_dkdv_splits(...) chunks (1 where the key tiles alone fill the GPU) */
+int nsa_swa_bwd_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, int window);
 int nsa_swa_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                      const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                      const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,

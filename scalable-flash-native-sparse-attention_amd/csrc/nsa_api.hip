@@ -30,6 +30,7 @@ Knob g_knobs[] = {
     {"dq_min_blocks", {0}, {false}},    // workgroups per CU of the dense dq kernel
     {"dkdv_key_blocks", {0}, {false}},  // 32-key blocks per wave of the dense dk/dv kernel
     {"topk_seg_blocks", {0}, {false}},  // selection blocks per segment of the block selector
+    {"swa_dkdv_splits", {0}, {false}},  // query chunks per key tile of the window dk/dv kernel (0: from the sizes)
     {"topk_two_pass", {0}, {false}},    // 0: the one-launch selector even when a workspace is given
 };
 Knob* find_knob(const char* name) {
@@ -80,7 +81,7 @@ int nsa_abi_version(void) { return 1; }
 int nsa_set_tuning(const char* name, int value) {
   Knob* k = name ? find_knob(name) : nullptr;
   NSA_REQUIRE(k != nullptr, NSA_ERR_BAD_ARG, "set_tuning: unknown name '%s' (fwd_variant, dq_min_blocks, "
-              "dkdv_key_blocks, topk_seg_blocks, topk_two_pass)", name ? name : "(null)");
+              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, topk_two_pass)", name ? name : "(null)");
   k->value.store(value);
   k->is_set.store(true);
   return NSA_OK;
@@ -289,36 +290,59 @@ int nsa_cmp_attn_bwd_dq_final(const void* q, int64_t q_st, int64_t q_sh, const v
                          x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream);
 }
 
+static int device_cus() {
+  static std::atomic<int> num_cus{0};
+  int n = num_cus.load(std::memory_order_relaxed);
+  if (n == 0) {
+    int dev = 0;
+    hipDeviceProp_t prop;
+    n = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
+         prop.multiProcessorCount > 0) ? prop.multiProcessorCount : 256;
+    num_cus.store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Time of a workgroup of the dk/dv kernel: a fixed part (K / V fragments, epilogue) plus its 64-row tiles, and how many
+// workgroups run at once (one per CU; two where 64 channels leave the kernel under 256 registers).
+struct DkdvCost {
+  double fixed_us, tile_us;
+  int slots;
+};
+static DkdvCost dkdv_cost(int D, int VD) {
+  if (D <= 64) return {12.0, 1.9, 2 * device_cus()};
+  return {12.0, 2.55 * (D + VD) / 256.0, device_cus()};
+}
+
 // Query tokens per work item of the compressed dk/dv kernel when the caller leaves the choice to the library.
 static int cmp_dkdv_q_chunk(int q_chunk_tokens, int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
                             int kernel_size, int stride) {
   if (q_chunk_tokens <= 0) {
-    // The kernel keeps one workgroup per CU, so a launch takes about
-    //   ceil(workgroups / CUs) * (fixed cost of a workgroup + its 64-row tiles * time per tile);
-    // a workgroup is one (128-key tile, query chunk that sees it, kv head, sequence).  The chunk (a power of two in
-    // [128, 2048]) that minimises this for the longest sequence is taken.  The constants (90 us, 2.4 us per tile
-    // at d = dv = 128) were fitted on MI355X to sweeps over one to eight sequences of 4K to 64K tokens, where the
-    // choice is within 1 % of the best chunk.
-    static int num_cus = 0;
-    if (num_cus == 0) {
-      int dev = 0;
-      hipDeviceProp_t prop;
-      num_cus = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-                 prop.multiProcessorCount > 0) ? prop.multiProcessorCount : 256;
-    }
-    const double tile_us = 2.4 * (D + VD) / 256.0, fixed_us = 90.0;
+    // A work item is one (128-key tile, query chunk that sees it, kv head, sequence).  The launch takes as long as its
+    // longest item when there are fewer items than workgroup slots, else about all the work over the slots plus a
+    // quarter of an item for the last, partly empty round.  The chunk (a power of two in [64, 2048]) that minimises
+    // this for the longest sequence is taken.  Fitted on MI355X to sweeps of all chunks over one to forty sequences of
+    // 1K to 64K tokens, d = 64, 128, 192: within 3 % of the best chunk on average, 16 % at most (chunk 64 / 128 / 512 /
+    // 2048 on one sequence of 4096 tokens, 16 q / 1 kv heads: 58 / 98 / 345 / 1294 us; of 65536 tokens: 3.46 / 3.17 /
+    // 3.00 / 3.99 ms).
+    const DkdvCost c = dkdv_cost(D, VD);
     const int G = QH / KH;
     double best = 0.0;
-    for (int chunk = 128; chunk <= 2048; chunk *= 2) {
+    for (int chunk = 64; chunk <= 2048; chunk *= 2) {
       const int64_t nch = (x_maxlen + chunk - 1) / chunk;
-      int64_t wgs = 0;
+      int64_t items = 0;
+      double rows = 0.0;
       for (int64_t kt = 0; kt * 128 < y_maxlen; kt++) {
-        const int64_t fc = ((int64_t)stride * kt * 128 + kernel_size - 1) / chunk;
-        wgs += nch - (fc < nch ? fc : nch);
+        const int64_t first = (int64_t)stride * kt * 128 + kernel_size - 1;
+        if (first >= x_maxlen) break;
+        items += nch - first / chunk;
+        rows += (double)(x_maxlen - first) * G;
       }
-      wgs *= (int64_t)B * KH;
-      const double rounds = (double)((wgs + num_cus - 1) / num_cus);
-      const double cost = rounds * (fixed_us + (double)chunk * G / 64.0 * tile_us);
+      items *= (int64_t)B * KH;
+      rows *= (double)B * KH;
+      const double item = c.fixed_us + (double)(chunk < x_maxlen ? chunk : x_maxlen) * G / 64.0 * c.tile_us;
+      const double all = (items * c.fixed_us + rows / 64.0 * c.tile_us) / c.slots + 0.25 * item;
+      const double cost = items <= c.slots || all < item ? item : all;
       if (q_chunk_tokens <= 0 || cost < best) { best = cost; q_chunk_tokens = chunk; }
     }
   }
@@ -430,6 +454,26 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
   return nsa_bwd_dq_tile_launch(p, 1, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
+int nsa_swa_bwd_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, int window) {
+  if (B <= 0 || x_maxlen <= 0 || QH <= 0 || KH <= 0) return 1;
+  const int knob = nsa_tuning_knob("swa_dkdv_splits", 0);
+  if (knob > 0) return knob > 16 ? 16 : knob;
+  // A key tile's queries are cut while the rounds of workgroups times the time of one keeps falling (by a tenth at
+  // least: every cut adds a pass of atomic additions).  1 / 2 / 4 / 8 / 16 chunks, d = 128: one sequence of 4096 tokens,
+  // 16 q / 1 kv heads 399 / 211 / 126 / 83 / 105 us, 64 q / 4 kv heads 423 / 244 / 260 / 280 / 359 us; 8192 tokens,
+  // 64 q / 4 kv heads 480 / 485 / 513 / 557 / 712 us.
+  const DkdvCost c = dkdv_cost(D, VD);
+  const int64_t wgs = (int64_t)((x_maxlen + 127) / 128) * B * KH;
+  const double tiles = (128.0 + (window < x_maxlen ? window : x_maxlen)) * (QH / KH) / 64.0;
+  int best = 1;
+  double best_cost = 0.0;
+  for (int s = 1; s <= 16; s *= 2) {
+    const double cost = (double)((wgs * s + c.slots - 1) / c.slots) * (c.fixed_us + tiles / s * c.tile_us);
+    if (s == 1 || cost < 0.9 * best_cost) { best = s; best_cost = cost; }
+  }
+  return best;
+}
+
 int nsa_swa_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                      const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                      const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
@@ -443,7 +487,10 @@ int nsa_swa_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
   NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
   p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
   p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
-  p.dkv_mode = dkv_is_f32 ? 1 : 0;
+  NSA_REQUIRE(dkv_is_f32 >= 0 && dkv_is_f32 <= 2, NSA_ERR_BAD_ARG, "swa_bwd_dkdv: dkv_is_f32 %d not in {0,1,2}",
+              dkv_is_f32);
+  p.dkv_mode = dkv_is_f32 == 2 ? 3 : dkv_is_f32;
+  p.grid_chunks = dkv_is_f32 == 2 ? nsa_swa_bwd_dkdv_splits(B, x_maxlen, QH, KH, D, VD, window) : 1;
   p.x_cu = x_cu; p.k_cu = x_cu;
   p.window = window;
   return nsa_bwd_dkdv_launch(p, 1, B, x_maxlen, x_maxlen, D, VD, 0, (hipStream_t)stream);

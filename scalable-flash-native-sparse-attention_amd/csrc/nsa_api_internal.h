@@ -89,8 +89,8 @@ struct NsaBwdTileParams {
   int G, KH;
   float scale_log2, sm_scale;
   int kernel_size, stride, window;
-  int q_chunk_tokens;          // compressed dkdv: query tokens per grid.x chunk
-  int grid_chunks;             // compressed dkdv: chunks per key tile in grid.x (set by the launcher)
+  int q_chunk_tokens;          // compressed / window dkdv: query tokens per grid.x chunk
+  int grid_chunks;             // window dkdv with dkv_mode 3: query chunks per key tile in grid.x
 };
 
 int nsa_bwd_dq_tile_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int D, int VD,

@@ -5,8 +5,8 @@
 //   dV^T += dO^T P,  dK^T += Q^T dS      (Q^T / dO^T fragments via ds_read_b64_tr_b16)
 // MODE_CMP: rows are all later queries of the sequence, split in chunks over grid.x, fp32 atomics
 //           (upstream flash_nsa/ops/compress_attn.py:193-376)
-// MODE_SWA: rows are the <= W+NW*32 queries whose window contains the keys, plain stores
-//           (upstream: FlashAttention backward, flash_nsa/ops/sliding_window_attention.py:98-157)
+// MODE_SWA: rows are the <= W+NW*32 queries whose window contains the keys: one workgroup per key tile and plain
+//           stores, or, where that leaves CUs without work, cut over grid.x with fp32 atomics (upstream: FlashAttention backward, flash_nsa/ops/sliding_window_attention.py:98-157)
 // MODE_SLC: rows are gathered through the inverse index (selection block -> tokens that selected it), lists are
 //           cut into chunks over grid.x, fp32 atomics (upstream flash_nsa/ops/select_attn.py:147-328)
 #include "nsa_common.h"
@@ -18,8 +18,10 @@ constexpr int MODE_CMP = 0;
 constexpr int MODE_SWA = 1;
 constexpr int MODE_SLC = 2;
 
+// Up to 64 channels the accumulators and K / V fragments leave room for two waves per SIMD (window branch, 40 ragged
+// sequences, 16 q / 2 kv heads: 430 -> 191 us together with the epilogue through LDS).
 template <int D, int VD, int MODE, int NW, int KB>
-__global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(NsaBwdTileParams p) {
+__global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_kernel(NsaBwdTileParams p) {
   constexpr int NT = NW * 64;
   constexpr int KPW = 32 * KB;   // keys per wave: KB blocks of 32, every Q / dO fragment read from LDS serves KB MFMAs
   constexpr int KW = NW * KPW;
@@ -27,8 +29,9 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(NsaBwdTileParams p) {
   constexpr int QLD = D + NSA_LDS_PAD;
   constexpr int OLD = VD + NSA_LDS_PAD;
   constexpr int T_INVALID = -0x40000000;
-  __shared__ __attribute__((aligned(16))) bf16_t Qs[RT * QLD];
-  __shared__ __attribute__((aligned(16))) bf16_t dOs[RT * OLD];
+  __shared__ __attribute__((aligned(16))) bf16_t rows_s[RT * (QLD + OLD)];  // Q rows, dO rows; epilogue: dK / dV rows
+  bf16_t* const Qs = rows_s;
+  bf16_t* const dOs = rows_s + RT * QLD;
   __shared__ __attribute__((aligned(16))) float lse_s[RT];
   __shared__ __attribute__((aligned(16))) float delta_s[RT];
   __shared__ __attribute__((aligned(16))) int t_s[RT];
@@ -103,10 +106,12 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(NsaBwdTileParams p) {
     // sub-block of a wide one, leaves the upper waves without keys)
     if (MODE == MODE_SLC) nkeys = min(xl, (key0 / p.block_size + 1) * p.block_size);
     if (MODE == MODE_SWA) {
-      key0 = blockIdx.x * KW;
+      const int ktile = blockIdx.x / p.grid_chunks;
+      key0 = ktile * KW;
       if (key0 >= nkeys) return;
-      row_begin = key0 * G;
-      row_end = min(xl, key0 + KW + p.window) * G;
+      const int ta = key0 + (blockIdx.x - ktile * p.grid_chunks) * p.q_chunk_tokens;
+      row_begin = ta * G;
+      row_end = min(min(xl, key0 + KW + p.window), ta + p.q_chunk_tokens) * G;
     } else if (key0 >= nkeys) {
       return;
     }
@@ -500,47 +505,72 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(NsaBwdTileParams p) {
   int64_t slot = 0;
   if (MODE == MODE_CMP) slot = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * p.KH + kh;
   else if (MODE == MODE_SLC) slot = ((int64_t)kh * gridDim.x + blockIdx.x) * gridDim.y + blockIdx.y;
-  auto emit = [&](void* base, int64_t off, f32x4 val) {
-    if (p.dkv_mode == 0) {
-      *reinterpret_cast<bf16x4*>((bf16_t*)base + off) = pack4(val[0], val[1], val[2], val[3]);
-    } else if (p.dkv_mode == 1 || p.dkv_mode == 4) {
-      *reinterpret_cast<f32x4*>((float*)base + off) = val;
-    } else {
-      float* dst = (float*)base + off;
+  // The accumulators hold one key per lane, so writing them as they lie would touch 32 rows with every instruction
+  // (and turn every fp32 atomic addition into a cache line of its own).  They pass through LDS instead, CW channels of
+  // the wave's 32 keys at a time, and leave as whole row pieces: one addition per lane on CW consecutive floats.
+  // Fixed cost of a workgroup (128 keys, d = 128): about 90 -> 12 us.
+  constexpr int WAVE_BYTES = RT * (QLD + OLD) * 2 / NW / 16 * 16;
+  constexpr int CW = WAVE_BYTES >= 32 * 68 * 4 ? 64 : (WAVE_BYTES >= 32 * 36 * 4 ? 32 : 16);
+  constexpr int ELD = CW + 4;
+  static_assert(32 * ELD * 4 <= WAVE_BYTES, "the row tiles hold the epilogue's strip of every wave");
+  static_assert(CW <= D || D == 32, "");
+  __syncthreads();  // all waves are done with the row tiles
+  if (!wave_has_keys) return;
+  float* const strip = reinterpret_cast<float*>(reinterpret_cast<char*>(rows_s) + wave * WAVE_BYTES);
+  auto emit = [&](auto& acc, auto width_tag, void* base, int64_t off, int64_t row_stride, float scale, int n_keys) {
+    constexpr int W = decltype(width_tag)::value;
+    constexpr int C = CW < W ? CW : W;  // channels per strip
 #pragma unroll
-      for (int e = 0; e < 4; e++) unsafeAtomicAdd(dst + e, val[e]);
+    for (int c0 = 0; c0 < W; c0 += C) {
+#pragma unroll
+      for (int q4 = 0; q4 < C / 8; q4++) {
+        const int dt = (c0 + q4 * 8) / 32, i4 = q4 % 4;
+        // strips of 16 channels start inside a 32-channel accumulator block
+        const int i0 = (C < 32 ? ((c0 % 32) / 8 + q4) : i4) * 4;
+        *reinterpret_cast<f32x4*>(&strip[l32 * ELD + q4 * 8 + hl * 4]) =
+            f32x4{acc[dt][i0] * scale, acc[dt][i0 + 1] * scale, acc[dt][i0 + 2] * scale, acc[dt][i0 + 3] * scale};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (p.dkv_mode == 3) {
+        constexpr int RPI = 64 / C;  // rows per instruction
+        const int r0 = lane / C, col = lane % C;
+#pragma unroll
+        for (int r = 0; r < 32; r += RPI)
+          if (r + r0 < n_keys)
+            unsafeAtomicAdd((float*)base + off + (int64_t)(r + r0) * row_stride + c0 + col, strip[(r + r0) * ELD + col]);
+      } else {
+        constexpr int LPR = C / 4;   // lanes per row, four channels each
+        const int r0 = lane / LPR, col = (lane % LPR) * 4;
+#pragma unroll
+        for (int r = 0; r < 32; r += 64 / LPR) {
+          if (r + r0 >= n_keys) continue;
+          const f32x4 val = *reinterpret_cast<const f32x4*>(&strip[(r + r0) * ELD + col]);
+          const int64_t at = off + (int64_t)(r + r0) * row_stride + c0 + col;
+          if (p.dkv_mode == 0) *reinterpret_cast<bf16x4*>((bf16_t*)base + at) = pack4(val[0], val[1], val[2], val[3]);
+          else *reinterpret_cast<f32x4*>((float*)base + at) = val;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   };
 #pragma unroll
   for (int kb = 0; kb < KB; kb++) {
-    const int my_key = kw0 + kb * 32 + l32;
-    if (my_key >= nkeys) continue;
-    int64_t koff = ((int64_t)kbase + my_key) * p.dk_sr + (int64_t)kh * p.dk_sh;
-    int64_t voff = ((int64_t)kbase + my_key) * p.dv_sr + (int64_t)kh * p.dv_sh;
-    void* dk_base = p.dk;
-    void* dv_base = p.dv;
+    const int k0 = kw0 + kb * 32;
+    const int n_keys = min(32, nkeys - k0);
+    if (n_keys <= 0) continue;
     if (p.dkv_mode == 4) {
-      koff = (slot * KW + (my_key - key0)) * D;
-      voff = (slot * KW + (my_key - key0)) * VD;
-      dk_base = p.part_dk;
-      dv_base = p.part_dv;
+      const int64_t row = slot * KW + (k0 - key0);
+      emit(dkacc[kb], std::integral_constant<int, D>{}, p.part_dk, row * D, D, osc, n_keys);
+      emit(dvacc[kb], std::integral_constant<int, VD>{}, p.part_dv, row * VD, VD, 1.f, n_keys);
+    } else {
+      const int64_t row = (int64_t)kbase + k0;
+      emit(dkacc[kb], std::integral_constant<int, D>{}, p.dk, row * p.dk_sr + (int64_t)kh * p.dk_sh, p.dk_sr, osc, n_keys);
+      emit(dvacc[kb], std::integral_constant<int, VD>{}, p.dv, row * p.dv_sr + (int64_t)kh * p.dv_sh, p.dv_sr, 1.f, n_keys);
     }
-#pragma unroll
-    for (int dt = 0; dt < D / 32; dt++)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        int d = dt * 32 + i4 * 8 + hl * 4;
-        emit(dk_base, koff + d, f32x4{dkacc[kb][dt][i4 * 4 + 0] * osc, dkacc[kb][dt][i4 * 4 + 1] * osc,
-                                   dkacc[kb][dt][i4 * 4 + 2] * osc, dkacc[kb][dt][i4 * 4 + 3] * osc});
-      }
-#pragma unroll
-    for (int dt = 0; dt < VD / 32; dt++)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        int d = dt * 32 + i4 * 8 + hl * 4;
-        emit(dv_base, voff + d, f32x4{dvacc[kb][dt][i4 * 4 + 0], dvacc[kb][dt][i4 * 4 + 1], dvacc[kb][dt][i4 * 4 + 2],
-                                   dvacc[kb][dt][i4 * 4 + 3]});
-      }
   }
 }
 
@@ -570,14 +600,17 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
     }
   } else if (mode == MODE_SWA) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;
+    const int KW = 4 * 32 * (kb_cmp == 2 ? 2 : 1);
+    p.grid_chunks = p.dkv_mode == 3 ? p.grid_chunks : 1;
+    p.q_chunk_tokens = cdiv_i(KW + p.window, p.grid_chunks);
     if constexpr (KB2_BUILT) {
       if (kb_cmp == 2) {
-        dim3 grid(cdiv_i(max_k_len, 256), B, p.KH);
+        dim3 grid(cdiv_i(max_k_len, 256) * p.grid_chunks, B, p.KH);
         bwd_dkdv_kernel<D, VD, MODE_SWA, 4, 2><<<grid, 256, 0, stream>>>(p);
         return nsa_check_launch("bwd_dkdv_kernel");
       }
     }
-    dim3 grid(cdiv_i(max_k_len, 128), B, p.KH);
+    dim3 grid(cdiv_i(max_k_len, 128) * p.grid_chunks, B, p.KH);
     bwd_dkdv_kernel<D, VD, MODE_SWA, 4, 1><<<grid, 256, 0, stream>>>(p);
   } else {
     if (n_items_bound <= 0) return NSA_OK;

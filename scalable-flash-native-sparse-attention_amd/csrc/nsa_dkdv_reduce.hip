@@ -8,45 +8,52 @@
 
 namespace {
 
-// compressed branch: grid (key tiles, B, KH).  The work items of a key tile are consecutive in the dk/dv kernel's
-// grid.x (key-tile major), one per query chunk that sees the tile.
+// compressed branch: grid (key tiles x pieces of 256 sums, B, KH), one thread per four channels of a key.  The work
+// items of a key tile are consecutive in the dk/dv kernel's grid.x (key-tile major), one per query chunk that sees the
+// tile.  The sum is a chain of loads from slots that lie KH * KW rows apart: eight are in flight at once, and a tile is
+// spread over many workgroups, since short batches have few tiles and many chunks (one sequence of 4096 tokens, 16 q /
+// 1 kv heads, 64 chunks: 650 us with a workgroup per tile, 5 us so).
 template <int KW>
-__global__ __launch_bounds__(256) void cmp_dkdv_reduce_kernel(NsaBwdTileParams p, int D, int VD, int grid_x_items) {
-  const int ktile = blockIdx.x, b = blockIdx.y, kh = blockIdx.z;
+__global__ __launch_bounds__(256) void cmp_dkdv_reduce_kernel(NsaBwdTileParams p, int D, int VD, int grid_x_items,
+                                                              int pieces) {
+  const int ktile = blockIdx.x / pieces, b = blockIdx.y, kh = blockIdx.z;
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
   const int kbase = p.k_cu[b];
   const int nkeys = p.k_cu[b + 1] - kbase;
   const int key0 = ktile * KW;
-  if (key0 >= nkeys) return;
+  const int n4k = D / 4, n4v = VD / 4;
+  const int per_key = n4k + n4v;
+  const int e = (blockIdx.x - ktile * pieces) * 256 + threadIdx.x;
+  const int kl = e / per_key, c4 = e - kl * per_key;
+  if (kl >= min(KW, nkeys - key0)) return;
   // the enumeration of bwd_dkdv_kernel MODE_CMP
   const int nch = cdiv_i(xl, p.q_chunk_tokens);
   int start = 0;
   for (int kt = 0; kt < ktile; kt++)
     start += nch - min(nch, (p.stride * kt * KW + p.kernel_size - 1) / p.q_chunk_tokens);
-  const int fc = min(nch, (p.stride * key0 + p.kernel_size - 1) / p.q_chunk_tokens);
-  const int first = p.stride * key0 + p.kernel_size - 1;
-  const int n4k = D / 4, n4v = VD / 4;
-  const int per_key = n4k + n4v;
-  const int nk_here = min(KW, nkeys - key0);
-  for (int e = threadIdx.x; e < nk_here * per_key; e += 256) {
-    const int kl = e / per_key, c4 = e - kl * per_key;
-    const bool is_v = c4 >= n4k;
-    const int d = (is_v ? c4 - n4k : c4) * 4;
-    const int W = is_v ? VD : D;
-    const float* part = is_v ? p.part_dv : p.part_dk;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ch = fc; ch < nch; ch++) {
-      // chunks without a visible row wrote nothing
-      if (max(ch * p.q_chunk_tokens, first) >= min((ch + 1) * p.q_chunk_tokens, xl)) continue;
-      const int64_t slot = ((int64_t)b * grid_x_items + start + (ch - fc)) * p.KH + kh;
-      const f32x4 x = *reinterpret_cast<const f32x4*>(part + (slot * KW + kl) * W + d);
-      acc[0] += x[0]; acc[1] += x[1]; acc[2] += x[2]; acc[3] += x[3];
-    }
-    float* dst = is_v ? (float*)p.dv + ((int64_t)kbase + key0 + kl) * p.dv_sr + (int64_t)kh * p.dv_sh + d
-                      : (float*)p.dk + ((int64_t)kbase + key0 + kl) * p.dk_sr + (int64_t)kh * p.dk_sh + d;
-    *reinterpret_cast<f32x4*>(dst) = acc;
+  // chunk fc holds the tile's first visible row (there is one: the tile has keys)
+  const int fc = (p.stride * key0 + p.kernel_size - 1) / p.q_chunk_tokens;
+  const bool is_v = c4 >= n4k;
+  const int d = (is_v ? c4 - n4k : c4) * 4;
+  const int W = is_v ? VD : D;
+  const int64_t slot0 = ((int64_t)b * grid_x_items + start) * p.KH + kh;
+  const float* src = (is_v ? p.part_dv : p.part_dk) + (slot0 * KW + kl) * W + d;
+  const int64_t step = (int64_t)p.KH * KW * W;
+  const int n = nch - fc;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int ch = 0;
+  for (; ch + 8 <= n; ch += 8) {
+    f32x4 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = *reinterpret_cast<const f32x4*>(src + (ch + u) * step);
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc += x[u];
   }
+  for (; ch < n; ch++) acc += *reinterpret_cast<const f32x4*>(src + ch * step);
+  float* dst = is_v ? (float*)p.dv + ((int64_t)kbase + key0 + kl) * p.dv_sr + (int64_t)kh * p.dv_sh + d
+                    : (float*)p.dk + ((int64_t)kbase + key0 + kl) * p.dk_sr + (int64_t)kh * p.dk_sh + d;
+  *reinterpret_cast<f32x4*>(dst) = acc;
 }
 
 // selected branch: grid (selection blocks, sub-blocks, KH).  The work items of a block are the chunks of its token
@@ -97,9 +104,10 @@ int nsa_dkdv_reduce_cmp_launch(const NsaBwdTileParams& p, int B, int max_q_len, 
   const int grid_x_items = (int)(nsa_bwd_dkdv_cmp_slots(1, 1, max_q_len, max_k_len, p.q_chunk_tokens, p.kernel_size,
                                                          p.stride));
   if (grid_x_items <= 0) return NSA_OK;
-  dim3 grid(cdiv_i(max_k_len, KW), B, p.KH);
-  if (KW == 128) cmp_dkdv_reduce_kernel<128><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items);
-  else cmp_dkdv_reduce_kernel<256><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items);
+  const int pieces = cdiv_i(KW * (D + VD) / 4, 256);
+  dim3 grid(cdiv_i(max_k_len, KW) * pieces, B, p.KH);
+  if (KW == 128) cmp_dkdv_reduce_kernel<128><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces);
+  else cmp_dkdv_reduce_kernel<256><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces);
   return nsa_check_launch("cmp_dkdv_reduce_kernel");
 }
 

@@ -1,4 +1,6 @@
 """Argument checks shared by the operator wrappers."""
+import math
+
 import torch
 
 
@@ -28,6 +30,13 @@ def delta_of(o, do):
     _lib.call("nsa_delta", o.data_ptr(), o.stride(0), o.stride(1), do.data_ptr(), do.stride(0), do.stride(1),
               delta.data_ptr(), T, H, D, _lib.stream_ptr())
     return delta
+
+
+def zeros_pair(shape_a, shape_b, device):
+    """Two zero-filled fp32 tensors out of one allocation and one fill launch."""
+    a, b = math.prod(shape_a), math.prod(shape_b)
+    buf = torch.zeros(a + b, device=device, dtype=torch.float32)
+    return buf[:a].view(shape_a), buf[a:].view(shape_b)
 
 
 def dq_target(q, dq):

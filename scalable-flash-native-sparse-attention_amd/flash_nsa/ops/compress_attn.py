@@ -3,7 +3,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
-from ._common import check_thd, default_scale, delta_of, dq_target
+from ._common import check_thd, default_scale, delta_of, dq_target, zeros_pair
 
 
 def cmp_attn_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
@@ -24,16 +24,22 @@ def cmp_attn_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
     return o, lse
 
 
+# most scratch for the partial dk / dv of the compressed branch.  Slots and their sum are as fast as atomic additions
+# (d = 128, 64 q / 4 kv heads, atomics / slots: T = 1024 56 / 55 us, 4096 125 / 115, 8192 290 / 280, 16384 820 / 815),
+# but their size grows with the square of the sequence length.
+DKDV_SLOTS_LIMIT = 512 << 20
+
+
 def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None, helper=NSAHelper, delta=None,
                  q_chunk_tokens=0, finalize_dq=False, parts="both"):
     """Backward of compressed attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer, which is added into; with finalize_dq the fp32 buffer is
     only read and the returned dq is a fresh tensor in q's dtype holding buffer + this branch.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None).
-    dk, dv: fp32 [y_len,KH,*].  dkdv_repeat=False (default, as upstream): the work items (query chunks) add their
-    partial results with fp32 atomics, so the summation order changes from run to run; dkdv_repeat=True (or
-    NSAHelper.set_deterministic(True)): every work item stores into its own slot of a scratch buffer and a second
-    launch sums the slots in a fixed order -- bit-identical results across runs.
+    dk, dv: fp32 [y_len,KH,*].  Every work item (query chunk of a key tile) stores its partial result into its own slot
+    of a scratch buffer and a second launch sums the slots in a fixed order -- bit-identical results across runs.
+    Where the slots would take more than DKDV_SLOTS_LIMIT bytes and neither dkdv_repeat nor
+    NSAHelper.set_deterministic(True) asks for that order, the work items add with fp32 atomics instead.
     delta may be passed when already known (delta[T,QH] fp32 = rowsum(o*do)).
     q_chunk_tokens: queries per work item of the dk/dv kernel (0: chosen by the library from the sizes)."""
     check_thd(do, "do")
@@ -61,15 +67,19 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
             _lib.call("nsa_cmp_attn_bwd_dq", *common, dq_buf.data_ptr(), dq_buf.stride(0), dq_buf.stride(1), mode,
                       *tail)
     if parts in ("both", "dkdv"):
-        dk = torch.zeros(Y, KH, D, device=q.device, dtype=torch.float32)
-        dv = torch.zeros(Y, KH, VD, device=q.device, dtype=torch.float32)
         sizes = (helper.batch, helper.x_maxlen, helper.y_maxlen, QH, KH, D, VD, helper.kernel_size, helper.stride,
                  q_chunk_tokens)
+        need = _lib.value("nsa_cmp_attn_bwd_dkdv_det_bytes", *sizes)
+        slots = dkdv_repeat or getattr(helper, "deterministic", False) or need <= DKDV_SLOTS_LIMIT
+        if slots:
+            dk = torch.empty(Y, KH, D, device=q.device, dtype=torch.float32)
+            dv = torch.empty(Y, KH, VD, device=q.device, dtype=torch.float32)
+        else:
+            dk, dv = zeros_pair((Y, KH, D), (Y, KH, VD), q.device)
         args = (*common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0), dv.stride(1),
                 helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), *sizes, sm_scale)
-        if dkdv_repeat or getattr(helper, "deterministic", False):
-            ws = torch.empty(max(_lib.value("nsa_cmp_attn_bwd_dkdv_det_bytes", *sizes), 1), dtype=torch.uint8,
-                             device=q.device)
+        if slots:
+            ws = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
             _lib.call("nsa_cmp_attn_bwd_dkdv_det", *args, ws.data_ptr(), ws.numel(), _lib.stream_ptr())
         else:
             _lib.call("nsa_cmp_attn_bwd_dkdv", *args, _lib.stream_ptr())

@@ -4,7 +4,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
-from ._common import check_thd, default_scale, delta_of, dq_target
+from ._common import check_thd, default_scale, delta_of, dq_target, zeros_pair
 
 
 def swa_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
@@ -24,7 +24,8 @@ def swa_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
 
 def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq=None, dkv_fp32=False, parts="both"):
     """Backward of the window branch.  Returns (dq, dk, dv); dq is a fresh bf16 tensor or the caller's fp32
-    buffer (added into); dk/dv are freshly written (bf16, or fp32 when dkv_fp32), one writer per element.
+    buffer (added into); dk/dv are fresh (bf16, or fp32 when dkv_fp32): one writer per element, or, for batches that do
+    not fill the GPU and unless NSAHelper.set_deterministic is on, summed in fp32 with atomics.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None), so that a caller can put the
     two on different streams."""
     check_thd(do, "do")
@@ -43,12 +44,21 @@ def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq
                   helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH, KH, D, VD, helper.window_size,
                   sm_scale, _lib.stream_ptr())
     if parts in ("both", "dkdv"):
-        kv_dtype = torch.float32 if dkv_fp32 else k.dtype
-        dk = torch.empty(T, KH, D, device=q.device, dtype=kv_dtype)
-        dv = torch.empty(T, KH, VD, device=q.device, dtype=kv_dtype)
+        # batches whose key tiles do not fill the GPU: the queries of a tile are cut as well and added with atomics
+        split = (not helper.deterministic and
+                 _lib.value("nsa_swa_bwd_dkdv_splits", helper.batch, helper.x_maxlen, QH, KH, D, VD,
+                            helper.window_size) > 1)
+        if split:
+            dk, dv = zeros_pair((T, KH, D), (T, KH, VD), q.device)
+        else:
+            kv_dtype = torch.float32 if dkv_fp32 else k.dtype
+            dk = torch.empty(T, KH, D, device=q.device, dtype=kv_dtype)
+            dv = torch.empty(T, KH, VD, device=q.device, dtype=kv_dtype)
         _lib.call("nsa_swa_bwd_dkdv", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(),
-                  dv.stride(0), dv.stride(1), int(dkv_fp32), helper.x_cu_seqlens.data_ptr(), helper.batch,
-                  helper.x_maxlen, QH, KH, D, VD, helper.window_size, sm_scale, _lib.stream_ptr())
+                  dv.stride(0), dv.stride(1), 2 if split else int(dkv_fp32), helper.x_cu_seqlens.data_ptr(),
+                  helper.batch, helper.x_maxlen, QH, KH, D, VD, helper.window_size, sm_scale, _lib.stream_ptr())
+        if split and not dkv_fp32:
+            dk, dv = dk.to(k.dtype), dv.to(v.dtype)
     return dq_buf, dk, dv
 
 

@@ -481,3 +481,39 @@ def test_deterministic_dk_dv(device, block_size, lens, QH, KH):
     c = run()
     for name, x, y in zip(("dq", "dk", "dv", "dw"), a, c):
         assert_close(x, y.float(), f"{name}: deterministic vs default mode", atol=2e-3, rtol=8e-3, row_scale=True)
+
+
+@pytest.mark.parametrize("QH,KH,D", [(16, 2, 128), (4, 4, 64), (6, 2, 32)])
+@pytest.mark.parametrize("splits", [2, 16])
+def test_dk_dv_query_chunks(device, QH, KH, D, splits, monkeypatch):
+    """The window dk/dv kernel with the queries of a key tile cut into chunks (fewer rows than chunks in the short
+    sequences) against one workgroup per key tile, and the compressed one with atomic additions against slots.  The
+    products are the same, only the order of the fp32 sums over at most 16 / 12 partial results differs: at most
+    16 x 2^-24 of the sum of their magnitudes, which stays below 1e-4 of the row's rms for these inputs."""
+    from flash_nsa import _lib
+    from flash_nsa.ops import compress_attn as ca
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.sliding_window_attention import swa_fwd, swa_bwd
+    cu = make_cu([700, 0, 1, 129, 33])
+    T = int(cu[-1])
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, seed=140)]
+    do = randn_bf16(T, QH, D, seed=144).to(device)
+    setup_helper(cu.to(device), window_size=200)
+    o, lse = swa_fwd(q, k, v)
+    runs = {}
+    try:
+        for s in (1, splits):
+            _lib.call("nsa_set_tuning", b"swa_dkdv_splits", s)
+            runs[s] = swa_bwd(q, k, v, o, lse, do, dkv_fp32=True, parts="dkdv")[1:]
+    finally:
+        _lib.call("nsa_reset_tuning")
+    for a, b, name in zip(runs[splits], runs[1], ("dk", "dv")):
+        assert_close(a, b, f"window {name}", atol=1e-5, rtol=1e-4, row_scale=True)
+    ck, cv = mean_pooling_fwd(k), mean_pooling_fwd(v)
+    o, lse = ca.cmp_attn_fwd(q, ck, cv)
+    slots = ca.cmp_attn_bwd(q, ck, cv, o, lse, do, parts="dkdv", q_chunk_tokens=64)[1:]
+    monkeypatch.setattr(ca, "DKDV_SLOTS_LIMIT", 0)
+    atomics = ca.cmp_attn_bwd(q, ck, cv, o, lse, do, parts="dkdv", q_chunk_tokens=64)[1:]
+    for a, b, name in zip(atomics, slots, ("dk", "dv")):
+        assert_close(a, b, f"compressed {name}", atol=1e-5, rtol=1e-4, row_scale=True)
+    setup_helper(cu.to(device))
