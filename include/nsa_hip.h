@@ -93,12 +93,30 @@ int nsa_topk_select_ws(const void* q, int64_t q_st, int64_t q_sh, const void* ck
                        const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D, int kernel_size, int stride,
                        int block_size, int top_n, int num_init, int num_local, int ignore_index, float sm_scale,
                        int total_tokens, void* workspace, int64_t workspace_bytes, void* stream);
+/* nsa_topk_select_ws without the selection of the queries at positions below t_begin: where the two launches run, their
+ * topk rows are not written */
+int nsa_topk_select_ws_from(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
+                            const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                            int64_t tk_st, float* imp_out, int64_t imp_sh, int64_t imp_st, int imp_cols,
+                            const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
+                            int kernel_size, int stride, int block_size, int top_n, int num_init, int num_local,
+                            int ignore_index, float sm_scale, int total_tokens, int t_begin, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 /* flash_nsa/ops/select_attn.py:439-507 slc_attn_fwd */
 int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                      const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st,
                      void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
                      const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD, int block_size,
                      int top_n, float sm_scale, void* stream);
+/* the same where the caller knows that the queries at positions below all_below (<= top_n * block_size) select every
+ * block they can see, as the selector's own output does: they run as full causal attention on the dense tile kernel and
+ * their topk rows are not read.  Likewise nsa_slc_attn_bwd_dq_full and nsa_paged_slc_attn_fwd_full (max_context: a bound
+ * of the longest context, 0 if unknown) */
+int nsa_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                          const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh,
+                          int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st,
+                          int64_t lse_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
+                          int block_size, int top_n, int all_below, float sm_scale, void* stream);
 
 /* ---- backward ----
  * dq_mode: 0 = store bf16, 1 = store fp32, 2 = add into an existing fp32 buffer (single writer per element).
@@ -171,6 +189,23 @@ int nsa_slc_attn_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
                         int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream);
+int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
+                        int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
+                        int KH, int D, int VD, int block_size, int top_n, int all_below,
+                        float sm_scale, void* stream);
+/* dk/dv of the queries at positions below all_below, added into the caller's fp32 buffers; with an inverse index that
+ * leaves them out (nsa_build_inverse_index_from) this completes nsa_slc_attn_bwd_dkdv.  ordered: the summation order does
+ * not change between runs */
+int nsa_slc_attn_bwd_dkdv_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                                const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st,
+                                int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta,
+                                int64_t delta_st, int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh,
+                                float* dv, int64_t dv_sr, int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen,
+                                int QH, int KH, int D, int VD, int all_below, int ordered, float sm_scale,
+                                void* stream);
 /* flash_nsa/ops/topk.py:889-945 get_bind_from_find: inverse of the selection as a CSR.
  *   csr_off  [KH][nblk_total+1] absolute start of each (kv head, global block) list inside csr_tok
  *   csr_tok  [KH*T*top_n]       query tokens (index local to their sequence), ascending within a list
@@ -185,6 +220,11 @@ int nsa_build_inverse_index(const int32_t* topk, int64_t tk_sh, int64_t tk_st, i
                             const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
                             int chunk_tokens, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
                             int32_t* workspace, int64_t workspace_elems, void* stream);
+/* the same over the queries at positions >= t_begin only */
+int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
+                                 const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
+                                 int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
+                                 int32_t* workspace, int64_t workspace_elems, void* stream);
 /* flash_nsa/ops/select_attn.py:593-637 (_dkdv_kernel launch): fp32 atomic adds into dk/dv [T,KH,*];
  * blk_seq [nblk_total] = sequence of each global block; n_items_bound >= max over kv heads of item_off[kh][nblk_total] */
 int nsa_slc_attn_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
@@ -246,6 +286,14 @@ int nsa_paged_topk_select_ws(const void* q, int64_t q_st, int64_t q_sh, const vo
                              int block_size, int top_n, int num_init, int num_local, int ignore_index,
                              float sm_scale, int total_tokens, void* workspace, int64_t workspace_bytes,
                              void* stream);
+int nsa_paged_topk_select_ws_from(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+                                  int64_t k_sh, const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk,
+                                  int64_t tk_sh, int64_t tk_st, const int32_t* x_cu, const int32_t* context_lens,
+                                  const int32_t* cmp_block_tables, int table_stride, int page_size, int B,
+                                  int x_maxlen, int fixed_num_slc_blocks, int QH, int KH, int D, int kernel_size,
+                                  int stride, int block_size, int top_n, int num_init, int num_local,
+                                  int ignore_index, float sm_scale, int total_tokens, int t_begin, void* workspace,
+                                  int64_t workspace_bytes, void* stream);
 /* flash_nsa/inference/select_attn.py:103-166 slc_attn_prefill */
 int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
                            int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, const int32_t* topk,
@@ -253,6 +301,13 @@ int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
                            int QH, int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream);
+int nsa_paged_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+                           int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, const int32_t* topk,
+                           int64_t tk_sh, int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse,
+                           int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
+                           const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
+                           int QH, int KH, int D, int VD, int block_size, int top_n, int all_below,
+                           int max_context, float sm_scale, void* stream);
 
 /* flash_nsa/inference/compress_kv.py:191-220 mean_pooling_prefill (in-pool write at flat row slot) */
 int nsa_paged_pool_prefill(void* cache, int64_t c_sr, int64_t c_sh, const int32_t* y_cu, const int32_t* block_tables,

@@ -8,6 +8,7 @@
 #include <atomic>
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include "../../include/nsa_hip.h"
 
 static thread_local char g_err[512] = "";
 
@@ -137,7 +138,7 @@ static int topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const voi
                             int64_t tk_st, float* imp_out, int64_t imp_sh, int64_t imp_st, int imp_cols,
                             const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
                             int kernel_size, int stride, int block_size, int top_n, int num_init, int num_local,
-                            int ignore_index, float sm_scale, int total_tokens, void* workspace,
+                            int ignore_index, float sm_scale, int total_tokens, int t_begin, void* workspace,
                             int64_t workspace_bytes, void* stream) {
   int rc = check_heads("topk_select", QH, KH, D, 32);
   if (rc) return rc;
@@ -159,6 +160,7 @@ static int topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const voi
   p.top_n = top_n; p.num_init = num_init; p.num_local = num_local; p.ignore_index = ignore_index;
   p.nb_max = (x_maxlen + block_size - 1) / block_size;
   if (p.nb_max < 1) p.nb_max = 1;
+  p.t_begin = t_begin;
   if (workspace != nullptr && nsa_tuning_knob("topk_two_pass", 1) != 0 && nsa_topk_two_pass_supported(p, D))
     return nsa_topk_two_pass_launch(p, false, B, x_maxlen, total_tokens, D, workspace, workspace_bytes,
                                     (hipStream_t)stream);
@@ -173,7 +175,7 @@ int nsa_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void* ck, i
                     void* stream) {
   return topk_select_impl(q, q_st, q_sh, ck, ck_sr, ck_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, imp_out, imp_sh,
                           imp_st, imp_cols, x_cu, y_cu, B, x_maxlen, QH, KH, D, kernel_size, stride, block_size,
-                          top_n, num_init, num_local, ignore_index, sm_scale, 0, nullptr, 0, stream);
+                          top_n, num_init, num_local, ignore_index, sm_scale, 0, 0, nullptr, 0, stream);
 }
 
 int64_t nsa_topk_workspace_bytes(int total_tokens, int max_blocks, int KH) {
@@ -187,12 +189,33 @@ int nsa_topk_select_ws(const void* q, int64_t q_st, int64_t q_sh, const void* ck
                        const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D, int kernel_size, int stride,
                        int block_size, int top_n, int num_init, int num_local, int ignore_index, float sm_scale,
                        int total_tokens, void* workspace, int64_t workspace_bytes, void* stream) {
+  return nsa_topk_select_ws_from(q, q_st, q_sh, ck, ck_sr, ck_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, imp_out,
+                                 imp_sh, imp_st, imp_cols, x_cu, y_cu, B, x_maxlen, QH, KH, D, kernel_size, stride,
+                                 block_size, top_n, num_init, num_local, ignore_index, sm_scale, total_tokens, 0,
+                                 workspace, workspace_bytes, stream);
+}
+
+int nsa_topk_select_ws_from(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
+                            const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                            int64_t tk_st, float* imp_out, int64_t imp_sh, int64_t imp_st, int imp_cols,
+                            const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
+                            int kernel_size, int stride, int block_size, int top_n, int num_init, int num_local,
+                            int ignore_index, float sm_scale, int total_tokens, int t_begin, void* workspace,
+                            int64_t workspace_bytes, void* stream) {
   NSA_REQUIRE(total_tokens >= 0 && (workspace == nullptr || workspace_bytes > 0), NSA_ERR_BAD_ARG,
               "topk_select_ws: bad token count %d or workspace size %lld", total_tokens, (long long)workspace_bytes);
   return topk_select_impl(q, q_st, q_sh, ck, ck_sr, ck_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, imp_out, imp_sh,
                           imp_st, imp_cols, x_cu, y_cu, B, x_maxlen, QH, KH, D, kernel_size, stride, block_size,
-                          top_n, num_init, num_local, ignore_index, sm_scale, total_tokens, workspace,
+                          top_n, num_init, num_local, ignore_index, sm_scale, total_tokens, t_begin, workspace,
                           workspace_bytes, stream);
+}
+
+// The queries at positions below all_below (at most top_n blocks) select every block they can see: full causal
+// attention, on the dense tile kernel, whose 64-key tiles serve eight tokens instead of one.
+static int check_all_below(const char* who, int all_below, int top_n, int block_size) {
+  NSA_REQUIRE(all_below >= 0 && all_below <= top_n * block_size, NSA_ERR_BAD_ARG,
+              "%s: all_below %d exceeds top_n %d blocks of %d", who, all_below, top_n, block_size);
+  return NSA_OK;
 }
 
 int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
@@ -200,11 +223,37 @@ int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
                      void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
                      const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD, int block_size,
                      int top_n, float sm_scale, void* stream) {
+  return nsa_slc_attn_fwd_full(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, topk, tk_sh, tk_st, o, o_st, o_sh, lse,
+                               lse_st, lse_sh, x_cu, B, x_maxlen, QH, KH, D, VD, block_size, top_n, 0, sm_scale,
+                               stream);
+}
+
+int nsa_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                          const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh,
+                          int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st,
+                          int64_t lse_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
+                          int block_size, int top_n, int all_below, float sm_scale, void* stream) {
   int rc = check_heads("slc_attn_fwd", QH, KH, D, VD);
   if (rc) return rc;
   NSA_REQUIRE(block_size % 32 == 0 && block_size > 0, NSA_ERR_UNSUPPORTED,
               "slc_attn_fwd: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "slc_attn_fwd: top_n %d must be in [1,64]", top_n);
+  rc = check_all_below("slc_attn_fwd", all_below, top_n, block_size);
+  if (rc) return rc;
+  if (all_below > 0) {
+    NsaFwdTileParams p{};
+    p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
+    p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
+    p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
+    p.o = (bf16_t*)o; p.o_st = o_st; p.o_sh = o_sh;
+    p.lse = lse; p.lse_st = lse_st; p.lse_sh = lse_sh;
+    p.x_cu = x_cu; p.k_cu = x_cu;
+    p.G = QH / KH; p.KH = KH;
+    p.scale_log2 = sm_scale * NSA_LOG2E;
+    p.kernel_size = 1; p.stride = 1; p.window = all_below; p.t_end = all_below;
+    rc = nsa_fwd_tile_launch(p, 1, false, B, x_maxlen, D, VD, (hipStream_t)stream);
+    if (rc) return rc;
+  }
   NsaSlcParams p{};
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
@@ -215,6 +264,7 @@ int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
   p.x_cu = x_cu;
   p.G = QH / KH; p.KH = KH; p.top_n = top_n; p.block_size = block_size;
   p.scale_log2 = sm_scale * NSA_LOG2E;
+  p.t_begin = all_below;
   return nsa_slc_fwd_launch(p, false, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
@@ -502,13 +552,38 @@ int nsa_slc_attn_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
                         int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream) {
+  return nsa_slc_attn_bwd_dq_full(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh,
+                                  delta, delta_st, delta_sh, topk, tk_sh, tk_st, dq, dq_st, dq_sh, dq_mode, x_cu, B,
+                                  x_maxlen, QH, KH, D, VD, block_size, top_n, 0, sm_scale, stream);
+}
+
+int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
+                        int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
+                        int KH, int D, int VD, int block_size, int top_n, int all_below,
+                        float sm_scale, void* stream) {
   int rc = check_heads("slc_attn_bwd_dq", QH, KH, D, VD);
   if (rc) return rc;
   NSA_REQUIRE(block_size % 32 == 0 && block_size > 0, NSA_ERR_UNSUPPORTED,
               "slc_attn_bwd_dq: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "slc_attn_bwd_dq: top_n %d must be in [1,64]", top_n);
   NSA_REQUIRE(dq_mode >= 0 && dq_mode <= 2, NSA_ERR_BAD_ARG, "slc_attn_bwd_dq: dq_mode %d not in {0,1,2}", dq_mode);
+  rc = check_all_below("slc_attn_bwd_dq", all_below, top_n, block_size);
+  if (rc) return rc;
+  if (all_below > 0) {
+    BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+                delta_sh};
+    NsaBwdTileParams t = make_bwd(c, QH, KH, sm_scale);
+    t.dq = dq; t.dq_st = dq_st; t.dq_sh = dq_sh; t.dq_mode = dq_mode;
+    t.x_cu = x_cu; t.k_cu = x_cu;
+    t.window = all_below; t.t_end = all_below;
+    rc = nsa_bwd_dq_tile_launch(t, 1, B, x_maxlen, D, VD, (hipStream_t)stream);
+    if (rc) return rc;
+  }
   NsaSlcBwdDqParams p{};
+  p.t_begin = all_below;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
   p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
@@ -521,6 +596,30 @@ int nsa_slc_attn_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k
   p.G = QH / KH; p.KH = KH; p.top_n = top_n; p.block_size = block_size;
   p.scale_log2 = sm_scale * NSA_LOG2E; p.sm_scale = sm_scale;
   return nsa_slc_bwd_dq_launch(p, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
+int nsa_slc_attn_bwd_dkdv_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                                const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st,
+                                int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta,
+                                int64_t delta_st, int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh,
+                                float* dv, int64_t dv_sr, int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen,
+                                int QH, int KH, int D, int VD, int all_below, int ordered, float sm_scale,
+                                void* stream) {
+  int rc = check_heads("slc_attn_bwd_dkdv_dense", QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(all_below > 0, NSA_ERR_BAD_ARG, "slc_attn_bwd_dkdv_dense: all_below %d must be positive", all_below);
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
+  p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
+  p.dkv_mode = 3;
+  const int len = x_maxlen < all_below ? x_maxlen : all_below;
+  // one workgroup per key tile adds exactly once to every element: no order to vary
+  p.grid_chunks = ordered ? 1 : nsa_swa_bwd_dkdv_splits(B, len, QH, KH, D, VD, len);
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.window = all_below; p.t_end = all_below;
+  return nsa_bwd_dkdv_launch(p, 1, B, x_maxlen, x_maxlen, D, VD, 0, (hipStream_t)stream);
 }
 
 static int slc_attn_bwd_dkdv_impl(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
@@ -639,15 +738,12 @@ int nsa_paged_cmp_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
   return nsa_fwd_tile_launch(p, 0, true, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
-int nsa_paged_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
-                      const void* v_cache, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh,
-                      float* lse, int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
-                      const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen, int QH,
-                      int KH, int D, int VD, int window, float sm_scale, void* stream) {
-  int rc = check_heads("paged_swa_fwd", QH, KH, D, VD);
-  if (rc) return rc;
-  rc = check_page("paged_swa_fwd", page_size);
-  if (rc) return rc;
+static NsaFwdTileParams paged_window_params(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+                                            int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, void* o,
+                                            int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
+                                            const int32_t* x_cu, const int32_t* context_lens,
+                                            const int32_t* block_tables, int table_stride, int page_size, int QH,
+                                            int KH, int window, int t_end, float sm_scale) {
   NsaFwdTileParams p{};
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k_cache; p.k_sr = k_sr; p.k_sh = k_sh;
@@ -658,8 +754,23 @@ int nsa_paged_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_c
   p.table = block_tables; p.table_stride = table_stride; p.page_size = page_size;
   p.G = QH / KH; p.KH = KH;
   p.scale_log2 = sm_scale * NSA_LOG2E;
-  p.kernel_size = 1; p.stride = 1; p.window = window;
-  return nsa_fwd_tile_launch(p, 1, true, B, x_maxlen, D, VD, (hipStream_t)stream);
+  p.kernel_size = 1; p.stride = 1; p.window = window; p.t_end = t_end;
+  return p;
+}
+
+int nsa_paged_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                      const void* v_cache, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh,
+                      float* lse, int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
+                      const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen, int QH,
+                      int KH, int D, int VD, int window, float sm_scale, void* stream) {
+  int rc = check_heads("paged_swa_fwd", QH, KH, D, VD);
+  if (rc) return rc;
+  rc = check_page("paged_swa_fwd", page_size);
+  if (rc) return rc;
+  return nsa_fwd_tile_launch(paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh,
+                                                 lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
+                                                 page_size, QH, KH, window, 0, sm_scale),
+                             1, true, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
 static int paged_topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
@@ -668,7 +779,7 @@ static int paged_topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, con
                           const int32_t* cmp_block_tables, int table_stride, int page_size, int B, int x_maxlen,
                           int fixed_num_slc_blocks, int QH, int KH, int D, int kernel_size, int stride,
                           int block_size, int top_n, int num_init, int num_local, int ignore_index, float sm_scale,
-                          int total_tokens, void* workspace, int64_t workspace_bytes, void* stream) {
+                          int total_tokens, int t_begin, void* workspace, int64_t workspace_bytes, void* stream) {
   int rc = check_heads("paged_topk_select", QH, KH, D, 32);
   if (rc) return rc;
   rc = check_nsa_sizes("paged_topk_select", kernel_size, stride, block_size);
@@ -691,6 +802,7 @@ static int paged_topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, con
   p.kernel_size = kernel_size; p.stride = stride; p.block_size = block_size;
   p.top_n = top_n; p.num_init = num_init; p.num_local = num_local; p.ignore_index = ignore_index;
   p.nb_max = fixed_num_slc_blocks;
+  p.t_begin = t_begin;
   if (workspace != nullptr && nsa_tuning_knob("topk_two_pass", 1) != 0 && nsa_topk_two_pass_supported(p, D))
     return nsa_topk_two_pass_launch(p, true, B, x_maxlen, total_tokens, D, workspace, workspace_bytes,
                                     (hipStream_t)stream);
@@ -707,7 +819,7 @@ int nsa_paged_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void*
   return paged_topk_select_impl(q, q_st, q_sh, k_cache, k_sr, k_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, x_cu,
                                 context_lens, cmp_block_tables, table_stride, page_size, B, x_maxlen,
                                 fixed_num_slc_blocks, QH, KH, D, kernel_size, stride, block_size, top_n, num_init,
-                                num_local, ignore_index, sm_scale, 0, nullptr, 0, stream);
+                                num_local, ignore_index, sm_scale, 0, 0, nullptr, 0, stream);
 }
 
 int nsa_paged_topk_select_ws(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
@@ -718,13 +830,29 @@ int nsa_paged_topk_select_ws(const void* q, int64_t q_st, int64_t q_sh, const vo
                              int block_size, int top_n, int num_init, int num_local, int ignore_index,
                              float sm_scale, int total_tokens, void* workspace, int64_t workspace_bytes,
                              void* stream) {
+  return nsa_paged_topk_select_ws_from(q, q_st, q_sh, k_cache, k_sr, k_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st,
+                                       x_cu, context_lens, cmp_block_tables, table_stride, page_size, B, x_maxlen,
+                                       fixed_num_slc_blocks, QH, KH, D, kernel_size, stride, block_size, top_n,
+                                       num_init, num_local, ignore_index, sm_scale, total_tokens, 0, workspace,
+                                       workspace_bytes, stream);
+}
+
+int nsa_paged_topk_select_ws_from(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+                                  int64_t k_sh, const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk,
+                                  int64_t tk_sh, int64_t tk_st, const int32_t* x_cu, const int32_t* context_lens,
+                                  const int32_t* cmp_block_tables, int table_stride, int page_size, int B,
+                                  int x_maxlen, int fixed_num_slc_blocks, int QH, int KH, int D, int kernel_size,
+                                  int stride, int block_size, int top_n, int num_init, int num_local,
+                                  int ignore_index, float sm_scale, int total_tokens, int t_begin, void* workspace,
+                                  int64_t workspace_bytes, void* stream) {
   NSA_REQUIRE(total_tokens >= 0 && (workspace == nullptr || workspace_bytes > 0), NSA_ERR_BAD_ARG,
               "paged_topk_select_ws: bad token count %d or workspace size %lld", total_tokens,
               (long long)workspace_bytes);
   return paged_topk_select_impl(q, q_st, q_sh, k_cache, k_sr, k_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, x_cu,
                                 context_lens, cmp_block_tables, table_stride, page_size, B, x_maxlen,
                                 fixed_num_slc_blocks, QH, KH, D, kernel_size, stride, block_size, top_n, num_init,
-                                num_local, ignore_index, sm_scale, total_tokens, workspace, workspace_bytes, stream);
+                                num_local, ignore_index, sm_scale, total_tokens, t_begin, workspace, workspace_bytes,
+                                stream);
 }
 
 int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
@@ -733,6 +861,18 @@ int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
                            int QH, int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream) {
+  return nsa_paged_slc_attn_fwd_full(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, topk, tk_sh, tk_st, o,
+                                     o_st, o_sh, lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
+                                     page_size, B, x_maxlen, QH, KH, D, VD, block_size, top_n, 0, 0, sm_scale, stream);
+}
+
+int nsa_paged_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+                           int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, const int32_t* topk,
+                           int64_t tk_sh, int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse,
+                           int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
+                           const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
+                           int QH, int KH, int D, int VD, int block_size, int top_n, int all_below,
+                           int max_context, float sm_scale, void* stream) {
   int rc = check_heads("paged_slc_attn_fwd", QH, KH, D, VD);
   if (rc) return rc;
   rc = check_page("paged_slc_attn_fwd", page_size);
@@ -740,7 +880,17 @@ int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
   NSA_REQUIRE(block_size % 32 == 0 && block_size > 0, NSA_ERR_UNSUPPORTED,
               "paged_slc_attn_fwd: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "paged_slc_attn_fwd: top_n %d must be in [1,64]", top_n);
+  rc = check_all_below("paged_slc_attn_fwd", all_below, top_n, block_size);
+  if (rc) return rc;
+  if (all_below > 0) {
+    rc = nsa_fwd_tile_launch(paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh,
+                                                 lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
+                                                 page_size, QH, KH, all_below, all_below, sm_scale),
+                             1, true, B, x_maxlen, D, VD, (hipStream_t)stream);
+    if (rc || (max_context > 0 && max_context <= all_below)) return rc;
+  }
   NsaSlcParams p{};
+  p.t_begin = all_below;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k_cache; p.k_sr = k_sr; p.k_sh = k_sh;
   p.v = (const bf16_t*)v_cache; p.v_sr = v_sr; p.v_sh = v_sh;

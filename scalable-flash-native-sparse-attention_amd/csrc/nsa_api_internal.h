@@ -18,6 +18,7 @@ struct NsaFwdTileParams {
   int G, KH;
   float scale_log2;
   int kernel_size, stride, window;
+  int t_end;                                // > 0: only queries at positions below it
 };
 
 struct NsaSlcParams {
@@ -32,6 +33,7 @@ struct NsaSlcParams {
   const int32_t* table; int table_stride; int page_size;
   int G, KH, top_n, block_size;
   float scale_log2;
+  int t_begin;                                // only queries at positions from here on
 };
 
 struct NsaTopkParams {
@@ -48,6 +50,7 @@ struct NsaTopkParams {
   float scale_log2;
   int kernel_size, stride, block_size, top_n, num_init, num_local, ignore_index;
   int nb_max;  // selection blocks of the longest context
+  int t_begin;     // two-launch form: queries at positions below it need no selection (their topk rows stay unwritten)
   int seg_blocks;  // set by the launcher: 0 = an LDS score row holds all nb_max blocks; else blocks per segment
 };
 
@@ -89,6 +92,7 @@ struct NsaBwdTileParams {
   int G, KH;
   float scale_log2, sm_scale;
   int kernel_size, stride, window;
+  int t_end;                   // window mode: > 0: only queries at positions below it
   int q_chunk_tokens;          // compressed / window dkdv: query tokens per grid.x chunk
   int grid_chunks;             // window dkdv with dkv_mode 3: query chunks per key tile in grid.x
 };
@@ -117,6 +121,7 @@ struct NsaSlcBwdDqParams {
   const int32_t* topk; int64_t tk_sh, tk_st;
   const int32_t* x_cu;
   int G, KH, top_n, block_size;
+  int t_begin;                                // only queries at positions from here on
   float scale_log2, sm_scale;
 };
 int nsa_slc_bwd_dq_launch(const NsaSlcBwdDqParams& p, int B, int max_q_len, int D, int VD, hipStream_t stream);

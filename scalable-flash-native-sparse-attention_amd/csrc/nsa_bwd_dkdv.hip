@@ -76,7 +76,8 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
     b = blockIdx.y;
   }
   const int x0 = p.x_cu[b];
-  const int xl = p.x_cu[b + 1] - x0;
+  int xl = p.x_cu[b + 1] - x0;
+  if (MODE == MODE_SWA && p.t_end > 0) xl = min(xl, p.t_end);  // queries, and so keys, of the sequence's start only
   int nkeys, kbase;
   if (MODE == MODE_CMP) {
     kbase = p.k_cu[b];
@@ -600,6 +601,7 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
     }
   } else if (mode == MODE_SWA) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;
+    if (p.t_end > 0 && p.t_end < max_k_len) max_k_len = p.t_end;
     const int KW = 4 * 32 * (kb_cmp == 2 ? 2 : 1);
     p.grid_chunks = p.dkv_mode == 3 ? p.grid_chunks : 1;
     p.q_chunk_tokens = cdiv_i(KW + p.window, p.grid_chunks);

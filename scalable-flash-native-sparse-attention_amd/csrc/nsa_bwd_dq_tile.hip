@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
 
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int rows_total = xl * G;
+  const int rows_total = (MODE == MODE_SWA && p.t_end > 0 ? min(xl, p.t_end) : xl) * G;
   const int r0 = blockIdx.x * ROWS_WG;
   if (r0 >= rows_total) return;
   int nkeys, kbase;
@@ -228,6 +228,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
 template <int MODE>
 int dispatch(const NsaBwdTileParams& p, int B, int max_q_len, int D, int VD, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
+  if (MODE == MODE_SWA && p.t_end > 0 && p.t_end < max_q_len) max_q_len = p.t_end;
   dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
   const int minb = nsa_tuning_knob("dq_min_blocks", 2);
   if (D == 128 && VD == 128) {

@@ -59,11 +59,11 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int rows_total = xl * G;
-  const int r0 = blockIdx.x * ROWS_WG;
-  if (r0 >= rows_total) return;
   const int ctx = PAGED ? p.ctx_lens[b] : xl;
   const int qoff = ctx - xl;
+  const int rows_total = (MODE == MODE_SWA && p.t_end > 0 ? min(xl, p.t_end - qoff) : xl) * G;
+  const int r0 = blockIdx.x * ROWS_WG;
+  if (r0 >= rows_total) return;
   int nkeys, kbase = 0;
   if (MODE == MODE_CMP) {
     nkeys = ctx >= p.kernel_size ? (ctx - p.kernel_size) / p.stride + 1 : 0;
@@ -390,6 +390,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 template <int D, int VD, int MODE, bool PAGED>
 int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
+  if (MODE == MODE_SWA && p.t_end > 0 && p.t_end < max_q_len) max_q_len = p.t_end;
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there;
   // the window branch, with its short key loops, and d=192, whose swizzled addresses cost registers, are faster with
   // register staging); 1..4 force one variant for experiments

@@ -5,6 +5,7 @@
 // Upstream: flash_nsa/ops/topk.py:782-945 (get_bind_from_find, dense scatter + per-row sort).
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include "../../include/nsa_hip.h"
 
 namespace {
 
@@ -23,7 +24,8 @@ __device__ __forceinline__ int find_seq(const int32_t* x_cu, int B, int tok) {
 
 // grid (nchunks, KH), 256 threads, dynamic LDS nblk ints
 __global__ void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
-                                 const int32_t* kblk_cu, int B, int T, int nblk, int block_size, int32_t* chunk_cnt) {
+                                 const int32_t* kblk_cu, int B, int T, int nblk, int block_size, int t_begin,
+                                 int32_t* chunk_cnt) {
   extern __shared__ int hist[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
   for (int i = threadIdx.x; i < nblk; i += blockDim.x) hist[i] = 0;
@@ -36,7 +38,7 @@ __global__ void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_
     int s = idx % top_n;
     int b = find_seq(x_cu, B, tok);
     int n = tok - x_cu[b];
-    if (s < min(top_n, n / block_size + 1)) {
+    if (n >= t_begin && s < min(top_n, n / block_size + 1)) {
       int j = topk[(int64_t)kh * tk_sh + (int64_t)tok * tk_st + s];
       int nb = kblk_cu[b + 1] - kblk_cu[b];
       if (j >= 0 && j < nb) atomicAdd(&hist[kblk_cu[b] + j], 1);
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
 // grid (nchunks, KH), 64 threads: in-order fill
 __global__ __launch_bounds__(64) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
                                                       const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
-                                                      int nblk, int block_size, const int32_t* chunk_base,
+                                                      int nblk, int block_size, int t_begin, const int32_t* chunk_base,
                                                       const int32_t* csr_off, int32_t* csr_tok) {
   extern __shared__ int cursor[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(64) void csr_fill_kernel(const int32_t* topk, int64
         x_begin = x_cu[b], x_end = x_cu[b + 1], kb_begin = kblk_cu[b], nb = kblk_cu[b + 1] - kb_begin;
       }
       const int n = tok - x_begin;
-      const int nvalid = min(top_n, n / block_size + 1);
+      const int nvalid = n >= t_begin ? min(top_n, n / block_size + 1) : 0;
       if (lane < nvalid) {
         const int j = cur[u];
         if (j >= 0 && j < nb) {
@@ -171,6 +173,14 @@ int nsa_build_inverse_index(const int32_t* topk, int64_t tk_sh, int64_t tk_st, i
                             const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
                             int chunk_tokens, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
                             int32_t* workspace, int64_t workspace_elems, void* stream) {
+  return nsa_build_inverse_index_from(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, KH, nblk_total, block_size,
+                                      chunk_tokens, 0, csr_off, csr_tok, item_off, workspace, workspace_elems, stream);
+}
+
+int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
+                                 const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
+                                 int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
+                                 int32_t* workspace, int64_t workspace_elems, void* stream) {
   if (T <= 0 || B <= 0 || nblk_total <= 0) return NSA_OK;
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "build_inverse_index: top_n %d must be in [1,64]", top_n);
   NSA_REQUIRE(chunk_tokens >= 1, NSA_ERR_BAD_ARG, "build_inverse_index: chunk_tokens must be positive");
@@ -186,7 +196,7 @@ int nsa_build_inverse_index(const int32_t* topk, int64_t tk_sh, int64_t tk_st, i
   size_t lds = (size_t)nblk_total * sizeof(int);
   dim3 grid(nchunks, KH);
   csr_count_kernel<<<grid, 256, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
-                                          workspace);
+                                          t_begin, workspace);
   int rc = nsa_check_launch("csr_count_kernel");
   if (rc) return rc;
   csr_scan_kernel<<<KH, 1024, 0, s>>>(workspace, nchunks, nblk_total, (int64_t)T * top_n, chunk_tokens, csr_off,
@@ -194,7 +204,7 @@ int nsa_build_inverse_index(const int32_t* topk, int64_t tk_sh, int64_t tk_st, i
   rc = nsa_check_launch("csr_scan_kernel");
   if (rc) return rc;
   csr_fill_kernel<<<grid, 64, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
-                                        workspace, csr_off, csr_tok);
+                                        t_begin, workspace, csr_off, csr_tok);
   return nsa_check_launch("csr_fill_kernel");
 }
 

@@ -30,7 +30,7 @@ __global__ __launch_bounds__(256, 2) void slc_dq_kernel(NsaSlcBwdDqParams p) {
 
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int n = blockIdx.x * 4 + wave;
+  const int n = p.t_begin + blockIdx.x * 4 + wave;
   if (n >= xl) return;
   const int t = n;
   const int64_t tok = x0 + n;
@@ -185,6 +185,7 @@ __global__ __launch_bounds__(256, 2) void slc_dq_kernel(NsaSlcBwdDqParams p) {
 }  // namespace
 
 int nsa_slc_bwd_dq_launch(const NsaSlcBwdDqParams& p, int B, int max_q_len, int D, int VD, hipStream_t stream) {
+  max_q_len -= p.t_begin;
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
   dim3 grid(cdiv_i(max_q_len, 4), B, p.KH * ((p.G + 15) / 16));
   if (D == 128 && VD == 128) slc_dq_kernel<128, 128><<<grid, 256, 0, stream>>>(p);

@@ -37,9 +37,9 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
 
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int n = blockIdx.x * 4 + wave;
-  if (n >= xl) return;
   const int ctx = PAGED ? p.ctx_lens[b] : xl;
+  const int n = (p.t_begin > 0 ? max(p.t_begin - (ctx - xl), 0) : 0) + blockIdx.x * 4 + wave;
+  if (n >= xl) return;
   const int t = n + (ctx - xl);
   const int64_t tok = x0 + n;
   const int32_t* table = PAGED ? p.table + (int64_t)b * p.table_stride : nullptr;
@@ -223,6 +223,7 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
 
 template <int D, int VD, bool PAGED>
 int launch_slc(const NsaSlcParams& p, int B, int max_q_len, hipStream_t stream) {
+  if (!PAGED) max_q_len -= p.t_begin;
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
   dim3 grid(cdiv_i(max_q_len, 4), B, p.KH * ((p.G + 15) / 16));
   slc_fwd_kernel<D, VD, PAGED><<<grid, 256, 0, stream>>>(p);

@@ -47,7 +47,6 @@ struct SlotMap {
 
 struct ScoreWs {
   float* imp;      // [KH][ntok][row_stride] block scores of the chunk's tokens
-  int32_t* pos;    // [ntok] absolute position of the token in its context, -1: token not in this launch
   int tok_lo, tok_hi, row_stride;
 };
 
@@ -95,6 +94,7 @@ __global__ __launch_bounds__(256, NSA_TOPK_SCORE_WAVES) void topk_score_kernel(N
 
   // workgroup: keys that its last token sees, tiles to score and tiles to fold (every block up to the last token's)
   const int t_hi_wg = min(n0 + TWG - 1, xl - 1) + qoff;
+  if (t_hi_wg < p.t_begin) return;  // no token of the workgroup needs a selection
   const int key_end = t_hi_wg >= Kz - 1 ? min((t_hi_wg - Kz + 1) / St + 1, nkeys) : 0;
   const int n_score = (key_end + KT - 1) / KT;
   const int n_fold = (t_hi_wg / Bs) / BPT + 1;
@@ -264,21 +264,15 @@ __global__ __launch_bounds__(256, NSA_TOPK_SCORE_WAVES) void topk_score_kernel(N
     do_tile(tile, std::integral_constant<int, 0>{});
     if (tile + 1 < ntiles) do_tile(tile + 1, std::integral_constant<int, 1>{});
   }
-  // positions of the workgroup's tokens, for the pick kernel (kv head 0 writes them)
-  if (kh == 0 && tid < TWG) {
-    const int n = n0 + tid;
-    const int64_t tok = (int64_t)x0 + n;
-    if (n < xl && tok >= ws.tok_lo && tok < ws.tok_hi) ws.pos[tok - ws.tok_lo] = n + qoff;
-  }
 }
 
 struct PickParams {
   const float* imp;      // [KH][ntok][row_stride]
-  const int32_t* pos;    // [ntok]
+  const int32_t* x_cu; const int32_t* ctx_lens; int B;  // ctx_lens: null where the context is the sequence itself
   int32_t* topk; int64_t tk_sh, tk_st;
   float* imp_out; int64_t imp_sh, imp_st; int imp_cols;
   int ntok, tok_lo, row_stride, nb_max, KH;
-  int block_size, top_n, num_init, num_local, ignore_index;
+  int block_size, top_n, num_init, num_local, ignore_index, t_begin;
 };
 
 __global__ __launch_bounds__(256) void topk_pick_kernel(PickParams p) {
@@ -288,10 +282,19 @@ __global__ __launch_bounds__(256) void topk_pick_kernel(PickParams p) {
   if (r >= (int64_t)p.KH * p.ntok) return;
   const int kh = (int)(r / p.ntok);
   const int tr = (int)(r - (int64_t)kh * p.ntok);
-  const int t = __builtin_amdgcn_readfirstlane(p.pos[tr]);
-  if (t < 0) return;
-  const float* imp = p.imp + r * p.row_stride;
   const int64_t tok = (int64_t)p.tok_lo + tr;
+  // sequence of the token: its number of sequence ends at or before the token, counted 64 at a time
+  int b = 0;
+  for (int i0 = 0; i0 < p.B; i0 += 64) {
+    const bool before = i0 + lane < p.B && p.x_cu[i0 + lane + 1] <= tok;
+    b += (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
+  }
+  if (b >= p.B) return;  // past the last sequence
+  const int x_end = p.x_cu[b + 1];
+  const int t = __builtin_amdgcn_readfirstlane((p.ctx_lens != nullptr ? p.ctx_lens[b] : x_end - p.x_cu[b]) - x_end +
+                                               (int)tok);
+  if (t < p.t_begin) return;
+  const float* imp = p.imp + r * p.row_stride;
   const int nk = t / p.block_size;
   const int jmax = min(nk, p.nb_max - 1);
   if (p.imp_out != nullptr) {
@@ -307,11 +310,6 @@ __global__ __launch_bounds__(256) void topk_pick_kernel(PickParams p) {
   else if (jmax < 1024) result = select_blocks_short_list<16>(imp, t, min(cap, 1024), p, lane, cand_v[wave], cand_i[wave]);
   else result = select_blocks_short_list<32>(imp, t, min(cap, 2048), p, lane, cand_v[wave], cand_i[wave]);
   if (lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + tok * p.tk_st + lane] = result;
-}
-
-__global__ void fill_i32_kernel(int32_t* dst, int n, int32_t value) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = value;
 }
 
 template <int D, int GP, bool PAGED>
@@ -344,8 +342,8 @@ bool nsa_topk_two_pass_supported(const NsaTopkParams& p, int D) {
   return p.nb_max <= 2048;
 }
 
-// bytes per token of the chunk: its score rows for every kv head and its position
-int64_t nsa_topk_two_pass_bytes_per_token(int KH, int nb_max) { return (int64_t)KH * row_stride_of(nb_max) * 4 + 4; }
+// bytes per token of the chunk: its score rows for every kv head
+int64_t nsa_topk_two_pass_bytes_per_token(int KH, int nb_max) { return (int64_t)KH * row_stride_of(nb_max) * 4; }
 
 int nsa_topk_two_pass_launch(const NsaTopkParams& p, bool paged, int B, int max_q_len, int total_tokens, int D,
                              void* workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -363,16 +361,15 @@ int nsa_topk_two_pass_launch(const NsaTopkParams& p, bool paged, int B, int max_
     const int ntok = (int)min((int64_t)total_tokens - lo, chunk);
     ScoreWs ws;
     ws.imp = (float*)workspace;
-    ws.pos = (int32_t*)((char*)workspace + (((int64_t)p.KH * ntok * rs * 4 + 255) & ~(int64_t)255));
     ws.tok_lo = (int)lo; ws.tok_hi = (int)lo + ntok; ws.row_stride = rs;
-    fill_i32_kernel<<<cdiv_i(ntok, 256), 256, 0, stream>>>(ws.pos, ntok, -1);
     if (D == 128) paged ? dispatch_score<128, true>(p, ws, B, max_q_len, stream) : dispatch_score<128, false>(p, ws, B, max_q_len, stream);
     else if (D == 64) paged ? dispatch_score<64, true>(p, ws, B, max_q_len, stream) : dispatch_score<64, false>(p, ws, B, max_q_len, stream);
     else paged ? dispatch_score<192, true>(p, ws, B, max_q_len, stream) : dispatch_score<192, false>(p, ws, B, max_q_len, stream);
     int rc = nsa_check_launch("topk_score_kernel");
     if (rc) return rc;
     PickParams pp{};
-    pp.imp = ws.imp; pp.pos = ws.pos;
+    pp.imp = ws.imp;
+    pp.x_cu = p.x_cu; pp.ctx_lens = paged ? p.ctx_lens : nullptr; pp.B = B; pp.t_begin = p.t_begin;
     pp.topk = p.topk; pp.tk_sh = p.tk_sh; pp.tk_st = p.tk_st;
     pp.imp_out = p.imp_out; pp.imp_sh = p.imp_sh; pp.imp_st = p.imp_st; pp.imp_cols = p.imp_cols;
     pp.ntok = ntok; pp.tok_lo = (int)lo; pp.row_stride = rs; pp.nb_max = p.nb_max; pp.KH = p.KH;

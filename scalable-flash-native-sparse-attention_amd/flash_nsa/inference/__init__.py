@@ -34,6 +34,8 @@ def nsa_prefill(q, k, v, w, x_cu_seqlens, y_cu_seqlens, x_maxlen, y_maxlen, cont
                              kernel_size=kernel_size, stride=stride)
         mean_pooling_prefill(v, y_cu_seqlens, y_maxlen, block_table=block_tables, slot_mapping=cmp_slot_mapping,
                              kernel_size=kernel_size, stride=stride)
+    # queries with at most top_n blocks in sight select them all; y_maxlen rows are complete below this many tokens
+    full = dict(all_below=top_n * block_size, max_context=kernel_size + int(y_maxlen) * stride - 1)
     cmp_o, lse = cmp_attn_prefill(q, k, v, x_cu_seqlens, x_maxlen, block_tables=cmp_block_tables,
                                   context_lens=context_lens, kernel_size=kernel_size, stride=stride,
                                   sm_scale=sm_scale)
@@ -41,9 +43,9 @@ def nsa_prefill(q, k, v, w, x_cu_seqlens, y_cu_seqlens, x_maxlen, y_maxlen, cont
                         context_lens=context_lens, fixed_y_maxlen=fixed_y_maxlen,
                         fixed_num_slc_blocks=fixed_num_slc_blocks, sm_scale=sm_scale, kernel_size=kernel_size,
                         stride=stride, block_size=block_size, top_n=top_n, num_inital=num_init_blocks,
-                        num_local=num_local_blocks)
+                        num_local=num_local_blocks, **full)
     slc_o, _ = slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables=block_tables,
-                                context_lens=context_lens, block_size=block_size, top_n=top_n, sm_scale=sm_scale)
+                                context_lens=context_lens, block_size=block_size, top_n=top_n, sm_scale=sm_scale, **full)
     swa_o = swa_prefill(q, k, v, x_cu_seqlens, x_maxlen, block_tables=block_tables, context_lens=context_lens,
                         window_size=window_size, sm_scale=sm_scale)
     return combine_prefill(cmp_o, slc_o, swa_o, w)

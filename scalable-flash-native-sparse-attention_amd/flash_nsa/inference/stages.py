@@ -129,8 +129,10 @@ def cmp_attn_decode(q, k, v, block_tables, context_lens, num_splits=0, kernel_si
 # ------------------------------------------------------------------------------------------------ top-k
 def topk_prefill(q, k, lse, x_cu_seqlens, x_maxlen, y_maxlen, block_tables, context_lens, fixed_y_maxlen=8192,
                  fixed_num_slc_blocks=2048, sm_scale=None, kernel_size=32, stride=16, block_size=64, top_n=16,
-                 num_inital=1, num_local=2):
-    """-> topk [KH,t,top_n] int32, unused slots = -1.  lse [QH,t] from cmp_attn_prefill."""
+                 num_inital=1, num_local=2, all_below=0, max_context=0):
+    """-> topk [KH,t,top_n] int32, unused slots = -1.  lse [QH,t] from cmp_attn_prefill.  all_below (<= top_n *
+    block_size): the rows of queries at positions below it, which select every block they can see, may stay
+    unwritten; max_context: a bound of the longest context (0: unknown)."""
     check_bf16(q)
     page, KH, D, ksr, ksh = _pool_args(k)
     t, QH, _ = q.shape
@@ -138,12 +140,14 @@ def topk_prefill(q, k, lse, x_cu_seqlens, x_maxlen, y_maxlen, block_tables, cont
     sm_scale = q.size(-1) ** -0.5 if sm_scale is None else sm_scale
     assert lse.dtype == torch.float32 and lse.shape == (QH, t)
     topk = torch.empty(KH, t, top_n, device=q.device, dtype=torch.int32)
+    if 0 < max_context <= all_below:
+        return topk
     ws = topk_workspace(t, int(fixed_num_slc_blocks), KH, q.device)
-    _lib.call("nsa_paged_topk_select_ws", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh,
+    _lib.call("nsa_paged_topk_select_ws_from", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh,
               lse.data_ptr(), lse.stride(1), lse.stride(0), topk.data_ptr(), topk.stride(0), topk.stride(1),
               _i32(x_cu_seqlens).data_ptr(), _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(),
               block_tables.stride(0), page, B, int(x_maxlen), int(fixed_num_slc_blocks), QH, KH, D, kernel_size,
-              stride, block_size, top_n, num_inital, num_local, -1, sm_scale, t, _lib.ptr(ws),
+              stride, block_size, top_n, num_inital, num_local, -1, sm_scale, t, all_below, _lib.ptr(ws),
               ws.numel() if ws is not None else 0, _lib.stream_ptr())
     return topk
 
@@ -159,8 +163,10 @@ def topk_decode(q, k, lse, block_tables, context_lens, fixed_y_maxlen=8192, fixe
 
 # ------------------------------------------------------------------------------------------------ selected / window
 def slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables, context_lens, block_size=64, top_n=16,
-                     sm_scale=None):
-    """-> (o [t,QH,VD], lse [t,QH])"""
+                     sm_scale=None, all_below=0, max_context=0):
+    """-> (o [t,QH,VD], lse [t,QH]).  all_below: the queries at positions below it are known to select every block they
+    can see (all_below <= top_n * block_size) and their rows of topk are not read; max_context: a bound of the longest
+    context (0: unknown)."""
     check_bf16(q)
     page, KH, D, ksr, ksh = _pool_args(k)
     _, _, VD, vsr, vsh = _pool_args(v)
@@ -170,11 +176,12 @@ def slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables, contex
     assert topk.dtype == torch.int32 and topk.shape == (KH, t, top_n) and topk.stride(-1) == 1
     o = torch.empty(t, QH, VD, device=q.device, dtype=q.dtype)
     lse = torch.empty(t, QH, device=q.device, dtype=torch.float32)
-    _lib.call("nsa_paged_slc_attn_fwd", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(),
+    _lib.call("nsa_paged_slc_attn_fwd_full", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(),
               vsr, vsh, topk.data_ptr(), topk.stride(0), topk.stride(1), o.data_ptr(), o.stride(0), o.stride(1),
               lse.data_ptr(), lse.stride(0), lse.stride(1), _i32(x_cu_seqlens).data_ptr(),
               _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(), block_tables.stride(0), page, B,
-              int(x_maxlen), QH, KH, D, VD, block_size, top_n, sm_scale, _lib.stream_ptr())
+              int(x_maxlen), QH, KH, D, VD, block_size, top_n, all_below, int(max_context), sm_scale,
+              _lib.stream_ptr())
     return o, lse
 
 

@@ -96,8 +96,8 @@ class NSAFunction(torch.autograd.Function):
         win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, H.cmp_k_method)
         win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method)
         cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
-        topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale)
-        slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale)
+        topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=H.all_below())
+        slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, all_below=H.all_below())
         swa_o, swa_lse = swa_fwd(q, k, v, sm_scale=sm_scale)
         out = combine_fwd(cmp_o, slc_o, swa_o, combine_weight)
 
@@ -127,7 +127,7 @@ class NSAFunction(torch.autograd.Function):
         if cmp_o is None:
             cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale, helper=helper)
         if slc_o is None:
-            slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, helper=helper)
+            slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, helper=helper, all_below=helper.all_below())
         if swa_o is None:
             swa_o, swa_lse = swa_fwd(q, k, v, sm_scale=sm_scale, helper=helper)
 
@@ -135,13 +135,14 @@ class NSAFunction(torch.autograd.Function):
         dcmp_o, dslc_o, dswa_o, dw, delta = combine_bwd(cmp_o, slc_o, swa_o, combine_weight, do, return_delta=True)
         dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         kw = dict(sm_scale=sm_scale, helper=helper)
+        skw = dict(kw, all_below=helper.all_below())
         if OVERLAP_STREAMS:
             main, side = torch.cuda.current_stream(), _side_stream(q.device)
             side.wait_stream(main)
             with torch.cuda.stream(side):
                 # dq chain: the selected branch (memory bound) stores, the window branch (matrix bound, with
                 # bandwidth to spare for the read-modify-write) adds, the compressed branch adds and writes q's dtype
-                slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **kw)
+                slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **skw)
                 swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dq=dq32, parts="dq", **kw)
                 dq, _, _ = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0],
                                         finalize_dq=True, parts="dq", **kw)
@@ -154,13 +155,13 @@ class NSAFunction(torch.autograd.Function):
             _, dcmp_k, dcmp_v = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, delta=delta[0], parts="dkdv",
                                              **kw)
             _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **skw)
         else:
             # the selected branch stores dq, the window branch adds to it and writes every element of dk / dv, to
             # which the selected branch then adds
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **skw)
             _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dq=dq32, dkv_fp32=True, **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **skw)
             dq, dcmp_k, dcmp_v = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0],
                                               finalize_dq=True, **kw)
         _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)

@@ -3,12 +3,14 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
-from ._common import check_thd, default_scale, delta_of, dq_target
+from ._common import check_thd, default_scale, delta_of, dq_target, zeros_pair
 
 
-def slc_attn_fwd(q, k, v, topk, sm_scale=None, helper=NSAHelper):
+def slc_attn_fwd(q, k, v, topk, sm_scale=None, helper=NSAHelper, all_below=0):
     """q [T,QH,D], k [T,KH,D], v [T,KH,VD], topk [KH,T,top_n] int32 -> o [T,QH,VD], lse [T,QH] fp32 (log2).
-    Query t of a sequence attends the keys <= t of the blocks in its first min(top_n, t//block+1) slots."""
+    Query t of a sequence attends the keys <= t of the blocks in its first min(top_n, t//block+1) slots.
+    all_below: the queries at positions below it are known to select every block they can see (as slc_topk_indices
+    lets them for all_below <= top_n * block_size); their rows of topk are then not read."""
     check_thd(q, "q"), check_thd(k, "k"), check_thd(v, "v")
     T, QH, D = q.shape
     _, KH, VD = v.shape
@@ -16,23 +18,24 @@ def slc_attn_fwd(q, k, v, topk, sm_scale=None, helper=NSAHelper):
     sm_scale = default_scale(q, sm_scale)
     o = torch.empty(T, QH, VD, device=q.device, dtype=q.dtype)
     lse = torch.empty(T, QH, device=q.device, dtype=torch.float32)
-    _lib.call("nsa_slc_attn_fwd", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
+    _lib.call("nsa_slc_attn_fwd_full", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
               v.data_ptr(), v.stride(0), v.stride(1), topk.data_ptr(), topk.stride(0), topk.stride(1), o.data_ptr(),
               o.stride(0), o.stride(1), lse.data_ptr(), lse.stride(0), lse.stride(1),
               helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH, KH, D, VD, helper.block_size,
-              topk.size(-1), sm_scale, _lib.stream_ptr())
+              topk.size(-1), all_below, sm_scale, _lib.stream_ptr())
     return o, lse
 
 
 def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=None, helper=NSAHelper, delta=None,
-                 bind=None, parts="both", dkdv_repeat=False):
+                 bind=None, parts="both", dkdv_repeat=False, all_below=0):
     """Backward of selected attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer (added into).  dk/dv: fp32 [T,KH,*]; the caller's buffers
     are added into, otherwise zero-filled ones are created.  dkdv_repeat=False (default): with fp32 atomics, so the
     summation order changes from run to run (as upstream's dkdv_repeat=False); dkdv_repeat=True (or
     NSAHelper.set_deterministic(True)): the work items store into slots of a scratch buffer that a second launch adds
     in a fixed order -- bit-identical results across runs.  `bind` is the inverse index from get_bind_from_find (built here when absent).
-    parts = "dq" / "dkdv" launches only that kernel (the other results are None)."""
+    parts = "dq" / "dkdv" launches only that kernel (the other results are None).
+    all_below: as in slc_attn_fwd (a given `bind` then has to leave those queries out)."""
     from .topk import get_bind_from_find
     check_thd(do, "do")
     T, QH, D = q.shape
@@ -46,23 +49,33 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     dq_buf = None
     if parts in ("both", "dq"):
         dq_buf, mode = dq_target(q, dq)
-        _lib.call("nsa_slc_attn_bwd_dq", *common, topk.data_ptr(), topk.stride(0), topk.stride(1), dq_buf.data_ptr(),
+        _lib.call("nsa_slc_attn_bwd_dq_full", *common, topk.data_ptr(), topk.stride(0), topk.stride(1), dq_buf.data_ptr(),
                   dq_buf.stride(0), dq_buf.stride(1), mode, helper.x_cu_seqlens.data_ptr(), helper.batch,
-                  helper.x_maxlen, QH, KH, D, VD, helper.block_size, topk.size(-1), sm_scale, _lib.stream_ptr())
+                  helper.x_maxlen, QH, KH, D, VD, helper.block_size, topk.size(-1), all_below, sm_scale,
+                  _lib.stream_ptr())
     if parts == "dq":
         return dq_buf, None, None
-    if dk is None:
+    if dk is None and dv is None:
+        dk, dv = zeros_pair((T, KH, D), (T, KH, VD), q.device)
+    elif dk is None:
         dk = torch.zeros(T, KH, D, device=q.device, dtype=torch.float32)
-    if dv is None:
+    elif dv is None:
         dv = torch.zeros(T, KH, VD, device=q.device, dtype=torch.float32)
     assert dk.dtype == torch.float32 and dv.dtype == torch.float32
+    ordered = dkdv_repeat or getattr(helper, "deterministic", False)
+    if all_below > 0:
+        _lib.call("nsa_slc_attn_bwd_dkdv_dense", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(),
+                  dv.stride(0), dv.stride(1), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH, KH, D,
+                  VD, all_below, int(ordered), sm_scale, _lib.stream_ptr())
+        if helper.x_maxlen <= all_below:
+            return dq_buf, dk, dv
     if bind is None:
-        bind = get_bind_from_find(topk, helper)
+        bind = get_bind_from_find(topk, helper, t_begin=all_below)
     args = (*common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0), dv.stride(1),
             helper.x_cu_seqlens.data_ptr(), helper.k_cu_seqlens.data_ptr(), helper.blk_seq.data_ptr(),
             bind["csr_off"].data_ptr(), bind["csr_tok"].data_ptr(), bind["item_off"].data_ptr(), bind["nblk"],
             bind["chunk_tokens"], bind["n_items_bound"], helper.batch, QH, KH, D, VD, helper.block_size, sm_scale)
-    if dkdv_repeat or getattr(helper, "deterministic", False):
+    if ordered:
         nbytes = _lib.value("nsa_slc_attn_bwd_dkdv_det_bytes", bind["n_items_bound"], KH, D, VD, helper.block_size)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=q.device)
         _lib.call("nsa_slc_attn_bwd_dkdv_det", *args, ws.data_ptr(), ws.numel(), _lib.stream_ptr())
@@ -73,10 +86,11 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
 
 class _SelectAttn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, topk, sm_scale):
-        o, lse = slc_attn_fwd(q, k, v, topk, sm_scale)
+    def forward(ctx, q, k, v, topk, sm_scale, all_below):
+        o, lse = slc_attn_fwd(q, k, v, topk, sm_scale, all_below=all_below)
         ctx.save_for_backward(q, k, v, topk, o, lse)
         ctx.sm_scale = sm_scale
+        ctx.all_below = all_below
         ctx.helper = NSAHelper.get_bwd_helper()
         return o
 
@@ -84,10 +98,11 @@ class _SelectAttn(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, topk, o, lse = ctx.saved_tensors
         do = do if do.stride(-1) == 1 else do.contiguous()
-        dq, dk, dv = slc_attn_bwd(q, k, v, topk, o, lse, do, sm_scale=ctx.sm_scale, helper=ctx.helper)
-        return dq, dk.to(k.dtype), dv.to(v.dtype), None, None
+        dq, dk, dv = slc_attn_bwd(q, k, v, topk, o, lse, do, sm_scale=ctx.sm_scale, helper=ctx.helper,
+                                  all_below=ctx.all_below)
+        return dq, dk.to(k.dtype), dv.to(v.dtype), None, None, None
 
 
-def select_attn(q, k, v, topk, sm_scale=None):
-    """Differentiable selected-block attention (no gradient flows into topk)."""
-    return _SelectAttn.apply(q, k, v, topk, sm_scale)
+def select_attn(q, k, v, topk, sm_scale=None, all_below=0):
+    """Differentiable selected-block attention (no gradient flows into topk); all_below as in slc_attn_fwd."""
+    return _SelectAttn.apply(q, k, v, topk, sm_scale, all_below)

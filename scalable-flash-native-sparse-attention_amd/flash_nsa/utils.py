@@ -164,6 +164,11 @@ class NSAHelper:
         cls._registered, cls._registered_version = x_cu_seqlens, x_cu_seqlens._version
 
     @classmethod
+    def all_below(cls):
+        """Positions whose queries select every block they can see: they have at most top_n blocks."""
+        return cls.top_n * cls.block_size
+
+    @classmethod
     def clear_tensor_data(cls, *tensors):
         for t in tensors:
             if isinstance(t, torch.Tensor):
@@ -185,3 +190,6 @@ class BwdNSAHelper:
     def __init__(self):
         for f in self._FIELDS:
             setattr(self, f, getattr(NSAHelper, f))
+
+    def all_below(self):
+        return self.top_n * self.block_size

@@ -517,3 +517,41 @@ def test_dk_dv_query_chunks(device, QH, KH, D, splits, monkeypatch):
     for a, b, name in zip(atomics, slots, ("dk", "dv")):
         assert_close(a, b, f"compressed {name}", atol=1e-5, rtol=1e-4, row_scale=True)
     setup_helper(cu.to(device))
+
+
+@pytest.mark.parametrize("QH,KH,D,block_size", [(16, 1, 128, 64), (3, 1, 64, 32), (24, 1, 128, 96)])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_selected_attention_of_queries_that_select_everything(device, QH, KH, D, block_size, ordered):
+    """slc_attn_fwd / slc_attn_bwd with all_below (dense tiles for the queries that see at most top_n blocks, gather for
+    the rest) against the gather for all of them: sequences that end one before, at and one after the boundary, inside
+    the first tile and far past it.  The two round P to bf16 against another running maximum, so each side's sum of
+    p v is off by at most 2^-9 of the sum of p |v| (below 1 for these N(0,1) values wherever more than one p counts,
+    and exact where one does), and an output by that twice plus its own rounding: 2^-8 + 2^-7 |o|.  The gradients are
+    taken from the same lse and outputs, so P is the same to fp32 rounding; its and dS's bf16 rounding may flip, by
+    2^-8 of a term in sums of many: 2^-7 of the row's rms and 2e-3."""
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
+    from flash_nsa.ops.topk import slc_topk_indices
+    n = 4 * block_size
+    cu = make_cu([n - 1, n, 0, n + 1, 1, 5 * n + 7, 33])
+    T = int(cu[-1])
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, seed=150)]
+    do = randn_bf16(T, QH, D, seed=154).to(device)
+    setup_helper(cu.to(device), block_size=block_size, top_n=4)
+    _, lse_c = cmp_attn_fwd(q, mean_pooling_fwd(k), mean_pooling_fwd(v))
+    full, _ = slc_topk_indices(q, mean_pooling_fwd(k), lse_c)
+    part = torch.full_like(full, -7)
+    topk, _ = slc_topk_indices(q, mean_pooling_fwd(k), lse_c, all_below=n)
+    pos = torch.cat([torch.arange(b - a) for a, b in zip(cu[:-1].tolist(), cu[1:].tolist())]).to(device)
+    part[:, pos >= n] = topk[:, pos >= n]
+    assert torch.equal(part[:, pos >= n], full[:, pos >= n])
+    ref = slc_attn_fwd(q, k, v, full)
+    out = slc_attn_fwd(q, k, v, part, all_below=n)   # rows of part below the boundary are invalid and must not be read
+    assert_close(out[0], ref[0].float(), "o", atol=2 ** -8, rtol=2 ** -7)
+    assert_close(out[1], ref[1], "lse", atol=1e-5, rtol=1e-5)
+    g_ref = slc_attn_bwd(q, k, v, full, *ref, do, dkdv_repeat=ordered)
+    g_out = slc_attn_bwd(q, k, v, part, *ref, do, dkdv_repeat=ordered, all_below=n)
+    for name, a, b in zip(("dq", "dk", "dv"), g_out, g_ref):
+        assert_close(a, b.float(), name, atol=2e-3, rtol=2 ** -7, row_scale=True)
+    setup_helper(cu.to(device))
