@@ -472,6 +472,22 @@ int nsa_decode_fused(const void* q, int64_t q_st, int64_t q_sh, const void* k_ca
                      int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks, int kernel_size, int stride,
                      int block_size, int top_n, int num_init, int num_local, int ignore_index, int window,
                      float sm_scale, void* stream);
+/* the same with scratch memory (16-byte aligned, nothing is kept in it between calls) of
+ * nsa_decode_fused_scratch_bytes(...): where that is not 0, large batches run two workgroups per CU instead of one and
+ * keep the probabilities that LDS does not hold in the scratch; with 192 q/k channels the scratch is required */
+int64_t nsa_decode_fused_scratch_bytes(int B, int KH, int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks,
+                                       int table_stride, int page_size);
+int nsa_decode_fused_ws(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
+                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
+                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                     int64_t tk_st, const int32_t* context_lens, const int32_t* block_tables, int table_stride,
+                     const int32_t* cmp_block_tables, int cmp_table_stride,
+                     const int32_t* cmp_slot_mapping, const void* new_k, int64_t nk_st, int64_t nk_sh,
+                     const void* new_v, int64_t nv_st, int64_t nv_sh, const int32_t* slot_mapping, int page_size, int B, int QH, int KH,
+                     int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks, int kernel_size, int stride,
+                     int block_size, int top_n, int num_init, int num_local, int ignore_index, int window,
+                     float sm_scale, void* scratch, int64_t scratch_bytes, void* stream);
 
 #ifdef __cplusplus
 }

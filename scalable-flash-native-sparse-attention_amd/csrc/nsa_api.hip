@@ -31,6 +31,7 @@ Knob g_knobs[] = {
     {"dq_min_blocks", {0}, {false}},    // workgroups per CU of the dense dq kernel
     {"dkdv_key_blocks", {0}, {false}},  // 32-key blocks per wave of the dense dk/dv kernel
     {"topk_seg_blocks", {0}, {false}},  // selection blocks per segment of the block selector
+    {"decode_waves", {0}, {false}},     // waves per workgroup of the one-launch decode kernel (0: from the batch; 4, 8)
     {"swa_dkdv_splits", {0}, {false}},  // query chunks per key tile of the window dk/dv kernel (0: from the sizes)
     {"topk_two_pass", {0}, {false}},    // 0: the one-launch selector even when a workspace is given
 };
@@ -53,6 +54,19 @@ int nsa_check_launch(const char* what) {
     return NSA_ERR_LAUNCH;
   }
   return NSA_OK;
+}
+
+int nsa_device_cus() {
+  static std::atomic<int> num_cus{0};
+  int n = num_cus.load(std::memory_order_relaxed);
+  if (n == 0) {
+    int dev = 0;
+    hipDeviceProp_t prop;
+    n = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
+         prop.multiProcessorCount > 0) ? prop.multiProcessorCount : 256;
+    num_cus.store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 static int check_heads(const char* who, int QH, int KH, int D, int VD) {
@@ -82,7 +96,7 @@ int nsa_abi_version(void) { return 1; }
 int nsa_set_tuning(const char* name, int value) {
   Knob* k = name ? find_knob(name) : nullptr;
   NSA_REQUIRE(k != nullptr, NSA_ERR_BAD_ARG, "set_tuning: unknown name '%s' (fwd_variant, dq_min_blocks, "
-              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, topk_two_pass)", name ? name : "(null)");
+              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, decode_waves, topk_two_pass)", name ? name : "(null)");
   k->value.store(value);
   k->is_set.store(true);
   return NSA_OK;
@@ -340,19 +354,6 @@ int nsa_cmp_attn_bwd_dq_final(const void* q, int64_t q_st, int64_t q_sh, const v
                          x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream);
 }
 
-static int device_cus() {
-  static std::atomic<int> num_cus{0};
-  int n = num_cus.load(std::memory_order_relaxed);
-  if (n == 0) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    n = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-         prop.multiProcessorCount > 0) ? prop.multiProcessorCount : 256;
-    num_cus.store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // Time of a workgroup of the dk/dv kernel: a fixed part (K / V fragments, epilogue) plus its 64-row tiles, and how many
 // workgroups run at once (one per CU; two where 64 channels leave the kernel under 256 registers).
 struct DkdvCost {
@@ -360,8 +361,8 @@ struct DkdvCost {
   int slots;
 };
 static DkdvCost dkdv_cost(int D, int VD) {
-  if (D <= 64) return {12.0, 1.9, 2 * device_cus()};
-  return {12.0, 2.55 * (D + VD) / 256.0, device_cus()};
+  if (D <= 64) return {12.0, 1.9, 2 * nsa_device_cus()};
+  return {12.0, 2.55 * (D + VD) / 256.0, nsa_device_cus()};
 }
 
 // Query tokens per work item of the compressed dk/dv kernel when the caller leaves the choice to the library.
@@ -1036,7 +1037,7 @@ static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const vo
   p.lse_out = lse; p.lse_st = lse_st; p.lse_sh = lse_sh;
   p.topk = topk; p.tk_sh = tk_sh; p.tk_st = tk_st;
   p.sp_m = sp_m; p.sp_l = sp_l; p.sp_o = sp_o;
-  p.sp_keep_p = (_Float16*)sp_keep_p; p.sp_keep_m = sp_keep_m; p.nsplit = nsplit;
+  p.sp_keep_p = sp_keep_p; p.sp_keep_m = sp_keep_m; p.nsplit = nsplit;
   p.ctx_lens = context_lens;
   p.cmp_slots = cmp_slot_mapping;
   p.table = block_tables;
@@ -1143,6 +1144,15 @@ int nsa_decode_fused_fits(int D, int VD, int fixed_y_maxlen, int fixed_num_slc_b
   return nsa_decode_fused_lds_bytes(p, D, VD) > 0 ? 1 : 0;
 }
 
+int64_t nsa_decode_fused_scratch_bytes(int B, int KH, int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks,
+                                       int table_stride, int page_size) {
+  if (B <= 0 || KH <= 0 || fixed_y_maxlen < 1 || fixed_num_slc_blocks < 1 || table_stride < 1 || page_size < 1) return 0;
+  NsaDecodeParams p{};
+  p.KH = KH;
+  p.y_cap = fixed_y_maxlen; p.nb_cap = fixed_num_slc_blocks; p.table_stride = table_stride; p.page_size = page_size;
+  return nsa_decode_fused_scratch(p, B, D, VD);
+}
+
 int nsa_decode_fused(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
                      const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
                      void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
@@ -1154,6 +1164,25 @@ int nsa_decode_fused(const void* q, int64_t q_st, int64_t q_sh, const void* k_ca
                      int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks, int kernel_size, int stride,
                      int block_size, int top_n, int num_init, int num_local, int ignore_index, int window,
                      float sm_scale, void* stream) {
+  return nsa_decode_fused_ws(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, w, w_st, w_sh, out, o_st, o_sh,
+                             cmp_o, slc_o, swa_o, co_st, co_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st,
+                             context_lens, block_tables, table_stride, cmp_block_tables, cmp_table_stride,
+                             cmp_slot_mapping, new_k, nk_st, nk_sh, new_v, nv_st, nv_sh, slot_mapping, page_size, B,
+                             QH, KH, D, VD, fixed_y_maxlen, fixed_num_slc_blocks, kernel_size, stride, block_size,
+                             top_n, num_init, num_local, ignore_index, window, sm_scale, nullptr, 0, stream);
+}
+
+int nsa_decode_fused_ws(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
+                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
+                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                     int64_t tk_st, const int32_t* context_lens, const int32_t* block_tables, int table_stride,
+                     const int32_t* cmp_block_tables, int cmp_table_stride,
+                     const int32_t* cmp_slot_mapping, const void* new_k, int64_t nk_st, int64_t nk_sh,
+                     const void* new_v, int64_t nv_st, int64_t nv_sh, const int32_t* slot_mapping, int page_size, int B, int QH, int KH,
+                     int D, int VD, int fixed_y_maxlen, int fixed_num_slc_blocks, int kernel_size, int stride,
+                     int block_size, int top_n, int num_init, int num_local, int ignore_index, int window,
+                     float sm_scale, void* scratch, int64_t scratch_bytes, void* stream) {
   int rc = check_heads("decode_fused", QH, KH, D, VD);
   if (rc) return rc;
   rc = check_nsa_sizes("decode_fused", kernel_size, stride, block_size);
@@ -1194,6 +1223,12 @@ int nsa_decode_fused(const void* q, int64_t q_st, int64_t q_sh, const void* k_ca
   p.kernel_size = kernel_size; p.stride = stride; p.block_size = block_size; p.window = window;
   p.top_n = top_n; p.num_init = num_init; p.num_local = num_local; p.ignore_index = ignore_index;
   p.y_cap = fixed_y_maxlen; p.nb_cap = fixed_num_slc_blocks;
+  const int64_t need = nsa_decode_fused_scratch(p, B, D, VD);
+  if (scratch != nullptr && need > 0) {
+    NSA_REQUIRE(scratch_bytes >= need, NSA_ERR_WORKSPACE, "decode_fused: scratch of %lld bytes, %lld needed",
+                (long long)scratch_bytes, (long long)need);
+    p.sp_keep_p = scratch;
+  }
   return nsa_decode_fused_launch(p, B, D, VD, (hipStream_t)stream);
 }
 

@@ -174,6 +174,7 @@ enum {
 void nsa_set_error(const char* fmt, ...);
 int nsa_tuning_knob(const char* name, int default_value);  // value given to nsa_set_tuning for this name, else the default
 int nsa_check_launch(const char* what);
+int nsa_device_cus();  // compute units of the current device
 
 #define NSA_REQUIRE(cond, code, ...)        \
   do {                                      \

@@ -29,10 +29,21 @@ constexpr int SEL_INTS = 192;  // LDS words of a selecting wave: 64 selected blo
 // K and V rows of a unit are fetched as whole rows (16 lanes x 16 bytes per row: every cache line is requested once
 // and used completely), held in registers while the previous unit is computed, and pass through one wave-private
 // LDS slot: first the K rows (read back as MFMA A fragments), then the V rows (read back transposed).
-// With KEEP the un-normalised probabilities exp2((s - m_unit) * c) of every unit are kept in LDS as fp16 together
-// with the m_unit they refer to, so that the importance pass needs no second pass over the keys.
-template <int D, int VD>
+// The un-normalised probabilities exp2((s - m_unit) * c) of every unit can be kept (in LDS, or spilled to scratch
+// memory, or both), together with the m_unit they refer to, so that the importance pass needs no second pass over the
+// keys: as fp16, or, with 192 channels, as fp32.
+// TWO_DEEP: two sets of K / V registers, the next unit is loaded while one is computed.  Otherwise one set, whose K and
+// V halves are loaded again as soon as their rows have gone to LDS: half the registers (192 channels do not fit two sets
+// into 256), the loads in flight for most of a unit instead of all of it.
+// STREAMS: a unit's m_unit is the running maximum of its stream, the units of the wave a fixed step apart; the wave
+// walks that many streams in turn.  With two of them (units dealt to four waves instead of eight) the kept values are
+// those of the eight-wave kernel.
+// KEEP: where kept probabilities go.
+constexpr int KEEP_LDS = 0, KEEP_MEM = 1, KEEP_BOTH = 2;
+template <int D, int VD, int KEEP = KEEP_LDS, int STREAMS = 1, bool TWO_DEEP = (D <= 128)>
 struct UnitFlash {
+  using keep_t = std::conditional_t<(D <= 128), _Float16, float>;
+  typedef keep_t keep4 __attribute__((ext_vector_type(4)));
   static constexpr int KC = D / 32;
   static constexpr int KJ = (UK * (D / 8)) / 64;
   static constexpr int VJ = (UK * (VD / 8)) / 64;
@@ -49,9 +60,12 @@ struct UnitFlash {
   float sc;
   int l16, kq, lane;
   bf16_t* Ss;          // wave-private staging slot
-  _Float16* keep_p;    // [16][keep_ld] (keep_ld > 0), [units][16][UK] (keep_ld == 0: whole units contiguous), or null
+  keep_t* keep_p;      // LDS [16][keep_ld], the units that start below key keep_lds_end
+  keep_t* spill_p;     // memory [units][16][UK] (whole units contiguous), the other units
   float* keep_m;       // [units][16]
-  int keep_ld;
+  int keep_ld, keep_lds_end;
+  int keep_end;        // probabilities of the units that start below this key are kept
+  float m_even, m_odd;  // STREAMS 2: running maxima of the stream of the next unit, of the other one
 
   NSA_DEVICE void init(const bf16_t* qrow, float scale_log2, int lane_, bf16_t* slot) {
     lane = lane_;
@@ -59,9 +73,11 @@ struct UnitFlash {
     kq = lane >> 4;
     sc = scale_log2;
     Ss = slot;
-    keep_p = nullptr;
+    keep_p = spill_p = nullptr;
     keep_m = nullptr;
-    keep_ld = 0;
+    keep_ld = keep_lds_end = 0;
+    keep_end = 0;
+    m_even = m_odd = NSA_NEG_INF;
 #pragma unroll
     for (int kc = 0; kc < KC; kc++) qf[kc] = ld_global_b128(qrow + kq * 8 + kc * 32);
 #pragma unroll
@@ -75,16 +91,23 @@ struct UnitFlash {
     for (int dt = 0; dt < VD / 16; dt++) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     m_run = NSA_NEG_INF;
     l_run = 0.f;
-    keep_p = nullptr;
+    keep_end = 0;
   }
   // loads of the unit starting at key0 (wave-uniform); keys outside [klo, khi] are replaced by a clamped key
   // (masked later).  A unit spans at most two pages: the page of its first usable key is looked up once.
+  template <bool K = true, bool V = true>
   NSA_DEVICE void issue(int key0, int klo, int khi, const int* tab_s, int page, const bf16_t* kbase, int64_t k_sr,
                         const bf16_t* vbase, int64_t v_sr, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ]) {
     const int ks = __builtin_amdgcn_readfirstlane(max(klo, min(key0, khi)));
     const int pi = ks / page;
     const int rem0 = ks - pi * page;
-    if constexpr (64 % (D / 8) == 0 && 64 % (VD / 8) == 0) {
+    // (a row of 192 channels is 24 sixteen-byte pieces: three groups of 64 lanes are eight whole rows, so three
+    // per-lane offsets that never change)
+    constexpr int KP = D / 8, VP = VD / 8;
+    constexpr int KG = 64 % KP == 0 ? 1 : KP / 8, VG = 64 % VP == 0 ? 1 : VP / 8;  // groups of 64 lanes per period
+    constexpr int KR = 64 * KG / KP, VR = 64 * VG / VP;                            // rows of a period
+    static_assert(64 * KG % KP == 0 && 64 * VG % VP == 0 && KJ % KG == 0 && VJ % VG == 0, "");
+    {
       // A unit that lies inside [klo, khi] and inside one page (nearly all of them) is UK consecutive pool rows:
       // one wave-uniform row address per group of 64 lanes' rows, and a per-lane byte offset that never changes.
       const int k0 = __builtin_amdgcn_readfirstlane(key0);
@@ -93,40 +116,48 @@ struct UnitFlash {
         const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(tab_s[pi]) * page + rem0;
         const char* kp = reinterpret_cast<const char*>(kbase + row0 * k_sr);
         const char* vp = reinterpret_cast<const char*>(vbase + row0 * v_sr);
-        const uint32_t koff = (uint32_t)(lane / (D / 8)) * (uint32_t)k_sr * 2u + (uint32_t)(lane % (D / 8)) * 16u;
-        const uint32_t voff = (uint32_t)(lane / (VD / 8)) * (uint32_t)v_sr * 2u + (uint32_t)(lane % (VD / 8)) * 16u;
+        uint32_t koff[KG], voff[VG];
 #pragma unroll
-        for (int j = 0; j < KJ; j++)
-          kf[j] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)(j * (64 / (D / 8))) * k_sr * 2 + koff);
+        for (int g = 0; g < KG; g++)
+          koff[g] = (uint32_t)((lane + g * 64) / KP) * (uint32_t)k_sr * 2u + (uint32_t)((lane + g * 64) % KP) * 16u;
 #pragma unroll
-        for (int j = 0; j < VJ; j++)
-          vr[j] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)(j * (64 / (VD / 8))) * v_sr * 2 + voff);
+        for (int g = 0; g < VG; g++)
+          voff[g] = (uint32_t)((lane + g * 64) / VP) * (uint32_t)v_sr * 2u + (uint32_t)((lane + g * 64) % VP) * 16u;
+#pragma unroll
+        for (int j = 0; j < (K ? KJ : 0); j++)
+          kf[j] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)(j / KG * KR) * k_sr * 2 + koff[j % KG]);
+#pragma unroll
+        for (int j = 0; j < (V ? VJ : 0); j++)
+          vr[j] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)(j / VG * VR) * v_sr * 2 + voff[j % VG]);
         return;
       }
     }
     const int64_t base0 = (int64_t)tab_s[pi] * page;
     const int64_t base1 = (rem0 + UK > page && (int64_t)(pi + 1) * page <= khi) ? (int64_t)tab_s[pi + 1] * page - page : base0;
 #pragma unroll
-    for (int j = 0; j < KJ; j++) {
+    for (int j = 0; j < (K ? KJ : 0); j++) {
       int pc = lane + j * 64;
       int r = rem0 + max(klo, min(key0 + pc / (D / 8), khi)) - ks;
       int64_t row = (r >= page ? base1 : base0) + r;
       kf[j] = ld_global_b128(kbase + row * k_sr + (pc % (D / 8)) * 8);
     }
 #pragma unroll
-    for (int j = 0; j < VJ; j++) {
+    for (int j = 0; j < (V ? VJ : 0); j++) {
       int pc = lane + j * 64;
       int r = rem0 + max(klo, min(key0 + pc / (VD / 8), khi)) - ks;
       int64_t row = (r >= page ? base1 : base0) + r;
       vr[j] = ld_global_b128(vbase + row * v_sr + (pc % (VD / 8)) * 8);
     }
   }
-  NSA_DEVICE void compute(int key0, int klo, int khi, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ]) {
+  // next_k / next_v run as soon as the K / V registers have gone to LDS (they may load the next unit into them)
+  template <class NextK, class NextV>
+  NSA_DEVICE void compute(int key0, int klo, int khi, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ], NextK next_k, NextV next_v) {
 #pragma unroll
     for (int j = 0; j < KJ; j++) {
       int pc = lane + j * 64;
       *reinterpret_cast<bf16x8*>(&Ss[(pc / (D / 8)) * KLD + (pc % (D / 8)) * 8]) = kf[j];
     }
+    next_k();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -147,6 +178,7 @@ struct UnitFlash {
       int pc = lane + j * 64;
       *reinterpret_cast<bf16x8*>(&Ss[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
     }
+    next_v();
     if (key0 < klo || key0 + UK - 1 > khi) {  // wave-uniform: only boundary units are masked
 #pragma unroll
       for (int jt = 0; jt < 2; jt++)
@@ -166,6 +198,29 @@ struct UnitFlash {
     const float msc = m_safe * sc;
     m_run = m_new;
     float psum = 0.f;
+    auto keep = [&](const f32x4 (&x)[2], float m_unit) {
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++) {
+        const keep4 hv = {(keep_t)x[jt][0], (keep_t)x[jt][1], (keep_t)x[jt][2], (keep_t)x[jt][3]};
+        if (KEEP == KEEP_LDS || (KEEP == KEEP_BOTH && key0 < keep_lds_end))
+          *reinterpret_cast<keep4*>(&keep_p[l16 * keep_ld + key0 + jt * 16 + kq * 4]) = hv;
+        else
+          *reinterpret_cast<keep4*>(&spill_p[(key0 / UK) * (16 * UK) + l16 * UK + jt * 16 + kq * 4]) = hv;
+      }
+      if (kq == 0) keep_m[(key0 / UK) * 16 + l16] = m_unit;
+    };
+    if (STREAMS == 2 && key0 < keep_end) {  // relative to the stream's maximum
+      const float ms = fmaxf(m_even, tmax);
+      m_even = m_odd;
+      m_odd = ms;
+      const float m_unit = ms == NSA_NEG_INF ? 0.f : ms, ksc = m_unit * sc;
+      f32x4 x[2];
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[jt][i] = fast_exp2(__builtin_fmaf(sacc[jt][i], sc, -ksc));
+      keep(x, m_unit);
+    }
 #pragma unroll
     for (int jt = 0; jt < 2; jt++)
 #pragma unroll
@@ -174,17 +229,7 @@ struct UnitFlash {
         sacc[jt][i] = pv;
         psum += pv;
       }
-    if (keep_p != nullptr) {
-      typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-      for (int jt = 0; jt < 2; jt++) {
-        h4 hv = {(_Float16)sacc[jt][0], (_Float16)sacc[jt][1], (_Float16)sacc[jt][2], (_Float16)sacc[jt][3]};
-        const int at = keep_ld > 0 ? l16 * keep_ld + key0 + jt * 16 + kq * 4
-                                   : (key0 / UK) * (16 * UK) + l16 * UK + jt * 16 + kq * 4;
-        *reinterpret_cast<h4*>(&keep_p[at]) = hv;
-      }
-      if (kq == 0) keep_m[(key0 / UK) * 16 + l16] = m_safe;
-    }
+    if (STREAMS == 1 && key0 < keep_end) keep(sacc, m_safe);
     if (__builtin_amdgcn_ballot_w64(m_new != m_old) != 0) {
       const float alpha = fast_exp2((m_old - m_safe) * sc);
       l_run *= alpha;
@@ -224,6 +269,24 @@ struct UnitFlash {
   template <bool USE_PRE = false, class KeyFn>
   NSA_DEVICE void run(int first, int step, int nu, int klo, int khi, KeyFn key0_of, const int* tab_s, int page,
                       const bf16_t* kbase, int64_t k_sr, const bf16_t* vbase, int64_t v_sr) {
+    if constexpr (!TWO_DEEP) {
+      static_assert(!USE_PRE, "");
+      bf16x8 kf[KJ], vr[VJ];
+      if (first >= nu) return;
+      int key = key0_of(first);
+      issue(key, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr);
+      for (int u = first; u < nu; u += step) {
+        const bool more = u + step < nu;
+        const int nxt = more ? key0_of(u + step) : 0;
+        compute(
+            key, klo, khi, kf, vr,
+            [&]() { if (more) issue<true, false>(nxt, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr); },
+            [&]() { if (more) issue<false, true>(nxt, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr); });
+        key = nxt;
+      }
+      return;
+    } else {
+    auto none = []() {};
     bf16x8 kfA[KJ], kfB[KJ], vrA[VJ], vrB[VJ];
     int keyA = 0, keyB = 0;
     if (USE_PRE) {
@@ -239,14 +302,15 @@ struct UnitFlash {
     for (int u = first; u < nu; u += 2 * step) {
       const bool hasB = u + step < nu;
       if (hasB) { keyB = key0_of(u + step); issue(keyB, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kfB, vrB); }
-      compute(keyA, klo, khi, kfA, vrA);
+      compute(keyA, klo, khi, kfA, vrA, none, none);
       if (hasB) {
         if (u + 2 * step < nu) {
           keyA = key0_of(u + 2 * step);
           issue(keyA, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kfA, vrA);
         }
-        compute(keyB, klo, khi, kfB, vrB);
+        compute(keyB, klo, khi, kfB, vrB, none, none);
       }
+    }
     }
   }
   // wave partial -> LDS slot: m (raw units), l, o[16 heads][VD]
@@ -438,7 +502,8 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_cmp_topk_kernel(NsaDeco
   const int keep_ld = n_units_cap * UK + 8;  // +8 halves: the 16 head rows start in different banks
   float* after_tab = reinterpret_cast<float*>(tab_s + ((ntab + 3) & ~3));
   float* keep_m = after_tab;                                               // KEEP
-  _Float16* keep_p = reinterpret_cast<_Float16*>(keep_m + n_units_cap * 16);  // KEEP
+  using keep_t = typename UF::keep_t;
+  keep_t* keep_p = reinterpret_cast<keep_t*>(keep_m + n_units_cap * 16);  // KEEP
   float* pg = KEEP ? reinterpret_cast<float*>(dyn_raw) : after_tab;
 
   const int tid = threadIdx.x;
@@ -468,6 +533,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_cmp_topk_kernel(NsaDeco
     uf.keep_p = keep_p;
     uf.keep_m = keep_m;
     uf.keep_ld = keep_ld;
+    uf.keep_end = uf.keep_lds_end = y;
   }
   const int nu = (y + UK - 1) / UK;
 
@@ -551,7 +617,7 @@ constexpr int SPLIT_WAVES = 4;
 // grid (B, KH, nsplit): compressed attention over the units u = s*4 + wave (mod 4*nsplit)
 template <int D, int VD>
 __global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(NsaDecodeParams p) {
-  using UF = UnitFlash<D, VD>;
+  using UF = UnitFlash<D, VD, KEEP_MEM>;
   constexpr int NW = SPLIT_WAVES;
   constexpr int SLOT = UF::SLOT;
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn_raw[];
@@ -609,9 +675,10 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(Ns
   uf.init(p.q + (int64_t)b * p.q_st + (int64_t)head * p.q_sh, p.scale_log2, lane, Vs_all + wave * SLOT);
   if (p.sp_keep_p != nullptr) {  // spill the un-normalised probabilities of every unit for the final kernel
     const int nuc = (p.y_cap + UK - 1) / UK;
-    uf.keep_ld = 0;  // unit-major: a wave writes the 1 KB of a unit as whole cache lines
-    uf.keep_p = p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * nuc * UK;
+    // unit-major: a wave writes the 1 KB of a unit as whole cache lines
+    uf.spill_p = (typename UF::keep_t*)p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * nuc * UK;
     uf.keep_m = p.sp_keep_m + ((int64_t)b * p.KH + kh) * nuc * 16;
+    uf.keep_end = y;
   }
   const int nu = (y + UK - 1) / UK;
   uf.run(sp * NW + wave, NW * nsplit, nu, 0, y - 1, [&](int u) { return u * UK; }, tab_s, page, kbase, p.k_sr,
@@ -796,7 +863,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     // Prologue of the two-launch split path: merge the statistics of the parts of the compressed branch, turn the
     // spilled fp16 probabilities into head-summed probabilities (over the not-yet-used staging slots) and fold them
     // into block scores.  The same arithmetic as the one-launch kernel.
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef typename UF::keep4 h4;
     const int y = L >= p.kernel_size ? min((L - p.kernel_size) / p.stride + 1, p.y_cap) : 0;
     const int nuc = (p.y_cap + UK - 1) / UK, keep_ld = nuc * UK;
     const int nsplit = p.nsplit;
@@ -804,7 +871,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     imp = reinterpret_cast<float*>(tab_s + ((p.table_stride + 3) & ~3));
     float* fac = imp + ((p.nb_cap + 3) & ~3);
     const int64_t sp_base = ((int64_t)b * p.KH + kh) * nsplit * 16;
-    const _Float16* keep_p = p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * keep_ld;
+    const typename UF::keep_t* keep_p = (const typename UF::keep_t*)p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * keep_ld;
     const float* keep_m = p.sp_keep_m + ((int64_t)b * p.KH + kh) * nuc * 16;
     // all (m, l) of the parts in one round trip, then one thread per head
     float* st_m = fac;
@@ -1038,10 +1105,10 @@ __global__ __launch_bounds__(256) void decode_split_final_kernel(NsaDecodeParams
 // attention -> gated combine.  Nothing but the final output (and, on request, topk / the branch outputs) goes
 // back to global memory; the compressed-branch output stays in registers, the window partials in the LDS region
 // that held the fp16 probabilities.
-template <int D, int VD>
-__global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeParams p) {
-  using UF = UnitFlash<D, VD>;
-  constexpr int NW = DEC_WAVES;
+template <int D, int VD, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void decode_fused_kernel(NsaDecodeParams p, int keep_units) {
+  using UF = UnitFlash<D, VD, (D > 128) ? KEEP_MEM : (NW == DEC_WAVES ? KEEP_LDS : KEEP_BOTH),
+                       (D > 128) ? 1 : DEC_WAVES / NW, NW == DEC_WAVES>;
   constexpr int SLOT = UF::SLOT;
   constexpr int NTHREADS = NW * 64;
   constexpr int NV4 = 16 * VD / 4;                             // groups of four merged output values
@@ -1061,10 +1128,11 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeP
   int* ctab_s = blk_s + SEL_INTS;
   const int ntab_c = (p.y_cap + p.page_size - 1) / p.page_size;
   int* tab_s = ctab_s + ((ntab_c + 3) & ~3);
+  const int keep_ld = keep_units * UK + 8;
   const int n_units_cap = (p.y_cap + UK - 1) / UK;
-  const int keep_ld = n_units_cap * UK + 8;
+  using keep_t = typename UF::keep_t;
   float* keep_m = reinterpret_cast<float*>(tab_s + ((p.table_stride + 3) & ~3));
-  _Float16* keep_p = reinterpret_cast<_Float16*>(keep_m + n_units_cap * 16);
+  keep_t* keep_p = reinterpret_cast<keep_t*>(keep_m + n_units_cap * 16);
   float* swa_o = reinterpret_cast<float*>(keep_p);  // [NW-1][16][VD], after the probabilities are consumed
   float* pg = reinterpret_cast<float*>(dyn_raw);    // over the staging slots, between the phases
 
@@ -1151,6 +1219,11 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeP
   uf.keep_p = keep_p;
   uf.keep_m = keep_m;
   uf.keep_ld = keep_ld;
+  const int y_keep = min(y, keep_units * UK);  // keys whose probabilities stay in LDS; the others go to scratch memory
+  const keep_t* spill = (const keep_t*)p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * n_units_cap * UK;
+  uf.spill_p = const_cast<keep_t*>(spill);
+  uf.keep_lds_end = y_keep;
+  uf.keep_end = y;
   const int nu = (y + UK - 1) / UK;
 
   // ---- compressed attention, units dealt round-robin to the waves ----
@@ -1162,7 +1235,8 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeP
   const int swa_k0 = (swa_klo / UK) * UK;
   const int swa_nu = t >= 0 ? (t - swa_k0) / UK + 1 : 0;
   auto swa_key = [&](int u) { return swa_k0 + u * UK; };
-  constexpr bool PREFETCH_SWA = true;
+  // (with two workgroups per CU the other one hides that latency, and the prefetched unit's registers would spill)
+  constexpr bool PREFETCH_SWA = NW == DEC_WAVES;
   // When the newest token's row was stored by waves 0 / 1 after the first barrier (nothing pooled at this step),
   // only the next barrier orders that store before other waves' reads of the row, and the window's last unit holds
   // it: the prefetch then waits for the barrier (workgroup-uniform condition).
@@ -1196,14 +1270,21 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeP
   // four consecutive keys (one unit, so one set of 16 per-head factors) ----
   for (int key = tid * 4; key < y; key += NTHREADS * 4) {
     const float* um = keep_m + (key / UK) * 16;
+    typename UF::keep4 kp[16];
+    if (NW == DEC_WAVES || (D <= 128 && key < y_keep)) {
+#pragma unroll
+      for (int h = 0; h < 16; h++) kp[h] = *reinterpret_cast<const typename UF::keep4*>(&keep_p[h * keep_ld + key]);
+    } else {
+      const keep_t* up = spill + (int64_t)(key / UK) * (16 * UK) + (key % UK);
+#pragma unroll
+      for (int h = 0; h < 16; h++) kp[h] = *reinterpret_cast<const typename UF::keep4*>(up + h * UK);
+    }
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int h = 0; h < 16; h++) {
       const float fac = h < G ? fast_exp2(__builtin_fmaf(um[h], p.scale_log2, -lse_s[h])) : 0.f;
-      typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-      const h4 kp = *reinterpret_cast<const h4*>(&keep_p[h * keep_ld + key]);
-      acc[0] += (float)kp[0] * fac; acc[1] += (float)kp[1] * fac;
-      acc[2] += (float)kp[2] * fac; acc[3] += (float)kp[3] * fac;
+      acc[0] += (float)kp[h][0] * fac; acc[1] += (float)kp[h][1] * fac;
+      acc[2] += (float)kp[h][2] * fac; acc[3] += (float)kp[h][3] * fac;
     }
     *reinterpret_cast<f32x4*>(&pg[key]) = acc;
   }
@@ -1263,9 +1344,9 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_fused_kernel(NsaDecodeP
 
 }  // namespace
 
-template <class K>
-static int launch_dyn(K kern, dim3 grid, size_t dyn, const NsaDecodeParams& p, hipStream_t stream, const char* name,
-                      size_t static_lds = 0) {
+template <class K, class... Args>
+static int launch_dyn(K kern, dim3 grid, int waves, size_t dyn, hipStream_t stream, const char* name,
+                      size_t static_lds, Args... args) {
   if (dyn + static_lds > 160 * 1024) {
     nsa_set_error("%s: %zu bytes of LDS needed (fixed_y_maxlen / fixed_num_slc_blocks too large)", name,
                   dyn + static_lds);
@@ -1276,31 +1357,37 @@ static int launch_dyn(K kern, dim3 grid, size_t dyn, const NsaDecodeParams& p, h
     nsa_set_error("%s: hipFuncSetAttribute(%zu) failed: %s", name, dyn, hipGetErrorString(e));
     return NSA_ERR_LAUNCH;
   }
-  kern<<<grid, DEC_WAVES * 64, dyn, stream>>>(p);
+  kern<<<grid, waves * 64, dyn, stream>>>(args...);
   return nsa_check_launch(name);
 }
 
 template <int D, int VD>
-static size_t slot_bytes() { return (size_t)DEC_WAVES * UnitFlash<D, VD>::SLOT * 2; }
+static size_t slot_bytes(int waves = DEC_WAVES) { return (size_t)waves * UnitFlash<D, VD>::SLOT * 2; }
 
 // LDS of the fused compressed-attention + selection kernel; `keep` adds the fp16 probabilities of every compressed
 // key and the per-unit maxima (no second pass over the keys) and drops the separate pg array
-static size_t cmp_topk_lds(size_t slots, const NsaDecodeParams& p, bool keep) {
+static size_t cmp_topk_lds(size_t slots, size_t keep_size, const NsaDecodeParams& p, bool keep) {
   const size_t ntab = (size_t)(p.y_cap + p.page_size - 1) / p.page_size;
   const size_t units = (size_t)(p.y_cap + UK - 1) / UK;
   size_t n = slots + (size_t)(2 * DEC_WAVES * 16 + 16 + p.nb_cap + ((ntab + 3) & ~(size_t)3)) * sizeof(float);
-  if (keep) n += units * 16 * sizeof(float) + 16 * (units * UK + 8) * sizeof(_Float16);
+  if (keep) n += units * 16 * sizeof(float) + 16 * (units * UK + 8) * keep_size;
   else n += (size_t)p.y_cap * sizeof(float);
   return n;
 }
 
 template <int D, int VD>
 static int launch_cmp_topk(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
-  const size_t keep_bytes = cmp_topk_lds(slot_bytes<D, VD>(), p, true);
+  const size_t keep_bytes = cmp_topk_lds(slot_bytes<D, VD>(), sizeof(typename UnitFlash<D, VD>::keep_t), p, true);
   if (keep_bytes <= 160 * 1024)
-    return launch_dyn(decode_cmp_topk_kernel<D, VD, true>, grid, keep_bytes, p, stream, "decode_cmp_topk_kernel");
-  return launch_dyn(decode_cmp_topk_kernel<D, VD, false>, grid, cmp_topk_lds(slot_bytes<D, VD>(), p, false), p, stream,
-                    "decode_cmp_topk_kernel");
+    return launch_dyn(decode_cmp_topk_kernel<D, VD, true>, grid, DEC_WAVES, keep_bytes, stream, "decode_cmp_topk_kernel",
+                      0, p);
+  return launch_dyn(decode_cmp_topk_kernel<D, VD, false>, grid, DEC_WAVES, cmp_topk_lds(slot_bytes<D, VD>(), 0, p, false),
+                    stream, "decode_cmp_topk_kernel", 0, p);
+}
+
+static int bad_decode_dims(int D, int VD) {
+  nsa_set_error("decode: unsupported head dims D=%d VD=%d (built: 128/128, 64/64, 192/128)", D, VD);
+  return NSA_ERR_UNSUPPORTED;
 }
 
 int nsa_decode_cmp_topk_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream) {
@@ -1308,8 +1395,14 @@ int nsa_decode_cmp_topk_launch(const NsaDecodeParams& p, int B, int D, int VD, h
   dim3 grid(B, p.KH);
   if (D == 128 && VD == 128) return launch_cmp_topk<128, 128>(p, grid, stream);
   if (D == 64 && VD == 64) return launch_cmp_topk<64, 64>(p, grid, stream);
-  nsa_set_error("decode: unsupported head dims D=%d VD=%d (built: 128/128, 64/64)", D, VD);
-  return NSA_ERR_UNSUPPORTED;
+  if (D == 192 && VD == 128) return launch_cmp_topk<192, 128>(p, grid, stream);
+  return bad_decode_dims(D, VD);
+}
+
+template <int D, int VD>
+static int launch_slc_swa(const NsaDecodeParams& p, dim3 grid, size_t dyn, hipStream_t stream) {
+  return launch_dyn(decode_slc_swa_kernel<D, VD>, grid, DEC_WAVES, dyn, stream, "decode_slc_swa_kernel",
+                    SLC_SWA_STATIC_LDS, p);
 }
 
 int nsa_decode_slc_swa_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream) {
@@ -1317,39 +1410,36 @@ int nsa_decode_slc_swa_launch(const NsaDecodeParams& p, int B, int D, int VD, hi
   dim3 grid(B, p.KH);
   size_t extra = (size_t)(2 * DEC_WAVES * 16 + SEL_INTS + ((p.table_stride + 3) & ~3)) * sizeof(float);
   if (p.pg != nullptr) extra += (size_t)((p.nb_cap + 3) & ~3) * sizeof(float);  // block scores
-  if (D == 128 && VD == 128)
-    return launch_dyn(decode_slc_swa_kernel<128, 128>, grid, slot_bytes<128, 128>() + extra, p, stream,
-                      "decode_slc_swa_kernel", SLC_SWA_STATIC_LDS);
-  if (D == 64 && VD == 64)
-    return launch_dyn(decode_slc_swa_kernel<64, 64>, grid, slot_bytes<64, 64>() + extra, p, stream,
-                      "decode_slc_swa_kernel", SLC_SWA_STATIC_LDS);
-  nsa_set_error("decode: unsupported head dims D=%d VD=%d (built: 128/128, 64/64)", D, VD);
-  return NSA_ERR_UNSUPPORTED;
+  if (D == 128 && VD == 128) return launch_slc_swa<128, 128>(p, grid, slot_bytes<128, 128>() + extra, stream);
+  if (D == 64 && VD == 64) return launch_slc_swa<64, 64>(p, grid, slot_bytes<64, 64>() + extra, stream);
+  if (D == 192 && VD == 128) return launch_slc_swa<192, 128>(p, grid, slot_bytes<192, 128>() + extra, stream);
+  return bad_decode_dims(D, VD);
+}
+
+template <int D, int VD>
+static int launch_cmp_partial(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
+  const int ntab = (p.y_cap + p.page_size - 1) / p.page_size;
+  return launch_dyn(decode_cmp_partial_kernel<D, VD>, grid, SPLIT_WAVES,
+                    slot_bytes<D, VD>(SPLIT_WAVES) + (size_t)(2 * SPLIT_WAVES * 16 + ntab) * 4, stream,
+                    "decode_cmp_partial_kernel", 0, p);
+}
+
+template <int D, int VD>
+static int launch_cmp_split(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
+  const int rc = launch_cmp_partial<D, VD>(p, grid, stream);
+  if (rc) return rc;
+  const size_t ntab = (size_t)(p.y_cap + p.page_size - 1) / p.page_size;
+  decode_importance_kernel<D, VD><<<grid, SPLIT_WAVES * 64, ntab * 4, stream>>>(p);
+  return nsa_check_launch("decode_importance_kernel");
 }
 
 int nsa_decode_cmp_split_launch(const NsaDecodeParams& p, int B, int nsplit, int D, int VD, hipStream_t stream) {
   if (B <= 0) return NSA_OK;
   dim3 grid(B, p.KH, nsplit);
-  int ntab = (p.y_cap + p.page_size - 1) / p.page_size;
-  size_t dyn1 = (size_t)SPLIT_WAVES * (D == 128 ? UnitFlash<128, 128>::SLOT : UnitFlash<64, 64>::SLOT) * 2 +
-                (size_t)(2 * SPLIT_WAVES * 16 + ntab) * 4;
-  size_t dyn2 = (size_t)ntab * 4;
-  if (!((D == 128 && VD == 128) || (D == 64 && VD == 64))) {
-    nsa_set_error("decode: unsupported head dims D=%d VD=%d (built: 128/128, 64/64)", D, VD);
-    return NSA_ERR_UNSUPPORTED;
-  }
-  if (D == 128) {
-    decode_cmp_partial_kernel<128, 128><<<grid, SPLIT_WAVES * 64, dyn1, stream>>>(p);
-    int rc = nsa_check_launch("decode_cmp_partial_kernel");
-    if (rc) return rc;
-    decode_importance_kernel<128, 128><<<grid, SPLIT_WAVES * 64, dyn2, stream>>>(p);
-  } else {
-    decode_cmp_partial_kernel<64, 64><<<grid, SPLIT_WAVES * 64, dyn1, stream>>>(p);
-    int rc = nsa_check_launch("decode_cmp_partial_kernel");
-    if (rc) return rc;
-    decode_importance_kernel<64, 64><<<grid, SPLIT_WAVES * 64, dyn2, stream>>>(p);
-  }
-  return nsa_check_launch("decode_importance_kernel");
+  if (D == 128 && VD == 128) return launch_cmp_split<128, 128>(p, grid, stream);
+  if (D == 64 && VD == 64) return launch_cmp_split<64, 64>(p, grid, stream);
+  if (D == 192 && VD == 128) return launch_cmp_split<192, 128>(p, grid, stream);
+  return bad_decode_dims(D, VD);
 }
 
 // ---- two-launch split path: partial kernel with the probability spill, then the final kernel ----
@@ -1366,10 +1456,22 @@ static size_t split_final_lds(const NsaDecodeParams& p) {
 int nsa_decode_split_lds_bytes(const NsaDecodeParams& p, int D, int VD) {
   if (D == 128 && VD == 128) return (int)split_final_lds<128, 128>(p);
   if (D == 64 && VD == 64) return (int)split_final_lds<64, 64>(p);
+  if (D == 192 && VD == 128) return (int)split_final_lds<192, 128>(p);
   return 0;
 }
 
 int nsa_decode_split_static_lds_bytes() { return (int)SLC_SWA_STATIC_LDS; }
+
+template <int D, int VD>
+static int launch_split(const NsaDecodeParams& p, int B, size_t lds2, hipStream_t stream) {
+  const int S = p.slc_nsplit > 1 ? p.slc_nsplit : 1;
+  int rc = launch_cmp_partial<D, VD>(p, dim3(B, p.KH, p.nsplit), stream);
+  if (rc) return rc;
+  rc = launch_slc_swa<D, VD>(p, dim3(B, p.KH, S), lds2, stream);
+  if (rc || S == 1) return rc;
+  decode_split_final_kernel<VD><<<dim3(B, p.KH), 256, 0, stream>>>(p);
+  return nsa_check_launch("decode_split_final_kernel");
+}
 
 int nsa_decode_split_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream) {
   if (B <= 0) return NSA_OK;
@@ -1379,63 +1481,104 @@ int nsa_decode_split_launch(const NsaDecodeParams& p, int B, int D, int VD, hipS
                   "not fit the final kernel's LDS", D, VD, p.y_cap, p.nb_cap, p.table_stride);
     return NSA_ERR_UNSUPPORTED;
   }
-  const int S = p.slc_nsplit > 1 ? p.slc_nsplit : 1;
-  dim3 grid1(B, p.KH, p.nsplit), grid2(B, p.KH, S);
-  const int ntab = (p.y_cap + p.page_size - 1) / p.page_size;
-  const size_t dyn1 = (size_t)SPLIT_WAVES * (D == 128 ? UnitFlash<128, 128>::SLOT : UnitFlash<64, 64>::SLOT) * 2 +
-                      (size_t)(2 * SPLIT_WAVES * 16 + ntab) * 4;
-  if (D == 128) {
-    decode_cmp_partial_kernel<128, 128><<<grid1, SPLIT_WAVES * 64, dyn1, stream>>>(p);
-    int rc = nsa_check_launch("decode_cmp_partial_kernel");
-    if (rc) return rc;
-    rc = launch_dyn(decode_slc_swa_kernel<128, 128>, grid2, (size_t)lds2, p, stream, "decode_slc_swa_kernel",
-                    SLC_SWA_STATIC_LDS);
-    if (rc || S == 1) return rc;
-    decode_split_final_kernel<128><<<dim3(B, p.KH), 256, 0, stream>>>(p);
-    return nsa_check_launch("decode_split_final_kernel");
-  }
-  decode_cmp_partial_kernel<64, 64><<<grid1, SPLIT_WAVES * 64, dyn1, stream>>>(p);
-  int rc = nsa_check_launch("decode_cmp_partial_kernel");
-  if (rc) return rc;
-  rc = launch_dyn(decode_slc_swa_kernel<64, 64>, grid2, (size_t)lds2, p, stream, "decode_slc_swa_kernel",
-                  SLC_SWA_STATIC_LDS);
-  if (rc || S == 1) return rc;
-  decode_split_final_kernel<64><<<dim3(B, p.KH), 256, 0, stream>>>(p);
-  return nsa_check_launch("decode_split_final_kernel");
+  if (D == 128) return launch_split<128, 128>(p, B, (size_t)lds2, stream);
+  if (D == 64) return launch_split<64, 64>(p, B, (size_t)lds2, stream);
+  return launch_split<192, 128>(p, B, (size_t)lds2, stream);
 }
 
-// LDS of the one-launch decode kernel; 0 when it does not fit (the caller then takes the two-launch path)
+// LDS of the one-launch decode kernel with `waves` waves that keeps the probabilities of keep_units units
 template <int D, int VD>
-static size_t fused_lds(const NsaDecodeParams& p) {
+static size_t fused_lds(const NsaDecodeParams& p, int waves, size_t keep_units) {
   const size_t ntab_c = (size_t)(p.y_cap + p.page_size - 1) / p.page_size;
   const size_t units = (size_t)(p.y_cap + UK - 1) / UK;
-  size_t region = 16 * (units * UK + 8) * sizeof(_Float16);
-  const size_t swa_part = (size_t)(DEC_WAVES - 1) * 16 * UnitFlash<D, VD>::OLD * sizeof(float);
+  size_t region = 16 * (keep_units * UK + 8) * sizeof(typename UnitFlash<D, VD>::keep_t);
+  const size_t swa_part = (size_t)(waves - 1) * 16 * UnitFlash<D, VD>::OLD * sizeof(float);
   if (region < swa_part) region = swa_part;
   region = (region + 15) & ~(size_t)15;
-  size_t n = slot_bytes<D, VD>() +
-             (size_t)(4 * DEC_WAVES * 16 + 16 + (((size_t)p.nb_cap + 3) & ~(size_t)3) + SEL_INTS + ((ntab_c + 3) & ~(size_t)3) +
-                      (((size_t)p.table_stride + 3) & ~(size_t)3) + units * 16) * sizeof(float) + region;
-  if ((size_t)p.y_cap * sizeof(float) > slot_bytes<D, VD>()) return 0;
-  return n <= 160 * 1024 ? n : 0;
+  return slot_bytes<D, VD>(waves) +
+         (size_t)(4 * waves * 16 + 16 + (((size_t)p.nb_cap + 3) & ~(size_t)3) + SEL_INTS + ((ntab_c + 3) & ~(size_t)3) +
+                  (((size_t)p.table_stride + 3) & ~(size_t)3) + units * 16) * sizeof(float) + region;
+}
+
+// Shape of a one-launch decode: waves per workgroup and units whose probabilities stay in LDS (those of the others are
+// spilled to scratch memory, if the caller gives it); lds 0: it does not fit (the caller then takes a path with more
+// launches).
+//   * One workgroup of 8 waves per CU, all probabilities in LDS, while the (request, kv head) pairs fill the CUs less
+//     than twice: the waves share a request's units, so more of them shorten the longest request.
+//   * From there on two workgroups of 4 waves per CU, so that the serial sections of one (merges, block scores,
+//     selection) run beside the loads of the other; their 80 KB hold the probabilities of about 1000 keys (contexts of
+//     16K tokens).  64 q / 4 kv heads, d = 128, one / two workgroups: 512 x 4K 505 / 400 us (1.9 GB: 4.7 TB/s, what a
+//     copy reaches), 256 x 8K 287 / 231, 128 x 16K 173 / 146, 128 x 4K-32K 171 / 155; with one pair per CU two lose:
+//     64 x 4K-32K 78 / 83, 64 x 32K 118 / 126.  With one set of K / V registers per wave (two sets spill: 423 us).
+//   * 192 channels: four waves, fp32 probabilities in scratch memory.
+struct FusedShape {
+  int waves, keep_units;
+  size_t lds;
+  bool spills;
+};
+template <int D, int VD>
+static FusedShape fused_shape(const NsaDecodeParams& p, int pairs, bool may_spill) {
+  const int units = (p.y_cap + UK - 1) / UK;
+  auto pg_fits = [&](int waves) { return (size_t)p.y_cap * sizeof(float) <= slot_bytes<D, VD>(waves); };
+  if (D > 128) {
+    const size_t lds = fused_lds<D, VD>(p, 4, 0);
+    return pg_fits(4) && lds <= 160 * 1024 ? FusedShape{4, 0, lds, true} : FusedShape{0, 0, 0, false};
+  }
+  const size_t lds8 = fused_lds<D, VD>(p, DEC_WAVES, units);
+  const FusedShape one = pg_fits(DEC_WAVES) && lds8 <= 160 * 1024 ? FusedShape{DEC_WAVES, units, lds8, false}
+                                                                  : FusedShape{0, 0, 0, false};
+  const int forced = nsa_tuning_knob("decode_waves", 0);
+  const bool many = forced ? forced == 4 : pairs >= 2 * nsa_device_cus();
+  if (one.lds == 0 || !many || !pg_fits(4)) return one;
+  // (64 channels: three workgroups per CU, what their registers allow)
+  constexpr size_t budget = 160 * 1024 / (D <= 64 ? 3 : 2);
+  int keep = units;
+  while (keep > 0 && fused_lds<D, VD>(p, 4, keep) > budget) keep--;
+  const size_t lds = fused_lds<D, VD>(p, 4, keep);
+  return lds <= budget && (keep == units || may_spill) ? FusedShape{4, keep, lds, keep < units} : one;
+}
+
+static FusedShape fused_shape_of(const NsaDecodeParams& p, int pairs, bool may_spill, int D, int VD) {
+  if (D == 128 && VD == 128) return fused_shape<128, 128>(p, pairs, may_spill);
+  if (D == 64 && VD == 64) return fused_shape<64, 64>(p, pairs, may_spill);
+  if (D == 192 && VD == 128) return fused_shape<192, 128>(p, pairs, may_spill);
+  return {0, 0, 0, false};
 }
 
 int nsa_decode_fused_lds_bytes(const NsaDecodeParams& p, int D, int VD) {
-  if (D == 128 && VD == 128) return (int)fused_lds<128, 128>(p);
-  if (D == 64 && VD == 64) return (int)fused_lds<64, 64>(p);
-  return 0;
+  return (int)fused_shape_of(p, 1, true, D, VD).lds;
+}
+
+int64_t nsa_decode_fused_scratch(const NsaDecodeParams& p, int B, int D, int VD) {
+  if (!fused_shape_of(p, B * p.KH, true, D, VD).spills) return 0;
+  return (int64_t)B * p.KH * 16 * ((p.y_cap + UK - 1) / UK * UK) * (D <= 128 ? 2 : 4);
+}
+
+template <int D, int VD>
+static int launch_fused(const NsaDecodeParams& p, const FusedShape& s, dim3 grid, hipStream_t stream) {
+  if constexpr (D <= 128) {
+    if (s.waves == DEC_WAVES)
+      return launch_dyn(decode_fused_kernel<D, VD, DEC_WAVES>, grid, DEC_WAVES, s.lds, stream, "decode_fused_kernel", 0,
+                        p, s.keep_units);
+  }
+  return launch_dyn(decode_fused_kernel<D, VD, 4>, grid, 4, s.lds, stream, "decode_fused_kernel", 0, p, s.keep_units);
 }
 
 int nsa_decode_fused_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream) {
   if (B <= 0) return NSA_OK;
-  dim3 grid(B, p.KH);
-  const int dyn = nsa_decode_fused_lds_bytes(p, D, VD);
-  if (dyn == 0) {
+  const FusedShape s = fused_shape_of(p, B * p.KH, p.sp_keep_p != nullptr, D, VD);
+  if (s.spills && p.sp_keep_p == nullptr) {
+    nsa_set_error("decode_fused: head dims %d/%d need scratch memory", D, VD);
+    return NSA_ERR_WORKSPACE;
+  }
+  if (s.lds == 0) {
     nsa_set_error("decode_fused: head dims %d/%d or fixed_y_maxlen %d / fixed_num_slc_blocks %d / table width %d do "
                   "not fit the one-launch kernel (160 KB of LDS); use the two-launch path", D, VD, p.y_cap, p.nb_cap,
                   p.table_stride);
     return NSA_ERR_UNSUPPORTED;
   }
-  if (D == 128) return launch_dyn(decode_fused_kernel<128, 128>, grid, (size_t)dyn, p, stream, "decode_fused_kernel");
-  return launch_dyn(decode_fused_kernel<64, 64>, grid, (size_t)dyn, p, stream, "decode_fused_kernel");
+  const dim3 grid(B, p.KH);
+  if (D == 128) return launch_fused<128, 128>(p, s, grid, stream);
+  if (D == 64) return launch_fused<64, 64>(p, s, grid, stream);
+  return launch_fused<192, 128>(p, s, grid, stream);
 }

@@ -116,6 +116,8 @@ int nsa_decode_split_static(const void* q, int64_t q_st, int64_t q_sh, const voi
   NSA_REQUIRE(B >= 0 && KH > 0 && VD > 0 && nsplit >= 1 && nsplit <= 64 && fixed_y_maxlen >= 1, NSA_ERR_BAD_ARG,
               "decode_split_static: bad sizes B %d, kv heads %d, VD %d, nsplit %d, fixed_y_maxlen %d", B, KH, VD,
               nsplit, fixed_y_maxlen);
+  NSA_REQUIRE(D <= 128, NSA_ERR_UNSUPPORTED, "decode_split_static: head dim %d (the static scratch holds fp16 "
+              "probabilities: 64 or 128 q/k channels)", D);
   const ScratchLayout s = layout(B, KH, VD, nsplit, fixed_y_maxlen);
   NSA_REQUIRE(s.total <= STATIC_SCRATCH_BYTES, NSA_ERR_UNSUPPORTED,
               "decode_split_static: B %d x kv heads %d x nsplit %d at fixed_y_maxlen %d needs %zu bytes of scratch, "

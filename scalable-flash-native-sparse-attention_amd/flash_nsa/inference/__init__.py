@@ -51,7 +51,7 @@ def nsa_prefill(q, k, v, w, x_cu_seqlens, y_cu_seqlens, x_maxlen, y_maxlen, cont
     return combine_prefill(cmp_o, slc_o, swa_o, w)
 
 
-def auto_cmp_splits(batch, num_kv_heads, fixed_y_maxlen, num_cus=256, one_launch_fits=None):
+def auto_cmp_splits(batch, num_kv_heads, fixed_y_maxlen, num_cus=256, one_launch_fits=None, qk_dim=128):
     """Parts the compressed branch of a decode step is cut into per (request, kv head); 1 = not cut.
     one_launch_fits: whether the one-launch kernel holds this capacity (None: assumed up to 2048 compressed rows).
     Measured on MI355X (4 kv heads, d = 128, graph replay, microseconds for 1 / 2 / 4 / 8 parts):
@@ -61,13 +61,24 @@ def auto_cmp_splits(batch, num_kv_heads, fixed_y_maxlen, num_cus=256, one_launch
       capacity 8192 rows (two launches without parts): 8 x 64K 105 / 72 / 68 / 64, 16 x 64K 114 / 80 / 77 / 80,
       16 x 128K 192 / 127 / 114 / 114, 32 x 64K 140 / 111 / 119 / 126, 32 x 128K 240 / 185 / 188 / 191;
       8 / 16 / 32 / 64 parts: 1 x 128K 61.3 / 58.8 / 61.1 / 69.1, 2 x 128K 64.8 / 62.7 / 65.9 / 76.8, 4 x 128K
-      67.9 / 68.3 / 76.7 / 89.6 -- 16 parts pay for up to 8 pairs."""
+      67.9 / 68.3 / 76.7 / 89.6 -- 16 parts pay for up to 8 pairs.
+    192 q/k channels (2 kv heads, four waves in the one-launch kernel whatever the capacity, 1 / 2 / 4 / 8 / 16 parts):
+      16 x 1K-32K 72 / 63 / 63 / 59 / 64, 32 x 1K-32K 80 / 70 / 70 / 71 / 80, 64 x 4K 67 / 66 / 70 / 68 / 82, 64 x 1K-32K
+      92 / 88 / 87 / 94 / 115, 128 x 4K-32K 127 / 137 / 127 / 139 / 173; capacity 8192: 4 x 128K 148 / 109 / 87 / 71 / 68,
+      16 x 128K 173 / 126 / 97 / 86 / 94, 32 x 128K 181 / 141 / 123 / 124 / 130."""
     pairs = batch * num_kv_heads
     if fixed_y_maxlen < 1024:
         return 1
     if one_launch_fits is None:
         one_launch_fits = fixed_y_maxlen <= 2048
     scale = num_cus / 256.0
+    if qk_dim > 128:
+        if pairs <= 8 * scale and fixed_y_maxlen >= 8192:
+            return 16
+        for parts, most in ((8, 32), (4, 64), (2 if fixed_y_maxlen < 8192 else 4, 128)):
+            if pairs <= most * scale:
+                return parts
+        return 1
     if one_launch_fits:
         return 8 if pairs <= 16 * scale else 1
     if pairs <= 8 * scale and fixed_y_maxlen >= 8192:
@@ -103,7 +114,8 @@ def nsa_decode(q, k, v, w, context_lens, block_tables, cmp_slot_mapping, cmp_blo
         # q-heads per kv head)
         if fused_decode_supported(q, k, v):
             fits = decode_one_launch_fits(q, k, v, block_tables, fixed_y_maxlen, fixed_num_slc_blocks)
-            cmp_num_splits = auto_cmp_splits(q.size(0), k.size(2), fixed_y_maxlen, one_launch_fits=fits)
+            cmp_num_splits = auto_cmp_splits(q.size(0), k.size(2), fixed_y_maxlen, one_launch_fits=fits,
+                                             qk_dim=q.size(-1))
         else:
             cmp_num_splits = 1
     one_launch = (fused_decode_supported(q, k, v) and cmp_num_splits <= 1 and

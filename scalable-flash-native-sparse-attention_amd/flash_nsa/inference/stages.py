@@ -230,7 +230,7 @@ def combine_decode(a, b, c, w):
 # ------------------------------------------------------------------------------------------------ fused decode
 def fused_decode_supported(q, k, v):
     QH, KH = q.size(1), k.size(2)
-    return QH // KH <= 16 and (q.size(-1), v.size(-1)) in ((128, 128), (64, 64))
+    return QH // KH <= 16 and (q.size(-1), v.size(-1)) in ((128, 128), (64, 64), (192, 128))
 
 
 def decode_one_launch_fits(q, k, v, block_tables, fixed_y_maxlen, fixed_num_slc_blocks):
@@ -264,7 +264,10 @@ def decode_one_launch(q, k, v, w, block_tables, cmp_block_tables, context_lens, 
         assert new_v.shape == (B, KH, VD) and new_k.stride(-1) == 1 and new_v.stride(-1) == 1
     topk = torch.empty(KH, B, top_n, device=dev, dtype=torch.int32) if return_parts else None
     lse = torch.empty(B, QH, device=dev, dtype=torch.float32) if return_parts else None
-    _lib.call("nsa_decode_fused", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(), vsr,
+    need = _lib.value("nsa_decode_fused_scratch_bytes", B, KH, D, VD, int(fixed_y_maxlen), int(fixed_num_slc_blocks),
+                      block_tables.stride(0), page)
+    scratch = torch.empty(need, device=dev, dtype=torch.uint8) if need else None
+    _lib.call("nsa_decode_fused_ws", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(), vsr,
               vsh, w.data_ptr(), w.stride(0), w.stride(1), out.data_ptr(), out.stride(0), out.stride(1),
               _lib.ptr(parts[0]), _lib.ptr(parts[1]), _lib.ptr(parts[2]), out.stride(0), out.stride(1),
               _lib.ptr(lse), lse.stride(0) if return_parts else 0, lse.stride(1) if return_parts else 0,
@@ -276,7 +279,7 @@ def decode_one_launch(q, k, v, w, block_tables, cmp_block_tables, context_lens, 
               new_v.stride(0) if store else 0, new_v.stride(1) if store else 0,
               _i32(slot_mapping).data_ptr() if store else None, page, B, QH, KH, D, VD,
               int(fixed_y_maxlen), int(fixed_num_slc_blocks), kernel_size, stride, block_size, top_n, num_inital,
-              num_local, -1, window_size, sm_scale, _lib.stream_ptr())
+              num_local, -1, window_size, sm_scale, _lib.ptr(scratch), need, _lib.stream_ptr())
     if return_parts:
         return out, parts[0], parts[1], parts[2], topk, lse
     return out
@@ -385,7 +388,8 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
     ycap32 = (int(fixed_y_maxlen) + 31) // 32 * 32
     sp_ml = torch.empty(2, B, KH, nsplit, 16, device=dev, dtype=torch.float32)
     sp_o = torch.empty(B, KH, nsplit, 16, VD, device=dev, dtype=torch.float32)
-    keep_p = torch.empty(B, KH, 16, ycap32, device=dev, dtype=torch.float16)
+    # 192 q/k channels: the probabilities of the block scores stay fp32
+    keep_p = torch.empty(B, KH, 16, ycap32, device=dev, dtype=torch.float16 if D <= 128 else torch.float32)
     keep_m = torch.empty(B, KH, ycap32 // 32, 16, device=dev, dtype=torch.float32)
     args = (q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(), vsr,
             vsh, w.data_ptr(), w.stride(0), w.stride(1), out.data_ptr(), out.stride(0), out.stride(1),
