@@ -56,6 +56,13 @@ int nsa_combine_fwd(const void* a, const void* b, const void* c, int64_t i_st, i
 int nsa_combine_bwd(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
                     int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
                     void* dc, void* dw, float* delta3, int64_t T, int H, int D, void* stream);
+/* the same with b = selected and c = window branch, folding the selected branch's gradient over the window's keys into the
+ * window's for the tokens at positions below all_below (log-sum-exps of the two branches [T,H] with strides l_st, l_sh) */
+int nsa_combine_bwd_tail(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
+                         int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
+                         void* dc, void* dw, float* delta3, const float* slc_lse, const float* swa_lse, int64_t l_st,
+                         int64_t l_sh, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D,
+                         void* stream);
 /* flash_nsa/ops/compress_attn.py:160-184 _bwd_preprocess: delta[T,H] fp32 = rowsum(o*do) */
 int nsa_delta(const void* o, int64_t o_st, int64_t o_sh, const void* dO, int64_t d_st, int64_t d_sh, float* delta,
               int64_t T, int H, int D, void* stream);
@@ -70,6 +77,18 @@ int nsa_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_
                 const void* v, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh, float* lse,
                 int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D,
                 int VD, int window, float sm_scale, void* stream);
+/* nsa_swa_fwd, and in the same launch
+ *   - the selected branch of the queries at positions below all_below, which select every block they can see: the window
+ *     branch continued over the keys before the window -> slc_o / slc_lse (may be null) of those queries;
+ *   - with `out`: the gated sum of the three branches (nsa_combine_fwd), the selected branch of the other queries read
+ *     from slc_o.  store_branches 0: o and slc_o are then scratch that may or may not be written. */
+int nsa_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                     const void* v, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh, float* lse,
+                     int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh, float* slc_lse,
+                     int64_t sl_st, int64_t sl_sh, int all_below, const void* cmp_o, int64_t co_st, int64_t co_sh,
+                     const void* w, int64_t w_st, int64_t w_sh, void* out, int64_t out_st, int64_t out_sh,
+                     int store_branches, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
+                     int window, float sm_scale, void* stream);
 /* flash_nsa/ops/topk.py:630-775 slc_topk_indices; topk int32 addressed kh*tk_sh + tok*tk_st + slot;
  * imp_out optional fp32 block scores [KH, T, imp_cols] */
 int nsa_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
@@ -108,15 +127,14 @@ int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
                      void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
                      const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD, int block_size,
                      int top_n, float sm_scale, void* stream);
-/* the same where the caller knows that the queries at positions below all_below (<= top_n * block_size) select every
- * block they can see, as the selector's own output does: they run as full causal attention on the dense tile kernel and
- * their topk rows are not read.  Likewise nsa_slc_attn_bwd_dq_full and nsa_paged_slc_attn_fwd_full (max_context: a bound
- * of the longest context, 0 if unknown) */
-int nsa_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+/* the same for the queries at positions >= t_begin only, as nsa_slc_attn_bwd_dq_from, nsa_paged_slc_attn_fwd_from and
+ * nsa_build_inverse_index_from: the queries below top_n * block_size select every block they can see, and
+ * nsa_swa_fwd_tail / nsa_swa_bwd_dq_tail / nsa_combine_bwd_tail finish their selected branch with the window's */
+int nsa_slc_attn_fwd_from(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                           const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh,
                           int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st,
                           int64_t lse_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
-                          int block_size, int top_n, int all_below, float sm_scale, void* stream);
+                          int block_size, int top_n, int t_begin, float sm_scale, void* stream);
 
 /* ---- backward ----
  * dq_mode: 0 = store bf16, 1 = store fp32, 2 = add into an existing fp32 buffer (single writer per element).
@@ -172,6 +190,15 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
                    const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                    int64_t delta_sh, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu,
                    int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
+/* nsa_swa_bwd_dq with dq_mode 2 (add into fp32) for gradients from nsa_combine_bwd_tail: the queries at positions below
+ * all_below also take the selected branch's keys before their window, and their dq is stored instead of added */
+int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
+                        int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                        int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
+                        int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
 /* same upstream site.  dkv_is_f32 0 / 1: dk/dv are stored (every key row has exactly one writer), bf16 / fp32; 2: added
  * with fp32 atomics into the caller's initialised fp32 buffers, which lets the launch cut the queries of a key tile into
  * nsa_swa_bwd_dkdv_splits(...) chunks (1 where the key tiles alone fill the GPU) */
@@ -189,23 +216,24 @@ int nsa_slc_attn_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
                         int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream);
-int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+int nsa_slc_attn_bwd_dq_from(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                         const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                         const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
-                        int KH, int D, int VD, int block_size, int top_n, int all_below,
+                        int KH, int D, int VD, int block_size, int top_n, int t_begin,
                         float sm_scale, void* stream);
-/* dk/dv of the queries at positions below all_below, added into the caller's fp32 buffers; with an inverse index that
- * leaves them out (nsa_build_inverse_index_from) this completes nsa_slc_attn_bwd_dkdv.  ordered: the summation order does
- * not change between runs */
-int nsa_slc_attn_bwd_dkdv_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
-                                const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st,
-                                int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta,
-                                int64_t delta_st, int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh,
-                                float* dv, int64_t dv_sr, int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen,
-                                int QH, int KH, int D, int VD, int all_below, int ordered, float sm_scale,
-                                void* stream);
+/* dk/dv of the selected branch of the queries at positions below all_below over the keys before their window, added into
+ * the caller's fp32 buffers (the keys of the window are in the window branch's gradient: nsa_combine_bwd_tail).  ordered:
+ * the summation order does not change between runs */
+int nsa_slc_attn_bwd_dkdv_before_window(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr,
+                                        int64_t k_sh, const void* v, int64_t v_sr, int64_t v_sh, const void* dO,
+                                        int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st,
+                                        int64_t lse_sh, const float* delta, int64_t delta_st, int64_t delta_sh,
+                                        float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                                        int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH,
+                                        int D, int VD, int window, int all_below, int ordered, float sm_scale,
+                                        void* stream);
 /* flash_nsa/ops/topk.py:889-945 get_bind_from_find: inverse of the selection as a CSR.
  *   csr_off  [KH][nblk_total+1] absolute start of each (kv head, global block) list inside csr_tok
  *   csr_tok  [KH*T*top_n]       query tokens (index local to their sequence), ascending within a list
@@ -269,6 +297,15 @@ int nsa_paged_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_c
                       float* lse, int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                       const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen, int QH,
                       int KH, int D, int VD, int window, float sm_scale, void* stream);
+int nsa_paged_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                           const void* v_cache, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh,
+                           float* lse, int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh,
+                           float* slc_lse, int64_t sl_st, int64_t sl_sh, int all_below, const void* cmp_o,
+                           int64_t co_st, int64_t co_sh, const void* w, int64_t w_st, int64_t w_sh, void* out,
+                           int64_t out_st, int64_t out_sh, int store_branches, const int32_t* x_cu,
+                           const int32_t* context_lens, const int32_t* block_tables, int table_stride, int page_size,
+                           int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale,
+                           void* stream);
 /* flash_nsa/inference/topk.py:184-298 topk_prefill / :495-623 topk_decode (causality is masked per row here) */
 int nsa_paged_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
                           int64_t k_sh, const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk,
@@ -301,13 +338,13 @@ int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
                            int QH, int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream);
-int nsa_paged_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+int nsa_paged_slc_attn_fwd_from(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
                            int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, const int32_t* topk,
                            int64_t tk_sh, int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse,
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
-                           int QH, int KH, int D, int VD, int block_size, int top_n, int all_below,
-                           int max_context, float sm_scale, void* stream);
+                           int QH, int KH, int D, int VD, int block_size, int top_n, int t_begin,
+                           float sm_scale, void* stream);
 
 /* flash_nsa/inference/compress_kv.py:191-220 mean_pooling_prefill (in-pool write at flat row slot) */
 int nsa_paged_pool_prefill(void* cache, int64_t c_sr, int64_t c_sh, const int32_t* y_cu, const int32_t* block_tables,

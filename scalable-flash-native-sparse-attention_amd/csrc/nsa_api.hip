@@ -147,6 +147,49 @@ int nsa_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_
   return nsa_fwd_tile_launch(p, 1, false, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
+static int fill_swa_tail(NsaFwdTileParams& p, const char* who, void* slc_o, int64_t so_st, int64_t so_sh,
+                         float* slc_lse, int64_t sl_st, int64_t sl_sh, int all_below, const void* cmp_o,
+                         int64_t co_st, int64_t co_sh, const void* w, int64_t w_st, int64_t w_sh, void* out,
+                         int64_t out_st, int64_t out_sh, int store_branches) {
+  NSA_REQUIRE(all_below >= 0 && slc_o != nullptr && p.o != nullptr, NSA_ERR_BAD_ARG,
+              "%s: all_below %d must be >= 0 and both branch outputs given", who, all_below);
+  NSA_REQUIRE(out == nullptr || (cmp_o != nullptr && w != nullptr), NSA_ERR_BAD_ARG,
+              "%s: the combined output needs the compressed branch and the gates", who);
+  p.all_below = all_below; p.store_branches = store_branches;
+  p.slc_o = (bf16_t*)slc_o; p.so_st = so_st; p.so_sh = so_sh;
+  p.slc_lse = slc_lse; p.sl_st = sl_st; p.sl_sh = sl_sh;
+  p.cmp_o = (const bf16_t*)cmp_o; p.co_st = co_st; p.co_sh = co_sh;
+  p.w = (const bf16_t*)w; p.w_st = w_st; p.w_sh = w_sh;
+  p.out = (bf16_t*)out; p.out_st = out_st; p.out_sh = out_sh;
+  return NSA_OK;
+}
+
+int nsa_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                     const void* v, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh, float* lse,
+                     int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh, float* slc_lse,
+                     int64_t sl_st, int64_t sl_sh, int all_below, const void* cmp_o, int64_t co_st, int64_t co_sh,
+                     const void* w, int64_t w_st, int64_t w_sh, void* out, int64_t out_st, int64_t out_sh,
+                     int store_branches, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
+                     int window, float sm_scale, void* stream) {
+  int rc = check_heads("swa_fwd_tail", QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0, NSA_ERR_BAD_ARG, "swa_fwd_tail: window %d must be >= 0", window);
+  NsaFwdTileParams p{};
+  p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
+  p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
+  p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
+  p.o = (bf16_t*)o; p.o_st = o_st; p.o_sh = o_sh;
+  p.lse = lse; p.lse_st = lse_st; p.lse_sh = lse_sh;
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.G = QH / KH; p.KH = KH;
+  p.scale_log2 = sm_scale * NSA_LOG2E;
+  p.kernel_size = 1; p.stride = 1; p.window = window;
+  rc = fill_swa_tail(p, "swa_fwd_tail", slc_o, so_st, so_sh, slc_lse, sl_st, sl_sh, all_below, cmp_o, co_st, co_sh, w,
+                     w_st, w_sh, out, out_st, out_sh, store_branches);
+  if (rc) return rc;
+  return nsa_fwd_tile_launch(p, 2, false, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
 static int topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
                             const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
                             int64_t tk_st, float* imp_out, int64_t imp_sh, int64_t imp_st, int imp_cols,
@@ -224,11 +267,8 @@ int nsa_topk_select_ws_from(const void* q, int64_t q_st, int64_t q_sh, const voi
                           workspace_bytes, stream);
 }
 
-// The queries at positions below all_below (at most top_n blocks) select every block they can see: full causal
-// attention, on the dense tile kernel, whose 64-key tiles serve eight tokens instead of one.
-static int check_all_below(const char* who, int all_below, int top_n, int block_size) {
-  NSA_REQUIRE(all_below >= 0 && all_below <= top_n * block_size, NSA_ERR_BAD_ARG,
-              "%s: all_below %d exceeds top_n %d blocks of %d", who, all_below, top_n, block_size);
+static int check_positions(const char* who, int pos) {
+  NSA_REQUIRE(pos >= 0, NSA_ERR_BAD_ARG, "%s: position %d must be >= 0", who, pos);
   return NSA_OK;
 }
 
@@ -237,37 +277,23 @@ int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
                      void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
                      const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD, int block_size,
                      int top_n, float sm_scale, void* stream) {
-  return nsa_slc_attn_fwd_full(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, topk, tk_sh, tk_st, o, o_st, o_sh, lse,
+  return nsa_slc_attn_fwd_from(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, topk, tk_sh, tk_st, o, o_st, o_sh, lse,
                                lse_st, lse_sh, x_cu, B, x_maxlen, QH, KH, D, VD, block_size, top_n, 0, sm_scale,
                                stream);
 }
 
-int nsa_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+int nsa_slc_attn_fwd_from(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                           const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh,
                           int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st,
                           int64_t lse_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
-                          int block_size, int top_n, int all_below, float sm_scale, void* stream) {
+                          int block_size, int top_n, int t_begin, float sm_scale, void* stream) {
   int rc = check_heads("slc_attn_fwd", QH, KH, D, VD);
   if (rc) return rc;
   NSA_REQUIRE(block_size % 32 == 0 && block_size > 0, NSA_ERR_UNSUPPORTED,
               "slc_attn_fwd: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "slc_attn_fwd: top_n %d must be in [1,64]", top_n);
-  rc = check_all_below("slc_attn_fwd", all_below, top_n, block_size);
+  rc = check_positions("slc_attn_fwd", t_begin);
   if (rc) return rc;
-  if (all_below > 0) {
-    NsaFwdTileParams p{};
-    p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
-    p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
-    p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
-    p.o = (bf16_t*)o; p.o_st = o_st; p.o_sh = o_sh;
-    p.lse = lse; p.lse_st = lse_st; p.lse_sh = lse_sh;
-    p.x_cu = x_cu; p.k_cu = x_cu;
-    p.G = QH / KH; p.KH = KH;
-    p.scale_log2 = sm_scale * NSA_LOG2E;
-    p.kernel_size = 1; p.stride = 1; p.window = all_below; p.t_end = all_below;
-    rc = nsa_fwd_tile_launch(p, 1, false, B, x_maxlen, D, VD, (hipStream_t)stream);
-    if (rc) return rc;
-  }
   NsaSlcParams p{};
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
@@ -278,7 +304,7 @@ int nsa_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void*
   p.x_cu = x_cu;
   p.G = QH / KH; p.KH = KH; p.top_n = top_n; p.block_size = block_size;
   p.scale_log2 = sm_scale * NSA_LOG2E;
-  p.t_begin = all_below;
+  p.t_begin = t_begin;
   return nsa_slc_fwd_launch(p, false, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
@@ -505,6 +531,30 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
   return nsa_bwd_dq_tile_launch(p, 1, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
+int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
+                        int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                        int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
+                        int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream) {
+  int rc = check_heads("swa_bwd_dq_tail", QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0 && all_below >= 0, NSA_ERR_BAD_ARG, "swa_bwd_dq_tail: window %d and all_below %d must be >= 0",
+              window, all_below);
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh; p.dq_mode = 2;
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.window = window;
+  p.all_below = all_below;
+  p.dO2 = (const bf16_t*)slc_dO; p.do2_st = sdo_st; p.do2_sh = sdo_sh;
+  p.lse2 = slc_lse; p.lse2_st = sl_st; p.lse2_sh = sl_sh;
+  p.delta2 = slc_delta; p.delta2_st = sd_st; p.delta2_sh = sd_sh;
+  return nsa_bwd_dq_tile_launch(p, 2, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
 int nsa_swa_bwd_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, int window) {
   if (B <= 0 || x_maxlen <= 0 || QH <= 0 || KH <= 0) return 1;
   const int knob = nsa_tuning_knob("swa_dkdv_splits", 0);
@@ -553,17 +603,17 @@ int nsa_slc_attn_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
                         int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream) {
-  return nsa_slc_attn_bwd_dq_full(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh,
+  return nsa_slc_attn_bwd_dq_from(q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh,
                                   delta, delta_st, delta_sh, topk, tk_sh, tk_st, dq, dq_st, dq_sh, dq_mode, x_cu, B,
                                   x_maxlen, QH, KH, D, VD, block_size, top_n, 0, sm_scale, stream);
 }
 
-int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+int nsa_slc_attn_bwd_dq_from(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                         const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                         const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                         int64_t delta_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st, void* dq,
                         int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu, int B, int x_maxlen, int QH,
-                        int KH, int D, int VD, int block_size, int top_n, int all_below,
+                        int KH, int D, int VD, int block_size, int top_n, int t_begin,
                         float sm_scale, void* stream) {
   int rc = check_heads("slc_attn_bwd_dq", QH, KH, D, VD);
   if (rc) return rc;
@@ -571,20 +621,10 @@ int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const vo
               "slc_attn_bwd_dq: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "slc_attn_bwd_dq: top_n %d must be in [1,64]", top_n);
   NSA_REQUIRE(dq_mode >= 0 && dq_mode <= 2, NSA_ERR_BAD_ARG, "slc_attn_bwd_dq: dq_mode %d not in {0,1,2}", dq_mode);
-  rc = check_all_below("slc_attn_bwd_dq", all_below, top_n, block_size);
+  rc = check_positions("slc_attn_bwd_dq", t_begin);
   if (rc) return rc;
-  if (all_below > 0) {
-    BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
-                delta_sh};
-    NsaBwdTileParams t = make_bwd(c, QH, KH, sm_scale);
-    t.dq = dq; t.dq_st = dq_st; t.dq_sh = dq_sh; t.dq_mode = dq_mode;
-    t.x_cu = x_cu; t.k_cu = x_cu;
-    t.window = all_below; t.t_end = all_below;
-    rc = nsa_bwd_dq_tile_launch(t, 1, B, x_maxlen, D, VD, (hipStream_t)stream);
-    if (rc) return rc;
-  }
   NsaSlcBwdDqParams p{};
-  p.t_begin = all_below;
+  p.t_begin = t_begin;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
   p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
@@ -599,27 +639,30 @@ int nsa_slc_attn_bwd_dq_full(const void* q, int64_t q_st, int64_t q_sh, const vo
   return nsa_slc_bwd_dq_launch(p, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
-int nsa_slc_attn_bwd_dkdv_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
-                                const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st,
-                                int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta,
-                                int64_t delta_st, int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh,
-                                float* dv, int64_t dv_sr, int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen,
-                                int QH, int KH, int D, int VD, int all_below, int ordered, float sm_scale,
-                                void* stream) {
-  int rc = check_heads("slc_attn_bwd_dkdv_dense", QH, KH, D, VD);
+int nsa_slc_attn_bwd_dkdv_before_window(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr,
+                                        int64_t k_sh, const void* v, int64_t v_sr, int64_t v_sh, const void* dO,
+                                        int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st,
+                                        int64_t lse_sh, const float* delta, int64_t delta_st, int64_t delta_sh,
+                                        float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                                        int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH,
+                                        int D, int VD, int window, int all_below, int ordered, float sm_scale,
+                                        void* stream) {
+  int rc = check_heads("slc_attn_bwd_dkdv_before_window", QH, KH, D, VD);
   if (rc) return rc;
-  NSA_REQUIRE(all_below > 0, NSA_ERR_BAD_ARG, "slc_attn_bwd_dkdv_dense: all_below %d must be positive", all_below);
+  NSA_REQUIRE(window >= 0 && all_below >= 0, NSA_ERR_BAD_ARG,
+              "slc_attn_bwd_dkdv_before_window: window %d and all_below %d must be >= 0", window, all_below);
+  const int len = (x_maxlen < all_below ? x_maxlen : all_below) - window - 1;  // positions that are some query's keys
+  if (len <= 0) return NSA_OK;
   BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
               delta_sh};
   NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
   p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
   p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
   p.dkv_mode = 3;
-  const int len = x_maxlen < all_below ? x_maxlen : all_below;
   // one workgroup per key tile adds exactly once to every element: no order to vary
   p.grid_chunks = ordered ? 1 : nsa_swa_bwd_dkdv_splits(B, len, QH, KH, D, VD, len);
   p.x_cu = x_cu; p.k_cu = x_cu;
-  p.window = all_below; p.t_end = all_below;
+  p.min_dist = window + 1; p.window = all_below; p.t_end = all_below;
   return nsa_bwd_dkdv_launch(p, 1, B, x_maxlen, x_maxlen, D, VD, 0, (hipStream_t)stream);
 }
 
@@ -744,7 +787,7 @@ static NsaFwdTileParams paged_window_params(const void* q, int64_t q_st, int64_t
                                             int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh,
                                             const int32_t* x_cu, const int32_t* context_lens,
                                             const int32_t* block_tables, int table_stride, int page_size, int QH,
-                                            int KH, int window, int t_end, float sm_scale) {
+                                            int KH, int window, float sm_scale) {
   NsaFwdTileParams p{};
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k_cache; p.k_sr = k_sr; p.k_sh = k_sh;
@@ -755,7 +798,7 @@ static NsaFwdTileParams paged_window_params(const void* q, int64_t q_st, int64_t
   p.table = block_tables; p.table_stride = table_stride; p.page_size = page_size;
   p.G = QH / KH; p.KH = KH;
   p.scale_log2 = sm_scale * NSA_LOG2E;
-  p.kernel_size = 1; p.stride = 1; p.window = window; p.t_end = t_end;
+  p.kernel_size = 1; p.stride = 1; p.window = window;
   return p;
 }
 
@@ -770,8 +813,31 @@ int nsa_paged_swa_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k_c
   if (rc) return rc;
   return nsa_fwd_tile_launch(paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh,
                                                  lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
-                                                 page_size, QH, KH, window, 0, sm_scale),
+                                                 page_size, QH, KH, window, sm_scale),
                              1, true, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
+int nsa_paged_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                           const void* v_cache, int64_t v_sr, int64_t v_sh, void* o, int64_t o_st, int64_t o_sh,
+                           float* lse, int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh,
+                           float* slc_lse, int64_t sl_st, int64_t sl_sh, int all_below, const void* cmp_o,
+                           int64_t co_st, int64_t co_sh, const void* w, int64_t w_st, int64_t w_sh, void* out,
+                           int64_t out_st, int64_t out_sh, int store_branches, const int32_t* x_cu,
+                           const int32_t* context_lens, const int32_t* block_tables, int table_stride, int page_size,
+                           int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale,
+                           void* stream) {
+  int rc = check_heads("paged_swa_fwd_tail", QH, KH, D, VD);
+  if (rc) return rc;
+  rc = check_page("paged_swa_fwd_tail", page_size);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0, NSA_ERR_BAD_ARG, "paged_swa_fwd_tail: window %d must be >= 0", window);
+  NsaFwdTileParams p = paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh, lse,
+                                           lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride, page_size,
+                                           QH, KH, window, sm_scale);
+  rc = fill_swa_tail(p, "paged_swa_fwd_tail", slc_o, so_st, so_sh, slc_lse, sl_st, sl_sh, all_below, cmp_o, co_st,
+                     co_sh, w, w_st, w_sh, out, out_st, out_sh, store_branches);
+  if (rc) return rc;
+  return nsa_fwd_tile_launch(p, 2, true, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
 static int paged_topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
@@ -862,18 +928,18 @@ int nsa_paged_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
                            int QH, int KH, int D, int VD, int block_size, int top_n, float sm_scale, void* stream) {
-  return nsa_paged_slc_attn_fwd_full(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, topk, tk_sh, tk_st, o,
+  return nsa_paged_slc_attn_fwd_from(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, topk, tk_sh, tk_st, o,
                                      o_st, o_sh, lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
-                                     page_size, B, x_maxlen, QH, KH, D, VD, block_size, top_n, 0, 0, sm_scale, stream);
+                                     page_size, B, x_maxlen, QH, KH, D, VD, block_size, top_n, 0, sm_scale, stream);
 }
 
-int nsa_paged_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
+int nsa_paged_slc_attn_fwd_from(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
                            int64_t k_sh, const void* v_cache, int64_t v_sr, int64_t v_sh, const int32_t* topk,
                            int64_t tk_sh, int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse,
                            int64_t lse_st, int64_t lse_sh, const int32_t* x_cu, const int32_t* context_lens,
                            const int32_t* block_tables, int table_stride, int page_size, int B, int x_maxlen,
-                           int QH, int KH, int D, int VD, int block_size, int top_n, int all_below,
-                           int max_context, float sm_scale, void* stream) {
+                           int QH, int KH, int D, int VD, int block_size, int top_n, int t_begin,
+                           float sm_scale, void* stream) {
   int rc = check_heads("paged_slc_attn_fwd", QH, KH, D, VD);
   if (rc) return rc;
   rc = check_page("paged_slc_attn_fwd", page_size);
@@ -881,17 +947,10 @@ int nsa_paged_slc_attn_fwd_full(const void* q, int64_t q_st, int64_t q_sh, const
   NSA_REQUIRE(block_size % 32 == 0 && block_size > 0, NSA_ERR_UNSUPPORTED,
               "paged_slc_attn_fwd: block_size %d must be a multiple of 32", block_size);
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "paged_slc_attn_fwd: top_n %d must be in [1,64]", top_n);
-  rc = check_all_below("paged_slc_attn_fwd", all_below, top_n, block_size);
+  rc = check_positions("paged_slc_attn_fwd", t_begin);
   if (rc) return rc;
-  if (all_below > 0) {
-    rc = nsa_fwd_tile_launch(paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh,
-                                                 lse, lse_st, lse_sh, x_cu, context_lens, block_tables, table_stride,
-                                                 page_size, QH, KH, all_below, all_below, sm_scale),
-                             1, true, B, x_maxlen, D, VD, (hipStream_t)stream);
-    if (rc || (max_context > 0 && max_context <= all_below)) return rc;
-  }
   NsaSlcParams p{};
-  p.t_begin = all_below;
+  p.t_begin = t_begin;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k_cache; p.k_sr = k_sr; p.k_sh = k_sh;
   p.v = (const bf16_t*)v_cache; p.v_sr = v_sr; p.v_sh = v_sh;

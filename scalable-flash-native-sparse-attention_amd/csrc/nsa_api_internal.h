@@ -18,7 +18,16 @@ struct NsaFwdTileParams {
   int G, KH;
   float scale_log2;
   int kernel_size, stride, window;
-  int t_end;                                // > 0: only queries at positions below it
+  // window mode with a tail: the queries at positions below all_below select every block they can see, so their
+  // selected branch is the window branch plus the keys before the window; its output and log-sum-exp go to slc_o /
+  // slc_lse.  With `out` the gated sum of the three branches is formed as well (the selected branch of the other queries
+  // is read from slc_o), and o / slc_o are written only if store_branches is set.
+  int all_below, store_branches;
+  bf16_t* slc_o; int64_t so_st, so_sh;
+  float* slc_lse; int64_t sl_st, sl_sh;
+  const bf16_t* cmp_o; int64_t co_st, co_sh;
+  const bf16_t* w; int64_t w_st, w_sh;      // gates [tokens, QH, 3]
+  bf16_t* out; int64_t out_st, out_sh;
 };
 
 struct NsaSlcParams {
@@ -55,7 +64,7 @@ struct NsaTopkParams {
 };
 
 int nsa_fwd_tile_launch(const NsaFwdTileParams& p, int mode, bool paged, int B, int max_q_len, int D, int VD,
-                        hipStream_t stream);
+                        hipStream_t stream);  // mode 0: compressed, 1: window, 2: window with a tail
 int nsa_slc_fwd_launch(const NsaSlcParams& p, bool paged, int B, int max_q_len, int D, int VD, hipStream_t stream);
 int nsa_topk_launch(const NsaTopkParams& p, bool paged, int B, int max_q_len, int D, hipStream_t stream);
 // two launches with the block scores in a workspace (nsa_topk_two_pass.hip)
@@ -92,7 +101,15 @@ struct NsaBwdTileParams {
   int G, KH;
   float scale_log2, sm_scale;
   int kernel_size, stride, window;
-  int t_end;                   // window mode: > 0: only queries at positions below it
+  // window mode: keys at distances min_dist .. window before the query (0: the window itself), of the queries at
+  // positions below t_end (0: all)
+  int min_dist, t_end;
+  // dq of the window with a tail: queries at positions below all_below also take the keys before their window, with the
+  // selected branch's dO2 / lse2 / delta2; their dq is stored, not added
+  int all_below;
+  const bf16_t* dO2; int64_t do2_st, do2_sh;
+  const float* lse2; int64_t lse2_st, lse2_sh;
+  const float* delta2; int64_t delta2_st, delta2_sh;
   int q_chunk_tokens;          // compressed / window dkdv: query tokens per grid.x chunk
   int grid_chunks;             // window dkdv with dkv_mode 3: query chunks per key tile in grid.x
 };

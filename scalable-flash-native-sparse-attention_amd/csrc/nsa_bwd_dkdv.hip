@@ -110,7 +110,7 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
       const int ktile = blockIdx.x / p.grid_chunks;
       key0 = ktile * KW;
       if (key0 >= nkeys) return;
-      const int ta = key0 + (blockIdx.x - ktile * p.grid_chunks) * p.q_chunk_tokens;
+      const int ta = key0 + p.min_dist + (blockIdx.x - ktile * p.grid_chunks) * p.q_chunk_tokens;
       row_begin = ta * G;
       row_end = min(min(xl, key0 + KW + p.window), ta + p.q_chunk_tokens) * G;
     } else if (key0 >= nkeys) {
@@ -392,8 +392,8 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
       any_vis = t_max >= p.stride * kw0 + p.kernel_size - 1;
       full_vis = (n_in == RT) && (t_min >= p.stride * (kw0 + KL) + p.kernel_size - 1) && (kw0 + KL < nkeys);
     } else if (MODE == MODE_SWA) {
-      any_vis = (kw0 <= t_max) && (kw0 + KL >= t_min - p.window);
-      full_vis = (n_in == RT) && (kw0 + KL <= t_min) && (kw0 >= t_max - p.window) && (kw0 + KL < nkeys);
+      any_vis = (kw0 <= t_max - p.min_dist) && (kw0 + KL >= t_min - p.window);
+      full_vis = (n_in == RT) && (kw0 + KL <= t_min - p.min_dist) && (kw0 >= t_max - p.window) && (kw0 + KL < nkeys);
     } else {
       any_vis = kw0 <= t_max;
       full_vis = (n_in == RT) && (kw0 + KL <= t_min) && (kw0 + KL < nkeys);
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
               const int my_key = kw0 + kb * 32 + l32;
               bool vis;
               if (MODE == MODE_CMP) vis = (my_key < nkeys) && (tr >= p.stride * my_key + p.kernel_size - 1);
-              else if (MODE == MODE_SWA) vis = (my_key <= tr) && (my_key >= tr - p.window) && (my_key < nkeys);
+              else if (MODE == MODE_SWA) vis = (my_key <= tr - p.min_dist) && (my_key >= tr - p.window) && (my_key < nkeys);
               else vis = (my_key <= tr) && (my_key < nkeys);
               sacc[kb][i4 * 4 + ii] = vis ? sacc[kb][i4 * 4 + ii] : 0.f;
             }
@@ -602,9 +602,11 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
   } else if (mode == MODE_SWA) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;
     if (p.t_end > 0 && p.t_end < max_k_len) max_k_len = p.t_end;
+    max_k_len -= p.min_dist;  // the last min_dist positions are no query's keys
+    if (max_k_len <= 0) return NSA_OK;
     const int KW = 4 * 32 * (kb_cmp == 2 ? 2 : 1);
     p.grid_chunks = p.dkv_mode == 3 ? p.grid_chunks : 1;
-    p.q_chunk_tokens = cdiv_i(KW + p.window, p.grid_chunks);
+    p.q_chunk_tokens = cdiv_i(KW + p.window - p.min_dist, p.grid_chunks);
     if constexpr (KB2_BUILT) {
       if (kb_cmp == 2) {
         dim3 grid(cdiv_i(max_k_len, 256) * p.grid_chunks, B, p.KH);

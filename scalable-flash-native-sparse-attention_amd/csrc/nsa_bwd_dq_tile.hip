@@ -10,6 +10,7 @@ namespace {
 
 constexpr int MODE_CMP = 0;
 constexpr int MODE_SWA = 1;
+constexpr int MODE_TAIL = 2;  // MODE_SWA; queries below all_below also take the keys before their window (selected branch)
 
 template <int D, int VD, int MODE, int MINB, bool DO_LDS>
 __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams p) {
@@ -35,7 +36,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
 
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int rows_total = (MODE == MODE_SWA && p.t_end > 0 ? min(xl, p.t_end) : xl) * G;
+  const int rows_total = xl * G;
   const int r0 = blockIdx.x * ROWS_WG;
   if (r0 >= rows_total) return;
   int nkeys, kbase;
@@ -69,8 +70,8 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       else dof[kc] = t8;
     }
   }
-  const float lse = p.lse[tok * p.lse_st + (int64_t)head * p.lse_sh];
-  const float delta = p.delta[tok * p.delta_st + (int64_t)head * p.delta_sh];
+  float lse = p.lse[tok * p.lse_st + (int64_t)head * p.lse_sh];
+  float delta = p.delta[tok * p.delta_st + (int64_t)head * p.delta_sh];
 
   const int rw_lo = r0 + wave * ROWS_W;
   const int rw_hi = min(rw_lo + ROWS_W - 1, rows_total - 1);
@@ -117,6 +118,9 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       vreg[j] = ld_global_b128(p.v + ((int64_t)kbase + kt + kr) * p.v_sr + (int64_t)kh * p.v_sh + dp * 8);
     }
   };
+  // window: keys t + klo .. t + khi; before the window: keys .. t + khi, of queries at positions below t_end
+  int klo = -p.window, khi = 0, t_end = 0x7fffffff;
+  auto run_keys = [&]() {
   if (key_begin < key_end) gload(key_begin);
 
   for (int kt = key_begin; kt < key_end; kt += KT) {
@@ -139,8 +143,9 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
       full_vis = (tw_lo >= p.stride * (kt + KT - 1) + p.kernel_size - 1) && (kt + KT <= nkeys);
     } else {
-      any_vis = (kt <= tw_hi) && (kt + KT - 1 >= tw_lo - p.window);
-      full_vis = (kt + KT - 1 <= tw_lo) && (kt >= tw_hi - p.window);
+      any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
+      full_vis = (kt + KT - 1 <= tw_lo + khi) && (kt >= tw_hi + klo);
+      if (MODE == MODE_TAIL) full_vis = full_vis && tw_hi < t_end;
     }
     if (!any_vis) continue;
 
@@ -170,6 +175,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
 #pragma unroll
       for (int i = 0; i < 16; i++) sacc[nt][i] = fast_exp2(__builtin_fmaf(sacc[nt][i], sc, -lsc));
     if (!full_vis) {  // wave-uniform
+      asm volatile("");  // keeps it a branch: if-converted, every tile would pay
 #pragma unroll
       for (int nt = 0; nt < 2; nt++)
 #pragma unroll
@@ -177,7 +183,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
           int key = kt + nt * 32 + (i >> 2) * 8 + hl * 4 + (i & 3);
           bool vis;
           if (MODE == MODE_CMP) vis = (key < nkeys) && (t >= p.stride * key + p.kernel_size - 1);
-          else vis = (key <= t) && (key >= t - p.window);
+          else vis = (key <= t + khi) && (key >= t + klo) && (MODE != MODE_TAIL || t < t_end);
           sacc[nt][i] = vis ? sacc[nt][i] : 0.f;
         }
     }
@@ -202,6 +208,32 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
     }
   }
 
+  };
+  run_keys();
+  if constexpr (MODE == MODE_TAIL) {
+    // The selected branch of these queries inside the window has been folded into the window's incoming gradient; what
+    // is left are the keys before the window.  40 samples of up to 1.2K tokens, 16 heads of 64: the selected dq kernel
+    // 401 -> 51 us, this one 98 -> 110 us; 8 x 6K tokens, 64 heads of 128: 6829 -> 6080 and 1914 -> 1924 us.
+    const int far_end = min(t_hi, p.all_below - 1) - p.window;  // keys before some query's window
+    if (far_end > 0 && t_lo < p.all_below) {                    // workgroup-uniform
+      const bf16_t* dp = p.dO2 + tok * p.do2_st + (int64_t)head * p.do2_sh + hl * 8;
+#pragma unroll
+      for (int kc = 0; kc < VD / 16; kc++) {
+        bf16x8 t8 = ld_global_b128(dp + kc * 16);
+        if (DO_LDS) *reinterpret_cast<bf16x8*>(&dOs[(wave * 32 + l32) * VLD + hl * 8 + kc * 16]) = t8;
+        else dof[kc] = t8;
+      }
+      lse = p.lse2[tok * p.lse2_st + (int64_t)head * p.lse2_sh];
+      delta = p.delta2[tok * p.delta2_st + (int64_t)head * p.delta2_sh];
+      key_begin = 0;
+      key_end = far_end;
+      klo = -0x40000000;
+      khi = -p.window - 1;
+      t_end = p.all_below;
+      run_keys();
+    }
+  }
+
   if (!valid) return;
   const float osc = p.sm_scale;
   const int64_t off = tok * p.dq_st + (int64_t)head * p.dq_sh;
@@ -219,7 +251,7 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
         *reinterpret_cast<bf16x4*>((bf16_t*)p.dq + off + d) = pack4(val[0], val[1], val[2], val[3]);
       } else {
         float* dst = (float*)p.dq + off + d;
-        if (p.dq_mode == 2) val += *reinterpret_cast<f32x4*>(dst);
+        if (p.dq_mode == 2 && (MODE != MODE_TAIL || t >= p.all_below)) val += *reinterpret_cast<f32x4*>(dst);
         *reinterpret_cast<f32x4*>(dst) = val;
       }
     }
@@ -228,7 +260,6 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
 template <int MODE>
 int dispatch(const NsaBwdTileParams& p, int B, int max_q_len, int D, int VD, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
-  if (MODE == MODE_SWA && p.t_end > 0 && p.t_end < max_q_len) max_q_len = p.t_end;
   dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
   const int minb = nsa_tuning_knob("dq_min_blocks", 2);
   if (D == 128 && VD == 128) {
@@ -249,6 +280,7 @@ int dispatch(const NsaBwdTileParams& p, int B, int max_q_len, int D, int VD, hip
 
 int nsa_bwd_dq_tile_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int D, int VD,
                            hipStream_t stream) {
+  if (mode == MODE_TAIL) return dispatch<MODE_TAIL>(p, B, max_q_len, D, VD, stream);
   return mode == MODE_CMP ? dispatch<MODE_CMP>(p, B, max_q_len, D, VD, stream)
                           : dispatch<MODE_SWA>(p, B, max_q_len, D, VD, stream);
 }

@@ -7,6 +7,7 @@
 //           flash_nsa/inference/combine.py:16-127.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include "../../include/nsa_hip.h"
 
 namespace {
 
@@ -205,10 +206,22 @@ __global__ void combine_fwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
 // backward: da,db,dc = dy*sig(w_k); dw_k = sig_k(1-sig_k) * sum_d dy*x_k; optional delta_k = rowsum(x_k * d x_k)
 // with the stored (bf16) d x_k, the softmax-backward correction term of branch k, written as delta[k][T][H] fp32.
 // D/8 consecutive lanes share one (t,h); D/8 must be a power of two <= 64.
+//
+// TAIL: for the tokens at positions below all_below, which select every block they can see, the selected branch b's
+// gradient over the window's keys is folded into the window branch c's.  With P_c = exp2(s - lse_c) and
+// P_b = r P_c, r = exp2(lse_c - lse_b), both branches' dS over a key of the window is
+//   P_c (dO_c . v - delta_c) + P_b (dO_b . v - delta_b) = P_c ((dO_c + r dO_b) . v - (delta_c + r delta_b)),
+// and likewise dV, so c gets dO_c + r dO_b, and what remains of b are the keys before the window.  delta_c is formed so
+// that it matches the rounded sum (b's share of it exactly, c's from what is left).
+struct CombineTail {
+  const float* lse_b; const float* lse_c; int64_t l_st, l_sh;
+  const int32_t* x_cu; int B, all_below;
+};
+template <bool TAIL>
 __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16_t* c, int64_t i_st, int64_t i_sh,
                                    const bf16_t* w, int64_t w_st, int64_t w_sh, const bf16_t* dy, int64_t dy_st,
                                    int64_t dy_sh, bf16_t* da, bf16_t* db, bf16_t* dc, bf16_t* dw, float* delta,
-                                   int64_t T, int H, int D) {
+                                   int64_t T, int H, int D, CombineTail tail) {
   const int C = D / 8;
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool ok = idx < T * H * C;
@@ -221,6 +234,16 @@ __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
   int64_t off = t * i_st + (int64_t)h * i_sh + cc * 8;
   bf16x8 va = ld_global_b128(a + off), vb = ld_global_b128(bb + off), vc = ld_global_b128(c + off);
   bf16x8 g = ld_global_b128(dy + t * dy_st + (int64_t)h * dy_sh + cc * 8);
+  float r = 0.f;  // share of b's gradient that c takes
+  if (TAIL) {
+    int lo = 0, hi = tail.B;  // last sequence that starts at or before t
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (tail.x_cu[mid] <= t) lo = mid; else hi = mid;
+    }
+    if (t - tail.x_cu[lo] < tail.all_below)
+      r = fast_exp2(tail.lse_c[t * tail.l_st + h * tail.l_sh] - tail.lse_b[t * tail.l_st + h * tail.l_sh]);
+  }
   // p_k = sum_d dy * x_k (gate gradient); q_k = sum_d round(dy * sig_k) * x_k: the correction term is formed from
   // the ROUNDED branch gradient, the one the attention backward kernels read, so that dP - delta cancels exactly
   // where a row's probabilities are one-hot (upstream forms it the same way from the stored bf16 tensors,
@@ -231,14 +254,18 @@ __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
   for (int e = 0; e < 8; e++) {
     float gf = (float)g[e];
     float xa = (float)va[e], xb = (float)vb[e], xc = (float)vc[e];
-    ra[e] = (bf16_t)(gf * s0); rb[e] = (bf16_t)(gf * s1); rc[e] = (bf16_t)(gf * s2);
+    ra[e] = (bf16_t)(gf * s0); rb[e] = (bf16_t)(gf * s1);
+    const float b_share = TAIL ? r * (float)rb[e] : 0.f;
+    rc[e] = (bf16_t)(TAIL ? __builtin_fmaf(gf, s2, b_share) : gf * s2);
     p0 += gf * xa; p1 += gf * xb; p2 += gf * xc;
-    q0 += (float)ra[e] * xa; q1 += (float)rb[e] * xb; q2 += (float)rc[e] * xc;
+    q0 += (float)ra[e] * xa; q1 += (float)rb[e] * xb;
+    q2 += ((float)rc[e] - b_share) * xc;
   }
   for (int o = C >> 1; o > 0; o >>= 1) {
     p0 += __shfl_xor(p0, o, 64); p1 += __shfl_xor(p1, o, 64); p2 += __shfl_xor(p2, o, 64);
     q0 += __shfl_xor(q0, o, 64); q1 += __shfl_xor(q1, o, 64); q2 += __shfl_xor(q2, o, 64);
   }
+  if (TAIL) q2 += r * q1;
   if (!ok) return;
   int64_t ooff = (t * H + h) * (int64_t)D + cc * 8;  // grads are contiguous [T,H,D]
   *reinterpret_cast<bf16x8*>(da + ooff) = ra;
@@ -597,13 +624,29 @@ int nsa_combine_fwd(const void* a, const void* b, const void* c, int64_t i_st, i
 int nsa_combine_bwd(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
                     int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
                     void* dc, void* dw, float* delta3, int64_t T, int H, int D, void* stream) {
+  return nsa_combine_bwd_tail(a, b, c, i_st, i_sh, w, w_st, w_sh, dy, dy_st, dy_sh, da, db, dc, dw, delta3, nullptr,
+                              nullptr, 0, 0, nullptr, 0, 0, T, H, D, stream);
+}
+
+int nsa_combine_bwd_tail(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
+                         int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
+                         void* dc, void* dw, float* delta3, const float* slc_lse, const float* swa_lse, int64_t l_st,
+                         int64_t l_sh, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D,
+                         void* stream) {
   int C = D / 8;
   NSA_REQUIRE(D % 8 == 0 && C > 0 && C <= 64 && (C & (C - 1)) == 0, NSA_ERR_BAD_ARG,
               "combine_bwd: head dim %d must be 8 * a power of two <= 512", D);
+  NSA_REQUIRE(all_below <= 0 || (slc_lse && swa_lse && x_cu && B > 0 && delta3), NSA_ERR_BAD_ARG,
+              "combine_bwd_tail: all_below needs the log-sum-exps, the sequence offsets and the delta output");
   if (T <= 0) return NSA_OK;
-  combine_bwd_kernel<<<blocks_for(T * H * C, 256), 256, 0, (hipStream_t)stream>>>(
-      (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)c, i_st, i_sh, (const bf16_t*)w, w_st, w_sh, (const bf16_t*)dy,
-      dy_st, dy_sh, (bf16_t*)da, (bf16_t*)db, (bf16_t*)dc, (bf16_t*)dw, delta3, T, H, D);
+  const CombineTail tail{slc_lse, swa_lse, l_st, l_sh, x_cu, B, all_below};
+  auto launch = [&](auto kern) {
+    kern<<<blocks_for(T * H * C, 256), 256, 0, (hipStream_t)stream>>>(
+        (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)c, i_st, i_sh, (const bf16_t*)w, w_st, w_sh,
+        (const bf16_t*)dy, dy_st, dy_sh, (bf16_t*)da, (bf16_t*)db, (bf16_t*)dc, (bf16_t*)dw, delta3, T, H, D, tail);
+  };
+  if (all_below > 0) launch(combine_bwd_kernel<true>);
+  else launch(combine_bwd_kernel<false>);
   return nsa_check_launch("combine_bwd");
 }
 

@@ -18,6 +18,7 @@ namespace {
 
 constexpr int MODE_CMP = 0;
 constexpr int MODE_SWA = 1;
+constexpr int MODE_TAIL = 2;  // MODE_SWA, and what can be finished in the same launch (below)
 
 typedef __attribute__((address_space(1))) const void* nsa_gptr_t;
 typedef __attribute__((address_space(3))) void* nsa_lptr_t;
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int xl = p.x_cu[b + 1] - x0;
   const int ctx = PAGED ? p.ctx_lens[b] : xl;
   const int qoff = ctx - xl;
-  const int rows_total = (MODE == MODE_SWA && p.t_end > 0 ? min(xl, p.t_end - qoff) : xl) * G;
+  const int rows_total = xl * G;
   const int r0 = blockIdx.x * ROWS_WG;
   if (r0 >= rows_total) return;
   int nkeys, kbase = 0;
@@ -111,6 +112,9 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     key_begin = (max(0, t_lo - p.window) / KT) * KT;
     key_end = min(t_hi + 1, nkeys);
   }
+
+  // window: keys t + klo .. t + khi; before the window: keys .. t + khi, of queries at positions below t_end
+  int klo = -p.window, khi = 0, t_end = 0x7fffffff;
 
   f32x16 oacc[RS][VD / 32];
   float m_run[RS], l_run[RS];
@@ -207,6 +211,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     }
     // ---- mask, online softmax (running max in raw score units; scale folded into the exp2 fma) ----
     if (masked) {  // wave-uniform: only tiles that straddle a visibility boundary pay for the mask
+      asm volatile("");  // keeps it a branch: if-converted, every tile would pay
       const int t = t_row[rs];
 #pragma unroll
       for (int nt = 0; nt < 2; nt++)
@@ -215,7 +220,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
           int key = kt + nt * 32 + (i >> 2) * 8 + hl * 4 + (i & 3);
           bool vis;
           if (MODE == MODE_CMP) vis = (key < nkeys) && (t >= p.stride * key + p.kernel_size - 1);
-          else vis = (key <= t) && (key >= t - p.window);
+          else vis = (key <= t + khi) && (key >= t + klo) && (MODE != MODE_TAIL || t < t_end);
           sacc[nt][i] = vis ? sacc[nt][i] : NSA_NEG_INF;
         }
     }
@@ -326,63 +331,147 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       }
     }
   };
-  if (key_begin < key_end) {
-    if constexpr (ASYNC) {
-      stage_async(key_begin, 0);
-    } else {
-      gload(key_begin);
-      stage(0);
-      if (key_begin + KT < key_end) gload(key_begin + KT);
-    }
-  }
-
-  int buf = 0;
-  for (int kt = key_begin; kt < key_end; kt += KT, buf ^= 1) {
-    if constexpr (ASYNC) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile kt have landed
-    __syncthreads();  // tile kt is visible; nobody reads the other buffer (tile kt - KT) any more
-    if (kt + KT < key_end) {
+  auto run_keys = [&]() {
+    if (key_begin < key_end) {
       if constexpr (ASYNC) {
-        stage_async(kt + KT, buf ^ 1);
+        stage_async(key_begin, 0);
       } else {
-        stage(buf ^ 1);
-        if (kt + 2 * KT < key_end) gload(kt + 2 * KT);
+        gload(key_begin);
+        stage(0);
+        if (key_begin + KT < key_end) gload(key_begin + KT);
       }
     }
-    if (!wave_active) continue;
+    int buf = 0;
+    for (int kt = key_begin; kt < key_end; kt += KT, buf ^= 1) {
+      if constexpr (ASYNC) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile kt have landed
+      __syncthreads();  // tile kt is visible; nobody reads the other buffer (tile kt - KT) any more
+      if (kt + KT < key_end) {
+        if constexpr (ASYNC) {
+          stage_async(kt + KT, buf ^ 1);
+        } else {
+          stage(buf ^ 1);
+          if (kt + 2 * KT < key_end) gload(kt + 2 * KT);
+        }
+      }
+      if (!wave_active) continue;
 
-    // wave-uniform visibility classification of this tile
-    bool any_vis, full_vis;
-    if (MODE == MODE_CMP) {
-      any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
-      full_vis = (tw_lo >= p.stride * (kt + KT - 1) + p.kernel_size - 1) && (kt + KT <= nkeys);
-    } else {
-      any_vis = (kt <= tw_hi) && (kt + KT - 1 >= tw_lo - p.window);
-      full_vis = (kt + KT - 1 <= tw_lo) && (kt >= tw_hi - p.window);
+      // wave-uniform visibility classification of this tile
+      bool any_vis, full_vis;
+      if (MODE == MODE_CMP) {
+        any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
+        full_vis = (tw_lo >= p.stride * (kt + KT - 1) + p.kernel_size - 1) && (kt + KT <= nkeys);
+      } else {
+        any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
+        full_vis = (kt + KT - 1 <= tw_lo + khi) && (kt >= tw_hi + klo);
+        if (MODE == MODE_TAIL) full_vis = full_vis && tw_hi < t_end;
+      }
+      if (!any_vis) continue;
+      process(!full_vis, std::integral_constant<int, 0>{}, kt, Ks2[buf], Vs2[buf]);
+      if constexpr (RS > 1) process(!full_vis, std::integral_constant<int, RS - 1>{}, kt, Ks2[buf], Vs2[buf]);
     }
-    if (!any_vis) continue;
-    process(!full_vis, std::integral_constant<int, 0>{}, kt, Ks2[buf], Vs2[buf]);
-    if constexpr (RS > 1) process(!full_vis, std::integral_constant<int, RS - 1>{}, kt, Ks2[buf], Vs2[buf]);
-  }
+  };
 
-  // ---- epilogue ----
-#pragma unroll
-  for (int rs = 0; rs < RS; rs++) {
-    float l_tot = xhalf_sum(l_run[rs]);
-    if (!valid[rs]) continue;
-    float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    bf16_t* op = p.o + tok[rs] * p.o_st + (int64_t)head[rs] * p.o_sh;
+  // Epilogue.  A lane holds 4-channel pieces of one row; stored (or combined with other tensors) as they lie, every
+  // instruction would touch 32 rows.  The rows pass through LDS instead (bf16, wave-private, 16-byte chunks swizzled by
+  // row) and are handled as whole rows, 16 bytes per lane.
+  constexpr int NC = VD / 8;                     // chunks per row
+  constexpr int RPI = 64 / NC;                   // rows per instruction
+  static_assert(32 * VD * 4 <= 2 * KT * KLD, "the K tiles hold the rows of the four waves");
+  bf16_t* const rows = &Ks2[0][0] + wave * 32 * VD;
+  auto chunk_at = [&](int row, int c) { return rows + row * VD + ((c ^ (row & (NC - 1))) * 8); };
+  // (token, head) of a row of the wave, from the lane that holds it; token -1: none
+  auto row_id = [&](auto rs_tag, int r) {
+    constexpr int rs = decltype(rs_tag)::value;
+    return make_int2(__shfl(valid[rs] ? t_row[rs] - qoff : -1, r, 64), __shfl(head[rs], r, 64));
+  };
+  auto rows_to_lds = [&](auto rs_tag, float inv) {
+    constexpr int rs = decltype(rs_tag)::value;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int dt = 0; dt < VD / 32; dt++)
 #pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        int d = dt * 32 + i4 * 8 + hl * 4;
-        bf16x4 w = pack4(oacc[rs][dt][i4 * 4 + 0] * inv, oacc[rs][dt][i4 * 4 + 1] * inv,
-                         oacc[rs][dt][i4 * 4 + 2] * inv, oacc[rs][dt][i4 * 4 + 3] * inv);
-        *reinterpret_cast<bf16x4*>(op + d) = w;
+      for (int i4 = 0; i4 < 4; i4++)
+        *reinterpret_cast<bf16x4*>(chunk_at(l32, dt * 4 + i4) + hl * 4) =
+            pack4(oacc[rs][dt][i4 * 4 + 0] * inv, oacc[rs][dt][i4 * 4 + 1] * inv, oacc[rs][dt][i4 * 4 + 2] * inv,
+                  oacc[rs][dt][i4 * 4 + 3] * inv);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // the branch output and log-sum-exp of the keys so far, of the queries at positions below `below`
+  auto emit = [&](bf16_t* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh, int below) {
+    auto one = [&](auto rs_tag) {
+      constexpr int rs = decltype(rs_tag)::value;
+      const float l_tot = xhalf_sum(l_run[rs]);
+      rows_to_lds(rs_tag, l_tot > 0.f ? 1.f / l_tot : 0.f);
+      const int c = lane % NC;
+#pragma unroll
+      for (int r = lane / NC; r < 32; r += RPI) {
+        const int2 th = row_id(rs_tag, r);
+        if (th.x < 0 || th.x + qoff >= below) continue;
+        *reinterpret_cast<bf16x8*>(o + ((int64_t)x0 + th.x) * o_st + (int64_t)th.y * o_sh + c * 8) =
+            *reinterpret_cast<const bf16x8*>(chunk_at(r, c));
       }
-    if (hl == 0 && p.lse != nullptr) {
-      float lse2 = l_tot > 0.f ? m_run[rs] * sc + fast_log2(l_tot) : 0.f;
-      p.lse[tok[rs] * p.lse_st + (int64_t)head[rs] * p.lse_sh] = lse2;
+      if (hl == 0 && lse != nullptr && valid[rs] && t_row[rs] < below)
+        lse[tok[rs] * lse_st + (int64_t)head[rs] * lse_sh] = l_tot > 0.f ? m_run[rs] * sc + fast_log2(l_tot) : 0.f;
+    };
+    one(std::integral_constant<int, 0>{});
+    if constexpr (RS > 1) one(std::integral_constant<int, RS - 1>{});
+  };
+  constexpr int ALL = 0x7fffffff;
+  run_keys();
+  __syncthreads();  // the tile buffers are free
+  if constexpr (MODE != MODE_TAIL) {
+    emit(p.o, p.o_st, p.o_sh, p.lse, p.lse_st, p.lse_sh, ALL);
+  } else {
+    static_assert(RS == 1, "");
+    // Queries at positions below all_below select every block they can see: their selected branch is the window branch
+    // continued over the keys before the window (nothing at all up to position `window`), instead of a second pass
+    // over all of their keys.  40 samples of up to 1.2K tokens, 16 heads of 64: selected kernel 278 -> 39 us, window
+    // kernel 69 -> 92 us; 8 x 6K tokens, 64 heads of 128: 4477 -> 3947 us, and with the gated sum at its end
+    // (one read of the branch outputs less) 1774 -> 1674 us.
+    const int far_end = min(t_hi, p.all_below - 1) - p.window;  // keys before some query's window
+    const bool far = far_end > 0 && t_lo < p.all_below;         // workgroup-uniform
+    const bool store = p.store_branches || p.out == nullptr;
+    if (store || far) emit(p.o, p.o_st, p.o_sh, p.lse, p.lse_st, p.lse_sh, ALL);
+    if (far) {
+      __syncthreads();  // the rows in the tile buffers have been stored
+      key_begin = 0;
+      key_end = far_end;
+      klo = -0x40000000;
+      khi = -p.window - 1;
+      t_end = p.all_below;
+      run_keys();
+      __syncthreads();
+    }
+    if (store && t_lo < p.all_below) emit(p.slc_o, p.so_st, p.so_sh, p.slc_lse, p.sl_st, p.sl_sh, p.all_below);
+    if (p.out != nullptr) {
+      // gated sum of the branch outputs, each rounded to bf16 as it is stored: the rows in LDS are the window branch or,
+      // behind the keys before the window, the selected branch
+      const float l_tot = xhalf_sum(l_run[0]);
+      rows_to_lds(std::integral_constant<int, 0>{}, l_tot > 0.f ? 1.f / l_tot : 0.f);
+      const int c = lane % NC;
+#pragma unroll
+      for (int r = lane / NC; r < 32; r += RPI) {
+        const int2 th = row_id(std::integral_constant<int, 0>{}, r);
+        if (th.x < 0) continue;
+        const int64_t tk = (int64_t)x0 + th.x, hd = th.y;
+        const bf16_t* wp = p.w + tk * p.w_st + hd * p.w_sh;
+        const bf16x8 vc = ld_global_b128(p.cmp_o + tk * p.co_st + hd * p.co_sh + c * 8);
+        bf16x8 vw = *reinterpret_cast<const bf16x8*>(chunk_at(r, c));
+        bf16x8 vs = vw;
+        if (th.x + qoff >= p.all_below) vs = ld_global_b128(p.slc_o + tk * p.so_st + hd * p.so_sh + c * 8);
+        if (far) vw = ld_global_b128(p.o + tk * p.o_st + hd * p.o_sh + c * 8);
+        const float s0 = 1.f / (1.f + __expf(-(float)wp[0])), s1 = 1.f / (1.f + __expf(-(float)wp[1])),
+                    s2 = 1.f / (1.f + __expf(-(float)wp[2]));
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = (float)vc[e] * s0 + (float)vs[e] * s1 + (float)vw[e] * s2;
+        *reinterpret_cast<bf16x8*>(p.out + tk * p.out_st + hd * p.out_sh + c * 8) =
+            pack8(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
+      }
     }
   }
 }
@@ -390,7 +479,6 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 template <int D, int VD, int MODE, bool PAGED>
 int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
-  if (MODE == MODE_SWA && p.t_end > 0 && p.t_end < max_q_len) max_q_len = p.t_end;
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there;
   // the window branch, with its short key loops, and d=192, whose swizzled addresses cost registers, are faster with
   // register staging); 1..4 force one variant for experiments
@@ -402,6 +490,9 @@ int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t
     dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 1, false><<<grid, 256, 0, stream>>>(p);
     return nsa_check_launch("fwd_tile_kernel");
+  } else if constexpr (MODE == MODE_TAIL) {
+    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
+    fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, false><<<grid, 256, 0, stream>>>(p);
   } else if (variant == 2) {
     dim3 grid(cdiv_i(max_q_len * p.G, 256), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 2, 1, false><<<grid, 256, 0, stream>>>(p);
@@ -436,6 +527,10 @@ int nsa_fwd_tile_launch(const NsaFwdTileParams& p, int mode, bool paged, int B, 
   if (mode == MODE_CMP) {
     return paged ? dispatch_fwd_tile<MODE_CMP, true>(p, B, max_q_len, D, VD, stream)
                  : dispatch_fwd_tile<MODE_CMP, false>(p, B, max_q_len, D, VD, stream);
+  }
+  if (mode == MODE_TAIL) {
+    return paged ? dispatch_fwd_tile<MODE_TAIL, true>(p, B, max_q_len, D, VD, stream)
+                 : dispatch_fwd_tile<MODE_TAIL, false>(p, B, max_q_len, D, VD, stream);
   }
   return paged ? dispatch_fwd_tile<MODE_SWA, true>(p, B, max_q_len, D, VD, stream)
                : dispatch_fwd_tile<MODE_SWA, false>(p, B, max_q_len, D, VD, stream);

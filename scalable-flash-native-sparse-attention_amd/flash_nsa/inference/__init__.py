@@ -5,7 +5,8 @@ them; they write the newly completed compressed rows into the same pool (mean po
 never synchronise with the host, so the decode step can be captured in a HIP graph."""
 from .stages import (mean_pooling_prefill, kv_mean_pooling_decode, cmp_attn_prefill, cmp_attn_decode, topk_prefill,
                      topk_decode, slc_attn_prefill, fused_slc_swa_attn_decode, swa_prefill, combine_prefill,
-                     combine_decode, mean_pooling_decode, slc_attn_decode, fused_decode_supported, decode_cmp_topk,
+                     swa_combine_prefill, combine_decode, mean_pooling_decode, slc_attn_decode,
+                     fused_decode_supported, decode_cmp_topk,
                      decode_slc_swa_combine, decode_cmp_split, decode_one_launch, decode_one_launch_fits,
                      store_kvcache, store_kvcache_and_pool_prefill, decode_split, decode_split_fits)
 from .paging import PageTableBuilder, allocate_kv_pools
@@ -45,10 +46,11 @@ def nsa_prefill(q, k, v, w, x_cu_seqlens, y_cu_seqlens, x_maxlen, y_maxlen, cont
                         stride=stride, block_size=block_size, top_n=top_n, num_inital=num_init_blocks,
                         num_local=num_local_blocks, **full)
     slc_o, _ = slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables=block_tables,
-                                context_lens=context_lens, block_size=block_size, top_n=top_n, sm_scale=sm_scale, **full)
-    swa_o = swa_prefill(q, k, v, x_cu_seqlens, x_maxlen, block_tables=block_tables, context_lens=context_lens,
-                        window_size=window_size, sm_scale=sm_scale)
-    return combine_prefill(cmp_o, slc_o, swa_o, w)
+                                context_lens=context_lens, block_size=block_size, top_n=top_n, sm_scale=sm_scale,
+                                t_begin=full["all_below"], max_context=full["max_context"])
+    return swa_combine_prefill(q, k, v, cmp_o, slc_o, w, x_cu_seqlens, x_maxlen, block_tables=block_tables,
+                               context_lens=context_lens, window_size=window_size, all_below=full["all_below"],
+                               sm_scale=sm_scale)
 
 
 def auto_cmp_splits(batch, num_kv_heads, fixed_y_maxlen, num_cus=256, one_launch_fits=None, qk_dim=128):

@@ -163,10 +163,9 @@ def topk_decode(q, k, lse, block_tables, context_lens, fixed_y_maxlen=8192, fixe
 
 # ------------------------------------------------------------------------------------------------ selected / window
 def slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables, context_lens, block_size=64, top_n=16,
-                     sm_scale=None, all_below=0, max_context=0):
-    """-> (o [t,QH,VD], lse [t,QH]).  all_below: the queries at positions below it are known to select every block they
-    can see (all_below <= top_n * block_size) and their rows of topk are not read; max_context: a bound of the longest
-    context (0: unknown)."""
+                     sm_scale=None, t_begin=0, max_context=0):
+    """-> (o [t,QH,VD], lse [t,QH]).  t_begin: only the queries at positions from here on (the other rows stay unwritten:
+    swa_combine_prefill); max_context: a bound of the longest context (0: unknown)."""
     check_bf16(q)
     page, KH, D, ksr, ksh = _pool_args(k)
     _, _, VD, vsr, vsh = _pool_args(v)
@@ -176,12 +175,13 @@ def slc_attn_prefill(q, k, v, topk, x_cu_seqlens, x_maxlen, block_tables, contex
     assert topk.dtype == torch.int32 and topk.shape == (KH, t, top_n) and topk.stride(-1) == 1
     o = torch.empty(t, QH, VD, device=q.device, dtype=q.dtype)
     lse = torch.empty(t, QH, device=q.device, dtype=torch.float32)
-    _lib.call("nsa_paged_slc_attn_fwd_full", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(),
+    if 0 < max_context <= t_begin:
+        return o, lse
+    _lib.call("nsa_paged_slc_attn_fwd_from", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(),
               vsr, vsh, topk.data_ptr(), topk.stride(0), topk.stride(1), o.data_ptr(), o.stride(0), o.stride(1),
               lse.data_ptr(), lse.stride(0), lse.stride(1), _i32(x_cu_seqlens).data_ptr(),
               _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(), block_tables.stride(0), page, B,
-              int(x_maxlen), QH, KH, D, VD, block_size, top_n, all_below, int(max_context), sm_scale,
-              _lib.stream_ptr())
+              int(x_maxlen), QH, KH, D, VD, block_size, top_n, t_begin, sm_scale, _lib.stream_ptr())
     return o, lse
 
 
@@ -199,6 +199,27 @@ def swa_prefill(q, k, v, x_cu_seqlens, x_maxlen, block_tables, context_lens, win
               _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(), block_tables.stride(0), page, B,
               int(x_maxlen), QH, KH, D, VD, window_size, sm_scale, _lib.stream_ptr())
     return o
+
+
+def swa_combine_prefill(q, k, v, cmp_o, slc_o, w, x_cu_seqlens, x_maxlen, block_tables, context_lens, window_size=512,
+                        all_below=0, sm_scale=None):
+    """swa_prefill, the selected branch of the queries at positions below all_below (they select every block they can
+    see; slc_o holds that of the others) and combine_prefill in one launch -> o [t,QH,VD]."""
+    check_bf16(q), check_bf16(w)
+    page, KH, D, ksr, ksh = _pool_args(k)
+    _, _, VD, vsr, vsh = _pool_args(v)
+    t, QH, _ = q.shape
+    B = x_cu_seqlens.numel() - 1
+    sm_scale = q.size(-1) ** -0.5 if sm_scale is None else sm_scale
+    assert cmp_o.shape == slc_o.shape == (t, QH, VD) and w.shape == (t, QH, 3)
+    swa_o = torch.empty(t, QH, VD, device=q.device, dtype=q.dtype)  # scratch of the launch
+    out = torch.empty_like(swa_o)
+    st = lambda x: (x.data_ptr(), x.stride(0), x.stride(1))
+    _lib.call("nsa_paged_swa_fwd_tail", *st(q), k.data_ptr(), ksr, ksh, v.data_ptr(), vsr, vsh, *st(swa_o), None, 0, 0,
+              *st(slc_o), None, 0, 0, all_below, *st(cmp_o), *st(w), *st(out), 0, _i32(x_cu_seqlens).data_ptr(),
+              _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(), block_tables.stride(0), page, B,
+              int(x_maxlen), QH, KH, D, VD, window_size, sm_scale, _lib.stream_ptr())
+    return out
 
 
 def slc_attn_decode(q, k, v, topk, block_tables, context_lens, num_splits=0, block_size=64, top_n=16,

@@ -85,10 +85,8 @@ class HFNSACore(torch.nn.Module):
         cmp_k = run("cmp_k", lambda: self.compress_k(k))
         cmp_v = run("cmp_v", lambda: self.compress_v(v))
         cmp_o, cmp_lse = run("cmp_o", lambda: compress_attn(q, cmp_k, cmp_v, sm_scale=self.sm_scale))
-        topk, _ = run("top_k", lambda: slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=self.sm_scale,
-                                                             all_below=NSAHelper.all_below()))
-        slc_o = run("slc_o", lambda: select_attn(q, k, v, topk, sm_scale=self.sm_scale,
-                                                        all_below=NSAHelper.all_below()))
+        topk, _ = run("top_k", lambda: slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=self.sm_scale))
+        slc_o = run("slc_o", lambda: select_attn(q, k, v, topk, sm_scale=self.sm_scale))
         swa_o = run("swa_o", lambda: swa_varlen_func(q, k, v, self.sm_scale))
         out = run("combine", lambda: fused_sigmoid_combine(cmp_o, slc_o, swa_o, combine_weight))
         if not bench:

@@ -10,11 +10,11 @@ from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
 from ..ops.compress_kv import construct_block_fwd, construct_block_bwd, mean_pooling_fwd, mean_pooling_bwd
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
-from ..ops.select_attn import slc_attn_fwd, slc_attn_bwd
+from ..ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
-from ..ops.combine import combine_fwd, combine_bwd
-from ..ops.sliding_window_attention import swa_fwd, swa_bwd
+from ..ops.combine import combine_bwd
+from ..ops.sliding_window_attention import swa_fwd_tail, swa_bwd, swa_bwd_dq_tail
 
 
 # The backward runs on two streams: the memory-bound selected-block dq kernel leaves the matrix cores idle and the
@@ -87,6 +87,16 @@ def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHel
     return dx, (dw_fn if async_dw else dw_fn())
 
 
+def slc_swa_fwd(q, k, v, topk, sm_scale, helper, cmp_o=None, w=None, store=True):
+    """Selected and window branch, and, with the compressed branch's output and the gates, the gated sum: the gather of
+    the queries that have blocks to choose from, then the window kernel, which finishes the rest.
+    -> (slc_o, slc_lse), (swa_o, swa_lse), out; with store=False only out is defined."""
+    all_below = helper.all_below()
+    slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, helper=helper, t_begin=all_below)
+    swa_o, swa_lse, out = swa_fwd_tail(q, k, v, slc_o, slc_lse, all_below, cmp_o, w, store, sm_scale, helper)
+    return (slc_o, slc_lse), (swa_o, swa_lse), out
+
+
 class NSAFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, combine_weight, cmp_k_weight, cmp_v_weight, sm_scale=None):
@@ -97,9 +107,10 @@ class NSAFunction(torch.autograd.Function):
         win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method)
         cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
         topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=H.all_below())
-        slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, all_below=H.all_below())
-        swa_o, swa_lse = swa_fwd(q, k, v, sm_scale=sm_scale)
-        out = combine_fwd(cmp_o, slc_o, swa_o, combine_weight)
+        (slc_o, slc_lse), (swa_o, swa_lse), out = slc_swa_fwd(q, k, v, topk, sm_scale, H, cmp_o, combine_weight,
+                                                              store=ctx is not None)
+        if ctx is None:
+            return out
 
         keep = lambda flag, *ts: [None if flag else t for t in ts]
         saved = [q, k, v, combine_weight, cmp_k_weight, cmp_v_weight, topk]
@@ -126,44 +137,55 @@ class NSAFunction(torch.autograd.Function):
             win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, v_method, helper)
         if cmp_o is None:
             cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale, helper=helper)
-        if slc_o is None:
-            slc_o, slc_lse = slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale, helper=helper, all_below=helper.all_below())
-        if swa_o is None:
-            swa_o, swa_lse = swa_fwd(q, k, v, sm_scale=sm_scale, helper=helper)
+        if slc_o is None or swa_o is None:
+            (slc_o, slc_lse), (swa_o, swa_lse), _ = slc_swa_fwd(q, k, v, topk, sm_scale, helper)
 
-        # the combine backward also yields rowsum(branch * dbranch) of the three branches
-        dcmp_o, dslc_o, dswa_o, dw, delta = combine_bwd(cmp_o, slc_o, swa_o, combine_weight, do, return_delta=True)
+        # the combine backward also yields rowsum(branch * dbranch) of the three branches, and folds what the selected
+        # branch of the first all_below tokens of a sequence has in common with the window branch into the latter
+        all_below = helper.all_below()
+        dcmp_o, dslc_o, dswa_o, dw, delta = combine_bwd(cmp_o, slc_o, swa_o, combine_weight, do, return_delta=True,
+                                                        all_below=all_below, slc_lse=slc_lse, swa_lse=swa_lse,
+                                                        helper=helper)
         dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         kw = dict(sm_scale=sm_scale, helper=helper)
-        skw = dict(kw, all_below=helper.all_below())
+
+        def dq_chain():
+            # the selected branch (memory bound) stores, the window branch (matrix bound, with bandwidth to spare for
+            # the read-modify-write) adds, or stores where the selected branch left rows out, and the compressed branch
+            # adds and writes q's dtype
+            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq",
+                         t_begin=all_below, **kw)
+            swa_bwd_dq_tail(q, k, v, swa_lse, dswa_o, delta[2], slc_lse, dslc_o, delta[1], all_below, dq32, **kw)
+            return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
+                                parts="dq", **kw)[0]
+
+        def dkdv_raw():
+            # the window branch writes every element of dk / dv, the selected branch then adds to them
+            _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
+            slc_attn_bwd_dkdv_before_window(q, k, v, slc_lse, dslc_o, delta[1], dk, dv, all_below, **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv",
+                         t_begin=all_below, **kw)
+            return dk, dv
+
+        def dkdv_cmp():
+            return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, delta=delta[0], parts="dkdv", **kw)[1:]
+
         if OVERLAP_STREAMS:
             main, side = torch.cuda.current_stream(), _side_stream(q.device)
             side.wait_stream(main)
             with torch.cuda.stream(side):
-                # dq chain: the selected branch (memory bound) stores, the window branch (matrix bound, with
-                # bandwidth to spare for the read-modify-write) adds, the compressed branch adds and writes q's dtype
-                slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **skw)
-                swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dq=dq32, parts="dq", **kw)
-                dq, _, _ = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0],
-                                        finalize_dq=True, parts="dq", **kw)
+                dq = dq_chain()
                 dq.record_stream(main)
             # dk/dv kernels on the caller's stream.  The compressed branch (matrix bound) goes first, next to the
             # selected dq kernel (bound by the gather path) on the other stream: 0.7-1.7 ms per step less at T = 64K
             # (67.7 -> 67.0 and 67.2 -> 65.5 ms on two GPUs) than the order window, selected, compressed, which ran the
-            # two selected kernels side by side.  The
-            # window branch writes every element of dk / dv, the selected branch then adds to them.
-            _, dcmp_k, dcmp_v = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, delta=delta[0], parts="dkdv",
-                                             **kw)
-            _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **skw)
+            # two selected kernels side by side.
+            dcmp_k, dcmp_v = dkdv_cmp()
+            dk, dv = dkdv_raw()
         else:
-            # the selected branch stores dq, the window branch adds to it and writes every element of dk / dv, to
-            # which the selected branch then adds
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq", **skw)
-            _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dq=dq32, dkv_fp32=True, **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv", **skw)
-            dq, dcmp_k, dcmp_v = cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0],
-                                              finalize_dq=True, **kw)
+            dq = dq_chain()
+            dk, dv = dkdv_raw()
+            dcmp_k, dcmp_v = dkdv_cmp()
         _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
         _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
         if OVERLAP_STREAMS:
@@ -183,6 +205,8 @@ def _store_into(buf):
 
 
 def flash_nsa_varlen_func(q, k, v, combine_weight, cmp_k_weight=None, cmp_v_weight=None, sm_scale=None):
+    if not torch.is_grad_enabled():  # nothing is kept for a backward: the branch outputs need not be stored
+        return NSAFunction.forward(None, q, k, v, combine_weight, cmp_k_weight, cmp_v_weight, sm_scale)
     return NSAFunction.apply(q, k, v, combine_weight, cmp_k_weight, cmp_v_weight, sm_scale)
 
 

@@ -19,9 +19,13 @@ def combine_fwd(a, b, c, w):
     return o
 
 
-def combine_bwd(a, b, c, w, do, return_delta=False):
+def combine_bwd(a, b, c, w, do, return_delta=False, all_below=0, slc_lse=None, swa_lse=None, helper=None):
     """Returns da, db, dc (contiguous [T,H,D]), dw [T,H,3] and optionally delta [3,T,H] fp32 with
-    delta[k] = rowsum(branch_k * d branch_k), which the attention backward kernels consume."""
+    delta[k] = rowsum(branch_k * d branch_k), which the attention backward kernels consume.
+    all_below > 0 (b = selected, c = window branch, with their log-sum-exps [T,H] and the batch's helper; needs
+    return_delta): for the tokens at positions below it, which select every block they can see, dc and delta[2] also
+    carry the selected branch's gradient over the window's keys (swa_bwd_dq_tail, slc_attn_bwd_dkdv_before_window take
+    the rest)."""
     T, H, D = a.shape
     assert a.stride() == b.stride() == c.stride()
     do = do if do.stride(-1) == 1 else do.contiguous()
@@ -30,9 +34,16 @@ def combine_bwd(a, b, c, w, do, return_delta=False):
     dc = torch.empty_like(da)
     dw = torch.empty(T, H, 3, device=a.device, dtype=w.dtype)
     delta = torch.empty(3, T, H, device=a.device, dtype=torch.float32) if return_delta else None
-    _lib.call("nsa_combine_bwd", a.data_ptr(), b.data_ptr(), c.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(),
+    tail = ()
+    name = "nsa_combine_bwd"
+    if all_below > 0:
+        assert slc_lse.stride() == swa_lse.stride() and return_delta
+        name = "nsa_combine_bwd_tail"
+        tail = (slc_lse.data_ptr(), swa_lse.data_ptr(), slc_lse.stride(0), slc_lse.stride(1),
+                helper.x_cu_seqlens.data_ptr(), helper.batch, all_below)
+    _lib.call(name, a.data_ptr(), b.data_ptr(), c.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(),
               w.stride(0), w.stride(1), do.data_ptr(), do.stride(0), do.stride(1), da.data_ptr(), db.data_ptr(),
-              dc.data_ptr(), dw.data_ptr(), _lib.ptr(delta), T, H, D, _lib.stream_ptr())
+              dc.data_ptr(), dw.data_ptr(), _lib.ptr(delta), *tail, T, H, D, _lib.stream_ptr())
     if return_delta:
         return da, db, dc, dw, delta
     return da, db, dc, dw

@@ -4,7 +4,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
-from ._common import check_thd, default_scale, delta_of, dq_target, zeros_pair
+from ._common import check_bf16, check_thd, default_scale, delta_of, dq_target, zeros_pair
 
 
 def swa_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
@@ -20,6 +20,42 @@ def swa_fwd(q, k, v, sm_scale=None, helper=NSAHelper):
               lse.stride(0), lse.stride(1), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH, KH, D,
               VD, helper.window_size, sm_scale, _lib.stream_ptr())
     return o, lse
+
+
+def swa_fwd_tail(q, k, v, slc_o, slc_lse, all_below, cmp_o=None, w=None, store=True, sm_scale=None,
+                 helper=NSAHelper):
+    """swa_fwd, finishing the selected branch of the queries at positions below all_below (they select every block they
+    can see: the window branch continued over the keys before it) into slc_o / slc_lse and, with cmp_o and the gates w,
+    forming the gated sum of the three branches.  -> (o, lse, out or None); with store=False only `out` is defined."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (slc_o, "slc_o")):
+        check_thd(t, n)
+    T, QH, D = q.shape
+    _, KH, VD = v.shape
+    sm_scale = default_scale(q, sm_scale)
+    o = torch.empty(T, QH, VD, device=q.device, dtype=q.dtype)
+    lse = torch.empty(T, QH, device=q.device, dtype=torch.float32) if store else None
+    out = None
+    if cmp_o is not None:
+        check_thd(cmp_o, "cmp_o"), check_bf16(w)
+        assert cmp_o.shape == o.shape and w.shape == (T, QH, 3)
+        out = torch.empty_like(o)
+    st = lambda t: (None, 0, 0) if t is None else (t.data_ptr(), t.stride(0), t.stride(1))
+    _lib.call("nsa_swa_fwd_tail", *st(q), *st(k), *st(v), *st(o), *st(lse), *st(slc_o), *st(slc_lse), all_below,
+              *st(cmp_o), *st(w), *st(out), int(store), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen,
+              QH, KH, D, VD, helper.window_size, sm_scale, _lib.stream_ptr())
+    return o, lse, out
+
+
+def swa_bwd_dq_tail(q, k, v, lse, do, delta, slc_lse, slc_do, slc_delta, all_below, dq, sm_scale=None,
+                    helper=NSAHelper):
+    """dq of the window branch added into the fp32 buffer dq, for gradients from combine_bwd with all_below: the queries
+    at positions below it also take the selected branch's keys before their window, and their dq is stored."""
+    T, QH, D = q.shape
+    _, KH, VD = v.shape
+    st = lambda t: (t.data_ptr(), t.stride(0), t.stride(1))
+    _lib.call("nsa_swa_bwd_dq_tail", *st(q), *st(k), *st(v), *st(do), *st(lse), *st(delta), *st(slc_do), *st(slc_lse),
+              *st(slc_delta), all_below, *st(dq), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH,
+              KH, D, VD, helper.window_size, default_scale(q, sm_scale), _lib.stream_ptr())
 
 
 def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq=None, dkv_fp32=False, parts="both"):

@@ -519,39 +519,72 @@ def test_dk_dv_query_chunks(device, QH, KH, D, splits, monkeypatch):
     setup_helper(cu.to(device))
 
 
-@pytest.mark.parametrize("QH,KH,D,block_size", [(16, 1, 128, 64), (3, 1, 64, 32), (24, 1, 128, 96)])
+@pytest.mark.parametrize("QH,KH,D,VD,block_size,window", [
+    (16, 1, 128, 128, 64, 100), (3, 1, 64, 64, 32, 0), (24, 1, 128, 128, 96, 512), (8, 2, 192, 128, 64, 255)])
 @pytest.mark.parametrize("ordered", [False, True])
-def test_selected_attention_of_queries_that_select_everything(device, QH, KH, D, block_size, ordered):
-    """slc_attn_fwd / slc_attn_bwd with all_below (dense tiles for the queries that see at most top_n blocks, gather for
-    the rest) against the gather for all of them: sequences that end one before, at and one after the boundary, inside
-    the first tile and far past it.  The two round P to bf16 against another running maximum, so each side's sum of
-    p v is off by at most 2^-9 of the sum of p |v| (below 1 for these N(0,1) values wherever more than one p counts,
-    and exact where one does), and an output by that twice plus its own rounding: 2^-8 + 2^-7 |o|.  The gradients are
-    taken from the same lse and outputs, so P is the same to fp32 rounding; its and dS's bf16 rounding may flip, by
-    2^-8 of a term in sums of many: 2^-7 of the row's rms and 2e-3."""
+def test_selected_attention_of_queries_that_select_everything(device, QH, KH, D, VD, block_size, window, ordered):
+    """The selected branch of the queries that see at most top_n blocks, finished by the window kernels (forward with and
+    without stored branches, dq, and what their keys before the window add to dk / dv), against the gather for all of
+    them: windows shorter and longer than top_n blocks, sequences that end one before, at and one after the boundary,
+    inside the first tile and far past it.  The two round P to bf16 against another running maximum, so each side's
+    sum of p v is off by at most 2^-9 of the sum of p |v| (below 1 for these N(0,1) values wherever more than one p
+    counts, and exact where one does), and an output by that twice plus its own rounding: 2^-8 + 2^-7 |o|.  In the
+    backward the two branches' gradients of a window key are summed before they are rounded to bf16 instead of after:
+    dP is then off by 2^-9 of the sum of |dO v| over the channels at most and 2^-9 sqrt(channels) typically (0.02),
+    which dq takes times the softmax scale and |k| (0.09 x 1 to 3 at 128 channels), on either side: the bar of 2e-2
+    plus 1e-2 of the row's rms covers it."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.combine import combine_fwd, combine_bwd
     from flash_nsa.ops.compress_attn import cmp_attn_fwd
     from flash_nsa.ops.compress_kv import mean_pooling_fwd
-    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
+    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window
+    from flash_nsa.ops.sliding_window_attention import swa_fwd, swa_bwd, swa_fwd_tail, swa_bwd_dq_tail
     from flash_nsa.ops.topk import slc_topk_indices
     n = 4 * block_size
     cu = make_cu([n - 1, n, 0, n + 1, 1, 5 * n + 7, 33])
     T = int(cu[-1])
-    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, seed=150)]
-    do = randn_bf16(T, QH, D, seed=154).to(device)
-    setup_helper(cu.to(device), block_size=block_size, top_n=4)
-    _, lse_c = cmp_attn_fwd(q, mean_pooling_fwd(k), mean_pooling_fwd(v))
-    full, _ = slc_topk_indices(q, mean_pooling_fwd(k), lse_c)
-    part = torch.full_like(full, -7)
-    topk, _ = slc_topk_indices(q, mean_pooling_fwd(k), lse_c, all_below=n)
+    q, k, v, w = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=150)]
+    do = randn_bf16(T, QH, VD, seed=154).to(device)
+    H = setup_helper(cu.to(device), block_size=block_size, top_n=4, window_size=window)
+    ck = mean_pooling_fwd(k)
+    cmp_o, lse_c = cmp_attn_fwd(q, ck, mean_pooling_fwd(v))
+    full, _ = slc_topk_indices(q, ck, lse_c)
+    topk, _ = slc_topk_indices(q, ck, lse_c, all_below=n)
     pos = torch.cat([torch.arange(b - a) for a, b in zip(cu[:-1].tolist(), cu[1:].tolist())]).to(device)
+    part = torch.full_like(full, -7)            # rows below the boundary are invalid and must not be read
     part[:, pos >= n] = topk[:, pos >= n]
     assert torch.equal(part[:, pos >= n], full[:, pos >= n])
-    ref = slc_attn_fwd(q, k, v, full)
-    out = slc_attn_fwd(q, k, v, part, all_below=n)   # rows of part below the boundary are invalid and must not be read
-    assert_close(out[0], ref[0].float(), "o", atol=2 ** -8, rtol=2 ** -7)
-    assert_close(out[1], ref[1], "lse", atol=1e-5, rtol=1e-5)
-    g_ref = slc_attn_bwd(q, k, v, full, *ref, do, dkdv_repeat=ordered)
-    g_out = slc_attn_bwd(q, k, v, part, *ref, do, dkdv_repeat=ordered, all_below=n)
-    for name, a, b in zip(("dq", "dk", "dv"), g_out, g_ref):
-        assert_close(a, b.float(), name, atol=2e-3, rtol=2 ** -7, row_scale=True)
+    so, sl = slc_attn_fwd(q, k, v, full)
+    wo, wl = swa_fwd(q, k, v)
+    ref = combine_fwd(cmp_o, so, wo, w)
+    for store in (True, False):
+        so2, sl2 = slc_attn_fwd(q, k, v, part, t_begin=n)
+        wo2, wl2, out = swa_fwd_tail(q, k, v, so2, sl2, n, cmp_o, w, store)
+        assert_close(out, ref.float(), "out", atol=2 ** -8, rtol=2 ** -7)
+    so2, sl2 = slc_attn_fwd(q, k, v, part, t_begin=n)
+    wo2, wl2, out = swa_fwd_tail(q, k, v, so2, sl2, n)
+    assert out is None and torch.equal(wo, wo2) and torch.equal(wl, wl2)
+    assert_close(so2, so.float(), "slc o", atol=2 ** -8, rtol=2 ** -7)
+    assert_close(sl2, sl, "slc lse", atol=1e-5, rtol=1e-5)
+    try:
+        NSAHelper.set_deterministic(ordered)
+        _, ds, dsw, dw, delta = combine_bwd(cmp_o, so2, wo2, w, do, return_delta=True)
+        dq = torch.zeros(T, QH, D, device=device)
+        slc_attn_bwd(q, k, v, full, so2, sl2, ds, dq, delta=delta[1], parts="dq")
+        swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dq=dq, parts="dq")
+        _, dk, dv = swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dkv_fp32=True, parts="dkdv")
+        slc_attn_bwd(q, k, v, full, so2, sl2, ds, None, dk, dv, delta=delta[1], parts="dkdv")
+        _, ds, dsw, dw2, delta = combine_bwd(cmp_o, so2, wo2, w, do, True, n, sl2, wl2, H)
+        assert torch.equal(dw, dw2)
+        dq2 = torch.full((T, QH, D), float("nan"), device=device)
+        dq2[pos >= n] = 0
+        slc_attn_bwd(q, k, v, part, so2, sl2, ds, dq2, delta=delta[1], parts="dq", t_begin=n)
+        swa_bwd_dq_tail(q, k, v, wl2, dsw, delta[2], sl2, ds, delta[1], n, dq2)
+        _, dk2, dv2 = swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dkv_fp32=True, parts="dkdv")
+        slc_attn_bwd_dkdv_before_window(q, k, v, sl2, ds, delta[1], dk2, dv2, n)
+        slc_attn_bwd(q, k, v, part, so2, sl2, ds, None, dk2, dv2, delta=delta[1], parts="dkdv", t_begin=n)
+    finally:
+        NSAHelper.set_deterministic(False)
+    for name, a, b in (("dq", dq2, dq), ("dk", dk2, dk), ("dv", dv2, dv)):
+        assert_close(a, b, name, row_scale=True)
     setup_helper(cu.to(device))
