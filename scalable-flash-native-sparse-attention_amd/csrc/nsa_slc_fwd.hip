@@ -3,31 +3,42 @@
 // Upstream: flash_nsa/ops/select_attn.py:21-108 (training), flash_nsa/inference/select_attn.py:21-100 (paged).
 //
 // The keys of the selected blocks are processed in units of 32.  The K and V rows of a unit are fetched as whole
-// coalesced rows (16 lanes x 16 bytes per row) into registers one unit ahead, pass through wave-private LDS
-// regions, and are read back as MFMA fragments (K row-major, V through ds_read_b64_tr_b16, which delivers the
+// coalesced rows (16 lanes x 16 bytes per row) into registers one unit ahead, pass through a wave-private LDS
+// region, and are read back as MFMA fragments (K row-major, V through ds_read_b64_tr_b16, which delivers the
 // key-contraction slices).  Keys are gathered by the per-token block list topk[kh, t, 0 .. min(top_n, t/block+1)).
+//
+// What bounds it is the gather: 512 KB of rows per token and kv head, from L2 while the keys of the sequences in flight
+// fit there, else from the memory-side cache (13.5 TB/s of requests at 64K tokens).  Two units in flight per wave and
+// separate K and V regions bought nothing over one, and took the registers and the LDS of a second workgroup per CU at
+// 192 channels: 32 heads, 16K tokens 1726 -> 1080 us; 64 heads of 128, 8 x 6K tokens 4207 -> 3920 us.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
 
 namespace {
 
+// waves per SIMD the register budget is cut for; at 256 channels two waves with 30 spilled registers beat one without
+// (1039 against 1165 us for 16 heads, 16K tokens)
+constexpr int slc_waves(int d) { return d <= 64 ? 4 : d <= 128 ? 3 : 2; }
+
 template <int D, int VD, bool PAGED>
-__global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
-  // Work unit = 32 keys (half of a 64-key tile).  The K fragments and the V rows of unit u+1 are loaded into
-  // registers while unit u is computed, so the gather latency overlaps the MFMAs of the previous unit.
-  constexpr int VLD = VD + NSA_LDS_PAD;
+__global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams p) {
+  // Work unit = 32 keys (half of a 64-key tile).  One set of registers holds the rows of the next unit: its K rows are
+  // requested when this unit's have gone to LDS, its V rows when this unit's have, which is when the scores are known
+  // and the K rows in LDS are no longer needed: K and V take turns in one LDS region.
   constexpr int UK = 32;                      // keys per unit
   constexpr int KC = D / 32;                  // K fragments per 16-key tile
   constexpr int VJ = (UK * (VD / 8)) / 64;    // 16-byte V loads per lane and unit
   constexpr int KJ = (UK * (D / 8)) / 64;     // 16-byte K loads per lane and unit
-  constexpr int KLD = D + NSA_LDS_PAD;
-  __shared__ __attribute__((aligned(16))) bf16_t Vs_all[4 * UK * VLD];
-  __shared__ __attribute__((aligned(16))) bf16_t Ks_all[4 * UK * KLD];
+  constexpr int KLD = D + NSA_LDS_PAD, VLD = VD + NSA_LDS_PAD;
+  constexpr int LD = KLD > VLD ? KLD : VLD;
+  constexpr int KP = D / 8, VP = VD / 8;                                             // 16-byte pieces per row
+  constexpr int KPAT = 64 % KP == 0 ? 1 : 3, VPAT = 64 % VP == 0 ? 1 : 3;            // 192 channels: 3 * 64 = 8 * 24
+  static_assert((KPAT * 64) % KP == 0 && (VPAT * 64) % VP == 0, "");
+  __shared__ __attribute__((aligned(16))) bf16_t rows_all[4 * UK * LD];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  bf16_t* Vs = Vs_all + wave * UK * VLD;
-  bf16_t* Ks = Ks_all + wave * UK * KLD;
+  bf16_t* const rows = rows_all + wave * UK * LD;
   const int l16 = lane & 15;
   const int kq = lane >> 4;
   const int b = blockIdx.y;
@@ -62,6 +73,7 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
   }
   int my_blk = 0;
   if (lane < nvalid) my_blk = p.topk[(int64_t)kh * p.tk_sh + tok * p.tk_st + lane];
+  my_blk = sort_blocks(my_blk, nvalid, lane);
 
   f32x4 oacc[VD / 16];
 #pragma unroll
@@ -69,77 +81,96 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
   float m_run = NSA_NEG_INF, l_run = 0.f;
   const float sc = p.scale_log2;
 
-  // first key of unit u; wave-uniform.  Units that start past the last attendable key (second half of the current
-  // block) and ignore values (negative ids) are reported as -1 and skipped.
-  auto unit_key0 = [&](int u) {
-    int slot = u / upb;
-    int blk = __builtin_amdgcn_readlane(my_blk, slot);
-    int key0 = blk * Bs + (u - slot * upb) * UK;
-    return (blk < 0 || key0 > key_last) ? -1 : key0;
+  // first key of the next unit with something to attend, at or behind unit u, -1: none left; wave-uniform.  Units that
+  // start past the last attendable key (second half of the current block) and ignore values (negative ids) are skipped.
+  auto next_unit = [&](int& u) {
+    for (; u < nu; u++) {
+      const int slot = u / upb;
+      const int blk = __builtin_amdgcn_readlane(my_blk, slot);
+      const int key0 = blk * Bs + (u - slot * upb) * UK;
+      if (blk >= 0 && key0 <= key_last) {
+        u++;
+        return key0;
+      }
+    }
+    return -1;
   };
-  // per-lane element offsets inside a unit are the same for every unit: the loads are (uniform base) + offset
   // K and V rows are fetched as whole 16-byte-per-lane coalesced rows (every cache line is requested once and used
-  // completely) and go through wave-private LDS; the MFMA fragments are read from there
-  int64_t koff[KJ], voff[VJ];
+  // completely) and go through wave-private LDS; the MFMA fragments are read from there.
+  // A unit's rows are fetched 64 pieces of 16 bytes at a time; after KPAT (VPAT) instructions the pieces fall on the same
+  // columns again, so the lane part of the addresses is KPAT + VPAT 32-bit offsets and the rest is wave-uniform.
+  uint32_t koff[KPAT], voff[VPAT];
 #pragma unroll
-  for (int j = 0; j < KJ; j++) {
+  for (int j = 0; j < KPAT; j++) {
     int pc = lane + j * 64;
-    koff[j] = (int64_t)(pc / (D / 8)) * p.k_sr + (pc % (D / 8)) * 8;
+    koff[j] = (uint32_t)(pc / KP) * (uint32_t)(p.k_sr * 2) + (pc % KP) * 16;
   }
 #pragma unroll
-  for (int j = 0; j < VJ; j++) {
+  for (int j = 0; j < VPAT; j++) {
     int pc = lane + j * 64;
-    voff[j] = (int64_t)(pc / (VD / 8)) * p.v_sr + (pc % (VD / 8)) * 8;
+    voff[j] = (uint32_t)(pc / VP) * (uint32_t)(p.v_sr * 2) + (pc % VP) * 16;
   }
-  auto issue = [&](int key0, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ]) {
-    if (key0 < 0) return;
-    int64_t row0;  // flat row of the unit's first key (a unit never straddles a page)
-    if (PAGED) row0 = (int64_t)__builtin_amdgcn_readfirstlane(table[key0 / p.page_size]) * p.page_size + (key0 % p.page_size);
-    else row0 = (int64_t)x0 + key0;
-    const bf16_t* kb = p.k + row0 * p.k_sr + (int64_t)kh * p.k_sh;
-    const bf16_t* vb = p.v + row0 * p.v_sr + (int64_t)kh * p.v_sh;
+  bf16x8 kr[KJ], vr[VJ];
+  auto flat_row = [&](int key0) -> int64_t {  // flat row of the unit's first key (a unit never straddles a page)
+    if (PAGED) return (int64_t)__builtin_amdgcn_readfirstlane(table[key0 / p.page_size]) * p.page_size + (key0 % p.page_size);
+    return (int64_t)x0 + key0;
+  };
+  // the unit holding the causal boundary: rows past it are replaced by the boundary row (masked later)
+  auto issue_k = [&](int key0) {
+    const bf16_t* kb = p.k + flat_row(key0) * p.k_sr + (int64_t)kh * p.k_sh;
     const int kmax = key_last - key0;  // >= 0
     if (kmax >= UK - 1) {
 #pragma unroll
-      for (int j = 0; j < KJ; j++) kf[j] = ld_global_b128(kb + koff[j]);
-#pragma unroll
-      for (int j = 0; j < VJ; j++) vr[j] = ld_global_b128(vb + voff[j]);
-    } else {  // the unit holding the causal boundary: rows past it are replaced by the boundary row (masked later)
+      for (int j = 0; j < KJ; j++)
+        kr[j] = ld_global_b128((const bf16_t*)((const char*)(kb + (j / KPAT) * (KPAT * 64 / KP) * p.k_sr) + koff[j % KPAT]));
+    } else {
 #pragma unroll
       for (int j = 0; j < KJ; j++) {
         int pc = lane + j * 64;
-        kf[j] = ld_global_b128(kb + (int64_t)min(pc / (D / 8), kmax) * p.k_sr + (pc % (D / 8)) * 8);
-      }
-#pragma unroll
-      for (int j = 0; j < VJ; j++) {
-        int pc = lane + j * 64;
-        vr[j] = ld_global_b128(vb + (int64_t)min(pc / (VD / 8), kmax) * p.v_sr + (pc % (VD / 8)) * 8);
+        kr[j] = ld_global_b128(kb + (int64_t)min(pc / KP, kmax) * p.k_sr + (pc % KP) * 8);
       }
     }
   };
-  auto compute = [&](int key0, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ]) {
-    if (key0 < 0) return;
+  auto issue_v = [&](int key0) {
+    const bf16_t* vb = p.v + flat_row(key0) * p.v_sr + (int64_t)kh * p.v_sh;
+    const int kmax = key_last - key0;  // >= 0
+    if (kmax >= UK - 1) {
 #pragma unroll
-    for (int j = 0; j < KJ; j++) {
-      int pc = lane + j * 64;
-      *reinterpret_cast<bf16x8*>(&Ks[(pc / (D / 8)) * KLD + (pc % (D / 8)) * 8]) = kf[j];
+      for (int j = 0; j < VJ; j++)
+        vr[j] = ld_global_b128((const bf16_t*)((const char*)(vb + (j / VPAT) * (VPAT * 64 / VP) * p.v_sr) + voff[j % VPAT]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < VJ; j++) {
+        int pc = lane + j * 64;
+        vr[j] = ld_global_b128(vb + (int64_t)min(pc / VP, kmax) * p.v_sr + (pc % VP) * 8);
+      }
     }
+  };
+  auto lds_order = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  int u = 0;
+  int key0 = next_unit(u);
+  if (key0 >= 0) { issue_k(key0); issue_v(key0); }
+  while (key0 >= 0) {
+    const int key_next = next_unit(u);
+#pragma unroll
+    for (int j = 0; j < KJ; j++) {
+      int pc = lane + j * 64;
+      *reinterpret_cast<bf16x8*>(&rows[(pc / KP) * KLD + (pc % KP) * 8]) = kr[j];
+    }
+    lds_order();
+    if (key_next >= 0) issue_k(key_next);
     f32x4 sacc[2];
 #pragma unroll
     for (int jt = 0; jt < 2; jt++) {
       sacc[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const bf16_t* kp = &Ks[(jt * 16 + l16) * KLD + kq * 8];
+      const bf16_t* kp = &rows[(jt * 16 + l16) * KLD + kq * 8];
 #pragma unroll
       for (int kc = 0; kc < KC; kc++) sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(kp + kc * 32), qf[kc], sacc[jt]);
-    }
-    // V rows -> wave-private LDS (previous unit's transpose reads are complete: LDS ops of a wave are in order)
-#pragma unroll
-    for (int j = 0; j < VJ; j++) {
-      int pc = lane + j * 64;
-      *reinterpret_cast<bf16x8*>(&Vs[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
     }
     const int kmax = key_last - key0;  // last usable key offset inside this unit
     if (kmax < UK - 1) {               // wave-uniform: only the unit holding the causal boundary is masked
@@ -176,9 +207,14 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
       for (int dt = 0; dt < VD / 16; dt++) oacc[dt] *= alpha;
     }
     l_run += psum;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    lds_order();
+#pragma unroll
+    for (int j = 0; j < VJ; j++) {
+      int pc = lane + j * 64;
+      *reinterpret_cast<bf16x8*>(&rows[(pc / VP) * VLD + (pc % VP) * 8]) = vr[j];
+    }
+    lds_order();
+    if (key_next >= 0) issue_v(key_next);
     // O^T += V^T P^T over the 32 keys of the unit
     bf16x8 pf = pack8(sacc[0][0], sacc[0][1], sacc[0][2], sacc[0][3], sacc[1][0], sacc[1][1], sacc[1][2], sacc[1][3]);
     const int kb0 = kq * 4 + (l16 >> 2);
@@ -186,24 +222,12 @@ __global__ __launch_bounds__(256, 2) void slc_fwd_kernel(NsaSlcParams p) {
 #pragma unroll
     for (int dt = 0; dt < VD / 16; dt++) {
       const int col = dt * 16 + 4 * (l16 & 3);
-      bf16x4 v0 = lds_read_tr(&Vs[kb0 * VLD + col]);
-      bf16x4 v1 = lds_read_tr(&Vs[kb1 * VLD + col]);
+      bf16x4 v0 = lds_read_tr(&rows[kb0 * VLD + col]);
+      bf16x4 v1 = lds_read_tr(&rows[kb1 * VLD + col]);
       oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  bf16x8 kfA[KJ], kfB[KJ], vrA[VJ], vrB[VJ];
-  int keyA = 0, keyB = 0;
-  if (nu > 0) { keyA = unit_key0(0); issue(keyA, kfA, vrA); }
-  for (int u = 0; u < nu; u += 2) {
-    if (u + 1 < nu) { keyB = unit_key0(u + 1); issue(keyB, kfB, vrB); }
-    compute(keyA, kfA, vrA);
-    if (u + 1 < nu) {
-      if (u + 2 < nu) { keyA = unit_key0(u + 2); issue(keyA, kfA, vrA); }
-      compute(keyB, kfB, vrB);
-    }
+    lds_order();
+    key0 = key_next;
   }
 
   float l_tot = xrow_sum(l_run);
