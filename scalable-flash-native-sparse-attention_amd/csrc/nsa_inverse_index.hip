@@ -2,6 +2,10 @@
 // selected the block, as a CSR (offsets + token ids), plus the prefix of fixed-size list chunks that the dK/dV
 // kernel uses as its work items.  Built by a deterministic counting sort: per-token-chunk histograms,
 // a scan over chunks and blocks, then an in-order fill, so no sort and no dense (block x token) scratch.
+// All three are bound by round trips to memory and LDS, not by bytes, and stand on the critical path in front of the
+// selected dK/dV kernel.  us for count + scan + fill, with one search per entry, a scan and a fill that wait for every
+// element -> as below: one sequence of 4K tokens, 1 kv head 79 -> 24, 40 of up to 1.2K, 2 kv heads 101 -> 31, 8 x 6K,
+// 4 kv heads 149 -> 58, 64K 171 -> 82.
 // Upstream: flash_nsa/ops/topk.py:782-945 (get_bind_from_find, dense scatter + per-row sort).
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
@@ -22,31 +26,58 @@ __device__ __forceinline__ int find_seq(const int32_t* x_cu, int B, int tok) {
   return lo;
 }
 
+// One thread per query token: where its sequence's blocks begin, how many there are and how many slots of its selection
+// count.  (One search per token; one per entry was most of the counting kernel.)
+struct TokenRow {
+  const int32_t* slots;
+  int n, kb, nb, nvalid;
+};
+__device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+                                              const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok, int t1, int kh,
+                                              int block_size, int t_begin) {
+  TokenRow r{topk, 0, 0, 0, 0};
+  if (tok >= t1) return r;
+  const int b = find_seq(x_cu, B, tok);
+  r.slots = topk + (int64_t)kh * tk_sh + (int64_t)tok * tk_st;
+  r.n = tok - x_cu[b];
+  r.kb = kblk_cu[b];
+  r.nb = kblk_cu[b + 1] - r.kb;
+  r.nvalid = r.n >= t_begin ? min(top_n, r.n / block_size + 1) : 0;
+  return r;
+}
+// fn(global block) for every block that the token selected; the ids are fetched ROW at a time, so that they share one
+// round trip to memory
+constexpr int ROW = 16;
+template <class Fn>
+__device__ __forceinline__ void for_each_block(const TokenRow& r, Fn fn) {
+  for (int s0 = 0; s0 < r.nvalid; s0 += ROW) {
+    int j[ROW];
+#pragma unroll
+    for (int s = 0; s < ROW; s++) j[s] = s0 + s < r.nvalid ? r.slots[s0 + s] : -1;
+#pragma unroll
+    for (int s = 0; s < ROW; s++)
+      if (j[s] >= 0 && j[s] < r.nb) fn(r.kb + j[s]);
+  }
+}
+
 // grid (nchunks, KH), 256 threads, dynamic LDS nblk ints
-__global__ void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
-                                 const int32_t* kblk_cu, int B, int T, int nblk, int block_size, int t_begin,
-                                 int32_t* chunk_cnt) {
+__global__ __launch_bounds__(256) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+                                                        const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
+                                                        int nblk, int block_size, int t_begin, int32_t* chunk_cnt) {
   extern __shared__ int hist[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x) hist[i] = 0;
+  for (int i = threadIdx.x; i < nblk; i += 256) hist[i] = 0;
   __syncthreads();
   const int CT = counting_chunk(T);
   const int t0 = chunk * CT;
   const int t1 = min(T, t0 + CT);
-  for (int idx = threadIdx.x; idx < (t1 - t0) * top_n; idx += blockDim.x) {
-    int tok = t0 + idx / top_n;
-    int s = idx % top_n;
-    int b = find_seq(x_cu, B, tok);
-    int n = tok - x_cu[b];
-    if (n >= t_begin && s < min(top_n, n / block_size + 1)) {
-      int j = topk[(int64_t)kh * tk_sh + (int64_t)tok * tk_st + s];
-      int nb = kblk_cu[b + 1] - kblk_cu[b];
-      if (j >= 0 && j < nb) atomicAdd(&hist[kblk_cu[b] + j], 1);
-    }
+  for (int tb = t0; tb < t1; tb += 256) {
+    const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + threadIdx.x, t1, kh, block_size, t_begin);
+    for_each_block(r, [&](int jb) { atomicAdd(&hist[jb], 1); });
   }
   __syncthreads();
   int32_t* dst = chunk_cnt + ((int64_t)kh * gridDim.x + chunk) * nblk;
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x) dst[i] = hist[i];
+  for (int i = threadIdx.x; i < nblk; i += 256) dst[i] = hist[i];
 }
 
 // grid (KH), 1024 threads: chunk counts -> chunk bases (in place), list offsets, work-item offsets
@@ -61,11 +92,18 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
   const int j0 = tid * per, j1 = min(nblk, j0 + per);
   int sum_a = 0, sum_b = 0;
   for (int j = j0; j < j1; j++) {
+    // counts are read SCAN at a time: reading and replacing them one by one is a chain of round trips to memory
+    constexpr int SCAN = 16;
     int base = 0;
-    for (int c = 0; c < nchunks; c++) {
-      int v = cnt[(int64_t)c * nblk + j];
-      cnt[(int64_t)c * nblk + j] = base;
-      base += v;
+    for (int c0 = 0; c0 < nchunks; c0 += SCAN) {
+      int v[SCAN];
+#pragma unroll
+      for (int u = 0; u < SCAN; u++) v[u] = c0 + u < nchunks ? cnt[(int64_t)(c0 + u) * nblk + j] : 0;
+#pragma unroll
+      for (int u = 0; u < SCAN; u++) {
+        if (c0 + u < nchunks) cnt[(int64_t)(c0 + u) * nblk + j] = base;
+        base += v[u];
+      }
     }
     // totals are parked in the output arrays and replaced by their prefixes below
     csr_off[(int64_t)kh * (nblk + 1) + j] = base;
@@ -99,62 +137,61 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
   }
 }
 
-// grid (nchunks, KH), 64 threads: in-order fill
-__global__ __launch_bounds__(64) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
-                                                      const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
-                                                      int nblk, int block_size, int t_begin, const int32_t* chunk_base,
-                                                      const int32_t* csr_off, int32_t* csr_tok) {
-  extern __shared__ int cursor[];
+// grid (nchunks, KH), 256 threads: in-order fill.  The position of a token in a block's list is the number of earlier
+// tokens that selected the block.  256 tokens at a time set their bit in the block's 256-bit mask, so the count is that
+// of the bits below the token's own and no token waits for another (a wave that walked the tokens one by one took as
+// long as 256 dependent LDS updates, whatever the size of the batch).  LDS holds the masks of FILL_BLOCKS blocks; more
+// blocks than that are taken in several rounds.
+constexpr int FILL_BLOCKS = 1024, FILL_WORDS = 256 / 32;
+__global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+                                                       const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
+                                                       int nblk, int block_size, int t_begin, const int32_t* chunk_base,
+                                                       const int32_t* csr_off, int32_t* csr_tok) {
+  __shared__ int cursor[FILL_BLOCKS];
+  __shared__ __attribute__((aligned(16))) uint32_t mask[FILL_BLOCKS * FILL_WORDS];
   const int chunk = blockIdx.x, kh = blockIdx.y;
-  const int lane = threadIdx.x;
-  const int32_t* base = chunk_base + ((int64_t)kh * gridDim.x + chunk) * nblk;
-  for (int i = lane; i < nblk; i += 64) cursor[i] = base[i] + csr_off[(int64_t)kh * (nblk + 1) + i];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int tid = threadIdx.x;
   const int CT = counting_chunk(T);
   const int t0 = chunk * CT;
   const int t1 = min(T, t0 + CT);
   if (t0 >= t1) return;
-  // The list positions depend on the order of the tokens, so the wave walks them one by one; the selection rows
-  // do not, and are fetched a batch ahead so that the walk never waits for memory.
-  constexpr int PF = 16;
-  int b = find_seq(x_cu, B, t0);
-  int x_begin = x_cu[b], x_end = x_cu[b + 1], kb_begin = kblk_cu[b], nb = kblk_cu[b + 1] - kb_begin;
-  const int32_t* row0 = topk + (int64_t)kh * tk_sh;
-  int nxt[PF], cur[PF];
-  auto fetch = [&](int tb) {
+  const int32_t* base = chunk_base + ((int64_t)kh * gridDim.x + chunk) * nblk;
+  const int32_t* off = csr_off + (int64_t)kh * (nblk + 1);
+  // the blocks of this chunk's sequences
+  const int b0 = find_seq(x_cu, B, t0), b1 = find_seq(x_cu, B, t1 - 1);
+  const int blk_lo = kblk_cu[b0];
+  const int blk_hi = kblk_cu[b1 + 1];
+  const int word = tid >> 5;
+  const uint32_t bit = 1u << (tid & 31);
+  for (int r0 = blk_lo; r0 < blk_hi; r0 += FILL_BLOCKS) {
+    const int nr = min(FILL_BLOCKS, blk_hi - r0);
+    for (int i = tid; i < nr; i += 256) cursor[i] = base[r0 + i] + off[r0 + i];
+    for (int tb = t0; tb < t1; tb += 256) {
+      for (int i = tid; i < nr * FILL_WORDS; i += 256) mask[i] = 0;
+      __syncthreads();
+      const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + tid, t1, kh, block_size, t_begin);
+      for_each_block(r, [&](int jb) {
+        if ((unsigned)(jb - r0) < (unsigned)nr) atomicOr(&mask[(jb - r0) * FILL_WORDS + word], bit);
+      });
+      __syncthreads();
+      for_each_block(r, [&](int jb) {
+        if ((unsigned)(jb - r0) >= (unsigned)nr) return;
+        const uint32_t* m = &mask[(jb - r0) * FILL_WORDS];
+        int pos = cursor[jb - r0];
 #pragma unroll
-    for (int u = 0; u < PF; u++)
-      nxt[u] = (tb + u < t1 && lane < top_n) ? row0[(int64_t)(tb + u) * tk_st + lane] : -1;
-  };
-  fetch(t0);
-  for (int tb = t0; tb < t1; tb += PF) {
+        for (int w = 0; w < FILL_WORDS; w++) pos += __popc(w < word ? m[w] : w == word ? m[w] & (bit - 1) : 0u);
+        csr_tok[pos] = r.n;
+      });
+      __syncthreads();
+      if (tb + 256 < t1) {
+        for (int i = tid; i < nr; i += 256) {
+          int add = 0;
 #pragma unroll
-    for (int u = 0; u < PF; u++) cur[u] = nxt[u];
-    if (tb + PF < t1) fetch(tb + PF);
-#pragma unroll
-    for (int u = 0; u < PF; u++) {
-      const int tok = tb + u;
-      if (tok >= t1) break;
-      if (tok >= x_end) {  // next (non-empty) sequence: the only loads inside the walk
-        do { b++; } while (tok >= x_cu[b + 1]);
-        x_begin = x_cu[b], x_end = x_cu[b + 1], kb_begin = kblk_cu[b], nb = kblk_cu[b + 1] - kb_begin;
-      }
-      const int n = tok - x_begin;
-      const int nvalid = n >= t_begin ? min(top_n, n / block_size + 1) : 0;
-      if (lane < nvalid) {
-        const int j = cur[u];
-        if (j >= 0 && j < nb) {
-          const int jb = kb_begin + j;
-          const int pos = cursor[jb];
-          cursor[jb] = pos + 1;
-          csr_tok[pos] = n;
+          for (int w = 0; w < FILL_WORDS; w++) add += __popc(mask[i * FILL_WORDS + w]);
+          cursor[i] += add;
         }
+        __syncthreads();
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   }
 }
@@ -203,7 +240,7 @@ int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_
                                       item_off);
   rc = nsa_check_launch("csr_scan_kernel");
   if (rc) return rc;
-  csr_fill_kernel<<<grid, 64, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
+  csr_fill_kernel<<<grid, 256, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
                                         t_begin, workspace, csr_off, csr_tok);
   return nsa_check_launch("csr_fill_kernel");
 }

@@ -133,6 +133,39 @@ def test_slc_attn_bwd(device, lens, QH, KH, D):
     setup_helper(cu.to(device))
 
 
+@pytest.mark.parametrize("lens,t_begin", [([1, 255, 256, 257, 64, 700], 0), ([70000], 1024), ([130000, 3, 9000], 100)],
+                         ids=["short", "two_rounds_of_blocks", "long_counting_chunks"])
+def test_inverse_index_is_the_stable_inverse(device, lens, t_begin):
+    """Sequences that begin inside a counting chunk, more blocks than the fill kernel's LDS masks hold, counting chunks of
+    more than 256 tokens, ignored slots: the lists are those of a stable sort by block."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.topk import get_bind_from_find
+    cu = make_cu(lens)
+    T, KH, N = int(cu[-1]), 2, 16
+    setup_helper(cu.to(device), top_n=N)
+    g = torch.Generator().manual_seed(7)
+    n = torch.cat([torch.arange(x) for x in lens])
+    nb = torch.cat([torch.full((x,), -(-x // 64)) for x in lens])
+    first = torch.cat([torch.full((x,), b) for x, b in zip(lens, NSAHelper.k_cu_seqlens.tolist())])
+    # distinct blocks per token: a random start and a stride that is coprime to what is wrapped around; -1: ignored
+    j = (torch.randint(0, 1 << 20, (KH, T, 1), generator=g) + torch.arange(N)) % torch.clamp(nb, min=N)[None, :, None]
+    topk = torch.where(j < nb[None, :, None], j, torch.full_like(j, -1)).to(torch.int32)
+    bind = get_bind_from_find(topk.to(device), chunk_tokens=100, t_begin=t_begin)
+    off, tok, items = bind["csr_off"].cpu().long(), bind["csr_tok"].cpu().long(), bind["item_off"].cpu().long()
+    nvalid = torch.where(n >= t_begin, torch.clamp(n // 64 + 1, max=N), torch.zeros_like(n))
+    for kh in range(KH):
+        use = (torch.arange(N) < nvalid[:, None]) & (topk[kh] >= 0)
+        blk = (first[:, None] + topk[kh])[use]
+        order = torch.sort(blk, stable=True).indices
+        counts = torch.bincount(blk, minlength=bind["nblk"])
+        want = n[:, None].expand(T, N)[use][order]
+        lo = int(off[kh, 0])
+        assert lo == kh * T * N
+        assert torch.equal(off[kh, 1:] - off[kh, :-1], counts)
+        assert torch.equal(tok[lo:lo + want.numel()], want)
+        assert torch.equal(items[kh, 1:] - items[kh, :-1], (counts + 99) // 100)
+
+
 def test_combine_bwd(device):
     from flash_nsa.ops.combine import combine_bwd
     a, b, c = [randn_bf16(300, 8, 128, seed=s) for s in (1, 2, 3)]
