@@ -239,8 +239,8 @@ int nsa_slc_attn_bwd_dkdv_before_window(const void* q, int64_t q_st, int64_t q_s
  *   csr_tok  [KH*T*top_n]       query tokens (index local to their sequence), ascending within a list
  *   item_off [KH][nblk_total+1] prefix count of list chunks of chunk_tokens tokens (work items of the dk/dv pass)
  *   workspace: int32 scratch of nsa_inverse_index_workspace_elems(T,KH,nblk_total) elements
- * nsa_slc_bwd_chunk_tokens: the chunk_tokens this library suggests for a batch of T tokens (1024 for long batches,
- * less when that would leave the dk/dv pass too few work items); any positive value is valid as long as the
+ * nsa_slc_bwd_chunk_tokens: the chunk_tokens this library suggests for a batch of T tokens (256, less when that
+ * would leave the dk/dv pass too few work items); any positive value is valid as long as the
  * builder and nsa_slc_attn_bwd_dkdv get the same one */
 int64_t nsa_inverse_index_workspace_elems(int T, int KH, int nblk_total);
 int nsa_slc_bwd_chunk_tokens(int T, int KH, int top_n);

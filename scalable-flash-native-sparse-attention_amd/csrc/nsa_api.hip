@@ -505,12 +505,15 @@ int nsa_cmp_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
 
 
 int nsa_slc_bwd_chunk_tokens(int T, int KH, int top_n) {
-  // list chunk (tokens per work item of the selected-attention dk/dv pass): 1024 for long batches, smaller when
-  // that would leave fewer than about 2048 two-wave work items; below 256 the fp32 atomic additions of the many
-  // items cost more than the idle CUs
-  const int64_t want = (int64_t)KH * T * top_n / 2048;
-  int c = 256;
-  while (c < 1024 && c * 2 <= want) c *= 2;
+  // List chunk (tokens per work item of the selected-attention dk/dv pass).  An item of 256 tokens takes 200 us at 128
+  // channels (16 q-heads per kv head), so a batch that has fewer of them than the 512 two-wave workgroups the GPU holds
+  // takes that long whatever its size: it is cut finer, down to 64.  Longer items than 256 only add imbalance; shorter
+  // ones than the GPU needs add fp32 atomics.  us at 64 / 128 / 256 / 512 / 1024 tokens, 16 q / 1 kv heads: 2K tokens
+  // 75 / 111 / 200 / 383 / 701, 4K 155 / 131 / 203 / 383 / 749, 8K 300 / 256 / 228 / 387 / 752; 64 / 4 heads: 16K 2043 /
+  // 1812 / 1807 / 1924 / 2071, 8 x 6K 4933 / 4530 / 4465 / 4776 / 5064, 64K 8478 / 7814 / 7584 / 7551 / 7777.
+  const int64_t want = (int64_t)KH * T * top_n / 512;
+  int c = 64;
+  while (c < 256 && c * 2 <= want) c *= 2;
   return c;
 }
 

@@ -69,13 +69,14 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     assert dk.dtype == torch.float32 and dv.dtype == torch.float32
     if 0 < helper.x_maxlen <= t_begin:
         return dq_buf, dk, dv
+    ordered = dkdv_repeat or getattr(helper, "deterministic", False)
     if bind is None:
-        bind = get_bind_from_find(topk, helper, t_begin=t_begin)
+        bind = get_bind_from_find(topk, helper, t_begin=t_begin, deterministic=ordered)
     args = (*common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0), dv.stride(1),
             helper.x_cu_seqlens.data_ptr(), helper.k_cu_seqlens.data_ptr(), helper.blk_seq.data_ptr(),
             bind["csr_off"].data_ptr(), bind["csr_tok"].data_ptr(), bind["item_off"].data_ptr(), bind["nblk"],
             bind["chunk_tokens"], bind["n_items_bound"], helper.batch, QH, KH, D, VD, helper.block_size, sm_scale)
-    if dkdv_repeat or getattr(helper, "deterministic", False):
+    if ordered:
         nbytes = _lib.value("nsa_slc_attn_bwd_dkdv_det_bytes", bind["n_items_bound"], KH, D, VD, helper.block_size)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=q.device)
         _lib.call("nsa_slc_attn_bwd_dkdv_det", *args, ws.data_ptr(), ws.numel(), _lib.stream_ptr())

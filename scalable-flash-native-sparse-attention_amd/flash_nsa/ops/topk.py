@@ -67,16 +67,23 @@ def topk_workspace(total_tokens, max_blocks, KH, device):
 
 
 @torch.no_grad()
-def get_bind_from_find(topk, helper=NSAHelper, chunk_tokens=None, t_begin=0):
+def get_bind_from_find(topk, helper=NSAHelper, chunk_tokens=None, t_begin=0, deterministic=None):
     """Inverse of the selection: for every (kv head, selection block) the ascending list of query tokens that
     selected it.  Returns a dict with the CSR (csr_off [KH,nblk+1], csr_tok [KH*T*top_n]), the work-item prefix
     (item_off [KH,nblk+1]) and the static bound on the number of work items per kv head.  Queries at positions below
-    t_begin are left out."""
+    t_begin are left out.  deterministic (default: the helper's): the work items are sized for the ordered sum."""
+    if deterministic is None:
+        deterministic = getattr(helper, "deterministic", False)
     KH, T, N = topk.shape
     dev = topk.device
     nblk = helper.k_len
     if chunk_tokens is None:
         chunk_tokens = _lib.value("nsa_slc_bwd_chunk_tokens", T, KH, N)
+        if deterministic:
+            # every work item holds a slot of 64 KB (at 128 channels) until the ordered sum: longer items for long
+            # batches, at most about 2048 + one per block and kv head
+            want = KH * T * N // 2048
+            chunk_tokens = 1024 if want >= 1024 else 512 if want >= 512 else 256
     csr_off = torch.empty(KH, nblk + 1, device=dev, dtype=torch.int32)
     item_off = torch.empty(KH, nblk + 1, device=dev, dtype=torch.int32)
     csr_tok = torch.empty(KH * T * N, device=dev, dtype=torch.int32)
