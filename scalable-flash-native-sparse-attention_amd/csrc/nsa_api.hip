@@ -1056,6 +1056,15 @@ int nsa_decode_split_lds_total(int D, int VD, int fixed_y_maxlen, int fixed_num_
   return dyn > 0 ? dyn + nsa_decode_split_static_lds_bytes() : 0;
 }
 
+int nsa_decode_split_window_parts(int window, int fixed_y_maxlen, int nsplit) {
+  // as many as give a wave of the window no more units than a wave of the compressed branch has
+  if (window < 0 || window > 65536 || nsplit <= 0) return 0;
+  const int units = window / 32 + 2;
+  const int cmp = (fixed_y_maxlen / 32 + 4 * nsplit - 1) / (4 * nsplit);
+  const int n = (units + 4 * (cmp > 2 ? cmp : 2) - 1) / (4 * (cmp > 2 ? cmp : 2));
+  return n < 4 ? n : 4;
+}
+
 static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
                      const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
                      void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
@@ -1066,7 +1075,7 @@ static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const vo
                      int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
                      int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
                      int num_local, int ignore_index, int window, float sm_scale, int slc_nsplit, float* sp2_ml,
-                     float* sp2_o, void* cmp_tmp, void* stream) {
+                     float* sp2_o, void* cmp_tmp, int win_parts, float* win_ml, float* win_o, void* stream) {
   int rc = check_heads("decode_split", QH, KH, D, VD);
   if (rc) return rc;
   rc = check_nsa_sizes("decode_split", kernel_size, stride, block_size);
@@ -1088,7 +1097,13 @@ static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const vo
               slc_nsplit);
   NSA_REQUIRE(slc_nsplit == 1 || (sp2_ml && sp2_o && cmp_tmp), NSA_ERR_BAD_ARG,
               "decode_split: slc_nsplit > 1 needs the three buffers of the window / selected parts");
+  NSA_REQUIRE(win_parts >= 0 && win_parts <= 4 && (win_parts == 0 || (win_ml && win_o)), NSA_ERR_BAD_ARG,
+              "decode_split: win_parts %d must be in [0,4], with its two buffers", win_parts);
+  NSA_REQUIRE(win_parts == 0 || (window >= 0 && window <= 65536), NSA_ERR_BAD_ARG,
+              "decode_split: window %d must be in [0,65536] to be attended in parts", window);
   NsaDecodeParams p{};
+  p.win_parts = win_parts; p.win_m = win_ml; p.win_o = win_o;
+  p.win_l = win_ml ? win_ml + (int64_t)B * KH * win_parts * 16 : nullptr;
   p.slc_nsplit = slc_nsplit; p.sp2_ml = sp2_ml; p.sp2_o = sp2_o; p.cmp_tmp = (bf16_t*)cmp_tmp;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.k = (const bf16_t*)k_cache; p.k_sr = k_sr; p.k_sh = k_sh;
@@ -1127,7 +1142,26 @@ int nsa_decode_split(const void* q, int64_t q_st, int64_t q_sh, const void* k_ca
                            sp_keep_m, nsplit, cmp_slot_mapping, context_lens, block_tables, table_stride,
                            cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD, fixed_y_maxlen,
                            fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init, num_local,
-                           ignore_index, window, sm_scale, 1, nullptr, nullptr, nullptr, stream);
+                           ignore_index, window, sm_scale, 1, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream);
+}
+
+int nsa_decode_split_window(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
+                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
+                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                     int64_t tk_st, float* sp_m, float* sp_l, float* sp_o, void* sp_keep_p, float* sp_keep_m,
+                     int nsplit, const int32_t* cmp_slot_mapping, const int32_t* context_lens,
+                     const int32_t* block_tables, int table_stride, const int32_t* cmp_block_tables,
+                     int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
+                     int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
+                     int num_local, int ignore_index, int window, float sm_scale, int win_parts,
+                     float* win_ml, float* win_o, void* stream) {
+  return decode_split_impl(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, w, w_st, w_sh, out, o_st, o_sh, cmp_o, slc_o,
+                           swa_o, co_st, co_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, sp_m, sp_l, sp_o, sp_keep_p,
+                           sp_keep_m, nsplit, cmp_slot_mapping, context_lens, block_tables, table_stride,
+                           cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD, fixed_y_maxlen,
+                           fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init, num_local,
+                           ignore_index, window, sm_scale, 1, nullptr, nullptr, nullptr, win_parts, win_ml, win_o, stream);
 }
 
 int nsa_decode_split_parts(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
@@ -1146,7 +1180,8 @@ int nsa_decode_split_parts(const void* q, int64_t q_st, int64_t q_sh, const void
                            sp_keep_m, nsplit, cmp_slot_mapping, context_lens, block_tables, table_stride,
                            cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD, fixed_y_maxlen,
                            fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init, num_local,
-                           ignore_index, window, sm_scale, slc_nsplit, sp2_ml, sp2_o, cmp_tmp, stream);
+                           ignore_index, window, sm_scale, slc_nsplit, sp2_ml, sp2_o, cmp_tmp, 0, nullptr,
+                           nullptr, stream);
 }
 
 int nsa_decode_slc_swa_combine(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,

@@ -176,6 +176,9 @@ struct NsaDecodeParams {
   // output, and a third launch merges and combines.  sp2_ml [B,KH,slc_nsplit,2 branches,2 (m,l),16],
   // sp2_o [B,KH,slc_nsplit,2,16,VD] fp32, cmp_tmp [B,QH,VD] bf16
   int slc_nsplit; float* sp2_ml; float* sp2_o; bf16_t* cmp_tmp;
+  // two-launch split path: win_parts (0..4) workgroups per (request, kv head) of the first launch attend the window;
+  // fp32 scratch [B,KH,win_parts,16] (m, l), [B,KH,win_parts,16,VD] (o).  0: the second launch does
+  int win_parts; float* win_m; float* win_l; float* win_o;
 };
 int nsa_decode_cmp_topk_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream);
 int nsa_decode_slc_swa_launch(const NsaDecodeParams& p, int B, int D, int VD, hipStream_t stream);

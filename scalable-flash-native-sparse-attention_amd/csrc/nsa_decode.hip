@@ -13,6 +13,7 @@
 // pool through the block tables.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include <algorithm>
 #include <type_traits>
 #include "nsa_select.h"
 
@@ -24,6 +25,48 @@ constexpr int DEC_WAVES = 8;
 constexpr size_t SLC_SWA_STATIC_LDS = (3 * 16 + 64 * 16) * sizeof(float);
 constexpr int UK = 32;  // keys per unit
 constexpr int SEL_INTS = 192;  // LDS words of a selecting wave: 64 selected blocks + candidate list (64 scores, 64 indices)
+
+// Sum of K raw rows from position st on, in row order in fp32: one 16-byte piece (col: its column in the pool).  The row
+// at position `given` is not read but taken from given_row (the lane has just stored it).  It stands in front of
+// everything else that the workgroup does and is a chain of round trips and of a lone wave's instructions, so the page is
+// divided out once (a window of at most a page touches two) and 16 rows are fetched at a time.  One-launch step at which
+// every request completes a compressed row, 64 q / 4 kv heads, us, row by row -> so: 16 x 4K 47.5 -> 36.5, 64 x 4K 63 -> 51,
+// 512 x 4K 398 -> 329; 64 ragged requests, four of which complete one, 78.8 -> 73.5.
+NSA_DEVICE void sum_rows(float (&a)[8], const bf16_t* col, int64_t c_sr, const int32_t* tab, int page, int st, int K,
+                         int given, bf16x8 given_row) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) a[e] = 0.f;
+  if (K > page) {
+    for (int n = st; n < st + K; n++) {
+      bf16x8 x = given_row;
+      if (n != given) x = ld_global_b128(col + ((int64_t)tab[n / page] * page + (n % page)) * c_sr);
+#pragma unroll
+      for (int e = 0; e < 8; e++) a[e] += (float)x[e];
+    }
+    return;
+  }
+  const int p0 = st / page, off = st - p0 * page;
+  const int64_t row0 = (int64_t)tab[p0] * page + off;
+  const int64_t row1 = off + K > page ? (int64_t)tab[p0 + 1] * page + off - page : row0;
+  const int skip = given - st;  // < K; negative: none
+  constexpr int RB = 16;
+  for (int r0 = 0; r0 < K; r0 += RB) {
+    bf16x8 x[RB];
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      int k = min(r0 + r, K - 1);
+      if (k == skip) k = max(k - 1, 0);
+      x[r] = ld_global_b128(col + ((off + k < page ? row0 : row1) + k) * c_sr);
+    }
+#pragma unroll
+    for (int r = 0; r < RB; r++)
+      if (r0 + r < K) {
+        if (r0 + r == skip) x[r] = given_row;
+#pragma unroll
+        for (int e = 0; e < 8; e++) a[e] += (float)x[r][e];
+      }
+  }
+}
 
 // One wave's flash-attention state over units of 32 keys for the 16 heads of a kv group.
 // K and V rows of a unit are fetched as whole rows (16 lanes x 16 bytes per row: every cache line is requested once
@@ -613,10 +656,15 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_cmp_topk_kernel(NsaDeco
 // ---- split variant of the compressed branch: requests are cut in NSPLIT key-interleaved parts so that long
 // contexts do not leave most CUs idle; partial (m, l, o) go through a small fp32 scratch in global memory.
 constexpr int SPLIT_WAVES = 4;
+// scratch of the caller: float-aligned
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// grid (B, KH, nsplit): compressed attention over the units u = s*4 + wave (mod 4*nsplit)
+// grid (B, KH, nsplit + win_parts): compressed attention over the units u = s*4 + wave (mod 4*nsplit); the last win_parts
+// parts of a pair attend the window in the same way, which needs nothing from the block selection and so stays out of
+// the second launch (0 / 1 / 2 / 3 / 4 parts, both launches: 1 x 32K 38.2 / 39.3 / 37.5 / 36.8 / 37.0 us, 16 x 128K
+// 99.9 / 98.0 / 97.7 / 97.8 / 99.9).  Two workgroups per CU, or the window's would wait for a CU.
 template <int D, int VD>
-__global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(NsaDecodeParams p) {
+__global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void decode_cmp_partial_kernel(NsaDecodeParams p) {
   using UF = UnitFlash<D, VD, KEEP_MEM>;
   constexpr int NW = SPLIT_WAVES;
   constexpr int SLOT = UF::SLOT;
@@ -630,13 +678,19 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(Ns
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.x, kh = blockIdx.y, sp = blockIdx.z;
-  const int nsplit = gridDim.z;
+  const int nsplit = gridDim.z - p.win_parts;
+  const bool in_window = sp >= nsplit;  // workgroup-uniform
   const int G = p.G;
   const int L = p.ctx_lens[b];
   const int y = L >= p.kernel_size ? min((L - p.kernel_size) / p.stride + 1, p.y_cap) : 0;
   const int32_t* ctab = p.cmp_table + (int64_t)b * p.cmp_table_stride;
   const int page = p.page_size;
-  for (int i = tid; i < (y + page - 1) / page; i += NW * 64) tab_s[i] = ctab[i];
+  const int t = L - 1;
+  const int klo = in_window ? max(0, t - p.window) : 0;
+  const int khi = in_window ? t : y - 1;
+  const int page0 = klo / page;  // tab_s: pages of the keys klo .. khi
+  if (in_window) ctab = p.table + (int64_t)b * p.table_stride;
+  for (int i = page0 + tid; i <= (khi < 0 ? -1 : khi / page); i += NW * 64) tab_s[i - page0] = ctab[i];
   // The compressed row that the newest token completes (mean of the last kernel_size raw rows, fp32 sums in row
   // order like nsa_paged_pool_decode; flash_nsa/inference/compress_kv.py:253-287 upstream) is written by the part
   // that attends it -- the one whose waves own the last unit -- wave 0 for K and wave 1 for V, one 16-byte piece per
@@ -650,14 +704,8 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(Ns
       if (lane < (wave == 0 ? D : VD) / 8) {
         const int32_t* tab = p.table + (int64_t)b * p.table_stride;
         const int st = ((L - p.kernel_size) / p.stride) * p.stride;
-        float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int r = 0; r < p.kernel_size; r++) {
-          const int n = st + r;
-          const int64_t row = (int64_t)tab[n / page] * page + (n % page);
-          const bf16x8 x = ld_global_b128(cache + row * c_sr + (int64_t)kh * c_sh + lane * 8);
-#pragma unroll
-          for (int e = 0; e < 8; e++) a[e] += (float)x[e];
-        }
+        float a[8];
+        sum_rows(a, cache + (int64_t)kh * c_sh + lane * 8, c_sr, tab, page, st, p.kernel_size, -1, zero_bf16x8());
         const float inv = 1.f / (float)p.kernel_size;
         *reinterpret_cast<bf16x8*>(cache + (int64_t)cmp_slot * c_sr + (int64_t)kh * c_sh + lane * 8) =
             pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -673,36 +721,43 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64) void decode_cmp_partial_kernel(Ns
 
   UF uf;
   uf.init(p.q + (int64_t)b * p.q_st + (int64_t)head * p.q_sh, p.scale_log2, lane, Vs_all + wave * SLOT);
-  if (p.sp_keep_p != nullptr) {  // spill the un-normalised probabilities of every unit for the final kernel
+  if (p.sp_keep_p != nullptr && !in_window) {  // spill the un-normalised probabilities of every unit for the final kernel
     const int nuc = (p.y_cap + UK - 1) / UK;
     // unit-major: a wave writes the 1 KB of a unit as whole cache lines
     uf.spill_p = (typename UF::keep_t*)p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * nuc * UK;
     uf.keep_m = p.sp_keep_m + ((int64_t)b * p.KH + kh) * nuc * 16;
     uf.keep_end = y;
   }
-  const int nu = (y + UK - 1) / UK;
-  uf.run(sp * NW + wave, NW * nsplit, nu, 0, y - 1, [&](int u) { return u * UK; }, tab_s, page, kbase, p.k_sr,
-         vbase, p.v_sr);
+  const int k0 = (klo / UK) * UK;
+  const int nu = khi < 0 ? 0 : (khi - k0) / UK + 1;
+  const int first = in_window ? (sp - nsplit) * NW + wave : sp * NW + wave;
+  uf.run(first, NW * (in_window ? p.win_parts : nsplit), nu, klo, khi, [&](int u) { return k0 + u * UK; }, tab_s - page0,
+         page, kbase, p.k_sr, vbase, p.v_sr);
   uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
   __syncthreads();
-  // merge the 4 waves; store the split's un-normalised partial
-  const int64_t base = (((int64_t)b * p.KH + kh) * nsplit + sp) * 16;
+  // merge the 4 waves; store the part's un-normalised partial
+  const int64_t pair = (int64_t)b * p.KH + kh;
+  const int64_t base = (in_window ? pair * p.win_parts + (sp - nsplit) : pair * nsplit + sp) * 16;
+  float* const m_dst = (in_window ? p.win_m : p.sp_m) + base;
+  float* const l_dst = (in_window ? p.win_l : p.sp_l) + base;
+  float* const o_dst = (in_window ? p.win_o : p.sp_o) + base * VD;
   const float* po = reinterpret_cast<const float*>(Vs_all);
-  for (int idx = tid; idx < 16 * VD; idx += NW * 64) {
-    int h = idx / VD, d = idx - h * VD;
+  for (int idx = tid * 4; idx < 16 * VD; idx += NW * 64 * 4) {
+    const int h = idx / VD, d = idx - h * VD;
     float m = NSA_NEG_INF;
     for (int w = 0; w < NW; w++) m = fmaxf(m, part_m[w * 16 + h]);
-    float l = 0.f, o = 0.f;
+    float l = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
     if (m != NSA_NEG_INF) {
       for (int w = 0; w < NW; w++) {
-        float mw = part_m[w * 16 + h];
-        float a = (mw == NSA_NEG_INF) ? 0.f : fast_exp2((mw - m) * p.scale_log2);
+        const float mw = part_m[w * 16 + h];
+        const float a = (mw == NSA_NEG_INF) ? 0.f : fast_exp2((mw - m) * p.scale_log2);
         l += a * part_l[w * 16 + h];
-        o += a * po[w * (SLOT / 2) + h * UF::OLD + d];
+        o += a * *reinterpret_cast<const f32x4*>(&po[w * (SLOT / 2) + h * UF::OLD + d]);
       }
     }
-    p.sp_o[(base + h) * VD + d] = o;
-    if (d == 0) { p.sp_m[base + h] = m; p.sp_l[base + h] = l; }
+    *reinterpret_cast<f32x4u*>(o_dst + idx) = o;
+    if (d == 0) { m_dst[h] = m; l_dst[h] = l; }
   }
 }
 
@@ -856,7 +911,16 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
                 "the host-side LDS budget must count this kernel's static arrays");
   constexpr int OPT = 16 * VD / NT;  // output values per thread
   static_assert((16 * VD) % NT == 0, "output values must divide over the threads");
-  float ocmp_pre[OPT];               // split path: merged compressed-branch output of this thread's values
+  // output values of a thread: OPT consecutive channels of one head
+  typedef float fvec __attribute__((ext_vector_type(OPT)));
+  typedef float fvecu __attribute__((ext_vector_type(OPT), aligned(4)));
+  typedef bf16_t bvecu __attribute__((ext_vector_type(OPT), aligned(2)));
+  const int oi = tid * OPT;
+  const int oh = oi / VD, od = oi - oh * VD;
+  const int W = p.win_parts;         // > 0: the first launch has attended the window
+  fvec ocmp_pre, o_swa_pre;          // merged outputs of the compressed branch (split path) and of the window
+#pragma unroll
+  for (int r = 0; r < OPT; r++) ocmp_pre[r] = o_swa_pre[r] = 0.f;
   float* imp = nullptr;              // block scores, when the selection runs here
   const bool select_here = p.sp_keep_p != nullptr || p.pg != nullptr;
   if (p.sp_keep_p != nullptr) {
@@ -873,12 +937,40 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     const int64_t sp_base = ((int64_t)b * p.KH + kh) * nsplit * 16;
     const typename UF::keep_t* keep_p = (const typename UF::keep_t*)p.sp_keep_p + ((int64_t)b * p.KH + kh) * 16 * keep_ld;
     const float* keep_m = p.sp_keep_m + ((int64_t)b * p.KH + kh) * nuc * 16;
-    // all (m, l) of the parts in one round trip, then one thread per head
+    // Everything that comes from the first launch is requested here, in one round trip to memory: statistics, outputs of
+    // the parts, maxima and the first probabilities (the rest of the prologue is a chain of short steps with barriers).
+    // Us of this launch, with a round trip per step and the window attended next to the selection -> so: one request of
+    // 32K tokens 28.9 -> 22.4, 16 of 128K 45.4 -> 36.0, 8 of up to 16K with 192 channels 29.8 -> 23.4; 1-2 us of it come
+    // from the window, the rest from the loads.
+    constexpr int PRE = 8, KM = 2, WMAX = 4;
     float* st_m = fac;
     float* st_l = fac + 64 * 16;
     for (int i = tid; i < nsplit * 16; i += NT) { st_m[i] = p.sp_m[sp_base + i]; st_l[i] = p.sp_l[sp_base + i]; }
+    const int64_t w_base = ((int64_t)b * p.KH + kh) * W * 16;
+    if (tid < W * 16) { part_m[tid] = p.win_m[w_base + tid]; part_l[tid] = p.win_l[w_base + tid]; }
+    auto part_out = [&](const float* o, int64_t base16, int s2) {
+      return (fvec)*reinterpret_cast<const fvecu*>(o + (base16 + s2 * 16 + oh) * VD + od);
+    };
+    fvec po[PRE], wo[WMAX];
+#pragma unroll
+    for (int s2 = 0; s2 < PRE; s2++) po[s2] = part_out(p.sp_o, sp_base, min(s2, nsplit - 1));
+    if (W > 0) {
+#pragma unroll
+      for (int s2 = 0; s2 < WMAX; s2++) wo[s2] = part_out(p.win_o, w_base, min(s2, W - 1));
+    }
+    const int nu = (y + UK - 1) / UK;
+    float km[KM];
+#pragma unroll
+    for (int r = 0; r < KM; r++) km[r] = tid + r * NT < nu * 16 ? keep_m[tid + r * NT] : 0.f;
+    h4 v[16];
+    auto fetch_probs = [&](int k4) {
+#pragma unroll
+      for (int h = 0; h < 16; h++)
+        v[h] = *reinterpret_cast<const h4*>(keep_p + (k4 / UK) * (16 * UK) + h * UK + (k4 % UK));
+    };
+    if (tid * 4 < y) fetch_probs(tid * 4);
     __syncthreads();
-    if (tid < 16) {
+    if (tid < 16) {  // one thread per head
       float m = NSA_NEG_INF;
       for (int s2 = 0; s2 < nsplit; s2++) m = fmaxf(m, st_m[s2 * 16 + tid]);
       float l = 0.f;
@@ -893,34 +985,42 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
       const float lse2 = (m != NSA_NEG_INF && l > 0.f) ? m * p.scale_log2 + fast_log2(l) : 0.f;
       sp_lse_s[tid] = lse2;
       if (tid < G && p.lse_out) p.lse_out[(int64_t)b * p.lse_st + (kh * G + tid) * p.lse_sh] = lse2;
+    } else if (wave == 1 && lane < 16 && W > 0) {
+      merge_weights(part_m, part_l, W, 16, lane, p.scale_log2);
     }
     __syncthreads();
-    // merge of the parts' outputs: independent loads, issued here so that they overlap the rest of the prologue
+    for (int s0 = 0; s0 < nsplit; s0 += PRE) {
+      if (s0 > 0) {
 #pragma unroll
-    for (int r = 0; r < OPT; r++) {
-      const int idx = tid + r * NT;
-      const int h = idx / VD, d = idx - h * VD;
-      float o = 0.f;
-      for (int s2 = 0; s2 < nsplit; s2++) o += sp_w_s[s2 * 16 + h] * p.sp_o[(sp_base + s2 * 16 + h) * VD + d];
-      ocmp_pre[r] = o;
+        for (int s2 = 0; s2 < PRE; s2++) po[s2] = part_out(p.sp_o, sp_base, min(s0 + s2, nsplit - 1));
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < PRE; s2++)
+        if (s0 + s2 < nsplit) ocmp_pre += sp_w_s[(s0 + s2) * 16 + oh] * po[s2];
     }
-    const int nu = (y + UK - 1) / UK;
-    for (int i = tid; i < nu * 16; i += NT) {
+    if (W > 0) {
+#pragma unroll
+      for (int s2 = 0; s2 < WMAX; s2++)
+        if (s2 < W) o_swa_pre += part_l[s2 * 16 + oh] * wo[s2];
+    }
+#pragma unroll
+    for (int r = 0; r < KM; r++) {
+      const int i = tid + r * NT, h = i & 15;
+      if (i < nu * 16) fac[i] = h < G ? fast_exp2(__builtin_fmaf(km[r], p.scale_log2, -sp_lse_s[h])) : 0.f;
+    }
+    for (int i = tid + KM * NT; i < nu * 16; i += NT) {
       const int h = i & 15;
       fac[i] = h < G ? fast_exp2(__builtin_fmaf(keep_m[i], p.scale_log2, -sp_lse_s[h])) : 0.f;
     }
     __syncthreads();
     for (int k4 = tid * 4; k4 < y; k4 += NT * 4) {
       const float* f = fac + (k4 / UK) * 16;
-      h4 v[16];
-#pragma unroll
-      for (int h = 0; h < 16; h++)
-        v[h] = *reinterpret_cast<const h4*>(keep_p + (k4 / UK) * (16 * UK) + h * UK + (k4 % UK));
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int h = 0; h < 16; h++)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[e] += (float)v[h][e] * f[h];
+      if (k4 + NT * 4 < y) fetch_probs(k4 + NT * 4);
       *reinterpret_cast<f32x4*>(pgs + k4) = acc;
     }
     __syncthreads();
@@ -937,7 +1037,10 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
   }
   __syncthreads();
 
-  // ---- window attention; when the selection runs here, wave 0 selects meanwhile ----
+  // ---- window attention, or, when the first launch has done it, the blocks that are selected whatever their score (they
+  // open the selected branch); when the selection runs here, wave 0 selects meanwhile ----
+  const int upb = Bs / UK;
+  const int n_forced = W > 0 ? min(p.num_init + p.num_local, nvalid) : 0;
   UF uf;
   uf.init(p.q + (int64_t)b * p.q_st + (int64_t)head * p.q_sh, p.scale_log2, lane, Vs_all + wave * SLOT);
   const int w_first = select_here ? 1 : 0;
@@ -947,13 +1050,18 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     if (p.topk && part == 0 && lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + (int64_t)b * p.tk_st + lane] = result;
   } else {
     if (t >= 0) {
-      const int klo = max(0, t - p.window);
+      const int klo = W > 0 ? 0 : max(0, t - p.window);
       const int k0 = (klo / UK) * UK;
-      const int nu = (t - k0) / UK + 1;
+      const int nu = W > 0 ? n_forced * upb : (t - k0) / UK + 1;
       uf.run(part * (NW - w_first) + wave - w_first, nparts * (NW - w_first), nu, klo, t,
-             [&](int u) { return k0 + u * UK; }, tab_s, page, kbase, p.k_sr, vbase, p.v_sr);
+             [&](int u) {
+               if (W == 0) return k0 + u * UK;
+               const int slot = u / upb;
+               return (slot < p.num_init ? slot : t / Bs - (slot - p.num_init)) * Bs + (u - slot * upb) * UK;
+             },
+             tab_s, page, kbase, p.k_sr, vbase, p.v_sr);
     }
-    uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
+    if (W == 0) uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
   }
   __syncthreads();
   const float* part_o = reinterpret_cast<const float*>(Vs_all);
@@ -983,7 +1091,6 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     __syncthreads();  // the slots are staging space again
     uf.reset();
     if (t >= 0) {
-      const int upb = Bs / UK;
       uf.run(part * NW + wave, nparts * NW, nvalid * upb, 0, t,
              [&](int u) { int slot = u / upb; return blk_s[slot] * Bs + (u - slot * upb) * UK; }, tab_s, page, kbase,
              p.k_sr, vbase, p.v_sr);
@@ -991,66 +1098,72 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
     uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
     __syncthreads();
     spill_part(0, 0, NW);
-    if (part == 0 && p.sp_keep_p != nullptr) {  // the compressed branch's output, merged in the prologue
+    if (part == 0 && p.sp_keep_p != nullptr && oh < G) {  // the compressed branch's output, merged in the prologue
+      bvecu c;
 #pragma unroll
-      for (int r = 0; r < OPT; r++) {
-        const int idx = tid + r * NT;
-        const int h = idx / VD, d = idx - h * VD;
-        if (h < G) p.cmp_tmp[(int64_t)b * p.co_st + (int64_t)(kh * G + h) * p.co_sh + d] = (bf16_t)ocmp_pre[r];
-      }
+      for (int r = 0; r < OPT; r++) c[r] = (bf16_t)ocmp_pre[r];
+      *reinterpret_cast<bvecu*>(p.cmp_tmp + (int64_t)b * p.co_st + (int64_t)(kh * G + oh) * p.co_sh + od) = c;
     }
     return;
   }
-  if (tid < 16) merge_weights(part_m + w_first * 16, part_l + w_first * 16, NW - w_first, 16, tid, p.scale_log2);
-  __syncthreads();
-  float o_swa_pre[OPT];
+  // the weighted sum of the partial outputs of waves w0 .. w0 + NP - 1
+  auto merged = [&](auto np, int w0) {
+    constexpr int NP = decltype(np)::value;
+    float wgt[NP];
+    merge_weights_local<NP>(part_m + w0 * 16, part_l + w0 * 16, 16, oh, p.scale_log2, wgt);
+    fvec o;
 #pragma unroll
-  for (int r = 0; r < OPT; r++) {
-    const int idx = tid + r * NT;
-    const int h = idx / VD, d = idx - h * VD;
-    o_swa_pre[r] = merge_value(part_l + w_first * 16, part_o + w_first * (SLOT / 2), NW - w_first, 16, SLOT / 2, h, d, UF::OLD);
+    for (int r = 0; r < OPT; r++) o[r] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NP; w++)
+      o += wgt[w] * *reinterpret_cast<const fvec*>(&part_o[(w0 + w) * (SLOT / 2) + oh * UF::OLD + od]);
+    return o;
+  };
+  if (W == 0) {
+    if (w_first) o_swa_pre = merged(std::integral_constant<int, NW - 1>{}, 1);
+    else o_swa_pre = merged(std::integral_constant<int, NW>{}, 0);
+    __syncthreads();  // the slots are staging space again
+    uf.reset();
   }
-  __syncthreads();  // the slots are staging space again
 
-  // ---- selected blocks, all waves ----
-  uf.reset();
+  // ---- selected blocks (behind the forced ones), all waves; the last wave and wave 0 have had fewest units so far ----
   if (t >= 0) {
-    const int upb = Bs / UK;
-    uf.run(wave, NW, nvalid * upb, 0, t,
-           [&](int u) { int slot = u / upb; return blk_s[slot] * Bs + (u - slot * upb) * UK; }, tab_s, page, kbase,
-           p.k_sr, vbase, p.v_sr);
+    uf.run(W > 0 ? (wave + 1) % NW : wave, NW, (nvalid - n_forced) * upb, 0, t,
+           [&](int u) { const int slot = u / upb; return blk_s[n_forced + slot] * Bs + (u - slot * upb) * UK; }, tab_s, page,
+           kbase, p.k_sr, vbase, p.v_sr);
+  }
+  // the gates come from memory: request them before the merge
+  float gate[3] = {0.f, 0.f, 0.f};
+  const int hq = kh * G + oh;
+  if (p.out && oh < G) {
+    const bf16_t* wp = p.w + (int64_t)b * p.w_st + (int64_t)hq * p.w_sh;
+#pragma unroll
+    for (int i = 0; i < 3; i++) gate[i] = 1.f / (1.f + __expf(-(float)wp[i]));
   }
   uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
   __syncthreads();
-  if (tid < 16) merge_weights(part_m, part_l, NW, 16, tid, p.scale_log2);
-  __syncthreads();
+  if (oh >= G) return;
+  const fvec o_slc = merged(std::integral_constant<int, NW>{}, 0);
+  const int64_t co = (int64_t)b * p.co_st + (int64_t)hq * p.co_sh + od;
+  // branch outputs are rounded to bf16 before the gated sum, as the three-kernel path stores them
+  bvecu slc, swa, cmp;
 #pragma unroll
-  for (int r = 0; r < OPT; r++) {
-    const int idx = tid + r * NT;
-    const int h = idx / VD, d = idx - h * VD;
-    if (h >= G) continue;
-    const int hq = kh * G + h;
-    float o_slc = merge_value(part_l, part_o, NW, 16, SLOT / 2, h, d, UF::OLD);
-    // branch outputs are rounded to bf16 before the gated sum, as the three-kernel path stores them
-    o_slc = (float)(bf16_t)o_slc;
-    const float o_swa = (float)(bf16_t)o_swa_pre[r];
-    if (p.slc_o) p.slc_o[(int64_t)b * p.co_st + (int64_t)hq * p.co_sh + d] = (bf16_t)o_slc;
-    if (p.swa_o) p.swa_o[(int64_t)b * p.co_st + (int64_t)hq * p.co_sh + d] = (bf16_t)o_swa;
-    if (p.out) {
-      const bf16_t* wp = p.w + (int64_t)b * p.w_st + (int64_t)hq * p.w_sh;
-      float s0 = 1.f / (1.f + __expf(-(float)wp[0]));
-      float s1 = 1.f / (1.f + __expf(-(float)wp[1]));
-      float s2 = 1.f / (1.f + __expf(-(float)wp[2]));
-      float o_cmp;
-      if (p.sp_keep_p != nullptr) {  // merged in the prologue
-        const float o = ocmp_pre[r];
-        if (p.cmp_o) p.cmp_o[(int64_t)b * p.co_st + (int64_t)hq * p.co_sh + d] = (bf16_t)o;
-        o_cmp = (float)(bf16_t)o;
-      } else {
-        o_cmp = (float)p.cmp_o[(int64_t)b * p.co_st + (int64_t)hq * p.co_sh + d];
-      }
-      p.out[(int64_t)b * p.o_st + (int64_t)hq * p.o_sh + d] = (bf16_t)(o_cmp * s0 + o_slc * s1 + o_swa * s2);
-    }
+  for (int r = 0; r < OPT; r++) { slc[r] = (bf16_t)o_slc[r]; swa[r] = (bf16_t)o_swa_pre[r]; }
+  if (p.slc_o) *reinterpret_cast<bvecu*>(p.slc_o + co) = slc;
+  if (p.swa_o) *reinterpret_cast<bvecu*>(p.swa_o + co) = swa;
+  if (p.sp_keep_p != nullptr) {  // merged in the prologue
+#pragma unroll
+    for (int r = 0; r < OPT; r++) cmp[r] = (bf16_t)ocmp_pre[r];
+    if (p.cmp_o) *reinterpret_cast<bvecu*>(p.cmp_o + co) = cmp;
+  } else if (p.out) {
+    cmp = *reinterpret_cast<const bvecu*>(p.cmp_o + co);
+  }
+  if (p.out) {
+    bvecu o;
+#pragma unroll
+    for (int r = 0; r < OPT; r++)
+      o[r] = (bf16_t)((float)cmp[r] * gate[0] + (float)slc[r] * gate[1] + (float)swa[r] * gate[2]);
+    *reinterpret_cast<bvecu*>(p.out + (int64_t)b * p.o_st + (int64_t)hq * p.o_sh + od) = o;
   }
 }
 
@@ -1184,19 +1297,9 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_fused_kernel(NsaDecodeParam
       if (pool_now) {
         const int32_t* tab = p.table + (int64_t)b * p.table_stride;
         const int st = ((L - p.kernel_size) / p.stride) * p.stride;
-        float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int r = 0; r < p.kernel_size; r++) {
-          const int n = st + r;
-          bf16x8 x;
-          if (raw_slot >= 0 && n == L - 1) {
-            x = newest;  // the row just stored: taken from the register, not read back
-          } else {
-            const int64_t row = (int64_t)tab[n / page] * page + (n % page);
-            x = ld_global_b128(cache + row * c_sr + (int64_t)kh * c_sh + lane * 8);
-          }
-#pragma unroll
-          for (int e = 0; e < 8; e++) a[e] += (float)x[e];
-        }
+        float a[8];
+        sum_rows(a, cache + (int64_t)kh * c_sh + lane * 8, c_sr, tab, page, st, p.kernel_size,
+                 raw_slot >= 0 ? L - 1 : -1, newest);
         const float inv = 1.f / (float)p.kernel_size;
         *reinterpret_cast<bf16x8*>(cache + (int64_t)cmp_slot * c_sr + (int64_t)kh * c_sh + lane * 8) =
             pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -1418,7 +1521,8 @@ int nsa_decode_slc_swa_launch(const NsaDecodeParams& p, int B, int D, int VD, hi
 
 template <int D, int VD>
 static int launch_cmp_partial(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
-  const int ntab = (p.y_cap + p.page_size - 1) / p.page_size;
+  const int ntab = std::max((p.y_cap + p.page_size - 1) / p.page_size,
+                            p.win_parts > 0 ? p.window / p.page_size + 2 : 0);
   return launch_dyn(decode_cmp_partial_kernel<D, VD>, grid, SPLIT_WAVES,
                     slot_bytes<D, VD>(SPLIT_WAVES) + (size_t)(2 * SPLIT_WAVES * 16 + ntab) * 4, stream,
                     "decode_cmp_partial_kernel", 0, p);
@@ -1465,7 +1569,7 @@ int nsa_decode_split_static_lds_bytes() { return (int)SLC_SWA_STATIC_LDS; }
 template <int D, int VD>
 static int launch_split(const NsaDecodeParams& p, int B, size_t lds2, hipStream_t stream) {
   const int S = p.slc_nsplit > 1 ? p.slc_nsplit : 1;
-  int rc = launch_cmp_partial<D, VD>(p, dim3(B, p.KH, p.nsplit), stream);
+  int rc = launch_cmp_partial<D, VD>(p, dim3(B, p.KH, p.nsplit + p.win_parts), stream);
   if (rc) return rc;
   rc = launch_slc_swa<D, VD>(p, dim3(B, p.KH, S), lds2, stream);
   if (rc || S == 1) return rc;

@@ -9,6 +9,7 @@
 #include <mutex>
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include "../../include/nsa_hip.h"
 
 namespace {
 
@@ -84,17 +85,6 @@ ScratchLayout layout(int B, int KH, int VD, int nsplit, int fixed_y_maxlen) {
 
 extern "C" {
 
-int nsa_decode_split(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
-                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
-                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
-                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
-                     int64_t tk_st, float* sp_m, float* sp_l, float* sp_o, void* sp_keep_p, float* sp_keep_m,
-                     int nsplit, const int32_t* cmp_slot_mapping, const int32_t* context_lens,
-                     const int32_t* block_tables, int table_stride, const int32_t* cmp_block_tables,
-                     int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
-                     int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
-                     int num_local, int ignore_index, int window, float sm_scale, void* stream);
-
 int64_t nsa_decode_split_static_capacity(void) { return (int64_t)STATIC_SCRATCH_BYTES; }
 
 int64_t nsa_decode_split_static_bytes(int B, int KH, int VD, int nsplit, int fixed_y_maxlen) {
@@ -127,13 +117,18 @@ int nsa_decode_split_static(const void* q, int64_t q_st, int64_t q_sh, const voi
   unsigned char* base = nullptr;
   int rc = scratch_base(out, &base);
   if (rc) return rc;
-  return nsa_decode_split(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, w, w_st, w_sh, out, o_st, o_sh,
+  // the window parts take what the array has left; a call that leaves too little attends the window in the second launch
+  int parts = nsa_decode_split_window_parts(window, fixed_y_maxlen, nsplit);
+  const size_t win_ml = round256(2 * (size_t)B * KH * parts * 16 * sizeof(float));
+  if (s.total + win_ml + (size_t)B * KH * parts * 16 * VD * sizeof(float) > STATIC_SCRATCH_BYTES) parts = 0;
+  return nsa_decode_split_window(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, w, w_st, w_sh, out, o_st, o_sh,
                           cmp_o, slc_o, swa_o, co_st, co_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st,
                           (float*)(base + s.m), (float*)(base + s.l), (float*)(base + s.o), base + s.keep_p,
                           (float*)(base + s.keep_m), nsplit, cmp_slot_mapping, context_lens, block_tables,
                           table_stride, cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD,
                           fixed_y_maxlen, fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init,
-                          num_local, ignore_index, window, sm_scale, stream);
+                          num_local, ignore_index, window, sm_scale, parts, (float*)(base + s.total),
+                          (float*)(base + s.total + win_ml), stream);
 }
 
 }  // extern "C"

@@ -64,6 +64,9 @@ def auto_cmp_splits(batch, num_kv_heads, fixed_y_maxlen, num_cus=256, one_launch
       16 x 128K 192 / 127 / 114 / 114, 32 x 64K 140 / 111 / 119 / 126, 32 x 128K 240 / 185 / 188 / 191;
       8 / 16 / 32 / 64 parts: 1 x 128K 61.3 / 58.8 / 61.1 / 69.1, 2 x 128K 64.8 / 62.7 / 65.9 / 76.8, 4 x 128K
       67.9 / 68.3 / 76.7 / 89.6 -- 16 parts pay for up to 8 pairs.
+      (With the later, shorter kernels of both paths the lines stay where they were: 1 / 2 / 4 / 8 parts, capacity 2048,
+      16 pairs: 32K tokens 47 / 45 / 40 / 38, 4K 29 / 34 / 32 / 31; 32 pairs: 49 / 46 / 43 / 42 and 30 / 35 / 34 / 34;
+      capacity 8192, 64 pairs: 32K 76 / 49 / 48 / 51.)
     192 q/k channels (2 kv heads, four waves in the one-launch kernel whatever the capacity, 1 / 2 / 4 / 8 / 16 parts):
       16 x 1K-32K 72 / 63 / 63 / 59 / 64, 32 x 1K-32K 80 / 70 / 70 / 71 / 80, 64 x 4K 67 / 66 / 70 / 68 / 82, 64 x 1K-32K
       92 / 88 / 87 / 94 / 115, 128 x 4K-32K 127 / 137 / 127 / 139 / 173; capacity 8192: 4 x 128K 148 / 109 / 87 / 71 / 68,
@@ -135,18 +138,12 @@ def nsa_decode(q, k, v, w, context_lens, block_tables, cmp_slot_mapping, cmp_blo
     if (fused_decode_supported(q, k, v) and cmp_num_splits > 1 and
             decode_split_fits(q, k, v, block_tables, fixed_y_maxlen, fixed_num_slc_blocks)):
         # small batches of long contexts: the compressed branch is cut in that many key-interleaved parts per
-        # (request, kv head); two launches.  From 8 requests on the first of them also pools the newest compressed
-        # row (2 us less than the pooling launch at 16-32 requests); below that the pooling, which sits in front of
-        # the one workgroup that owns the last unit, costs more than its launch (46 -> 49 us for one request).
-        fuse_pool = q.size(0) >= 8
-        if not fuse_pool:
-            kv_mean_pooling_decode(k, v, block_table=block_tables, slot_mapping=cmp_slot_mapping,
-                                   context_lens=context_lens, kernel_size=kernel_size, stride=stride)
+        # (request, kv head); two launches, the first of which also pools the newest compressed row
         return decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nsplit=cmp_num_splits,
                             fixed_y_maxlen=fixed_y_maxlen, fixed_num_slc_blocks=fixed_num_slc_blocks,
                             kernel_size=kernel_size, stride=stride, block_size=block_size, top_n=top_n,
                             num_inital=num_init_blocks, num_local=num_local_blocks, window_size=window_size,
-                            sm_scale=sm_scale, cmp_slot_mapping=cmp_slot_mapping if fuse_pool else None,
+                            sm_scale=sm_scale, cmp_slot_mapping=cmp_slot_mapping,
                             slc_nsplit=max(1, min(int(slc_num_splits), 16)))
     kv_mean_pooling_decode(k, v, block_table=block_tables, slot_mapping=cmp_slot_mapping, context_lens=context_lens,
                            kernel_size=kernel_size, stride=stride)

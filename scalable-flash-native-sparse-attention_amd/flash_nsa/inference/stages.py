@@ -407,8 +407,12 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
             return out, parts[0], parts[1], parts[2], topk, lse
         return out
     ycap32 = (int(fixed_y_maxlen) + 31) // 32 * 32
-    sp_ml = torch.empty(2, B, KH, nsplit, 16, device=dev, dtype=torch.float32)
-    sp_o = torch.empty(B, KH, nsplit, 16, VD, device=dev, dtype=torch.float32)
+    # one fp32 buffer: m, l and o of the parts of the compressed branch, then of the window's
+    n_win = 0 if slc_nsplit > 1 else _lib.value("nsa_decode_split_window_parts", window_size, int(fixed_y_maxlen), nsplit)
+    n_sp, n_wp = B * KH * nsplit * 16, B * KH * n_win * 16
+    sp = torch.empty((n_sp + n_wp) * (2 + VD), device=dev, dtype=torch.float32)
+    sp_ptr = sp.data_ptr()
+    win_ptr = sp_ptr + 4 * n_sp * (2 + VD)
     # 192 q/k channels: the probabilities of the block scores stay fp32
     keep_p = torch.empty(B, KH, 16, ycap32, device=dev, dtype=torch.float16 if D <= 128 else torch.float32)
     keep_m = torch.empty(B, KH, ycap32 // 32, 16, device=dev, dtype=torch.float32)
@@ -417,7 +421,7 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
             _lib.ptr(parts[0]), _lib.ptr(parts[1]), _lib.ptr(parts[2]), out.stride(0), out.stride(1),
             _lib.ptr(lse), lse.stride(0) if return_parts else 0, lse.stride(1) if return_parts else 0,
             _lib.ptr(topk), topk.stride(0) if return_parts else 0, topk.stride(1) if return_parts else 0,
-            sp_ml[0].data_ptr(), sp_ml[1].data_ptr(), sp_o.data_ptr(), keep_p.data_ptr(), keep_m.data_ptr(), nsplit,
+            sp_ptr, sp_ptr + 4 * n_sp, sp_ptr + 8 * n_sp, keep_p.data_ptr(), keep_m.data_ptr(), nsplit,
             _lib.ptr(None if cmp_slot_mapping is None else _i32(cmp_slot_mapping)), _i32(context_lens).data_ptr(),
             _i32(block_tables).data_ptr(), block_tables.stride(0),
             _i32(cmp_block_tables).data_ptr(), cmp_block_tables.stride(0), page, B, QH, KH, D, VD,
@@ -430,7 +434,7 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
         _lib.call("nsa_decode_split_parts", *args, int(slc_nsplit), sp2_ml.data_ptr(), sp2_o.data_ptr(),
                   cmp_tmp.data_ptr(), _lib.stream_ptr())
     else:
-        _lib.call("nsa_decode_split", *args, _lib.stream_ptr())
+        _lib.call("nsa_decode_split_window", *args, n_win, win_ptr, win_ptr + 8 * n_wp, _lib.stream_ptr())
     if return_parts:
         return out, parts[0], parts[1], parts[2], topk, lse
     return out

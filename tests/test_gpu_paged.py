@@ -569,6 +569,65 @@ def test_split_decode_with_window_and_selected_blocks_in_parts(device, QH, KH, D
     assert torch.equal(got[0], out2), "optional outputs must not change the result"
 
 
+@pytest.mark.parametrize("window,num_init,num_local,top_n", [(0, 1, 2, 16), (31, 0, 0, 4), (513, 2, 5, 7), (3000, 1, 2, 8)])
+@pytest.mark.parametrize("QH,KH,D,VD", [(64, 4, 128, 128), (12, 2, 64, 64), (16, 2, 192, 128)])
+def test_split_decode_attends_the_window_in_the_first_launch(device, monkeypatch, QH, KH, D, VD, window, num_init,
+                                                             num_local, top_n):
+    """win_parts 1..4 against 0 (window in the second launch): selection, lse and compressed branch bit for bit; the
+    other branches sum the same partial results in another order (one bf16 rounding of either side apart).  Windows that
+    end with a unit and that do not, shorter and longer than the context, all or none of the selection forced."""
+    from flash_nsa import _lib
+    from flash_nsa.inference import decode_split
+    ctx = [4096, 333, 48, 31, 1, 777, 2999, 65, 0, 513, 514]
+    case = build_pool([max(c, 1) for c in ctx], KH, D, VD, page=64, seed=71)
+    prepool(case, [max(c, 1) for c in ctx])
+    d = to_dev(case, device)
+    q, w = randn_bf16(len(ctx), QH, D, seed=72).to(device), randn_bf16(len(ctx), QH, 3, seed=73).to(device)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32, device=device)
+    live = ctx_t > 0
+    value = _lib.value
+
+    def run(parts):
+        monkeypatch.setattr(_lib, "value", lambda name, *a: parts if name == "nsa_decode_split_window_parts" else value(name, *a))
+        return decode_split(q, d["k"], d["v"], w, d["bt"], d["cbt"], ctx_t, return_parts=True, nsplit=3, fixed_y_maxlen=512,
+                            fixed_num_slc_blocks=64, top_n=top_n, window_size=window, num_inital=num_init,
+                            num_local=num_local)
+
+    ref = run(0)
+    for parts in (1, 2, 3, 4):
+        got = run(parts)
+        for i in (4, 5, 1):
+            a, b = (got[i][:, live], ref[i][:, live]) if i == 4 else (got[i][live], ref[i][live])
+            assert torch.equal(a, b), (parts, i)
+        assert_close(got[2][live], ref[2][live], "slc_o", atol=4e-3, rtol=1e-2)
+        assert_close(got[3][live], ref[3][live], "swa_o", atol=4e-3, rtol=1e-2)
+        assert_close(got[0][live], ref[0][live], "o", atol=8e-3, rtol=1e-2)
+        assert float(got[0][~live].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("kernel_size,stride,block", [(128, 64, 128), (32, 16, 64), (16, 16, 32)])
+def test_decode_kernels_pool_like_the_pooling_kernel(device, kernel_size, stride, block):
+    """The row that the decode kernels pool themselves, for windows longer than a page, inside one, across two and shorter
+    than a batch of fetched rows: the pools equal those of the pooling launch bit for bit."""
+    from flash_nsa.inference import decode_one_launch, decode_split, kv_mean_pooling_decode
+    QH, KH, D, page = 16, 1, 128, 64
+    ctx = [n * stride + kernel_size for n in (0, 1, 3, 9, 30)]
+    case = build_pool(ctx, KH, D, D, page=page, seed=81)
+    slots = torch.tensor([int(case["cbt"][b, 0]) * page + 5 for b in range(len(ctx))], dtype=torch.int32, device=device)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32, device=device)
+    q, w = randn_bf16(len(ctx), QH, D, seed=82).to(device), randn_bf16(len(ctx), QH, 3, seed=83).to(device)
+    d = [to_dev(case, device) for _ in range(3)]
+    for x in d:
+        x["k"], x["v"] = x["k"].clone(), x["v"].clone()
+    sizes = dict(kernel_size=kernel_size, stride=stride)
+    kw = dict(fixed_y_maxlen=512, fixed_num_slc_blocks=64, block_size=block, cmp_slot_mapping=slots, **sizes)
+    kv_mean_pooling_decode(d[0]["k"], d[0]["v"], block_table=d[0]["bt"], slot_mapping=slots, context_lens=ctx_t, **sizes)
+    decode_split(q, d[1]["k"], d[1]["v"], w, d[1]["bt"], d[1]["cbt"], ctx_t, nsplit=2, **kw)
+    decode_one_launch(q, d[2]["k"], d[2]["v"], w, d[2]["bt"], d[2]["cbt"], ctx_t, **kw)
+    for x in d[1:]:
+        assert torch.equal(d[0]["k"], x["k"]) and torch.equal(d[0]["v"], x["v"])
+
+
 def test_one_launch_decode_pools_the_new_row_itself(device):
     """nsa_decode's one-launch kernel with a slot mapping == pooling kernel followed by the same kernel without:
     the pools end bit-identical and so do the outputs."""
