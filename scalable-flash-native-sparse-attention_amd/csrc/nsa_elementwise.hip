@@ -15,6 +15,40 @@ NSA_DEVICE void acc8(float* a, bf16x8 v) {
 #pragma unroll
   for (int e = 0; e < 8; e++) a[e] += (float)v[e];
 }
+// Sum of K rows in row order, fetched eight at a time: one by one they are K round trips to memory, which is what bounds
+// the pooling of all but the longest batches (K and V, us, one by one -> so: 4K tokens, 1 kv head 28 -> 14; 16K tokens, 2
+// kv heads 33 -> 17; chunks of 16 x 2K tokens behind prefixes 67 -> 33; three short prompts with the cache write 15 -> 8.5).
+template <class RowPtr>
+NSA_DEVICE void sum_rows(float* a, int K, RowPtr ptr) {
+  for (int r = 0; r < K; r += 8) {
+    bf16x8 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = ld_global_b128(ptr(min(r + u, K - 1)));
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (r + u < K) acc8(a, x[u]);
+  }
+}
+// row number in the pool of K consecutive positions from st on: a window of at most a page touches two pages, whose table
+// entries are read once and without a division per row.  Positions from `end` on are not looked up.
+struct PagedRows {
+  const int32_t* tb;
+  int st, page, off;
+  bool two;
+  int64_t row0, row1;
+  NSA_DEVICE PagedRows(const int32_t* tb_, int st_, int K, int page_, int end = 0x7fffffff)
+      : tb(tb_), st(st_), page(page_), off(0), two(K <= page_), row0(0), row1(0) {
+    if (!two || st >= end) return;
+    const int p0 = st / page;
+    off = st - p0 * page;
+    row0 = (int64_t)tb[p0] * page + off;
+    row1 = off + min(K, end - st) > page ? (int64_t)tb[p0 + 1] * page + off - page : row0;
+  }
+  NSA_DEVICE int64_t operator()(int r) const {
+    if (two) return (off + r < page ? row0 : row1) + r;
+    return (int64_t)tb[(st + r) / page] * page + (st + r) % page;
+  }
+};
 NSA_DEVICE float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 
 // ------------------------------------------------------------------------------------------ mean pooling fwd
@@ -33,7 +67,7 @@ __global__ void mean_pool_fwd_kernel(const bf16_t* x, int64_t x_st, int64_t x_sh
   int i = idx / ((int64_t)C * H);
   float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   const bf16_t* xp = x + (int64_t)(x0 + (int64_t)S * i) * x_st + (int64_t)h * x_sh + c * 8;
-  for (int r = 0; r < K; r++) acc8(a, ld_global_b128(xp + r * x_st));
+  sum_rows(a, K, [&](int r) { return xp + r * x_st; });
   float inv = 1.f / (float)K;
   *reinterpret_cast<bf16x8*>(y + (int64_t)(y0 + i) * y_st + (int64_t)h * y_sh + c * 8) =
       pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -323,11 +357,9 @@ __global__ void paged_pool_prefill_kernel(bf16_t* cache, int64_t c_sr, int64_t c
   if (slot < 0) return;
   const int32_t* tb = table + (int64_t)b * table_stride;
   float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int r = 0; r < K; r++) {
-    int n = S * i + r;
-    int64_t row = (int64_t)tb[n / page] * page + (n % page);
-    acc8(a, ld_global_b128(cache + row * c_sr + (int64_t)h * c_sh + c * 8));
-  }
+  const PagedRows row(tb, S * i, K, page);
+  const bf16_t* col = cache + (int64_t)h * c_sh + c * 8;
+  sum_rows(a, K, [&](int r) { return col + row(r) * c_sr; });
   float inv = 1.f / (float)K;
   *reinterpret_cast<bf16x8*>(cache + (int64_t)slot * c_sr + (int64_t)h * c_sh + c * 8) =
       pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -352,31 +384,9 @@ __global__ void paged_pool_decode_kernel(bf16_t* kc, int64_t k_sr, int64_t k_sh,
   const int st = ((L - K) / S) * S;
   const int32_t* tb = table + (int64_t)b * table_stride;
   float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (K <= page) {
-    // the window touches at most two pages: both table entries are read up front, then the rows are fetched eight at
-    // a time (independent loads) and added in row order
-    const int p0 = st / page, r0 = st - p0 * page;
-    const int64_t base0 = (int64_t)tb[p0] * page + r0;
-    const int64_t base1 = r0 + K > page ? (int64_t)tb[p0 + 1] * page + r0 - page : base0;
-    const bf16_t* col = cache + (int64_t)h * c_sh + c * 8;
-    for (int r = 0; r < K; r += 8) {
-      bf16x8 x[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int rr = min(r + u, K - 1);
-        x[u] = ld_global_b128(col + ((r0 + rr < page ? base0 : base1) + rr) * c_sr);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (r + u < K) acc8(a, x[u]);
-    }
-  } else {
-    for (int r = 0; r < K; r++) {
-      int n = st + r;
-      int64_t row = (int64_t)tb[n / page] * page + (n % page);
-      acc8(a, ld_global_b128(cache + row * c_sr + (int64_t)h * c_sh + c * 8));
-    }
-  }
+  const PagedRows row(tb, st, K, page);
+  const bf16_t* col = cache + (int64_t)h * c_sh + c * 8;
+  sum_rows(a, K, [&](int r) { return col + row(r) * c_sr; });
   float inv = 1.f / (float)K;
   *reinterpret_cast<bf16x8*>(cache + (int64_t)slot * c_sr + (int64_t)h * c_sh + c * 8) =
       pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -436,15 +446,10 @@ __global__ void paged_store_pool_prefill_kernel(const bf16_t* key, int64_t k_st,
     if (slot < 0) return;
     const int32_t* tb = table + (int64_t)b * table_stride;
     float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int r = 0; r < K; r++) {
-      const int n = S * i + r;
-      if (n >= cached) {
-        acc8(a, ld_global_b128(src + (int64_t)(x0 + n - cached) * s_st + (int64_t)h * s_sh + c * 8));
-      } else {
-        const int64_t row = (int64_t)tb[n / page] * page + (n % page);
-        acc8(a, ld_global_b128(cache + row * c_sr + (int64_t)h * c_sh + c * 8));
-      }
-    }
+    const PagedRows row(tb, S * i, K, page, cached);
+    const bf16_t* fresh = src + (int64_t)(x0 + S * i - cached) * s_st + (int64_t)h * s_sh + c * 8;
+    const bf16_t* pool = cache + (int64_t)h * c_sh + c * 8;
+    sum_rows(a, K, [&](int r) { return S * i + r >= cached ? fresh + r * s_st : pool + row(r) * c_sr; });
     const float inv = 1.f / (float)K;
     *reinterpret_cast<bf16x8*>(cache + (int64_t)slot * c_sr + (int64_t)h * c_sh + c * 8) =
         pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);

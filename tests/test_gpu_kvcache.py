@@ -5,6 +5,7 @@ import torch
 
 from oracle import nsa_oracle as O
 from gpu_util import assert_close, randn_bf16
+from paged_util import build_pool
 
 pytestmark = pytest.mark.gpu
 
@@ -52,6 +53,50 @@ def test_fused_store_and_pool_prefill_equals_store_then_pool(device):
                                        st["cmp_slot_mapping"], st["block_tables"])
         assert torch.equal(k1, k2) and torch.equal(v1, v2), f"chunk {chunk}"
     assert float(k1.abs().sum()) > 0
+
+
+@pytest.mark.parametrize("K,S", [(32, 16), (128, 64), (24, 8), (4, 4)])
+def test_prefill_pooling_is_the_row_order_sum(device, K, S):
+    """Windows inside a page, across two, longer than one, and not a multiple of the rows fetched together: every pooled
+    row is the fp32 sum of its rows in row order times 1 / K, bit for bit, with and without the cache write."""
+    from flash_nsa.inference import mean_pooling_prefill, store_kvcache_and_pool_prefill
+    KH, D, page = 2, 64, 64
+    new, cached = [K + 3 * S, 1, 200, K], [0, 70, 130, 64 - K // 2]
+    total = [n + c for n, c in zip(new, cached)]
+    case = build_pool(total, KH, D, D, page=page, seed=91, kernel=K, stride=S)
+    ys = case["ys"]
+    slots = torch.tensor([int(case["cbt"][b, i // page]) * page + i % page for b in range(4) for i in range(ys[b])])
+    raw = [torch.tensor([int(case["bt"][b, i // page]) * page + i % page for i in range(n)]) for b, n in enumerate(total)]
+    cum = lambda x: torch.tensor([0] + x).cumsum(0).to(torch.int32).to(device)
+    want = {}
+    for name in ("k", "v"):
+        flat = case[name].clone().view(-1, KH, D)
+        pos = 0
+        for b in range(4):
+            rows = flat[raw[b]].float()
+            for i in range(ys[b]):
+                acc = torch.zeros(KH, D)
+                for r in range(K):
+                    acc = acc + rows[S * i + r]
+                flat[slots[pos]] = (acc * torch.tensor(1.0 / K)).to(torch.bfloat16)
+                pos += 1
+        want[name] = flat.view_as(case[name])
+    bt, slots = case["bt"].to(device), slots.to(torch.int32).to(device)
+    pools = {name: case[name].to(device) for name in ("k", "v")}
+    for name in ("k", "v"):
+        mean_pooling_prefill(pools[name], cum(ys), max(ys), bt, slots, kernel_size=K, stride=S)
+        assert torch.equal(pools[name].cpu(), want[name])
+    # the new rows handed over instead, their places in the pool still empty
+    fresh = {name: torch.cat([case[name].view(-1, KH, D)[raw[b][cached[b]:]] for b in range(4)]).to(device) for name in ("k", "v")}
+    to = torch.cat([raw[b][cached[b]:] for b in range(4)])
+    for name in ("k", "v"):
+        pools[name] = case[name].clone()
+        pools[name].view(-1, KH, D)[to] = 0
+        pools[name] = pools[name].to(device)
+    store_kvcache_and_pool_prefill(fresh["k"], fresh["v"], pools["k"], pools["v"], cum(new), max(new),
+                                   torch.tensor(total, dtype=torch.int32, device=device), to.to(torch.int32).to(device),
+                                   cum(ys), max(ys), slots, bt, kernel_size=K, stride=S)
+    assert torch.equal(pools["k"].cpu(), want["k"]) and torch.equal(pools["v"].cpu(), want["v"])
 
 
 @pytest.mark.parametrize("QH,KH,D,caps", [(64, 4, 128, (512, 64)), (16, 2, 128, (8192, 2048))])
