@@ -56,13 +56,14 @@ int nsa_combine_fwd(const void* a, const void* b, const void* c, int64_t i_st, i
 int nsa_combine_bwd(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
                     int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
                     void* dc, void* dw, float* delta3, int64_t T, int H, int D, void* stream);
-/* the same with b = selected and c = window branch, folding the selected branch's gradient over the window's keys into the
- * window's for the tokens at positions below all_below (log-sum-exps of the two branches [T,H] with strides l_st, l_sh) */
-int nsa_combine_bwd_tail(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
-                         int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
-                         void* dc, void* dw, float* delta3, const float* slc_lse, const float* swa_lse, int64_t l_st,
-                         int64_t l_sh, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D,
-                         void* stream);
+/* the same for kernels of the branches b = selected and c = window that read dy itself: da and delta3[0] as above;
+ * delta3[k] = rowsum(x_k * dy) and lse2 [2,T,H] = lse_k - log2 sigmoid(w_k) (lse_k: the branch's log-sum-exp, any strides)
+ * take the place of these branches' delta and lse.  For the tokens at positions below all_below, which select every block they can see,
+ * c's values also carry b's gradient over the window's keys */
+int nsa_combine_bwd_gates(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
+                          int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, const float* lse_b,
+                          int64_t lb_st, int64_t lb_sh, const float* lse_c, int64_t lc_st, int64_t lc_sh, void* da,
+                          void* dw, float* delta3, float* lse2, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D, void* stream);
 /* flash_nsa/ops/compress_attn.py:160-184 _bwd_preprocess: delta[T,H] fp32 = rowsum(o*do) */
 int nsa_delta(const void* o, int64_t o_st, int64_t o_sh, const void* dO, int64_t d_st, int64_t d_sh, float* delta,
               int64_t T, int H, int D, void* stream);
@@ -129,7 +130,7 @@ int nsa_slc_attn_fwd(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
                      int top_n, float sm_scale, void* stream);
 /* the same for the queries at positions >= t_begin only, as nsa_slc_attn_bwd_dq_from, nsa_paged_slc_attn_fwd_from and
  * nsa_build_inverse_index_from: the queries below top_n * block_size select every block they can see, and
- * nsa_swa_fwd_tail / nsa_swa_bwd_dq_tail / nsa_combine_bwd_tail finish their selected branch with the window's */
+ * nsa_swa_fwd_tail / nsa_swa_bwd_dq_tail / nsa_combine_bwd_gates finish their selected branch with the window's */
 int nsa_slc_attn_fwd_from(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                           const void* v, int64_t v_sr, int64_t v_sh, const int32_t* topk, int64_t tk_sh,
                           int64_t tk_st, void* o, int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st,
@@ -190,7 +191,7 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
                    const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                    int64_t delta_sh, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu,
                    int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
-/* nsa_swa_bwd_dq with dq_mode 2 (add into fp32) for gradients from nsa_combine_bwd_tail: the queries at positions below
+/* nsa_swa_bwd_dq with dq_mode 2 (add into fp32) for gradients from nsa_combine_bwd_gates: the queries at positions below
  * all_below also take the selected branch's keys before their window, and their dq is stored instead of added */
 int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                         const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
@@ -224,7 +225,7 @@ int nsa_slc_attn_bwd_dq_from(const void* q, int64_t q_st, int64_t q_sh, const vo
                         int KH, int D, int VD, int block_size, int top_n, int t_begin,
                         float sm_scale, void* stream);
 /* dk/dv of the selected branch of the queries at positions below all_below over the keys before their window, added into
- * the caller's fp32 buffers (the keys of the window are in the window branch's gradient: nsa_combine_bwd_tail).  ordered:
+ * the caller's fp32 buffers (the keys of the window are in the window branch's gradient: nsa_combine_bwd_gates).  ordered:
  * the summation order does not change between runs */
 int nsa_slc_attn_bwd_dkdv_before_window(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr,
                                         int64_t k_sh, const void* v, int64_t v_sr, int64_t v_sh, const void* dO,

@@ -240,22 +240,10 @@ __global__ void combine_fwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
 // backward: da,db,dc = dy*sig(w_k); dw_k = sig_k(1-sig_k) * sum_d dy*x_k; optional delta_k = rowsum(x_k * d x_k)
 // with the stored (bf16) d x_k, the softmax-backward correction term of branch k, written as delta[k][T][H] fp32.
 // D/8 consecutive lanes share one (t,h); D/8 must be a power of two <= 64.
-//
-// TAIL: for the tokens at positions below all_below, which select every block they can see, the selected branch b's
-// gradient over the window's keys is folded into the window branch c's.  With P_c = exp2(s - lse_c) and
-// P_b = r P_c, r = exp2(lse_c - lse_b), both branches' dS over a key of the window is
-//   P_c (dO_c . v - delta_c) + P_b (dO_b . v - delta_b) = P_c ((dO_c + r dO_b) . v - (delta_c + r delta_b)),
-// and likewise dV, so c gets dO_c + r dO_b, and what remains of b are the keys before the window.  delta_c is formed so
-// that it matches the rounded sum (b's share of it exactly, c's from what is left).
-struct CombineTail {
-  const float* lse_b; const float* lse_c; int64_t l_st, l_sh;
-  const int32_t* x_cu; int B, all_below;
-};
-template <bool TAIL>
 __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16_t* c, int64_t i_st, int64_t i_sh,
                                    const bf16_t* w, int64_t w_st, int64_t w_sh, const bf16_t* dy, int64_t dy_st,
                                    int64_t dy_sh, bf16_t* da, bf16_t* db, bf16_t* dc, bf16_t* dw, float* delta,
-                                   int64_t T, int H, int D, CombineTail tail) {
+                                   int64_t T, int H, int D) {
   const int C = D / 8;
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool ok = idx < T * H * C;
@@ -268,16 +256,6 @@ __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
   int64_t off = t * i_st + (int64_t)h * i_sh + cc * 8;
   bf16x8 va = ld_global_b128(a + off), vb = ld_global_b128(bb + off), vc = ld_global_b128(c + off);
   bf16x8 g = ld_global_b128(dy + t * dy_st + (int64_t)h * dy_sh + cc * 8);
-  float r = 0.f;  // share of b's gradient that c takes
-  if (TAIL) {
-    int lo = 0, hi = tail.B;  // last sequence that starts at or before t
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (tail.x_cu[mid] <= t) lo = mid; else hi = mid;
-    }
-    if (t - tail.x_cu[lo] < tail.all_below)
-      r = fast_exp2(tail.lse_c[t * tail.l_st + h * tail.l_sh] - tail.lse_b[t * tail.l_st + h * tail.l_sh]);
-  }
   // p_k = sum_d dy * x_k (gate gradient); q_k = sum_d round(dy * sig_k) * x_k: the correction term is formed from
   // the ROUNDED branch gradient, the one the attention backward kernels read, so that dP - delta cancels exactly
   // where a row's probabilities are one-hot (upstream forms it the same way from the stored bf16 tensors,
@@ -288,18 +266,14 @@ __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
   for (int e = 0; e < 8; e++) {
     float gf = (float)g[e];
     float xa = (float)va[e], xb = (float)vb[e], xc = (float)vc[e];
-    ra[e] = (bf16_t)(gf * s0); rb[e] = (bf16_t)(gf * s1);
-    const float b_share = TAIL ? r * (float)rb[e] : 0.f;
-    rc[e] = (bf16_t)(TAIL ? __builtin_fmaf(gf, s2, b_share) : gf * s2);
+    ra[e] = (bf16_t)(gf * s0); rb[e] = (bf16_t)(gf * s1); rc[e] = (bf16_t)(gf * s2);
     p0 += gf * xa; p1 += gf * xb; p2 += gf * xc;
-    q0 += (float)ra[e] * xa; q1 += (float)rb[e] * xb;
-    q2 += ((float)rc[e] - b_share) * xc;
+    q0 += (float)ra[e] * xa; q1 += (float)rb[e] * xb; q2 += (float)rc[e] * xc;
   }
   for (int o = C >> 1; o > 0; o >>= 1) {
     p0 += __shfl_xor(p0, o, 64); p1 += __shfl_xor(p1, o, 64); p2 += __shfl_xor(p2, o, 64);
     q0 += __shfl_xor(q0, o, 64); q1 += __shfl_xor(q1, o, 64); q2 += __shfl_xor(q2, o, 64);
   }
-  if (TAIL) q2 += r * q1;
   if (!ok) return;
   int64_t ooff = (t * H + h) * (int64_t)D + cc * 8;  // grads are contiguous [T,H,D]
   *reinterpret_cast<bf16x8*>(da + ooff) = ra;
@@ -317,6 +291,77 @@ __global__ void combine_bwd_kernel(const bf16_t* a, const bf16_t* bb, const bf16
       delta[2 * TH + t * H + h] = q2;
     }
   }
+}
+
+// The same backward for kernels of the selected branch b and the window branch c that read dy itself (the compressed branch
+// a gets its gradient da, as above).  The gradient of branch k is s_k dy (s_k its gate, one number per token and head), so
+// with P_k = exp2(S - lse_k), dP = dy . v and delta_k = rowsum(x_k * dy) its dS and the
+// operand of its dV are
+//   P_k (s_k dP - s_k delta_k) = P'_k (dP - delta_k),   s_k P_k = P'_k,   P'_k = exp2(S - (lse_k - log2 s_k)):
+// the gate goes into the log-sum-exp, and the gradients s_k dy are neither written nor rounded to bf16.
+// The tokens at positions below all_below select every block they can see.  Their selected branch b over the window's
+// keys goes into the window branch c: with r = exp2(lse_c - lse_b), P_b = r P_c there, and
+//   P_c ((s_c + r s_b) dP - (s_c delta_c + r s_b delta_b))
+// is the form above with the sum of the gates and the weighted mean of the deltas; b is left the keys before the window.
+// Folding the rounded gradients instead loses what their separate roundings average out: relative error of dq against 64
+// bits, 700 / 2300 tokens, unfolded 2.53e-3 / 2.53e-3, folded in bf16 3.17e-3 / 2.98e-3, so 2.49e-3 / 2.42e-3.  One tensor
+// is written instead of three: 64K tokens, 64 heads of 128 1398 -> 1048 us, 8 x 6K 1089 -> 741, 40 samples of up to 1.2K, 16
+// heads of 64 90 -> 55.
+struct Lse {
+  const float* p; int64_t st, sh;
+};
+__global__ void combine_bwd_gates_kernel(const bf16_t* a, const bf16_t* bb, const bf16_t* c, int64_t i_st, int64_t i_sh,
+                                         const bf16_t* w, int64_t w_st, int64_t w_sh, const bf16_t* dy, int64_t dy_st,
+                                         int64_t dy_sh, Lse lb, Lse lc, bf16_t* da, bf16_t* dw, float* delta,
+                                         float* lse, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D) {
+  const int C = D / 8;
+  int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  bool ok = idx < T * H * C;
+  if (!ok) idx = T * H * C - 1;
+  int cc = idx % C;
+  int h = (idx / C) % H;
+  int64_t t = idx / ((int64_t)C * H);
+  int64_t off = t * i_st + (int64_t)h * i_sh + cc * 8;
+  bf16x8 va = ld_global_b128(a + off), vb = ld_global_b128(bb + off), vc = ld_global_b128(c + off);
+  bf16x8 g = ld_global_b128(dy + t * dy_st + (int64_t)h * dy_sh + cc * 8);
+  const bf16_t* wp = w + t * w_st + (int64_t)h * w_sh;
+  const float s0 = sigmoidf_((float)wp[0]), s1 = sigmoidf_((float)wp[1]), s2 = sigmoidf_((float)wp[2]);
+  float p0 = 0.f, p1 = 0.f, p2 = 0.f, q0 = 0.f;
+  bf16x8 ra;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    float gf = (float)g[e];
+    ra[e] = (bf16_t)(gf * s0);
+    p0 += gf * (float)va[e]; p1 += gf * (float)vb[e]; p2 += gf * (float)vc[e];
+    q0 += (float)ra[e] * (float)va[e];
+  }
+  for (int o = C >> 1; o > 0; o >>= 1) {
+    p0 += __shfl_xor(p0, o, 64); p1 += __shfl_xor(p1, o, 64); p2 += __shfl_xor(p2, o, 64);
+    q0 += __shfl_xor(q0, o, 64);
+  }
+  if (!ok) return;
+  *reinterpret_cast<bf16x8*>(da + (t * H + h) * (int64_t)D + cc * 8) = ra;
+  if (cc != 0) return;
+  const float l1 = lb.p[t * lb.st + h * lb.sh], l2 = lc.p[t * lc.st + h * lc.sh];
+  bf16_t* dwp = dw + (t * H + h) * 3;
+  dwp[0] = (bf16_t)(s0 * (1.f - s0) * p0);
+  dwp[1] = (bf16_t)(s1 * (1.f - s1) * p1);
+  dwp[2] = (bf16_t)(s2 * (1.f - s2) * p2);
+  float sw = s2, dc = p2;
+  int lo = 0, hi = B;  // last sequence that starts at or before t
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (x_cu[mid] <= t) lo = mid; else hi = mid;
+  }
+  if (t - x_cu[lo] < all_below) {
+    const float rb = fast_exp2(l2 - l1) * s1;
+    sw = s2 + rb;
+    // (a gate of zero: P' is zero whatever delta is)
+    if (sw > 0.f) dc = p2 + (p1 - p2) * (rb / sw);
+  }
+  const int64_t TH = T * H, at = t * H + h;
+  delta[at] = q0; delta[TH + at] = p1; delta[2 * TH + at] = dc;
+  lse[at] = l1 - fast_log2(s1); lse[TH + at] = l2 - fast_log2(sw);
 }
 
 // delta[t,h] = sum_d o*do   (fp32, contiguous [T,H])
@@ -629,30 +674,30 @@ int nsa_combine_fwd(const void* a, const void* b, const void* c, int64_t i_st, i
 int nsa_combine_bwd(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
                     int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
                     void* dc, void* dw, float* delta3, int64_t T, int H, int D, void* stream) {
-  return nsa_combine_bwd_tail(a, b, c, i_st, i_sh, w, w_st, w_sh, dy, dy_st, dy_sh, da, db, dc, dw, delta3, nullptr,
-                              nullptr, 0, 0, nullptr, 0, 0, T, H, D, stream);
-}
-
-int nsa_combine_bwd_tail(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
-                         int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, void* da, void* db,
-                         void* dc, void* dw, float* delta3, const float* slc_lse, const float* swa_lse, int64_t l_st,
-                         int64_t l_sh, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D,
-                         void* stream) {
   int C = D / 8;
   NSA_REQUIRE(D % 8 == 0 && C > 0 && C <= 64 && (C & (C - 1)) == 0, NSA_ERR_BAD_ARG,
               "combine_bwd: head dim %d must be 8 * a power of two <= 512", D);
-  NSA_REQUIRE(all_below <= 0 || (slc_lse && swa_lse && x_cu && B > 0 && delta3), NSA_ERR_BAD_ARG,
-              "combine_bwd_tail: all_below needs the log-sum-exps, the sequence offsets and the delta output");
   if (T <= 0) return NSA_OK;
-  const CombineTail tail{slc_lse, swa_lse, l_st, l_sh, x_cu, B, all_below};
-  auto launch = [&](auto kern) {
-    kern<<<blocks_for(T * H * C, 256), 256, 0, (hipStream_t)stream>>>(
-        (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)c, i_st, i_sh, (const bf16_t*)w, w_st, w_sh,
-        (const bf16_t*)dy, dy_st, dy_sh, (bf16_t*)da, (bf16_t*)db, (bf16_t*)dc, (bf16_t*)dw, delta3, T, H, D, tail);
-  };
-  if (all_below > 0) launch(combine_bwd_kernel<true>);
-  else launch(combine_bwd_kernel<false>);
+  combine_bwd_kernel<<<blocks_for(T * H * C, 256), 256, 0, (hipStream_t)stream>>>(
+      (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)c, i_st, i_sh, (const bf16_t*)w, w_st, w_sh, (const bf16_t*)dy,
+      dy_st, dy_sh, (bf16_t*)da, (bf16_t*)db, (bf16_t*)dc, (bf16_t*)dw, delta3, T, H, D);
   return nsa_check_launch("combine_bwd");
+}
+
+int nsa_combine_bwd_gates(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
+                          int64_t w_st, int64_t w_sh, const void* dy, int64_t dy_st, int64_t dy_sh, const float* lse_b,
+                          int64_t lb_st, int64_t lb_sh, const float* lse_c, int64_t lc_st, int64_t lc_sh, void* da,
+                          void* dw, float* delta3, float* lse2, const int32_t* x_cu, int B, int all_below, int64_t T, int H, int D, void* stream) {
+  int C = D / 8;
+  NSA_REQUIRE(D % 8 == 0 && C > 0 && C <= 64 && (C & (C - 1)) == 0, NSA_ERR_BAD_ARG,
+              "combine_bwd_gates: head dim %d must be 8 * a power of two <= 512", D);
+  NSA_REQUIRE(lse_b && lse_c && delta3 && lse2 && x_cu && B > 0, NSA_ERR_BAD_ARG,
+              "combine_bwd_gates: the log-sum-exps, the sequence offsets and the two outputs are required");
+  if (T <= 0) return NSA_OK;
+  combine_bwd_gates_kernel<<<blocks_for(T * H * C, 256), 256, 0, (hipStream_t)stream>>>(
+      (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)c, i_st, i_sh, (const bf16_t*)w, w_st, w_sh, (const bf16_t*)dy,
+      dy_st, dy_sh, Lse{lse_b, lb_st, lb_sh}, Lse{lse_c, lc_st, lc_sh}, (bf16_t*)da, (bf16_t*)dw, delta3, lse2, x_cu, B, all_below, T, H, D);
+  return nsa_check_launch("combine_bwd_gates");
 }
 
 int nsa_delta(const void* o, int64_t o_st, int64_t o_sh, const void* dO, int64_t d_st, int64_t d_sh, float* delta,

@@ -13,7 +13,7 @@ from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
 from ..ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
-from ..ops.combine import combine_bwd
+from ..ops.combine import combine_bwd_gates
 from ..ops.sliding_window_attention import swa_fwd_tail, swa_bwd, swa_bwd_dq_tail
 
 
@@ -140,12 +140,12 @@ class NSAFunction(torch.autograd.Function):
         if slc_o is None or swa_o is None:
             (slc_o, slc_lse), (swa_o, swa_lse), _ = slc_swa_fwd(q, k, v, topk, sm_scale, helper)
 
-        # the combine backward also yields rowsum(branch * dbranch) of the three branches, and folds what the selected
-        # branch of the first all_below tokens of a sequence has in common with the window branch into the latter
+        # the kernels of the selected and the window branch read do itself, with the gates in their log-sum-exps; what the
+        # selected branch of the first all_below tokens of a sequence has in common with the window branch is folded into
+        # the latter
         all_below = helper.all_below()
-        dcmp_o, dslc_o, dswa_o, dw, delta = combine_bwd(cmp_o, slc_o, swa_o, combine_weight, do, return_delta=True,
-                                                        all_below=all_below, slc_lse=slc_lse, swa_lse=swa_lse,
-                                                        helper=helper)
+        dcmp_o, dw, delta, (lse_slc, lse_swa) = combine_bwd_gates(cmp_o, slc_o, swa_o, combine_weight, do, slc_lse, swa_lse,
+                                                                  all_below, helper)
         dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         kw = dict(sm_scale=sm_scale, helper=helper)
 
@@ -153,17 +153,17 @@ class NSAFunction(torch.autograd.Function):
             # the selected branch (memory bound) stores, the window branch (matrix bound, with bandwidth to spare for
             # the read-modify-write) adds, or stores where the selected branch left rows out, and the compressed branch
             # adds and writes q's dtype
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, _store_into(dq32), delta=delta[1], parts="dq",
+            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, _store_into(dq32), delta=delta[1], parts="dq",
                          t_begin=all_below, **kw)
-            swa_bwd_dq_tail(q, k, v, swa_lse, dswa_o, delta[2], slc_lse, dslc_o, delta[1], all_below, dq32, **kw)
+            swa_bwd_dq_tail(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, dq32, **kw)
             return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
                                 parts="dq", **kw)[0]
 
         def dkdv_raw():
             # the window branch writes every element of dk / dv, the selected branch then adds to them
-            _, dk, dv = swa_bwd(q, k, v, swa_o, swa_lse, dswa_o, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
-            slc_attn_bwd_dkdv_before_window(q, k, v, slc_lse, dslc_o, delta[1], dk, dv, all_below, **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, None, dk, dv, delta=delta[1], parts="dkdv",
+            _, dk, dv = swa_bwd(q, k, v, swa_o, lse_swa, do, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
+            slc_attn_bwd_dkdv_before_window(q, k, v, lse_slc, do, delta[1], dk, dv, all_below, **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, None, dk, dv, delta=delta[1], parts="dkdv",
                          t_begin=all_below, **kw)
             return dk, dv
 

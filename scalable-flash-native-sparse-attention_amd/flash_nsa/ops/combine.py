@@ -19,13 +19,9 @@ def combine_fwd(a, b, c, w):
     return o
 
 
-def combine_bwd(a, b, c, w, do, return_delta=False, all_below=0, slc_lse=None, swa_lse=None, helper=None):
+def combine_bwd(a, b, c, w, do, return_delta=False):
     """Returns da, db, dc (contiguous [T,H,D]), dw [T,H,3] and optionally delta [3,T,H] fp32 with
-    delta[k] = rowsum(branch_k * d branch_k), which the attention backward kernels consume.
-    all_below > 0 (b = selected, c = window branch, with their log-sum-exps [T,H] and the batch's helper; needs
-    return_delta): for the tokens at positions below it, which select every block they can see, dc and delta[2] also
-    carry the selected branch's gradient over the window's keys (swa_bwd_dq_tail, slc_attn_bwd_dkdv_before_window take
-    the rest)."""
+    delta[k] = rowsum(branch_k * d branch_k), which the attention backward kernels consume."""
     T, H, D = a.shape
     assert a.stride() == b.stride() == c.stride()
     do = do if do.stride(-1) == 1 else do.contiguous()
@@ -34,19 +30,33 @@ def combine_bwd(a, b, c, w, do, return_delta=False, all_below=0, slc_lse=None, s
     dc = torch.empty_like(da)
     dw = torch.empty(T, H, 3, device=a.device, dtype=w.dtype)
     delta = torch.empty(3, T, H, device=a.device, dtype=torch.float32) if return_delta else None
-    tail = ()
-    name = "nsa_combine_bwd"
-    if all_below > 0:
-        assert slc_lse.stride() == swa_lse.stride() and return_delta
-        name = "nsa_combine_bwd_tail"
-        tail = (slc_lse.data_ptr(), swa_lse.data_ptr(), slc_lse.stride(0), slc_lse.stride(1),
-                helper.x_cu_seqlens.data_ptr(), helper.batch, all_below)
-    _lib.call(name, a.data_ptr(), b.data_ptr(), c.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(),
+    _lib.call("nsa_combine_bwd", a.data_ptr(), b.data_ptr(), c.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(),
               w.stride(0), w.stride(1), do.data_ptr(), do.stride(0), do.stride(1), da.data_ptr(), db.data_ptr(),
-              dc.data_ptr(), dw.data_ptr(), _lib.ptr(delta), *tail, T, H, D, _lib.stream_ptr())
+              dc.data_ptr(), dw.data_ptr(), _lib.ptr(delta), T, H, D, _lib.stream_ptr())
     if return_delta:
         return da, db, dc, dw, delta
     return da, db, dc, dw
+
+
+def combine_bwd_gates(a, b, c, w, do, lse_b, lse_c, all_below, helper):
+    """Backward of the gated sum for kernels of the selected branch b and the window branch c that read do itself: the
+    gate of a branch goes into its log-sum-exp (lse_b, lse_c [T,H]).
+    Returns da (the compressed branch's gradient), dw [T,H,3], delta [3,T,H] and lse [2,T,H] (fp32), which the branches'
+    backward kernels take with do.
+    For the tokens at positions below all_below, which select every block they can see, delta[2] and lse[1] also carry
+    the selected branch's gradient over the window's keys (swa_bwd_dq_tail, slc_attn_bwd_dkdv_before_window take the
+    rest)."""
+    T, H, D = a.shape
+    assert a.stride() == b.stride() == c.stride() and do.stride(-1) == 1
+    da = torch.empty(T, H, D, device=a.device, dtype=a.dtype)
+    dw = torch.empty(T, H, 3, device=a.device, dtype=w.dtype)
+    delta, lse = torch.empty(5, T, H, device=a.device, dtype=torch.float32).split((3, 2))
+    _lib.call("nsa_combine_bwd_gates", a.data_ptr(), b.data_ptr(), c.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(),
+              w.stride(0), w.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse_b.data_ptr(), lse_b.stride(0),
+              lse_b.stride(1), lse_c.data_ptr(), lse_c.stride(0), lse_c.stride(1), da.data_ptr(), dw.data_ptr(),
+              delta.data_ptr(), lse.data_ptr(), helper.x_cu_seqlens.data_ptr(), helper.batch, all_below, T, H, D,
+              _lib.stream_ptr())
+    return da, dw, delta, lse
 
 
 class _Combine(torch.autograd.Function):

@@ -562,12 +562,12 @@ def test_selected_attention_of_queries_that_select_everything(device, QH, KH, D,
     inside the first tile and far past it.  The two round P to bf16 against another running maximum, so each side's
     sum of p v is off by at most 2^-9 of the sum of p |v| (below 1 for these N(0,1) values wherever more than one p
     counts, and exact where one does), and an output by that twice plus its own rounding: 2^-8 + 2^-7 |o|.  In the
-    backward the two branches' gradients of a window key are summed before they are rounded to bf16 instead of after:
-    dP is then off by 2^-9 of the sum of |dO v| over the channels at most and 2^-9 sqrt(channels) typically (0.02),
+    backward the gathered side rounds the two branches' gradients s do to bf16, this side reads do and has the gates in
+    the log-sum-exps: dP differs by 2^-9 of the sum of |dO v| over the channels at most and 2^-9 sqrt(channels) typically (0.02),
     which dq takes times the softmax scale and |k| (0.09 x 1 to 3 at 128 channels), on either side: the bar of 2e-2
     plus 1e-2 of the row's rms covers it."""
     from flash_nsa import NSAHelper
-    from flash_nsa.ops.combine import combine_fwd, combine_bwd
+    from flash_nsa.ops.combine import combine_fwd, combine_bwd, combine_bwd_gates
     from flash_nsa.ops.compress_attn import cmp_attn_fwd
     from flash_nsa.ops.compress_kv import mean_pooling_fwd
     from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window
@@ -607,15 +607,15 @@ def test_selected_attention_of_queries_that_select_everything(device, QH, KH, D,
         swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dq=dq, parts="dq")
         _, dk, dv = swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dkv_fp32=True, parts="dkdv")
         slc_attn_bwd(q, k, v, full, so2, sl2, ds, None, dk, dv, delta=delta[1], parts="dkdv")
-        _, ds, dsw, dw2, delta = combine_bwd(cmp_o, so2, wo2, w, do, True, n, sl2, wl2, H)
+        _, dw2, delta, (ls, lw) = combine_bwd_gates(cmp_o, so2, wo2, w, do, sl2, wl2, n, H)
         assert torch.equal(dw, dw2)
         dq2 = torch.full((T, QH, D), float("nan"), device=device)
         dq2[pos >= n] = 0
-        slc_attn_bwd(q, k, v, part, so2, sl2, ds, dq2, delta=delta[1], parts="dq", t_begin=n)
-        swa_bwd_dq_tail(q, k, v, wl2, dsw, delta[2], sl2, ds, delta[1], n, dq2)
-        _, dk2, dv2 = swa_bwd(q, k, v, wo2, wl2, dsw, delta=delta[2], dkv_fp32=True, parts="dkdv")
-        slc_attn_bwd_dkdv_before_window(q, k, v, sl2, ds, delta[1], dk2, dv2, n)
-        slc_attn_bwd(q, k, v, part, so2, sl2, ds, None, dk2, dv2, delta=delta[1], parts="dkdv", t_begin=n)
+        slc_attn_bwd(q, k, v, part, so2, ls, do, dq2, delta=delta[1], parts="dq", t_begin=n)
+        swa_bwd_dq_tail(q, k, v, lw, do, delta[2], ls, do, delta[1], n, dq2)
+        _, dk2, dv2 = swa_bwd(q, k, v, wo2, lw, do, delta=delta[2], dkv_fp32=True, parts="dkdv")
+        slc_attn_bwd_dkdv_before_window(q, k, v, ls, do, delta[1], dk2, dv2, n)
+        slc_attn_bwd(q, k, v, part, so2, ls, do, None, dk2, dv2, delta=delta[1], parts="dkdv", t_begin=n)
     finally:
         NSAHelper.set_deterministic(False)
     for name, a, b in (("dq", dq2, dq), ("dk", dk2, dk), ("dv", dv2, dv)):
