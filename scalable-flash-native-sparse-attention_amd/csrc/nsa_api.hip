@@ -380,15 +380,26 @@ int nsa_cmp_attn_bwd_dq_final(const void* q, int64_t q_st, int64_t q_sh, const v
                          x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream);
 }
 
-// Time of a workgroup of the dk/dv kernel: a fixed part (K / V fragments, epilogue) plus its 64-row tiles, and how many
-// workgroups run at once (one per CU; two where 64 channels leave the kernel under 256 registers).
+// Cost model of a dk/dv work item (128 keys x some query rows, 4 waves): fixed part (K / V fragments, epilogue, summing up)
+// and time per 64-row tile, alone on a CU (tile_us) and as the CU's throughput with `per_cu` of them on it (cu_tile_us).
+// Measured on MI355X; 8 / 16 / 32 / 64 heads per kv head: nsa_bwd_dkdv_dma.hip, else nsa_bwd_dkdv.hip.
 struct DkdvCost {
-  double fixed_us, tile_us;
-  int slots;
+  double fixed_us, tile_us, cu_tile_us;
+  int per_cu;
+  int slots() const { return per_cu * nsa_device_cus(); }
+  // one of `items` work items of `tiles` tiles, as many of them on a CU as there are
+  double item(int64_t items, double tiles) const {
+    const int64_t on_cu = (items + nsa_device_cus() - 1) / nsa_device_cus();
+    const double shared = (on_cu < per_cu ? on_cu : per_cu) * cu_tile_us;
+    return fixed_us + tiles * (shared > tile_us ? shared : tile_us);
+  }
 };
-static DkdvCost dkdv_cost(int D, int VD) {
-  if (D <= 64) return {12.0, 1.9, 2 * nsa_device_cus()};
-  return {12.0, 2.55 * (D + VD) / 256.0, nsa_device_cus()};
+static DkdvCost dkdv_cost(int G, int D, int VD) {
+  const bool dma = G == 8 || G == 16 || G == 32 || G == 64;
+  if (dma && D == 128) return {14.0, 2.3, 2.03, 2};
+  if (dma && D == 64) return {13.0, 1.45, 1.13, 3};
+  if (D <= 64) return {12.0, 0.95, 0.95, 2};
+  return {12.0, 2.55 * (D + VD) / 256.0, 2.55 * (D + VD) / 256.0, 1};
 }
 
 // Query tokens per work item of the compressed dk/dv kernel when the caller leaves the choice to the library.
@@ -397,15 +408,14 @@ static int cmp_dkdv_q_chunk(int q_chunk_tokens, int B, int x_maxlen, int y_maxle
   if (q_chunk_tokens <= 0) {
     // A work item is one (128-key tile, query chunk that sees it, kv head, sequence).  The launch takes as long as its
     // longest item when there are fewer items than workgroup slots, else about all the work over the slots plus a
-    // quarter of an item for the last, partly empty round.  The chunk (a power of two in [64, 2048]) that minimises
-    // this for the longest sequence is taken.  Fitted on MI355X to sweeps of all chunks over one to forty sequences of
-    // 1K to 64K tokens, d = 64, 128, 192: within 3 % of the best chunk on average, 16 % at most (chunk 64 / 128 / 512 /
-    // 2048 on one sequence of 4096 tokens, 16 q / 1 kv heads: 58 / 98 / 345 / 1294 us; of 65536 tokens: 3.46 / 3.17 /
-    // 3.00 / 3.99 ms).
-    const DkdvCost c = dkdv_cost(D, VD);
+    // quarter of an item for the last, partly empty round.  The chunk (a power of two in [32, 2048]) that minimises
+    // this for the longest sequence is taken.  Fitted to sweeps of all chunks over one to forty sequences of 600 to 64K
+    // tokens (chunk 64 / 128 / 256 / 512 / 2048, d = 128: 16 q / 1 kv heads, 4096 tokens 53 / 86 / 157 / 304 / 1150 us;
+    // 64 / 4 heads, 16K tokens 701 / 587 / 610 / 726 / 1166 us, 64K 10.3 / 9.3 / 8.6 / 8.1 / 8.8 ms).
     const int G = QH / KH;
+    const DkdvCost c = dkdv_cost(G, D, VD);
     double best = 0.0;
-    for (int chunk = 64; chunk <= 2048; chunk *= 2) {
+    for (int chunk = 32; chunk <= 2048; chunk *= 2) {
       const int64_t nch = (x_maxlen + chunk - 1) / chunk;
       int64_t items = 0;
       double rows = 0.0;
@@ -417,9 +427,9 @@ static int cmp_dkdv_q_chunk(int q_chunk_tokens, int B, int x_maxlen, int y_maxle
       }
       items *= (int64_t)B * KH;
       rows *= (double)B * KH;
-      const double item = c.fixed_us + (double)(chunk < x_maxlen ? chunk : x_maxlen) * G / 64.0 * c.tile_us;
-      const double all = (items * c.fixed_us + rows / 64.0 * c.tile_us) / c.slots + 0.25 * item;
-      const double cost = items <= c.slots || all < item ? item : all;
+      const double item = c.item(items, (double)(chunk < x_maxlen ? chunk : x_maxlen) * G / 64.0);
+      const double all = items * c.fixed_us / c.slots() + rows / 64.0 * c.cu_tile_us / nsa_device_cus() + 0.25 * item;
+      const double cost = items <= c.slots() || all < item ? item : all;
       if (q_chunk_tokens <= 0 || cost < best) { best = cost; q_chunk_tokens = chunk; }
     }
   }
@@ -573,9 +583,9 @@ static int swa_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, i
   if (knob > 0) return knob > 16 ? 16 : knob;
   // A key tile's queries are cut while the rounds of workgroups times the time of one keeps falling (by a tenth at
   // least: every cut adds a pass over partial results).  1 / 2 / 4 / 8 / 16 chunks, their sum included, d = 128: one
-  // sequence of 4096 tokens, 16 q / 1 kv heads 408 / 212 / 128 / 77 / 87 us, 64 q / 4 kv heads 409 / 228 / 254 / 291 /
-  // 345 us; 8192 tokens, 64 q / 4 kv heads 414 / 440 / 516 / 594 / 694 us.
-  const DkdvCost c = dkdv_cost(D, VD);
+  // sequence of 4096 tokens, 16 q / 1 kv heads 365 / 196 / 110 / 70 / 63 us, 64 q / 4 kv heads 389 / 224 / 167 / 206 /
+  // 256 us; 8192 tokens, 64 q / 4 kv heads 422 / 333 / 370 / 397 / 486 us.
+  const DkdvCost c = dkdv_cost(QH / KH, D, VD);
   const int64_t wgs = (int64_t)((x_maxlen + 127) / 128) * B * KH;
   const double tiles = (128.0 + (window < x_maxlen ? window : x_maxlen)) * (QH / KH) / 64.0;
   int best = 1;
@@ -583,7 +593,7 @@ static int swa_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, i
   int64_t dk_bytes;
   for (int s = 1; s <= 16; s *= 2) {
     if (s > 1 && swa_dkdv_slot_bytes(s, B, x_maxlen, KH, D, VD, &dk_bytes) > max_bytes) break;
-    const double cost = (double)((wgs * s + c.slots - 1) / c.slots) * (c.fixed_us + tiles / s * c.tile_us);
+    const double cost = (double)((wgs * s + c.slots() - 1) / c.slots()) * c.item(wgs * s, tiles / s);
     if (s == 1 || cost < 0.9 * best_cost) { best = s; best_cost = cost; }
   }
   return best;
@@ -731,6 +741,7 @@ static int slc_attn_bwd_dkdv_impl(const void* q, int64_t q_st, int64_t q_sh, con
   p.x_cu = x_cu; p.k_cu = x_cu;
   p.csr_off = csr_off; p.csr_tok = csr_tok; p.item_off = item_off; p.blk_seq = blk_seq; p.kblk_cu = kblk_cu;
   p.nblk_total = nblk_total; p.chunk_tokens = chunk_tokens; p.block_size = block_size;
+  p.csr_sh = nblk_total + 1;
   if (!deterministic) return nsa_bwd_dkdv_launch(p, 2, B, 0, 0, D, VD, n_items_bound, (hipStream_t)stream);
   if (n_items_bound <= 0) return NSA_OK;
   const int64_t slots = nsa_bwd_dkdv_slc_slots(KH, n_items_bound, block_size);

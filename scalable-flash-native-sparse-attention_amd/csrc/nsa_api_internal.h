@@ -92,12 +92,19 @@ struct NsaBwdTileParams {
   const int32_t* x_cu;
   const int32_t* k_cu;
   // gathered (selected-attention) row lists: CSR over (kv head, global selection block)
+  // (the per-head rows of csr_off / item_off are csr_sh apart)
   const int32_t* csr_off;      // [KH][nblk_total + 1] absolute positions into csr_tok
   const int32_t* csr_tok;      // [KH * T * top_n] local token index inside its sequence, ascending per list
   const int32_t* item_off;     // [KH][nblk_total + 1] prefix of work items (list chunks)
   const int32_t* blk_seq;      // [nblk_total] sequence id of a global block
   const int32_t* kblk_cu;      // [B+1] selection-block offsets
   int nblk_total, chunk_tokens, block_size;
+  int64_t csr_sh;
+  // selected dkdv that also stores dS (see nsa_slc_bwd_dq.hip for the layout): csr_slot names the slot of the token's
+  // selection that an entry of csr_tok stands for; ds holds the tokens from global token ds_tok0 on, heads ds_sh apart
+  bf16_t* ds; int64_t ds_sh;
+  const uint8_t* csr_slot;
+  int ds_tok0, ds_ntok, ds_dump, top_n;  // ds_dump: entry for the dS of rows that stand for nothing
   int G, KH;
   float scale_log2, sm_scale;
   int kernel_size, stride, window;
@@ -116,6 +123,9 @@ struct NsaBwdTileParams {
 
 int nsa_bwd_dq_tile_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int D, int VD,
                            hipStream_t stream);
+// the kernel for 8, 16, 32 or 64 q-heads per kv head (nsa_bwd_dkdv_dma.hip), with the grid of nsa_bwd_dkdv_launch
+bool nsa_bwd_dkdv_dma_takes(const NsaBwdTileParams& p, int D, int VD);
+int nsa_bwd_dkdv_dma_launch(const NsaBwdTileParams& p, int mode, dim3 grid, int D, int VD, hipStream_t stream);
 int nsa_bwd_dkdv_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int max_k_len, int D, int VD,
                         int n_items_bound, hipStream_t stream);
 // deterministic dk / dv (dkv_mode 4): slots a launch writes, and the ordered sums over them (nsa_dkdv_reduce.hip)
@@ -144,6 +154,24 @@ struct NsaSlcBwdDqParams {
   float scale_log2, sm_scale;
 };
 int nsa_slc_bwd_dq_launch(const NsaSlcBwdDqParams& p, int B, int max_q_len, int D, int VD, hipStream_t stream);
+
+// dQ = dS K from the stored dS of the tokens tok0 .. tok0 + ntok - 1 (global token numbers)
+struct NsaSlcDqDsParams {
+  const bf16_t* k; int64_t k_sr, k_sh;
+  const bf16_t* ds; int64_t ds_sh;
+  // 0: store bf16, 1: store fp32, 2: add into fp32, 3: bf16 store of (result + fp32 dq_partial), also of the queries before
+  // t_begin (whose result is 0)
+  void* dq; int64_t dq_st, dq_sh; int dq_mode;
+  const float* dq_partial; int64_t dqp_st, dqp_sh;
+  const int32_t* topk; int64_t tk_sh, tk_st;
+  const int32_t* x_cu;
+  int B, G, KH, top_n, block_size;
+  int t_begin, tok0, ntok;
+  float sm_scale;
+};
+int nsa_slc_dq_ds_launch(const NsaSlcDqDsParams& p, int D, hipStream_t stream);
+// elements of the dS of one (token, slot), all heads of one kv head; 0: this group size has no such layout
+int64_t nsa_slc_ds_entry_elems(int G, int block_size);
 
 // fused paged decode (one query token per request)
 struct NsaDecodeParams {

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
   int b, key0, row_begin, row_end;  // rows in the group-row space of sequence b (MODE_SLC: positions in the list)
   const int32_t* list = nullptr;
   if (MODE == MODE_SLC) {
-    const int32_t* ioff = p.item_off + (int64_t)kh * (p.nblk_total + 1);
+    const int32_t* ioff = p.item_off + kh * p.csr_sh;
     const int w = blockIdx.x;
     if (w >= ioff[p.nblk_total]) return;
     int lo = 0, hi = p.nblk_total;  // last jb with ioff[jb] <= w
@@ -68,8 +68,8 @@ __global__ __launch_bounds__(NW * 64, KB == 1 && D <= 64 ? 2 : 1) void bwd_dkdv_
     b = p.blk_seq[jb];
     // a selection block wider than the workgroup's NW*32 keys is cut into sub-blocks over grid.y (same token list)
     key0 = (jb - p.kblk_cu[b]) * p.block_size + blockIdx.y * (NW * 32 * KB);
-    const int s0 = p.csr_off[(int64_t)kh * (p.nblk_total + 1) + jb];
-    const int s1 = p.csr_off[(int64_t)kh * (p.nblk_total + 1) + jb + 1];
+    const int s0 = p.csr_off[kh * p.csr_sh + jb];
+    const int s1 = p.csr_off[kh * p.csr_sh + jb + 1];
     const int a = s0 + c * p.chunk_tokens;
     list = p.csr_tok + a;
     row_begin = 0;
@@ -584,6 +584,7 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
            hipStream_t stream) {
   NsaBwdTileParams p = p0;
   constexpr bool KB2_BUILT = kb2_built(D);
+  const bool dma = nsa_bwd_dkdv_dma_takes(p, D, VD) && nsa_tuning_knob("dkdv_key_blocks", 1) != 2;
   const int kb_cmp = KB2_BUILT ? nsa_tuning_knob("dkdv_key_blocks", 1) : 1;  // 32-key blocks per wave (cmp / swa)
   if (mode == MODE_CMP) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;
@@ -596,6 +597,7 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
     }
     if (total <= 0) return NSA_OK;
     dim3 grid(total, B, p.KH);
+    if (dma) return nsa_bwd_dkdv_dma_launch(p, mode, grid, D, VD, stream);
     if constexpr (KB2_BUILT) {
       if (kb_cmp == 2) bwd_dkdv_kernel<D, VD, MODE_CMP, 4, 2><<<grid, 256, 0, stream>>>(p);
       else bwd_dkdv_kernel<D, VD, MODE_CMP, 4, 1><<<grid, 256, 0, stream>>>(p);
@@ -621,6 +623,7 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
       }
     }
     dim3 grid(cdiv_i(max_k_len, 128) * p.grid_chunks, B, p.KH);
+    if (dma) return nsa_bwd_dkdv_dma_launch(p, mode, grid, D, VD, stream);
     bwd_dkdv_kernel<D, VD, MODE_SWA, 4, 1><<<grid, 256, 0, stream>>>(p);
   } else {
     if (n_items_bound <= 0) return NSA_OK;
@@ -632,9 +635,11 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
     // waves whose 32 keys lie past the end of the block only help staging the query rows
     if (p.block_size <= 64) {
       dim3 grid(n_items_bound, 1, p.KH);
+      if (dma) return nsa_bwd_dkdv_dma_launch(p, mode, grid, D, VD, stream);
       bwd_dkdv_kernel<D, VD, MODE_SLC, 2, 1><<<grid, 128, 0, stream>>>(p);
     } else {
       dim3 grid(n_items_bound, cdiv_i(p.block_size, 128), p.KH);
+      if (dma) return nsa_bwd_dkdv_dma_launch(p, mode, grid, D, VD, stream);
       bwd_dkdv_kernel<D, VD, MODE_SLC, 4, 1><<<grid, 256, 0, stream>>>(p);
     }
   }

@@ -44,6 +44,13 @@ NSA_DEVICE f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// the lane's number, computed where it is asked for instead of living in a register
+NSA_DEVICE int lane_id() {
+  int ones = -1;
+  asm volatile("" : "+s"(ones));
+  return __builtin_amdgcn_mbcnt_hi(ones, __builtin_amdgcn_mbcnt_lo(ones, 0));
+}
+
 NSA_DEVICE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 NSA_DEVICE float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 NSA_DEVICE float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }

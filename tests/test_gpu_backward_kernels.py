@@ -1,0 +1,54 @@
+"""The dk/dv kernel for 8, 16, 32 or 64 q-heads per kv head at the sizes where it can go wrong, against the oracle with the
+rounding points of a bf16 pipeline (the bar of test_gpu_backward.py)."""
+import pytest
+import torch
+
+from oracle import nsa_oracle as O
+from gpu_util import make_cu, make_qkvw, randn_bf16, assert_close
+from test_gpu_backward import setup_helper
+
+pytestmark = pytest.mark.gpu
+
+# tiles of 64 rows = 64 / (heads per kv head) tokens, key tiles of 64 / 128: one token, just below / at / above either
+EDGES = [1, 7, 8, 9, 63, 64, 65, 127, 129, 0, 300]
+
+
+@pytest.mark.parametrize("QH,KH,D,VD", [(8, 1, 64, 64), (16, 2, 128, 128), (32, 2, 192, 128), (32, 1, 128, 128),
+                                        (64, 1, 64, 64)])
+@pytest.mark.parametrize("block_size", [32, 64, 96, 256])
+def test_dkdv_of_every_branch(device, QH, KH, D, VD, block_size):
+    """All three branches, strided q and do, selection blocks narrower and wider than a workgroup's keys."""
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
+    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
+    from flash_nsa.ops.sliding_window_attention import swa_fwd, swa_bwd
+    from flash_nsa.ops.topk import slc_topk_indices
+    cu = make_cu(EDGES)
+    T = int(cu[-1])
+    q, k, v, _ = make_qkvw(T, QH, KH, D, VD, seed=300)
+    do = randn_bf16(T, QH, VD, seed=304)
+    setup_helper(cu.to(device), block_size=block_size, top_n=3, window_size=70)
+    cfg = O.OracleConfig(block_size=block_size, top_n=3, window_size=70)
+    wide = torch.zeros(T, QH + 1, D, dtype=torch.bfloat16, device=device)  # rows of q inside rows of something wider
+    wide[:, 1:] = q.to(device)
+    qd, kd, vd, dod = wide[:, 1:], k.to(device), v.to(device), do.to(device)
+    ck, cv = mean_pooling_fwd(kd), mean_pooling_fwd(vd)
+    rounded = dict(round_dtype=torch.bfloat16, round_mma=True)
+
+    def check(name, got, ref):
+        for g, n in zip(got, ("dq", "dk", "dv")):
+            if g is not None:
+                assert_close(g, ref[n], f"{name} {n}", row_scale=n != "dq")
+
+    co, cl = cmp_attn_fwd(qd, ck, cv)
+    ref = O.branch_forward_backward("cmp", q.float(), ck.float().cpu(), cv.float().cpu(), do.float(), cu, cfg, **rounded)
+    for chunk in (32, 256):
+        check(f"cmp, chunks of {chunk}", cmp_attn_bwd(qd, ck, cv, co, cl, dod, q_chunk_tokens=chunk), ref)
+    wo, wl = swa_fwd(qd, kd, vd)
+    check("swa", swa_bwd(qd, kd, vd, wo, wl, dod, dkv_fp32=True),
+          O.branch_forward_backward("swa", q.float(), k.float(), v.float(), do.float(), cu, cfg, **rounded))
+    topk, _ = slc_topk_indices(qd, ck, cl)
+    so, sl = slc_attn_fwd(qd, kd, vd, topk)
+    ref = O.branch_forward_backward("slc", q.float(), k.float(), v.float(), do.float(), cu, cfg, topk=topk.cpu(), **rounded)
+    check("slc", slc_attn_bwd(qd, kd, vd, topk, so, sl, dod), ref)
+    check("slc, dq recomputed", (slc_attn_bwd(qd, kd, vd, topk, so, sl, dod, parts="dq")[0], None, None), ref)
