@@ -8,11 +8,12 @@
 // key-contraction slices).  Keys are gathered by the per-token block list topk[kh, t, 0 .. min(top_n, t/block+1)).
 //
 // What bounds it is the gather: 512 KB of rows per token and kv head, from L2 while the keys of the sequences in flight
-// fit there, else from the memory-side cache (13.5 TB/s of requests at 64K tokens).  Two units in flight per wave and
-// separate K and V regions bought nothing over one, and took the registers and the LDS of a second workgroup per CU at
+// fit there (then the CU's address unit is busy 86 % of the cycles, LDS 67 %), else from the memory-side cache (13.5 TB/s of
+// requests at 64K tokens).  Two units in flight per wave and separate K and V regions bought nothing over one, and took the registers and the LDS of a second workgroup per CU at
 // 192 channels: 32 heads, 16K tokens 1726 -> 1080 us; 64 heads of 128, 8 x 6K tokens 4207 -> 3920 us.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
+#include "nsa_units.h"
 
 namespace {
 
@@ -35,13 +36,8 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   // and the K rows in LDS are no longer needed: K and V take turns in one LDS region.
   constexpr int UK = 32;                      // keys per unit
   constexpr int KC = D / 32;                  // K fragments per 16-key tile
-  constexpr int VJ = (UK * (VD / 8)) / 64;    // 16-byte V loads per lane and unit
-  constexpr int KJ = (UK * (D / 8)) / 64;     // 16-byte K loads per lane and unit
   constexpr int KLD = D + NSA_LDS_PAD, VLD = VD + NSA_LDS_PAD;
   constexpr int LD = KLD > VLD ? KLD : VLD;
-  constexpr int KP = D / 8, VP = VD / 8;                                             // 16-byte pieces per row
-  constexpr int KPAT = 64 % KP == 0 ? 1 : 3, VPAT = 64 % VP == 0 ? 1 : 3;            // 192 channels: 3 * 64 = 8 * 24
-  static_assert((KPAT * 64) % KP == 0 && (VPAT * 64) % VP == 0, "");
   __shared__ __attribute__((aligned(16))) bf16_t rows_all[4 * UK * LD];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -64,8 +60,7 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   const int32_t* table = PAGED ? p.table + (int64_t)b * p.table_stride : nullptr;
   const int Bs = p.block_size;
   const int nvalid = t >= 0 ? min(p.top_n, t / Bs + 1) : 0;  // t < 0: padded request, output row = 0
-  const int upb = Bs / UK;                    // units per selection block
-  const int nu = nvalid * upb;
+  const int nu = nvalid * (Bs / UK);
   const int key_last = min(ctx - 1, t);       // last key this token may attend
 
   int g = hc * 16 + l16;
@@ -89,72 +84,37 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   float m_run = NSA_NEG_INF, l_run = 0.f;
   const float sc = p.scale_log2;
 
-  // first key of the next unit with something to attend, at or behind unit u, -1: none left; wave-uniform.  Units that
-  // start past the last attendable key (second half of the current block) and ignore values (negative ids) are skipped.
-  auto next_unit = [&](int& u) {
-    for (; u < nu; u++) {
-      const int slot = u / upb;
-      const int blk = __builtin_amdgcn_readlane(my_blk, slot);
-      const int key0 = blk * Bs + (u - slot * upb) * UK;
-      if (blk >= 0 && key0 <= key_last) {
-        u++;
-        return key0;
-      }
-    }
-    return -1;
-  };
   // K and V rows are fetched as whole 16-byte-per-lane coalesced rows (every cache line is requested once and used
   // completely) and go through wave-private LDS; the MFMA fragments are read from there.
-  // A unit's rows are fetched 64 pieces of 16 bytes at a time; after KPAT (VPAT) instructions the pieces fall on the same
-  // columns again, so the lane part of the addresses is KPAT + VPAT 32-bit offsets and the rest is wave-uniform.
-  uint32_t koff[KPAT], voff[VPAT];
+  using KRows = UnitRows<D>;
+  using VRows = UnitRows<VD>;
+  uint32_t koff[KRows::PAT], voff[VRows::PAT];
 #pragma unroll
-  for (int j = 0; j < KPAT; j++) {
-    int pc = lane + j * 64;
-    koff[j] = (uint32_t)(pc / KP) * (uint32_t)(p.k_sr * 2) + (pc % KP) * 16;
-  }
+  for (int j = 0; j < KRows::PAT; j++) koff[j] = KRows::offset(j, lane, p.k_sr);
 #pragma unroll
-  for (int j = 0; j < VPAT; j++) {
-    int pc = lane + j * 64;
-    voff[j] = (uint32_t)(pc / VP) * (uint32_t)(p.v_sr * 2) + (pc % VP) * 16;
-  }
-  // (strides whose offsets within a period, up to 16 rows, leave 32 bits take the clamped form below: 64-bit rows)
-  const bool narrow = p.k_sr < (1 << 27) && p.v_sr < (1 << 27);
-  bf16x8 kr[KJ], vr[VJ];
-  auto flat_row = [&](int key0) -> int64_t {  // flat row of the unit's first key (a unit never straddles a page)
-    if (PAGED) return (int64_t)__builtin_amdgcn_readfirstlane(table[key0 / p.page_size]) * p.page_size + (key0 % p.page_size);
-    return (int64_t)x0 + key0;
+  for (int j = 0; j < VRows::PAT; j++) voff[j] = VRows::offset(j, lane, p.v_sr);
+  KRows kr;
+  VRows vr;
+  UnitList ul;
+  // flat row of the first key of unit i (a unit never straddles a page)
+  auto flat_row = [&](int i) -> int64_t {
+    if (PAGED) return (int64_t)__builtin_amdgcn_readlane(ul.page, i) * p.page_size + __builtin_amdgcn_readlane(ul.off, i);
+    return (int64_t)x0 + __builtin_amdgcn_readlane(ul.key0, i);
   };
-  // the unit holding the causal boundary: rows past it are replaced by the boundary row (masked later)
-  auto issue_k = [&](int key0) {
-    const bf16_t* kb = p.k + flat_row(key0) * p.k_sr + (int64_t)kh * p.k_sh;
-    const int kmax = key_last - key0;  // >= 0
-    if (kmax >= UK - 1 && narrow) {
-#pragma unroll
-      for (int j = 0; j < KJ; j++)
-        kr[j] = ld_global_b128((const bf16_t*)((const char*)(kb + (j / KPAT) * (KPAT * 64 / KP) * p.k_sr) + koff[j % KPAT]));
-    } else {
-#pragma unroll
-      for (int j = 0; j < KJ; j++) {
-        int pc = lane + j * 64;
-        kr[j] = ld_global_b128(kb + (int64_t)min(pc / KP, kmax) * p.k_sr + (pc % KP) * 8);
-      }
-    }
+  // how the rows of a unit are requested: not at all, the unit is known to be full, or with the rows past the causal boundary
+  // replaced by the boundary row (masked later) and any stride
+  enum { NONE, FULL, ANY };
+  auto issue_k = [&](auto how, int i) {
+    if constexpr (decltype(how)::value == NONE) return;
+    const bf16_t* kb = p.k + flat_row(i) * p.k_sr + (int64_t)kh * p.k_sh;
+    if constexpr (decltype(how)::value == FULL) kr.load(kb, p.k_sr, koff);
+    else kr.load_clamped(kb, p.k_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
   };
-  auto issue_v = [&](int key0) {
-    const bf16_t* vb = p.v + flat_row(key0) * p.v_sr + (int64_t)kh * p.v_sh;
-    const int kmax = key_last - key0;  // >= 0
-    if (kmax >= UK - 1 && narrow) {
-#pragma unroll
-      for (int j = 0; j < VJ; j++)
-        vr[j] = ld_global_b128((const bf16_t*)((const char*)(vb + (j / VPAT) * (VPAT * 64 / VP) * p.v_sr) + voff[j % VPAT]));
-    } else {
-#pragma unroll
-      for (int j = 0; j < VJ; j++) {
-        int pc = lane + j * 64;
-        vr[j] = ld_global_b128(vb + (int64_t)min(pc / VP, kmax) * p.v_sr + (pc % VP) * 8);
-      }
-    }
+  auto issue_v = [&](auto how, int i) {
+    if constexpr (decltype(how)::value == NONE) return;
+    const bf16_t* vb = p.v + flat_row(i) * p.v_sr + (int64_t)kh * p.v_sh;
+    if constexpr (decltype(how)::value == FULL) vr.load(vb, p.v_sr, voff);
+    else vr.load_clamped(vb, p.v_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
   };
   auto lds_order = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -162,18 +122,15 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
 
-  int u = 0;
-  int key0 = next_unit(u);
-  if (key0 >= 0) { issue_k(key0); issue_v(key0); }
-  while (key0 >= 0) {
-    const int key_next = next_unit(u);
-#pragma unroll
-    for (int j = 0; j < KJ; j++) {
-      int pc = lane + j * 64;
-      *reinterpret_cast<bf16x8*>(&rows[(pc / KP) * KLD + (pc % KP) * 8]) = kr[j];
-    }
+  // Unit i, the rows of unit i + 1 being requested meanwhile.  How is fixed per copy of the code: with a branch around the
+  // requests the compiler cannot tell this unit's V rows from them and waits for both.  With the unit list in lanes: 64 heads
+  // of 128, 8 x 6K tokens 3.85 -> 3.60 ms, paged, 16 x 2K queries behind up to 16K 3.11 -> 3.06 ms; 16 heads, one sequence of
+  // 4K tokens 113 -> 109 us; 32 heads of 192, 16K tokens 1072 -> 1043 us.
+  auto unit = [&](auto how_next, int i) {
+    const int key0 = __builtin_amdgcn_readlane(ul.key0, i);
+    kr.to_lds(rows, KLD, lane);
     lds_order();
-    if (key_next >= 0) issue_k(key_next);
+    issue_k(how_next, i + 1);
     f32x4 sacc[2];
 #pragma unroll
     for (int jt = 0; jt < 2; jt++) {
@@ -183,12 +140,12 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
       for (int kc = 0; kc < KC; kc++) sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(kp + kc * 32), qf[kc], sacc[jt]);
     }
     const int kmax = key_last - key0;  // last usable key offset inside this unit
-    if (kmax < UK - 1) {               // wave-uniform: only the unit holding the causal boundary is masked
+    if (decltype(how_next)::value != FULL && kmax < UK - 1) {  // wave-uniform: the unit holding the causal boundary
 #pragma unroll
       for (int jt = 0; jt < 2; jt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          int ko = jt * 16 + kq * 4 + i;
+          int ko = jt * 16 + (lane_id() >> 4) * 4 + i;
           if (ko > kmax) sacc[jt][i] = NSA_NEG_INF;
         }
     }
@@ -218,13 +175,9 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
     }
     l_run += psum;
     lds_order();
-#pragma unroll
-    for (int j = 0; j < VJ; j++) {
-      int pc = lane + j * 64;
-      *reinterpret_cast<bf16x8*>(&rows[(pc / VP) * VLD + (pc % VP) * 8]) = vr[j];
-    }
+    vr.to_lds(rows, VLD, lane);
     lds_order();
-    if (key_next >= 0) issue_v(key_next);
+    issue_v(how_next, i + 1);
     // O^T += V^T P^T over the 32 keys of the unit
     bf16x8 pf = pack8(sacc[0][0], sacc[0][1], sacc[0][2], sacc[0][3], sacc[1][0], sacc[1][1], sacc[1][2], sacc[1][3]);
     const int kb0 = kq * 4 + (l16 >> 2);
@@ -237,7 +190,17 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
       oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
     }
     lds_order();
-    key0 = key_next;
+  };
+  for (int base = 0; base < nu; base += 64) {
+    ul = unit_list<PAGED>(my_blk, nvalid, base, Bs, key_last, table, p.page_size, lane, [](int, int, int) { return 0; });
+    if (ul.n == 0) continue;
+    const int n_full = p.k_sr < KRows::NARROW && p.v_sr < VRows::NARROW ? ul.n_full : 0;
+    int i = 0;
+    issue_k(std::integral_constant<int, ANY>{}, 0);
+    issue_v(std::integral_constant<int, ANY>{}, 0);
+    for (; i + 1 < n_full; i++) unit(std::integral_constant<int, FULL>{}, i);
+    for (; i + 1 < ul.n; i++) unit(std::integral_constant<int, ANY>{}, i);
+    unit(std::integral_constant<int, NONE>{}, i);
   }
 
   float l_tot = xrow_sum(l_run);

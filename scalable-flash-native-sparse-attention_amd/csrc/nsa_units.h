@@ -1,0 +1,90 @@
+// The 32-key units that a query token's selected blocks consist of, as a list in the lanes of a wave.
+#pragma once
+#include "nsa_common.h"
+
+// Lane i of a wave holds unit i of a list of `n` (lanes from n on: leftovers).  Made for 64 units at a time by all lanes in
+// parallel: a loop over them then reads its next unit with one readlane per number instead of finding it step by step (slot
+// and part of the block by division, skipped units, page lookup).  The unit that holds the causal boundary comes last: the
+// query's own block is among the first selected, and all others can be loaded and scored without looking at the boundary.
+struct UnitList {
+  int n;
+  int n_full;     // how many of them end at or before key_last: the first ones
+  int key0;       // first key, position inside the sequence
+  int page, off;  // paged: page id and row inside the page; else unused
+  int aux;        // caller's number of the unit (unit_list's aux_of)
+};
+
+// Units base .. base + 63 of the blocks blk[0 .. nvalid-1] (lane s: block of position s, negative: ignored), block_size /
+// 32 of them per block, without those that start behind key_last.  aux_of(position, part of the block, lanes' blk).
+template <bool PAGED, class Aux>
+NSA_DEVICE UnitList unit_list(int blk, int nvalid, int base, int block_size, int key_last, const int32_t* table, int page_size,
+                              int lane, Aux aux_of) {
+  const int upb = block_size / 32;
+  const int u = base + lane;
+  const int pos = upb == 2 ? u >> 1 : u / upb, part = u - pos * upb;
+  const int b = __shfl(blk, min(pos, 63), 64);
+  const int key0 = b * block_size + part * 32;
+  const bool ok = pos < nvalid && b >= 0 && key0 <= key_last;
+  const bool full = ok && key0 + 31 <= key_last;
+  const uint64_t mask = __builtin_amdgcn_ballot_w64(ok), mask_full = __builtin_amdgcn_ballot_w64(full);
+  UnitList l;
+  l.n = __popcll(mask);
+  l.n_full = __popcll(mask_full);
+  const uint64_t below = (1ull << lane) - 1;
+  const int before = __popcll(mask & below), before_full = __popcll(mask_full & below);
+  // (the ones that are no units behind them, so that every lane is written)
+  const int dest = (full ? before_full : ok ? l.n_full + before - before_full : l.n + lane - before) * 4;
+  l.key0 = __builtin_amdgcn_ds_permute(dest, key0);
+  l.aux = __builtin_amdgcn_ds_permute(dest, aux_of(pos, part, b));
+  l.page = l.off = 0;
+  if (PAGED && lane < l.n) {
+    const int pg = l.key0 / page_size;
+    l.page = table[pg];
+    l.off = l.key0 - pg * page_size;
+  }
+  return l;
+}
+
+// Rows of one unit as 16-byte pieces of a wave, N instructions of 64 pieces with P pieces per row: after PAT instructions
+// the pieces fall on the same columns again.
+template <int CHANNELS>
+struct UnitRows {
+  static constexpr int P = CHANNELS / 8;
+  static constexpr int N = 32 * P / 64;
+  static constexpr int PAT = 64 % P == 0 ? 1 : 3;  // 192 channels: 3 * 64 = 8 * 24
+  static_assert((PAT * 64) % P == 0, "");
+  bf16x8 r[N];
+
+  // byte offset of this lane's piece of instruction j (j < PAT) from the unit's first row
+  static NSA_DEVICE uint32_t offset(int j, int lane, int64_t row_stride) {
+    const int pc = lane + j * 64;
+    return (uint32_t)(pc / P) * (uint32_t)(row_stride * 2) + (pc % P) * 16;
+  }
+  // all 32 rows: scalar base + 32-bit lane offsets (row strides below NARROW elements)
+  static constexpr int64_t NARROW = 1 << 27;
+  NSA_DEVICE void load(const bf16_t* first, int64_t row_stride, const uint32_t (&off)[PAT]) {
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+      const char* at = reinterpret_cast<const char*>(first + (j / PAT) * (PAT * 64 / P) * row_stride);
+      uint32_t o = off[j % PAT];
+      asm volatile("" : "+s"(at), "+v"(o));  // (the compiler would widen the offset outside of the loop and add 64 bits per lane)
+      r[j] = *(const __attribute__((address_space(1))) bf16x8*)((const __attribute__((address_space(1))) char*)at + o);
+    }
+  }
+  // rows past row `last` replaced by it; any stride
+  NSA_DEVICE void load_clamped(const bf16_t* first, int64_t row_stride, int last) {
+    const int lane = lane_id();  // (nothing of this rarely taken path is to be held in registers)
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+      const int pc = lane + j * 64;
+      r[j] = ld_global_b128(first + (int64_t)min(pc / P, last) * row_stride + (pc % P) * 8);
+    }
+  }
+  NSA_DEVICE void to_lds(bf16_t* rows, int ld, int lane) const {
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+      const int pc = lane + j * 64;
+      *reinterpret_cast<bf16x8*>(&rows[(pc / P) * ld + (pc % P) * 8]) = r[j];
+    }
+  }
+};

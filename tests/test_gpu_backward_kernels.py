@@ -1,5 +1,5 @@
 """The dk/dv kernel for 8, 16, 32 or 64 q-heads per kv head at the sizes where it can go wrong, against the oracle with the
-rounding points of a bf16 pipeline (the bar of test_gpu_backward.py)."""
+rounding points of a bf16 pipeline (the bar of test_gpu_backward.py); the selected forward's lists of key units."""
 import pytest
 import torch
 
@@ -52,3 +52,28 @@ def test_dkdv_of_every_branch(device, QH, KH, D, VD, block_size):
     ref = O.branch_forward_backward("slc", q.float(), k.float(), v.float(), do.float(), cu, cfg, topk=topk.cpu(), **rounded)
     check("slc", slc_attn_bwd(qd, kd, vd, topk, so, sl, dod), ref)
     check("slc, dq recomputed", (slc_attn_bwd(qd, kd, vd, topk, so, sl, dod, parts="dq")[0], None, None), ref)
+
+
+@pytest.mark.parametrize("QH,KH,D,VD", [(16, 2, 64, 64), (16, 1, 128, 128), (32, 2, 192, 128)])
+def test_selected_forward_with_long_unit_lists(device, QH, KH, D, VD):
+    """More than 64 units of 32 keys, the blocks in any order and negative ids between them, against masked attention."""
+    from flash_nsa.ops.select_attn import slc_attn_fwd
+    T, bs = 2310, 256
+    n = -(-T // bs)
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=330)]
+    setup_helper(make_cu([T]).to(device), block_size=bs, top_n=n + 1)
+    own = (torch.arange(T, device=device) // bs)[None, :, None]
+    rank = torch.rand(KH, T, n, generator=torch.Generator().manual_seed(331)).to(device)
+    topk = torch.where(torch.arange(n, device=device) <= own, rank, 2.0).argsort(-1).int()
+    topk = torch.where((rank[..., :1] < 0.3) & (topk != own) & (topk == 1), -1, topk)
+    topk = torch.cat([topk, torch.zeros_like(topk[..., :1])], -1).contiguous()
+    o, lse = slc_attn_fwd(q, k, v, topk)
+    taken = torch.zeros(KH, T, n + 1, dtype=torch.bool, device=device).scatter_(2, topk[..., :n].long() % (n + 1), True)
+    keys = torch.arange(T, device=device)
+    seen = taken[:, :, :n].repeat_interleave(bs, 2)[:, :, :T] & (keys <= keys[:, None])
+    for h in range(QH):
+        kh = h // (QH // KH)
+        s = (q[:, h].float() @ k[:, kh].float().t() * D ** -0.5).masked_fill(~seen[kh], float("-inf"))
+        # P and o are rounded to bf16 once each: 2 * 2^-9 of the largest value
+        assert (o[:, h].float() - s.softmax(-1) @ v[:, kh].float()).abs().max() <= 2 ** -8 * v.float().abs().max()
+        assert (lse[:, h] - s.logsumexp(-1) * 1.4426950408889634).abs().max() < 1e-4
