@@ -161,6 +161,15 @@ int nsa_cmp_attn_bwd_dq_final(const void* q, int64_t q_st, int64_t q_sh, const v
                               int64_t dqp_st, int64_t dqp_sh, void* dq, int64_t dq_st, int64_t dq_sh,
                               const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
                               int VD, int kernel_size, int stride, float sm_scale, void* stream);
+/* the same where the selected branch's dq is still to be added: dq of the positions below final_below, and this branch's dq
+ * added into dq_partial for the others */
+int nsa_cmp_attn_bwd_dq_final_below(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr,
+                                    int64_t ck_sh, const void* cv, int64_t cv_sr, int64_t cv_sh, const void* dO,
+                                    int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh,
+                                    const float* delta, int64_t delta_st, int64_t delta_sh, float* dq_partial,
+                                    int64_t dqp_st, int64_t dqp_sh, void* dq, int64_t dq_st, int64_t dq_sh, int final_below,
+                                    const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
+                                    int VD, int kernel_size, int stride, float sm_scale, void* stream);
 /* flash_nsa/ops/compress_attn.py:650-690 (_cmp_dkdv_kernel launch, dkdv_repeat=False): fp32 atomic adds into
  * dck/dcv [y_len,KH,*], which the caller zero-fills; queries are cut into chunks of q_chunk_tokens
  * (<= 0: chosen from the sizes so that short batches still fill the GPU) */
@@ -202,6 +211,14 @@ int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k
                         int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
                         int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
                         int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
+/* the same where this branch is the first to write dq: stores for every query */
+int nsa_swa_bwd_dq_tail_store(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                              const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                              const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                              int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
+                              int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                              int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
+                              int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
 /* same upstream site; dk/dv are stored (every key row has exactly one writer), bf16 or fp32 */
 int nsa_swa_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                      const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
@@ -264,6 +281,13 @@ int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_
                                  const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
                                  int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
                                  int32_t* workspace, int64_t workspace_elems, void* stream);
+/* the same over the tokens tok0 .. tok0 + T - 1 of the batch (csr_tok [KH*T*top_n]); csr_slot (or NULL) [KH*T*top_n]: the
+ * position in the token's selection that an entry of csr_tok stands for */
+int nsa_build_inverse_index_slots(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
+                                  const int32_t* kblk_cu, int B, int tok0, int T, int KH, int nblk_total,
+                                  int block_size, int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok,
+                                  uint8_t* csr_slot, int32_t* item_off, int32_t* workspace, int64_t workspace_elems,
+                                  void* stream);
 /* flash_nsa/ops/select_attn.py:593-637 (_dkdv_kernel launch): fp32 atomic adds into dk/dv [T,KH,*];
  * blk_seq [nblk_total] = sequence of each global block; n_items_bound >= max over kv heads of item_off[kh][nblk_total] */
 int nsa_slc_attn_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
@@ -274,6 +298,27 @@ int nsa_slc_attn_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void*
                           const int32_t* blk_seq, const int32_t* csr_off, const int32_t* csr_tok,
                           const int32_t* item_off, int nblk_total, int chunk_tokens, int n_items_bound, int B,
                           int QH, int KH, int D, int VD, int block_size, float sm_scale, void* stream);
+/* nsa_slc_attn_bwd_dkdv and nsa_slc_attn_bwd_dq_from for the tokens tok0 .. tok0 + ntok - 1 of the batch (with the index that
+ * nsa_build_inverse_index_slots makes of them): the dk/dv pass leaves its dS in `ds` (nsa_slc_bwd_ds_bytes(ntok, ...) bytes),
+ * from which the dq pass has dq = dS k.  dq_mode 3: bf16 store of the result added to the fp32 dq_partial.  nsa_slc_bwd_ds_tokens: tokens per call for a batch of T tokens, T where one call does;
+ * 0: shapes, strides or a scale that take the other entry points. */
+int nsa_slc_bwd_ds_tokens(int T, int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, int block_size,
+                          int top_n, float sm_scale);
+int64_t nsa_slc_bwd_ds_bytes(int ntok, int QH, int KH, int block_size, int top_n);
+int nsa_slc_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                             const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                             const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                             int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                             int64_t dv_sh, const int32_t* x_cu, const int32_t* kblk_cu, const int32_t* blk_seq,
+                             const int32_t* csr_off, const int32_t* csr_tok, const uint8_t* csr_slot,
+                             const int32_t* item_off, int nblk_total, int chunk_tokens, int n_items_bound, int B, int QH,
+                             int KH, int D, int VD, int block_size, int top_n, int tok0, int ntok, float sm_scale, void* ds,
+                             int64_t ds_bytes, void* stream);
+int nsa_slc_attn_bwd_dq_ds(const void* k, int64_t k_sr, int64_t k_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st,
+                           void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const float* dq_partial, int64_t dqp_st,
+                           int64_t dqp_sh, const int32_t* x_cu, int B, int QH, int KH, int D, int VD, int block_size,
+                           int top_n, int t_begin, int tok0, int ntok, float sm_scale, const void* ds, int64_t ds_bytes,
+                           void* stream);
 /* The same with a run-independent summation order (upstream's dkdv_repeat=True, flash_nsa/ops/select_attn.py:528-531,
  * 639-641): every work item (a chunk of a block's token list) stores its partial result in its own slot of
  * `workspace` (nsa_slc_attn_bwd_dkdv_det_bytes(...) bytes), a second launch adds the slots of a block to dk / dv in

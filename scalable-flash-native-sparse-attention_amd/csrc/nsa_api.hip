@@ -33,6 +33,7 @@ Knob g_knobs[] = {
     {"topk_seg_blocks", {0}, {false}},  // selection blocks per segment of the block selector
     {"decode_waves", {0}, {false}},     // waves per workgroup of the one-launch decode kernel (0: from the batch; 4, 8)
     {"swa_dkdv_splits", {0}, {false}},  // query chunks per key tile of the window dk/dv kernel (0: from the sizes)
+    {"slc_ds_mb", {0}, {false}},        // scratch for the dS of the selected branch, MB (0: dq and dk/dv computed apart)
     {"topk_two_pass", {0}, {false}},    // 0: the one-launch selector even when a workspace is given
 };
 Knob* find_knob(const char* name) {
@@ -96,7 +97,7 @@ int nsa_abi_version(void) { return 1; }
 int nsa_set_tuning(const char* name, int value) {
   Knob* k = name ? find_knob(name) : nullptr;
   NSA_REQUIRE(k != nullptr, NSA_ERR_BAD_ARG, "set_tuning: unknown name '%s' (fwd_variant, dq_min_blocks, "
-              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, decode_waves, topk_two_pass)", name ? name : "(null)");
+              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, decode_waves, slc_ds_mb, topk_two_pass)", name ? name : "(null)");
   k->value.store(value);
   k->is_set.store(true);
   return NSA_OK;
@@ -338,9 +339,9 @@ NsaBwdTileParams make_bwd(const BwdCommon& c, int QH, int KH, float sm_scale) {
 extern "C" {
 
 static int cmp_bwd_dq_impl(const char* who, const BwdCommon& c, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode,
-                           const float* dq_partial, int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu,
+                           float* dq_partial, int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu,
                            const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D, int VD, int kernel_size,
-                           int stride, float sm_scale, void* stream) {
+                           int stride, float sm_scale, void* stream, int final_below = 0) {
   int rc = check_heads(who, QH, KH, D, VD);
   if (rc) return rc;
   rc = check_nsa_sizes(who, kernel_size, stride, 0);
@@ -350,6 +351,7 @@ static int cmp_bwd_dq_impl(const char* who, const BwdCommon& c, void* dq, int64_
   p.dq_partial = dq_partial; p.dqp_st = dqp_st; p.dqp_sh = dqp_sh;
   p.x_cu = x_cu; p.k_cu = y_cu;
   p.kernel_size = kernel_size; p.stride = stride;
+  p.all_below = final_below;
   return nsa_bwd_dq_tile_launch(p, 0, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
@@ -376,8 +378,22 @@ int nsa_cmp_attn_bwd_dq_final(const void* q, int64_t q_st, int64_t q_sh, const v
   NSA_REQUIRE(dq_partial != nullptr && dq != nullptr, NSA_ERR_BAD_ARG, "cmp_attn_bwd_dq_final: null dq buffers");
   BwdCommon c{q, q_st, q_sh, ck, ck_sr, ck_sh, cv, cv_sr, cv_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta,
               delta_st, delta_sh};
-  return cmp_bwd_dq_impl("cmp_attn_bwd_dq_final", c, dq, dq_st, dq_sh, 3, dq_partial, dqp_st, dqp_sh, x_cu, y_cu, B,
-                         x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream);
+  return cmp_bwd_dq_impl("cmp_attn_bwd_dq_final", c, dq, dq_st, dq_sh, 3, const_cast<float*>(dq_partial), dqp_st, dqp_sh,
+                         x_cu, y_cu, B, x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream);
+}
+
+int nsa_cmp_attn_bwd_dq_final_below(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr,
+                                    int64_t ck_sh, const void* cv, int64_t cv_sr, int64_t cv_sh, const void* dO,
+                                    int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh,
+                                    const float* delta, int64_t delta_st, int64_t delta_sh, float* dq_partial,
+                                    int64_t dqp_st, int64_t dqp_sh, void* dq, int64_t dq_st, int64_t dq_sh, int final_below,
+                                    const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH, int D,
+                                    int VD, int kernel_size, int stride, float sm_scale, void* stream) {
+  NSA_REQUIRE(dq_partial != nullptr && dq != nullptr, NSA_ERR_BAD_ARG, "cmp_attn_bwd_dq_final_below: null dq buffers");
+  BwdCommon c{q, q_st, q_sh, ck, ck_sr, ck_sh, cv, cv_sr, cv_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta,
+              delta_st, delta_sh};
+  return cmp_bwd_dq_impl("cmp_attn_bwd_dq_final_below", c, dq, dq_st, dq_sh, 4, dq_partial, dqp_st, dqp_sh, x_cu, y_cu, B,
+                         x_maxlen, QH, KH, D, VD, kernel_size, stride, sm_scale, stream, final_below);
 }
 
 // Cost model of a dk/dv work item (128 keys x some query rows, 4 waves): fixed part (K / V fragments, epilogue, summing up)
@@ -544,7 +560,7 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
   return nsa_bwd_dq_tile_launch(p, 1, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
-int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+static int swa_bwd_dq_tail_impl(int dq_mode, const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                         const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                         const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                         int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
@@ -558,7 +574,7 @@ int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k
   BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
               delta_sh};
   NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
-  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh; p.dq_mode = 2;
+  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh; p.dq_mode = dq_mode;
   p.x_cu = x_cu; p.k_cu = x_cu;
   p.window = window;
   p.all_below = all_below;
@@ -566,6 +582,30 @@ int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k
   p.lse2 = slc_lse; p.lse2_st = sl_st; p.lse2_sh = sl_sh;
   p.delta2 = slc_delta; p.delta2_st = sd_st; p.delta2_sh = sd_sh;
   return nsa_bwd_dq_tile_launch(p, 2, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
+int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
+                        int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                        int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
+                        int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream) {
+  return swa_bwd_dq_tail_impl(2, q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+                              delta_sh, slc_dO, sdo_st, sdo_sh, slc_lse, sl_st, sl_sh, slc_delta, sd_st, sd_sh, all_below, dq,
+                              dq_st, dq_sh, x_cu, B, x_maxlen, QH, KH, D, VD, window, sm_scale, stream);
+}
+
+int nsa_swa_bwd_dq_tail_store(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                              const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                              const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                              int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh, const float* slc_lse,
+                              int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                              int all_below, float* dq, int64_t dq_st, int64_t dq_sh, const int32_t* x_cu, int B,
+                              int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream) {
+  return swa_bwd_dq_tail_impl(1, q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+                              delta_sh, slc_dO, sdo_st, sdo_sh, slc_lse, sl_st, sl_sh, slc_delta, sd_st, sd_sh, all_below, dq,
+                              dq_st, dq_sh, x_cu, B, x_maxlen, QH, KH, D, VD, window, sm_scale, stream);
 }
 
 // bytes of the partial dk / dv of the window branch with `splits` query chunks per key tile; dk_bytes: those of dk
@@ -795,7 +835,112 @@ int nsa_slc_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
                                 block_size, sm_scale, true, workspace, workspace_bytes, stream);
 }
 
+// dK / dV and dQ of the selected branch in one go: the dK/dV kernel leaves the dS of every (token, block) behind, and dQ = dS K
+// gathers half of what the kernel gathers that computes S and dP again.  Both kernels alone on the GPU, 64 heads of 128: 64K
+// tokens dQ 10.3 -> 5.55, dK/dV 6.4 -> 6.7 ms, 8 x 6K tokens 5.2 -> 2.93 and 3.84 -> 4.01 ms.
+// The dS of a token takes 32 KB per kv head (16 q-heads, 16 blocks of 64 keys), and 2 GB of it in flight do: longer batches
+// are cut into ranges of tokens (64K tokens, whole step with 1 / 2 / 4 / 8.6 GB: 55.5 / 55.3 / 55.7 / 56.3 ms; 32K tokens 20.5
+// / 20.6 / 20.5 / 20.5 ms), of 512 tokens at least.
+// No rule on the number of tokens: a query's dq is to be the same bits whatever follows it in the batch.  Steps with dq
+// recomputed / from the dS, us: 16 heads of 128, 16K tokens 2315 / 2277; 64 heads, 4K 1730 / 1744, 8K 3980 / 3863; 32 heads of
+// 192, 4K 1340 / 1402, 16K 6660 / 6630; 16 heads of 64 in 2 groups, 16K 1632 / 1642, 48K 6448 / 6105.
+static bool slc_bwd_ds_takes(int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, int block_size,
+                             int top_n, float sm_scale) {
+  if (KH <= 0 || QH % KH != 0 || block_size <= 0 || block_size % 32 != 0 || block_size > 2048) return false;
+  if (top_n < 1 || top_n > 64 || k_sr < 0 || k_sr >= (1 << 27)) return false;
+  NsaBwdTileParams p{};
+  p.G = QH / KH; p.q_sh = q_sh; p.do_sh = do_sh; p.scale_log2 = sm_scale * NSA_LOG2E;
+  return nsa_bwd_dkdv_dma_takes(p, D, VD);
+}
 
+int nsa_slc_bwd_ds_tokens(int T, int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, int block_size,
+                          int top_n, float sm_scale) {
+  if (T <= 0 || !slc_bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, block_size, top_n, sm_scale)) return 0;
+  const int64_t budget = (int64_t)nsa_tuning_knob("slc_ds_mb", 2048) << 20;
+  const int64_t per_token = nsa_slc_ds_entry_elems(QH / KH, block_size) * 2 * top_n * KH;
+  if (budget <= 0) return 0;
+  const int64_t fit = budget / per_token > 512 ? budget / per_token : 512;
+  if (fit >= T) return T;
+  const int64_t ranges = (T + fit - 1) / fit;
+  return (int)((T + ranges - 1) / ranges);
+}
+
+int64_t nsa_slc_bwd_ds_bytes(int ntok, int QH, int KH, int block_size, int top_n) {
+  if (ntok <= 0) return 0;
+  const int G = QH / KH;
+  // per kv head one more entry, for the dS of rows that stand for nothing
+  return KH * ((int64_t)ntok * top_n + 1) * nsa_slc_ds_entry_elems(G, block_size) * 2;
+}
+
+static int slc_ds_check(const char* who, int QH, int KH, int D, int VD, int block_size, int top_n, int tok0, int ntok, int B,
+                        const void* ds, int64_t ds_bytes, bool takes) {
+  int rc = check_heads(who, QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(tok0 >= 0 && ntok >= 0 && B >= 1, NSA_ERR_BAD_ARG, "%s: tokens %d + %d of %d sequences", who, tok0, ntok, B);
+  NSA_REQUIRE(takes, NSA_ERR_UNSUPPORTED, "%s: these shapes take slc_attn_bwd_dq and slc_attn_bwd_dkdv", who);
+  const int64_t need = nsa_slc_bwd_ds_bytes(ntok, QH, KH, block_size, top_n);
+  NSA_REQUIRE(ntok == 0 || (ds != nullptr && ds_bytes >= need), NSA_ERR_WORKSPACE, "%s: dS buffer of %lld bytes, %lld needed", who,
+              (long long)ds_bytes, (long long)need);
+  return NSA_OK;
+}
+
+int nsa_slc_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                             const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                             const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                             int64_t delta_sh, float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                             int64_t dv_sh, const int32_t* x_cu, const int32_t* kblk_cu, const int32_t* blk_seq,
+                             const int32_t* csr_off, const int32_t* csr_tok, const uint8_t* csr_slot,
+                             const int32_t* item_off, int nblk_total, int chunk_tokens, int n_items_bound, int B, int QH,
+                             int KH, int D, int VD, int block_size, int top_n, int tok0, int ntok, float sm_scale, void* ds,
+                             int64_t ds_bytes, void* stream) {
+  int rc = slc_ds_check("slc_attn_bwd_dkdv_ds", QH, KH, D, VD, block_size, top_n, tok0, ntok, B, ds, ds_bytes,
+                        slc_bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, block_size, top_n, sm_scale));
+  if (rc) return rc;
+  if (ntok == 0 || n_items_bound <= 0) return NSA_OK;
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
+  p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
+  p.dkv_mode = 3;
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.csr_off = csr_off; p.csr_tok = csr_tok; p.item_off = item_off; p.blk_seq = blk_seq; p.kblk_cu = kblk_cu;
+  p.nblk_total = nblk_total; p.chunk_tokens = chunk_tokens; p.block_size = block_size;
+  p.csr_sh = nblk_total + 1;
+  p.ds = (bf16_t*)ds; p.csr_slot = csr_slot;
+  p.ds_sh = ((int64_t)ntok * top_n + 1) * nsa_slc_ds_entry_elems(p.G, block_size);
+  p.ds_tok0 = tok0; p.ds_ntok = ntok; p.top_n = top_n;
+  p.ds_dump = ntok * top_n * (p.G > 16 ? p.G / 16 : 1);
+  NSA_REQUIRE(nsa_bwd_dkdv_dma_takes(p, D, VD), NSA_ERR_UNSUPPORTED,
+              "slc_attn_bwd_dkdv_ds: chunk_tokens %d exceeds what a work item's kernel holds", chunk_tokens);
+  return nsa_bwd_dkdv_launch(p, 2, B, 0, 0, D, VD, n_items_bound, (hipStream_t)stream);
+}
+
+int nsa_slc_attn_bwd_dq_ds(const void* k, int64_t k_sr, int64_t k_sh, const int32_t* topk, int64_t tk_sh, int64_t tk_st,
+                           void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const float* dq_partial, int64_t dqp_st,
+                           int64_t dqp_sh, const int32_t* x_cu, int B, int QH, int KH, int D, int VD, int block_size,
+                           int top_n, int t_begin, int tok0, int ntok, float sm_scale, const void* ds, int64_t ds_bytes,
+                           void* stream) {
+  int rc = slc_ds_check("slc_attn_bwd_dq_ds", QH, KH, D, VD, block_size, top_n, tok0, ntok, B, ds, ds_bytes,
+                        slc_bwd_ds_takes(0, 0, k_sr, QH, KH, D, VD, block_size, top_n, sm_scale));
+  if (rc) return rc;
+  NSA_REQUIRE(dq_mode >= 0 && dq_mode <= 3 && (dq_mode != 3 || dq_partial != nullptr), NSA_ERR_BAD_ARG,
+              "slc_attn_bwd_dq_ds: dq_mode %d not in {0,1,2,3}, or 3 without dq_partial", dq_mode);
+  rc = check_positions("slc_attn_bwd_dq_ds", t_begin);
+  if (rc) return rc;
+  NsaSlcDqDsParams p{};
+  p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
+  p.G = QH / KH;
+  p.ds = (const bf16_t*)ds; p.ds_sh = ((int64_t)ntok * top_n + 1) * nsa_slc_ds_entry_elems(p.G, block_size);
+  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh; p.dq_mode = dq_mode;
+  p.dq_partial = dq_partial; p.dqp_st = dqp_st; p.dqp_sh = dqp_sh;
+  p.topk = topk; p.tk_sh = tk_sh; p.tk_st = tk_st;
+  p.x_cu = x_cu;
+  p.B = B; p.KH = KH; p.top_n = top_n; p.block_size = block_size;
+  p.t_begin = t_begin; p.tok0 = tok0; p.ntok = ntok;
+  p.sm_scale = sm_scale;
+  return nsa_slc_dq_ds_launch(p, D, (hipStream_t)stream);
+}
 
 }  // extern "C"
 

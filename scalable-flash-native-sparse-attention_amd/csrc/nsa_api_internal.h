@@ -83,7 +83,8 @@ struct NsaBwdTileParams {
   const float* delta; int64_t delta_st, delta_sh;
   void* dq; int64_t dq_st, dq_sh; int dq_mode;      // 0: store bf16, 1: store fp32, 2: add into fp32,
                                                     // 3 (dq tile kernel): bf16 store of (result + fp32 dq_partial)
-  const float* dq_partial; int64_t dqp_st, dqp_sh;
+                                                    // 4: 3 for the positions below all_below, else add into dq_partial
+  float* dq_partial; int64_t dqp_st, dqp_sh;
   void* dk; int64_t dk_sr, dk_sh;                   // dkdv kernels
   void* dv; int64_t dv_sr, dv_sh;
   int dkv_mode;                                     // 0: store bf16, 1: store fp32, 3: atomic add into fp32,
@@ -100,7 +101,7 @@ struct NsaBwdTileParams {
   const int32_t* kblk_cu;      // [B+1] selection-block offsets
   int nblk_total, chunk_tokens, block_size;
   int64_t csr_sh;
-  // selected dkdv that also stores dS (see nsa_slc_bwd_dq.hip for the layout): csr_slot names the slot of the token's
+  // selected dkdv that also stores dS (see nsa_slc_bwd_dq_ds.hip for the layout): csr_slot names the slot of the token's
   // selection that an entry of csr_tok stands for; ds holds the tokens from global token ds_tok0 on, heads ds_sh apart
   bf16_t* ds; int64_t ds_sh;
   const uint8_t* csr_slot;
@@ -159,8 +160,7 @@ int nsa_slc_bwd_dq_launch(const NsaSlcBwdDqParams& p, int B, int max_q_len, int 
 struct NsaSlcDqDsParams {
   const bf16_t* k; int64_t k_sr, k_sh;
   const bf16_t* ds; int64_t ds_sh;
-  // 0: store bf16, 1: store fp32, 2: add into fp32, 3: bf16 store of (result + fp32 dq_partial), also of the queries before
-  // t_begin (whose result is 0)
+  // 0: store bf16, 1: store fp32, 2: add into fp32, 3: bf16 store of (result + fp32 dq_partial)
   void* dq; int64_t dq_st, dq_sh; int dq_mode;
   const float* dq_partial; int64_t dqp_st, dqp_sh;
   const int32_t* topk; int64_t tk_sh, tk_st;

@@ -584,7 +584,7 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
            hipStream_t stream) {
   NsaBwdTileParams p = p0;
   constexpr bool KB2_BUILT = kb2_built(D);
-  const bool dma = nsa_bwd_dkdv_dma_takes(p, D, VD) && nsa_tuning_knob("dkdv_key_blocks", 1) != 2;
+  const bool dma = p.ds != nullptr || (nsa_bwd_dkdv_dma_takes(p, D, VD) && nsa_tuning_knob("dkdv_key_blocks", 1) != 2);
   const int kb_cmp = KB2_BUILT ? nsa_tuning_knob("dkdv_key_blocks", 1) : 1;  // 32-key blocks per wave (cmp / swa)
   if (mode == MODE_CMP) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;

@@ -62,7 +62,7 @@ constexpr int DMA_LIST = 1024;  // tokens of a work item that the kernel holds i
 constexpr int dma_waves(int d) { return d <= 128 ? 2 : 1; }
 
 // DSH > 0 (MODE_SLC): the dS of every (token, block) is also stored, in blobs of DSH heads, for the dQ of the same tokens
-// (nsa_slc_bwd_dq.hip).  No path through the tile loop leaves the stores out (rows without an entry go to a blob that nobody
+// (nsa_slc_bwd_dq_ds.hip).  No path through the tile loop leaves the stores out (rows without an entry go to a blob that nobody
 // reads): where one did, the compiler waited for all of them and not just for the next tile's loads.
 template <int D, int VD, int MODE, bool NARROW, int DSH>
 __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdTileParams p) {

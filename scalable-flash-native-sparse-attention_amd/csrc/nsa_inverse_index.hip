@@ -45,7 +45,7 @@ __device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh
   r.nvalid = r.n >= t_begin ? min(top_n, r.n / block_size + 1) : 0;
   return r;
 }
-// fn(global block) for every block that the token selected; the ids are fetched ROW at a time, so that they share one
+// fn(global block, slot) for every block that the token selected; the ids are fetched ROW at a time, so that they share one
 // round trip to memory
 constexpr int ROW = 16;
 template <class Fn>
@@ -56,24 +56,25 @@ __device__ __forceinline__ void for_each_block(const TokenRow& r, Fn fn) {
     for (int s = 0; s < ROW; s++) j[s] = s0 + s < r.nvalid ? r.slots[s0 + s] : -1;
 #pragma unroll
     for (int s = 0; s < ROW; s++)
-      if (j[s] >= 0 && j[s] < r.nb) fn(r.kb + j[s]);
+      if (j[s] >= 0 && j[s] < r.nb) fn(r.kb + j[s], s0 + s);
   }
 }
 
 // grid (nchunks, KH), 256 threads, dynamic LDS nblk ints
 __global__ __launch_bounds__(256) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
-                                                        const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
-                                                        int nblk, int block_size, int t_begin, int32_t* chunk_cnt) {
+                                                        const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
+                                                        int T, int nblk, int block_size, int t_begin,
+                                                        int32_t* chunk_cnt) {
   extern __shared__ int hist[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
   for (int i = threadIdx.x; i < nblk; i += 256) hist[i] = 0;
   __syncthreads();
   const int CT = counting_chunk(T);
-  const int t0 = chunk * CT;
-  const int t1 = min(T, t0 + CT);
+  const int t0 = tok0 + chunk * CT;
+  const int t1 = min(tok0 + T, t0 + CT);
   for (int tb = t0; tb < t1; tb += 256) {
     const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + threadIdx.x, t1, kh, block_size, t_begin);
-    for_each_block(r, [&](int jb) { atomicAdd(&hist[jb], 1); });
+    for_each_block(r, [&](int jb, int) { atomicAdd(&hist[jb], 1); });
   }
   __syncthreads();
   int32_t* dst = chunk_cnt + ((int64_t)kh * gridDim.x + chunk) * nblk;
@@ -144,16 +145,17 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
 // blocks than that are taken in several rounds.
 constexpr int FILL_BLOCKS = 1024, FILL_WORDS = 256 / 32;
 __global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
-                                                       const int32_t* x_cu, const int32_t* kblk_cu, int B, int T,
-                                                       int nblk, int block_size, int t_begin, const int32_t* chunk_base,
-                                                       const int32_t* csr_off, int32_t* csr_tok) {
+                                                       const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
+                                                       int T, int nblk, int block_size, int t_begin,
+                                                       const int32_t* chunk_base, const int32_t* csr_off,
+                                                       int32_t* csr_tok, uint8_t* csr_slot) {
   __shared__ int cursor[FILL_BLOCKS];
   __shared__ __attribute__((aligned(16))) uint32_t mask[FILL_BLOCKS * FILL_WORDS];
   const int chunk = blockIdx.x, kh = blockIdx.y;
   const int tid = threadIdx.x;
   const int CT = counting_chunk(T);
-  const int t0 = chunk * CT;
-  const int t1 = min(T, t0 + CT);
+  const int t0 = tok0 + chunk * CT;
+  const int t1 = min(tok0 + T, t0 + CT);
   if (t0 >= t1) return;
   const int32_t* base = chunk_base + ((int64_t)kh * gridDim.x + chunk) * nblk;
   const int32_t* off = csr_off + (int64_t)kh * (nblk + 1);
@@ -170,17 +172,18 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int6
       for (int i = tid; i < nr * FILL_WORDS; i += 256) mask[i] = 0;
       __syncthreads();
       const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + tid, t1, kh, block_size, t_begin);
-      for_each_block(r, [&](int jb) {
+      for_each_block(r, [&](int jb, int) {
         if ((unsigned)(jb - r0) < (unsigned)nr) atomicOr(&mask[(jb - r0) * FILL_WORDS + word], bit);
       });
       __syncthreads();
-      for_each_block(r, [&](int jb) {
+      for_each_block(r, [&](int jb, int slot) {
         if ((unsigned)(jb - r0) >= (unsigned)nr) return;
         const uint32_t* m = &mask[(jb - r0) * FILL_WORDS];
         int pos = cursor[jb - r0];
 #pragma unroll
         for (int w = 0; w < FILL_WORDS; w++) pos += __popc(w < word ? m[w] : w == word ? m[w] & (bit - 1) : 0u);
         csr_tok[pos] = r.n;
+        if (csr_slot != nullptr) csr_slot[pos] = (uint8_t)slot;
       });
       __syncthreads();
       if (tb + 256 < t1) {
@@ -218,6 +221,16 @@ int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_
                                  const int32_t* kblk_cu, int B, int T, int KH, int nblk_total, int block_size,
                                  int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok, int32_t* item_off,
                                  int32_t* workspace, int64_t workspace_elems, void* stream) {
+  return nsa_build_inverse_index_slots(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, 0, T, KH, nblk_total, block_size,
+                                       chunk_tokens, t_begin, csr_off, csr_tok, nullptr, item_off, workspace,
+                                       workspace_elems, stream);
+}
+
+int nsa_build_inverse_index_slots(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n, const int32_t* x_cu,
+                                  const int32_t* kblk_cu, int B, int tok0, int T, int KH, int nblk_total,
+                                  int block_size, int chunk_tokens, int t_begin, int32_t* csr_off, int32_t* csr_tok,
+                                  uint8_t* csr_slot, int32_t* item_off, int32_t* workspace, int64_t workspace_elems,
+                                  void* stream) {
   if (T <= 0 || B <= 0 || nblk_total <= 0) return NSA_OK;
   NSA_REQUIRE(top_n >= 1 && top_n <= 64, NSA_ERR_BAD_ARG, "build_inverse_index: top_n %d must be in [1,64]", top_n);
   NSA_REQUIRE(chunk_tokens >= 1, NSA_ERR_BAD_ARG, "build_inverse_index: chunk_tokens must be positive");
@@ -232,7 +245,7 @@ int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_
   int nchunks = (T + CT - 1) / CT;
   size_t lds = (size_t)nblk_total * sizeof(int);
   dim3 grid(nchunks, KH);
-  csr_count_kernel<<<grid, 256, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
+  csr_count_kernel<<<grid, 256, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
                                           t_begin, workspace);
   int rc = nsa_check_launch("csr_count_kernel");
   if (rc) return rc;
@@ -240,8 +253,8 @@ int nsa_build_inverse_index_from(const int32_t* topk, int64_t tk_sh, int64_t tk_
                                       item_off);
   rc = nsa_check_launch("csr_scan_kernel");
   if (rc) return rc;
-  csr_fill_kernel<<<grid, 256, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, T, nblk_total, block_size,
-                                        t_begin, workspace, csr_off, csr_tok);
+  csr_fill_kernel<<<grid, 256, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
+                                        t_begin, workspace, csr_off, csr_tok, csr_slot);
   return nsa_check_launch("csr_fill_kernel");
 }
 

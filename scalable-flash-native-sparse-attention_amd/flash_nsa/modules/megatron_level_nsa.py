@@ -11,7 +11,8 @@ from ..utils import NSAHelper
 from ..ops._common import thd_rows
 from ..ops.compress_kv import construct_block_fwd, construct_block_bwd, mean_pooling_fwd, mean_pooling_bwd
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
-from ..ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window
+from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window,
+                               slc_bwd_ds_tokens)
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
 from ..ops.combine import combine_bwd_gates
@@ -19,9 +20,9 @@ from ..ops.sliding_window_attention import (slc_fwd_first_queries, swa_fwd, swa_
                                             swa_bwd_dq_tail)
 
 
-# The backward runs on two streams: the memory-bound selected-block dq kernel leaves the matrix cores idle and the
-# dense dk/dv kernels leave the memory side idle, so the dq chain (selected -> window -> compressed) runs next to the
-# dk/dv kernels (measured: about 1 ms of a 75 ms step; the same split of the forward gained nothing).
+# The backward runs on two streams, the dense dq kernels next to the dk/dv passes: batches that do not fill the GPU gain
+# (eight samples of up to 2.8K tokens, 16 heads of 128: 1705 -> 1488 us; 64 heads, 4K tokens 1825 -> 1744), full ones neither
+# gain nor lose (64K tokens 55.0 ms either way); the same split of the forward gained nothing.
 # Setting this module attribute to False puts everything back on the caller's stream.
 OVERLAP_STREAMS = True
 _side_streams = {}
@@ -156,37 +157,56 @@ class NSAFunction(torch.autograd.Function):
         dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         kw = dict(sm_scale=sm_scale, helper=helper)
 
-        def dq_chain():
-            # the selected branch (memory bound) stores, the window branch (matrix bound, with bandwidth to spare for
-            # the read-modify-write) adds, or stores where the selected branch left rows out, and the compressed branch
-            # adds and writes q's dtype
-            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, _store_into(dq32), delta=delta[1], parts="dq",
-                         t_begin=all_below, **kw)
-            swa_bwd_dq_tail(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, dq32, **kw)
-            return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
-                                parts="dq", **kw)[0]
+        # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
+        # branches' and writes q's dtype (the compressed branch does for the queries that the gather leaves out).  Else it
+        # stores first, the window branch (matrix bound, with bandwidth to spare for the read-modify-write) adds, or stores
+        # where the selected branch left rows out, and the compressed branch adds and writes q's dtype.
+        stored_ds = helper.x_maxlen > all_below and slc_bwd_ds_tokens(q, k, v, do, topk, **kw) > 0
+        dq_last = torch.empty_like(q) if stored_ds else None
 
-        def dkdv_raw():
+        def dq_chain():
+            if not stored_ds:
+                slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, _store_into(dq32), delta=delta[1], parts="dq",
+                             t_begin=all_below, **kw)
+            swa_bwd_dq_tail(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, dq32, store=stored_ds, **kw)
+            return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
+                                parts="dq", finalize_below=(dq_last, all_below) if stored_ds else None, **kw)[0]
+
+        def dkdv_raw(dq_after=None):
             # the window branch writes every element of dk / dv, the selected branch then adds to them
             _, dk, dv = swa_bwd(q, k, v, swa_o, lse_swa, do, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
             slc_attn_bwd_dkdv_before_window(q, k, v, lse_slc, do, delta[1], dk, dv, all_below, **kw)
-            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, None, dk, dv, delta=delta[1], parts="dkdv",
-                         t_begin=all_below, **kw)
+            last = dict(dq=dq32, finalize_dq=dq_last, dq_after=dq_after) if stored_ds else dict(parts="dkdv")
+            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, dk=dk, dv=dv, delta=delta[1], t_begin=all_below, **last, **kw)
             return dk, dv
 
         def dkdv_cmp():
             return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, delta=delta[0], parts="dkdv", **kw)[1:]
 
-        if OVERLAP_STREAMS:
-            main, side = torch.cuda.current_stream(), _side_stream(q.device)
+        main = torch.cuda.current_stream()
+        if OVERLAP_STREAMS and stored_ds:
+            # the dense dq kernels next to the dk / dv passes whose dS the selected dq waits for, the compressed dk / dv
+            # next to the selected dq
+            side = _side_stream(q.device)
+            side.wait_stream(main)
+            with torch.cuda.stream(side):
+                dq = dq_chain()
+                dense_dq = side.record_event()
+                dcmp_k, dcmp_v = dkdv_cmp()
+                dcmp_k.record_stream(main)
+                dcmp_v.record_stream(main)
+            dk, dv = dkdv_raw(dense_dq)
+            main.wait_stream(side)
+        elif OVERLAP_STREAMS:
+            side = _side_stream(q.device)
             side.wait_stream(main)
             with torch.cuda.stream(side):
                 dq = dq_chain()
                 dq.record_stream(main)
-            # dk/dv kernels on the caller's stream.  The compressed branch (matrix bound) goes first, next to the
-            # selected dq kernel (bound by the gather path) on the other stream: 0.7-1.7 ms per step less at T = 64K
-            # (67.7 -> 67.0 and 67.2 -> 65.5 ms on two GPUs) than the order window, selected, compressed, which ran the
-            # two selected kernels side by side.
+            # dk/dv kernels on the caller's stream.  The compressed branch (matrix bound) goes first, next to the selected
+            # dq kernel (bound by the gather path) on the other stream: 0.7-1.7 ms per step less at T = 64K (67.7 -> 67.0
+            # and 67.2 -> 65.5 ms on two GPUs) than the order window, selected, compressed, which ran the two selected
+            # kernels side by side.
             dcmp_k, dcmp_v = dkdv_cmp()
             dk, dv = dkdv_raw()
         else:

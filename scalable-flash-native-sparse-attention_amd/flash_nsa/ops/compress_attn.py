@@ -32,10 +32,12 @@ DKDV_SLOTS_LIMIT = 80 << 20
 
 
 def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None, helper=NSAHelper, delta=None,
-                 q_chunk_tokens=0, finalize_dq=False, parts="both"):
+                 q_chunk_tokens=0, finalize_dq=False, parts="both", finalize_below=None):
     """Backward of compressed attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer, which is added into; with finalize_dq the fp32 buffer is
-    only read and the returned dq is a fresh tensor in q's dtype holding buffer + this branch.
+    only read and the returned dq is a fresh tensor in q's dtype holding buffer + this branch.  finalize_below (with
+    finalize_dq): a tensor of q's dtype and n; that sum is for the queries at positions below n stored there, for the others
+    kept in the buffer.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None).
     dk, dv: fp32 [y_len,KH,*].  Every work item (query chunk of a key tile) stores its partial result into its own slot
     of a scratch buffer and a second launch sums the slots in a fixed order -- bit-identical results across runs.
@@ -60,9 +62,13 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
             # last branch of a fused backward: dq (fp32 sum of the other branches) + this branch -> fresh tensor in
             # q's dtype
             assert dq is not None and dq.dtype == torch.float32 and dq.shape == q.shape and dq.stride(-1) == 1
-            dq_buf = torch.empty_like(q)
-            _lib.call("nsa_cmp_attn_bwd_dq_final", *common, dq.data_ptr(), dq.stride(0), dq.stride(1),
-                      dq_buf.data_ptr(), dq_buf.stride(0), dq_buf.stride(1), *tail)
+            bufs = lambda out: (dq.data_ptr(), dq.stride(0), dq.stride(1), out.data_ptr(), out.stride(0), out.stride(1))
+            if finalize_below is not None:
+                dq_buf, below = finalize_below
+                _lib.call("nsa_cmp_attn_bwd_dq_final_below", *common, *bufs(dq_buf), below, *tail)
+            else:
+                dq_buf = torch.empty_like(q)
+                _lib.call("nsa_cmp_attn_bwd_dq_final", *common, *bufs(dq_buf), *tail)
         else:
             dq_buf, mode = dq_target(q, dq)
             _lib.call("nsa_cmp_attn_bwd_dq", *common, dq_buf.data_ptr(), dq_buf.stride(0), dq_buf.stride(1), mode,

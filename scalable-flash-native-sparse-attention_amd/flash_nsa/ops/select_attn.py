@@ -27,8 +27,49 @@ def slc_attn_fwd(q, k, v, topk, sm_scale=None, helper=NSAHelper, t_begin=0):
     return o, lse
 
 
+def slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale=None, helper=NSAHelper):
+    """Tokens per call of the backward that computes dq from the dS of the dk / dv pass, 0 where dq and dk / dv are computed
+    apart.  The scratch holds the dS of so many tokens (2 GB at most: 32 KB per token and kv head for 16 q-heads, 16 blocks
+    of 64 keys)."""
+    T, QH, D = q.shape
+    _, KH, VD = v.shape
+    if getattr(helper, "deterministic", False):
+        return 0
+    return _lib.value("nsa_slc_bwd_ds_tokens", T, q.stride(1), do.stride(1), k.stride(0), QH, KH, D, VD, helper.block_size,
+                      topk.size(-1), default_scale(q, sm_scale))
+
+
+def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, t_begin, sm_scale, helper, dq_after):
+    T, QH, KH, D, VD = shape
+    N, nblk, dev = topk.size(-1), helper.k_len, topk.device
+    chunk = _lib.value("nsa_slc_bwd_chunk_tokens", tokens, KH, N)
+    ds = torch.empty(_lib.value("nsa_slc_bwd_ds_bytes", tokens, QH, KH, helper.block_size, N), dtype=torch.uint8, device=dev)
+    ws_elems = _lib.value("nsa_inverse_index_workspace_elems", tokens, KH, nblk)
+    offs = torch.empty(2, KH, nblk + 1, device=dev, dtype=torch.int32)
+    index = torch.empty(KH * tokens * N + ws_elems, device=dev, dtype=torch.int32)  # list, then the builder's scratch
+    slot = torch.empty(KH * tokens * N, device=dev, dtype=torch.uint8)
+    x_cu, k_cu = helper.x_cu_seqlens.data_ptr(), helper.k_cu_seqlens.data_ptr()
+    tk = (topk.data_ptr(), topk.stride(0), topk.stride(1))
+    heads = (helper.batch, QH, KH, D, VD, helper.block_size, N)
+    dqs = (dq.data_ptr(), dq.stride(0), dq.stride(1), dq_mode)
+    dqs += (None, 0, 0) if partial is None else (partial.data_ptr(), partial.stride(0), partial.stride(1))
+    for tok0 in range(0, T, tokens):
+        n = min(tokens, T - tok0)
+        _lib.call("nsa_build_inverse_index_slots", *tk, N, x_cu, k_cu, helper.batch, tok0, n, KH, nblk, helper.block_size,
+                  chunk, t_begin, offs[0].data_ptr(), index.data_ptr(), slot.data_ptr(), offs[1].data_ptr(),
+                  index[KH * tokens * N:].data_ptr(), ws_elems, _lib.stream_ptr())
+        _lib.call("nsa_slc_attn_bwd_dkdv_ds", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0),
+                  dv.stride(1), x_cu, k_cu, helper.blk_seq.data_ptr(), offs[0].data_ptr(), index.data_ptr(),
+                  slot.data_ptr(), offs[1].data_ptr(), nblk, chunk, (n * N + chunk - 1) // chunk + nblk, *heads, tok0, n,
+                  sm_scale, ds.data_ptr(), ds.numel(), _lib.stream_ptr())
+        if tok0 == 0 and dq_after is not None:
+            torch.cuda.current_stream().wait_event(dq_after)
+        _lib.call("nsa_slc_attn_bwd_dq_ds", *common[3:6], *tk, *dqs, x_cu, *heads, t_begin, tok0, n, sm_scale, ds.data_ptr(),
+                  ds.numel(), _lib.stream_ptr())
+
+
 def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=None, helper=NSAHelper, delta=None,
-                 bind=None, parts="both", dkdv_repeat=False, t_begin=0):
+                 bind=None, parts="both", dkdv_repeat=False, t_begin=0, finalize_dq=None, dq_after=None):
     """Backward of selected attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer (added into).  dk/dv: fp32 [T,KH,*]; the caller's buffers
     are added into, otherwise zero-filled ones are created.  dkdv_repeat=False (default): with fp32 atomics, so the
@@ -37,7 +78,9 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     in a fixed order -- bit-identical results across runs.
     `bind` is the inverse index from get_bind_from_find (built here when absent).
     parts = "dq" / "dkdv" launches only that kernel (the other results are None).
-    t_begin: only the queries at positions from here on (a given `bind` then has to leave the others out)."""
+    t_begin: only the queries at positions from here on (a given `bind` then has to leave the others out).
+    finalize_dq (where slc_bwd_ds_tokens > 0): a tensor of q's dtype that takes the sum of this branch's dq and dq, the fp32
+    sum of the others, which is ready when the event dq_after is."""
     from .topk import get_bind_from_find
     check_thd(do, "do")
     T, QH, D = q.shape
@@ -49,8 +92,16 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
               v.stride(0), v.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse.data_ptr(), lse.stride(0),
               lse.stride(1), delta.data_ptr(), delta.stride(0), delta.stride(1))
     dq_buf = None
-    if parts in ("both", "dq"):
-        dq_buf, mode = dq_target(q, dq)
+    ordered = dkdv_repeat or getattr(helper, "deterministic", False)
+    ds_tokens = 0
+    if parts == "both" and not ordered and bind is None and not 0 < helper.x_maxlen <= t_begin:
+        ds_tokens = slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale, helper)
+    if finalize_dq is not None:
+        assert ds_tokens and dq.dtype == torch.float32 and dq.shape == q.shape and dq.stride(-1) == 1
+        dq_buf, mode, partial = finalize_dq, 3, dq
+    elif parts in ("both", "dq"):
+        (dq_buf, mode), partial = dq_target(q, dq), None
+    if parts in ("both", "dq") and not ds_tokens:
         _lib.call("nsa_slc_attn_bwd_dq_from", *common, topk.data_ptr(), topk.stride(0), topk.stride(1), dq_buf.data_ptr(),
                   dq_buf.stride(0), dq_buf.stride(1), mode, helper.x_cu_seqlens.data_ptr(), helper.batch,
                   helper.x_maxlen, QH, KH, D, VD, helper.block_size, topk.size(-1), t_begin, sm_scale,
@@ -66,7 +117,10 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     assert dk.dtype == torch.float32 and dv.dtype == torch.float32
     if 0 < helper.x_maxlen <= t_begin:
         return dq_buf, dk, dv
-    ordered = dkdv_repeat or getattr(helper, "deterministic", False)
+    if ds_tokens:
+        _slc_attn_bwd_ds(common, topk, dq_buf, mode, partial, dk, dv, (T, QH, KH, D, VD), ds_tokens, t_begin, sm_scale,
+                         helper, dq_after)
+        return dq_buf, dk, dv
     if bind is None:
         bind = get_bind_from_find(topk, helper, t_begin=t_begin, deterministic=ordered)
     args = (*common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0), dv.stride(1),

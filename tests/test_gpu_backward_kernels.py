@@ -77,3 +77,41 @@ def test_selected_forward_with_long_unit_lists(device, QH, KH, D, VD):
         # P and o are rounded to bf16 once each: 2 * 2^-9 of the largest value
         assert (o[:, h].float() - s.softmax(-1) @ v[:, kh].float()).abs().max() <= 2 ** -8 * v.float().abs().max()
         assert (lse[:, h] - s.logsumexp(-1) * 1.4426950408889634).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("QH,KH,D,VD", [(16, 1, 128, 128), (32, 1, 192, 128)])
+def test_selected_gradients_over_ranges_of_tokens(device, QH, KH, D, VD):
+    """dq from stored dS with a scratch that holds 2048 tokens: ranges that cut sequences, queries below t_begin left out,
+    added into fp32 -- against dq recomputed and dk / dv without ranges.  dS is the same bf16 value either way up to its last
+    place, so dq may differ by 2^-8 of a term's size; dk / dv only by the order of their fp32 sums."""
+    from flash_nsa import _lib
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd
+    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd, slc_bwd_ds_tokens
+    from flash_nsa.ops.topk import slc_topk_indices
+    cu = make_cu([1, 1500, 0, 3001, 77])
+    T, t_begin = int(cu[-1]), 300
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=350)]
+    do = randn_bf16(T, QH, VD, seed=354).to(device)
+    setup_helper(cu.to(device), top_n=5)
+    ck, cv = mean_pooling_fwd(k), mean_pooling_fwd(v)
+    _, cl = cmp_attn_fwd(q, ck, cv)
+    topk, _ = slc_topk_indices(q, ck, cl)
+    o, lse = slc_attn_fwd(q, k, v, topk)
+    base = torch.randn(T, QH, D, generator=torch.Generator().manual_seed(355)).to(device)
+    entry_kb = QH // KH * 5 * 64 * 2 / 1024
+    results = []
+    for mb in (-(-2048 * entry_kb // 1024), 0):
+        _lib.call("nsa_set_tuning", b"slc_ds_mb", int(mb))
+        try:
+            assert (0 < slc_bwd_ds_tokens(q, k, v, do, topk) < T) == (mb > 0)
+            results.append(slc_attn_bwd(q, k, v, topk, o, lse, do, base.clone(), t_begin=t_begin))
+        finally:
+            _lib.call("nsa_reset_tuning")
+    (dq, dk, dv), (dq_ref, dk_ref, dv_ref) = results
+    early = torch.cat([torch.arange(a, min(a + t_begin, b)) for a, b in zip(cu[:-1].tolist(), cu[1:].tolist())])
+    assert torch.equal(dq[early], base[early])
+    scale = (dq_ref - base).pow(2).mean().sqrt()
+    assert (dq - dq_ref).abs().max() <= 2 ** -6 * scale + 2 ** -8 * (dq_ref - base).abs().max()
+    for a, b in ((dk, dk_ref), (dv, dv_ref)):
+        assert (a - b).norm() <= 1e-4 * b.norm()
