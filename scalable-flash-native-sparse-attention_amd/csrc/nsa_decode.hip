@@ -918,6 +918,13 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
   typedef bf16_t bvecu __attribute__((ext_vector_type(OPT), aligned(2)));
   const int oi = tid * OPT;
   const int oh = oi / VD, od = oi - oh * VD;
+  const int hq = kh * G + oh;
+  bf16_t gate_raw[3] = {};           // requested long before the merge that uses them
+  if (p.out && oh < G) {
+    const bf16_t* wp = p.w + (int64_t)b * p.w_st + (int64_t)hq * p.w_sh;
+#pragma unroll
+    for (int i = 0; i < 3; i++) gate_raw[i] = wp[i];
+  }
   const int W = p.win_parts;         // > 0: the first launch has attended the window
   fvec ocmp_pre, o_swa_pre;          // merged outputs of the compressed branch (split path) and of the window
 #pragma unroll
@@ -1133,14 +1140,9 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
            [&](int u) { const int slot = u / upb; return blk_s[n_forced + slot] * Bs + (u - slot * upb) * UK; }, tab_s, page,
            kbase, p.k_sr, vbase, p.v_sr);
   }
-  // the gates come from memory: request them before the merge
-  float gate[3] = {0.f, 0.f, 0.f};
-  const int hq = kh * G + oh;
-  if (p.out && oh < G) {
-    const bf16_t* wp = p.w + (int64_t)b * p.w_st + (int64_t)hq * p.w_sh;
+  float gate[3];
 #pragma unroll
-    for (int i = 0; i < 3; i++) gate[i] = 1.f / (1.f + __expf(-(float)wp[i]));
-  }
+  for (int i = 0; i < 3; i++) gate[i] = 1.f / (1.f + __expf(-(float)gate_raw[i]));
   uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
   __syncthreads();
   if (oh >= G) return;

@@ -91,12 +91,14 @@ NSA_DEVICE float wave_fmax_uniform(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 63));
 }
 
-// The same selection as select_blocks_regs, with the repeated arg-max run over a short list instead of the NV
-// registers of every lane: the R-th largest of the 64 lane maxima is a lower bound of the R-th largest score (R =
-// number of arg-max rounds), so only the scores at or above it can be selected; they are compacted (ballot + prefix
-// count) into a wave-private list of at most 64 entries in LDS (cand_v / cand_i), one per lane, and a round is one
-// wave reduction plus one compare.  The picks and their order are those of select_blocks_regs (descending score,
-// lowest index on ties); rows with more than 64 scores at the bound (many equal values) take that function.
+// The same selection as select_blocks_regs over a short list instead of the NV registers of every lane: the R-th largest
+// of the 64 lane maxima is a lower bound of the R-th largest score (R = number of scored slots), so only the scores at or
+// above it can be selected; they are compacted (ballot + prefix count) into a wave-private list of at most 64 entries in LDS
+// (cand_v / cand_i), one per lane, in ascending order of the block.  Bound and places come from counting: every lane
+// compares its value with all others, broadcast one by one, which are independent instructions.  (Repeated wave-wide maxima
+// are a dependent chain of about 200 ns per round, twice R of them: one request of 32K tokens, 512 blocks, the selection 5.5
+// -> 2.7 us; 16 of 128K, 2048 blocks, 8.0 -> 5.1.)  The picks and their order are those of select_blocks_regs
+// (descending score, lowest index on ties); rows with more than 64 scores at the bound (many equal values) take that function.
 template <int NV, class P>
 NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, const P& p, int lane, float* cand_v,
                                         int* cand_i) {
@@ -122,18 +124,12 @@ NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, con
     v[k] = x;
     m = fmaxf(m, x);
   }
-  // bound: the lane maxima in descending order until `rounds` lanes are counted
-  float theta = -1.f;
-  int counted = 0;
-  for (int r = 0; r < rounds; r++) {
-    const float mx = wave_fmax_uniform(m);
-    if (mx < -1.f) { theta = -1.f; break; }  // fewer lanes than rounds hold a candidate: everything is listed
-    theta = mx;
-    const bool hit = m == mx;
-    counted += __builtin_popcountll(__builtin_amdgcn_ballot_w64(hit));
-    if (hit) m = -4.f;
-    if (counted >= rounds) break;
-  }
+  // bound: the smallest lane maximum that fewer than `rounds` exceed; -1 where fewer lanes than rounds hold a candidate
+  int above = 0;
+#pragma unroll
+  for (int j = 0; j < 64; j++)
+    above += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j)) > m;
+  const float theta = fmaxf(-wave_fmax_uniform(above < rounds ? -m : -__builtin_inff()), -1.f);
   // compaction of the scores >= theta, register by register (ascending block number within a register)
   int base = 0;
 #pragma unroll
@@ -148,12 +144,20 @@ NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, con
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  float cv = lane < base ? cand_v[lane] : -3.f;
-  int ci = lane < base ? cand_i[lane] : 0x7fffffff;
-  for (int slot = forced; slot < nsel; slot++) {
-    const int w = wave_argmax_lowest(cv, ci, ci != 0x7fffffff);
-    if (lane == slot) result = w;
-    if (ci == w) ci = 0x7fffffff;
+  const float cv = lane < base ? cand_v[lane] : -3.f;
+  const int ci = lane < base ? cand_i[lane] : 0;
+  int place = 0;  // scores ahead of this lane's: greater ones, and equal ones of lower blocks
+#pragma unroll 4
+  for (int j = 0; j < base; j++) {
+    const float other = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cv), j));
+    place += other > cv || (other == cv && j < lane);
   }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (lane < base && place < rounds) cand_i[place] = ci;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (lane >= forced && lane < nsel) result = lane - forced < base ? cand_i[lane - forced] : 0x7fffffff;
   return result;
 }
