@@ -504,6 +504,20 @@ int nsa_decode_split_window(const void* q, int64_t q_st, int64_t q_sh, const voi
                      int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
                      int num_local, int ignore_index, int window, float sm_scale, int win_parts,
                      float* win_ml, float* win_o, void* stream);
+/* the same (win_parts > 0), launch (1) also writing the newest token's K / V new_k / new_v [B,KH,*] to the flat pool rows
+ * slot_mapping [B] (-1: none), as nsa_decode_fused does */
+int nsa_decode_split_window_store(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
+                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
+                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                     int64_t tk_st, float* sp_m, float* sp_l, float* sp_o, void* sp_keep_p, float* sp_keep_m,
+                     int nsplit, const int32_t* cmp_slot_mapping, const int32_t* context_lens,
+                     const int32_t* block_tables, int table_stride, const int32_t* cmp_block_tables,
+                     int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
+                     int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
+                     int num_local, int ignore_index, int window, float sm_scale, int win_parts,
+                     float* win_ml, float* win_o, const void* new_k, int64_t nk_st, int64_t nk_sh, const void* new_v,
+                     int64_t nv_st, int64_t nv_sh, const int32_t* slot_mapping, void* stream);
 /* nsa_decode_split with launch (2) cut as well: upstream's slc_num_splits (flash_nsa/inference/__init__.py:195-196,
  * inference/select_attn.py:329-331,492-498 -- the selected blocks of one token dealt over several programs, merged
  * through fp32 partials).  Here slc_nsplit workgroups per (request, kv head) share the window units and the selected

@@ -1280,7 +1280,9 @@ static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const vo
                      int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
                      int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
                      int num_local, int ignore_index, int window, float sm_scale, int slc_nsplit, float* sp2_ml,
-                     float* sp2_o, void* cmp_tmp, int win_parts, float* win_ml, float* win_o, void* stream) {
+                     float* sp2_o, void* cmp_tmp, int win_parts, float* win_ml, float* win_o, void* stream,
+                     const void* new_k = nullptr, int64_t nk_st = 0, int64_t nk_sh = 0, const void* new_v = nullptr,
+                     int64_t nv_st = 0, int64_t nv_sh = 0, const int32_t* slot_mapping = nullptr) {
   int rc = check_heads("decode_split", QH, KH, D, VD);
   if (rc) return rc;
   rc = check_nsa_sizes("decode_split", kernel_size, stride, block_size);
@@ -1306,7 +1308,13 @@ static int decode_split_impl(const void* q, int64_t q_st, int64_t q_sh, const vo
               "decode_split: win_parts %d must be in [0,4], with its two buffers", win_parts);
   NSA_REQUIRE(win_parts == 0 || (window >= 0 && window <= 65536), NSA_ERR_BAD_ARG,
               "decode_split: window %d must be in [0,65536] to be attended in parts", window);
+  NSA_REQUIRE((new_k == nullptr) == (new_v == nullptr) && (new_k == nullptr) == (slot_mapping == nullptr) &&
+                  (new_k == nullptr || win_parts > 0),
+              NSA_ERR_BAD_ARG, "decode_split: new_k, new_v and slot_mapping must be given together, and with win_parts > 0");
   NsaDecodeParams p{};
+  p.new_k = (const bf16_t*)new_k; p.nk_st = nk_st; p.nk_sh = nk_sh;
+  p.new_v = (const bf16_t*)new_v; p.nv_st = nv_st; p.nv_sh = nv_sh;
+  p.raw_slots = slot_mapping;
   p.win_parts = win_parts; p.win_m = win_ml; p.win_o = win_o;
   p.win_l = win_ml ? win_ml + (int64_t)B * KH * win_parts * 16 : nullptr;
   p.slc_nsplit = slc_nsplit; p.sp2_ml = sp2_ml; p.sp2_o = sp2_o; p.cmp_tmp = (bf16_t*)cmp_tmp;
@@ -1367,6 +1375,27 @@ int nsa_decode_split_window(const void* q, int64_t q_st, int64_t q_sh, const voi
                            cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD, fixed_y_maxlen,
                            fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init, num_local,
                            ignore_index, window, sm_scale, 1, nullptr, nullptr, nullptr, win_parts, win_ml, win_o, stream);
+}
+
+int nsa_decode_split_window_store(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                     const void* v_cache, int64_t v_sr, int64_t v_sh, const void* w, int64_t w_st, int64_t w_sh,
+                     void* out, int64_t o_st, int64_t o_sh, void* cmp_o, void* slc_o, void* swa_o, int64_t co_st,
+                     int64_t co_sh, float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
+                     int64_t tk_st, float* sp_m, float* sp_l, float* sp_o, void* sp_keep_p, float* sp_keep_m,
+                     int nsplit, const int32_t* cmp_slot_mapping, const int32_t* context_lens,
+                     const int32_t* block_tables, int table_stride, const int32_t* cmp_block_tables,
+                     int cmp_table_stride, int page_size, int B, int QH, int KH, int D, int VD, int fixed_y_maxlen,
+                     int fixed_num_slc_blocks, int kernel_size, int stride, int block_size, int top_n, int num_init,
+                     int num_local, int ignore_index, int window, float sm_scale, int win_parts,
+                     float* win_ml, float* win_o, const void* new_k, int64_t nk_st, int64_t nk_sh, const void* new_v,
+                     int64_t nv_st, int64_t nv_sh, const int32_t* slot_mapping, void* stream) {
+  return decode_split_impl(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, w, w_st, w_sh, out, o_st, o_sh, cmp_o, slc_o,
+                           swa_o, co_st, co_sh, lse, lse_st, lse_sh, topk, tk_sh, tk_st, sp_m, sp_l, sp_o, sp_keep_p,
+                           sp_keep_m, nsplit, cmp_slot_mapping, context_lens, block_tables, table_stride,
+                           cmp_block_tables, cmp_table_stride, page_size, B, QH, KH, D, VD, fixed_y_maxlen,
+                           fixed_num_slc_blocks, kernel_size, stride, block_size, top_n, num_init, num_local,
+                           ignore_index, window, sm_scale, 1, nullptr, nullptr, nullptr, win_parts, win_ml, win_o, stream,
+                           new_k, nk_st, nk_sh, new_v, nv_st, nv_sh, slot_mapping);
 }
 
 int nsa_decode_split_parts(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,

@@ -193,13 +193,17 @@ struct UnitFlash {
     }
   }
   // next_k / next_v run as soon as the K / V registers have gone to LDS (they may load the next unit into them)
-  template <class NextK, class NextV>
-  NSA_DEVICE void compute(int key0, int klo, int khi, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ], NextK next_k, NextV next_v) {
+  // PATCH: row patch_row is not (or not yet) in the pool, its K pieces are in `patch` of the lanes from 0 on, its V pieces
+  // in those of the lanes from 32 on
+  template <bool PATCH, class NextK, class NextV>
+  NSA_DEVICE void compute(int key0, int klo, int khi, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ], NextK next_k, NextV next_v,
+                          int patch_row = 0, bf16x8 patch = bf16x8{}) {
 #pragma unroll
     for (int j = 0; j < KJ; j++) {
       int pc = lane + j * 64;
       *reinterpret_cast<bf16x8*>(&Ss[(pc / (D / 8)) * KLD + (pc % (D / 8)) * 8]) = kf[j];
     }
+    if (PATCH && lane < D / 8) *reinterpret_cast<bf16x8*>(&Ss[patch_row * KLD + lane * 8]) = patch;
     next_k();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -221,6 +225,8 @@ struct UnitFlash {
       int pc = lane + j * 64;
       *reinterpret_cast<bf16x8*>(&Ss[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
     }
+    if (PATCH && lane >= 32 && lane < 32 + VD / 8)
+      *reinterpret_cast<bf16x8*>(&Ss[patch_row * VLD + (lane - 32) * 8]) = patch;
     next_v();
     if (key0 < klo || key0 + UK - 1 > khi) {  // wave-uniform: only boundary units are masked
 #pragma unroll
@@ -321,7 +327,7 @@ struct UnitFlash {
       for (int u = first; u < nu; u += step) {
         const bool more = u + step < nu;
         const int nxt = more ? key0_of(u + step) : 0;
-        compute(
+        compute<false>(
             key, klo, khi, kf, vr,
             [&]() { if (more) issue<true, false>(nxt, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr); },
             [&]() { if (more) issue<false, true>(nxt, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr); });
@@ -345,16 +351,27 @@ struct UnitFlash {
     for (int u = first; u < nu; u += 2 * step) {
       const bool hasB = u + step < nu;
       if (hasB) { keyB = key0_of(u + step); issue(keyB, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kfB, vrB); }
-      compute(keyA, klo, khi, kfA, vrA, none, none);
+      compute<false>(keyA, klo, khi, kfA, vrA, none, none);
       if (hasB) {
         if (u + 2 * step < nu) {
           keyA = key0_of(u + 2 * step);
           issue(keyA, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kfA, vrA);
         }
-        compute(keyB, klo, khi, kfB, vrB, none, none);
+        compute<false>(keyB, klo, khi, kfB, vrB, none, none);
       }
     }
     }
+  }
+  // One unit, one row of which row_of() returns: called when the unit's rows have been requested (attend: the row belongs to
+  // the unit).  Apart from run(): inside its loop the exchange of a row costs every unit (16 x 128K 106.4 -> 108.6 us).
+  template <class RowFn>
+  NSA_DEVICE void run_patched(bool attend, int key, int klo, int khi, const int* tab_s, int page, const bf16_t* kbase,
+                              int64_t k_sr, const bf16_t* vbase, int64_t v_sr, int patch_row, RowFn row_of) {
+    bf16x8 kf[KJ], vr[VJ];
+    if (attend) issue(key, klo, khi, tab_s, page, kbase, k_sr, vbase, v_sr, kf, vr);
+    const bf16x8 patch = row_of();
+    auto none = []() {};
+    if (attend) compute<true>(key, klo, khi, kf, vr, none, none, patch_row, patch);
   }
   // wave partial -> LDS slot: m (raw units), l, o[16 heads][VD]
   NSA_DEVICE void publish(float* pm, float* pl, float* po) {
@@ -663,7 +680,9 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // parts of a pair attend the window in the same way, which needs nothing from the block selection and so stays out of
 // the second launch (0 / 1 / 2 / 3 / 4 parts, both launches: 1 x 32K 38.2 / 39.3 / 37.5 / 36.8 / 37.0 us, 16 x 128K
 // 99.9 / 98.0 / 97.7 / 97.8 / 99.9).  Two workgroups per CU, or the window's would wait for a CU.
-template <int D, int VD>
+// STORE: the caller passes the newest token's row.  (A kernel of its own: the launch is short, and the code that it does not
+// need costs the others 0.6 us.)
+template <int D, int VD, bool STORE>
 __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void decode_cmp_partial_kernel(NsaDecodeParams p) {
   using UF = UnitFlash<D, VD, KEEP_MEM>;
   constexpr int NW = SPLIT_WAVES;
@@ -691,6 +710,13 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void decode_cmp_partial_kernel
   const int page0 = klo / page;  // tab_s: pages of the keys klo .. khi
   if (in_window) ctab = p.table + (int64_t)b * p.table_stride;
   for (int i = page0 + tid; i <= (khi < 0 ? -1 : khi / page); i += NW * 64) tab_s[i - page0] = ctab[i];
+  // The newest token's row (upstream store_kvcache) is written by the wave that owns the window's
+  // last unit, which attends it from its registers; nobody else reads it in this launch (8 requests with 192 channels, 42.6
+  // us with a launch of its own in front, 39.5 so).  in_place: the block table has the caller's slot for it, else the
+  // table's row is what is attended.
+  const int new_slot = STORE ? p.raw_slots[b] : -1;
+  const bool newest_in_place =
+      STORE && new_slot >= 0 && t >= 0 && (int64_t)p.table[(int64_t)b * p.table_stride + t / page] * page + t % page == new_slot;
   // The compressed row that the newest token completes (mean of the last kernel_size raw rows, fp32 sums in row
   // order like nsa_paged_pool_decode; flash_nsa/inference/compress_kv.py:253-287 upstream) is written by the part
   // that attends it -- the one whose waves own the last unit -- wave 0 for K and wave 1 for V, one 16-byte piece per
@@ -705,7 +731,11 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void decode_cmp_partial_kernel
         const int32_t* tab = p.table + (int64_t)b * p.table_stride;
         const int st = ((L - p.kernel_size) / p.stride) * p.stride;
         float a[8];
-        sum_rows(a, cache + (int64_t)kh * c_sh + lane * 8, c_sr, tab, page, st, p.kernel_size, -1, zero_bf16x8());
+        bf16x8 newest = zero_bf16x8();
+        if (newest_in_place)
+          newest = ld_global_b128((wave == 0 ? p.new_k + (int64_t)b * p.nk_st + (int64_t)kh * p.nk_sh
+                                             : p.new_v + (int64_t)b * p.nv_st + (int64_t)kh * p.nv_sh) + lane * 8);
+        sum_rows(a, cache + (int64_t)kh * c_sh + lane * 8, c_sr, tab, page, st, p.kernel_size, newest_in_place ? t : -1, newest);
         const float inv = 1.f / (float)p.kernel_size;
         *reinterpret_cast<bf16x8*>(cache + (int64_t)cmp_slot * c_sr + (int64_t)kh * c_sh + lane * 8) =
             pack8(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, a[4] * inv, a[5] * inv, a[6] * inv, a[7] * inv);
@@ -732,8 +762,26 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void decode_cmp_partial_kernel
   const int nu = khi < 0 ? 0 : (khi - k0) / UK + 1;
   const int first = in_window ? (sp - nsplit) * NW + wave : sp * NW + wave;
   const int key_base = page0 * page;  // keys are counted from the first page in tab_s (a multiple of UK)
-  uf.run(first, NW * (in_window ? p.win_parts : nsplit), nu, klo - key_base, khi - key_base,
-         [&](int u) { return k0 - key_base + u * UK; }, tab_s, page, kbase, p.k_sr, vbase, p.v_sr);
+  auto key0_of = [&](int u) { return k0 - key_base + u * UK; };
+  const int step = NW * (in_window ? p.win_parts : nsplit);
+  const int last = max(nu - 1, 0);
+  const bool new_here = STORE && in_window && new_slot >= 0 && first == last % step;
+  uf.run(first, step, new_here && newest_in_place ? last : nu, klo - key_base, khi - key_base, key0_of, tab_s, page, kbase,
+         p.k_sr, vbase, p.v_sr);
+  if (new_here)
+    uf.run_patched(newest_in_place, key0_of(last), klo - key_base, khi - key_base, tab_s, page, kbase, p.k_sr, vbase, p.v_sr,
+                   khi - key_base - key0_of(last), [&]() {  // K in the lanes from 0 on, V in the lanes from 32 on
+                     const bool of_v = lane >= 32;
+                     const int c = (lane & 31) * 8;
+                     bf16x8 row = zero_bf16x8();
+                     if (c < (of_v ? VD : D)) {
+                       row = ld_global_b128((of_v ? p.new_v + (int64_t)b * p.nv_st + (int64_t)kh * p.nv_sh
+                                                  : p.new_k + (int64_t)b * p.nk_st + (int64_t)kh * p.nk_sh) + c);
+                       bf16_t* const cache = const_cast<bf16_t*>(of_v ? p.v : p.k) + (int64_t)kh * (of_v ? p.v_sh : p.k_sh);
+                       *reinterpret_cast<bf16x8*>(cache + (int64_t)new_slot * (of_v ? p.v_sr : p.k_sr) + c) = row;
+                     }
+                     return row;
+                   });
   uf.publish(part_m + wave * 16, part_l + wave * 16, reinterpret_cast<float*>(Vs_all + wave * SLOT));
   __syncthreads();
   // merge the 4 waves; store the part's un-normalised partial
@@ -1536,7 +1584,7 @@ static size_t cmp_partial_lds(const NsaDecodeParams& p) {
 
 template <int D, int VD>
 static int launch_cmp_partial(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
-  return launch_dyn(decode_cmp_partial_kernel<D, VD>, grid, SPLIT_WAVES, cmp_partial_lds<D, VD>(p), stream,
+  return launch_dyn(p.raw_slots != nullptr ? decode_cmp_partial_kernel<D, VD, true> : decode_cmp_partial_kernel<D, VD, false>, grid, SPLIT_WAVES, cmp_partial_lds<D, VD>(p), stream,
                     "decode_cmp_partial_kernel", 0, p);
 }
 

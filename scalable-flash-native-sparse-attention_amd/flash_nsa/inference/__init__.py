@@ -142,18 +142,20 @@ def nsa_decode(q, k, v, w, context_lens, block_tables, cmp_slot_mapping, cmp_blo
                                  num_inital=num_init_blocks, num_local=num_local_blocks, window_size=window_size,
                                  sm_scale=sm_scale, cmp_slot_mapping=cmp_slot_mapping, new_k=new_k, new_v=new_v,
                                  slot_mapping=slot_mapping)
-    if new_k is not None:
-        store_kvcache(new_k, new_v, k, v, slot_mapping)
     if (fused_decode_supported(q, k, v) and cmp_num_splits > 1 and
             decode_split_fits(q, k, v, block_tables, fixed_y_maxlen, fixed_num_slc_blocks)):
         # small batches of long contexts: the compressed branch is cut in that many key-interleaved parts per
-        # (request, kv head); two launches, the first of which also pools the newest compressed row
+        # (request, kv head); two launches, the first of which also writes the newest token's row and pools the newest
+        # compressed row
         return decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nsplit=cmp_num_splits,
                             fixed_y_maxlen=fixed_y_maxlen, fixed_num_slc_blocks=fixed_num_slc_blocks,
                             kernel_size=kernel_size, stride=stride, block_size=block_size, top_n=top_n,
                             num_inital=num_init_blocks, num_local=num_local_blocks, window_size=window_size,
                             sm_scale=sm_scale, cmp_slot_mapping=cmp_slot_mapping,
-                            slc_nsplit=max(1, min(int(slc_num_splits), 16)))
+                            slc_nsplit=max(1, min(int(slc_num_splits), 16)), new_k=new_k, new_v=new_v,
+                            slot_mapping=slot_mapping)
+    if new_k is not None:
+        store_kvcache(new_k, new_v, k, v, slot_mapping)
     kv_mean_pooling_decode(k, v, block_table=block_tables, slot_mapping=cmp_slot_mapping, context_lens=context_lens,
                            kernel_size=kernel_size, stride=stride)
     # capacities beyond the LDS of these kernels too (192 channels: from about 13K compressed rows on): stage by stage

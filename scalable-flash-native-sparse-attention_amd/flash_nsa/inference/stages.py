@@ -38,6 +38,13 @@ def store_kvcache(key, value, k_cache, v_cache, slot_mapping):
     """Scatter of new K/V rows into the paged pools (upstream nano-vllm/nanovllm/layers/attention.py:123-153):
     key [N,KH,D], value [N,KH,VD] -> flat pool rows slot_mapping[n] of k_cache / v_cache [pages,page,KH,*]
     (-1: skip the token)."""
+    N, KH, D, VD = _check_new_rows(key, value, k_cache, v_cache, slot_mapping)
+    _lib.call("nsa_store_kvcache", key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0),
+              k_cache.data_ptr(), KH * D, v_cache.data_ptr(), KH * VD, _i32(slot_mapping).data_ptr(), N, KH * D,
+              KH * VD, _lib.stream_ptr())
+
+
+def _check_new_rows(key, value, k_cache, v_cache, slot_mapping):
     check_bf16(key)
     N, KH, D = key.shape
     VD = value.size(-1)
@@ -46,9 +53,7 @@ def store_kvcache(key, value, k_cache, v_cache, slot_mapping):
     assert k_cache.dim() == 4 and k_cache.is_contiguous() and v_cache.is_contiguous()
     assert k_cache.shape[2:] == (KH, D) and v_cache.shape[2:] == (KH, VD)
     assert slot_mapping.numel() == N
-    _lib.call("nsa_store_kvcache", key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0),
-              k_cache.data_ptr(), KH * D, v_cache.data_ptr(), KH * VD, _i32(slot_mapping).data_ptr(), N, KH * D,
-              KH * VD, _lib.stream_ptr())
+    return N, KH, D, VD
 
 
 def store_kvcache_and_pool_prefill(key, value, k_cache, v_cache, x_cu_seqlens, x_maxlen, context_lens, slot_mapping,
@@ -372,13 +377,15 @@ def decode_two_launch_fits(q, k, v, block_tables, fixed_y_maxlen, fixed_num_slc_
 def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nsplit=4, fixed_y_maxlen=8192,
                  fixed_num_slc_blocks=2048, kernel_size=32, stride=16, block_size=64, top_n=16, num_inital=1,
                  num_local=2, window_size=512, sm_scale=None, return_parts=False, cmp_slot_mapping=None,
-                 static_scratch=False, slc_nsplit=1):
+                 static_scratch=False, slc_nsplit=1, new_k=None, new_v=None, slot_mapping=None):
     """The decode step in two launches, for small batches of long contexts: the compressed branch cut into `nsplit`
     parts per (request, kv head) so that it fills the GPU, then one workgroup per pair for the merge, the block
     selection, selected + window attention and the gated combine.  -> o [B,QH,VD]
     (return_parts: also cmp_o, slc_o, swa_o, topk [KH,B,top_n], lse [B,QH]).
     cmp_slot_mapping [B] (-1: none): the first launch also pools the compressed row that the newest token completes;
     None: that row is in the pool already.
+    new_k / new_v [B,KH,*] with slot_mapping [B]: the newest token's K/V are written to these flat pool rows (-1: none), by
+    the first launch where it attends the window, else by a launch of its own in front.
     static_scratch: the library's own static device buffer holds the parts' partial results (entry point
     nsa_decode_split_static, which allocates nothing); sizes beyond that buffer raise.
     slc_nsplit > 1: the second launch runs with that many workgroups per (request, kv head), which share the window
@@ -390,6 +397,13 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
     B, QH, _ = q.shape
     sm_scale = q.size(-1) ** -0.5 if sm_scale is None else sm_scale
     dev = q.device
+    n_win = 0 if slc_nsplit > 1 or static_scratch else _lib.value("nsa_decode_split_window_parts", window_size,
+                                                                  int(fixed_y_maxlen), nsplit)
+    if new_k is not None:
+        _check_new_rows(new_k, new_v, k, v, slot_mapping)
+        if n_win == 0 or new_k.size(0) != B:
+            store_kvcache(new_k, new_v, k, v, slot_mapping)
+            new_k = None
     out = torch.empty(B, QH, VD, device=dev, dtype=q.dtype)
     parts = [torch.empty_like(out) for _ in range(3)] if return_parts else [None] * 3
     topk = torch.empty(KH, B, top_n, device=dev, dtype=torch.int32) if return_parts else None
@@ -414,7 +428,6 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
         return out
     ycap32 = (int(fixed_y_maxlen) + 31) // 32 * 32
     # one fp32 buffer: m, l and o of the parts of the compressed branch, then of the window's
-    n_win = 0 if slc_nsplit > 1 else _lib.value("nsa_decode_split_window_parts", window_size, int(fixed_y_maxlen), nsplit)
     n_sp, n_wp = B * KH * nsplit * 16, B * KH * n_win * 16
     sp = torch.empty((n_sp + n_wp) * (2 + VD), device=dev, dtype=torch.float32)
     sp_ptr = sp.data_ptr()
@@ -439,6 +452,10 @@ def decode_split(q, k, v, w, block_tables, cmp_block_tables, context_lens, nspli
         cmp_tmp = torch.empty_like(out)
         _lib.call("nsa_decode_split_parts", *args, int(slc_nsplit), sp2_ml.data_ptr(), sp2_o.data_ptr(),
                   cmp_tmp.data_ptr(), _lib.stream_ptr())
+    elif new_k is not None:
+        _lib.call("nsa_decode_split_window_store", *args, n_win, win_ptr, win_ptr + 8 * n_wp, new_k.data_ptr(),
+                  new_k.stride(0), new_k.stride(1), new_v.data_ptr(), new_v.stride(0), new_v.stride(1),
+                  _i32(slot_mapping).data_ptr(), _lib.stream_ptr())
     else:
         _lib.call("nsa_decode_split_window", *args, n_win, win_ptr, win_ptr + 8 * n_wp, _lib.stream_ptr())
     if return_parts:
