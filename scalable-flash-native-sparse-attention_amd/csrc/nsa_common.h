@@ -71,6 +71,13 @@ NSA_DEVICE int sort_blocks(int blk, int n, int lane) {
   return __builtin_amdgcn_ds_permute(rank * 4, blk);
 }
 
+// Blocks in ascending order (sort_blocks), rotated so that the first one at or behind block `start` comes first.
+NSA_DEVICE int rotate_blocks(int blk, int n, int lane, int start) {
+  const int below = __popcll(__builtin_amdgcn_ballot_w64(lane < n && blk < start));
+  const int to = lane < n ? (lane < below ? lane + n - below : lane - below) : lane;
+  return __builtin_amdgcn_ds_permute(to * 4, blk);
+}
+
 NSA_DEVICE bf16x8 zero_bf16x8() {
   u32x4 z = {0, 0, 0, 0};
   return __builtin_bit_cast(bf16x8, z);

@@ -115,3 +115,31 @@ def test_selected_gradients_over_ranges_of_tokens(device, QH, KH, D, VD):
     assert (dq - dq_ref).abs().max() <= 2 ** -6 * scale + 2 ** -8 * (dq_ref - base).abs().max()
     for a, b in ((dk, dk_ref), (dv, dv_ref)):
         assert (a - b).norm() <= 1e-4 * b.norm()
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,T", [(16, 1, 128, 128, 8292), (16, 2, 64, 64, 16484), (16, 1, 192, 128, 6653)])
+def test_selected_forward_around_the_length_from_which_blocks_are_rotated(device, QH, KH, D, VD, T):
+    """The last 200 queries, some on either side of the line, blocks in any order and negative ids, against masked attention."""
+    from flash_nsa.ops.select_attn import slc_attn_fwd
+    bs, top_n, first = 64, 16, T - 200
+    n = -(-T // bs)
+    assert first < (4 << 20) // ((D + VD) * 2) < T - 1
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=360)]
+    setup_helper(make_cu([T]).to(device), block_size=bs, top_n=top_n)
+    own = (torch.arange(first, T, device=device) // bs)[None, :, None]
+    rank = torch.rand(KH, T - first, n, generator=torch.Generator().manual_seed(361)).to(device)
+    rank = torch.where(torch.arange(n, device=device) == own, -1.0, rank)  # the own block is among the selected
+    picked = torch.where(torch.arange(n, device=device) <= own, rank, 2.0).argsort(-1)[..., :top_n].int()
+    picked = torch.where((picked % 7 == 3) & (picked != own), -1, picked).roll(5, -1)
+    topk = torch.zeros(KH, T, top_n, dtype=torch.int32, device=device)
+    topk[:, first:] = picked
+    o, lse = slc_attn_fwd(q, k, v, topk, t_begin=first)
+    taken = torch.zeros(KH, T - first, n + 1, dtype=torch.bool, device=device).scatter_(2, picked.long() % (n + 1), True)
+    keys = torch.arange(T, device=device)
+    seen = taken[:, :, :n].repeat_interleave(bs, 2)[:, :, :T] & (keys <= keys[first:, None])
+    for h in range(QH):
+        kh = h // (QH // KH)
+        s = (q[first:, h].float() @ k[:, kh].float().t() * D ** -0.5).masked_fill(~seen[kh], float("-inf"))
+        # P and o are rounded to bf16 once each: 2 * 2^-9 of the largest value
+        assert (o[first:, h].float() - s.softmax(-1) @ v[:, kh].float()).abs().max() <= 2 ** -8 * v.float().abs().max()
+        assert (lse[first:, h] - s.logsumexp(-1) * 1.4426950408889634).abs().max() < 1e-4
