@@ -161,7 +161,8 @@ class NSAFunction(torch.autograd.Function):
         # branches' and writes q's dtype (the compressed branch does for the queries that the gather leaves out).  Else it
         # stores first, the window branch (matrix bound, with bandwidth to spare for the read-modify-write) adds, or stores
         # where the selected branch left rows out, and the compressed branch adds and writes q's dtype.
-        stored_ds = helper.x_maxlen > all_below and slc_bwd_ds_tokens(q, k, v, do, topk, **kw) > 0
+        ds_tokens = slc_bwd_ds_tokens(q, k, v, do, topk, **kw) if helper.x_maxlen > all_below else 0
+        stored_ds = ds_tokens > 0
         dq_last = torch.empty_like(q) if stored_ds else None
 
         def dq_chain():
@@ -176,7 +177,7 @@ class NSAFunction(torch.autograd.Function):
             # the window branch writes every element of dk / dv, the selected branch then adds to them
             _, dk, dv = swa_bwd(q, k, v, swa_o, lse_swa, do, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
             slc_attn_bwd_dkdv_before_window(q, k, v, lse_slc, do, delta[1], dk, dv, all_below, **kw)
-            last = dict(dq=dq32, finalize_dq=dq_last, dq_after=dq_after) if stored_ds else dict(parts="dkdv")
+            last = dict(dq=dq32, finalize_dq=dq_last, dq_after=dq_after, ds_tokens=ds_tokens) if stored_ds else dict(parts="dkdv")
             slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, dk=dk, dv=dv, delta=delta[1], t_begin=all_below, **last, **kw)
             return dk, dv
 

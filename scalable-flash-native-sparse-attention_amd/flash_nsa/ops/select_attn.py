@@ -43,11 +43,18 @@ def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, 
     T, QH, KH, D, VD = shape
     N, nblk, dev = topk.size(-1), helper.k_len, topk.device
     chunk = _lib.value("nsa_slc_bwd_chunk_tokens", tokens, KH, N)
-    ds = torch.empty(_lib.value("nsa_slc_bwd_ds_bytes", tokens, QH, KH, helper.block_size, N), dtype=torch.uint8, device=dev)
+    ds_bytes = _lib.value("nsa_slc_bwd_ds_bytes", tokens, QH, KH, helper.block_size, N)
     ws_elems = _lib.value("nsa_inverse_index_workspace_elems", tokens, KH, nblk)
-    offs = torch.empty(2, KH, nblk + 1, device=dev, dtype=torch.int32)
-    index = torch.empty(KH * tokens * N + ws_elems, device=dev, dtype=torch.int32)  # list, then the builder's scratch
-    slot = torch.empty(KH * tokens * N, device=dev, dtype=torch.uint8)
+    # one buffer: dS, token list, the list builder's scratch, list and item offsets, slot of every list entry
+    entries, n_off, index_at = KH * tokens * N, KH * (nblk + 1), (ds_bytes + 255) // 256 * 256
+    buf = torch.empty(index_at + 4 * (entries + ws_elems + 2 * n_off) + entries, dtype=torch.uint8, device=dev)
+    ds = buf.data_ptr()
+    index = ds + index_at
+    scratch = index + 4 * entries
+    csr_off = scratch + 4 * ws_elems
+    item_off = csr_off + 4 * n_off
+    slot = item_off + 4 * n_off
+    stream = _lib.stream_ptr()
     x_cu, k_cu = helper.x_cu_seqlens.data_ptr(), helper.k_cu_seqlens.data_ptr()
     tk = (topk.data_ptr(), topk.stride(0), topk.stride(1))
     heads = (helper.batch, QH, KH, D, VD, helper.block_size, N)
@@ -56,20 +63,19 @@ def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, 
     for tok0 in range(0, T, tokens):
         n = min(tokens, T - tok0)
         _lib.call("nsa_build_inverse_index_slots", *tk, N, x_cu, k_cu, helper.batch, tok0, n, KH, nblk, helper.block_size,
-                  chunk, t_begin, offs[0].data_ptr(), index.data_ptr(), slot.data_ptr(), offs[1].data_ptr(),
-                  index[KH * tokens * N:].data_ptr(), ws_elems, _lib.stream_ptr())
+                  chunk, t_begin, csr_off, index, slot, item_off, scratch, ws_elems, stream)
         _lib.call("nsa_slc_attn_bwd_dkdv_ds", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0),
-                  dv.stride(1), x_cu, k_cu, helper.blk_seq.data_ptr(), offs[0].data_ptr(), index.data_ptr(),
-                  slot.data_ptr(), offs[1].data_ptr(), nblk, chunk, (n * N + chunk - 1) // chunk + nblk, *heads, tok0, n,
-                  sm_scale, ds.data_ptr(), ds.numel(), _lib.stream_ptr())
+                  dv.stride(1), x_cu, k_cu, helper.blk_seq.data_ptr(), csr_off, index, slot, item_off, nblk, chunk,
+                  (n * N + chunk - 1) // chunk + nblk, *heads, tok0, n, sm_scale, ds, ds_bytes, stream)
         if tok0 == 0 and dq_after is not None:
             torch.cuda.current_stream().wait_event(dq_after)
-        _lib.call("nsa_slc_attn_bwd_dq_ds", *common[3:6], *tk, *dqs, x_cu, *heads, t_begin, tok0, n, sm_scale, ds.data_ptr(),
-                  ds.numel(), _lib.stream_ptr())
+        _lib.call("nsa_slc_attn_bwd_dq_ds", *common[3:6], *tk, *dqs, x_cu, *heads, t_begin, tok0, n, sm_scale, ds, ds_bytes,
+                  stream)
 
 
 def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=None, helper=NSAHelper, delta=None,
-                 bind=None, parts="both", dkdv_repeat=False, t_begin=0, finalize_dq=None, dq_after=None):
+                 bind=None, parts="both", dkdv_repeat=False, t_begin=0, finalize_dq=None, dq_after=None,
+                 ds_tokens=None):
     """Backward of selected attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer (added into).  dk/dv: fp32 [T,KH,*]; the caller's buffers
     are added into, otherwise zero-filled ones are created.  dkdv_repeat=False (default): with fp32 atomics, so the
@@ -79,6 +85,7 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     `bind` is the inverse index from get_bind_from_find (built here when absent).
     parts = "dq" / "dkdv" launches only that kernel (the other results are None).
     t_begin: only the queries at positions from here on (a given `bind` then has to leave the others out).
+    ds_tokens: what slc_bwd_ds_tokens has returned for these tensors, if the caller has asked.
     finalize_dq (where slc_bwd_ds_tokens > 0): a tensor of q's dtype that takes the sum of this branch's dq and dq, the fp32
     sum of the others, which is ready when the event dq_after is."""
     from .topk import get_bind_from_find
@@ -93,8 +100,9 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
               lse.stride(1), delta.data_ptr(), delta.stride(0), delta.stride(1))
     dq_buf = None
     ordered = dkdv_repeat or getattr(helper, "deterministic", False)
-    ds_tokens = 0
-    if parts == "both" and not ordered and bind is None and not 0 < helper.x_maxlen <= t_begin:
+    if parts != "both" or ordered or bind is not None or 0 < helper.x_maxlen <= t_begin:
+        ds_tokens = 0
+    elif ds_tokens is None:
         ds_tokens = slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale, helper)
     if finalize_dq is not None:
         assert ds_tokens and dq.dtype == torch.float32 and dq.shape == q.shape and dq.stride(-1) == 1
