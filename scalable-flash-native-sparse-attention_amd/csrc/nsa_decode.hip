@@ -193,8 +193,10 @@ struct UnitFlash {
     }
   }
   // next_k / next_v run as soon as the K / V registers have gone to LDS (they may load the next unit into them)
-  // PATCH: row patch_row is not (or not yet) in the pool, its K pieces are in `patch` of the lanes from 0 on, its V pieces
-  // in those of the lanes from 32 on
+  // PATCH: row patch_row, that of key khi, is not (or not yet) in the pool, its K pieces are in `patch` of the lanes from 0 on,
+  // its V pieces in those of the lanes from 32 on.  issue() has read the pool's row of khi also for every key clamped to it:
+  // those V rows are zeroed, since what a slot held before it was first written may be infinite or NaN, which a probability
+  // of 0 does not remove (a masked key's scores are replaced, whatever its K row holds).
   template <bool PATCH, class NextK, class NextV>
   NSA_DEVICE void compute(int key0, int klo, int khi, bf16x8 (&kf)[KJ], bf16x8 (&vr)[VJ], NextK next_k, NextV next_v,
                           int patch_row = 0, bf16x8 patch = bf16x8{}) {
@@ -223,6 +225,7 @@ struct UnitFlash {
 #pragma unroll
     for (int j = 0; j < VJ; j++) {
       int pc = lane + j * 64;
+      if (PATCH && (key0 + pc / (VD / 8) >= khi || klo >= khi)) vr[j] = zero_bf16x8();
       *reinterpret_cast<bf16x8*>(&Ss[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
     }
     if (PATCH && lane >= 32 && lane < 32 + VD / 8)

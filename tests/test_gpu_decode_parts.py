@@ -47,6 +47,47 @@ def test_newest_row_written_by_the_first_launch(device, D, VD, KH, G, page, wind
             assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("D,VD,KH,G", [(128, 128, 2, 16), (192, 128, 2, 16), (64, 64, 2, 8)])
+@pytest.mark.parametrize("page,window", [(64, 512), (256, 100), (128, 0)])
+def test_newest_row_into_a_slot_never_written(device, D, VD, KH, G, page, window):
+    """As above, bit for bit, where every pool row that holds no token yet, the newest's own slot among them, is NaN (a new
+    pool is uninitialised memory): the newest row first, in the middle and last in a unit, and the only one of its window."""
+    from flash_nsa.inference import store_kvcache
+    from flash_nsa.inference.stages import decode_split
+    ctx = [1, 2, 31, 32, 33, 48, 64, 65, 257, 800, 1024, 1025, 4096]
+    B = len(ctx)
+    case = build_pool(ctx, KH, D, VD, page=page, seed=4)
+    prepool(case, [n - 1 for n in ctx])
+    slots, cmp_slots, written = [], [], []
+    for b, n in enumerate(ctx):
+        rows = [int(case["bt"][b, i // page]) * page + i % page for i in range(n)]
+        written += rows[:-1]
+        slots.append(rows[-1])
+        y = max((n - 1 - 32) // 16 + 1, 0)
+        written += [cmp_row_slot(case, b, i) for i in range(y)]
+        cmp_slots.append(cmp_row_slot(case, b, y) if case["ys"][b] > y else -1)
+    for name in ("k", "v"):
+        flat = case[name].view(-1, *case[name].shape[2:])
+        empty = torch.ones(len(flat), dtype=torch.bool)
+        empty[written] = False
+        flat[empty] = float("nan")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
+    q, w = randn_bf16(B, KH * G, D, seed=15).to(device), randn_bf16(B, KH * G, 3, seed=16).to(device)
+    new_k, new_v = randn_bf16(B, KH, D, seed=17).to(device), randn_bf16(B, KH, VD, seed=18).to(device)
+    kw = dict(fixed_y_maxlen=512, fixed_num_slc_blocks=64, window_size=window, cmp_slot_mapping=i32(cmp_slots), top_n=8)
+    for nsplit in (2, 16):
+        results = []
+        for new in ({}, dict(new_k=new_k, new_v=new_v, slot_mapping=i32(slots))):
+            k, v = case["k"].to(device), case["v"].to(device)
+            if not new:
+                store_kvcache(new_k, new_v, k, v, i32(slots))
+            o = decode_split(q, k, v, w, case["bt"].to(device), case["cbt"].to(device), i32(ctx), nsplit=nsplit, **new, **kw)
+            results.append((o, k, v))
+        assert torch.isfinite(results[0][0]).all()
+        for x, y in zip(*results):
+            assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
 @pytest.mark.parametrize("blocks", [20, 64, 65, 512, 513, 2048])
 @pytest.mark.parametrize("values", [1, 3, 40, 100000])
 def test_selection_by_counting(device, blocks, values):
