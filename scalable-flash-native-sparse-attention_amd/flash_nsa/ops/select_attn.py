@@ -44,7 +44,8 @@ def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, 
     N, nblk, dev = topk.size(-1), helper.k_len, topk.device
     chunk = _lib.value("nsa_slc_bwd_chunk_tokens", tokens, KH, N)
     ds_bytes = _lib.value("nsa_slc_bwd_ds_bytes", tokens, QH, KH, helper.block_size, N)
-    ws_elems = _lib.value("nsa_inverse_index_workspace_elems", tokens, KH, nblk)
+    # (the last range, the only shorter one, may need more: short ranges are counted in shorter chunks)
+    ws_elems = max(_lib.value("nsa_inverse_index_workspace_elems", n, KH, nblk) for n in {tokens, (T - 1) % tokens + 1})
     # one buffer: dS, token list, the list builder's scratch, list and item offsets, slot of every list entry
     entries, n_off, index_at = KH * tokens * N, KH * (nblk + 1), (ds_bytes + 255) // 256 * 256
     buf = torch.empty(index_at + 4 * (entries + ws_elems + 2 * n_off) + entries, dtype=torch.uint8, device=dev)

@@ -158,6 +158,42 @@ def test_inverse_index_refuses_more_blocks_than_its_histogram_holds():
                   None, None, 0, None)
 
 
+@pytest.mark.parametrize("T", [700, 131072, 131073, 262144, 262145, 300001])
+@pytest.mark.parametrize("QH,KH,top_n", [(16, 1, 6), (8, 1, 8), (64, 4, 16)])
+def test_selected_backward_scratch_holds_every_range(monkeypatch, T, QH, KH, top_n):
+    """Every range of tokens gets the dS, list and builder's scratch that the library asks for, all inside the one buffer."""
+    import types
+    from flash_nsa import _lib
+    from flash_nsa.ops import select_attn
+    nblk = -(-T // 64)
+    one = torch.zeros(1, dtype=torch.int32)
+    helper = types.SimpleNamespace(block_size=64, k_len=nblk, batch=1, x_cu_seqlens=one, k_cu_seqlens=one, blk_seq=one)
+    tokens = _lib.value("nsa_slc_bwd_ds_tokens", T, 128, 128, KH * 128, QH, KH, 128, 128, 64, top_n, 128 ** -0.5)
+    assert 0 < tokens <= T
+    calls, buffers = [], []
+    monkeypatch.setattr(select_attn._lib, "call", lambda *a: calls.append(a))
+    monkeypatch.setattr(select_attn._lib, "stream_ptr", lambda: 0)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: buffers.append(empty(*a, **kw)) or buffers[-1])
+    meta = empty(KH, T, top_n, dtype=torch.int32)  # (never touched)
+    grad = torch.zeros(1, 1, 1)
+    select_attn._slc_attn_bwd_ds((0,) * 18, meta, grad, 2, None, grad, grad, (T, QH, KH, 128, 128), tokens, 0, 0.1, helper, None)
+    (buf,) = buffers
+    lo, hi = buf.data_ptr(), buf.data_ptr() + buf.numel()
+    built = [a[1:] for a in calls if a[0] == "nsa_build_inverse_index_slots"]
+    assert sum(a[8] for a in built) == T and [a[7] for a in built] == [sum(b[8] for b in built[:i]) for i in range(len(built))]
+    for a in built:
+        n, (csr_off, csr_tok, csr_slot, item_off, ws, ws_elems) = a[8], a[14:20]
+        assert ws_elems >= _lib.value("nsa_inverse_index_workspace_elems", n, KH, nblk)
+        parts = [(csr_off, 4 * KH * (nblk + 1)), (csr_tok, 4 * KH * n * top_n), (csr_slot, KH * n * top_n),
+                 (item_off, 4 * KH * (nblk + 1)), (ws, 4 * ws_elems),
+                 (lo, _lib.value("nsa_slc_bwd_ds_bytes", n, QH, KH, 64, top_n))]
+        ends = [(at, at + size) for at, size in sorted(parts)]
+        assert ends[0][0] >= lo and ends[-1][1] <= hi and all(x[1] <= y[0] for x, y in zip(ends, ends[1:]))
+    del buf
+    buffers.clear()
+
+
 def test_tuning_values_are_set_by_name_not_by_environment():
     from flash_nsa import _lib
     _lib.call("nsa_set_tuning", b"topk_seg_blocks", 64)
