@@ -38,6 +38,7 @@ __device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh
   TokenRow r{topk, 0, 0, 0, 0};
   if (tok >= t1) return r;
   const int b = find_seq(x_cu, B, tok);
+  if (tok >= x_cu[b + 1]) return r;  // behind the last sequence
   r.slots = topk + (int64_t)kh * tk_sh + (int64_t)tok * tk_st;
   r.n = tok - x_cu[b];
   r.kb = kblk_cu[b];

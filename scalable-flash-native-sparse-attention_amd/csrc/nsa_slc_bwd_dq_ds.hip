@@ -51,16 +51,17 @@ __global__ __launch_bounds__(dq_ds_waves(D) * 64) void slc_dq_ds_kernel(NsaSlcDq
   }
   const int x0 = p.x_cu[b];
   const int t = tok - x0;
-  if (t < p.t_begin) return;
+  if (t < p.t_begin || tok >= p.x_cu[b + 1]) return;  // (rows behind the last sequence are left alone)
   const int Bs = p.block_size, upb = Bs / UK;
   const int nvalid = min(p.top_n, t / Bs + 1);
   const int nu = nvalid * upb;
 
-  // blocks in ascending order, each with its position in the selection (at most 64)
+  // blocks in ascending order, each with its position in the selection (at most 64); ids that no key up to t belongs to
+  // are no blocks
   int mine = -1;
   if (lane < nvalid) {
     const int blk = p.topk[(int64_t)kh * p.tk_sh + (int64_t)tok * p.tk_st + lane];
-    mine = blk < 0 ? -1 : blk * 64 + lane;
+    mine = (unsigned)blk > (unsigned)(t / Bs) ? -1 : blk * 64 + lane;
   }
   mine = sort_blocks(mine, nvalid, lane);
 

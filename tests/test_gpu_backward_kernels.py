@@ -143,3 +143,41 @@ def test_selected_forward_around_the_length_from_which_blocks_are_rotated(device
         # P and o are rounded to bf16 once each: 2 * 2^-9 of the largest value
         assert (o[first:, h].float() - s.softmax(-1) @ v[:, kh].float()).abs().max() <= 2 ** -8 * v.float().abs().max()
         assert (lse[first:, h] - s.logsumexp(-1) * 1.4426950408889634).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("block_size", [64, 256])
+def test_selected_gradients_with_rows_behind_the_last_sequence(device, block_size):
+    """Rows of q behind cu_seqlens[-1] belong to no sequence: whatever topk holds there, their dq is left alone and dk / dv are
+    those of the batch without them, up to the order of their fp32 sums.  Ids of blocks that do not exist count as none."""
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd
+    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
+    from flash_nsa.ops.topk import slc_topk_indices
+    cu = make_cu([100, 0, 1400, 333])
+    T, more, QH, KH, D = int(cu[-1]), 70, 16, 1, 128
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T + more, QH, KH, D, seed=370)]
+    do = randn_bf16(T + more, QH, D, seed=374).to(device)
+    setup_helper(cu.to(device), top_n=5, block_size=block_size)
+    ck, cv = mean_pooling_fwd(k[:T]), mean_pooling_fwd(v[:T])
+    _, cl = cmp_attn_fwd(q[:T], ck, cv)
+    topk, _ = slc_topk_indices(q[:T], ck, cl)
+    o, lse = slc_attn_fwd(q[:T], k[:T], v[:T], topk)
+    base = torch.randn(T + more, QH, D, generator=torch.Generator().manual_seed(375)).to(device)
+    ref = slc_attn_bwd(q[:T], k[:T], v[:T], topk, o, lse, do[:T], base[:T].clone())
+    behind = torch.randint(0, 3, (KH, more, 5), generator=torch.Generator().manual_seed(376)).int().to(device)
+    behind[:, 1::4], behind[:, 2::4, 1], behind[:, 3::4, 0] = 2 ** 31 - 1, 2 ** 25 + 1, 2 ** 23 + 1
+    pad = lambda t, value: torch.cat([t, torch.full((more, *t.shape[1:]), value, dtype=t.dtype, device=device)])
+    wide = torch.cat([topk, behind], 1)
+    got = slc_attn_bwd(q, k, v, wide, pad(o, 0.5), pad(lse, 1.0), do, base.clone())
+    assert torch.equal(got[0][T:], base[T:]) and torch.equal(got[0][:T], ref[0])
+    for a, b in zip(got[1:], ref[1:]):
+        assert (a[:T] - b).norm() <= 1e-4 * b.norm() and not a[T:].any()
+    # an id no key up to the query belongs to, in the place of the last block: as if the place were empty
+    last = (torch.arange(1400, device=device) // block_size).clamp(max=4)
+    results = []
+    for value in (-1, 2 ** 31 - 1, 2 ** 25 + 1):
+        t = topk.clone()
+        rows = t[0, 100:1500]
+        rows.scatter_(1, last[:, None], torch.where(last > 2, value, rows.gather(1, last[:, None])[:, 0])[:, None].int())
+        results.append(slc_attn_bwd(q[:T], k[:T], v[:T], t, o, lse, do[:T], base[:T].clone())[0])
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
