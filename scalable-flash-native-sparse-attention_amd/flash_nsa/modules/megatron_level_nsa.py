@@ -216,7 +216,7 @@ class NSAFunction(torch.autograd.Function):
             dcmp_k, dcmp_v = dkdv_cmp()
         _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
         _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
-        if OVERLAP_STREAMS:
+        if OVERLAP_STREAMS and not stored_ds:
             main.wait_stream(side)
         return dq, dk, dv, dw, dwk, dwv, None, None
 
