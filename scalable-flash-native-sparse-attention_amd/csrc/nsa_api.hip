@@ -840,7 +840,10 @@ int nsa_slc_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
 // tokens dQ 10.3 -> 5.55, dK/dV 6.4 -> 6.7 ms, 8 x 6K tokens 5.2 -> 2.93 and 3.84 -> 4.01 ms.
 // The dS of a token takes 32 KB per kv head (16 q-heads, 16 blocks of 64 keys), and 2 GB of it in flight do: longer batches
 // are cut into ranges of tokens (64K tokens, whole step with 1 / 2 / 4 / 8.6 GB: 55.5 / 55.3 / 55.7 / 56.3 ms; 32K tokens 20.5
-// / 20.6 / 20.5 / 20.5 ms), of 512 tokens at least.
+// / 20.6 / 20.5 / 20.5 ms).  The ranges do not grow with the batch, so a block's list per range gets shorter: index, dK/dV and
+// dQ with dq recomputed / with 1 / 2 / 4 / 8 GB, ms, 64 heads: 128K tokens 38.7 / 28.8 / 27.6 / 28.3 / 28.5, 256K 86.4 / 66.5 /
+// 61.0 / 60.9 / 62.1, 512K 184 / 172 / 147 / 144 / 144.  Shapes of which 2 GB do not hold 512 tokens (8 kv heads of 16 q-heads
+// with 64 blocks of 512 keys: 4 GB) compute dq and dk/dv apart: the lists of such ranges would be a few tokens long.
 // No rule on the number of tokens: a query's dq is to be the same bits whatever follows it in the batch.  Steps with dq
 // recomputed / from the dS, us: 16 heads of 128, 16K tokens 2315 / 2277; 64 heads, 4K 1730 / 1744, 8K 3980 / 3863; 32 heads of
 // 192, 4K 1340 / 1402, 16K 6660 / 6630; 16 heads of 64 in 2 groups, 16K 1632 / 1642, 48K 6448 / 6105.
@@ -859,7 +862,8 @@ int nsa_slc_bwd_ds_tokens(int T, int64_t q_sh, int64_t do_sh, int64_t k_sr, int 
   const int64_t budget = (int64_t)nsa_tuning_knob("slc_ds_mb", 2048) << 20;
   const int64_t per_token = nsa_slc_ds_entry_elems(QH / KH, block_size) * 2 * top_n * KH;
   if (budget <= 0) return 0;
-  const int64_t fit = budget / per_token > 512 ? budget / per_token : 512;
+  const int64_t fit = budget / per_token;
+  if (fit < 512) return 0;
   if (fit >= T) return T;
   const int64_t ranges = (T + fit - 1) / fit;
   return (int)((T + ranges - 1) / ranges);

@@ -29,8 +29,8 @@ def slc_attn_fwd(q, k, v, topk, sm_scale=None, helper=NSAHelper, t_begin=0):
 
 def slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale=None, helper=NSAHelper):
     """Tokens per call of the backward that computes dq from the dS of the dk / dv pass, 0 where dq and dk / dv are computed
-    apart.  The scratch holds the dS of so many tokens (2 GB at most: 32 KB per token and kv head for 16 q-heads, 16 blocks
-    of 64 keys)."""
+    apart.  The scratch holds the dS of so many tokens (32 KB per token and kv head for 16 q-heads, 16 blocks of 64 keys), 2 GB
+    at most; shapes of which that does not hold 512 tokens are computed apart."""
     T, QH, D = q.shape
     _, KH, VD = v.shape
     if getattr(helper, "deterministic", False):

@@ -194,6 +194,26 @@ def test_selected_backward_scratch_holds_every_range(monkeypatch, T, QH, KH, top
     buffers.clear()
 
 
+@pytest.mark.parametrize("QH,KH", [(16, 1), (8, 1), (64, 1), (64, 4), (128, 8)])
+@pytest.mark.parametrize("block_size,top_n", [(32, 1), (64, 16), (64, 64), (512, 64), (2048, 64)])
+@pytest.mark.parametrize("limit_mb", [None, 64])
+def test_selected_backward_scratch_has_a_limit(QH, KH, block_size, top_n, limit_mb):
+    """The stored dS keeps to its limit (beside one spare entry per kv head) at every length, or the shape takes the other
+    kernels: also at every length, since a query's dq does not depend on the batch around it."""
+    from flash_nsa import _lib
+    if limit_mb is not None:
+        _lib.call("nsa_set_tuning", b"slc_ds_mb", limit_mb)
+    limit = (2048 if limit_mb is None else limit_mb) << 20
+    size = lambda n: _lib.value("nsa_slc_bwd_ds_bytes", n, QH, KH, block_size, top_n)
+    per_token = size(2) - size(1)
+    taken = set()
+    for T in (1, 100, 511, 513, 5000, 65536, 1000003):
+        n = _lib.value("nsa_slc_bwd_ds_tokens", T, 128, 128, KH * 128, QH, KH, 128, 128, block_size, top_n, 128 ** -0.5)
+        assert 0 <= n <= T and n * per_token <= limit
+        taken.add(n > 0)
+    assert taken == {512 * per_token <= limit}
+
+
 def test_tuning_values_are_set_by_name_not_by_environment():
     from flash_nsa import _lib
     _lib.call("nsa_set_tuning", b"topk_seg_blocks", 64)
