@@ -901,6 +901,7 @@ int nsa_slc_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const vo
                         slc_bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, block_size, top_n, sm_scale));
   if (rc) return rc;
   if (ntok == 0 || n_items_bound <= 0) return NSA_OK;
+  NSA_REQUIRE(csr_slot != nullptr, NSA_ERR_BAD_ARG, "slc_attn_bwd_dkdv_ds: csr_slot, the place of every entry's dS, is null");
   BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
               delta_sh};
   NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);

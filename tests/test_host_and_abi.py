@@ -32,6 +32,9 @@ def test_entry_points_reject_bad_arguments_without_a_gpu():
     with pytest.raises(RuntimeError, match="unsupported head dims"):
         _lib.call("nsa_swa_fwd", None, 0, 0, None, 0, 0, None, 0, 0, None, 0, 0, None, 0, 0, None, 1, 8, 16, 1, 96,
                   96, 512, 1.0, None)
+    with pytest.raises(RuntimeError, match="csr_slot"):  # the list of nsa_build_inverse_index_from, without the places of dS
+        _lib.call("nsa_slc_attn_bwd_dkdv_ds", *(None, 128, 128) * 6, None, 128, 128, None, 128, 128, None, None, None, None, None,
+                  None, None, 1, 64, 1, 1, 16, 1, 128, 128, 64, 4, 0, 8, 0.1, 1 << 20, 1 << 30, None)
 
 
 def test_nsa_helper_metadata():
