@@ -398,7 +398,12 @@ int nsa_cmp_attn_bwd_dq_final_below(const void* q, int64_t q_st, int64_t q_sh, c
 
 // Cost model of a dk/dv work item (128 keys x some query rows, 4 waves): fixed part (K / V fragments, epilogue, summing up)
 // and time per 64-row tile, alone on a CU (tile_us) and as the CU's throughput with `per_cu` of them on it (cu_tile_us).
-// Measured on MI355X; 8 / 16 / 32 / 64 heads per kv head: nsa_bwd_dkdv_dma.hip, else nsa_bwd_dkdv.hip.
+// Measured on MI355X; 8 / 16 / 32 / 64 heads per kv head with 64 or 128 channels: nsa_bwd_dkdv_dma.hip, the others on
+// nsa_bwd_dkdv.hip.  192 / 128 channels run in the former but keep the latter's row (3.2 us per tile, where 2.65 are measured;
+// the comparisons that the rules make hardly move).  us of the cut that the rules take and of the best one there, 32 q / 2 kv
+// heads: compressed, 1200 tokens 41 / 41, 4K 67 / 67, 16K 595 / 567, 64K 7094 / 7094, 8 x 6K 763 / 762, 64 / 4 heads 16K 966 /
+// 966; window, 1200 tokens 74 / 74, 4K 144 / 144, 16K 561 / 545, 64K 2033 / 1999, 8 x 6K 1813 / 1679, 64 / 4 heads 16K 1023 /
+// 1015.
 struct DkdvCost {
   double fixed_us, tile_us, cu_tile_us;
   int per_cu;
@@ -531,12 +536,17 @@ int nsa_cmp_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
 
 
 int nsa_slc_bwd_chunk_tokens(int T, int KH, int top_n) {
-  // List chunk (tokens per work item of the selected-attention dk/dv pass).  An item of 256 tokens takes 200 us at 128
-  // channels (16 q-heads per kv head), so a batch that has fewer of them than the 512 two-wave workgroups the GPU holds
-  // takes that long whatever its size: it is cut finer, down to 64.  Longer items than 256 only add imbalance; shorter
-  // ones than the GPU needs add fp32 atomics.  us at 64 / 128 / 256 / 512 / 1024 tokens, 16 q / 1 kv heads: 2K tokens
-  // 75 / 111 / 200 / 383 / 701, 4K 155 / 131 / 203 / 383 / 749, 8K 300 / 256 / 228 / 387 / 752; 64 / 4 heads: 16K 2043 /
-  // 1812 / 1807 / 1924 / 2071, 8 x 6K 4933 / 4530 / 4465 / 4776 / 5064, 64K 8478 / 7814 / 7584 / 7551 / 7777.
+  // List chunk (tokens per work item of the selected-attention dk/dv pass; T: the tokens of one call, a range of the batch
+  // where the dS is stored).  An item of 256 tokens alone takes 110 us at 128 channels (16 q-heads per kv head), so a batch that
+  // has fewer of them than the 512 workgroups the GPU holds (two per CU at 128 channels) takes that long whatever its size: it
+  // is cut finer, down to 64.  Longer items than 256 only add imbalance; shorter ones than the GPU needs add K / V loads and
+  // fp32 atomics.  us of the kernel that stores dS at 32 / 64 / 128 / 256 / 512 / 1024 tokens, the rule's marked: 16 q / 1 kv
+  // heads of 128, 2K tokens 86 / *59 / 70 / 114 / 212 / 409, 4K 162 / 122 / *103 / 120 / 210 / 408, 8K 302 / 240 / 244 / *265 /
+  // 274 / 411, 16K 548 / 469 / 438 / *468 / 574 / 508; 64 / 4 heads, 4K 512 / 407 / 379 / *381 / 475 / 505, 16K 2207 / 1755 /
+  // 1624 / *1619 / 1603 / 1713, 8 x 6K 7108 / 5634 / 5226 / *5228 / 5395 / 5836, 64K 9276 / 7355 / 6759 / *6530 / 6617 / 6773;
+  // 32 / 2 heads of 192 (one workgroup per CU), 4K 524 / 424 / 353 / *319 / 529 / 567, 16K 2204 / 1640 / 1427 / *1377 / 1431 /
+  // 1450; 16 / 2 heads of 64, 2K 65 / 51 / *38 / 55 / 75 / 140, 16K 431 / 300 / 271 / *264 / 279 / 300, 40 samples of up to
+  // 1.2K 321 / 216 / 181 / *191 / 225 / 253.
   const int64_t want = (int64_t)KH * T * top_n / 512;
   int c = 64;
   while (c < 256 && c * 2 <= want) c *= 2;
