@@ -24,8 +24,8 @@ PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 # what the same counter reads for a 1 GiB copy: x2.000 and x1.000), measured on the T=65536 workload of this file;
 # reported as roofline.traffic for that workload only.
 MEASURED_TRAFFIC_T64K = {
-    "cmp_dkdv": 30.80e9, "slc_fwd": 58.10e9, "cmp_dq": 6.62e9, "topk": 2.28e9, "cmp_fwd": 2.27e9, "swa_dkdv": 11.43e9,
-    "swa_dq": 7.61e9, "swa_fwd": 3.24e9,
+    "slc_bwd": 78.07e9, "cmp_dkdv": 30.80e9, "slc_fwd": 58.10e9, "cmp_dq": 6.62e9, "topk": 2.28e9, "cmp_fwd": 2.27e9,
+    "swa_dkdv": 11.43e9, "swa_dq": 7.61e9, "swa_fwd": 3.24e9,
 }
 PEAK_HBM_GBS = 8000.0
 
@@ -153,18 +153,29 @@ def staged_step(timer, q, k, v, w, wv, do, sm_scale):
     R("cmp_v_bwd", cmp_v_bwd)
 
 
+def selection_pattern(name, T, KH, dev, seed=7):
+    """Block lists [KH, T, 16] of 64-token blocks, all different: the first, the own and the one before it, and, one from each
+    thirteenth of a stretch, of all earlier blocks (`random`) or of the 64 nearest (`clustered`)."""
+    import torch
+    cur = (torch.arange(T, device=dev) // 64)[:, None]
+    i = torch.arange(13, device=dev)
+    first = torch.ones_like(cur) if name == "random" else (cur - 65).clamp(min=1)
+    n = cur - 1 - first
+    lo, hi = first + n * i // 13, first + n * (i + 1) // 13
+    u = torch.rand(KH, T, 13, generator=torch.Generator(device=dev).manual_seed(seed), device=dev)
+    free = torch.where(cur >= 16, lo + (u * (hi - lo)).long().clamp(max=hi - lo - 1), 1 + i)
+    forced = torch.cat([torch.zeros_like(cur), cur, cur - 1], -1)[None].expand(KH, T, 3)
+    return torch.cat([forced, free], -1).to(torch.int32).contiguous()
+
+
 def selected_attention_floor(q, k, v, do, KH, reps=3):
-    """Extra, not part of `value`: the selected-attention forward and dQ kernels on two synthetic selection patterns
-    of the benchmark shape -- `random` (3 forced blocks + 13 uniformly random earlier blocks per token and kv head:
-    what random q / k select, bound by the L2-miss path) and `clustered` (the 13 free blocks drawn from the 64
-    nearest: K/V stay in cache, which shows the kernels' own floor).  Milliseconds per launch."""
+    """Extra, not part of `value`: the selected branch's forward and backward (as the step runs it) on two synthetic
+    selection patterns of the benchmark shape: `random`, as random q / k select, bound by the L2-miss path, and `clustered`,
+    where K / V stay in cache, which shows the kernels' own floor.  Milliseconds per pass."""
     import torch
     from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
     T, QH, D = q.shape
     dev = q.device
-    g = torch.Generator(device=dev).manual_seed(7)
-    cur = torch.arange(T, device=dev) // 64
-    forced = torch.stack([torch.zeros_like(cur), cur, cur - 1], -1)[None].expand(KH, T, 3)
 
     def timed(fn):
         fn()
@@ -179,13 +190,12 @@ def selected_attention_floor(q, k, v, do, KH, reps=3):
 
     out = {}
     for name in ("random", "clustered"):
-        u = torch.rand(KH, T, 13, generator=g, device=dev)
-        free = (u * (cur + 1)[None, :, None]).long() if name == "random" else cur[None, :, None] - (u * 64).long()
-        topk = torch.cat([forced, free], -1).clamp_(min=0).to(torch.int32).contiguous()
+        topk = selection_pattern(name, T, KH, dev)
         o, lse = slc_attn_fwd(q, k, v, topk)
         dq = torch.zeros(T, QH, D, device=dev, dtype=torch.float32)
+        dk, dv = [torch.zeros(t.shape, device=dev, dtype=torch.float32) for t in (k, v)]
         out[name] = {"slc_fwd_ms": round(timed(lambda: slc_attn_fwd(q, k, v, topk)), 3),
-                     "slc_dq_ms": round(timed(lambda: slc_attn_bwd(q, k, v, topk, o, lse, do, dq=dq, parts="dq")), 3)}
+                     "slc_bwd_ms": round(timed(lambda: slc_attn_bwd(q, k, v, topk, o, lse, do, dq=dq, dk=dk, dv=dv)), 3)}
     return out
 
 
@@ -433,7 +443,7 @@ def main():
     fl = stage_flops([T], QH, D, D)
     total_flops = fl["fwd_total"] + fl["bwd_total"]
     mfma_stages = {s: stages[s] for s in stages if s in fl}
-    dom = max((s for s in mfma_stages if s != "slc_bwd"), key=mfma_stages.get)  # of the stages that are one kernel
+    dom = max(mfma_stages, key=mfma_stages.get)  # (slc_bwd: the kernels for dk/dv and dq from the stored dS together)
     achieved = fl[dom] / (stages[dom] * 1e-3) / 1e12
     traffic = MEASURED_TRAFFIC_T64K.get(dom) if T == 65536 else None
     result = {

@@ -81,6 +81,20 @@ def test_bench_flop_model_matches_closed_form():
     assert abs(f["bwd_total"] / 1e12 - 19.19) < 0.01
 
 
+@pytest.mark.parametrize("name", ["random", "clustered"])
+def test_bench_selection_patterns_name_every_block_once(name):
+    """The list builder counts on a query's blocks being different and none behind its own."""
+    import bench
+    T = 9000
+    topk = bench.selection_pattern(name, T, 2, "cpu")
+    cur = torch.arange(T) // 64
+    slot = torch.arange(16)
+    used = slot < (cur[:, None] + 1).clamp(max=16)
+    ids = torch.where(used, topk, -1 - slot.int())
+    assert (ids.sort(-1).values.diff(dim=-1) > 0).all()
+    assert ((topk >= 0) & (topk <= cur[:, None]))[used.expand_as(topk)].all()
+
+
 def test_helper_does_not_confuse_a_new_tensor_with_the_registered_one():
     """A second cu_seqlens tensor with other lengths must be re-registered even when it is as long as the first one
     (an allocator may even hand it the same address); the same unmodified object is recognised without a read."""
