@@ -300,8 +300,9 @@ int nsa_slc_attn_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void*
                           int QH, int KH, int D, int VD, int block_size, float sm_scale, void* stream);
 /* nsa_slc_attn_bwd_dkdv and nsa_slc_attn_bwd_dq_from for the tokens tok0 .. tok0 + ntok - 1 of the batch (with the index that
  * nsa_build_inverse_index_slots makes of them): the dk/dv pass leaves its dS in `ds` (nsa_slc_bwd_ds_bytes(ntok, ...) bytes),
- * from which the dq pass has dq = dS k.  dq_mode 3: bf16 store of the result added to the fp32 dq_partial.  nsa_slc_bwd_ds_tokens: tokens per call for a batch of T tokens, T where one call does;
- * 0: shapes, strides or a scale that take the other entry points. */
+ * from which the dq pass has dq = dS k.  dq_mode 3: bf16 store of the result added to the fp32 dq_partial.
+ * nsa_slc_bwd_ds_tokens: tokens per call for a batch of T tokens, T where one call does; 0: shapes, strides or a scale that
+ * take the other entry points, or shapes of which the scratch's limit (2 GB) does not hold 512 tokens. */
 int nsa_slc_bwd_ds_tokens(int T, int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, int block_size,
                           int top_n, float sm_scale);
 int64_t nsa_slc_bwd_ds_bytes(int ntok, int QH, int KH, int block_size, int top_n);

@@ -5,7 +5,8 @@
 // stored beside it; 32 heads of 192 / 128 (one wave per SIMD), 16K tokens, selected 4574 -> 1535.
 //
 // What bounds it: LDS reads and matrix instructions about equally (each of the four operands is read once per matrix
-// instruction of 32 cycles and SIMD, 4 KB per CU, which LDS delivers in 32 cycles), then instruction issue.  So nothing is
+// instruction of 32 cycles and SIMD, 4 KB per CU, which LDS delivers in 32 cycles; compressed branch at 64K tokens: LDS busy
+// 53 % of the cycles, matrix cores 60 %, at the 1.64 GHz that the power limit leaves), then instruction issue.  So nothing is
 // computed per lane that is uniform, and the order of reads, matrix instructions and softmax arithmetic is fixed (below).
 //
 // A wave keeps the K and V fragments of 32 keys and their dK / dV accumulators in registers (192 of 256 at 128 channels);

@@ -1588,8 +1588,8 @@ static size_t cmp_partial_lds(const NsaDecodeParams& p) {
 
 template <int D, int VD>
 static int launch_cmp_partial(const NsaDecodeParams& p, dim3 grid, hipStream_t stream) {
-  return launch_dyn(p.raw_slots != nullptr ? decode_cmp_partial_kernel<D, VD, true> : decode_cmp_partial_kernel<D, VD, false>, grid, SPLIT_WAVES, cmp_partial_lds<D, VD>(p), stream,
-                    "decode_cmp_partial_kernel", 0, p);
+  return launch_dyn(p.raw_slots != nullptr ? decode_cmp_partial_kernel<D, VD, true> : decode_cmp_partial_kernel<D, VD, false>,
+                    grid, SPLIT_WAVES, cmp_partial_lds<D, VD>(p), stream, "decode_cmp_partial_kernel", 0, p);
 }
 
 template <int D, int VD>

@@ -113,7 +113,8 @@ def nsa_decode(q, k, v, w, context_lens, block_tables, cmp_slot_mapping, cmp_blo
     GPU without it.  Measured, it does not pay on MI355X (one request of 128K tokens: 61.5 us with or without).
     As upstream, the newest token's K/V are expected in the pools already; alternatively pass them as new_k / new_v
     [B,KH,*] with their flat pool rows slot_mapping [B] (-1: padding) and the cache write happens here (inside the
-    single decode launch when that path is taken)."""
+    decode launch that attends the window where that is a fused one).  The rows that a call writes, raw and compressed, have
+    to belong to one request's context each: requests of a batch may share pages, but not a row that this call writes."""
     assert k.size(1) % 64 == 0, "page size must be a multiple of 64"
     check_bf16(w)
     assert all(a >= b for a, b in zip(w.shape, (q.size(0), q.size(1), 3))), "w must be [B,QH,3]"

@@ -59,14 +59,14 @@ def slc_fwd_first_queries(q, k, v, slc_o, slc_lse, all_below, sm_scale=None, hel
 
 def swa_bwd_dq_tail(q, k, v, lse, do, delta, slc_lse, slc_do, slc_delta, all_below, dq, sm_scale=None,
                     helper=NSAHelper, store=False):
-    """dq of the window branch added into (store: written to) the fp32 buffer dq.  lse, delta and slc_lse, slc_delta are combine_bwd_gates'
-    (lse[1], delta[2] and lse[0], delta[1], with the gates in them), with the same all_below: the queries at positions
-    below it also take the selected branch's keys before their window, and their dq is stored."""
+    """dq of the window branch added into (store: written to) the fp32 buffer dq.  lse, delta and slc_lse, slc_delta are
+    combine_bwd_gates' (lse[1], delta[2] and lse[0], delta[1], with the gates in them), with the same all_below: the queries
+    at positions below it also take the selected branch's keys before their window, and their dq is stored."""
     T, QH, D = q.shape
     _, KH, VD = v.shape
     st = lambda t: (t.data_ptr(), t.stride(0), t.stride(1))
-    _lib.call("nsa_swa_bwd_dq_tail_store" if store else "nsa_swa_bwd_dq_tail", *st(q), *st(k), *st(v), *st(do), *st(lse), *st(delta), *st(slc_do), *st(slc_lse),
-              *st(slc_delta), all_below, *st(dq), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH,
+    _lib.call("nsa_swa_bwd_dq_tail_store" if store else "nsa_swa_bwd_dq_tail", *st(q), *st(k), *st(v), *st(do), *st(lse),
+              *st(delta), *st(slc_do), *st(slc_lse), *st(slc_delta), all_below, *st(dq), helper.x_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH,
               KH, D, VD, helper.window_size, default_scale(q, sm_scale), _lib.stream_ptr())
 
 
