@@ -97,12 +97,14 @@ NSA_DEVICE float wave_fmax_uniform(float x) {
 // (cand_v / cand_i), one per lane, in ascending order of the block.  The picks and their order are those of
 // select_blocks_regs (descending score, lowest index on ties); rows with more than 64 scores at the bound (many equal values)
 // take that function.
-// COUNT: bound and places come from counting: every lane compares its value with all others, broadcast one by one, which are
-// independent instructions.  Repeated wave-wide maxima instead are a dependent chain of about 200 ns per round, twice R of
-// them: one request of 32K tokens, 512 blocks, the selection 5.5 -> 2.7 us; 16 of 128K, 2048 blocks, 8.0 -> 5.1.  Where other
-// waves have work of that length beside it (the one-launch decode kernel: the window), the chain costs nothing and the
-// counting's code does: 64 requests of 4K to 32K tokens 73.8 us with the chain, 74.3 counted; 48 of 1K to 9K 46.3 and 46.7.
-template <bool COUNT, int NV, class P>
+// Bound and places come from counting: every lane compares its value with all others, broadcast one by one, which are
+// independent instructions.  (Repeated wave-wide maxima are a dependent chain of about 200 ns per round, twice R of them: one
+// request of 32K tokens, 512 blocks, the selection 5.5 -> 2.7 us; 16 of 128K, 2048 blocks, 8.0 -> 5.1; in the one-launch decode
+// kernel, beside the window, 24 requests of 1K to 4K, 16 / 2 heads of 64, 28.9 -> 26.7 us, 64 / 4 heads of 128, 33.8 -> 33.3.)
+// UNROLL: of the bound's loop.  64 where nothing runs beside the selection (with 8 one request of 32K tokens 35.5 -> 35.7 us);
+// 8 in the one-launch kernel, where more code costs batches that wait for memory and not for this (64 requests of 4K to 32K
+// tokens 73.8 us with maxima, 73.8 with 8, 74.2 with 64; 64 of up to 2K 46.1, 46.4, 46.6).
+template <int UNROLL, int NV, class P>
 NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, const P& p, int lane, float* cand_v,
                                         int* cand_i) {
   const int nk = t >= 0 ? t / p.block_size : -1;
@@ -127,27 +129,12 @@ NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, con
     v[k] = x;
     m = fmaxf(m, x);
   }
-  float theta = -1.f;
-  if constexpr (COUNT) {
-    // bound: the smallest lane maximum that fewer than `rounds` exceed; -1 where fewer lanes than rounds hold a candidate
-    int above = 0;
-#pragma unroll
-    for (int j = 0; j < 64; j++)
-      above += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j)) > m;
-    theta = fmaxf(-wave_fmax_uniform(above < rounds ? -m : -__builtin_inff()), -1.f);
-  } else {
-    // bound: the lane maxima in descending order until `rounds` lanes are counted
-    int counted = 0;
-    for (int r = 0; r < rounds; r++) {
-      const float mx = wave_fmax_uniform(m);
-      if (mx < -1.f) { theta = -1.f; break; }  // fewer lanes than rounds hold a candidate: everything is listed
-      theta = mx;
-      const bool hit = m == mx;
-      counted += __builtin_popcountll(__builtin_amdgcn_ballot_w64(hit));
-      if (hit) m = -4.f;
-      if (counted >= rounds) break;
-    }
-  }
+  // bound: the smallest lane maximum that fewer than `rounds` exceed; -1 where fewer lanes than rounds hold a candidate
+  int above = 0;
+#pragma unroll UNROLL
+  for (int j = 0; j < 64; j++)
+    above += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j)) > m;
+  const float theta = fmaxf(-wave_fmax_uniform(above < rounds ? -m : -__builtin_inff()), -1.f);
   // compaction of the scores >= theta, register by register (ascending block number within a register)
   int base = 0;
 #pragma unroll
@@ -163,15 +150,6 @@ NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, con
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   const float cv = lane < base ? cand_v[lane] : -3.f;
-  if constexpr (!COUNT) {
-    int ci = lane < base ? cand_i[lane] : 0x7fffffff;
-    for (int slot = forced; slot < nsel; slot++) {
-      const int w = wave_argmax_lowest(cv, ci, ci != 0x7fffffff);
-      if (lane == slot) result = w;
-      if (ci == w) ci = 0x7fffffff;
-    }
-    return result;
-  }
   const int ci = lane < base ? cand_i[lane] : 0;
   int place = 0;  // scores ahead of this lane's: greater ones, and equal ones of lower blocks
 #pragma unroll 4

@@ -306,9 +306,9 @@ __global__ __launch_bounds__(256) void topk_pick_kernel(PickParams p) {
   __shared__ float cand_v[4][64];
   __shared__ int cand_i[4][64];
   int result;
-  if (jmax < 512) result = select_blocks_short_list<true, 8>(imp, t, min(cap, 512), p, lane, cand_v[wave], cand_i[wave]);
-  else if (jmax < 1024) result = select_blocks_short_list<true, 16>(imp, t, min(cap, 1024), p, lane, cand_v[wave], cand_i[wave]);
-  else result = select_blocks_short_list<true, 32>(imp, t, min(cap, 2048), p, lane, cand_v[wave], cand_i[wave]);
+  if (jmax < 512) result = select_blocks_short_list<64, 8>(imp, t, min(cap, 512), p, lane, cand_v[wave], cand_i[wave]);
+  else if (jmax < 1024) result = select_blocks_short_list<64, 16>(imp, t, min(cap, 1024), p, lane, cand_v[wave], cand_i[wave]);
+  else result = select_blocks_short_list<64, 32>(imp, t, min(cap, 2048), p, lane, cand_v[wave], cand_i[wave]);
   if (lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + tok * p.tk_st + lane] = result;
 }
 

@@ -113,3 +113,25 @@ def test_selection_by_counting(device, blocks, values):
         rest = [j for j in range(1, blocks - 2)]
         ref = forced + sorted(rest, key=lambda j: (-float(score[kh, j]), j))[:top_n - 3]
         assert topk[kh, 0].tolist() == ref
+
+
+@pytest.mark.parametrize("QH,KH,D", [(16, 2, 64), (32, 2, 128)])
+@pytest.mark.parametrize("blocks", [72, 600])
+def test_one_launch_selection_is_the_oracles(device, QH, KH, D, blocks):
+    """The one-launch kernel's picks against the oracle's, which may differ only between blocks whose scores lie within 1e-3 of
+    each other; capacities of fewer and of more blocks than its smallest selector holds."""
+    from flash_nsa.inference import decode_one_launch
+    from oracle import nsa_oracle as O
+    ctx = [1, 640, 1025, 1777, 4097]
+    case = build_pool(ctx, KH, D, D, seed=21)
+    prepool(case, ctx)
+    q, w = randn_bf16(len(ctx), QH, D, seed=22), randn_bf16(len(ctx), QH, 3, seed=23)
+    lens, cu = torch.tensor(ctx, dtype=torch.int32), torch.arange(len(ctx) + 1, dtype=torch.int32)
+    _, parts = O.nsa_paged_forward(q.float(), case["k"].float(), case["v"].float(), w.float(), cu, lens, case["bt"], case["cbt"],
+                                   O.OracleConfig(block_size=64, top_n=16), return_parts=True)
+    own = torch.cat([p["topk"] for p in parts], 1)
+    topk = decode_one_launch(*[t.to(device) for t in (q, case["k"], case["v"], w, case["bt"], case["cbt"], lens)],
+                             fixed_y_maxlen=512, fixed_num_slc_blocks=blocks, block_size=64, top_n=16, return_parts=True)[4].cpu()
+    _, differ, wrong = O.topk_mismatch_report(topk, own, [p["imp"] for p in parts], cu, 64, 16, tie_tol=1e-3,
+                                              t_offsets=[n - 1 for n in ctx])
+    assert wrong == 0 and differ <= 1
