@@ -43,7 +43,7 @@ struct NsaSlcParams {
   int G, KH, top_n, block_size;
   float scale_log2;
   int t_begin;                                // only queries at positions from here on
-  int sweep;                                  // queries that the GPU holds at once (set by the launcher)
+  int sweep;                                  // queries that the GPU holds at once (set by the launcher; 0: blocks in key order)
 };
 
 struct NsaTopkParams {

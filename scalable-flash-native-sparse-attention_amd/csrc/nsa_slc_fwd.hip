@@ -81,9 +81,9 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   // Where a head's K and V do not fit the 4 MB of an XCD's L2, the waves that run at the same time should be at the same part
   // of the sequence, whenever they started: `sweep` queries run at once, one starts whenever another ends, so query t starts
   // its way through the blocks at the part of them that the others have reached by then, (t / sweep) mod 1.  Every wave still
-  // goes once round, in an order that depends on its position alone.  64 heads of 128, 64K tokens 10.03 -> 8.97 ms; 32 heads
-  // of 192, 16K tokens 1078 -> 1000 us; paged, 16 x 2K queries behind up to 16K 3147 -> 3093 us; below that length 1 % slower.
-  if (t > (4 << 20) / ((D + VD) * 2))
+  // goes once round, in an order that depends on its position (and, paged, on the launch: walk_together) alone.  64 heads of
+  // 128, 64K tokens 10.03 -> 8.97 ms; 32 heads of 192, 16K tokens 1078 -> 1000 us; below that length 1 % slower.
+  if (p.sweep > 0 && t > (4 << 20) / ((D + VD) * 2))
     my_blk = rotate_blocks(my_blk, nvalid, lane, (int)((int64_t)(t % p.sweep) * (t / Bs + 1) / p.sweep));
 
   f32x4 oacc[VD / 16];
@@ -226,13 +226,32 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   }
 }
 
+// Paged: queries far behind their sequence's start are in flight from the launch's first moment on.  The first `sweep` of them
+// start together, and so do the next ones, when those end: all are at the same part of the sequence anyhow, until the waves
+// have drifted apart, and orders that expect starts spread over a wave's time (above) only spread them.  The wider the head,
+// the longer a wave and the later that is.  Chunks shorter than a sweep share it with other sequences and stay close anyhow.
+// Prefill calls without / with the rotation, us, contexts of 8K to 16K before the chunk:
+//   64 / 4 heads of 128 (sweep 3072): 16 x 256 1144 / 1207, 16 x 1024 3157 / 3646, 16 x 1536 4949 / 5009, 16 x 2048 6351 / 6178,
+//     16 x 2560 7971 / 7606, 8 x 2048 3267 / 3238, 4 x 2048 1691 / 1713, 1 x 2048 416 / 449, 5 x 2560 2438 / 2361, 1 x 4096 928 /
+//     909, 4 x 8192 7442 / 6625, 16 / 1 heads: 16 x 2048 1523 / 1556, 4 x 4096 917 / 903, 1 x 8192 494 / 483
+//   32 / 2 heads of 192 (2048): 16 x 1024 2386 / 2783, 4 x 2048 1285 / 1407, 8 x 2048 2443 / 2623, 2 x 4096 1333 / 1460, 4 x 4096
+//     2634 / 2770, 1 x 8192 1464 / 1545, 4 x 8192 6067 / 5827, 1 x 32K from the start 5566 / 5264
+//   16 / 2 heads of 64 (4096): 16 x 1024 849 / 926, 16 x 2048 1550 / 1549, 8 x 3072 1262 / 1232, 4 x 3072 646 / 645, 1 x 4096
+//     260 / 261, 2 x 3.5K to 5K 540 / 524, 2 x 8192 917 / 865
+bool walk_together(int D, int chunk, int64_t queries, int sweep) {
+  if (D <= 128 && chunk * 3 >= sweep * 4) return true;
+  return chunk * 3 >= sweep * 2 && queries / sweep >= (D <= 64 ? 4 : D <= 128 ? 12 : 24);
+}
+
 template <int D, int VD, bool PAGED>
 int launch_slc(const NsaSlcParams& p, int B, int max_q_len, hipStream_t stream) {
   if (!PAGED) max_q_len -= p.t_begin;
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
   dim3 grid(cdiv_i(max_q_len, 4), B, p.KH * ((p.G + 15) / 16));
   NsaSlcParams p2 = p;
-  p2.sweep = nsa_device_cus() * slc_waves(D) * 4;
+  const int sweep = nsa_device_cus() * slc_waves(D) * 4;
+  const bool together = !PAGED || walk_together(D, max_q_len, (int64_t)max_q_len * grid.y * grid.z, sweep);
+  p2.sweep = together ? sweep : 0;
   slc_fwd_kernel<D, VD, PAGED><<<grid, 256, 0, stream>>>(p2);
   return nsa_check_launch("slc_fwd_kernel");
 }

@@ -181,3 +181,28 @@ def test_selected_gradients_with_rows_behind_the_last_sequence(device, block_siz
         rows.scatter_(1, last[:, None], torch.where(last > 2, value, rows.gather(1, last[:, None])[:, 0])[:, None].int())
         results.append(slc_attn_bwd(q[:T], k[:T], v[:T], t, o, lse, do[:T], base[:T].clone())[0])
     assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
+@pytest.mark.parametrize("KH,D,VD,chunk,same", [(1, 128, 128, 4096, True), (1, 128, 128, 130, False), (2, 192, 128, 4096, False)])
+def test_paged_selected_attention_rotates_blocks_in_long_chunks_only(device, KH, D, VD, chunk, same):
+    """A chunk at the end of 9000 tokens: the bits of the unpaged launch where both rotate, else its values up to the order."""
+    from flash_nsa.inference.stages import slc_attn_prefill
+    from flash_nsa.ops.select_attn import slc_attn_fwd
+    from paged_util import build_pool
+    bs, top_n, T, QH = 64, 16, 9000, 16 * KH
+    case = build_pool([T], KH, D, VD, page=128, seed=380)
+    k, v = [O.gather_rows(case[n], case["bt"][0], T).to(device) for n in ("k", "v")]
+    q = randn_bf16(T, QH, D, seed=381).to(device)
+    n = torch.arange(T, device=device) // bs + 1  # blocks up to the own one
+    step = torch.arange(top_n, device=device) * 5 + torch.arange(KH, device=device)[:, None, None]
+    topk = torch.where(n[:, None] > 80, (n[:, None] - 1 - step) % n[:, None], torch.arange(top_n, device=device)).int()
+    setup_helper(make_cu([T]).to(device), block_size=bs, top_n=top_n)
+    first = T - chunk
+    ref, ref_lse = [x[first:] for x in slc_attn_fwd(q, k, v, topk)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
+    o, lse = slc_attn_prefill(q[first:], case["k"].to(device), case["v"].to(device), topk[:, first:], i32([0, chunk]), chunk,
+                              case["bt"].to(device), i32([T]), block_size=bs, top_n=top_n)
+    assert torch.equal(o, ref) == same
+    # P and o are rounded to bf16 once each in either: 4 * 2^-9 of the largest value
+    assert (o.float() - ref.float()).abs().max() <= 2 ** -7 * v.float().abs().max()
+    assert (lse - ref_lse).abs().max() < 1e-4
