@@ -334,6 +334,60 @@ int nsa_slc_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
                               const int32_t* item_off, int nblk_total, int chunk_tokens, int n_items_bound, int B,
                               int QH, int KH, int D, int VD, int block_size, float sm_scale, void* workspace,
                               int64_t workspace_bytes, void* stream);
+/* dQ of the range-keyed branches from the dS that their dk / dv kernels leave behind (8, 16, 32 or 64 q-heads per kv head with
+ * head dims 128/128 or 192/128): the dk / dv kernel of a branch also stores dS, bf16, in tiles of 64 rows, and one
+ * launch forms dQ = dS K of the compressed branch, the window and the keys before the window (of the queries below all_below)
+ * together.  The batch (T rows) is processed in ranges of tokens [tok0, tok1) in ascending order (tok1 = 0: all of it in one;
+ * otherwise the range of 128-position groups of a sequence whose first token it holds), so that the scratch stays bounded:
+ * nsa_bwd_ds_next gives the end of the range that begins at tok0 (T: the last one).
+ * nsa_bwd_ds_takes: 1 where these shapes, strides and scale have this path.  nsa_*_ds_bytes: scratch of a branch; `ring` is
+ * the length of the longest range (0: one range).  The window's scratch holds what the next range needs: the same buffer is
+ * passed for all ranges, and a range's dk / dv kernels run after the dq launch of the range before. */
+int nsa_bwd_ds_takes(int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, float sm_scale);
+int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window);
+int64_t nsa_cmp_attn_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int tok0,
+                                  int tok1);
+int64_t nsa_swa_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int window, int ring);
+int64_t nsa_slc_bwd_before_window_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int window, int all_below, int ring);
+/* nsa_cmp_attn_bwd_dkdv that stores dS.  Without workspace dck / dcv are added into with fp32 atomics; with
+ * nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(...) bytes of it the work items' sums are added in a fixed order and stored (add: added
+ * to what the ranges before have left). */
+int64_t nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
+                                            int kernel_size, int stride, int tok0, int tok1);
+int nsa_cmp_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
+                             const void* cv, int64_t cv_sr, int64_t cv_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                             const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                             int64_t delta_sh, float* dck, int64_t dck_sr, int64_t dck_sh, float* dcv, int64_t dcv_sr,
+                             int64_t dcv_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int y_maxlen,
+                             int QH, int KH, int D, int VD, int kernel_size, int stride, float sm_scale, int T, int tok0,
+                             int tok1, void* ds, int64_t ds_bytes, void* workspace, int64_t workspace_bytes, int add,
+                             void* stream);
+/* nsa_swa_bwd_dkdv_ws and nsa_slc_attn_bwd_dkdv_before_window that store dS: keys of the range, every key once. */
+int64_t nsa_swa_bwd_dkdv_ds_ws_bytes(int T, int B, int x_maxlen, int QH, int KH, int D, int VD, int window, int tok0,
+                                     int tok1);
+int nsa_swa_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, void* dk, int64_t dk_sr, int64_t dk_sh, void* dv, int64_t dv_sr,
+                        int64_t dv_sh, int dkv_is_f32, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D,
+                        int VD, int window, float sm_scale, int T, int ring, int tok0, int tok1, void* ds,
+                        int64_t ds_bytes, void* workspace, int64_t workspace_bytes, void* stream);
+int nsa_slc_attn_bwd_dkdv_before_window_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr,
+                                           int64_t k_sh, const void* v, int64_t v_sr, int64_t v_sh, const void* dO,
+                                           int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st,
+                                           int64_t lse_sh, const float* delta, int64_t delta_st, int64_t delta_sh,
+                                           float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                                           int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH,
+                                           int D, int VD, int window, int all_below, float sm_scale, int T, int ring,
+                                           int tok0, int tok1, void* ds, int64_t ds_bytes, void* stream);
+/* dq of the tokens of a range from what the calls above have stored (a null dS leaves the branch out).  dq_mode 0: bf16, 1:
+ * fp32, 2: added into fp32, 3: bf16 to dq at positions below all_below, fp32 to dq_partial for the others. */
+int nsa_attn_bwd_dq_ds(const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cmp_ds, int64_t cmp_ds_bytes, const void* k,
+                       int64_t k_sr, int64_t k_sh, const void* swa_ds, int64_t swa_ds_bytes, const void* far_ds,
+                       int64_t far_ds_bytes, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, float* dq_partial,
+                       int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH,
+                       int KH, int D, int VD, int kernel_size, int stride, int window, int all_below, float sm_scale, int T,
+                       int ring, int tok0, int tok1, void* stream);
 
 /* ---- paged KV (inference).  Caches are [num_pages, page_size, KH, D]; *_sr is the stride of a flat row
  * (page*page_size + offset), *_sh the head stride.  Request b's raw token n lives at flat row

@@ -34,6 +34,7 @@ Knob g_knobs[] = {
     {"decode_waves", {0}, {false}},     // waves per workgroup of the one-launch decode kernel (0: from the batch; 4, 8)
     {"swa_dkdv_splits", {0}, {false}},  // query chunks per key tile of the window dk/dv kernel (0: from the sizes)
     {"slc_ds_mb", {0}, {false}},        // scratch for the dS of the selected branch, MB (0: dq and dk/dv computed apart)
+    {"dense_ds_mb", {0}, {false}},      // scratch for the dS of the compressed branch, and for the window's, MB
     {"topk_two_pass", {0}, {false}},    // 0: the one-launch selector even when a workspace is given
 };
 Knob* find_knob(const char* name) {
@@ -97,7 +98,8 @@ int nsa_abi_version(void) { return 1; }
 int nsa_set_tuning(const char* name, int value) {
   Knob* k = name ? find_knob(name) : nullptr;
   NSA_REQUIRE(k != nullptr, NSA_ERR_BAD_ARG, "set_tuning: unknown name '%s' (fwd_variant, dq_min_blocks, "
-              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, decode_waves, slc_ds_mb, topk_two_pass)", name ? name : "(null)");
+              "dkdv_key_blocks, topk_seg_blocks, swa_dkdv_splits, decode_waves, slc_ds_mb, dense_ds_mb, "
+              "topk_two_pass)", name ? name : "(null)");
   k->value.store(value);
   k->is_set.store(true);
   return NSA_OK;
@@ -425,30 +427,32 @@ static DkdvCost dkdv_cost(int G, int D, int VD) {
 
 // Query tokens per work item of the compressed dk/dv kernel when the caller leaves the choice to the library.
 static int cmp_dkdv_q_chunk(int q_chunk_tokens, int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
-                            int kernel_size, int stride) {
+                            int kernel_size, int stride, int lo = 0) {
   if (q_chunk_tokens <= 0) {
     // A work item is one (128-key tile, query chunk that sees it, kv head, sequence).  The launch takes as long as its
     // longest item when there are fewer items than workgroup slots, else about all the work over the slots plus a
     // quarter of an item for the last, partly empty round.  The chunk (a power of two in [32, 2048]) that minimises
-    // this for the longest sequence is taken.  Fitted to sweeps of all chunks over one to forty sequences of 600 to 64K
-    // tokens (chunk 64 / 128 / 256 / 512 / 2048, d = 128: 16 q / 1 kv heads, 4096 tokens 53 / 86 / 157 / 304 / 1150 us;
-    // 64 / 4 heads, 16K tokens 701 / 587 / 610 / 726 / 1166 us, 64K 10.3 / 9.3 / 8.6 / 8.1 / 8.8 ms).
+    // this for the longest sequence (its queries from position lo on) is taken.  Fitted to sweeps of all chunks over one to
+    // forty sequences of 600 to 64K tokens (chunk 64 / 128 / 256 / 512 / 2048, d = 128: 16 q / 1 kv heads, 4096 tokens 53 /
+    // 86 / 157 / 304 / 1150 us; 64 / 4 heads, 16K tokens 701 / 587 / 610 / 726 / 1166 us, 64K 10.3 / 9.3 / 8.6 / 8.1 / 8.8
+    // ms).
     const int G = QH / KH;
     const DkdvCost c = dkdv_cost(G, D, VD);
     double best = 0.0;
     for (int chunk = 32; chunk <= 2048; chunk *= 2) {
-      const int64_t nch = (x_maxlen + chunk - 1) / chunk;
+      const int64_t nch = (x_maxlen - lo + chunk - 1) / chunk;
       int64_t items = 0;
       double rows = 0.0;
       for (int64_t kt = 0; kt * 128 < y_maxlen; kt++) {
-        const int64_t first = (int64_t)stride * kt * 128 + kernel_size - 1;
-        if (first >= x_maxlen) break;
+        const int64_t at = (int64_t)stride * kt * 128 + kernel_size - 1, first = at > lo ? at - lo : 0;
+        if (first >= x_maxlen - lo) break;
         items += nch - first / chunk;
-        rows += (double)(x_maxlen - first) * G;
+        rows += (double)(x_maxlen - lo - first) * G;
       }
       items *= (int64_t)B * KH;
       rows *= (double)B * KH;
-      const double item = c.item(items, (double)(chunk < x_maxlen ? chunk : x_maxlen) * G / 64.0);
+      const int n = chunk < x_maxlen - lo ? chunk : x_maxlen - lo;
+      const double item = c.item(items, (double)n * G / 64.0);
       const double all = items * c.fixed_us / c.slots() + rows / 64.0 * c.cu_tile_us / nsa_device_cus() + 0.25 * item;
       const double cost = items <= c.slots() || all < item ? item : all;
       if (q_chunk_tokens <= 0 || cost < best) { best = cost; q_chunk_tokens = chunk; }
@@ -482,7 +486,8 @@ static int cmp_attn_bwd_dkdv_impl(const void* q, int64_t q_st, int64_t q_sh, con
   if (!deterministic) return nsa_bwd_dkdv_launch(p, 0, B, x_maxlen, y_maxlen, D, VD, 0, (hipStream_t)stream);
   if (B <= 0 || y_maxlen <= 0) return NSA_OK;
   // every work item stores into its own slot, then one pass sums the slots of a key in ascending chunk order
-  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, q_chunk_tokens, kernel_size, stride);
+  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, q_chunk_tokens, kernel_size, stride, 0, 0,
+                                               B);
   const int64_t kw = nsa_bwd_dkdv_slot_keys(0, 0, D);
   const int64_t dk_bytes = (slots * kw * D * 4 + 255) & ~(int64_t)255;
   const int64_t need = dk_bytes + slots * kw * VD * 4;
@@ -494,7 +499,7 @@ static int cmp_attn_bwd_dkdv_impl(const void* q, int64_t q_st, int64_t q_sh, con
   p.part_dv = (float*)((char*)workspace + dk_bytes);
   rc = nsa_bwd_dkdv_launch(p, 0, B, x_maxlen, y_maxlen, D, VD, 0, (hipStream_t)stream);
   if (rc) return rc;
-  return nsa_dkdv_reduce_cmp_launch(p, B, x_maxlen, y_maxlen, D, VD, (hipStream_t)stream);
+  return nsa_dkdv_reduce_cmp_launch(p, false, B, x_maxlen, y_maxlen, D, VD, (hipStream_t)stream);
 }
 
 int nsa_cmp_attn_bwd_dkdv(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
@@ -514,7 +519,8 @@ int64_t nsa_cmp_attn_bwd_dkdv_det_bytes(int B, int x_maxlen, int y_maxlen, int Q
                                         int kernel_size, int stride, int q_chunk_tokens) {
   if (B <= 0 || x_maxlen <= 0 || y_maxlen <= 0 || KH <= 0 || QH <= 0 || stride <= 0) return 0;
   q_chunk_tokens = cmp_dkdv_q_chunk(q_chunk_tokens, B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride);
-  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, q_chunk_tokens, kernel_size, stride);
+  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, q_chunk_tokens, kernel_size, stride, 0, 0,
+                                               B);
   const int64_t kw = nsa_bwd_dkdv_slot_keys(0, 0, D);
   return ((slots * kw * D * 4 + 255) & ~(int64_t)255) + slots * kw * VD * 4;
 }
@@ -626,8 +632,10 @@ static int64_t swa_dkdv_slot_bytes(int splits, int B, int x_maxlen, int KH, int 
   return *dk_bytes + rows * VD * 4;
 }
 
-// Query chunks per key tile of the window branch's dk/dv; at most max_bytes of partial results.
-static int swa_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, int window, int64_t max_bytes) {
+// Query chunks per key tile of the window branch's dk/dv; at most max_bytes of partial results.  tokens: of the batch, where the
+// caller knows.
+static int swa_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, int window, int64_t max_bytes,
+                           int tokens = 0) {
   if (B <= 0 || x_maxlen <= 0 || QH <= 0 || KH <= 0) return 1;
   const int knob = nsa_tuning_knob("swa_dkdv_splits", 0);
   if (knob > 0) return knob > 16 ? 16 : knob;
@@ -636,7 +644,8 @@ static int swa_dkdv_splits(int B, int x_maxlen, int QH, int KH, int D, int VD, i
   // sequence of 4096 tokens, 16 q / 1 kv heads 365 / 196 / 110 / 70 / 63 us, 64 q / 4 kv heads 389 / 224 / 167 / 206 /
   // 256 us; 8192 tokens, 64 q / 4 kv heads 422 / 333 / 370 / 397 / 486 us.
   const DkdvCost c = dkdv_cost(QH / KH, D, VD);
-  const int64_t wgs = (int64_t)((x_maxlen + 127) / 128) * B * KH;
+  int64_t wgs = (int64_t)((x_maxlen + 127) / 128) * B * KH;
+  if (tokens > 0 && ((int64_t)tokens / 128 + B) * KH < wgs) wgs = ((int64_t)tokens / 128 + B) * KH;
   const double tiles = (128.0 + (window < x_maxlen ? window : x_maxlen)) * (QH / KH) / 64.0;
   int best = 1;
   double best_cost = 0.0;
@@ -955,6 +964,320 @@ int nsa_slc_attn_bwd_dq_ds(const void* k, int64_t k_sr, int64_t k_sh, const int3
   p.t_begin = t_begin; p.tok0 = tok0; p.ntok = ntok;
   p.sm_scale = sm_scale;
   return nsa_slc_dq_ds_launch(p, D, (hipStream_t)stream);
+}
+
+// ---- dQ of the range-keyed branches from stored dS.  A 64-row tile's dS takes 4 KB per 32 keys that it sees.
+// What it is worth: whole step with dq recomputed / from the dS, us: 64 heads of 128, 64K tokens 53.2 / 50.7 ms, 8 x 6K 20500 /
+// 19060, 16K 8200 / 7760; 32 heads of 192, 16K 6500 / 5800, 20 samples of up to 2K 4700 / 4320; 16 heads of 128, 4K 850 / 711,
+// 16K 2212 / 2115, 30 samples of up to 1.5K 1364 / 1201.  Not with 64 channels, whose dS is as large for half of the products:
+// 16 heads in 2 groups, 16K 1602 / 1699, 48K 5810 / 6207.
+namespace {
+struct DsLayout {
+  int tiles, seq_tiles, pitch;
+  int64_t sh, bytes;  // elements per kv head, bytes in all
+};
+// 68 KB behind the last tile that nobody reads
+DsLayout ds_layout(int64_t tiles, int seq_tiles, int pitch, int KH) {
+  DsLayout l;
+  l.tiles = (int)tiles; l.seq_tiles = seq_tiles; l.pitch = pitch;
+  l.sh = tiles * pitch * 2048;
+  l.bytes = (l.sh * KH + 68 * 512) * 2;
+  return l;
+}
+int64_t ds_all_tiles(int T, int B, int G) { return (int64_t)T * G / 64 + B + 1; }
+// compressed branch, the tokens tok0 .. tok1 - 1 (tok1 = 0: all).  Several sequences: any of them may be the longest.
+DsLayout ds_layout_cmp(int T, int B, int x_maxlen, int G, int KH, int kernel_size, int stride, int tok0, int tok1) {
+  const int end = B == 1 && tok1 > 0 && ((tok1 + 127) & ~127) < x_maxlen ? (tok1 + 127) & ~127 : x_maxlen;
+  const int keys = end >= kernel_size ? (end - kernel_size) / stride + 1 : 0;
+  int64_t tiles = ds_all_tiles(T, B, G);
+  if (tok1 > 0) {
+    const int64_t n = (int64_t)(tok1 - tok0 + 127) * G / 64 + B + 2;
+    if (n < tiles) tiles = n;
+  }
+  return ds_layout(tiles, 0, keys > 0 ? (keys + 31) / 32 : 1, KH);
+}
+// window, and the keys before it of the queries below all_below: ranges of up to `ring` tokens (0: all in one).  The keys of a
+// range leave dS for the tokens up to reach behind them, so the tiles of a range and of those are kept.
+int64_t ds_ring_tiles(int T, int B, int G, int ring, int64_t reach) {
+  const int64_t all = ds_all_tiles(T, B, G);
+  if (ring <= 0) return all;
+  const int64_t n = (ring + 127 + 128 + reach + 8) * G / 64 + B + 2;
+  return n < all ? n : all;
+}
+DsLayout ds_layout_win(int T, int B, int x_maxlen, int G, int KH, int window, int ring) {
+  const int w = window < x_maxlen ? window : x_maxlen;
+  int pitch = (w + 64 / G - 1) / 32 + 2;
+  if (pitch > (x_maxlen + 31) / 32) pitch = (x_maxlen + 31) / 32;
+  return ds_layout(ds_ring_tiles(T, B, G, ring, w), 0, pitch > 0 ? pitch : 1, KH);
+}
+// pitch 0: no query has such keys
+DsLayout ds_layout_far(int T, int B, int x_maxlen, int G, int KH, int window, int all_below, int ring) {
+  const int end = all_below < x_maxlen ? all_below : x_maxlen;
+  if ((int64_t)end - 1 - window - 1 < 0) return DsLayout{0, 0, 0, 0, 0};
+  const int pitch = (end - 1 - window - 1) / 32 + 1;
+  const int seq_tiles = (end * G + 63) / 64;
+  const int64_t tiles = ds_ring_tiles(T, B, G, ring, end);
+  if ((int64_t)seq_tiles * B < tiles) return ds_layout((int64_t)seq_tiles * B, seq_tiles, pitch, KH);
+  return ds_layout(tiles, 0, pitch, KH);
+}
+void set_ds(NsaBwdTileParams& p, const DsLayout& l, void* ds, int tok0, int tok1) {
+  p.ds = (bf16_t*)ds; p.ds_sh = l.sh;
+  p.ds_tiles = l.tiles; p.ds_seq_tiles = l.seq_tiles; p.ds_pitch = l.pitch;
+  p.tok0 = tok0; p.tok1 = tok1;
+}
+NsaDsOperand ds_operand(const DsLayout& l, const void* k, int64_t k_sr, int64_t k_sh, const void* ds) {
+  return NsaDsOperand{(const bf16_t*)k, k_sr, k_sh, (const bf16_t*)ds, l.sh, l.tiles, l.seq_tiles, l.pitch};
+}
+int check_ds(const char* who, int QH, int KH, int D, int VD, int T, int B, int x_maxlen, int tok0, int tok1, const void* ds,
+             int64_t ds_bytes, int64_t need, bool takes) {
+  int rc = check_heads(who, QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(T >= 0 && B >= 0 && x_maxlen >= 0 && x_maxlen <= T && tok0 >= 0 && tok1 >= 0 && (tok1 == 0 || tok0 < tok1),
+              NSA_ERR_BAD_ARG, "%s: tokens %d to %d of %d in %d sequences", who, tok0, tok1, T, B);
+  NSA_REQUIRE(takes, NSA_ERR_UNSUPPORTED, "%s: these shapes have no stored dS", who);
+  NSA_REQUIRE(ds != nullptr && ds_bytes >= need, NSA_ERR_WORKSPACE, "%s: dS buffer of %lld bytes, %lld needed", who,
+              (long long)ds_bytes, (long long)need);
+  return NSA_OK;
+}
+bool bwd_ds_takes(int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, float sm_scale) {
+  if (D < 128 || KH <= 0 || QH % KH != 0 || k_sr < 0 || k_sr >= (1 << 26)) return false;
+  if (nsa_tuning_knob("dkdv_key_blocks", 1) == 2) return false;
+  NsaBwdTileParams p{};
+  p.G = QH / KH; p.q_sh = q_sh; p.do_sh = do_sh; p.scale_log2 = sm_scale * NSA_LOG2E;
+  return nsa_bwd_dkdv_dma_takes(p, D, VD);
+}
+}  // namespace
+
+int nsa_bwd_ds_takes(int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, float sm_scale) {
+  return bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, sm_scale);
+}
+
+int64_t nsa_cmp_attn_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int tok0,
+                                  int tok1) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || stride <= 0) return 0;
+  return ds_layout_cmp(T, B, x_maxlen, QH / KH, KH, kernel_size, stride, tok0, tok1).bytes;
+}
+int64_t nsa_swa_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int window, int ring) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH) return 0;
+  return ds_layout_win(T, B, x_maxlen, QH / KH, KH, window, ring).bytes;
+}
+int64_t nsa_slc_bwd_before_window_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int window, int all_below, int ring) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH) return 0;
+  return ds_layout_far(T, B, x_maxlen, QH / KH, KH, window, all_below, ring).bytes;
+}
+
+// End of the range of tokens that begins at tok0: 4 GB for the compressed branch's dS, and the window's, but never fewer tokens
+// than give the dQ kernel 512 workgroups of 256 rows, and no shorter rest.  Whole step with 2 / 4 / 8 / 40 GB, 64 heads of 128,
+// ms: 64K tokens 52.7 / 52.2 / 51.8 / 52.2, 8 x 6K 19.9 / 19.2 / 19.2 / 19.2.  (As for the selected branch no rule on the number
+// of tokens decides whether dq comes from stored dS: a query's dq is to be the same bits whatever follows it in the batch.)
+int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || stride <= 0 || tok0 >= T) return T;
+  const int G = QH / KH;
+  const int64_t budget = (int64_t)nsa_tuning_knob("dense_ds_mb", 4096) << 20;
+  auto fits = [&](int tok1) {
+    return ds_layout_cmp(T, B, x_maxlen, G, KH, kernel_size, stride, tok0, tok1).bytes <= budget &&
+           ds_layout_win(T, B, x_maxlen, G, KH, window, tok1 - tok0).bytes <= budget;
+  };
+  if (fits(T)) return T;
+  const int least = (131072 / QH + 127) & ~127;
+  int lo = tok0 + least;
+  if (lo >= T) return T;
+  int hi = T;  // fits(lo) or lo is the least; !fits(hi)
+  while (hi - lo > 128) {
+    const int mid = lo + (((hi - lo) / 2 + 127) & ~127);
+    if (mid >= hi) break;
+    if (fits(mid)) lo = mid; else hi = mid;
+  }
+  return T - lo < least ? T : lo;
+}
+
+int64_t nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
+                                            int kernel_size, int stride, int tok0, int tok1) {
+  if (B <= 0 || x_maxlen <= 0 || y_maxlen <= 0 || KH <= 0 || QH < KH || stride <= 0) return 0;
+  int lo, hi;
+  nsa_local_range(tok0, tok1, 0, x_maxlen, lo, hi);
+  if (B > 1) { lo = 0; hi = x_maxlen; }
+  const int chunk = cmp_dkdv_q_chunk(0, B, hi, y_maxlen, QH, KH, D, VD, kernel_size, stride, lo);
+  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, chunk, kernel_size, stride, tok0, tok1, B);
+  const int64_t kw = nsa_bwd_dkdv_slot_keys(0, 0, D);
+  return ((slots * kw * D * 4 + 255) & ~(int64_t)255) + slots * kw * VD * 4;
+}
+
+int nsa_cmp_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
+                             const void* cv, int64_t cv_sr, int64_t cv_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                             const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                             int64_t delta_sh, float* dck, int64_t dck_sr, int64_t dck_sh, float* dcv, int64_t dcv_sr,
+                             int64_t dcv_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int y_maxlen,
+                             int QH, int KH, int D, int VD, int kernel_size, int stride, float sm_scale, int T, int tok0,
+                             int tok1, void* ds, int64_t ds_bytes, void* workspace, int64_t workspace_bytes, int add,
+                             void* stream) {
+  const DsLayout l = KH > 0 && QH >= KH && stride > 0
+                         ? ds_layout_cmp(T, B, x_maxlen, QH / KH, KH, kernel_size, stride, tok0, tok1) : DsLayout{};
+  int rc = check_ds("cmp_attn_bwd_dkdv_ds", QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, ds, ds_bytes, l.bytes,
+                    bwd_ds_takes(q_sh, do_sh, ck_sr, QH, KH, D, VD, sm_scale));
+  if (rc) return rc;
+  rc = check_nsa_sizes("cmp_attn_bwd_dkdv_ds", kernel_size, stride, 0);
+  if (rc) return rc;
+  if (B <= 0 || x_maxlen <= 0 || y_maxlen <= 0) return NSA_OK;
+  BwdCommon c{q, q_st, q_sh, ck, ck_sr, ck_sh, cv, cv_sr, cv_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta,
+              delta_st, delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dk = dck; p.dk_sr = dck_sr; p.dk_sh = dck_sh;
+  p.dv = dcv; p.dv_sr = dcv_sr; p.dv_sh = dcv_sh;
+  p.dkv_mode = 3;
+  p.x_cu = x_cu; p.k_cu = y_cu;
+  p.kernel_size = kernel_size; p.stride = stride;
+  set_ds(p, l, ds, tok0, tok1);
+  int lo, hi;
+  nsa_local_range(tok0, tok1, 0, x_maxlen, lo, hi);
+  if (B > 1) { lo = 0; hi = x_maxlen; }
+  p.q_chunk_tokens = cmp_dkdv_q_chunk(0, B, hi, y_maxlen, QH, KH, D, VD, kernel_size, stride, lo);
+  if (workspace == nullptr) return nsa_bwd_dkdv_launch(p, 0, B, x_maxlen, y_maxlen, D, VD, 0, (hipStream_t)stream);
+  const int64_t need = nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride, tok0, tok1);
+  NSA_REQUIRE(workspace_bytes >= need, NSA_ERR_WORKSPACE, "cmp_attn_bwd_dkdv_ds: workspace of %lld bytes, %lld needed",
+              (long long)workspace_bytes, (long long)need);
+  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, p.q_chunk_tokens, kernel_size, stride, tok0, tok1, B);
+  p.dkv_mode = 4;
+  p.part_dk = (float*)workspace;
+  p.part_dv = (float*)((char*)workspace + ((slots * nsa_bwd_dkdv_slot_keys(0, 0, D) * D * 4 + 255) & ~(int64_t)255));
+  rc = nsa_bwd_dkdv_launch(p, 0, B, x_maxlen, y_maxlen, D, VD, 0, (hipStream_t)stream);
+  if (rc) return rc;
+  return nsa_dkdv_reduce_cmp_launch(p, add != 0, B, x_maxlen, y_maxlen, D, VD, (hipStream_t)stream);
+}
+
+// The partial results of a ragged batch are mostly address space: slots are numbered by its longest sequence.
+static const int64_t SWA_DS_SLOTS_LIMIT = (int64_t)512 << 20;
+
+// length of the longest share of a sequence
+static int ds_share(int x_maxlen, int tok0, int tok1) {
+  return tok1 > 0 && tok1 - tok0 + 127 < x_maxlen ? tok1 - tok0 + 127 : x_maxlen;
+}
+
+static int swa_ds_splits(int T, int B, int x_maxlen, int QH, int KH, int D, int VD, int window, int tok0, int tok1) {
+  return swa_dkdv_splits(B, ds_share(x_maxlen, tok0, tok1), QH, KH, D, VD, window, SWA_DS_SLOTS_LIMIT,
+                         tok1 > 0 ? tok1 - tok0 : T);
+}
+
+int64_t nsa_swa_bwd_dkdv_ds_ws_bytes(int T, int B, int x_maxlen, int QH, int KH, int D, int VD, int window, int tok0,
+                                     int tok1) {
+  const int splits = swa_ds_splits(T, B, x_maxlen, QH, KH, D, VD, window, tok0, tok1);
+  int64_t dk_bytes;
+  return splits > 1 ? swa_dkdv_slot_bytes(splits, B, ds_share(x_maxlen, tok0, tok1), KH, D, VD, &dk_bytes) : 0;
+}
+
+int nsa_swa_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
+                        const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
+                        const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
+                        int64_t delta_sh, void* dk, int64_t dk_sr, int64_t dk_sh, void* dv, int64_t dv_sr,
+                        int64_t dv_sh, int dkv_is_f32, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D,
+                        int VD, int window, float sm_scale, int T, int ring, int tok0, int tok1, void* ds,
+                        int64_t ds_bytes, void* workspace, int64_t workspace_bytes, void* stream) {
+  const DsLayout l = KH > 0 && QH >= KH ? ds_layout_win(T, B, x_maxlen, QH / KH, KH, window, ring) : DsLayout{};
+  int rc = check_ds("swa_bwd_dkdv_ds", QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, ds, ds_bytes, l.bytes,
+                    bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, sm_scale));
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0 && (ring == 0 ? tok1 == 0 : tok1 > 0 && tok1 - tok0 <= ring), NSA_ERR_BAD_ARG,
+              "swa_bwd_dkdv_ds: window %d, tokens %d to %d in ranges of up to %d", window, tok0, tok1, ring);
+  if (B <= 0 || x_maxlen <= 0) return NSA_OK;
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
+  p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
+  p.dkv_mode = dkv_is_f32 ? 1 : 0;
+  const int share = ds_share(x_maxlen, tok0, tok1);
+  p.grid_chunks = workspace != nullptr ? swa_ds_splits(T, B, x_maxlen, QH, KH, D, VD, window, tok0, tok1) : 1;
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.window = window;
+  set_ds(p, l, ds, tok0, tok1);
+  if (p.grid_chunks > 1) {
+    int64_t dk_bytes;
+    const int64_t need = swa_dkdv_slot_bytes(p.grid_chunks, B, share, KH, D, VD, &dk_bytes);
+    NSA_REQUIRE(workspace_bytes >= need, NSA_ERR_WORKSPACE, "swa_bwd_dkdv_ds: workspace of %lld bytes, %lld needed",
+                (long long)workspace_bytes, (long long)need);
+    p.dkv_mode = 4;
+    p.part_dk = (float*)workspace;
+    p.part_dv = (float*)((char*)workspace + dk_bytes);
+  }
+  rc = nsa_bwd_dkdv_launch(p, 1, B, x_maxlen, x_maxlen, D, VD, 0, (hipStream_t)stream);
+  if (rc || p.grid_chunks == 1) return rc;
+  return nsa_dkdv_reduce_swa_launch(p, dkv_is_f32 != 0, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
+int nsa_slc_attn_bwd_dkdv_before_window_ds(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr,
+                                           int64_t k_sh, const void* v, int64_t v_sr, int64_t v_sh, const void* dO,
+                                           int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st,
+                                           int64_t lse_sh, const float* delta, int64_t delta_st, int64_t delta_sh,
+                                           float* dk, int64_t dk_sr, int64_t dk_sh, float* dv, int64_t dv_sr,
+                                           int64_t dv_sh, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH,
+                                           int D, int VD, int window, int all_below, float sm_scale, int T, int ring,
+                                           int tok0, int tok1, void* ds, int64_t ds_bytes, void* stream) {
+  const DsLayout l = KH > 0 && QH >= KH ? ds_layout_far(T, B, x_maxlen, QH / KH, KH, window, all_below, ring) : DsLayout{};
+  NSA_REQUIRE(window >= 0 && all_below >= 0 && all_below % 8 == 0 && (ring == 0 ? tok1 == 0 : tok1 > 0 && tok1 - tok0 <= ring),
+              NSA_ERR_BAD_ARG, "slc_attn_bwd_dkdv_before_window_ds: window %d, all_below %d, tokens %d to %d in ranges of up to %d",
+              window, all_below, tok0, tok1, ring);
+  if (l.pitch == 0) return NSA_OK;  // no query has keys before its window
+  int rc = check_ds("slc_attn_bwd_dkdv_before_window_ds", QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, ds, ds_bytes, l.bytes,
+                    bwd_ds_takes(q_sh, do_sh, k_sr, QH, KH, D, VD, sm_scale));
+  if (rc) return rc;
+  const int len = (x_maxlen < all_below ? x_maxlen : all_below) - window - 1;  // positions that are some query's keys
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dk = dk; p.dk_sr = dk_sr; p.dk_sh = dk_sh;
+  p.dv = dv; p.dv_sr = dv_sr; p.dv_sh = dv_sh;
+  p.dkv_mode = 3;
+  p.grid_chunks = swa_dkdv_splits(B, len, QH, KH, D, VD, len, INT64_MAX);
+  p.x_cu = x_cu; p.k_cu = x_cu;
+  p.min_dist = window + 1; p.window = all_below; p.t_end = all_below;
+  set_ds(p, l, ds, tok0, tok1);
+  return nsa_bwd_dkdv_launch(p, 1, B, x_maxlen, x_maxlen, D, VD, 0, (hipStream_t)stream);
+}
+
+int nsa_attn_bwd_dq_ds(const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cmp_ds, int64_t cmp_ds_bytes, const void* k,
+                       int64_t k_sr, int64_t k_sh, const void* swa_ds, int64_t swa_ds_bytes, const void* far_ds,
+                       int64_t far_ds_bytes, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, float* dq_partial,
+                       int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH,
+                       int KH, int D, int VD, int kernel_size, int stride, int window, int all_below, float sm_scale, int T,
+                       int ring, int tok0, int tok1, void* stream) {
+  const char* const who = "attn_bwd_dq_ds";
+  int rc = check_heads(who, QH, KH, D, VD);
+  if (rc) return rc;
+  NSA_REQUIRE(cmp_ds != nullptr || swa_ds != nullptr, NSA_ERR_BAD_ARG, "%s: no branch's dS", who);
+  NSA_REQUIRE(dq_mode >= 0 && dq_mode <= 3 && (dq_mode != 3 || dq_partial != nullptr) && window >= 0 && all_below % 8 == 0,
+              NSA_ERR_BAD_ARG, "%s: dq_mode %d, window %d, all_below %d", who, dq_mode, window, all_below);
+  const int G = QH / KH;
+  NsaDqDsParams p{};
+  if (cmp_ds != nullptr) {
+    rc = check_nsa_sizes(who, kernel_size, stride, 0);
+    if (rc) return rc;
+    const DsLayout l = ds_layout_cmp(T, B, x_maxlen, G, KH, kernel_size, stride, tok0, tok1);
+    rc = check_ds(who, QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, cmp_ds, cmp_ds_bytes, l.bytes,
+                  bwd_ds_takes(0, 0, ck_sr, QH, KH, D, VD, sm_scale));
+    if (rc) return rc;
+    p.cmp = ds_operand(l, ck, ck_sr, ck_sh, cmp_ds);
+  }
+  if (swa_ds != nullptr) {
+    const DsLayout l = ds_layout_win(T, B, x_maxlen, G, KH, window, ring);
+    rc = check_ds(who, QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, swa_ds, swa_ds_bytes, l.bytes,
+                  bwd_ds_takes(0, 0, k_sr, QH, KH, D, VD, sm_scale));
+    if (rc) return rc;
+    p.win = ds_operand(l, k, k_sr, k_sh, swa_ds);
+    const DsLayout f = ds_layout_far(T, B, x_maxlen, G, KH, window, all_below, ring);
+    if (far_ds != nullptr && f.pitch > 0) {
+      rc = check_ds(who, QH, KH, D, VD, T, B, x_maxlen, tok0, tok1, far_ds, far_ds_bytes, f.bytes, true);
+      if (rc) return rc;
+      p.far = ds_operand(f, k, k_sr, k_sh, far_ds);
+    }
+  }
+  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh; p.dq_mode = dq_mode;
+  p.dq_partial = dq_partial; p.dqp_st = dqp_st; p.dqp_sh = dqp_sh;
+  p.x_cu = x_cu; p.y_cu = y_cu;
+  p.G = G; p.KH = KH;
+  p.kernel_size = kernel_size; p.stride = stride; p.window = window; p.all_below = all_below;
+  p.tok0 = tok0; p.tok1 = tok1;
+  p.sm_scale = sm_scale;
+  return nsa_bwd_dq_ds_launch(p, B, x_maxlen, D, (hipStream_t)stream);
 }
 
 }  // extern "C"

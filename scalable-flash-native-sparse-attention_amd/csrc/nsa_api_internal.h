@@ -107,6 +107,10 @@ struct NsaBwdTileParams {
   bf16_t* ds; int64_t ds_sh;
   const uint8_t* csr_slot;
   int ds_tok0, ds_ntok, ds_dump, top_n;  // ds_dump: entry for the dS of rows that stand for nothing
+  // compressed / window dkdv that also stores dS (see nsa_bwd_dq_ds.hip for the layout), of the tokens tok0 .. tok1 - 1 (0: all):
+  // per kv head ds_tiles tiles of 64 rows with ds_pitch units of 32 keys (ds_seq_tiles: see nsa_ds_tile); then 68 KB that
+  // nobody reads
+  int tok0, tok1, ds_tiles, ds_seq_tiles, ds_pitch;
   int G, KH;
   float scale_log2, sm_scale;
   int kernel_size, stride, window;
@@ -131,11 +135,14 @@ int nsa_bwd_dkdv_dma_launch(const NsaBwdTileParams& p, int mode, dim3 grid, int 
 int nsa_bwd_dkdv_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int max_k_len, int D, int VD,
                         int n_items_bound, hipStream_t stream);
 // deterministic dk / dv (dkv_mode 4): slots a launch writes, and the ordered sums over them (nsa_dkdv_reduce.hip)
+// (of the tokens tok0 .. tok1 - 1 of a batch of n_seq sequences; tok1 = 0: all)
 int64_t nsa_bwd_dkdv_cmp_slots(int B, int KH, int max_q_len, int max_k_len, int D, int q_chunk_tokens,
-                               int kernel_size, int stride);
+                               int kernel_size, int stride, int tok0, int tok1, int n_seq);
+int nsa_swa_dkdv_q_chunk(const NsaBwdTileParams& p, int KW);
 int64_t nsa_bwd_dkdv_slc_slots(int KH, int n_items_bound, int block_size);
 int nsa_bwd_dkdv_slot_keys(int mode, int block_size, int D);
-int nsa_dkdv_reduce_cmp_launch(const NsaBwdTileParams& p, int B, int max_q_len, int max_k_len, int D, int VD,
+// (add: to what dk / dv hold)
+int nsa_dkdv_reduce_cmp_launch(const NsaBwdTileParams& p, bool add, int B, int max_q_len, int max_k_len, int D, int VD,
                                hipStream_t stream);
 int nsa_dkdv_reduce_swa_launch(const NsaBwdTileParams& p, bool to_f32, int B, int x_maxlen, int D, int VD,
                                hipStream_t stream);
@@ -173,6 +180,26 @@ struct NsaSlcDqDsParams {
 int nsa_slc_dq_ds_launch(const NsaSlcDqDsParams& p, int D, hipStream_t stream);
 // elements of the dS of one (token, slot), all heads of one kv head; 0: this group size has no such layout
 int64_t nsa_slc_ds_entry_elems(int G, int block_size);
+
+// dQ = dS K of the compressed branch (cmp), the window (win) and the keys before it (far, of the queries below all_below) from
+// their stored dS (null: the branch is left out)
+struct NsaDsOperand {
+  const bf16_t* k; int64_t k_sr, k_sh;
+  const bf16_t* ds; int64_t ds_sh;
+  int tiles, seq_tiles, pitch;                // as NsaBwdTileParams' ds_*
+};
+struct NsaDqDsParams {
+  NsaDsOperand cmp, win, far;                 // (far: win's keys)
+  // 0: store bf16, 1: store fp32, 2: add into fp32, 3: bf16 store to dq at positions below all_below, else fp32 to dq_partial
+  void* dq; int64_t dq_st, dq_sh; int dq_mode;
+  float* dq_partial; int64_t dqp_st, dqp_sh;
+  const int32_t* x_cu; const int32_t* y_cu;
+  int G, KH;
+  int kernel_size, stride, window, all_below;
+  int tok0, tok1;                             // tokens of the launch (tok1 = 0: all)
+  float sm_scale;
+};
+int nsa_bwd_dq_ds_launch(const NsaDqDsParams& p, int B, int max_q_len, int D, hipStream_t stream);
 
 // fused paged decode (one query token per request)
 struct NsaDecodeParams {

@@ -588,13 +588,8 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
   const int kb_cmp = KB2_BUILT ? nsa_tuning_knob("dkdv_key_blocks", 1) : 1;  // 32-key blocks per wave (cmp / swa)
   if (mode == MODE_CMP) {
     if (B <= 0 || max_k_len <= 0) return NSA_OK;
-    const int KW = 4 * 32 * (kb_cmp == 2 ? 2 : 1);
-    const int nch = cdiv_i(max_q_len, p.q_chunk_tokens);
-    int total = 0;
-    for (int kt = 0; kt * KW < max_k_len; kt++) {
-      const int fc = (p.stride * kt * KW + p.kernel_size - 1) / p.q_chunk_tokens;
-      total += nch - (nch < fc ? nch : fc);
-    }
+    const int total = (int)nsa_bwd_dkdv_cmp_slots(1, 1, max_q_len, max_k_len, D, p.q_chunk_tokens, p.kernel_size, p.stride,
+                                                  p.tok0, p.tok1, B);
     if (total <= 0) return NSA_OK;
     dim3 grid(total, B, p.KH);
     if (dma) return nsa_bwd_dkdv_dma_launch(p, mode, grid, D, VD, stream);
@@ -614,7 +609,8 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
     // no query is further from a key than the longest sequence: chunks cut from a wider window would start behind the
     // last query, and their row numbers (position x heads) leave the range of an int
     p.window = min(p.window, max_q_len);
-    p.q_chunk_tokens = cdiv_i(KW + p.window - p.min_dist, p.grid_chunks);
+    p.q_chunk_tokens = nsa_swa_dkdv_q_chunk(p, KW);
+    if (p.tok1 > 0) max_k_len = min(max_k_len, p.tok1 - p.tok0 + 127);
     if constexpr (KB2_BUILT) {
       if (kb_cmp == 2) {
         dim3 grid(cdiv_i(max_k_len, 256) * p.grid_chunks, B, p.KH);
@@ -650,15 +646,29 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
 
 // workgroups (= slots of the partial buffers) of a compressed-branch launch: grid.x * B * KH, as launch() sizes it
 int64_t nsa_bwd_dkdv_cmp_slots(int B, int KH, int max_q_len, int max_k_len, int D, int q_chunk_tokens,
-                               int kernel_size, int stride) {
+                               int kernel_size, int stride, int tok0, int tok1, int n_seq) {
   const int KW = nsa_bwd_dkdv_slot_keys(0, 0, D);
-  const int nch = cdiv_i(max_q_len, q_chunk_tokens);
+  // the share of the longest sequence; of several sequences that a range meets, one may have any share of that length
+  int lo, hi;
+  nsa_local_range(tok0, tok1, 0, max_q_len, lo, hi);
+  if (tok1 > 0 && n_seq > 1) {
+    lo = max_q_len - (max_q_len < tok1 - tok0 + 127 ? max_q_len : tok1 - tok0 + 127);
+    hi = max_q_len;
+  }
+  const int nch = hi > lo ? cdiv_i(hi - lo, q_chunk_tokens) : 0;
   int64_t total = 0;
-  for (int kt = 0; kt * KW < max_k_len; kt++) {
-    const int fc = (stride * kt * KW + kernel_size - 1) / q_chunk_tokens;
-    total += nch - (nch < fc ? nch : fc);
+  for (int64_t kt = 0; kt * KW < max_k_len; kt++) {
+    const int64_t first = stride * kt * KW + kernel_size - 1 - lo;
+    const int64_t fc = first > 0 ? first / q_chunk_tokens : 0;
+    if (fc >= nch) break;
+    total += nch - fc;
   }
   return total * B * KH;
+}
+// queries per work item of the window's dk/dv: with stored dS whole tiles of 64 rows
+int nsa_swa_dkdv_q_chunk(const NsaBwdTileParams& p, int KW) {
+  const int n = KW + p.window - p.min_dist;
+  return p.ds == nullptr ? cdiv_i(n, p.grid_chunks) : (cdiv_i(n + 8, p.grid_chunks) + 7) & ~7;
 }
 int64_t nsa_bwd_dkdv_slc_slots(int KH, int n_items_bound, int block_size) {
   return (int64_t)KH * n_items_bound * (block_size <= 64 ? 1 : cdiv_i(block_size, 128));

@@ -62,9 +62,10 @@ constexpr int DMA_LIST = 1024;  // tokens of a work item that the kernel holds i
 
 constexpr int dma_waves(int d) { return d <= 128 ? 2 : 1; }
 
-// DSH > 0 (MODE_SLC): the dS of every (token, block) is also stored, in blobs of DSH heads, for the dQ of the same tokens
-// (nsa_slc_bwd_dq_ds.hip).  No path through the tile loop leaves the stores out (rows without an entry go to a blob that nobody
-// reads): where one did, the compiler waited for all of them and not just for the next tile's loads.
+// DSH > 0: the dS is also stored, for the dQ of the same rows.  MODE_SLC: that of every (token, block), in blobs of DSH heads
+// (nsa_slc_bwd_dq_ds.hip); else that of every 64 rows and 32 keys, in four blobs of 16 rows (nsa_bwd_dq_ds.hip).  No path through
+// the tile loop leaves the stores out (rows without an entry, and waves that see nothing, store to a place that nobody reads):
+// where one did, the compiler waited for all of them and not just for the next tile's loads.
 template <int D, int VD, int MODE, bool NARROW, int DSH>
 __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdTileParams p) {
   constexpr bool DS = DSH > 0;
@@ -123,33 +124,41 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
   }
   const int x0 = p.x_cu[b];
   int xl = p.x_cu[b + 1] - x0;
+  const int tshift = 6 - gshift;  // log2 of the tokens of a 64-row tile
+  // stored dS of the range-keyed branches: tiles of 64 rows from the first of a sequence on
+  constexpr bool TILE_DS = DS && MODE != MODE_SLC;
+  int lo = 0, hi = xl;  // the launch's share of the sequence
+  if (TILE_DS) nsa_local_range(p.tok0, p.tok1, x0, xl, lo, hi);
   if (MODE == MODE_SWA && p.t_end > 0) xl = min(xl, p.t_end);
   int nkeys, kbase;
   if (MODE == MODE_CMP) {
     kbase = p.k_cu[b];
     nkeys = p.k_cu[b + 1] - kbase;
     // only the (key tile, query chunk) pairs that have visible rows, key-tile major, as nsa_bwd_dkdv.hip numbers them
-    const int nch = cdiv_i(xl, p.q_chunk_tokens);
+    const int nch = cdiv_i(max(hi - lo, 0), p.q_chunk_tokens);
     int rem = blockIdx.x, ktile = 0, ch = -1;
     for (; ktile * KW < nkeys; ktile++) {
-      const int fc = min(nch, (p.stride * ktile * KW + p.kernel_size - 1) / p.q_chunk_tokens);
+      const int fc = min(nch, max(p.stride * ktile * KW + p.kernel_size - 1 - lo, 0) / p.q_chunk_tokens);
       const int cnt = nch - fc;
       if (rem < cnt) { ch = fc + rem; break; }
       rem -= cnt;
     }
     if (ch < 0) return;
     key0 = ktile * KW;
-    n_begin = max(ch * p.q_chunk_tokens, p.stride * key0 + p.kernel_size - 1);
-    n_end = min((ch + 1) * p.q_chunk_tokens, xl);
+    n_begin = max(lo + ch * p.q_chunk_tokens, p.stride * key0 + p.kernel_size - 1);
+    n_end = min(lo + (ch + 1) * p.q_chunk_tokens, hi);
+    if (n_begin >= n_end) return;
+    if (TILE_DS) n_begin &= -(1 << tshift);  // (chunks and ranges begin with a tile)
   } else {
     kbase = x0;
     nkeys = xl;
     if (MODE == MODE_SLC) nkeys = min(xl, (key0 / p.block_size + 1) * p.block_size);
     if (MODE == MODE_SWA) {
       const int ktile = blockIdx.x / p.grid_chunks;
-      key0 = ktile * KW;
-      if (key0 >= nkeys) return;
-      n_begin = key0 + p.min_dist + (blockIdx.x - ktile * p.grid_chunks) * p.q_chunk_tokens;
+      key0 = lo + ktile * KW;
+      if (key0 >= min(nkeys, hi)) return;
+      n_begin = key0 + (TILE_DS ? p.min_dist & -(1 << tshift) : p.min_dist) +
+                (blockIdx.x - ktile * p.grid_chunks) * p.q_chunk_tokens;
       n_end = min(min(xl, key0 + KW + p.window), n_begin + p.q_chunk_tokens);
     } else if (key0 >= nkeys) {
       return;
@@ -178,15 +187,6 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
 #pragma unroll
     for (int kc = 0; kc < VD / 16; kc++) vf[kc] = ld_global_b128(vp + kc * 16);
   }
-  f32x16 dkacc[D / 32], dvacc[VD / 32];
-#pragma unroll
-  for (int dt = 0; dt < D / 32; dt++)
-#pragma unroll
-    for (int i = 0; i < 16; i++) dkacc[dt][i] = 0.f;
-#pragma unroll
-  for (int dt = 0; dt < VD / 32; dt++)
-#pragma unroll
-    for (int i = 0; i < 16; i++) dvacc[dt][i] = 0.f;
   const float sc = p.scale_log2;
 
   // ---- staging: wave w moves the row groups w and w + 4 of every tile
@@ -239,13 +239,30 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
   const int ta0 = rg * MT * 4 * GS * 2 + tr_row * 128 + (((g16 & 1) * 2 + ((i16 & 3) >> 1)) ^ tr_row) * 16 + (i16 & 1) * 8;
 
   float st_reg;
+  // stored dS: tile number of the work item's first tile, place for what nobody reads
+  int64_t ds_head = 0, ds_dump = 0;
+  int ds_tile = 0;
+  if (TILE_DS) {
+    ds_head = (int64_t)kh * p.ds_sh;
+    ds_dump = (int64_t)p.KH * p.ds_sh + ((blockIdx.x & 15) * 4 + wave) * 512;  // (and three blobs more)
+    ds_tile = nsa_ds_tile(p.ds_tiles, p.ds_seq_tiles, x0 >> tshift, b, n_begin >> tshift);
+  }
 
+  f32x16 dkacc[D / 32], dvacc[VD / 32];
+#pragma unroll
+  for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) dkacc[dt][i] = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < VD / 32; dt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) dvacc[dt][i] = 0.f;
   // one tile: `cur` holds it (its loads are in flight), `nxt` receives the next one
   auto step = [&](bf16_t* cur, bf16_t* nxt, int n0) {
     const int tv = tokens_of(n0), tvn = tokens_of(n0 + n_step);
     // lane i: place of the dS of row group i / 8 (rows without a token of the list, waves without keys: an entry nobody reads)
     int ds_ent = 0;
-    if (DS) {
+    if (MODE == MODE_SLC && DS) {
       const int grp = lane_id() >> 3, n = n0 + ((grp * 8) >> gshift);
       const int tok = x0 + tv - p.ds_tok0;
       const int e = (tok * p.top_n + slot_s[min(n, n_last)]) * (G > 16 ? G >> 4 : 1) + (((grp * 8) & (G - 1)) >> 4);
@@ -279,7 +296,15 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
       any_vis = kw0 <= t_max;
       full_vis = n_in == n_step && kw0 + 31 <= t_min && kw0 + 31 < nkeys;
     }
-    if (!DS && !(any_vis && wave_has_keys)) return;
+    const bool seen = any_vis && wave_has_keys;
+    if (!DS && !seen) return;
+    bf16_t* ds_out = nullptr;
+    if (TILE_DS) {
+      int tile = ds_tile + ((n0 - n_begin) >> tshift);
+      if (tile >= p.ds_tiles) tile -= p.ds_tiles;
+      const int unit = (kw0 >> 5) - (MODE == MODE_SWA ? max(0, n0 - p.window) >> 5 : 0);
+      ds_out = p.ds + (seen ? ds_head + ((int64_t)tile * p.ds_pitch + unit) * 2048 : ds_dump);
+    }
 
     // The A operands of a step's matrix instructions, in the order in which they are used: Q rows (S), dO rows (dP),
     // dO transposed (dV), Q transposed (dK).  They are read PF operands ahead, and the softmax arithmetic is placed between
@@ -376,7 +401,9 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
           constexpr int c = (f - F_DK) / nd, dt = (f - F_DK) % nd;
           dkacc[order_dt(dt, nd)] = mfma32(a, df[c], dkacc[order_dt(dt, nd)]);
           if (dt == 0 && c == 1 && mt + 1 < MT) init(s, 0, mt + 1);
-          if (DS && dt == 0) {
+          if (TILE_DS && dt == 0) {
+            __builtin_nontemporal_store(__builtin_bit_cast(u32x4, df[c]), reinterpret_cast<u32x4*>(ds_out + ((mt * 2 + c) * 512 + lane_id() * 8)));
+          } else if (DS && dt == 0) {
             const int upb = p.block_size >> 5, unit = min((int)blockIdx.y * NK + kg, upb - 1);  // 32-key units of the block
             auto entry = [&](int grp) { return (int64_t)__builtin_amdgcn_readlane(ds_ent, grp * 8) * upb + unit; };
             const int grp = (rg * MT + mt) * 4 + c * 2;
@@ -399,14 +426,48 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
     stage(tv, n_begin, tile_a);
     st_reg = stat_of(tv, n_begin);
   }
+  int n0 = n_begin;
+  // TILE_DS: tiles of which a wave sees nothing, two at a time: it only helps with the rows.  (Not a branch inside a step: the
+  // compiler then spills half of the accumulators.)
+  int n_stop = n_end;
+  auto skim = [&](bf16_t* cur, bf16_t* nxt) {
+    const int tvn = tokens_of(n0 + n_step);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(WAIT_LOADS);
+    asm volatile("" ::: "memory");
+    if (wave < 2) reinterpret_cast<float*>(cur + TILE)[wave * RT + lane_id()] = st_reg * s_mul;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(WAIT_LDS);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    stage(tvn, n0 + n_step, nxt);
+    st_reg = stat_of(tvn, n0 + n_step);
+    n0 += n_step;
+  };
+  if constexpr (TILE_DS) {
+    int n_first = MODE == MODE_CMP ? p.stride * kw0 + p.kernel_size - 1 : kw0 + p.min_dist;
+    if (!wave_has_keys) n_first = n_end;
+    if (MODE == MODE_SWA) n_stop = min(n_end, kw0 + 32 + p.window);
+    while (n0 + 2 * n_step <= n_first && n0 + 2 * n_step < n_end) {
+      skim(tile_a, tile_b);
+      skim(tile_b, tile_a);
+    }
+  }
   if (DS) __builtin_amdgcn_s_waitcnt(WAIT_LOADS);  // no stores behind the first tile's loads yet
-  for (int n0 = n_begin;;) {
+  for (;;) {
     step(tile_a, tile_b, n0);
     n0 += n_step;
     if (n0 >= n_end) break;
     step(tile_b, tile_a, n0);
     n0 += n_step;
-    if (n0 >= n_end) break;
+    if (n0 >= n_stop) break;
+  }
+  if constexpr (TILE_DS) {
+    while (n0 < n_end) {
+      skim(tile_a, tile_b);
+      if (n0 >= n_end) break;
+      skim(tile_b, tile_a);
+    }
   }
 
   // ---- epilogue: the tile buffers are free once the loads behind the last tile have landed
@@ -502,8 +563,14 @@ __global__ __launch_bounds__(256, dma_waves(D)) void bwd_dkdv_dma_kernel(NsaBwdT
 
 template <int D, int VD>
 int launch(const NsaBwdTileParams& p, int mode, dim3 grid, hipStream_t stream) {
-  if (mode == MODE_CMP) bwd_dkdv_dma_kernel<D, VD, MODE_CMP, false, 0><<<grid, 256, 0, stream>>>(p);
-  else if (mode == MODE_SWA) bwd_dkdv_dma_kernel<D, VD, MODE_SWA, false, 0><<<grid, 256, 0, stream>>>(p);
+  constexpr int TILE_DSH = D >= 128 ? 16 : 0;  // (64 channels: dq is faster without)
+  if (mode == MODE_CMP) {
+    if (TILE_DSH == 0 || p.ds == nullptr) bwd_dkdv_dma_kernel<D, VD, MODE_CMP, false, 0><<<grid, 256, 0, stream>>>(p);
+    else bwd_dkdv_dma_kernel<D, VD, MODE_CMP, false, TILE_DSH><<<grid, 256, 0, stream>>>(p);
+  } else if (mode == MODE_SWA) {
+    if (TILE_DSH == 0 || p.ds == nullptr) bwd_dkdv_dma_kernel<D, VD, MODE_SWA, false, 0><<<grid, 256, 0, stream>>>(p);
+    else bwd_dkdv_dma_kernel<D, VD, MODE_SWA, false, TILE_DSH><<<grid, 256, 0, stream>>>(p);
+  }
   else if (p.block_size <= 64) {
     if (p.ds == nullptr) bwd_dkdv_dma_kernel<D, VD, MODE_SLC, true, 0><<<grid, 256, 0, stream>>>(p);
     else if (p.G == 8) bwd_dkdv_dma_kernel<D, VD, MODE_SLC, true, 8><<<grid, 256, 0, stream>>>(p);

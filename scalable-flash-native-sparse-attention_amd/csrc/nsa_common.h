@@ -188,6 +188,22 @@ NSA_DEVICE int wave_argmax_lowest(float score, int index, bool has_candidate) {
 
 __host__ __device__ inline int cdiv_i(int a, int b) { return (a + b - 1) / b; }
 
+// The share of a sequence (tokens x0 .. x0 + xl - 1) that belongs to the tokens tok0 .. tok1 - 1 of a packed batch, in whole
+// groups of 128 positions: a group belongs to the range that holds its first token.  tok1 = 0: all of it.
+__host__ __device__ inline void nsa_local_range(int tok0, int tok1, int x0, int xl, int& lo, int& hi) {
+  lo = 0;
+  hi = xl;
+  if (tok1 <= 0) return;
+  const int a = (tok0 - x0 + 127) & ~127, e = (tok1 - x0 + 127) & ~127;
+  lo = a > 0 ? a : 0;
+  hi = e < xl ? e : xl;
+}
+// Place of a sequence's tile `i` among `tiles` of stored dS: numbered through the batch, in turn, or, with seq_tiles, so many
+// for every sequence.  x0_tiles: the sequence's first token / the tokens of a tile (rounded down).
+NSA_DEVICE int nsa_ds_tile(int tiles, int seq_tiles, int x0_tiles, int b, int i) {
+  return seq_tiles > 0 ? b * seq_tiles + i : __builtin_amdgcn_readfirstlane((x0_tiles + b + i) % tiles);
+}
+
 // error codes returned by the C entry points
 enum {
   NSA_OK = 0,

@@ -15,7 +15,7 @@ namespace {
 // 1 kv heads, 64 chunks: 650 us with a workgroup per tile, 5 us so).
 template <int KW>
 __global__ __launch_bounds__(256) void cmp_dkdv_reduce_kernel(NsaBwdTileParams p, int D, int VD, int grid_x_items,
-                                                              int pieces) {
+                                                              int pieces, bool add) {
   const int ktile = blockIdx.x / pieces, b = blockIdx.y, kh = blockIdx.z;
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
@@ -28,12 +28,16 @@ __global__ __launch_bounds__(256) void cmp_dkdv_reduce_kernel(NsaBwdTileParams p
   const int kl = e / per_key, c4 = e - kl * per_key;
   if (kl >= min(KW, nkeys - key0)) return;
   // the enumeration of bwd_dkdv_kernel MODE_CMP
-  const int nch = cdiv_i(xl, p.q_chunk_tokens);
+  int lo, hi;
+  nsa_local_range(p.tok0, p.tok1, x0, xl, lo, hi);
+  const int nch = cdiv_i(max(hi - lo, 0), p.q_chunk_tokens);
   int start = 0;
   for (int kt = 0; kt < ktile; kt++)
-    start += nch - min(nch, (p.stride * kt * KW + p.kernel_size - 1) / p.q_chunk_tokens);
-  // chunk fc holds the tile's first visible row (there is one: the tile has keys)
-  const int fc = (p.stride * key0 + p.kernel_size - 1) / p.q_chunk_tokens;
+    start += nch - min(nch, max(p.stride * kt * KW + p.kernel_size - 1 - lo, 0) / p.q_chunk_tokens);
+  // chunk fc holds the tile's first visible row, if the launch's share of the sequence holds one
+  const int seen = p.stride * key0 + p.kernel_size - 1;
+  const int fc = seen < hi ? max(seen - lo, 0) / p.q_chunk_tokens : nch;
+  if (add && fc >= nch) return;
   const bool is_v = c4 >= n4k;
   const int d = (is_v ? c4 - n4k : c4) * 4;
   const int W = is_v ? VD : D;
@@ -53,6 +57,7 @@ __global__ __launch_bounds__(256) void cmp_dkdv_reduce_kernel(NsaBwdTileParams p
   for (; ch < n; ch++) acc += *reinterpret_cast<const f32x4*>(src + ch * step);
   float* dst = is_v ? (float*)p.dv + ((int64_t)kbase + key0 + kl) * p.dv_sr + (int64_t)kh * p.dv_sh + d
                     : (float*)p.dk + ((int64_t)kbase + key0 + kl) * p.dk_sr + (int64_t)kh * p.dk_sh + d;
+  if (add) acc += *reinterpret_cast<const f32x4*>(dst);
   *reinterpret_cast<f32x4*>(dst) = acc;
 }
 
@@ -63,12 +68,14 @@ __global__ __launch_bounds__(256) void swa_dkdv_reduce_kernel(NsaBwdTileParams p
   const int ktile = blockIdx.x / pieces, b = blockIdx.y, kh = blockIdx.z;
   const int x0 = p.x_cu[b];
   const int xl = p.x_cu[b + 1] - x0;
-  const int key0 = ktile * KW;
+  int lo, hi;
+  nsa_local_range(p.tok0, p.tok1, x0, xl, lo, hi);
+  const int key0 = lo + ktile * KW;
   const int n4k = D / 4, n4v = VD / 4;
   const int per_key = n4k + n4v;
   const int e = (blockIdx.x - ktile * pieces) * 256 + threadIdx.x;
   const int kl = e / per_key, c4 = e - kl * per_key;
-  if (kl >= min(KW, xl - key0)) return;
+  if (kl >= min(KW, hi - key0)) return;
   const int rows = min(xl - key0, KW + p.window);
   const int n = min(p.grid_chunks, cdiv_i(rows, p.q_chunk_tokens));
   const bool is_v = c4 >= n4k;
@@ -133,17 +140,17 @@ __global__ __launch_bounds__(256) void slc_dkdv_reduce_kernel(NsaBwdTileParams p
 
 }  // namespace
 
-int nsa_dkdv_reduce_cmp_launch(const NsaBwdTileParams& p, int B, int max_q_len, int max_k_len, int D, int VD,
+int nsa_dkdv_reduce_cmp_launch(const NsaBwdTileParams& p, bool add, int B, int max_q_len, int max_k_len, int D, int VD,
                                hipStream_t stream) {
   if (B <= 0 || max_k_len <= 0) return NSA_OK;
   const int KW = nsa_bwd_dkdv_slot_keys(0, 0, D);
   const int grid_x_items = (int)nsa_bwd_dkdv_cmp_slots(1, 1, max_q_len, max_k_len, D, p.q_chunk_tokens, p.kernel_size,
-                                                       p.stride);
-  if (grid_x_items <= 0) return NSA_OK;
+                                                       p.stride, p.tok0, p.tok1, B);
+  if (grid_x_items <= 0 && add) return NSA_OK;
   const int pieces = cdiv_i(KW * (D + VD) / 4, 256);
   dim3 grid(cdiv_i(max_k_len, KW) * pieces, B, p.KH);
-  if (KW == 128) cmp_dkdv_reduce_kernel<128><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces);
-  else cmp_dkdv_reduce_kernel<256><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces);
+  if (KW == 128) cmp_dkdv_reduce_kernel<128><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces, add);
+  else cmp_dkdv_reduce_kernel<256><<<grid, 256, 0, stream>>>(p, D, VD, grid_x_items, pieces, add);
   return nsa_check_launch("cmp_dkdv_reduce_kernel");
 }
 
@@ -154,9 +161,10 @@ int nsa_dkdv_reduce_swa_launch(const NsaBwdTileParams& p0, bool to_f32, int B, i
   const int KW = nsa_bwd_dkdv_slot_keys(1, 0, D);
   // as the dk/dv launch cuts them
   p.window = min(p.window, x_maxlen);
-  p.q_chunk_tokens = cdiv_i(KW + p.window, p.grid_chunks);
+  p.q_chunk_tokens = nsa_swa_dkdv_q_chunk(p, KW);
   const int pieces = cdiv_i(KW * (D + VD) / 4, 256);
-  dim3 grid(cdiv_i(x_maxlen, KW) * pieces, B, p.KH);
+  const int len = p.tok1 > 0 ? min(x_maxlen, p.tok1 - p.tok0 + 127) : x_maxlen;
+  dim3 grid(cdiv_i(len, KW) * pieces, B, p.KH);
   if (to_f32) swa_dkdv_reduce_kernel<true><<<grid, 256, 0, stream>>>(p, KW, D, VD, pieces);
   else swa_dkdv_reduce_kernel<false><<<grid, 256, 0, stream>>>(p, KW, D, VD, pieces);
   return nsa_check_launch("swa_dkdv_reduce_kernel");

@@ -10,6 +10,7 @@ from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
 from ..ops._common import thd_rows
 from ..ops.compress_kv import construct_block_fwd, construct_block_bwd, mean_pooling_fwd, mean_pooling_bwd
+from ..ops import bwd_ds
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
 from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window,
                                slc_bwd_ds_tokens)
@@ -100,6 +101,60 @@ def slc_swa_fwd(q, k, v, topk, sm_scale, helper, cmp_o=None, w=None, store=True)
     return (slc_o, slc_lse), (swa_o, swa_lse), out
 
 
+def bwd_from_ds(q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa, delta, ds_tokens, sm_scale, helper):
+    """The backward of the three branches where all of them leave their dS behind -> dq, dk, dv, dcmp_k, dcmp_v.
+    ds_tokens: slc_bwd_ds_tokens; 0: every query selects all blocks it sees."""
+    all_below = helper.all_below()
+    dq = torch.empty_like(q)
+    dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32) if ds_tokens else None
+    # the window branch writes every element of dk / dv, the selected branch then adds to them
+    dk = torch.empty(k.shape, device=q.device, dtype=torch.float32)
+    dv = torch.empty(v.shape, device=q.device, dtype=torch.float32)
+    ds = bwd_ds.DenseDs(q, k, helper, all_below=all_below)
+
+    def dkdv_cmp(r, *sums):
+        return ds.dkdv_cmp(r, q, cmp_k, cmp_v, cmp_lse, dcmp_o, delta[0], sm_scale, *sums)
+
+    def dkdv_raw(r):
+        ds.dkdv_swa(r, q, k, v, lse_swa, do, delta[2], sm_scale, dk, dv)
+        ds.dkdv_far(r, q, k, v, lse_slc, do, delta[1], sm_scale, dk, dv)
+
+    def dense_dq(r):
+        # (the selected dq comes last and adds this one; the queries that the gather leaves out are done)
+        ds.dq(r, cmp_k, k, v.size(2), sm_scale, dq, 3 if ds_tokens else 0, dq32)
+
+    def selected(before_dq=None):
+        if ds_tokens:
+            slc_attn_bwd(q, k, v, topk, None, lse_slc, do, dq=dq32, dk=dk, dv=dv, delta=delta[1], t_begin=all_below,
+                         finalize_dq=dq, before_dq=before_dq, ds_tokens=ds_tokens, sm_scale=sm_scale, helper=helper)
+        elif before_dq is not None:
+            before_dq()
+
+    if OVERLAP_STREAMS and len(ds.ranges) == 1:
+        # the compressed dk / dv next to the window's, the dense dq next to the selected dk / dv
+        main, side, r = torch.cuda.current_stream(), _side_stream(q.device), ds.ranges[0]
+        side.wait_stream(main)
+        with torch.cuda.stream(side):
+            dcmp_k, dcmp_v = dkdv_cmp(r)
+        dkdv_raw(r)
+        window_done = main.record_event()
+        with torch.cuda.stream(side):
+            side.wait_event(window_done)
+            dense_dq(r)
+        dcmp_k.record_stream(main)
+        dcmp_v.record_stream(main)
+        selected(lambda: main.wait_stream(side))
+    else:  # ranges follow each other on one scratch, and each of them fills the GPU
+        sums = ()
+        for r in ds.ranges:
+            sums = dkdv_cmp(r, *sums)
+            dkdv_raw(r)
+            dense_dq(r)
+        dcmp_k, dcmp_v = sums
+        selected()
+    return dq, dk, dv, dcmp_k, dcmp_v
+
+
 class NSAFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, combine_weight, cmp_k_weight, cmp_v_weight, sm_scale=None, for_backward=True):
@@ -154,15 +209,23 @@ class NSAFunction(torch.autograd.Function):
         all_below = helper.all_below()
         dcmp_o, dw, delta, (lse_slc, lse_swa) = combine_bwd_gates(cmp_o, slc_o, swa_o, combine_weight, do, slc_lse, swa_lse,
                                                                   all_below, helper)
-        dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         kw = dict(sm_scale=sm_scale, helper=helper)
+
+        ds_tokens = slc_bwd_ds_tokens(q, k, v, do, topk, **kw) if helper.x_maxlen > all_below else 0
+        stored_ds = ds_tokens > 0
+        if (stored_ds or helper.x_maxlen <= all_below) and bwd_ds.takes(q, k, v, do, sm_scale, helper) and \
+                bwd_ds.takes(q, cmp_k, cmp_v, dcmp_o, sm_scale, helper):
+            dq, dk, dv, dcmp_k, dcmp_v = bwd_from_ds(q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa, delta,
+                                                     ds_tokens, sm_scale, helper)
+            _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+            _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+            return dq, dk, dv, dw, dwk, dwv, None, None
 
         # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
         # branches' and writes q's dtype (the compressed branch does for the queries that the gather leaves out).  Else it
         # stores first, the window branch (matrix bound, with bandwidth to spare for the read-modify-write) adds, or stores
         # where the selected branch left rows out, and the compressed branch adds and writes q's dtype.
-        ds_tokens = slc_bwd_ds_tokens(q, k, v, do, topk, **kw) if helper.x_maxlen > all_below else 0
-        stored_ds = ds_tokens > 0
+        dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         dq_last = torch.empty_like(q) if stored_ds else None
 
         def dq_chain():
@@ -173,11 +236,11 @@ class NSAFunction(torch.autograd.Function):
             return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
                                 parts="dq", finalize_below=(dq_last, all_below) if stored_ds else None, **kw)[0]
 
-        def dkdv_raw(dq_after=None):
+        def dkdv_raw(before_dq=None):
             # the window branch writes every element of dk / dv, the selected branch then adds to them
             _, dk, dv = swa_bwd(q, k, v, swa_o, lse_swa, do, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
             slc_attn_bwd_dkdv_before_window(q, k, v, lse_slc, do, delta[1], dk, dv, all_below, **kw)
-            last = dict(dq=dq32, finalize_dq=dq_last, dq_after=dq_after, ds_tokens=ds_tokens) if stored_ds else dict(parts="dkdv")
+            last = dict(dq=dq32, finalize_dq=dq_last, before_dq=before_dq, ds_tokens=ds_tokens) if stored_ds else dict(parts="dkdv")
             slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, dk=dk, dv=dv, delta=delta[1], t_begin=all_below, **last, **kw)
             return dk, dv
 
@@ -196,7 +259,7 @@ class NSAFunction(torch.autograd.Function):
                 dcmp_k, dcmp_v = dkdv_cmp()
                 dcmp_k.record_stream(main)
                 dcmp_v.record_stream(main)
-            dk, dv = dkdv_raw(dense_dq)
+            dk, dv = dkdv_raw(lambda: main.wait_event(dense_dq))
             main.wait_stream(side)
         elif OVERLAP_STREAMS:
             side = _side_stream(q.device)

@@ -3,6 +3,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
+from . import bwd_ds
 from ._common import check_thd, default_scale, delta_of, dq_target, zeros_pair
 
 
@@ -38,7 +39,8 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
     only read and the returned dq is a fresh tensor in q's dtype holding buffer + this branch.  finalize_below (with
     finalize_dq): a tensor of q's dtype and n; that sum is for the queries at positions below n stored there, for the others
     kept in the buffer.
-    parts = "dq" / "dkdv" launches only that kernel (the other results are None).
+    parts = "dq" / "dkdv" launches only that kernel (the other results are None); "both" forms dq from the dS that the dk / dv
+    kernel leaves behind where the shapes have that path (bwd_ds).
     dk, dv: fp32 [y_len,KH,*].  Every work item (query chunk of a key tile) stores its partial result into its own slot
     of a scratch buffer and a second launch sums the slots in a fixed order -- bit-identical results across runs.
     Where the slots would take more than DKDV_SLOTS_LIMIT bytes and neither dkdv_repeat nor
@@ -51,6 +53,13 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
     sm_scale = default_scale(q, sm_scale)
     if delta is None:
         delta = delta_of(o, do)
+    if parts == "both" and not (finalize_dq or dkdv_repeat or q_chunk_tokens) and bwd_ds.takes(q, k, v, do, sm_scale, helper):
+        ds, sums = bwd_ds.DenseDs(q, k, helper, with_swa=False), ()
+        dq_buf, mode = dq_target(q, dq)
+        for r in ds.ranges:
+            sums = ds.dkdv_cmp(r, q, k, v, lse, do, delta, sm_scale, *sums)
+            ds.dq(r, k, None, VD, sm_scale, dq_buf, mode)
+        return (dq_buf, *sums)
     common = (q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
               v.stride(0), v.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse.data_ptr(), lse.stride(1),
               lse.stride(0), delta.data_ptr(), delta.stride(0), delta.stride(1))

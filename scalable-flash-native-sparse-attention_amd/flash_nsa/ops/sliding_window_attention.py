@@ -4,6 +4,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
+from . import bwd_ds
 from ._common import check_bf16, check_thd, default_scale, delta_of, dq_target
 
 
@@ -75,13 +76,24 @@ def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq
     buffer (added into); dk/dv are fresh (bf16, or fp32 when dkv_fp32): one writer per element, or, for batches that do
     not fill the GPU, partial results added in a fixed order (up to 64 MB of scratch) -- bit-identical across runs.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None), so that a caller can put the
-    two on different streams."""
+    two on different streams; "both" forms dq from the dS that the dk / dv kernel leaves behind where the shapes have that
+    path (bwd_ds)."""
     check_thd(do, "do")
     T, QH, D = q.shape
     _, KH, VD = v.shape
     sm_scale = default_scale(q, sm_scale)
     if delta is None:
         delta = delta_of(o, do)
+    if parts == "both" and bwd_ds.takes(q, k, v, do, sm_scale, helper):
+        ds = bwd_ds.DenseDs(q, k, helper, with_cmp=False)
+        dq_buf, mode = dq_target(q, dq)
+        kv_dtype = torch.float32 if dkv_fp32 else k.dtype
+        dk = torch.empty(T, KH, D, device=q.device, dtype=kv_dtype)
+        dv = torch.empty(T, KH, VD, device=q.device, dtype=kv_dtype)
+        for r in ds.ranges:
+            ds.dkdv_swa(r, q, k, v, lse, do, delta, sm_scale, dk, dv)
+            ds.dq(r, None, k, VD, sm_scale, dq_buf, mode)
+        return dq_buf, dk, dv
     common = (q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
               v.stride(0), v.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse.data_ptr(), lse.stride(0),
               lse.stride(1), delta.data_ptr(), delta.stride(0), delta.stride(1))

@@ -1,0 +1,98 @@
+"""dq of the compressed and the window branch from the dS that their dk / dv kernels store, against the kernels that compute S
+and dP again (what the deterministic mode runs), over the shapes, sizes and ranges of tokens that the path takes."""
+import pytest
+import torch
+
+from gpu_util import assert_close, make_cu, make_qkvw, randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+def _grads(core, ts, cu, do, device):
+    ts = [t.to(device).requires_grad_() for t in ts]
+    out = core(*ts, cu)
+    out.backward(do)
+    return [out.detach()] + [t.grad for t in ts]
+
+
+# ends of tiles of 64 rows (8 .. 1 tokens), of units of 32 keys, of groups of 128 positions, and sequences without a
+# compressed row; ranged: a scratch limit of 1 MB, so that the ranges have the fewest tokens that they may have
+CASES = [
+    # QH, KH, D, VD, lens, ranged, settings
+    (8, 1, 128, 128, [1, 31, 32, 33, 700], False, {}),
+    (16, 1, 128, 128, [1024, 1025, 47, 1279], False, dict(top_n=4)),
+    (32, 1, 128, 128, [0, 515, 0, 640], False, dict(window_size=100, top_n=3)),
+    (64, 1, 128, 128, [513, 1, 129], False, dict(window_size=0, top_n=3)),
+    (64, 4, 128, 128, [4700], True, {}),
+    (64, 1, 128, 128, [2047, 300, 2500, 5], True, dict(top_n=6)),
+    (64, 4, 192, 128, [130, 4300], True, dict(window_size=300)),
+    (32, 2, 192, 128, [900, 64, 333], False, dict(block_size=96, kernel_size=64, stride=32, top_n=5)),
+    (16, 2, 128, 128, [1500, 200], False, dict(window_size=2000)),
+    (16, 1, 192, 128, [777], False, dict(kernel_size=16, stride=8, block_size=32, top_n=40)),
+]
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens,ranged,settings", CASES)
+def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ranged, settings):
+    from flash_nsa import NSAConfig, NSACore, _lib
+    from flash_nsa.ops import bwd_ds
+    from flash_nsa.utils import NSAHelper as H
+    T = sum(lens)
+    cu = make_cu(lens).to(device)
+    ts = make_qkvw(T, QH, KH, D, VD, seed=300)
+    do = randn_bf16(T, QH, VD, seed=301).to(device)
+    core = NSACore(NSAConfig(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH, **settings))
+    core = core.to(device=device, dtype=torch.bfloat16)
+    made, init = [], bwd_ds.DenseDs.__init__
+    bwd_ds.DenseDs.__init__ = lambda self, *a, **k: (init(self, *a, **k), made.append(self))[0]
+    if ranged:
+        _lib.call("nsa_set_tuning", b"dense_ds_mb", 1)
+    try:
+        got = _grads(core, ts, cu, do, device)
+        H.set_deterministic(True)
+        want = _grads(core, ts, cu, do, device)
+    finally:
+        H.set_deterministic(False)
+        _lib.call("nsa_reset_tuning")
+        bwd_ds.DenseDs.__init__ = init
+    assert len(made) == 1 and (len(made[0].ranges) > 1) == ranged
+    assert torch.equal(got[0], want[0])
+    # the same products of bf16 operands whose last bit may differ (P from differently rounded exponents): the bar that both
+    # are held to against the oracle
+    for a, b, name in zip(got[1:], want[1:], ("dq", "dk", "dv", "dw")):
+        assert_close(a, b, name, row_scale=name in ("dk", "dv"))
+        d = (a.double() - b.double()).norm() / b.double().norm()
+        assert d < 4e-3, (name, float(d))  # 2^-8
+
+
+@pytest.mark.parametrize("QH,KH,lens", [(16, 1, [1100, 40]), (64, 4, [2600, 2500])])
+def test_branch_backward_ranges_give_the_same_bits(device, QH, KH, lens):
+    """The two branches by themselves: whole and in ranges of tokens, dq bit for bit; into bf16, stored fp32 and added to fp32."""
+    from flash_nsa import _lib
+    from flash_nsa.ops._common import delta_of
+    from flash_nsa.ops.compress_attn import cmp_attn_bwd, cmp_attn_fwd
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.sliding_window_attention import swa_bwd, swa_fwd
+    from flash_nsa.utils import NSAHelper as H
+    T = sum(lens)
+    H.set_hyperparameters()
+    H.init_cu_seqlens(make_cu(lens).to(device))
+    q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, 128, 128, seed=310)]
+    do = randn_bf16(T, QH, 128, seed=311).to(device)
+    ck, cv = mean_pooling_fwd(k), mean_pooling_fwd(v)
+    for fwd, bwd, args in ((cmp_attn_fwd, cmp_attn_bwd, (q, ck, cv)), (swa_fwd, swa_bwd, (q, k, v))):
+        o, lse = fwd(*args)
+        delta = delta_of(o, do)
+        runs = []
+        for mb in (4096, 1):
+            _lib.call("nsa_set_tuning", b"dense_ds_mb", mb)
+            try:
+                runs.append(bwd(*args, o, lse, do, delta=delta))
+                base = torch.randn(T, QH, 128, device=device)
+                added = bwd(*args, o, lse, do, dq=base.clone(), delta=delta)[0]
+            finally:
+                _lib.call("nsa_reset_tuning")
+            assert_close((added - base).to(torch.bfloat16), runs[-1][0], "added dq", atol=1e-3)
+        assert torch.equal(runs[0][0], runs[1][0])
+        for a, b, name in zip(runs[0][1:], runs[1][1:], ("dk", "dv")):
+            assert_close(a, b, name, atol=2e-3, rtol=8e-3, row_scale=True)

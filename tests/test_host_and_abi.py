@@ -282,3 +282,25 @@ def test_unsupported_shapes_are_rejected_where_the_model_is_configured():
     for core in (NSACore, HFNSACore):
         with pytest.raises(AssertionError, match="not built"):
             core(loose)
+
+
+def test_ranges_of_stored_ds_cover_the_batch():
+    """Ranges of whole 128-token groups, none shorter than the rows that fill the GPU, up to the last token."""
+    from flash_nsa import _lib
+    for T, B, longest, QH, KH in ((65536, 1, 65536, 64, 4), (48362, 8, 8192, 64, 4), (1 << 20, 1, 1 << 20, 64, 4),
+                                  (70001, 3, 60000, 16, 1), (100, 2, 60, 8, 1)):
+        at, ranges = 0, []
+        while at < T:
+            end = _lib.value("nsa_bwd_ds_next", at, T, B, longest, QH, KH, 32, 16, 512)
+            ranges.append((at, end))
+            at = end
+        assert at == T and all(s % 128 == 0 for s, _ in ranges)
+        assert len(ranges) == 1 or min(e - s for s, e in ranges) * QH >= 131072
+        ring = max(e - s for s, e in ranges)
+        for s, e in ranges:  # a range's tiles fit what the whole batch would take
+            whole = _lib.value("nsa_cmp_attn_bwd_ds_bytes", T, B, longest, QH, KH, 32, 16, 0, 0)
+            assert 0 < _lib.value("nsa_cmp_attn_bwd_ds_bytes", T, B, longest, QH, KH, 32, 16, s, e) <= whole
+        assert 0 < _lib.value("nsa_swa_bwd_ds_bytes", T, B, longest, QH, KH, 512, ring) <= \
+            _lib.value("nsa_swa_bwd_ds_bytes", T, B, longest, QH, KH, 512, 0)
+    # no scratch where no query has keys before its window
+    assert _lib.value("nsa_slc_bwd_before_window_ds_bytes", 5000, 1, 5000, 64, 4, 2000, 1024, 0) == 0
