@@ -33,6 +33,13 @@ NSA_DEVICE constexpr int swz(int r) { return CP % 16 == 0 ? (r & 15) : ((r >> 1)
 template <int CP>
 NSA_DEVICE constexpr int swzv(int r) { return CP % 16 == 0 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1); }
 
+// a wave-uniform address in scalar registers (one that divisions went into is uniform and in vector registers)
+NSA_DEVICE const char* scalar_ptr(const void* x) {
+  const uint64_t v = reinterpret_cast<uint64_t>(x);
+  const uint32_t l = __builtin_amdgcn_readfirstlane((uint32_t)v), h = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const char*>(((uint64_t)h << 32) | l);
+}
+
 // ASYNC: the K/V tiles go from global memory straight into LDS (global_load_lds, 16 bytes per lane, no staging
 // registers, no ds_write); the tiles are then unpadded and swizzled instead of padded.
 template <int D, int VD, int MODE, bool PAGED, int RS, int MINB, bool ASYNC>
@@ -162,9 +169,10 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   // Fragment addresses.  Padded tiles: row * stride + column, the compiler folds everything but the lane part into
   // immediates.  Swizzled tiles with a power-of-two row size: byte address = lane part XOR (index << 5 or 6) +
   // compile-time row offset, with the lane parts computed once (kx, vxa, vxb), so a read costs at most one v_xor.
-  constexpr bool POW2 = (D == 64 || D == 128) && (VD == 64 || VD == 128);
+  // (192 channels: a row of three 128-byte pieces, the swizzle stays inside a piece)
+  constexpr bool XORED = (D == 64 || D == 128 || D == 192) && (VD == 64 || VD == 128);
   int kx = 0, vxa = 0, vxb = 0;
-  if constexpr (ASYNC && POW2) {
+  if constexpr (ASYNC && XORED) {
     const int s0 = swz<D / 8>(l32);
     kx = (l32 * D * 2 + ((hl ^ (s0 & 1)) << 4)) ^ ((s0 >> 1) << 5);
     const int sl = hl * 4 + (i16 >> 2);                 // row of the fragment inside its group of 16 rows
@@ -175,7 +183,10 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   }
   // K fragment: rows l32 + 32*half, chunk 2*kc + hl
   auto kfrag = [&](const bf16_t* Ks, int half, int kc) -> bf16x8 {
-    if constexpr (ASYNC && POW2)
+    if constexpr (ASYNC && XORED && D == 192)
+      return *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(Ks) + half * 32 * D * 2 + (kc >> 2) * 128 +
+                                              (kx ^ ((kc & 3) << 5)));
+    else if constexpr (ASYNC && XORED)
       return *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(Ks) + half * 32 * D * 2 + (kx ^ (kc << 5)));
     else if constexpr (ASYNC)
       return *reinterpret_cast<const bf16x8*>(
@@ -186,7 +197,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   // transposed V fragment piece: row kb + (i16 >> 2) (kb a multiple of 16, plus 8 for the second piece), columns
   // dt*32 + (g16&1)*16 + 4*(i16&3) ..
   auto vfrag = [&](const bf16_t* Vs, int kb16, int second, int dt) -> bf16x4 {
-    if constexpr (ASYNC && POW2) {
+    if constexpr (ASYNC && XORED) {
       const int x = (second ? vxb : vxa) ^ (dt << 6);
       return lds_read_tr(reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(Vs) + kb16 * VD * 2 + x));
     } else {
@@ -284,18 +295,22 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   };
   // ASYNC staging: lane L of a wave's j-th load fills LDS piece j*256 + wave*64 + L (row = piece / chunks per row,
   // position = piece % chunks per row), i.e. it fetches the chunk that the swizzle puts at that position
-  // per-lane byte offsets of its pieces from the first row of a tile (the same for every full tile)
-  int goffk[KJ], goffv[VJ];
+  // Per-lane byte offsets of its pieces from the first row of a tile (the same for every full tile): after KPAT / VPAT loads
+  // columns and swizzle repeat, KROWS / VROWS rows further.
+  constexpr int KPAT = 256 % KP == 0 ? 1 : 3, VPAT = 256 % VP == 0 ? 1 : 3;
+  constexpr int KROWS = KPAT * 256 / KP, VROWS = VPAT * 256 / VP;
+  static_assert(!ASYNC || (KROWS % 16 == 0 && VROWS % 16 == 0 && KJ % KPAT == 0 && VJ % VPAT == 0), "period of the swizzles");
+  uint32_t goffk[KPAT], goffv[VPAT];
   if constexpr (ASYNC) {
 #pragma unroll
-    for (int j = 0; j < KJ; j++) {
+    for (int j = 0; j < KPAT; j++) {
       const int pc = tid + j * 256, row = pc / KP;
-      goffk[j] = (int)((row * p.k_sr + ((pc % KP) ^ swz<KP>(row)) * 8) * 2);
+      goffk[j] = (uint32_t)((row * p.k_sr + ((pc % KP) ^ swz<KP>(row)) * 8) * 2);
     }
 #pragma unroll
-    for (int j = 0; j < VJ; j++) {
+    for (int j = 0; j < VPAT; j++) {
       const int pc = tid + j * 256, row = pc / VP;
-      goffv[j] = (int)((row * p.v_sr + ((pc % VP) ^ swzv<VP>(row)) * 8) * 2);
+      goffv[j] = (uint32_t)((row * p.v_sr + ((pc % VP) ^ swzv<VP>(row)) * 8) * 2);
     }
   }
   auto stage_async = [&](int kt, int buf) {
@@ -303,17 +318,19 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     if (PAGED) row0 = (int64_t)table[kt / p.page_size] * p.page_size + (kt % p.page_size);
     else row0 = (int64_t)kbase + kt;
     const int last = key_end - 1 - kt;  // >= 0; rows past it repeat it (masked)
-    const char* kb = reinterpret_cast<const char*>(p.k + row0 * p.k_sr + (int64_t)kh * p.k_sh);
-    const char* vb = reinterpret_cast<const char*>(p.v + row0 * p.v_sr + (int64_t)kh * p.v_sh);
+    const char* kb = scalar_ptr(p.k + row0 * p.k_sr + (int64_t)kh * p.k_sh);
+    const char* vb = scalar_ptr(p.v + row0 * p.v_sr + (int64_t)kh * p.v_sh);
     if (last >= KT - 1) {  // wave-uniform
 #pragma unroll
-      for (int j = 0; j < KJ; j++)
-        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(kb + goffk[j]),
-                                         (nsa_lptr_t)&Ks2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
+      for (int j = 0; j < KJ; j++) {
+        const char* at = kb + (int64_t)(j / KPAT) * KROWS * p.k_sr * 2;
+        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + goffk[j % KPAT]), (nsa_lptr_t)&Ks2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
+      }
 #pragma unroll
-      for (int j = 0; j < VJ; j++)
-        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(vb + goffv[j]),
-                                         (nsa_lptr_t)&Vs2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
+      for (int j = 0; j < VJ; j++) {
+        const char* at = vb + (int64_t)(j / VPAT) * VROWS * p.v_sr * 2;
+        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + goffv[j % VPAT]), (nsa_lptr_t)&Vs2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
+      }
     } else {
 #pragma unroll
       for (int j = 0; j < KJ; j++) {
@@ -516,12 +533,14 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 template <int D, int VD, int MODE, bool PAGED>
 int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
-  // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there;
-  // the window branch, with its short key loops, and d=192, whose swizzled addresses cost registers, are faster with
-  // register staging); 1..4 force one variant for experiments
+  // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there; the window
+  // branch, with its short key loops, is level with register staging) and for 192 channels everywhere: two of its unpadded
+  // tile buffers fill half of a CU's LDS, two padded ones more than that, which leaves one workgroup on a CU.  32 heads of 192,
+  // 16K tokens, register staging / so, us: staged forward 1921 / 1640, fused 1925 / 1587, training step 5830 / 5495; 8 x 2K paged
+  // queries behind up to 8K 1352 / 1118.  1..4 force one variant for experiments.
   const int variant = nsa_tuning_knob("fwd_variant", 0);
   constexpr bool pow2 = (D == 64 || D == 128) && (VD == 64 || VD == 128);
-  const bool async = variant == 4 || (variant == 0 && MODE == MODE_CMP && pow2);
+  const bool async = variant == 4 || (variant == 0 && ((MODE == MODE_CMP && pow2) || D == 192));
   if constexpr (D > 192 || VD > 128) {
     // head dims of 256: the output accumulators alone take 128 registers, one workgroup per CU
     dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
@@ -529,6 +548,12 @@ int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t
     return nsa_check_launch("fwd_tile_kernel");
   } else if constexpr (MODE == MODE_TAIL) {
     dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
+    if constexpr (D == 192) {
+      if (variant != 1) {
+        fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, true><<<grid, 256, 0, stream>>>(p);
+        return nsa_check_launch("fwd_tile_kernel");
+      }
+    }
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, false><<<grid, 256, 0, stream>>>(p);
   } else if (variant == 2) {
     dim3 grid(cdiv_i(max_q_len * p.G, 256), B, p.KH);

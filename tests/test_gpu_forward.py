@@ -272,3 +272,22 @@ def test_selected_and_window_branch_round_their_probabilities_apart(device, QH, 
     b = (swa_fwd(q, k, v)[0].double() - _attend64(q, k, v, near, D ** -0.5))[W + 1:]
     assert float((a * b).sum() / a.norm() / b.norm()) < 0.03
     setup_helper(cu.to(device))
+
+
+@pytest.mark.parametrize("QH,KH,lens", [(8, 1, [1, 31, 63, 64, 65, 129]), (32, 2, [700, 1100]), (12, 2, [513, 40])])
+def test_192_channels_staged_straight_into_lds(device, QH, KH, lens):
+    """192 q/k channels: both staging variants of the dense kernels do the same arithmetic in the same order, so the branches,
+    the window branch continued over earlier keys and the gated sum are the same bits."""
+    from flash_nsa import HFNSACore, NSAConfig, NSACore, _lib
+    cu = make_cu(lens).to(device)
+    args = [t.to(device) for t in make_qkvw(sum(lens), QH, KH, 192, 128, seed=71)]
+    cfg = NSAConfig(qk_head_dim=192, v_head_dim=128, num_heads=QH, num_kv_heads=KH, window_size=300)
+    for core in (NSACore(cfg), HFNSACore(cfg)):
+        with torch.no_grad():
+            got = core(*args, cu)
+            _lib.call("nsa_set_tuning", b"fwd_variant", 1)
+            try:
+                want = core(*args, cu)
+            finally:
+                _lib.call("nsa_reset_tuning")
+        assert torch.equal(got, want)
