@@ -28,6 +28,7 @@ struct NsaFwdTileParams {
   const bf16_t* cmp_o; int64_t co_st, co_sh;
   const bf16_t* w; int64_t w_st, w_sh;      // gates [tokens, QH, 3]
   bf16_t* out; int64_t out_st, out_sh;
+  bool last_first;                            // a sequence's last rows first (set by the launcher)
 };
 
 struct NsaSlcParams {

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int ctx = PAGED ? p.ctx_lens[b] : xl;
   const int qoff = ctx - xl;
   const int rows_total = xl * G;
-  const int r0 = blockIdx.x * ROWS_WG;
+  const int r0 = (p.last_first ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * ROWS_WG;
   if (r0 >= rows_total) return;
   int nkeys, kbase = 0;
   if (MODE == MODE_CMP) {
@@ -484,6 +484,34 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       };
+      // The gates of a row are computed by the lane that holds it, and everything else that a lane adds is requested before the
+      // first row comes out of LDS: one round trip instead of one per row and half.  Calls before / with this, us: 16 x 2K paged
+      // rows 5447 / 5370, 8 x 6K tokens 6060 / 5980, three short prompts 76.9 / 73.3; the same bits.
+      float gate[3] = {0.f, 0.f, 0.f};
+      if (valid[0]) {
+        const bf16_t* wp = p.w + tok[0] * p.w_st + (int64_t)head[0] * p.w_sh;
+#pragma unroll
+        for (int e = 0; e < 3; e++) gate[e] = 1.f / (1.f + __expf(-(float)wp[e]));
+      }
+      constexpr int NR = 32 / HRPI;              // rows of a lane
+      const int cl = lane % HC;
+      int2 th[NR];
+      bf16x8 vc[NR][2], vx[NR][2];               // compressed branch; selected or window branch where it is not in registers
+#pragma unroll
+      for (int k = 0; k < NR; k++) {
+        th[k] = row_id(std::integral_constant<int, 0>{}, lane / HC + k * HRPI);
+        const int64_t tk = (int64_t)x0 + max(th[k].x, 0), hd = th[k].y;
+        const bf16_t* const cp = p.cmp_o + tk * p.co_st + hd * p.co_sh + cl * 8;
+        const bool all_of_it = th[k].x + qoff < p.all_below;
+        const bf16_t* const xp = all_of_it ? p.o + tk * p.o_st + hd * p.o_sh + cl * 8
+                                           : p.slc_o + tk * p.so_st + hd * p.so_sh + cl * 8;
+        const bool stored = th[k].x >= 0 && (!all_of_it || th[k].x + qoff > p.window);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          vc[k][h] = th[k].x >= 0 ? ld_global_b128(cp + h * HC * 8) : zero_bf16x8();
+          vx[k][h] = stored ? ld_global_b128(xp + h * HC * 8) : zero_bf16x8();
+        }
+      }
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         lds_order();
@@ -494,35 +522,21 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
               f32x4{oacc[0][dt][i] * inv, oacc[0][dt][i + 1] * inv, oacc[0][dt][i + 2] * inv, oacc[0][dt][i + 3] * inv};
         }
         lds_order();
-        const int cl = lane % HC, c = h * HC + cl;
 #pragma unroll
-        for (int r = lane / HC; r < 32; r += HRPI) {
-          const int2 th = row_id(std::integral_constant<int, 0>{}, r);
-          if (th.x < 0) continue;
-          const int64_t tk = (int64_t)x0 + th.x, hd = th.y;
-          const bool all_of_it = th.x + qoff < p.all_below;
-          const bf16_t* wp = p.w + tk * p.w_st + hd * p.w_sh;
-          const bf16x8 vc = ld_global_b128(p.cmp_o + tk * p.co_st + hd * p.co_sh + c * 8);
+        for (int k = 0; k < NR; k++) {
+          const int r = lane / HC + k * HRPI;
+          const float s0 = __shfl(gate[0], r, 64), s1 = __shfl(gate[1], r, 64), s2 = __shfl(gate[2], r, 64);
+          if (th[k].x < 0) continue;
+          const bool all_of_it = th[k].x + qoff < p.all_below, from_o = all_of_it && th[k].x + qoff > p.window;
           const f32x4 x0v = *reinterpret_cast<const f32x4*>(half_at(r, cl));
           const f32x4 x1v = *reinterpret_cast<const f32x4*>(half_at(r, cl) + 4);
-          float vw[8], vs[8];
-#pragma unroll
-          for (int e = 0; e < 8; e++) vw[e] = vs[e] = e < 4 ? x0v[e] : x1v[e - 4];
-          if (!all_of_it) {
-            const bf16x8 x = ld_global_b128(p.slc_o + tk * p.so_st + hd * p.so_sh + c * 8);
-#pragma unroll
-            for (int e = 0; e < 8; e++) vs[e] = (float)x[e];
-          } else if (th.x + qoff > p.window) {
-            const bf16x8 x = ld_global_b128(p.o + tk * p.o_st + hd * p.o_sh + c * 8);
-#pragma unroll
-            for (int e = 0; e < 8; e++) vw[e] = (float)x[e];
-          }
-          const float s0 = 1.f / (1.f + __expf(-(float)wp[0])), s1 = 1.f / (1.f + __expf(-(float)wp[1])),
-                      s2 = 1.f / (1.f + __expf(-(float)wp[2]));
           float x[8];
 #pragma unroll
-          for (int e = 0; e < 8; e++) x[e] = (float)vc[e] * s0 + vs[e] * s1 + vw[e] * s2;
-          *reinterpret_cast<bf16x8*>(p.out + tk * p.out_st + hd * p.out_sh + c * 8) =
+          for (int e = 0; e < 8; e++) {
+            const float own = e < 4 ? x0v[e] : x1v[e - 4], other = (float)vx[k][h][e];
+            x[e] = (float)vc[k][h][e] * s0 + (all_of_it ? own : other) * s1 + (from_o ? other : own) * s2;
+          }
+          *reinterpret_cast<bf16x8*>(p.out + ((int64_t)x0 + th[k].x) * p.out_st + (int64_t)th[k].y * p.out_sh + (h * HC + cl) * 8) =
               pack8(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
         }
       }
@@ -531,8 +545,15 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 }
 
 template <int D, int VD, int MODE, bool PAGED>
-int launch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, hipStream_t stream) {
+int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_t stream) {
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
+  NsaFwdTileParams p = p0;
+  // Queries that select everything see 1 to 24 tiles of keys, the last rows of a short prompt the most: in a launch of few
+  // rounds of workgroups these go first.  Paged, 64 / 4 heads of 128, us, first / last rows first: 3 prompts of 60 to 700 tokens
+  // 73.5 / 72.5, 2 of 300 to 900 75.3 / 70.7, 6 of 60 to 1000 129.8 / 127.1, 12 252.0 / 252.5; one sequence of 4K tokens 159.4 /
+  // 163.9.
+  p.last_first = MODE == MODE_TAIL && max_q_len <= p.all_below &&
+                 (int64_t)cdiv_i(max_q_len * p.G, 128) * B * p.KH <= 16 * nsa_device_cus();
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there; the window
   // branch, with its short key loops, is level with register staging) and for 192 channels everywhere: two of its unpadded
   // tile buffers fill half of a CU's LDS, two padded ones more than that, which leaves one workgroup on a CU.  32 heads of 192,
