@@ -11,7 +11,10 @@
 // fit there (64 heads of 128, 8 x 6K tokens: the CU's address unit is busy 85 % of the cycles, LDS 66 %), else from the
 // memory-side cache (64K tokens: 15.3 TB/s of requests, 6.4 of them past L2).  Two units in flight per wave and separate K and V
 // regions bought nothing over one, and took the registers and the LDS of a second workgroup per CU at 192 channels: 32 heads,
-// 16K tokens 1726 -> 1080 us; 64 heads of 128, 8 x 6K tokens 4207 -> 3920 us.
+// 16K tokens 1726 -> 1080 us; 64 heads of 128, 8 x 6K tokens 4207 -> 3920 us.  The rows lie unpadded and swizzled in LDS
+// (UnitRows::place): padded by 48 bytes, a quarter of the cycles in which LDS worked were bank conflicts, and the padded offsets
+// took registers (14 spilled at 128 channels).  Whole calls, padded / so, us: 64 heads of 128, 64K tokens 18930 / 18590, 16 x 2K
+// paged queries 5290 / 5170, 16 heads, 4K tokens 185 / 182.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
 #include "nsa_units.h"
@@ -37,9 +40,10 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   // and the K rows in LDS are no longer needed: K and V take turns in one LDS region.
   constexpr int UK = 32;                      // keys per unit
   constexpr int KC = D / 32;                  // K fragments per 16-key tile
-  constexpr int KLD = D + NSA_LDS_PAD, VLD = VD + NSA_LDS_PAD;
+  constexpr bool SWZ = D >= 64 && VD >= 64;    // unpadded rows, chunks swizzled
+  constexpr int KLD = SWZ ? D : D + NSA_LDS_PAD, VLD = SWZ ? VD : VD + NSA_LDS_PAD;
   constexpr int LD = KLD > VLD ? KLD : VLD;
-  __shared__ __attribute__((aligned(16))) bf16_t rows_all[4 * UK * LD];
+  __shared__ __attribute__((aligned(1024))) bf16_t rows_all[4 * UK * LD];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -103,6 +107,15 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   for (int j = 0; j < VRows::PAT; j++) voff[j] = VRows::offset(j, lane, p.v_sr);
   KRows kr;
   VRows vr;
+  // place in LDS of the lane's piece of instruction j
+  int kput[KRows::SPAT], vput[VRows::SPAT];
+  if (SWZ) {
+#pragma unroll
+    for (int j = 0; j < KRows::SPAT; j++) kput[j] = KRows::place(j, lane);
+#pragma unroll
+    for (int j = 0; j < VRows::SPAT; j++) vput[j] = VRows::place(j, lane);
+  }
+  const int ksw = KRows::swz(l16), vsw = VRows::swz(kq * 4 + (l16 >> 2));
   UnitList ul;
   // flat row of the first key of unit i (a unit never straddles a page)
   auto flat_row = [&](int i) -> int64_t {
@@ -136,16 +149,19 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   // 4K tokens 113 -> 109 us; 32 heads of 192, 16K tokens 1072 -> 1043 us.
   auto unit = [&](auto how_next, int i) {
     const int key0 = __builtin_amdgcn_readlane(ul.key0, i);
-    kr.to_lds(rows, KLD, lane);
+    if (SWZ) kr.to_lds_swz(rows, kput);
+    else kr.to_lds(rows, KLD, lane);
     lds_order();
     issue_k(how_next, i + 1);
     f32x4 sacc[2];
 #pragma unroll
     for (int jt = 0; jt < 2; jt++) {
       sacc[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const bf16_t* kp = &rows[(jt * 16 + l16) * KLD + kq * 8];
 #pragma unroll
-      for (int kc = 0; kc < KC; kc++) sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(kp + kc * 32), qf[kc], sacc[jt]);
+      for (int kc = 0; kc < KC; kc++) {
+        const int at = SWZ ? KRows::col(kc * 4, kq ^ (ksw & 3), ksw & ~3) * 8 : kc * 32 + kq * 8;
+        sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(&rows[(jt * 16 + l16) * KLD + at]), qf[kc], sacc[jt]);
+      }
     }
     const int kmax = key_last - key0;  // last usable key offset inside this unit
     if (decltype(how_next)::value != FULL && kmax < UK - 1) {  // wave-uniform: the unit holding the causal boundary
@@ -183,7 +199,8 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
     }
     l_run += psum;
     lds_order();
-    vr.to_lds(rows, VLD, lane);
+    if (SWZ) vr.to_lds_swz(rows, vput);
+    else vr.to_lds(rows, VLD, lane);
     lds_order();
     issue_v(how_next, i + 1);
     // O^T += V^T P^T over the 32 keys of the unit
@@ -192,7 +209,7 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
     const int kb1 = kb0 + 16;
 #pragma unroll
     for (int dt = 0; dt < VD / 16; dt++) {
-      const int col = dt * 16 + 4 * (l16 & 3);
+      const int col = SWZ ? VRows::col(dt * 2, (l16 & 3) >> 1, vsw) * 8 + (l16 & 1) * 4 : dt * 16 + 4 * (l16 & 3);
       bf16x4 v0 = lds_read_tr(&rows[kb0 * VLD + col]);
       bf16x4 v1 = lds_read_tr(&rows[kb1 * VLD + col]);
       oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);

@@ -80,6 +80,25 @@ struct UnitRows {
       r[j] = ld_global_b128(first + (int64_t)min(pc / P, last) * row_stride + (pc % P) * 8);
     }
   }
+  // Rows in LDS without padding: row r holds its 16-byte chunk c at c ^ swz(r), which spreads row fragments (16 rows x 64 bytes)
+  // and transposed ones (16 rows x 32 bytes) over all banks.  swz: even, below 16 (rows of whole bank rounds) or 8.
+  static constexpr bool WIDE = CHANNELS % 128 == 0;
+  static constexpr int SPAT = 64 % P == 0 ? (64 / P < 8 ? (WIDE ? 8 * P / 64 : 2) : 1) : 3;  // instructions after which it repeats
+  static NSA_DEVICE int swz(int r) { return WIDE ? (r & 7) << 1 : ((r >> 1) & 3) << 1; }
+  static NSA_DEVICE int place(int j, int lane) {
+    const int pc = lane + j * 64, r = pc / P;
+    return r * CHANNELS + ((pc % P) ^ swz(r)) * 8;
+  }
+  // chunk c0 + c (c0 a constant multiple of what the swizzle's remaining bits sw count in), swizzled
+  static NSA_DEVICE int col(int c0, int c, int sw) {
+    constexpr int M = WIDE ? 16 : 8;
+    return c0 / M * M + (((c0 % M) ^ sw) + c);
+  }
+  NSA_DEVICE void to_lds_swz(bf16_t* rows, const int (&put)[SPAT]) const {
+#pragma unroll
+    for (int j = 0; j < N; j++)
+      *reinterpret_cast<bf16x8*>(&rows[put[j % SPAT] + j / SPAT * (SPAT * 64 / P) * CHANNELS]) = r[j];
+  }
   NSA_DEVICE void to_lds(bf16_t* rows, int ld, int lane) const {
 #pragma unroll
     for (int j = 0; j < N; j++) {
