@@ -291,3 +291,24 @@ def test_192_channels_staged_straight_into_lds(device, QH, KH, lens):
             finally:
                 _lib.call("nsa_reset_tuning")
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens", [
+    (16, 1, 128, 128, [511, 512, 513, 1, 700]),       # top_n * block_size = 512: the window kernel finishes rows below it
+    (12, 4, 64, 64, [40, 0, 640]),
+    (8, 2, 192, 128, [300, 33]),                      # no query has blocks to choose from
+])
+def test_staged_core_without_gradients_is_the_staged_core(device, QH, KH, D, VD, lens):
+    """Without gradients one function forms the gated sum (the window kernel, over the selected branch of the later queries
+    alone); with gradients every stage is a node of its own.  Sizes that the selector refuses are refused either way."""
+    from flash_nsa import HFNSACore, NSAConfig
+    cu = make_cu(lens).to(device)
+    args = [t.to(device) for t in make_qkvw(sum(lens), QH, KH, D, VD, seed=72)]
+    kw = dict(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH, top_n=8, window_size=128)
+    core = HFNSACore(NSAConfig(**kw))
+    want = core(*args, cu)
+    with torch.no_grad():
+        assert_close(core(*args, cu), want.detach(), "o")
+        core.num_local_blocks = 8  # with the initial block more than top_n
+        with pytest.raises(RuntimeError):
+            core(*args, cu)
