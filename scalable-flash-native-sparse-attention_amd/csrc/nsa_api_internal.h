@@ -45,6 +45,7 @@ struct NsaSlcParams {
   float scale_log2;
   int t_begin;                                // only queries at positions from here on
   int sweep;                                  // queries that the GPU holds at once (set by the launcher; 0: blocks in key order)
+  int reg_below;                              // queries at positions below it keep V out of LDS (set by the launcher)
 };
 
 struct NsaTopkParams {

@@ -4,7 +4,7 @@
 //
 // The keys of the selected blocks are processed in units of 32.  The K and V rows of a unit are fetched as whole
 // coalesced rows (16 lanes x 16 bytes per row) into registers one unit ahead, pass through a wave-private LDS
-// region, and are read back as MFMA fragments (K row-major, V through ds_read_b64_tr_b16, which delivers the
+// region (V: see below), and are read back as MFMA fragments (K row-major, V through ds_read_b64_tr_b16, which delivers the
 // key-contraction slices).  Keys are gathered by the per-token block list topk[kh, t, 0 .. min(top_n, t/block+1)).
 //
 // What bounds it is the gather: 512 KB of rows per token and kv head, from L2 while the keys of the sequences in flight
@@ -15,9 +15,15 @@
 // (UnitRows::place): padded by 48 bytes, a quarter of the cycles in which LDS worked were bank conflicts, and the padded offsets
 // took registers (14 spilled at 128 channels).  Whole calls, padded / so, us: 64 heads of 128, 64K tokens 18930 / 18590, 16 x 2K
 // paged queries 5290 / 5170, 16 heads, 4K tokens 185 / 182.
+// With 128 v channels the V rows of all but long sequences do not pass through LDS at all: an instruction fetches the rows whose
+// scores its lanes hold, so the transposition stays inside a lane (UnitColumns128).  LDS moves 16 KB per unit instead of 32 (a
+// quarter of them transposed reads, the slowest).  This kernel, us, through LDS / so: 64 heads of 128, 8 x 6K tokens 3830 / 3330
+// (25 TB/s of requests), 16 x 2K paged queries behind up to 16K 2941 / 2761, one sequence of 4K tokens, 16 heads 105 / 85; 32 heads of
+// 192, 16K tokens 964 / 869.  Outputs are the same bits.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
 #include "nsa_units.h"
+#include <type_traits>
 
 namespace {
 
@@ -90,157 +96,179 @@ __global__ __launch_bounds__(256, slc_waves(D)) void slc_fwd_kernel(NsaSlcParams
   if (p.sweep > 0 && t > (4 << 20) / ((D + VD) * 2))
     my_blk = rotate_blocks(my_blk, nvalid, lane, (int)((int64_t)(t % p.sweep) * (t / Bs + 1) / p.sweep));
 
-  f32x4 oacc[VD / 16];
+  auto attend = [&](auto vreg_tag) {
+    constexpr bool VREG = decltype(vreg_tag)::value;  // V is transposed in registers
+    f32x4 oacc[VD / 16];
 #pragma unroll
-  for (int dt = 0; dt < VD / 16; dt++) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = NSA_NEG_INF, l_run = 0.f;
-  const float sc = p.scale_log2;
+    for (int dt = 0; dt < VD / 16; dt++) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = NSA_NEG_INF, l_run = 0.f;
+    const float sc = p.scale_log2;
 
-  // K and V rows are fetched as whole 16-byte-per-lane coalesced rows (every cache line is requested once and used
-  // completely) and go through wave-private LDS; the MFMA fragments are read from there.
-  using KRows = UnitRows<D>;
-  using VRows = UnitRows<VD>;
-  uint32_t koff[KRows::PAT], voff[VRows::PAT];
+    // K and V rows are fetched as whole 16-byte-per-lane coalesced rows (every cache line is requested once and used
+    // completely) and go through wave-private LDS; the MFMA fragments are read from there.
+    using KRows = UnitRows<D>;
+    using VRows = std::conditional_t<VREG, UnitColumns128, UnitRows<VD>>;
+    uint32_t koff[KRows::PAT], voff[VRows::PAT];
 #pragma unroll
-  for (int j = 0; j < KRows::PAT; j++) koff[j] = KRows::offset(j, lane, p.k_sr);
+    for (int j = 0; j < KRows::PAT; j++) koff[j] = KRows::offset(j, lane, p.k_sr);
 #pragma unroll
-  for (int j = 0; j < VRows::PAT; j++) voff[j] = VRows::offset(j, lane, p.v_sr);
-  KRows kr;
-  VRows vr;
-  // place in LDS of the lane's piece of instruction j
-  int kput[KRows::SPAT], vput[VRows::SPAT];
-  if (SWZ) {
+    for (int j = 0; j < VRows::PAT; j++) voff[j] = VRows::offset(j, lane, p.v_sr);
+    KRows kr;
+    VRows vr;
+    // place in LDS of the lane's piece of instruction j
+    int kput[KRows::SPAT], vput[UnitRows<VD>::SPAT];
+    if (SWZ) {
 #pragma unroll
-    for (int j = 0; j < KRows::SPAT; j++) kput[j] = KRows::place(j, lane);
+      for (int j = 0; j < KRows::SPAT; j++) kput[j] = KRows::place(j, lane);
 #pragma unroll
-    for (int j = 0; j < VRows::SPAT; j++) vput[j] = VRows::place(j, lane);
-  }
-  const int ksw = KRows::swz(l16), vsw = VRows::swz(kq * 4 + (l16 >> 2));
-  UnitList ul;
-  // flat row of the first key of unit i (a unit never straddles a page)
-  auto flat_row = [&](int i) -> int64_t {
-    if (PAGED) return (int64_t)__builtin_amdgcn_readlane(ul.page, i) * p.page_size + __builtin_amdgcn_readlane(ul.off, i);
-    return (int64_t)x0 + __builtin_amdgcn_readlane(ul.key0, i);
-  };
-  // how the rows of a unit are requested: not at all, the unit is known to be full, or with the rows past the causal boundary
-  // replaced by the boundary row (masked later) and any stride
-  enum { NONE, FULL, ANY };
-  auto issue_k = [&](auto how, int i) {
-    if constexpr (decltype(how)::value == NONE) return;
-    const bf16_t* kb = p.k + flat_row(i) * p.k_sr + (int64_t)kh * p.k_sh;
-    if constexpr (decltype(how)::value == FULL) kr.load(kb, p.k_sr, koff);
-    else kr.load_clamped(kb, p.k_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
-  };
-  auto issue_v = [&](auto how, int i) {
-    if constexpr (decltype(how)::value == NONE) return;
-    const bf16_t* vb = p.v + flat_row(i) * p.v_sr + (int64_t)kh * p.v_sh;
-    if constexpr (decltype(how)::value == FULL) vr.load(vb, p.v_sr, voff);
-    else vr.load_clamped(vb, p.v_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
-  };
-  auto lds_order = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
-
-  // Unit i, the rows of unit i + 1 being requested meanwhile.  How is fixed per copy of the code: with a branch around the
-  // requests the compiler cannot tell this unit's V rows from them and waits for both.  With the unit list in lanes: 64 heads
-  // of 128, 8 x 6K tokens 3.85 -> 3.60 ms, paged, 16 x 2K queries behind up to 16K 3.11 -> 3.06 ms; 16 heads, one sequence of
-  // 4K tokens 113 -> 109 us; 32 heads of 192, 16K tokens 1072 -> 1043 us.
-  auto unit = [&](auto how_next, int i) {
-    const int key0 = __builtin_amdgcn_readlane(ul.key0, i);
-    if (SWZ) kr.to_lds_swz(rows, kput);
-    else kr.to_lds(rows, KLD, lane);
-    lds_order();
-    issue_k(how_next, i + 1);
-    f32x4 sacc[2];
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++) {
-      sacc[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kc = 0; kc < KC; kc++) {
-        const int at = SWZ ? KRows::col(kc * 4, kq ^ (ksw & 3), ksw & ~3) * 8 : kc * 32 + kq * 8;
-        sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(&rows[(jt * 16 + l16) * KLD + at]), qf[kc], sacc[jt]);
-      }
+      for (int j = 0; j < UnitRows<VD>::SPAT; j++) vput[j] = UnitRows<VD>::place(j, lane);
     }
-    const int kmax = key_last - key0;  // last usable key offset inside this unit
-    if (decltype(how_next)::value != FULL && kmax < UK - 1) {  // wave-uniform: the unit holding the causal boundary
+    const int ksw = KRows::swz(l16), vsw = UnitRows<VD>::swz(kq * 4 + (l16 >> 2));
+    UnitList ul;
+    // flat row of the first key of unit i (a unit never straddles a page)
+    auto flat_row = [&](int i) -> int64_t {
+      if (PAGED) return (int64_t)__builtin_amdgcn_readlane(ul.page, i) * p.page_size + __builtin_amdgcn_readlane(ul.off, i);
+      return (int64_t)x0 + __builtin_amdgcn_readlane(ul.key0, i);
+    };
+    // how the rows of a unit are requested: not at all, the unit is known to be full, or with the rows past the causal boundary
+    // replaced by the boundary row (masked later) and any stride
+    enum { NONE, FULL, ANY };
+    auto issue_k = [&](auto how, int i) {
+      if constexpr (decltype(how)::value == NONE) return;
+      const bf16_t* kb = p.k + flat_row(i) * p.k_sr + (int64_t)kh * p.k_sh;
+      if constexpr (decltype(how)::value == FULL) kr.load(kb, p.k_sr, koff);
+      else kr.load_clamped(kb, p.k_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
+    };
+    auto issue_v = [&](auto how, int i) {
+      if constexpr (decltype(how)::value == NONE) return;
+      const bf16_t* vb = p.v + flat_row(i) * p.v_sr + (int64_t)kh * p.v_sh;
+      if constexpr (decltype(how)::value == FULL) vr.load(vb, p.v_sr, voff);
+      else vr.load_clamped(vb, p.v_sr, min(key_last - __builtin_amdgcn_readlane(ul.key0, i), UK - 1));
+    };
+    auto lds_order = [&]() {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+
+    // Unit i, the rows of unit i + 1 being requested meanwhile.  How is fixed per copy of the code: with a branch around the
+    // requests the compiler cannot tell this unit's V rows from them and waits for both.  With the unit list in lanes: 64 heads
+    // of 128, 8 x 6K tokens 3.85 -> 3.60 ms, paged, 16 x 2K queries behind up to 16K 3.11 -> 3.06 ms; 16 heads, one sequence of
+    // 4K tokens 113 -> 109 us; 32 heads of 192, 16K tokens 1072 -> 1043 us.
+    auto unit = [&](auto how_next, int i) {
+      const int key0 = __builtin_amdgcn_readlane(ul.key0, i);
+      if (SWZ) kr.to_lds_swz(rows, kput);
+      else kr.to_lds(rows, KLD, lane);
+      lds_order();
+      issue_k(how_next, i + 1);
+      f32x4 sacc[2];
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++) {
+        sacc[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kc = 0; kc < KC; kc++) {
+          const int at = SWZ ? KRows::col(kc * 4, kq ^ (ksw & 3), ksw & ~3) * 8 : kc * 32 + kq * 8;
+          sacc[jt] = mfma16(*reinterpret_cast<const bf16x8*>(&rows[(jt * 16 + l16) * KLD + at]), qf[kc], sacc[jt]);
+        }
+      }
+      const int kmax = key_last - key0;  // last usable key offset inside this unit
+      if (decltype(how_next)::value != FULL && kmax < UK - 1) {  // wave-uniform: the unit holding the causal boundary
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            int ko = jt * 16 + (lane_id() >> 4) * 4 + i;
+            if (ko > kmax) sacc[jt][i] = NSA_NEG_INF;
+          }
+      }
+      float tmax = fmaxf(fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3])),
+                         fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
+      tmax = xrow_max(tmax);
+      tmax = xhalf_max(tmax);
+      const float m_old = m_run;
+      const float m_new = fmaxf(m_old, tmax);
+      const float m_safe = (m_new == NSA_NEG_INF) ? 0.f : m_new;
+      const float msc = __builtin_fmaf(m_safe, sc, -SLC_P_LOG2);
+      m_run = m_new;
+      float psum = 0.f;
 #pragma unroll
       for (int jt = 0; jt < 2; jt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          int ko = jt * 16 + (lane_id() >> 4) * 4 + i;
-          if (ko > kmax) sacc[jt][i] = NSA_NEG_INF;
+          float pv = fast_exp2(__builtin_fmaf(sacc[jt][i], sc, -msc));
+          sacc[jt][i] = pv;
+          psum += pv;
         }
-    }
-    float tmax = fmaxf(fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3])),
-                       fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
-    tmax = xrow_max(tmax);
-    tmax = xhalf_max(tmax);
-    const float m_old = m_run;
-    const float m_new = fmaxf(m_old, tmax);
-    const float m_safe = (m_new == NSA_NEG_INF) ? 0.f : m_new;
-    const float msc = __builtin_fmaf(m_safe, sc, -SLC_P_LOG2);
-    m_run = m_new;
-    float psum = 0.f;
+      if (__builtin_amdgcn_ballot_w64(m_new != m_old) != 0) {
+        const float alpha = fast_exp2((m_old - m_safe) * sc);
+        l_run *= alpha;
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        float pv = fast_exp2(__builtin_fmaf(sacc[jt][i], sc, -msc));
-        sacc[jt][i] = pv;
-        psum += pv;
+        for (int dt = 0; dt < VD / 16; dt++) oacc[dt] *= alpha;
       }
-    if (__builtin_amdgcn_ballot_w64(m_new != m_old) != 0) {
-      const float alpha = fast_exp2((m_old - m_safe) * sc);
-      l_run *= alpha;
+      l_run += psum;
+      // O^T += V^T P^T over the 32 keys of the unit
+      const bf16x8 pf = pack8(sacc[0][0], sacc[0][1], sacc[0][2], sacc[0][3], sacc[1][0], sacc[1][1], sacc[1][2], sacc[1][3]);
+      if constexpr (VREG) {
+        vr.multiply(oacc, pf, std::make_integer_sequence<int, 8>{});
+        issue_v(how_next, i + 1);
+      } else {
+        lds_order();
+        if (SWZ) vr.to_lds_swz(rows, vput);
+        else vr.to_lds(rows, VLD, lane);
+        lds_order();
+        issue_v(how_next, i + 1);
+        const int kb0 = kq * 4 + (l16 >> 2);
+        const int kb1 = kb0 + 16;
 #pragma unroll
-      for (int dt = 0; dt < VD / 16; dt++) oacc[dt] *= alpha;
+        for (int dt = 0; dt < VD / 16; dt++) {
+          const int col = SWZ ? UnitRows<VD>::col(dt * 2, (l16 & 3) >> 1, vsw) * 8 + (l16 & 1) * 4 : dt * 16 + 4 * (l16 & 3);
+          bf16x4 v0 = lds_read_tr(&rows[kb0 * VLD + col]);
+          bf16x4 v1 = lds_read_tr(&rows[kb1 * VLD + col]);
+          oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
+        }
+      }
+      lds_order();
+    };
+    for (int base = 0; base < nu; base += 64) {
+      ul = unit_list<PAGED>(my_blk, nvalid, base, Bs, key_last, table, p.page_size, lane, [](int, int, int) { return 0; });
+      if (ul.n == 0) continue;
+      const int n_full = p.k_sr < KRows::NARROW && p.v_sr < VRows::NARROW ? ul.n_full : 0;
+      int i = 0;
+      issue_k(std::integral_constant<int, ANY>{}, 0);
+      issue_v(std::integral_constant<int, ANY>{}, 0);
+      for (; i + 1 < n_full; i++) unit(std::integral_constant<int, FULL>{}, i);
+      for (; i + 1 < ul.n; i++) unit(std::integral_constant<int, ANY>{}, i);
+      unit(std::integral_constant<int, NONE>{}, i);
     }
-    l_run += psum;
-    lds_order();
-    if (SWZ) vr.to_lds_swz(rows, vput);
-    else vr.to_lds(rows, VLD, lane);
-    lds_order();
-    issue_v(how_next, i + 1);
-    // O^T += V^T P^T over the 32 keys of the unit
-    bf16x8 pf = pack8(sacc[0][0], sacc[0][1], sacc[0][2], sacc[0][3], sacc[1][0], sacc[1][1], sacc[1][2], sacc[1][3]);
-    const int kb0 = kq * 4 + (l16 >> 2);
-    const int kb1 = kb0 + 16;
-#pragma unroll
-    for (int dt = 0; dt < VD / 16; dt++) {
-      const int col = SWZ ? VRows::col(dt * 2, (l16 & 3) >> 1, vsw) * 8 + (l16 & 1) * 4 : dt * 16 + 4 * (l16 & 3);
-      bf16x4 v0 = lds_read_tr(&rows[kb0 * VLD + col]);
-      bf16x4 v1 = lds_read_tr(&rows[kb1 * VLD + col]);
-      oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
-    }
-    lds_order();
-  };
-  for (int base = 0; base < nu; base += 64) {
-    ul = unit_list<PAGED>(my_blk, nvalid, base, Bs, key_last, table, p.page_size, lane, [](int, int, int) { return 0; });
-    if (ul.n == 0) continue;
-    const int n_full = p.k_sr < KRows::NARROW && p.v_sr < VRows::NARROW ? ul.n_full : 0;
-    int i = 0;
-    issue_k(std::integral_constant<int, ANY>{}, 0);
-    issue_v(std::integral_constant<int, ANY>{}, 0);
-    for (; i + 1 < n_full; i++) unit(std::integral_constant<int, FULL>{}, i);
-    for (; i + 1 < ul.n; i++) unit(std::integral_constant<int, ANY>{}, i);
-    unit(std::integral_constant<int, NONE>{}, i);
-  }
 
-  float l_tot = xrow_sum(l_run);
-  l_tot = xhalf_sum(l_tot);
-  if (!head_ok) return;
-  float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  bf16_t* op = p.o + tok * p.o_st + (int64_t)head * p.o_sh + kq * 4;
+    float l_tot = xrow_sum(l_run);
+    l_tot = xhalf_sum(l_tot);
+    if (!head_ok) return;
+    float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    bf16_t* const op = p.o + tok * p.o_st + (int64_t)head * p.o_sh;
+    if constexpr (VREG) {
 #pragma unroll
-  for (int dt = 0; dt < VD / 16; dt++) {
-    bf16x4 w = pack4(oacc[dt][0] * inv, oacc[dt][1] * inv, oacc[dt][2] * inv, oacc[dt][3] * inv);
-    *reinterpret_cast<bf16x4*>(op + dt * 16) = w;
+      for (int i = 0; i < 4; i++)
+        *reinterpret_cast<bf16x8*>(op + (kq * 4 + i) * 8) =
+            pack8(oacc[0][i] * inv, oacc[1][i] * inv, oacc[2][i] * inv, oacc[3][i] * inv, oacc[4][i] * inv, oacc[5][i] * inv,
+                  oacc[6][i] * inv, oacc[7][i] * inv);
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < VD / 16; dt++)
+        *reinterpret_cast<bf16x4*>(op + kq * 4 + dt * 16) =
+            pack4(oacc[dt][0] * inv, oacc[dt][1] * inv, oacc[dt][2] * inv, oacc[dt][3] * inv);
+    }
+    if (kq == 0 && p.lse != nullptr) {
+      p.lse[tok * p.lse_st + (int64_t)head * p.lse_sh] = l_tot > 0.f ? __builtin_fmaf(m_run, sc, -SLC_P_LOG2) + fast_log2(l_tot) : 0.f;
+    }
+  };
+  if constexpr (VD == 128) {
+    if (t < p.reg_below) {  // wave-uniform
+      attend(std::true_type{});
+      return;
+    }
   }
-  if (kq == 0 && p.lse != nullptr) {
-    p.lse[tok * p.lse_st + (int64_t)head * p.lse_sh] = l_tot > 0.f ? __builtin_fmaf(m_run, sc, -SLC_P_LOG2) + fast_log2(l_tot) : 0.f;
-  }
+  attend(std::false_type{});
 }
 
 // Paged: queries far behind their sequence's start are in flight from the launch's first moment on.  The first `sweep` of them
@@ -269,6 +297,15 @@ int launch_slc(const NsaSlcParams& p, int B, int max_q_len, hipStream_t stream) 
   const int sweep = nsa_device_cus() * slc_waves(D) * 4;
   const bool together = !PAGED || walk_together(D, max_q_len, (int64_t)max_q_len * grid.y * grid.z, sweep);
   p2.sweep = together ? sweep : 0;
+  // V in registers while the sequence fits the L2 of an XCD about one and a half times: LDS is what the gather waits for there.
+  // Beyond, memory is, and waves that wait for LDS in turn keep more together: 64K tokens with V in registers everywhere have 11 %
+  // more L2 misses.  Calls with V in registers below 0 / 6 / infinitely many MB of K and V per head, us, 64 / 4 heads of 128: one
+  // sequence of 8K tokens 1072 / 1012 / 1003, 16K 2489 / 2395 / 2354, 24K 4159 / 4074 / 4136, 32K 6168 / 6060 / 6604, 64K 18988 /
+  // 18979 / 19789; paged, 16 x 2K queries behind 2K 4425 / 4295 / 4264, behind 12K 6625 / 6687 / 6998.  192 channels, at two waves per
+  // SIMD, 0 / 6 / 10 MB / all: 16K tokens 1583 / 1532 / 1490 / 1518, 48K 8407 / 8270 / 8325 / 8388, paged, 8 x 2K queries behind 12K
+  // 1945 / 1947 / 1971 / 1966, behind 16K 2235 / 2235 / 2234 / 2432.  64 channels gain nothing (4K to 8K tokens the same to 0.3 %,
+  // 16K 550 -> 567).
+  p2.reg_below = ((D > 128 && !PAGED ? 10 : 6) << 20) / ((D + VD) * 2);
   slc_fwd_kernel<D, VD, PAGED><<<grid, 256, 0, stream>>>(p2);
   return nsa_check_launch("slc_fwd_kernel");
 }

@@ -1,5 +1,6 @@
 // The 32-key units that a query token's selected blocks consist of, as a list in the lanes of a wave.
 #pragma once
+#include <utility>
 #include "nsa_common.h"
 
 // Lane i of a wave holds unit i of a list of `n` (lanes from n on: leftovers).  Made for 64 units at a time by all lanes in
@@ -105,5 +106,52 @@ struct UnitRows {
       const int pc = lane + j * 64;
       *reinterpret_cast<bf16x8*>(&rows[(pc / P) * ld + (pc % P) * 8]) = r[j];
     }
+  }
+};
+
+// Rows of one unit as the operand whose contraction index is the row (V^T of O^T = V^T P^T): transposed in the lanes' own
+// registers instead of through LDS.  Lane (kq, l16) holds of every row that it loads the channels 8 l16 .. 8 l16 + 7: of the rows
+// jt * 16 + kq * 4 + i (jt < 2, i < 4), whose scores it holds (result rows of v_mfma_f32_16x16x32).  The operand of channel e of
+// all pieces is element e of the lane's own eight rows, four v_perm_b32; the matrix instruction with it yields the channels
+// 8 c + e, so lane (kq, head) ends up with the pieces c = kq * 4 + i, eight neighbouring channels each.
+struct UnitColumns128 {
+  static constexpr int N = 8, PAT = 1;
+  static constexpr int64_t NARROW = UnitRows<128>::NARROW;
+  bf16x8 r[N];
+
+  static constexpr int row(int j) { return (j >> 2) * 16 + (j & 3); }  // of the lanes with kq 0
+  static NSA_DEVICE uint32_t offset(int, int lane, int64_t row_stride) {
+    return (uint32_t)((lane >> 4) * 4) * (uint32_t)(row_stride * 2) + (lane & 15) * 16;
+  }
+  // all 32 rows (row strides below NARROW elements)
+  NSA_DEVICE void load(const bf16_t* first, int64_t row_stride, const uint32_t (&off)[PAT]) {
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+      const char* at = reinterpret_cast<const char*>(first + row(j) * row_stride);
+      uint32_t o = off[0];
+      asm volatile("" : "+s"(at), "+v"(o));  // (scalar base + 32-bit lane offset, as in UnitRows)
+      r[j] = *(const __attribute__((address_space(1))) bf16x8*)((const __attribute__((address_space(1))) char*)at + o);
+    }
+  }
+  // rows past row `last` replaced by it; any stride
+  NSA_DEVICE void load_clamped(const bf16_t* first, int64_t row_stride, int last) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int j = 0; j < N; j++)
+      r[j] = ld_global_b128(first + (int64_t)min(row(j) + (lane >> 4) * 4, last) * row_stride + (lane & 15) * 8);
+  }
+  template <int E>
+  NSA_DEVICE bf16x8 operand() const {
+    u32x4 x;
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      x[m] = __builtin_amdgcn_perm(__builtin_bit_cast(u32x4, r[2 * m + 1])[E / 2], __builtin_bit_cast(u32x4, r[2 * m])[E / 2],
+                                   E % 2 ? 0x07060302u : 0x05040100u);
+    return __builtin_bit_cast(bf16x8, x);
+  }
+  // acc[e] += operand e times b
+  template <int... E>
+  NSA_DEVICE void multiply(f32x4 (&acc)[N], bf16x8 b, std::integer_sequence<int, E...>) const {
+    ((acc[E] = mfma16(operand<E>(), b, acc[E])), ...);
   }
 };

@@ -1,5 +1,6 @@
 """GPU parity of the forward operators against the CPU oracle (same seeded bf16 inputs).
 Mirrors upstream test.py --func mean/construct/cmp/topk/slc/combine (test.py:74-318), with asserted tolerances."""
+import math
 import pytest
 import torch
 
@@ -312,3 +313,29 @@ def test_staged_core_without_gradients_is_the_staged_core(device, QH, KH, D, VD,
         core.num_local_blocks = 8  # with the initial block more than top_n
         with pytest.raises(RuntimeError):
             core(*args, cu)
+
+
+@pytest.mark.parametrize("G,D,edge", [(16, 128, 12288), (5, 128, 12288), (16, 192, 16384)])
+def test_selected_branch_either_side_of_the_length_that_v_stays_in_registers_for(device, G, D, edge):
+    """128 v channels: queries below `edge` transpose V in registers, later ones through LDS.  Both are the selected attention
+    of their blocks, with a boundary unit of every size among them."""
+    from flash_nsa.ops.select_attn import slc_attn_fwd
+    T, first, top_n = edge + 70, edge - 70, 16
+    cu = make_cu([T]).to(device)
+    setup_helper(cu, top_n=top_n)
+    q, k, v, _ = [x.to(device) for x in make_qkvw(T, G, 1, D, 128, seed=83)]
+    g = torch.Generator().manual_seed(84)
+    topk = torch.stack([torch.randperm(t // 64, generator=g)[:top_n] for t in range(first, T)]).to(torch.int32)
+    topk[:, 5] = torch.arange(first, T) // 64  # the query's own block
+    full = torch.zeros(1, T, top_n, dtype=torch.int32)
+    full[0, first:] = topk
+    o, lse = slc_attn_fwd(q, k, v, full.to(device), t_begin=first)
+    keys = (topk.long()[:, :, None] * 64 + torch.arange(64)).reshape(T - first, -1).to(device)
+    t = torch.arange(first, T, device=device)
+    kk, vv = k[:, 0].float()[keys.clamp(max=T - 1)], v[:, 0].float()[keys.clamp(max=T - 1)]
+    s = torch.matmul(q[first:].float(), kk.transpose(1, 2).contiguous()) * D ** -0.5
+    s = s.masked_fill((keys > t[:, None])[:, None], float("-inf"))
+    want = torch.matmul(s.softmax(-1), vv)
+    assert_close(o[first:], want, "slc_o")
+    assert_close(lse[first:], s.logsumexp(-1) / math.log(2.0), "slc_lse", atol=1e-3, rtol=1e-4)
+    setup_helper(make_cu([64]).to(device))
