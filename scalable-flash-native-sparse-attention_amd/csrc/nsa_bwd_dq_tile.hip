@@ -56,6 +56,8 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
   const int t = n;
   const int64_t tok = x0 + n;
   const int head = kh * G + g;
+  int key_lo = t - p.window, key_hi = t;  // first and last key that the row sees
+  if (MODE == MODE_CMP) key_hi = t >= p.kernel_size - 1 ? min((t - p.kernel_size + 1) / p.stride, nkeys - 1) : -1;
 
   bf16x8 qf[D / 16], dof[DO_LDS ? 1 : VD / 16];
   {
@@ -138,14 +140,14 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
     __syncthreads();
     if (kt + KT < key_end) gload(kt + KT);
     if (!wave_active) continue;
-    bool any_vis, full_vis;
+    bool any_vis, mask_hi, mask_lo = false;
     if (MODE == MODE_CMP) {
       any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
-      full_vis = (tw_lo >= p.stride * (kt + KT - 1) + p.kernel_size - 1) && (kt + KT <= nkeys);
+      mask_hi = tw_lo < p.stride * (kt + KT - 1) + p.kernel_size - 1 || kt + KT > nkeys;
     } else {
       any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
-      full_vis = (kt + KT - 1 <= tw_lo + khi) && (kt >= tw_hi + klo);
-      if (MODE == MODE_TAIL) full_vis = full_vis && tw_hi < t_end;
+      mask_hi = kt + KT - 1 > tw_lo + khi || (MODE == MODE_TAIL && tw_hi >= t_end);
+      mask_lo = kt < tw_hi + klo;
     }
     if (!any_vis) continue;
 
@@ -174,18 +176,23 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
     for (int nt = 0; nt < 2; nt++)
 #pragma unroll
       for (int i = 0; i < 16; i++) sacc[nt][i] = fast_exp2(__builtin_fmaf(sacc[nt][i], sc, -lsc));
-    if (!full_vis) {  // wave-uniform
+    // wave-uniform: a tile that straddles a visibility boundary compares each key's place in it with the row's bound (as the
+    // forward kernel does)
+    if (mask_hi) {
       asm volatile("");  // keeps it a branch: if-converted, every tile would pay
+      const int bound = key_hi - kt - hl * 4;
 #pragma unroll
       for (int nt = 0; nt < 2; nt++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          int key = kt + nt * 32 + (i >> 2) * 8 + hl * 4 + (i & 3);
-          bool vis;
-          if (MODE == MODE_CMP) vis = (key < nkeys) && (t >= p.stride * key + p.kernel_size - 1);
-          else vis = (key <= t + khi) && (key >= t + klo) && (MODE != MODE_TAIL || t < t_end);
-          sacc[nt][i] = vis ? sacc[nt][i] : 0.f;
-        }
+        for (int i = 0; i < 16; i++) sacc[nt][i] = nt * 32 + (i >> 2) * 8 + (i & 3) <= bound ? sacc[nt][i] : 0.f;
+    }
+    if (MODE != MODE_CMP && mask_lo) {
+      asm volatile("");
+      const int bound = key_lo - kt - hl * 4;
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) sacc[nt][i] = nt * 32 + (i >> 2) * 8 + (i & 3) >= bound ? sacc[nt][i] : 0.f;
     }
 #pragma unroll
     for (int nt = 0; nt < 2; nt++)
@@ -230,6 +237,8 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       klo = -0x40000000;
       khi = -p.window - 1;
       t_end = p.all_below;
+      key_lo = 0;
+      key_hi = t < t_end ? t + khi : -1;
       run_keys();
     }
   }

@@ -87,6 +87,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   bool valid[RS];
   int64_t tok[RS];
   int head[RS];
+  int key_hi[RS];  // MODE_CMP: the last key that the row sees
   bf16x8 qf[RS][D / 16];
 #pragma unroll
   for (int rs = 0; rs < RS; rs++) {
@@ -96,6 +97,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     int n = rr / G;
     int g = rr - n * G;
     t_row[rs] = n + qoff;
+    if (MODE == MODE_CMP) key_hi[rs] = t_row[rs] >= p.kernel_size - 1 ? min((t_row[rs] - p.kernel_size + 1) / p.stride, nkeys - 1) : -1;
     tok[rs] = x0 + n;
     head[rs] = kh * G + g;
     const bf16_t* qp = p.q + tok[rs] * p.q_st + (int64_t)head[rs] * p.q_sh + hl * 8;
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       else return lds_read_tr(Vs + row * VLD + col);
     }
   };
-  auto process = [&](bool masked, auto rs_tag, int kt, const bf16_t* Ks, const bf16_t* Vs) {
+  auto process = [&](bool mask_hi, bool mask_lo, auto rs_tag, int kt, const bf16_t* Ks, const bf16_t* Vs) {
     constexpr int rs = decltype(rs_tag)::value;
     // ---- S^T = K Q^T : two 32-key sub tiles, interleaved accumulators ----
     f32x16 sacc[2];
@@ -221,19 +223,27 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       sacc[1] = mfma32(k1, qf[rs][kc], sacc[1]);
     }
     // ---- mask, online softmax (running max in raw score units; scale folded into the exp2 fma) ----
-    if (masked) {  // wave-uniform: only tiles that straddle a visibility boundary pay for the mask
+    // Wave-uniform: only tiles that straddle a visibility boundary pay for its mask, which compares the key's place in the tile
+    // (a constant) with the row's bound: two instructions per score.  (Three terms per score in one test: four and two scalar
+    // ones, 64 more of a wave's 250 vector instructions per tile; short sequences mask two to four of their 2 to 12 tiles.)
+    if (mask_hi) {
       asm volatile("");  // keeps it a branch: if-converted, every tile would pay
-      const int t = t_row[rs];
+      const int bound = (MODE == MODE_CMP ? key_hi[rs] : MODE == MODE_TAIL && t_row[rs] >= t_end ? -0x40000000 : t_row[rs] + khi) -
+                        kt - hl * 4;
 #pragma unroll
       for (int nt = 0; nt < 2; nt++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          int key = kt + nt * 32 + (i >> 2) * 8 + hl * 4 + (i & 3);
-          bool vis;
-          if (MODE == MODE_CMP) vis = (key < nkeys) && (t >= p.stride * key + p.kernel_size - 1);
-          else vis = (key <= t + khi) && (key >= t + klo) && (MODE != MODE_TAIL || t < t_end);
-          sacc[nt][i] = vis ? sacc[nt][i] : NSA_NEG_INF;
-        }
+        for (int i = 0; i < 16; i++)
+          sacc[nt][i] = nt * 32 + (i >> 2) * 8 + (i & 3) <= bound ? sacc[nt][i] : NSA_NEG_INF;
+    }
+    if (MODE != MODE_CMP && mask_lo) {
+      asm volatile("");
+      const int bound = t_row[rs] + klo - kt - hl * 4;
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+          sacc[nt][i] = nt * 32 + (i >> 2) * 8 + (i & 3) >= bound ? sacc[nt][i] : NSA_NEG_INF;
     }
     float tmax = NSA_NEG_INF;
 #pragma unroll
@@ -373,18 +383,18 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       if (!wave_active) continue;
 
       // wave-uniform visibility classification of this tile
-      bool any_vis, full_vis;
+      bool any_vis, mask_hi, mask_lo = false;
       if (MODE == MODE_CMP) {
         any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
-        full_vis = (tw_lo >= p.stride * (kt + KT - 1) + p.kernel_size - 1) && (kt + KT <= nkeys);
+        mask_hi = tw_lo < p.stride * (kt + KT - 1) + p.kernel_size - 1 || kt + KT > nkeys;
       } else {
         any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
-        full_vis = (kt + KT - 1 <= tw_lo + khi) && (kt >= tw_hi + klo);
-        if (MODE == MODE_TAIL) full_vis = full_vis && tw_hi < t_end;
+        mask_hi = kt + KT - 1 > tw_lo + khi || (MODE == MODE_TAIL && tw_hi >= t_end);
+        mask_lo = kt < tw_hi + klo;
       }
       if (!any_vis) continue;
-      process(!full_vis, std::integral_constant<int, 0>{}, kt, Ks2[buf], Vs2[buf]);
-      if constexpr (RS > 1) process(!full_vis, std::integral_constant<int, RS - 1>{}, kt, Ks2[buf], Vs2[buf]);
+      process(mask_hi, mask_lo, std::integral_constant<int, 0>{}, kt, Ks2[buf], Vs2[buf]);
+      if constexpr (RS > 1) process(mask_hi, mask_lo, std::integral_constant<int, RS - 1>{}, kt, Ks2[buf], Vs2[buf]);
     }
   };
 
