@@ -21,8 +21,8 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
   constexpr int VLD = VD + NSA_LDS_PAD;
   __shared__ __attribute__((aligned(16))) bf16_t Ks[KT * KLD];
   __shared__ __attribute__((aligned(16))) bf16_t Vs[KT * VLD];
-  // with DO_LDS the dO fragments of a wave's 32 rows live in a wave-private LDS region instead of 32 registers,
-  // which brings the kernel under 256 registers (two workgroups per CU)
+  // with DO_LDS the dO fragments of a wave's 32 rows live in a wave-private LDS region instead of 32 registers (16 at 64
+  // channels), which brings the kernel under 256 registers (two workgroups per CU; three at 64 channels)
   __shared__ __attribute__((aligned(16))) bf16_t dOs[DO_LDS ? 4 * 32 * VLD : 8];
 
   const int tid = threadIdx.x;
@@ -278,8 +278,12 @@ int dispatch(const NsaBwdTileParams& p, int B, int max_q_len, int D, int VD, hip
   if (D == 128 && VD == 128) {
     if (minb == 2) bwd_dq_tile_kernel<128, 128, MODE, 2, true><<<grid, 256, 0, stream>>>(p);
     else bwd_dq_tile_kernel<128, 128, MODE, 1, false><<<grid, 256, 0, stream>>>(p);
-  } else if (D == 64 && VD == 64) bwd_dq_tile_kernel<64, 64, MODE, 2, false><<<grid, 256, 0, stream>>>(p);
-  else if (D == 192 && VD == 128) bwd_dq_tile_kernel<192, 128, MODE, 1, false><<<grid, 256, 0, stream>>>(p);
+  } else if (D == 64 && VD == 64) {
+    // dO fragments in LDS: three waves fit on a SIMD instead of two.  16 / 2 heads, whole steps, us: 40 samples of 17 to 1200 tokens
+    // 964 -> 950, of 500 to 1000 854 -> 822, 80 of up to 600 709 -> 693, one sequence of 16K 1579 -> 1564, 48K 5771 -> 5735.
+    // (Three waves with dO in registers spill 10 to 20 of them: 971 -> 1000.)
+    bwd_dq_tile_kernel<64, 64, MODE, 3, true><<<grid, 256, 0, stream>>>(p);
+  } else if (D == 192 && VD == 128) bwd_dq_tile_kernel<192, 128, MODE, 1, false><<<grid, 256, 0, stream>>>(p);
   else if (D == 256 && VD == 256) bwd_dq_tile_kernel<256, 256, MODE, 1, false><<<grid, 256, 0, stream>>>(p);
   else if (D == 32 && VD == 32) bwd_dq_tile_kernel<32, 32, MODE, 2, false><<<grid, 256, 0, stream>>>(p);
   else {
