@@ -24,7 +24,7 @@ typedef __attribute__((address_space(3))) void* nsa_lptr_t;
 // waves per workgroup: as many units in flight as LDS holds (18 KB per wave at 128 channels, 26 KB at 192)
 constexpr int dq_ds_waves(int d) { return d <= 128 ? 4 : 2; }
 
-template <int D, int DSH>
+template <int D, int DSH, bool STREAM>
 __global__ __launch_bounds__(dq_ds_waves(D) * 64) void slc_dq_ds_kernel(NsaSlcDqDsParams p) {
   constexpr int NW = dq_ds_waves(D);
   constexpr int UK = 32;
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(dq_ds_waves(D) * 64) void slc_dq_ds_kernel(NsaSlcDq
     const char* at = reinterpret_cast<const char*>(dbase + ((int64_t)(aux >> 6) * n_hc * upb + (aux & 63)) * (DSH * 32));
     uint32_t off = DSH == 8 ? (lane & 31) * 16 : lane * 16;  // (8 heads: the blob twice)
     asm volatile("" : "+s"(at), "+v"(off));
-    __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + off), (nsa_lptr_t)(buf + KEL), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + off), (nsa_lptr_t)(buf + KEL), 16, 0, STREAM ? 2 : 0);  // (2: non-temporal)
   };
 
   f32x4 dqacc[D / 16];
@@ -188,8 +188,17 @@ __global__ __launch_bounds__(dq_ds_waves(D) * 64) void slc_dq_ds_kernel(NsaSlcDq
 template <int D>
 int launch(const NsaSlcDqDsParams& p, hipStream_t stream) {
   const dim3 grid(cdiv_i(p.ntok, dq_ds_waves(D)), p.KH * (p.G > 16 ? p.G / 16 : 1));
-  if (p.G == 8) slc_dq_ds_kernel<D, 8><<<grid, dq_ds_waves(D) * 64, 0, stream>>>(p);
-  else slc_dq_ds_kernel<D, 16><<<grid, dq_ds_waves(D) * 64, 0, stream>>>(p);
+  // The dS is read once: where it is more than the 256 MB that the memory-side cache holds, so that all of it comes from memory
+  // anyhow, it is not to push K rows out of L2.  This kernel, us, kept / so: 64 heads of 128, 64K tokens 5500 / 5320, 8 x 6K tokens
+  // 2972 / 2947, 16 heads of 64, 16K tokens (0.5 GB) 348 / 324, 32 heads of 192, 16K tokens 860 / 850; 16 heads of 128, 4K tokens
+  // (0.13 GB) 51.3 / 53.9.
+  auto run = [&](auto stream_tag) {
+    constexpr bool S = decltype(stream_tag)::value;
+    if (p.G == 8) slc_dq_ds_kernel<D, 8, S><<<grid, dq_ds_waves(D) * 64, 0, stream>>>(p);
+    else slc_dq_ds_kernel<D, 16, S><<<grid, dq_ds_waves(D) * 64, 0, stream>>>(p);
+  };
+  if (p.ds_sh * p.KH * 2 > (int64_t)256 << 20) run(std::true_type{});
+  else run(std::false_type{});
   return nsa_check_launch("slc_dq_ds_kernel");
 }
 
