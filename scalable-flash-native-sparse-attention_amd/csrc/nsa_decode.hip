@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "nsa_select.h"
+#include "nsa_units.h"
 
 namespace {
 
@@ -71,7 +72,7 @@ NSA_DEVICE void sum_rows(float (&a)[8], const bf16_t* col, int64_t c_sr, const i
 // One wave's flash-attention state over units of 32 keys for the 16 heads of a kv group.
 // K and V rows of a unit are fetched as whole rows (16 lanes x 16 bytes per row: every cache line is requested once
 // and used completely), held in registers while the previous unit is computed, and pass through one wave-private
-// LDS slot: first the K rows (read back as MFMA A fragments), then the V rows (read back transposed).
+// LDS slot: first the K rows (read back as MFMA A fragments), then the V rows (read back transposed; VREG: these do not).
 // The un-normalised probabilities exp2((s - m_unit) * c) of every unit can be kept (in LDS, or spilled to scratch
 // memory, or both), together with the m_unit they refer to, so that the importance pass needs no second pass over the
 // keys: as fp16, or, with 192 channels, as fp32.
@@ -90,6 +91,15 @@ struct UnitFlash {
   static constexpr int KC = D / 32;
   static constexpr int KJ = (UK * (D / 8)) / 64;
   static constexpr int VJ = (UK * (VD / 8)) / 64;
+  // 128 v channels: V is transposed in the lanes' registers (UnitColumns128), the slot takes K alone, and a unit is a shorter
+  // chain.  Calls through the slot / so, us: one request of 32K tokens 31.7 / 30.1, 8 of up to 16K with 192 channels 39.7 / 38.9, 64 of
+  // 4K to 32K 73.9 / 73.2, 16 of 128K 106.8 / 106.5.  Not with four waves and two workgroups on a CU, which wait for memory: 512 of
+  // 4K 330.2 / 331.0.
+  static constexpr bool VREG = VD == 128 && STREAMS == 1;
+  typedef UnitColumns128 Cols;
+  // row of the unit and first channel that V register j of a lane holds
+  static NSA_DEVICE int v_row(int j, int lane) { return VREG ? Cols::row(j) + (lane >> 4) * 4 : (lane + j * 64) / (VD / 8); }
+  static NSA_DEVICE int v_chunk(int j, int lane) { return VREG ? lane & 15 : (lane + j * 64) % (VD / 8); }
   static constexpr int KLD = D + NSA_LDS_PAD;
   static constexpr int VLD = VD + NSA_LDS_PAD;
   static constexpr int SLOT = UK * (KLD > VLD ? KLD : VLD);  // bf16 elements of a wave's staging slot
@@ -165,13 +175,13 @@ struct UnitFlash {
           koff[g] = (uint32_t)((lane + g * 64) / KP) * (uint32_t)k_sr * 2u + (uint32_t)((lane + g * 64) % KP) * 16u;
 #pragma unroll
         for (int g = 0; g < VG; g++)
-          voff[g] = (uint32_t)((lane + g * 64) / VP) * (uint32_t)v_sr * 2u + (uint32_t)((lane + g * 64) % VP) * 16u;
+          voff[g] = (uint32_t)v_row(g, lane) * (uint32_t)v_sr * 2u + (uint32_t)v_chunk(g, lane) * 16u;
 #pragma unroll
         for (int j = 0; j < (K ? KJ : 0); j++)
           kf[j] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)(j / KG * KR) * k_sr * 2 + koff[j % KG]);
 #pragma unroll
         for (int j = 0; j < (V ? VJ : 0); j++)
-          vr[j] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)(j / VG * VR) * v_sr * 2 + voff[j % VG]);
+          vr[j] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)(VREG ? Cols::row(j) : j / VG * VR) * v_sr * 2 + voff[j % VG]);
         return;
       }
     }
@@ -186,10 +196,9 @@ struct UnitFlash {
     }
 #pragma unroll
     for (int j = 0; j < (V ? VJ : 0); j++) {
-      int pc = lane + j * 64;
-      int r = rem0 + max(klo, min(key0 + pc / (VD / 8), khi)) - ks;
+      int r = rem0 + max(klo, min(key0 + v_row(j, lane), khi)) - ks;
       int64_t row = (r >= page ? base1 : base0) + r;
-      vr[j] = ld_global_b128(vbase + row * v_sr + (pc % (VD / 8)) * 8);
+      vr[j] = ld_global_b128(vbase + row * v_sr + v_chunk(j, lane) * 8);
     }
   }
   // next_k / next_v run as soon as the K / V registers have gone to LDS (they may load the next unit into them)
@@ -222,15 +231,30 @@ struct UnitFlash {
     // the K fragments are consumed (LDS operations of a wave complete in order): the slot now takes the V rows
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    if (PATCH) {
 #pragma unroll
-    for (int j = 0; j < VJ; j++) {
-      int pc = lane + j * 64;
-      if (PATCH && (key0 + pc / (VD / 8) >= khi || klo >= khi)) vr[j] = zero_bf16x8();
-      *reinterpret_cast<bf16x8*>(&Ss[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
+      for (int j = 0; j < VJ; j++)
+        if (key0 + v_row(j, lane) >= khi || klo >= khi) vr[j] = zero_bf16x8();
+      if constexpr (VREG) {
+        const u32x4 x = __builtin_bit_cast(u32x4, patch);
+        u32x4 mine;
+#pragma unroll
+        for (int e = 0; e < 4; e++) mine[e] = __shfl(x[e], 32 + l16, 64);
+#pragma unroll
+        for (int j = 0; j < VJ; j++)
+          if (v_row(j, lane) == patch_row) vr[j] = __builtin_bit_cast(bf16x8, mine);
+      }
     }
-    if (PATCH && lane >= 32 && lane < 32 + VD / 8)
-      *reinterpret_cast<bf16x8*>(&Ss[patch_row * VLD + (lane - 32) * 8]) = patch;
-    next_v();
+    if constexpr (!VREG) {
+#pragma unroll
+      for (int j = 0; j < VJ; j++) {
+        int pc = lane + j * 64;
+        *reinterpret_cast<bf16x8*>(&Ss[(pc / (VD / 8)) * VLD + (pc % (VD / 8)) * 8]) = vr[j];
+      }
+      if (PATCH && lane >= 32 && lane < 32 + VD / 8)
+        *reinterpret_cast<bf16x8*>(&Ss[patch_row * VLD + (lane - 32) * 8]) = patch;
+      next_v();
+    }
     if (key0 < klo || key0 + UK - 1 > khi) {  // wave-uniform: only boundary units are masked
 #pragma unroll
       for (int jt = 0; jt < 2; jt++)
@@ -289,18 +313,26 @@ struct UnitFlash {
       for (int dt = 0; dt < VD / 16; dt++) oacc[dt] *= alpha;
     }
     l_run += psum;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     bf16x8 pf = pack8(sacc[0][0], sacc[0][1], sacc[0][2], sacc[0][3], sacc[1][0], sacc[1][1], sacc[1][2], sacc[1][3]);
-    const int kb0 = kq * 4 + (l16 >> 2);
-    const int kb1 = kb0 + 16;
+    if constexpr (VREG) {
+      Cols cols;
 #pragma unroll
-    for (int dt = 0; dt < VD / 16; dt++) {
-      const int col = dt * 16 + 4 * (l16 & 3);
-      bf16x4 v0 = lds_read_tr(&Ss[kb0 * VLD + col]);
-      bf16x4 v1 = lds_read_tr(&Ss[kb1 * VLD + col]);
-      oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
+      for (int j = 0; j < VJ; j++) cols.r[j] = vr[j];
+      cols.multiply(oacc, pf, std::make_integer_sequence<int, 8>{});
+      next_v();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int kb0 = kq * 4 + (l16 >> 2);
+      const int kb1 = kb0 + 16;
+#pragma unroll
+      for (int dt = 0; dt < VD / 16; dt++) {
+        const int col = dt * 16 + 4 * (l16 & 3);
+        bf16x4 v0 = lds_read_tr(&Ss[kb0 * VLD + col]);
+        bf16x4 v1 = lds_read_tr(&Ss[kb1 * VLD + col]);
+        oacc[dt] = mfma16(cat4(v0, v1), pf, oacc[dt]);
+      }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -381,9 +413,18 @@ struct UnitFlash {
     float l_tot = xrow_sum(l_run);
     l_tot = xhalf_sum(l_tot);
     if (kq == 0) { pm[l16] = m_run; pl[l16] = l_tot; }
+    if constexpr (VREG) {
 #pragma unroll
-    for (int dt = 0; dt < VD / 16; dt++)
-      *reinterpret_cast<f32x4*>(&po[l16 * OLD + dt * 16 + kq * 4]) = oacc[dt];
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          *reinterpret_cast<f32x4*>(&po[l16 * OLD + (kq * 4 + i) * 8 + h * 4]) =
+              f32x4{oacc[h * 4][i], oacc[h * 4 + 1][i], oacc[h * 4 + 2][i], oacc[h * 4 + 3][i]};
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < VD / 16; dt++)
+        *reinterpret_cast<f32x4*>(&po[l16 * OLD + dt * 16 + kq * 4]) = oacc[dt];
+    }
   }
 };
 
