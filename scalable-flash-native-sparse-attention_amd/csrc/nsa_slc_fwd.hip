@@ -8,7 +8,7 @@
 // key-contraction slices).  Keys are gathered by the per-token block list topk[kh, t, 0 .. min(top_n, t/block+1)).
 //
 // What bounds it is the gather: 512 KB of rows per token and kv head, from L2 while the keys of the sequences in flight
-// fit there (64 heads of 128, 8 x 6K tokens: the CU's address unit is busy 85 % of the cycles, LDS 66 %), else from the
+// fit there (64 heads of 128, 8 x 6K tokens: the CU's address unit is busy 96 % of the cycles, LDS 32 %), else from the
 // memory-side cache (64K tokens: 15.3 TB/s of requests, 6.4 of them past L2).  Two units in flight per wave and separate K and V
 // regions bought nothing over one, and took the registers and the LDS of a second workgroup per CU at 192 channels: 32 heads,
 // 16K tokens 1726 -> 1080 us; 64 heads of 128, 8 x 6K tokens 4207 -> 3920 us.  The rows lie unpadded and swizzled in LDS
