@@ -117,6 +117,7 @@ struct UnitRows {
 struct UnitColumns128 {
   static constexpr int N = 8, PAT = 1;
   static constexpr int64_t NARROW = UnitRows<128>::NARROW;
+  static_assert(12 * NARROW * 2 + 256 <= (int64_t)1 << 32, "a lane's offset: up to twelve rows and a piece");
   bf16x8 r[N];
 
   static constexpr int row(int j) { return (j >> 2) * 16 + (j & 3); }  // of the lanes with kq 0
