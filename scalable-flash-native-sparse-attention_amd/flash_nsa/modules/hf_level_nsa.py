@@ -6,13 +6,12 @@ import torch
 from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
 from ..ops.compress_kv import construct_block, mean_pooling
-from ..ops.compress_attn import cmp_attn_fwd, compress_attn
+from ..ops.compress_attn import compress_attn
 from ..ops.select_attn import select_attn
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_impl, sigmoid_mul_impl
 from ..ops.combine import fused_sigmoid_combine
 from ..ops.sliding_window_attention import swa_varlen_func
-from .megatron_level_nsa import slc_swa_fwd
 
 _METHODS = ("mean", "sigmoid-mul", "swiglu", "linear")
 
@@ -44,23 +43,6 @@ class CompressKV(torch.nn.Module):
         return swiglu_impl(hidden)
 
 
-class _GatedAttention(torch.autograd.Function):
-    """The three branches and their gated sum where nothing is kept for a backward: the window kernel forms the sum, and the
-    selected branch of the first queries, which select all that they see, is the window's, continued.  32 / 2 heads of
-    192 / 128, 16K tokens: 1640 -> 1600 us, by three outputs that are written and read once less and the gather of those
-    queries.  (An autograd function of its own, so that transforms that the single stages refuse stay refused.)"""
-
-    @staticmethod
-    def forward(ctx, q, k, v, cmp_k, cmp_v, w, sm_scale):
-        cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
-        topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=NSAHelper.all_below())
-        return slc_swa_fwd(q, k, v, topk, sm_scale, NSAHelper, cmp_o, w, store=False)[2]
-
-    @staticmethod
-    def backward(ctx, do):
-        raise RuntimeError("this forward pass has kept nothing for a backward")
-
-
 class HFNSACore(torch.nn.Module):
     def __init__(self, config: NSAConfig):
         super().__init__()
@@ -86,12 +68,6 @@ class HFNSACore(torch.nn.Module):
                                       window_size=self.window_size, top_n=self.top_n,
                                       num_init_blocks=self.num_init_blocks, num_local_blocks=self.num_local_blocks)
 
-    def _selection_sizes_ok(self):
-        # the block selector's own conditions: batches of short sequences don't reach it in _GatedAttention, so that sizes which
-        # it refuses go to the single stages, which ask it for every batch
-        init, local = self.num_init_blocks, self.num_local_blocks
-        return 1 <= self.top_n <= 64 and init >= 0 and local >= 0 and init + local <= self.top_n
-
     def forward(self, q, k, v, combine_weight, cu_seqlens, bench: bool = False, print_result: bool = True):
         """q [T,QH,Dqk], k [T,KH,Dqk], v [T,KH,Dv], combine_weight [T,QH,3], cu_seqlens int32 [B+1] -> o [T,QH,Dv].
         With bench=True also returns a pandas Series of per-stage forward milliseconds."""
@@ -108,8 +84,6 @@ class HFNSACore(torch.nn.Module):
 
         cmp_k = run("cmp_k", lambda: self.compress_k(k))
         cmp_v = run("cmp_v", lambda: self.compress_v(v))
-        if not bench and not torch.is_grad_enabled() and self._selection_sizes_ok():
-            return _GatedAttention.apply(q, k, v, cmp_k, cmp_v, combine_weight, self.sm_scale)
         cmp_o, cmp_lse = run("cmp_o", lambda: compress_attn(q, cmp_k, cmp_v, sm_scale=self.sm_scale))
         topk, _ = run("top_k", lambda: slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=self.sm_scale))
         slc_o = run("slc_o", lambda: select_attn(q, k, v, topk, sm_scale=self.sm_scale))

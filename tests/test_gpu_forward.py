@@ -300,19 +300,20 @@ def test_192_channels_staged_straight_into_lds(device, QH, KH, lens):
     (8, 2, 192, 128, [300, 33]),                      # no query has blocks to choose from
 ])
 def test_staged_core_without_gradients_is_the_staged_core(device, QH, KH, D, VD, lens):
-    """Without gradients one function forms the gated sum (the window kernel, over the selected branch of the later queries
-    alone); with gradients every stage is a node of its own.  Sizes that the selector refuses are refused either way."""
+    """Evaluation gives the training forward's output, bit for bit (a reentrant activation checkpoint runs its first pass
+    without gradients and its second with them).  Sizes that the selector refuses are refused either way."""
     from flash_nsa import HFNSACore, NSAConfig
     cu = make_cu(lens).to(device)
-    args = [t.to(device) for t in make_qkvw(sum(lens), QH, KH, D, VD, seed=72)]
+    q, k, v, w = [t.to(device) for t in make_qkvw(sum(lens), QH, KH, D, VD, seed=72)]
     kw = dict(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH, top_n=8, window_size=128)
     core = HFNSACore(NSAConfig(**kw))
-    want = core(*args, cu)
+    want = core(q.clone().requires_grad_(), k, v, w, cu)
     with torch.no_grad():
-        assert_close(core(*args, cu), want.detach(), "o")
+        got = core(q, k, v, w, cu)
+        assert want.requires_grad and not got.requires_grad and torch.equal(got, want)
         core.num_local_blocks = 8  # with the initial block more than top_n
         with pytest.raises(RuntimeError):
-            core(*args, cu)
+            core(q, k, v, w, cu)
 
 
 @pytest.mark.parametrize("G,D,edge", [(16, 128, 12288), (5, 128, 12288), (16, 192, 16384)])
