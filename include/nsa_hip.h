@@ -351,7 +351,10 @@ int64_t nsa_swa_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int win
 int64_t nsa_slc_bwd_before_window_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int window, int all_below, int ring);
 /* nsa_cmp_attn_bwd_dkdv that stores dS.  Without workspace dck / dcv are added into with fp32 atomics; with
  * nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(...) bytes of it the work items' sums are added in a fixed order and stored (add: added
- * to what the ranges before have left). */
+ * to what the ranges before have left).  nsa_cmp_attn_bwd_dkdv_ds_items: work items of the launch per sequence and kv head,
+ * with q_chunk_tokens query tokens in one (0: as many as the launch takes); one slot each. */
+int64_t nsa_cmp_attn_bwd_dkdv_ds_items(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD, int kernel_size,
+                                       int stride, int q_chunk_tokens, int tok0, int tok1);
 int64_t nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
                                             int kernel_size, int stride, int tok0, int tok1);
 int nsa_cmp_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,

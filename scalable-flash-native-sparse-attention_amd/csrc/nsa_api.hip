@@ -1091,14 +1091,27 @@ int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int ke
   return T - lo < least ? T : lo;
 }
 
-int64_t nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
-                                            int kernel_size, int stride, int tok0, int tok1) {
-  if (B <= 0 || x_maxlen <= 0 || y_maxlen <= 0 || KH <= 0 || QH < KH || stride <= 0) return 0;
+// query tokens per work item of a range's launch (one sequence: of its share; of several, one may have any share)
+static int cmp_ds_q_chunk(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD, int kernel_size, int stride,
+                          int tok0, int tok1) {
   int lo, hi;
   nsa_local_range(tok0, tok1, 0, x_maxlen, lo, hi);
   if (B > 1) { lo = 0; hi = x_maxlen; }
-  const int chunk = cmp_dkdv_q_chunk(0, B, hi, y_maxlen, QH, KH, D, VD, kernel_size, stride, lo);
-  const int64_t slots = nsa_bwd_dkdv_cmp_slots(B, KH, x_maxlen, y_maxlen, D, chunk, kernel_size, stride, tok0, tok1, B);
+  return cmp_dkdv_q_chunk(0, B, hi, y_maxlen, QH, KH, D, VD, kernel_size, stride, lo);
+}
+
+int64_t nsa_cmp_attn_bwd_dkdv_ds_items(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD, int kernel_size,
+                                       int stride, int q_chunk_tokens, int tok0, int tok1) {
+  if (B <= 0 || x_maxlen <= 0 || y_maxlen <= 0 || KH <= 0 || QH < KH || stride <= 0) return 0;
+  if (q_chunk_tokens <= 0)
+    q_chunk_tokens = cmp_ds_q_chunk(B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride, tok0, tok1);
+  return nsa_bwd_dkdv_cmp_slots(1, 1, x_maxlen, y_maxlen, D, q_chunk_tokens, kernel_size, stride, tok0, tok1, B);
+}
+
+int64_t nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(int B, int x_maxlen, int y_maxlen, int QH, int KH, int D, int VD,
+                                            int kernel_size, int stride, int tok0, int tok1) {
+  const int64_t slots = B * (int64_t)KH *
+                        nsa_cmp_attn_bwd_dkdv_ds_items(B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride, 0, tok0, tok1);
   const int64_t kw = nsa_bwd_dkdv_slot_keys(0, 0, D);
   return ((slots * kw * D * 4 + 255) & ~(int64_t)255) + slots * kw * VD * 4;
 }
@@ -1128,10 +1141,7 @@ int nsa_cmp_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const vo
   p.x_cu = x_cu; p.k_cu = y_cu;
   p.kernel_size = kernel_size; p.stride = stride;
   set_ds(p, l, ds, tok0, tok1);
-  int lo, hi;
-  nsa_local_range(tok0, tok1, 0, x_maxlen, lo, hi);
-  if (B > 1) { lo = 0; hi = x_maxlen; }
-  p.q_chunk_tokens = cmp_dkdv_q_chunk(0, B, hi, y_maxlen, QH, KH, D, VD, kernel_size, stride, lo);
+  p.q_chunk_tokens = cmp_ds_q_chunk(B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride, tok0, tok1);
   if (workspace == nullptr) return nsa_bwd_dkdv_launch(p, 0, B, x_maxlen, y_maxlen, D, VD, 0, (hipStream_t)stream);
   const int64_t need = nsa_cmp_attn_bwd_dkdv_ds_slot_bytes(B, x_maxlen, y_maxlen, QH, KH, D, VD, kernel_size, stride, tok0, tok1);
   NSA_REQUIRE(workspace_bytes >= need, NSA_ERR_WORKSPACE, "cmp_attn_bwd_dkdv_ds: workspace of %lld bytes, %lld needed",

@@ -648,15 +648,22 @@ int launch(const NsaBwdTileParams& p0, int mode, int B, int max_q_len, int max_k
 int64_t nsa_bwd_dkdv_cmp_slots(int B, int KH, int max_q_len, int max_k_len, int D, int q_chunk_tokens,
                                int kernel_size, int stride, int tok0, int tok1, int n_seq) {
   const int KW = nsa_bwd_dkdv_slot_keys(0, 0, D);
-  // the share of the longest sequence; of several sequences that a range meets, one may have any share of that length
+  int64_t total = 0;
+  if (tok1 > 0 && n_seq > 1) {
+    // A range's share of a sequence may begin and end anywhere in it, and its chunks are cut from its first row on.  A key tile
+    // meets at most all chunks of the longest share, and at most one more than the rows behind the tile's first one fill.
+    const int share = max_q_len < tok1 - tok0 + 127 ? max_q_len : tok1 - tok0 + 127;
+    for (int64_t kt = 0; kt * KW < max_k_len; kt++) {
+      const int64_t seeing = max_q_len - (stride * kt * KW + kernel_size - 1);  // rows that see the tile, of the longest sequence
+      if (seeing <= 0) break;
+      const int64_t n = (seeing + q_chunk_tokens - 1) / q_chunk_tokens + 1, all = cdiv_i(share, q_chunk_tokens);
+      total += n < all ? n : all;
+    }
+    return total * B * KH;
+  }
   int lo, hi;
   nsa_local_range(tok0, tok1, 0, max_q_len, lo, hi);
-  if (tok1 > 0 && n_seq > 1) {
-    lo = max_q_len - (max_q_len < tok1 - tok0 + 127 ? max_q_len : tok1 - tok0 + 127);
-    hi = max_q_len;
-  }
   const int nch = hi > lo ? cdiv_i(hi - lo, q_chunk_tokens) : 0;
-  int64_t total = 0;
   for (int64_t kt = 0; kt * KW < max_k_len; kt++) {
     const int64_t first = stride * kt * KW + kernel_size - 1 - lo;
     const int64_t fc = first > 0 ? first / q_chunk_tokens : 0;

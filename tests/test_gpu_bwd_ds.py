@@ -16,19 +16,21 @@ def _grads(core, ts, cu, do, device):
 
 
 # ends of tiles of 64 rows (8 .. 1 tokens), of units of 32 keys, of groups of 128 positions, and sequences without a
-# compressed row; ranged: a scratch limit of 1 MB, so that the ranges have the fewest tokens that they may have
+# compressed row; ranged: a scratch limit in MB, 1: the ranges have the fewest tokens that they may have
 CASES = [
     # QH, KH, D, VD, lens, ranged, settings
-    (8, 1, 128, 128, [1, 31, 32, 33, 700], False, {}),
-    (16, 1, 128, 128, [1024, 1025, 47, 1279], False, dict(top_n=4)),
-    (32, 1, 128, 128, [0, 515, 0, 640], False, dict(window_size=100, top_n=3)),
-    (64, 1, 128, 128, [513, 1, 129], False, dict(window_size=0, top_n=3)),
-    (64, 4, 128, 128, [4700], True, {}),
-    (64, 1, 128, 128, [2047, 300, 2500, 5], True, dict(top_n=6)),
-    (64, 4, 192, 128, [130, 4300], True, dict(window_size=300)),
-    (32, 2, 192, 128, [900, 64, 333], False, dict(block_size=96, kernel_size=64, stride=32, top_n=5)),
-    (16, 2, 128, 128, [1500, 200], False, dict(window_size=2000)),
-    (16, 1, 192, 128, [777], False, dict(kernel_size=16, stride=8, block_size=32, top_n=40)),
+    (8, 1, 128, 128, [1, 31, 32, 33, 700], 0, {}),
+    (16, 1, 128, 128, [1024, 1025, 47, 1279], 0, dict(top_n=4)),
+    (32, 1, 128, 128, [0, 515, 0, 640], 0, dict(window_size=100, top_n=3)),
+    (64, 1, 128, 128, [513, 1, 129], 0, dict(window_size=0, top_n=3)),
+    (64, 4, 128, 128, [4700], 1, {}),
+    (64, 1, 128, 128, [2047, 300, 2500, 5], 1, dict(top_n=6)),
+    (64, 4, 192, 128, [130, 4300], 1, dict(window_size=300)),
+    (32, 2, 192, 128, [900, 64, 333], 0, dict(block_size=96, kernel_size=64, stride=32, top_n=5)),
+    (16, 2, 128, 128, [1500, 200], 0, dict(window_size=2000)),
+    (16, 1, 192, 128, [777], 0, dict(kernel_size=16, stride=8, block_size=32, top_n=40)),
+    # chunks of 256 queries, cut from the first row of a share in the middle of a sequence
+    (32, 2, 128, 128, [3063, 9859], 64, {}),
 ]
 
 
@@ -46,7 +48,7 @@ def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ra
     made, init = [], bwd_ds.DenseDs.__init__
     bwd_ds.DenseDs.__init__ = lambda self, *a, **k: (init(self, *a, **k), made.append(self))[0]
     if ranged:
-        _lib.call("nsa_set_tuning", b"dense_ds_mb", 1)
+        _lib.call("nsa_set_tuning", b"dense_ds_mb", ranged)
     try:
         got = _grads(core, ts, cu, do, device)
         H.set_deterministic(True)
@@ -55,7 +57,7 @@ def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ra
         H.set_deterministic(False)
         _lib.call("nsa_reset_tuning")
         bwd_ds.DenseDs.__init__ = init
-    assert len(made) == 1 and (len(made[0].ranges) > 1) == ranged
+    assert len(made) == 1 and (len(made[0].ranges) > 1) == (ranged > 0)
     assert torch.equal(got[0], want[0])
     # the same products of bf16 operands whose last bit may differ (P from differently rounded exponents): the bar that both
     # are held to against the oracle

@@ -304,3 +304,43 @@ def test_ranges_of_stored_ds_cover_the_batch():
             _lib.value("nsa_swa_bwd_ds_bytes", T, B, longest, QH, KH, 512, 0)
     # no scratch where no query has keys before its window
     assert _lib.value("nsa_slc_bwd_before_window_ds_bytes", 5000, 1, 5000, 64, 4, 2000, 1024, 0) == 0
+
+
+def test_grid_of_the_storing_dkdv_covers_every_share_of_a_range():
+    """The compressed dk / dv launch that stores dS has one grid for all sequences of a range, in which each of them numbers
+    its work items (key tile of 128, chunk of queries that sees it) from its own first row on."""
+    import random
+    from flash_nsa import _lib
+    QH, KH, D, VD, W = 64, 4, 128, 128, 512
+    rng = random.Random(5)
+    batches = [([20480] * 2, 32, 16), ([45056] * 2, 32, 16), ([12288] * 10, 32, 16), ([65000], 32, 16), ([700] * 3, 32, 16)]
+    for _ in range(60):
+        longest = int(2 ** rng.uniform(9, 16))
+        batches.append(([rng.randint(1, longest) for _ in range(rng.randint(1, 12))], *rng.choice(((32, 16), (64, 32), (16, 8)))))
+    tight = 0
+    for lens, kernel_size, stride in batches:
+        T, B, longest = sum(lens), len(lens), max(lens)
+        y = [max((n - kernel_size) // stride + 1, 0) for n in lens]
+        cuts, at = [], 0
+        while at < T:
+            end = _lib.value("nsa_bwd_ds_next", at, T, B, longest, QH, KH, kernel_size, stride, W)
+            cuts.append((at, end))
+            at = end
+        for a in range(0, T, max(T // 3 // 128, 1) * 128):  # and others than the library's
+            cuts.append((a, min(a + rng.randint(1, 200) * 128, T)))
+        for tok0, tok1 in ([(0, 0)] if len(cuts) == 1 else cuts):
+            for chunk in (32, 64, 128, 256, 512, 1024, 2048):
+                have = _lib.value("nsa_cmp_attn_bwd_dkdv_ds_items", B, longest, max(y), QH, KH, D, VD, kernel_size, stride,
+                                  chunk, tok0, tok1)
+                x0 = 0
+                for n, keys in zip(lens, y):
+                    lo, hi = 0, n
+                    if tok1:
+                        lo, hi = max(-(-(tok0 - x0) // 128) * 128, 0), min(-(-(tok1 - x0) // 128) * 128, n)
+                    chunks, need = -(-max(hi - lo, 0) // chunk), 0
+                    for first in range(kernel_size - 1, min(hi, kernel_size - 1 + stride * keys), stride * 128):
+                        need += chunks - min(chunks, max(first - lo, 0) // chunk)
+                    assert need <= have, (lens, (tok0, tok1), chunk, need, have)
+                    tight += need == have > 0
+                    x0 += n
+    assert tight > 100
