@@ -40,6 +40,9 @@ NSA_DEVICE const char* scalar_ptr(const void* x) {
   return reinterpret_cast<const char*>(((uint64_t)h << 32) | l);
 }
 
+// The widest row stride of ASYNC: a lane's offset inside a period of its loads (up to 32 rows, 64 of 32 channels) has 32 bits.
+constexpr int64_t async_row_stride(int D, int VD) { return D >= 64 && VD >= 64 ? 1 << 26 : 1 << 25; }
+
 // ASYNC: the K/V tiles go from global memory straight into LDS (global_load_lds, 16 bytes per lane, no staging
 // registers, no ds_write); the tiles are then unpadded and swizzled instead of padded.
 template <int D, int VD, int MODE, bool PAGED, int RS, int MINB, bool ASYNC>
@@ -310,6 +313,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   constexpr int KPAT = 256 % KP == 0 ? 1 : 3, VPAT = 256 % VP == 0 ? 1 : 3;
   constexpr int KROWS = KPAT * 256 / KP, VROWS = VPAT * 256 / VP;
   static_assert(!ASYNC || (KROWS % 16 == 0 && VROWS % 16 == 0 && KJ % KPAT == 0 && VJ % VPAT == 0), "period of the swizzles");
+  static_assert(!ASYNC || ((KROWS > VROWS ? KROWS : VROWS) - 1) * async_row_stride(D, VD) * 2 + 512 < (int64_t)1 << 32, "a lane's offset");
   uint32_t goffk[KPAT], goffv[VPAT];
   if constexpr (ASYNC) {
 #pragma unroll
@@ -571,7 +575,8 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   // queries behind up to 8K 1352 / 1118.  1..4 force one variant for experiments.
   const int variant = nsa_tuning_knob("fwd_variant", 0);
   constexpr bool pow2 = (D == 64 || D == 128) && (VD == 64 || VD == 128);
-  const bool async = variant == 4 || (variant == 0 && ((MODE == MODE_CMP && pow2) || D == 192));
+  const bool narrow = p.k_sr >= 0 && p.v_sr >= 0 && p.k_sr <= async_row_stride(D, VD) && p.v_sr <= async_row_stride(D, VD);
+  const bool async = narrow && (variant == 4 || (variant == 0 && ((MODE == MODE_CMP && pow2) || D == 192)));
   if constexpr (D > 192 || VD > 128) {
     // head dims of 256: the output accumulators alone take 128 registers, one workgroup per CU
     dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
@@ -580,7 +585,7 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   } else if constexpr (MODE == MODE_TAIL) {
     dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     if constexpr (D == 192) {
-      if (variant != 1) {
+      if (variant != 1 && narrow) {
         fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, true><<<grid, 256, 0, stream>>>(p);
         return nsa_check_launch("fwd_tile_kernel");
       }

@@ -340,3 +340,26 @@ def test_selected_branch_either_side_of_the_length_that_v_stays_in_registers_for
     assert_close(o[first:], want, "slc_o")
     assert_close(lse[first:], s.logsumexp(-1) / math.log(2.0), "slc_lse", atol=1e-3, rtol=1e-4)
     setup_helper(make_cu([64]).to(device))
+
+
+@pytest.mark.parametrize("D", [128, 192])
+def test_row_strides_that_a_32_bit_offset_does_not_hold(device, D):
+    """K and V rows 302 MB apart (15 of them are more than 4 GB), full tiles of 64 and a partial one: the same bits as
+    contiguous rows."""
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd
+    from flash_nsa.ops.sliding_window_attention import swa_fwd
+    sr, n, G = (1 << 27) + (1 << 24), 74, 8
+    for fwd, T in ((swa_fwd, n), (cmp_attn_fwd, 16 * (n - 1) + 32)):
+        setup_helper(make_cu([T]).to(device))
+        q = randn_bf16(T, G, D, seed=90).to(device)
+        k, v = randn_bf16(n, 1, D, seed=91).to(device), randn_bf16(n, 1, 128, seed=92).to(device)
+        want = fwd(q, k, v)
+        wide = []
+        for t in (k, v):
+            wide.append(torch.empty((n - 1) * sr + 192, dtype=torch.bfloat16, device=device).as_strided(t.shape, (sr, 192, 1)))
+            wide[-1].copy_(t)
+        got = fwd(q, *wide)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        del wide
+    torch.cuda.empty_cache()
+    setup_helper(make_cu([64]).to(device))
