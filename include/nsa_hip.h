@@ -339,11 +339,16 @@ int nsa_slc_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
  * launch forms dQ = dS K of the compressed branch, the window and the keys before the window (of the queries below all_below)
  * together.  The batch (T rows) is processed in ranges of tokens [tok0, tok1) in ascending order (tok1 = 0: all of it in one;
  * otherwise the range of 128-position groups of a sequence whose first token it holds), so that the scratch stays bounded:
- * nsa_bwd_ds_next gives the end of the range that begins at tok0 (T: the last one).
+ * nsa_bwd_ds_range_end gives the end of the range that begins at tok0 (T: the last one), in which no branch takes more than
+ * 4 GB (stride 0: without the compressed branch, window -1: without the window), or -1 where a range that fills the GPU would:
+ * such batches have dq computed apart.  nsa_bwd_ds_next: the same ranges of the compressed branch and the window alone, at least
+ * as long as fills the GPU, whatever they take.
  * nsa_bwd_ds_takes: 1 where these shapes, strides and scale have this path.  nsa_*_ds_bytes: scratch of a branch; `ring` is
  * the length of the longest range (0: one range).  The window's scratch holds what the next range needs: the same buffer is
  * passed for all ranges, and a range's dk / dv kernels run after the dq launch of the range before. */
 int nsa_bwd_ds_takes(int64_t q_sh, int64_t do_sh, int64_t k_sr, int QH, int KH, int D, int VD, float sm_scale);
+int nsa_bwd_ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
+                         int all_below);
 int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window);
 int64_t nsa_cmp_attn_bwd_ds_bytes(int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int tok0,
                                   int tok1);

@@ -34,7 +34,7 @@ Knob g_knobs[] = {
     {"decode_waves", {0}, {false}},     // waves per workgroup of the one-launch decode kernel (0: from the batch; 4, 8)
     {"swa_dkdv_splits", {0}, {false}},  // query chunks per key tile of the window dk/dv kernel (0: from the sizes)
     {"slc_ds_mb", {0}, {false}},        // scratch for the dS of the selected branch, MB (0: dq and dk/dv computed apart)
-    {"dense_ds_mb", {0}, {false}},      // scratch for the dS of the compressed branch, and for the window's, MB
+    {"dense_ds_mb", {0}, {false}},      // scratch for the dS of the compressed branch, the window's, the keys' before it, MB each
     {"topk_two_pass", {0}, {false}},    // 0: the one-launch selector even when a workspace is given
 };
 Knob* find_knob(const char* name) {
@@ -1066,21 +1066,29 @@ int64_t nsa_slc_bwd_before_window_ds_bytes(int T, int B, int x_maxlen, int QH, i
   return ds_layout_far(T, B, x_maxlen, QH / KH, KH, window, all_below, ring).bytes;
 }
 
-// End of the range of tokens that begins at tok0: 4 GB for the compressed branch's dS, and the window's, but never fewer tokens
-// than give the dQ kernel 512 workgroups of 256 rows, and no shorter rest.  Whole step with 2 / 4 / 8 / 40 GB, 64 heads of 128,
-// ms: 64K tokens 52.7 / 52.2 / 51.8 / 52.2, 8 x 6K 19.9 / 19.2 / 19.2 / 19.2.  (As for the selected branch no rule on the number
-// of tokens decides whether dq comes from stored dS: a query's dq is to be the same bits whatever follows it in the batch.)
-int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window) {
-  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || stride <= 0 || tok0 >= T) return T;
+// End of the range of tokens that begins at tok0: 4 GB for each branch's dS (stride 0: without the compressed branch, window -1:
+// without the window, all_below 0: without the keys before it), but never fewer tokens than give the dQ kernel 512 workgroups of
+// 256 rows, and no shorter rest; *fit: whether that holds the 4 GB.  Whole step with 2 / 4 / 8 / 40 GB, 64 heads of 128, ms: 64K
+// tokens 52.7 / 52.2 / 51.8 / 52.2, 8 x 6K 19.9 / 19.2 / 19.2 / 19.2.  (As for the selected branch no rule on the number of tokens
+// decides whether dq comes from stored dS: a query's dq is to be the same bits whatever follows it in the batch.  The exceptions
+// are what even the least range does not hold, and batches beside it: sequences past a quarter of a million tokens, and, where
+// top_n * block_size is far beyond the window, of more than so many keys before it.)
+static int ds_least(int QH) { return (131072 / QH + 127) & ~127; }
+static int ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
+                        int all_below, bool* fit) {
   const int G = QH / KH;
   const int64_t budget = (int64_t)nsa_tuning_knob("dense_ds_mb", 4096) << 20;
   auto fits = [&](int tok1) {
-    return ds_layout_cmp(T, B, x_maxlen, G, KH, kernel_size, stride, tok0, tok1).bytes <= budget &&
-           ds_layout_win(T, B, x_maxlen, G, KH, window, tok1 - tok0).bytes <= budget;
+    if (stride > 0 && ds_layout_cmp(T, B, x_maxlen, G, KH, kernel_size, stride, tok0, tok1).bytes > budget) return false;
+    if (window < 0) return true;
+    return ds_layout_win(T, B, x_maxlen, G, KH, window, tok1 - tok0).bytes <= budget &&
+           ds_layout_far(T, B, x_maxlen, G, KH, window, all_below, tok1 - tok0).bytes <= budget;
   };
+  *fit = true;
   if (fits(T)) return T;
-  const int least = (131072 / QH + 127) & ~127;
+  const int least = ds_least(QH);
   int lo = tok0 + least;
+  *fit = lo < T && fits(lo);
   if (lo >= T) return T;
   int hi = T;  // fits(lo) or lo is the least; !fits(hi)
   while (hi - lo > 128) {
@@ -1088,7 +1096,25 @@ int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int ke
     if (mid >= hi) break;
     if (fits(mid)) lo = mid; else hi = mid;
   }
-  return T - lo < least ? T : lo;
+  if (T - lo >= least) return lo;
+  if (!*fit) return T;
+  const int half = ((T - tok0) / 2 + 127) & ~127;
+  return T - tok0 - half >= least ? tok0 + half : lo;
+}
+
+int nsa_bwd_ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
+                         int all_below) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || tok0 < 0 || tok0 >= T) return T;
+  bool fit;
+  const int end = ds_range_end(tok0, T, B, x_maxlen, QH, KH, kernel_size, stride, window, all_below, &fit);
+  return fit ? end : -1;
+}
+
+int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window) {
+  if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || stride <= 0 || tok0 >= T) return T;
+  bool fit;
+  const int end = ds_range_end(tok0, T, B, x_maxlen, QH, KH, kernel_size, stride, window, 0, &fit);
+  return T - end < ds_least(QH) ? T : end;
 }
 
 // query tokens per work item of a range's launch (one sequence: of its share; of several, one may have any share)

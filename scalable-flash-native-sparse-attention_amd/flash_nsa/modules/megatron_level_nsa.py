@@ -101,16 +101,15 @@ def slc_swa_fwd(q, k, v, topk, sm_scale, helper, cmp_o=None, w=None, store=True)
     return (slc_o, slc_lse), (swa_o, swa_lse), out
 
 
-def bwd_from_ds(q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa, delta, ds_tokens, sm_scale, helper):
+def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa, delta, ds_tokens, sm_scale, helper):
     """The backward of the three branches where all of them leave their dS behind -> dq, dk, dv, dcmp_k, dcmp_v.
-    ds_tokens: slc_bwd_ds_tokens; 0: every query selects all blocks it sees."""
+    ds: the scratch of the dense branches; ds_tokens: slc_bwd_ds_tokens; 0: every query selects all blocks it sees."""
     all_below = helper.all_below()
     dq = torch.empty_like(q)
     dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32) if ds_tokens else None
     # the window branch writes every element of dk / dv, the selected branch then adds to them
     dk = torch.empty(k.shape, device=q.device, dtype=torch.float32)
     dv = torch.empty(v.shape, device=q.device, dtype=torch.float32)
-    ds = bwd_ds.DenseDs(q, k, helper, all_below=all_below)
 
     def dkdv_cmp(r, *sums):
         return ds.dkdv_cmp(r, q, cmp_k, cmp_v, cmp_lse, dcmp_o, delta[0], sm_scale, *sums)
@@ -151,6 +150,7 @@ def bwd_from_ds(q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_s
             dkdv_raw(r)
             dense_dq(r)
         dcmp_k, dcmp_v = sums
+        ds.release()  # (in stream order, before the selected branch takes its own)
         selected()
     return dq, dk, dv, dcmp_k, dcmp_v
 
@@ -215,11 +215,13 @@ class NSAFunction(torch.autograd.Function):
         stored_ds = ds_tokens > 0
         if (stored_ds or helper.x_maxlen <= all_below) and bwd_ds.takes(q, k, v, do, sm_scale, helper) and \
                 bwd_ds.takes(q, cmp_k, cmp_v, dcmp_o, sm_scale, helper):
-            dq, dk, dv, dcmp_k, dcmp_v = bwd_from_ds(q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa, delta,
-                                                     ds_tokens, sm_scale, helper)
-            _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
-            _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
-            return dq, dk, dv, dw, dwk, dwv, None, None
+            ds = bwd_ds.DenseDs(q, k, helper, all_below=all_below)
+            if ds.fits:
+                dq, dk, dv, dcmp_k, dcmp_v = bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa,
+                                                         delta, ds_tokens, sm_scale, helper)
+                _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+                _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+                return dq, dk, dv, dw, dwk, dwv, None, None
 
         # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
         # branches' and writes q's dtype (the compressed branch does for the queries that the gather leaves out).  Else it

@@ -22,8 +22,8 @@ def _st(t):
 
 class DenseDs:
     """The scratch of one backward of the compressed branch (with_cmp), the window (with_swa) and, with all_below > 0, the keys
-    before the window of the queries below it; `ranges` are the (tok0, tok1) that dkdv_cmp, dkdv_swa and dq are called for, in
-    this order."""
+    before the window of the queries below it, up to 4 GB each; `ranges` are the (tok0, tok1) that dkdv_cmp, dkdv_swa and dq are
+    called for, in this order.  `fits`: whether there are such ranges (else dq and dk / dv are to be computed apart)."""
 
     def __init__(self, q, k, helper=NSAHelper, with_cmp=True, with_swa=True, all_below=0):
         T, QH, D = q.shape
@@ -31,9 +31,13 @@ class DenseDs:
         self.all_below = all_below
         sizes = (T, helper.batch, helper.x_maxlen, QH, self.KH)
         cmp_sizes = (helper.kernel_size, helper.stride)
-        cuts, at = [], 0
+        branches = (*(cmp_sizes if with_cmp else (0, 0)), helper.window_size if with_swa else -1, all_below)
+        cuts, at, self.fits = [], 0, True
         while at < T:
-            end = _lib.value("nsa_bwd_ds_next", at, *sizes, *cmp_sizes, helper.window_size)
+            end = _lib.value("nsa_bwd_ds_range_end", at, *sizes, *branches)
+            if end < 0:
+                self.fits, self.ranges = False, []
+                return
             cuts.append((at, end))
             at = end
         if len(cuts) == 1:
@@ -50,6 +54,10 @@ class DenseDs:
         self.cmp = (base if n_cmp else None, n_cmp)
         self.swa = (base + n_cmp if n_swa else None, n_swa)
         self.far = (base + n_cmp + n_swa if n_far else None, n_far)
+
+    def release(self):
+        """Gives the scratch back (to the current stream's pool)."""
+        self.buf = None
 
     def dkdv_cmp(self, r, q, k, v, lse, do, delta, sm_scale, dk=None, dv=None):
         """dk, dv of the compressed rows from the queries of range r, added to those of the ranges before (dk, dv)."""

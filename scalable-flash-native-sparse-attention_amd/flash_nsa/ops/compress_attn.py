@@ -55,11 +55,12 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
         delta = delta_of(o, do)
     if parts == "both" and not (finalize_dq or dkdv_repeat or q_chunk_tokens) and bwd_ds.takes(q, k, v, do, sm_scale, helper):
         ds, sums = bwd_ds.DenseDs(q, k, helper, with_swa=False), ()
-        dq_buf, mode = dq_target(q, dq)
-        for r in ds.ranges:
-            sums = ds.dkdv_cmp(r, q, k, v, lse, do, delta, sm_scale, *sums)
-            ds.dq(r, k, None, VD, sm_scale, dq_buf, mode)
-        return (dq_buf, *sums)
+        if ds.fits:
+            dq_buf, mode = dq_target(q, dq)
+            for r in ds.ranges:
+                sums = ds.dkdv_cmp(r, q, k, v, lse, do, delta, sm_scale, *sums)
+                ds.dq(r, k, None, VD, sm_scale, dq_buf, mode)
+            return (dq_buf, *sums)
     common = (q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
               v.stride(0), v.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse.data_ptr(), lse.stride(1),
               lse.stride(0), delta.data_ptr(), delta.stride(0), delta.stride(1))

@@ -86,14 +86,15 @@ def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq
         delta = delta_of(o, do)
     if parts == "both" and bwd_ds.takes(q, k, v, do, sm_scale, helper):
         ds = bwd_ds.DenseDs(q, k, helper, with_cmp=False)
-        dq_buf, mode = dq_target(q, dq)
-        kv_dtype = torch.float32 if dkv_fp32 else k.dtype
-        dk = torch.empty(T, KH, D, device=q.device, dtype=kv_dtype)
-        dv = torch.empty(T, KH, VD, device=q.device, dtype=kv_dtype)
-        for r in ds.ranges:
-            ds.dkdv_swa(r, q, k, v, lse, do, delta, sm_scale, dk, dv)
-            ds.dq(r, None, k, VD, sm_scale, dq_buf, mode)
-        return dq_buf, dk, dv
+        if ds.fits:
+            dq_buf, mode = dq_target(q, dq)
+            kv_dtype = torch.float32 if dkv_fp32 else k.dtype
+            dk = torch.empty(T, KH, D, device=q.device, dtype=kv_dtype)
+            dv = torch.empty(T, KH, VD, device=q.device, dtype=kv_dtype)
+            for r in ds.ranges:
+                ds.dkdv_swa(r, q, k, v, lse, do, delta, sm_scale, dk, dv)
+                ds.dq(r, None, k, VD, sm_scale, dq_buf, mode)
+            return dq_buf, dk, dv
     common = (q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
               v.stride(0), v.stride(1), do.data_ptr(), do.stride(0), do.stride(1), lse.data_ptr(), lse.stride(0),
               lse.stride(1), delta.data_ptr(), delta.stride(0), delta.stride(1))

@@ -344,3 +344,37 @@ def test_grid_of_the_storing_dkdv_covers_every_share_of_a_range():
                     tight += need == have > 0
                     x0 += n
     assert tight > 100
+
+
+@pytest.mark.parametrize("lens,shape,settings", [
+    ([65536], (64, 4), {}), ([8192] * 6, (64, 4), {}), ([20480] * 2, (64, 4), {}), ([1000] * 100, (64, 4), {}),
+    ([4096] * 16, (64, 4), dict(top_n=64)),
+    ([4096] * 64, (64, 4), dict(top_n=64, window_size=64)),
+    ([8192] * 16, (64, 4), dict(block_size=128, top_n=64, window_size=64)),
+    ([70001, 300, 2500], (16, 1), dict(top_n=40, window_size=0)),
+    ([250000], (64, 4), {}), ([1 << 20], (64, 4), {}), ([1 << 20], (8, 1), {}), ([300000, 500], (32, 2), {}),
+])
+def test_scratch_of_stored_ds_is_bounded(lens, shape, settings):
+    """No branch's dS takes more than its limit of 4 GB, whatever the settings; where a range that fills the GPU would, there
+    are no ranges.  A lower limit holds as well."""
+    from flash_nsa import NSAHelper, _lib
+    from flash_nsa.ops import bwd_ds
+    T, (QH, KH) = sum(lens), shape
+    q, k = torch.empty(T, QH, 128, device="meta"), torch.empty(T, KH, 128, device="meta")
+    NSAHelper.set_hyperparameters(**settings)
+    cu = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
+    NSAHelper.init_cu_seqlens(cu)
+    fitted = 0
+    for mb in (4096, 700, 0):
+        _lib.call("nsa_set_tuning", b"dense_ds_mb", mb)
+        for with_cmp, with_swa in ((True, True), (True, False), (False, True)):
+            ds = bwd_ds.DenseDs(q, k, with_cmp=with_cmp, with_swa=with_swa,
+                                all_below=NSAHelper.all_below() if with_cmp and with_swa else 0)
+            if not ds.fits:
+                assert not ds.ranges
+                continue
+            fitted += 1
+            assert max(n for _, n in (ds.cmp, ds.swa, ds.far)) <= mb << 20
+            assert (ds.cmp[1] > 0) == with_cmp and (ds.swa[1] > 0) == with_swa
+    assert fitted > 0
+    NSAHelper.set_hyperparameters()
