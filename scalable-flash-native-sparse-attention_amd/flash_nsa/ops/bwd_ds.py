@@ -16,38 +16,92 @@ def takes(q, k, v, do, sm_scale, helper=NSAHelper):
                            v.size(2), sm_scale))
 
 
-def _st(t):
-    return t.data_ptr(), t.stride(0), t.stride(1)
+def _st(t, row=0):
+    """Address of row `row` of t, strides."""
+    return t.data_ptr() + row * t.stride(0) * t.element_size(), t.stride(0), t.stride(1)
+
+
+class _Part:
+    """Sequences b0 .. b1 - 1 of a batch as a batch of their own: its first token x0 and compressed row y0, lengths, offsets from
+    there on, and the ranges of its T tokens (one range: (0, 0)), `ring` tokens the longest of them (one range: 0)."""
+
+    def __init__(self, helper, b0=0, b1=None, T=0):
+        b1 = helper.batch if b1 is None else b1
+        self.batch = b1 - b0
+        if self.batch == helper.batch:
+            self.x0 = self.y0 = 0
+            self.T, self.x_maxlen, self.y_maxlen = T, helper.x_maxlen, helper.y_maxlen
+            self.x_cu, self.y_cu = helper.x_cu_seqlens, helper.y_cu_seqlens
+            return
+        lens = [e - s for s, e in zip(helper._host_cu, helper._host_cu[1:])]
+        y = [max((n - helper.kernel_size) // helper.stride + 1, 0) for n in lens[:b1]]
+        self.x0, self.y0 = sum(lens[:b0]), sum(y[:b0])
+        self.T, self.x_maxlen, self.y_maxlen = sum(lens[b0:b1]), max(lens[b0:b1]), max(y[b0:b1])
+        self.x_cu = helper.x_cu_seqlens[b0:b1 + 1] - self.x0
+        self.y_cu = helper.y_cu_seqlens[b0:b1 + 1] - self.y0
+
+    def plan(self, end_of):
+        self.ranges, at = [], 0
+        while at < self.T:
+            end = end_of(at, self.T, self.batch, self.x_maxlen)
+            if end < 0:
+                return False
+            self.ranges.append((at, end))
+            at = end
+        if len(self.ranges) == 1:
+            self.ranges = [(0, 0)]
+        self.ring = max(e - s for s, e in self.ranges)
+        return True
+
+
+def _cut(cu, b0, b1, end_of):
+    """The sequences b0 .. b1 - 1 (offsets cu) in consecutive groups that one range holds, or of one sequence: halved, by tokens,
+    while they do not.  A tile's dS is as wide as the longest sequence beside it, so a range over a long and many short ones is
+    short: one of 60K tokens before 400 of 350, 64 / 4 heads of 128, 105 ms in 29 ranges of the whole batch, 85 with dq
+    recomputed, 77 so."""
+    n = cu[b1] - cu[b0]
+    if n == 0:
+        return []
+    if b1 - b0 == 1 or end_of(0, n, b1 - b0, max(e - s for s, e in zip(cu[b0:b1], cu[b0 + 1:b1 + 1]))) == n:
+        return [(b0, b1)]
+    at = min(range(b0 + 1, b1), key=lambda b: abs(2 * (cu[b] - cu[b0]) - n))
+    return _cut(cu, b0, at, end_of) + _cut(cu, at, b1, end_of)
 
 
 class DenseDs:
     """The scratch of one backward of the compressed branch (with_cmp), the window (with_swa) and, with all_below > 0, the keys
-    before the window of the queries below it, up to 4 GB each; `ranges` are the (tok0, tok1) that dkdv_cmp, dkdv_swa and dq are
-    called for, in this order.  `fits`: whether there are such ranges (else dq and dk / dv are to be computed apart)."""
+    before the window of the queries below it, up to 4 GB each; `ranges` are the (part of the batch, tok0, tok1) that dkdv_cmp,
+    dkdv_swa and dq are called for, in this order.  `fits`: whether there are such ranges (else dq and dk / dv are to be computed
+    apart)."""
 
     def __init__(self, q, k, helper=NSAHelper, with_cmp=True, with_swa=True, all_below=0):
         T, QH, D = q.shape
-        self.h, self.T, self.QH, self.KH, self.D = helper, T, QH, k.size(1), D
+        self.h, self.QH, self.KH, self.D = helper, QH, k.size(1), D
         self.all_below = all_below
-        sizes = (T, helper.batch, helper.x_maxlen, QH, self.KH)
         cmp_sizes = (helper.kernel_size, helper.stride)
         branches = (*(cmp_sizes if with_cmp else (0, 0)), helper.window_size if with_swa else -1, all_below)
-        cuts, at, self.fits = [], 0, True
-        while at < T:
-            end = _lib.value("nsa_bwd_ds_range_end", at, *sizes, *branches)
-            if end < 0:
-                self.fits, self.ranges = False, []
-                return
-            cuts.append((at, end))
-            at = end
-        if len(cuts) == 1:
-            cuts = [(0, 0)]
-        self.ranges = cuts
-        self.ring = max(e - s for s, e in cuts)
-        n_cmp = max(_lib.value("nsa_cmp_attn_bwd_ds_bytes", *sizes, *cmp_sizes, *r) for r in cuts) if with_cmp else 0
-        n_swa = _lib.value("nsa_swa_bwd_ds_bytes", *sizes, helper.window_size, self.ring) if with_swa else 0
-        n_far = (_lib.value("nsa_slc_bwd_before_window_ds_bytes", *sizes, helper.window_size, all_below, self.ring)
-                 if with_swa and all_below else 0)
+
+        def end_of(at, T, batch, longest):
+            return _lib.value("nsa_bwd_ds_range_end", at, T, batch, longest, QH, self.KH, *branches)
+
+        parts = [_Part(helper, T=T)]
+        self.fits = parts[0].plan(end_of)
+        host = getattr(helper, "_host_cu", None)
+        if host is not None and helper.batch > 1 and len(parts[0].ranges) != 1:
+            parts = [_Part(helper, *g) for g in _cut(host, 0, helper.batch, end_of)]
+            self.fits = all([p.plan(end_of) for p in parts])
+        self.ranges = [(p, *r) for p in parts for r in p.ranges] if self.fits else []
+        if not self.fits:
+            return
+        n_cmp = n_swa = n_far = 0
+        for p in parts:
+            sizes = (p.T, p.batch, p.x_maxlen, QH, self.KH)
+            if with_cmp:
+                n_cmp = max(n_cmp, *(_lib.value("nsa_cmp_attn_bwd_ds_bytes", *sizes, *cmp_sizes, *r) for r in p.ranges))
+            if with_swa:
+                n_swa = max(n_swa, _lib.value("nsa_swa_bwd_ds_bytes", *sizes, helper.window_size, p.ring))
+            if with_swa and all_below:
+                n_far = max(n_far, _lib.value("nsa_slc_bwd_before_window_ds_bytes", *sizes, helper.window_size, all_below, p.ring))
         n_cmp, n_swa, n_far = ((n + 255) // 256 * 256 for n in (n_cmp, n_swa, n_far))
         self.buf = torch.empty(n_cmp + n_swa + n_far, dtype=torch.uint8, device=q.device)
         base = self.buf.data_ptr()
@@ -61,11 +115,14 @@ class DenseDs:
 
     def dkdv_cmp(self, r, q, k, v, lse, do, delta, sm_scale, dk=None, dv=None):
         """dk, dv of the compressed rows from the queries of range r, added to those of the ranges before (dk, dv)."""
+        p, *r = r
         h, VD = self.h, v.size(2)
-        sizes = (h.batch, h.x_maxlen, h.y_maxlen, self.QH, self.KH, self.D, VD, h.kernel_size, h.stride)
-        first = dk is None
-        if first:
-            self.cmp_slots = max(_lib.value("nsa_cmp_attn_bwd_dkdv_ds_slot_bytes", *sizes, *x) for x in self.ranges)
+
+        def sizes(p):
+            return p.batch, p.x_maxlen, p.y_maxlen, self.QH, self.KH, self.D, VD, h.kernel_size, h.stride
+
+        if dk is None:
+            self.cmp_slots = max(_lib.value("nsa_cmp_attn_bwd_dkdv_ds_slot_bytes", *sizes(x), *t) for x, *t in self.ranges)
             shapes = (k.shape, v.shape)
             if self.cmp_slots <= compress_attn.DKDV_SLOTS_LIMIT:
                 dk, dv = (torch.empty(s, device=q.device, dtype=torch.float32) for s in shapes)
@@ -73,36 +130,40 @@ class DenseDs:
                 dk, dv = zeros_pair(*shapes, q.device)
         n = self.cmp_slots if self.cmp_slots <= compress_attn.DKDV_SLOTS_LIMIT else 0
         ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
-        _lib.call("nsa_cmp_attn_bwd_dkdv_ds", *_st(q), *_st(k), *_st(v), *_st(do), lse.data_ptr(), lse.stride(1),
-                  lse.stride(0), *_st(delta), *_st(dk), *_st(dv), h.x_cu_seqlens.data_ptr(), h.y_cu_seqlens.data_ptr(),
-                  *sizes, sm_scale, self.T, *r, *self.cmp, _lib.ptr(ws), n, int(not first), _lib.stream_ptr())
+        _lib.call("nsa_cmp_attn_bwd_dkdv_ds", *_st(q, p.x0), *_st(k, p.y0), *_st(v, p.y0), *_st(do, p.x0),
+                  lse.data_ptr() + 4 * p.x0 * lse.stride(1), lse.stride(1), lse.stride(0), *_st(delta, p.x0), *_st(dk, p.y0),
+                  *_st(dv, p.y0), p.x_cu.data_ptr(), p.y_cu.data_ptr(), *sizes(p), sm_scale, p.T, *r, *self.cmp, _lib.ptr(ws), n,
+                  int(r[0] > 0), _lib.stream_ptr())
         return dk, dv
 
     def dkdv_swa(self, r, q, k, v, lse, do, delta, sm_scale, dk, dv):
         """dk, dv (bf16 or fp32) of the keys of range r."""
-        h, VD = self.h, v.size(2)
-        sizes = (h.batch, h.x_maxlen, self.QH, self.KH, self.D, VD, h.window_size)
-        n = _lib.value("nsa_swa_bwd_dkdv_ds_ws_bytes", self.T, *sizes, *r)
+        p, *r = r
+        h, x = self.h, p.x0
+        sizes = (p.batch, p.x_maxlen, self.QH, self.KH, self.D, v.size(2), h.window_size)
+        n = _lib.value("nsa_swa_bwd_dkdv_ds_ws_bytes", p.T, *sizes, *r)
         ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
-        _lib.call("nsa_swa_bwd_dkdv_ds", *_st(q), *_st(k), *_st(v), *_st(do), *_st(lse), *_st(delta), *_st(dk), *_st(dv),
-                  int(dk.dtype == torch.float32), h.x_cu_seqlens.data_ptr(), *sizes, sm_scale, self.T, self.ring, *r,
-                  *self.swa, _lib.ptr(ws), n, _lib.stream_ptr())
+        _lib.call("nsa_swa_bwd_dkdv_ds", *_st(q, x), *_st(k, x), *_st(v, x), *_st(do, x), *_st(lse, x), *_st(delta, x), *_st(dk, x),
+                  *_st(dv, x), int(dk.dtype == torch.float32), p.x_cu.data_ptr(), *sizes, sm_scale, p.T, p.ring, *r, *self.swa,
+                  _lib.ptr(ws), n, _lib.stream_ptr())
 
     def dkdv_far(self, r, q, k, v, lse, do, delta, sm_scale, dk, dv):
         """slc_attn_bwd_dkdv_before_window for the keys of range r."""
         if not self.far[1]:
             return
-        h, VD = self.h, v.size(2)
-        _lib.call("nsa_slc_attn_bwd_dkdv_before_window_ds", *_st(q), *_st(k), *_st(v), *_st(do), *_st(lse), *_st(delta),
-                  *_st(dk), *_st(dv), h.x_cu_seqlens.data_ptr(), h.batch, h.x_maxlen, self.QH, self.KH, self.D, VD,
-                  h.window_size, self.all_below, sm_scale, self.T, self.ring, *r, *self.far, _lib.stream_ptr())
+        p, *r = r
+        h, x = self.h, p.x0
+        _lib.call("nsa_slc_attn_bwd_dkdv_before_window_ds", *_st(q, x), *_st(k, x), *_st(v, x), *_st(do, x), *_st(lse, x),
+                  *_st(delta, x), *_st(dk, x), *_st(dv, x), p.x_cu.data_ptr(), p.batch, p.x_maxlen, self.QH, self.KH, self.D,
+                  v.size(2), h.window_size, self.all_below, sm_scale, p.T, p.ring, *r, *self.far, _lib.stream_ptr())
 
     def dq(self, r, ck, k, VD, sm_scale, dq, mode, partial=None):
         """dq of the tokens of range r from the compressed rows ck and / or the keys k: mode as nsa_attn_bwd_dq_ds."""
+        p, *r = r
         h = self.h
         none = (None, 0, 0)
-        _lib.call("nsa_attn_bwd_dq_ds", *(none if ck is None else _st(ck)), *self.cmp, *(none if k is None else _st(k)),
-                  *self.swa, *self.far, *_st(dq), mode, *(none if partial is None else _st(partial)),
-                  h.x_cu_seqlens.data_ptr(), h.y_cu_seqlens.data_ptr(), h.batch, h.x_maxlen, self.QH, self.KH, self.D, VD,
-                  h.kernel_size, h.stride, h.window_size, self.all_below, sm_scale, self.T, self.ring, *r,
+        _lib.call("nsa_attn_bwd_dq_ds", *(none if ck is None else _st(ck, p.y0)), *self.cmp,
+                  *(none if k is None else _st(k, p.x0)), *self.swa, *self.far, *_st(dq, p.x0), mode,
+                  *(none if partial is None else _st(partial, p.x0)), p.x_cu.data_ptr(), p.y_cu.data_ptr(), p.batch, p.x_maxlen,
+                  self.QH, self.KH, self.D, VD, h.kernel_size, h.stride, h.window_size, self.all_below, sm_scale, p.T, p.ring, *r,
                   _lib.stream_ptr())

@@ -186,7 +186,7 @@ class BwdNSAHelper:
     _FIELDS = ("kernel_size", "stride", "block_size", "window_size", "top_n", "num_init_blocks", "num_local_blocks",
                "x_cu_seqlens", "x_seqlens", "x_maxlen", "y_cu_seqlens", "y_seqlens", "y_maxlen", "y_len",
                "k_cu_seqlens", "k_seqlens", "k_maxlen", "k_len", "blk_seq", "batch", "cmp_k_method", "cmp_v_method",
-               "deterministic")
+               "deterministic", "_host_cu")
 
     def __init__(self):
         for f in self._FIELDS:

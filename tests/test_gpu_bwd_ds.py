@@ -9,33 +9,45 @@ pytestmark = pytest.mark.gpu
 
 
 def _grads(core, ts, cu, do, device):
-    ts = [t.to(device).requires_grad_() for t in ts]
+    ts = [t.to(device).detach().requires_grad_() for t in ts]
     out = core(*ts, cu)
     out.backward(do)
     return [out.detach()] + [t.grad for t in ts]
 
 
 # ends of tiles of 64 rows (8 .. 1 tokens), of units of 32 keys, of groups of 128 positions, and sequences without a
-# compressed row; ranged: a scratch limit in MB that needs several ranges
+# compressed row; mb: a scratch limit in MB that needs several ranges; whole: ranges of the whole batch, as where a helper does not
+# have the lengths on the host, else of parts of it
 CASES = [
-    # QH, KH, D, VD, lens, ranged, settings
-    (8, 1, 128, 128, [1, 31, 32, 33, 700], 0, {}),
-    (16, 1, 128, 128, [1024, 1025, 47, 1279], 0, dict(top_n=4)),
-    (32, 1, 128, 128, [0, 515, 0, 640], 0, dict(window_size=100, top_n=3)),
-    (64, 1, 128, 128, [513, 1, 129], 0, dict(window_size=0, top_n=3)),
-    (64, 4, 128, 128, [4700], 300, {}),
-    (64, 1, 128, 128, [2047, 300, 2500, 5], 200, dict(top_n=6)),
-    (64, 4, 192, 128, [130, 4300], 190, dict(window_size=300)),
-    (32, 2, 192, 128, [900, 64, 333], 0, dict(block_size=96, kernel_size=64, stride=32, top_n=5)),
-    (16, 2, 128, 128, [1500, 200], 0, dict(window_size=2000)),
-    (16, 1, 192, 128, [777], 0, dict(kernel_size=16, stride=8, block_size=32, top_n=40)),
+    # QH, KH, D, VD, lens, mb, whole, settings
+    (8, 1, 128, 128, [1, 31, 32, 33, 700], 0, False, {}),
+    (16, 1, 128, 128, [1024, 1025, 47, 1279], 0, False, dict(top_n=4)),
+    (32, 1, 128, 128, [0, 515, 0, 640], 0, False, dict(window_size=100, top_n=3)),
+    (64, 1, 128, 128, [513, 1, 129], 0, False, dict(window_size=0, top_n=3)),
+    (64, 4, 128, 128, [4700], 300, False, {}),
+    (64, 1, 128, 128, [2047, 300, 2500, 5], 200, True, dict(top_n=6)),
+    (64, 1, 128, 128, [2047, 300, 2500, 5], 200, False, dict(top_n=6)),
+    (64, 4, 192, 128, [130, 4300], 190, True, dict(window_size=300)),
+    (64, 4, 192, 128, [130, 4300], 165, False, dict(window_size=300)),
+    (32, 2, 192, 128, [900, 64, 333], 0, False, dict(block_size=96, kernel_size=64, stride=32, top_n=5)),
+    (16, 2, 128, 128, [1500, 200], 0, False, dict(window_size=2000)),
+    (16, 1, 192, 128, [777], 0, False, dict(kernel_size=16, stride=8, block_size=32, top_n=40)),
     # chunks of 256 queries, cut from the first row of a share in the middle of a sequence
-    (32, 2, 128, 128, [3063, 9859], 200, {}),
+    (32, 2, 128, 128, [3063, 9859], 200, True, {}),
+    # the keys before the window in places taken in turn
+    (64, 1, 128, 128, [1100, 1024, 1300, 1111, 1029], 500, True, dict(window_size=100)),
+    # a long sequence between many short ones
+    (64, 4, 128, 128, [40, 0, 350, 5, 350, 350, 4500, 33, 350, 350, 0, 350, 31], 300, False, {}),
 ]
 
 
-@pytest.mark.parametrize("QH,KH,D,VD,lens,ranged,settings", CASES)
-def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ranged, settings):
+def _wide(t):
+    """t in rows twice as long"""
+    return torch.cat([t, t], -1)[..., :t.size(-1)]
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens,mb,whole,settings", CASES)
+def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, mb, whole, settings):
     from flash_nsa import NSAConfig, NSACore, _lib
     from flash_nsa.ops import bwd_ds
     from flash_nsa.utils import NSAHelper as H
@@ -43,12 +55,21 @@ def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ra
     cu = make_cu(lens).to(device)
     ts = make_qkvw(T, QH, KH, D, VD, seed=300)
     do = randn_bf16(T, QH, VD, seed=301).to(device)
+    if mb:
+        ts, do = [*map(_wide, ts[:3]), ts[3]], _wide(do)
     core = NSACore(NSAConfig(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH, **settings))
     core = core.to(device=device, dtype=torch.bfloat16)
     made, init = [], bwd_ds.DenseDs.__init__
-    bwd_ds.DenseDs.__init__ = lambda self, *a, **k: (init(self, *a, **k), made.append(self))[0]
-    if ranged:
-        _lib.call("nsa_set_tuning", b"dense_ds_mb", ranged)
+
+    def recorded(self, *a, **k):
+        host, H._host_cu = H._host_cu, None if whole else H._host_cu
+        init(self, *a, **k)
+        H._host_cu = host
+        made.append(self)
+
+    bwd_ds.DenseDs.__init__ = recorded
+    if mb:
+        _lib.call("nsa_set_tuning", b"dense_ds_mb", mb)
     try:
         got = _grads(core, ts, cu, do, device)
         H.set_deterministic(True)
@@ -57,7 +78,8 @@ def test_dq_from_stored_ds_is_the_recomputed_one(device, QH, KH, D, VD, lens, ra
         H.set_deterministic(False)
         _lib.call("nsa_reset_tuning")
         bwd_ds.DenseDs.__init__ = init
-    assert len(made) == 1 and (len(made[0].ranges) > 1) == (ranged > 0)
+    assert len(made) == 1 and (len(made[0].ranges) > 1) == (mb > 0)
+    assert len({id(p) for p, *_ in made[0].ranges}) == 1 or not whole
     assert torch.equal(got[0], want[0])
     # the same products of bf16 operands whose last bit may differ (P from differently rounded exponents): the bar that both
     # are held to against the oracle

@@ -378,3 +378,39 @@ def test_scratch_of_stored_ds_is_bounded(lens, shape, settings):
             assert (ds.cmp[1] > 0) == with_cmp and (ds.swa[1] > 0) == with_swa
     assert fitted > 0
     NSAHelper.set_hyperparameters()
+
+
+@pytest.mark.parametrize("lens,most", [
+    ([60000] + [350] * 400, 8), ([350] * 200 + [60000] + [350] * 200, 9), ([16384] + [512] * 96, 3), ([20480] * 2, 2),
+    ([12288] * 10, 4), ([1000] * 100, 2), ([0, 60000, 0, 0, 31, 500, 0], 7), ([65536], 6), ([300] * 20, 1),
+])
+def test_parts_of_a_batch_whose_stored_ds_takes_several_ranges(lens, most):
+    """A batch that one range does not hold is cut between its sequences, so that short ones do not get the width of the longest:
+    every token in one part, in order; several ranges in parts of one sequence alone."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops import bwd_ds
+    T, QH, KH = sum(lens), 64, 4
+    NSAHelper.set_hyperparameters()
+    cu = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
+    NSAHelper.init_cu_seqlens(cu)
+    ds = bwd_ds.DenseDs(torch.empty(T, QH, 128, device="meta"), torch.empty(T, KH, 128, device="meta"),
+                        all_below=NSAHelper.all_below())
+    assert ds.fits and len(ds.ranges) <= most
+    parts = list(dict.fromkeys(p for p, *_ in ds.ranges))
+    x, y = cu.tolist(), NSAHelper.y_cu_seqlens.tolist()
+    seqs, at = [], 0
+    for p in parts:
+        b0 = max(b for b in range(len(lens)) if x[b] == p.x0 and lens[b:b + p.batch] and
+                 [c + p.x0 for c in p.x_cu.tolist()] == x[b:b + p.batch + 1])
+        assert p.x0 == at and p.T == p.x_cu.tolist()[-1] and p.y0 == y[b0]
+        assert [c + p.y0 for c in p.y_cu.tolist()] == y[b0:b0 + p.batch + 1]
+        assert p.x_maxlen == max(lens[b0:b0 + p.batch])
+        assert p.y_maxlen == max(d - c for c, d in zip(p.y_cu.tolist(), p.y_cu.tolist()[1:]))
+        assert len(p.ranges) == 1 or p.batch == 1
+        seqs += range(b0, b0 + p.batch)
+        at += p.T
+        ends = [r[2] for r in ds.ranges if r[0] is p]
+        starts = [r[1] for r in ds.ranges if r[0] is p]
+        assert (starts, ends) == ([0], [0]) or (starts == [0] + ends[:-1] and ends[-1] == p.T and p.ring > 0)
+    assert at == T and set(range(len(lens))) - set(seqs) <= {b for b, n in enumerate(lens) if n == 0}
+    NSAHelper.set_hyperparameters()
