@@ -122,12 +122,12 @@ def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, l
         # (the selected dq comes last and adds this one; the queries that the gather leaves out are done)
         ds.dq(r, cmp_k, k, v.size(2), sm_scale, dq, 3 if ds_tokens else 0, dq32)
 
-    def selected(before_dq=None):
+    def selected(dq_after=None):
         if ds_tokens:
             slc_attn_bwd(q, k, v, topk, None, lse_slc, do, dq=dq32, dk=dk, dv=dv, delta=delta[1], t_begin=all_below,
-                         finalize_dq=dq, before_dq=before_dq, ds_tokens=ds_tokens, sm_scale=sm_scale, helper=helper)
-        elif before_dq is not None:
-            before_dq()
+                         finalize_dq=dq, dq_after=dq_after, ds_tokens=ds_tokens, sm_scale=sm_scale, helper=helper)
+        elif dq_after is not None:
+            torch.cuda.current_stream().wait_event(dq_after)
 
     if OVERLAP_STREAMS and len(ds.ranges) == 1:
         # the compressed dk / dv next to the window's, the dense dq next to the selected dk / dv
@@ -140,9 +140,10 @@ def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, l
         with torch.cuda.stream(side):
             side.wait_event(window_done)
             dense_dq(r)
+            dq_done = side.record_event()
         dcmp_k.record_stream(main)
         dcmp_v.record_stream(main)
-        selected(lambda: main.wait_stream(side))
+        selected(dq_done)
     else:  # ranges follow each other on one scratch, and each of them fills the GPU
         sums = ()
         for r in ds.ranges:
@@ -238,11 +239,11 @@ class NSAFunction(torch.autograd.Function):
             return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
                                 parts="dq", finalize_below=(dq_last, all_below) if stored_ds else None, **kw)[0]
 
-        def dkdv_raw(before_dq=None):
+        def dkdv_raw(dq_after=None):
             # the window branch writes every element of dk / dv, the selected branch then adds to them
             _, dk, dv = swa_bwd(q, k, v, swa_o, lse_swa, do, delta=delta[2], dkv_fp32=True, parts="dkdv", **kw)
             slc_attn_bwd_dkdv_before_window(q, k, v, lse_slc, do, delta[1], dk, dv, all_below, **kw)
-            last = dict(dq=dq32, finalize_dq=dq_last, before_dq=before_dq, ds_tokens=ds_tokens) if stored_ds else dict(parts="dkdv")
+            last = dict(dq=dq32, finalize_dq=dq_last, dq_after=dq_after, ds_tokens=ds_tokens) if stored_ds else dict(parts="dkdv")
             slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, dk=dk, dv=dv, delta=delta[1], t_begin=all_below, **last, **kw)
             return dk, dv
 
@@ -261,7 +262,7 @@ class NSAFunction(torch.autograd.Function):
                 dcmp_k, dcmp_v = dkdv_cmp()
                 dcmp_k.record_stream(main)
                 dcmp_v.record_stream(main)
-            dk, dv = dkdv_raw(lambda: main.wait_event(dense_dq))
+            dk, dv = dkdv_raw(dense_dq)
             main.wait_stream(side)
         elif OVERLAP_STREAMS:
             side = _side_stream(q.device)

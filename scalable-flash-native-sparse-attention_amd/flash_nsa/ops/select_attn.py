@@ -39,7 +39,7 @@ def slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale=None, helper=NSAHelper):
                       topk.size(-1), default_scale(q, sm_scale))
 
 
-def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, t_begin, sm_scale, helper, before_dq):
+def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, t_begin, sm_scale, helper, dq_after):
     T, QH, KH, D, VD = shape
     N, nblk, dev = topk.size(-1), helper.k_len, topk.device
     chunk = _lib.value("nsa_slc_bwd_chunk_tokens", tokens, KH, N)
@@ -68,14 +68,14 @@ def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, 
         _lib.call("nsa_slc_attn_bwd_dkdv_ds", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0),
                   dv.stride(1), x_cu, k_cu, helper.blk_seq.data_ptr(), csr_off, index, slot, item_off, nblk, chunk,
                   (n * N + chunk - 1) // chunk + nblk, *heads, tok0, n, sm_scale, ds, ds_bytes, stream)
-        if tok0 == 0 and before_dq is not None:
-            before_dq()
+        if tok0 == 0 and dq_after is not None:
+            torch.cuda.current_stream().wait_event(dq_after)
         _lib.call("nsa_slc_attn_bwd_dq_ds", *common[3:6], *tk, *dqs, x_cu, *heads, t_begin, tok0, n, sm_scale, ds, ds_bytes,
                   stream)
 
 
 def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=None, helper=NSAHelper, delta=None,
-                 bind=None, parts="both", dkdv_repeat=False, t_begin=0, finalize_dq=None, before_dq=None,
+                 bind=None, parts="both", dkdv_repeat=False, t_begin=0, finalize_dq=None, dq_after=None,
                  ds_tokens=None):
     """Backward of selected attention.  Returns (dq, dk, dv).
     dq: fresh bf16 tensor, or the caller's fp32 buffer (added into).  dk/dv: fp32 [T,KH,*]; the caller's buffers
@@ -88,7 +88,7 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     t_begin: only the queries at positions from here on (a given `bind` then has to leave the others out).
     ds_tokens: what slc_bwd_ds_tokens has returned for these tensors, if the caller has asked.
     finalize_dq (where slc_bwd_ds_tokens > 0): a tensor of q's dtype that takes the sum of this branch's dq and dq, the fp32
-    sum of the others; before_dq is called before the launch that reads it."""
+    sum of the others, which is ready when the event dq_after is."""
     from .topk import get_bind_from_find
     check_thd(do, "do")
     T, QH, D = q.shape
@@ -128,7 +128,7 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
         return dq_buf, dk, dv
     if ds_tokens:
         _slc_attn_bwd_ds(common, topk, dq_buf, mode, partial, dk, dv, (T, QH, KH, D, VD), ds_tokens, t_begin, sm_scale,
-                         helper, before_dq)
+                         helper, dq_after)
         return dq_buf, dk, dv
     if bind is None:
         bind = get_bind_from_find(topk, helper, t_begin=t_begin, deterministic=ordered)

@@ -414,3 +414,10 @@ def test_parts_of_a_batch_whose_stored_ds_takes_several_ranges(lens, most):
         assert (starts, ends) == ([0], [0]) or (starts == [0] + ends[:-1] and ends[-1] == p.T and p.ring > 0)
     assert at == T and set(range(len(lens))) - set(seqs) <= {b for b, n in enumerate(lens) if n == 0}
     NSAHelper.set_hyperparameters()
+
+
+def test_backward_of_the_selected_branch_takes_the_event_of_the_other_dq():
+    import inspect
+    from flash_nsa.ops.select_attn import slc_attn_bwd
+    names = list(inspect.signature(slc_attn_bwd).parameters)
+    assert names[-3:] == ["finalize_dq", "dq_after", "ds_tokens"]
