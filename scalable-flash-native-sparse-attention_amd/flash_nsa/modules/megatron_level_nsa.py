@@ -13,7 +13,7 @@ from ..ops.compress_kv import construct_block_fwd, construct_block_bwd, mean_poo
 from ..ops import bwd_ds
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
 from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window,
-                               slc_bwd_ds_tokens)
+                               slc_bwd_ds_tokens, wait_for)
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
 from ..ops.combine import combine_bwd_gates
@@ -126,8 +126,8 @@ def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, l
         if ds_tokens:
             slc_attn_bwd(q, k, v, topk, None, lse_slc, do, dq=dq32, dk=dk, dv=dv, delta=delta[1], t_begin=all_below,
                          finalize_dq=dq, dq_after=dq_after, ds_tokens=ds_tokens, sm_scale=sm_scale, helper=helper)
-        elif dq_after is not None:
-            torch.cuda.current_stream().wait_event(dq_after)
+        else:
+            wait_for(dq_after)
 
     if OVERLAP_STREAMS and len(ds.ranges) == 1:
         # the compressed dk / dv next to the window's, the dense dq next to the selected dk / dv
@@ -140,10 +140,9 @@ def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, l
         with torch.cuda.stream(side):
             side.wait_event(window_done)
             dense_dq(r)
-            dq_done = side.record_event()
         dcmp_k.record_stream(main)
         dcmp_v.record_stream(main)
-        selected(dq_done)
+        selected(side)
     else:  # ranges follow each other on one scratch, and each of them fills the GPU
         sums = ()
         for r in ds.ranges:

@@ -39,6 +39,14 @@ def slc_bwd_ds_tokens(q, k, v, do, topk, sm_scale=None, helper=NSAHelper):
                       topk.size(-1), default_scale(q, sm_scale))
 
 
+def wait_for(done):
+    """The current stream waits for an event, or for what has been launched on another stream (None: for nothing)."""
+    if isinstance(done, torch.cuda.Stream):
+        torch.cuda.current_stream().wait_stream(done)
+    elif done is not None:
+        torch.cuda.current_stream().wait_event(done)
+
+
 def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, t_begin, sm_scale, helper, dq_after):
     T, QH, KH, D, VD = shape
     N, nblk, dev = topk.size(-1), helper.k_len, topk.device
@@ -68,8 +76,8 @@ def _slc_attn_bwd_ds(common, topk, dq, dq_mode, partial, dk, dv, shape, tokens, 
         _lib.call("nsa_slc_attn_bwd_dkdv_ds", *common, dk.data_ptr(), dk.stride(0), dk.stride(1), dv.data_ptr(), dv.stride(0),
                   dv.stride(1), x_cu, k_cu, helper.blk_seq.data_ptr(), csr_off, index, slot, item_off, nblk, chunk,
                   (n * N + chunk - 1) // chunk + nblk, *heads, tok0, n, sm_scale, ds, ds_bytes, stream)
-        if tok0 == 0 and dq_after is not None:
-            torch.cuda.current_stream().wait_event(dq_after)
+        if tok0 == 0:
+            wait_for(dq_after)
         _lib.call("nsa_slc_attn_bwd_dq_ds", *common[3:6], *tk, *dqs, x_cu, *heads, t_begin, tok0, n, sm_scale, ds, ds_bytes,
                   stream)
 
@@ -88,7 +96,7 @@ def slc_attn_bwd(q, k, v, topk, o, lse, do, dq=None, dk=None, dv=None, sm_scale=
     t_begin: only the queries at positions from here on (a given `bind` then has to leave the others out).
     ds_tokens: what slc_bwd_ds_tokens has returned for these tensors, if the caller has asked.
     finalize_dq (where slc_bwd_ds_tokens > 0): a tensor of q's dtype that takes the sum of this branch's dq and dq, the fp32
-    sum of the others, which is ready when the event dq_after is."""
+    sum of the others, which is ready when the event dq_after is, or what has been launched on the stream dq_after."""
     from .topk import get_bind_from_find
     check_thd(do, "do")
     T, QH, D = q.shape
