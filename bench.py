@@ -20,12 +20,12 @@ sys.path.insert(0, os.path.join(ROOT, "scalable-flash-native-sparse-attention_am
 sys.path.insert(0, ROOT)
 
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
-# Bytes per launch crossing the L2 <-> memory-side boundary (rocprofv3 --pmc FETCH_SIZE + WRITE_SIZE, each scaled by
+# Bytes per step crossing the L2 <-> memory-side boundary (rocprofv3 --pmc FETCH_SIZE + WRITE_SIZE, each scaled by
 # what the same counter reads for a 1 GiB copy: x2.000 and x1.000), measured on the T=65536 workload of this file;
 # reported as roofline.traffic for that workload only.
 MEASURED_TRAFFIC_T64K = {
-    "slc_bwd": 78.07e9, "cmp_dkdv": 30.80e9, "slc_fwd": 58.10e9, "cmp_dq": 6.62e9, "topk": 2.28e9, "cmp_fwd": 2.27e9,
-    "swa_dkdv": 11.43e9, "swa_dq": 7.61e9, "swa_fwd": 3.24e9,
+    "slc_bwd": 76.19e9, "slc_fwd": 56.89e9, "cmp_dkdv": 42.76e9, "dense_dq": 25.86e9, "swa_dkdv": 18.26e9, "swa_fwd": 6.31e9,
+    "topk": 2.27e9, "cmp_fwd": 2.25e9,
 }
 PEAK_HBM_GBS = 8000.0
 
@@ -54,103 +54,62 @@ def stage_flops(lens, QH, D, VD, **kw):
     for br in ("cmp", "swa"):
         f[br + "_dkdv"] = 2.0 * f[br + "_fwd"]
         f[br + "_dq"] = 0.5 * f[br + "_fwd"]
+    f["dense_dq"] = f["cmp_dq"] + f["swa_dq"]
     f["fwd_total"] = f["cmp_fwd"] + f["topk"] + f["slc_fwd"] + f["swa_fwd"]
     f["bwd_total"] = 2.5 * (f["cmp_fwd"] + f["slc_fwd"] + f["swa_fwd"])
     return f
 
 
+# stage of a C entry point, by the start of its name; the others are stages of their own
+_STAGES = (("nsa_cmp_attn_fwd", "cmp_fwd"), ("nsa_topk_select", "topk"), ("nsa_slc_attn_fwd", "slc_fwd"),
+           ("nsa_swa_fwd", "swa_fwd"),  # with the selected branch of the first queries and the gated sum
+           ("nsa_cmp_attn_bwd_dkdv", "cmp_dkdv"), ("nsa_cmp_attn_bwd_dq", "cmp_dq"), ("nsa_swa_bwd_dkdv", "swa_dkdv"),
+           ("nsa_slc_attn_bwd_dkdv_before_window", "swa_dkdv"), ("nsa_swa_bwd_dq", "swa_dq"),
+           ("nsa_attn_bwd_dq_ds", "dense_dq"),  # of the compressed and the window branch, from stored dS
+           ("nsa_slc_attn_bwd", "slc_bwd"), ("nsa_build_inverse_index", "slc_bwd"))
+
+
 class StageTimer:
-    """HIP-event timing of named stages on the current stream."""
+    """HIP-event times of every C entry point that a step calls, on one stream, by stage."""
 
     def __init__(self):
         self.events = []
+        self.steps = 0
 
-    def run(self, name, fn):
+    def _call(self, name, *args):
         import torch
         s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         s.record()
-        out = fn()
+        self.run(name, *args)
         e.record()
-        self.events.append((name, s, e))
-        return out
+        self.events.append((next((stage for start, stage in _STAGES if name.startswith(start)), name[4:]), s, e))
+
+    def step(self, fn):
+        import torch
+        from flash_nsa import _lib
+        from flash_nsa.modules import megatron_level_nsa as core
+        s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        overlap, core.OVERLAP_STREAMS = core.OVERLAP_STREAMS, False
+        self.run, _lib.call = _lib.call, self._call
+        try:
+            s.record()
+            fn()
+            e.record()
+        finally:
+            core.OVERLAP_STREAMS, _lib.call = overlap, self.run
+        self.events.append(("step", s, e))
+        self.steps += 1
 
     def summary(self):
+        """Milliseconds per step of every stage; `rest`: library products, casts, fills and gaps."""
         import torch
         torch.cuda.synchronize()
         acc = {}
         for name, s, e in self.events:
-            acc.setdefault(name, []).append(s.elapsed_time(e))
-        return {k: sum(v) / len(v) for k, v in acc.items()}
-
-
-def staged_step(timer, q, k, v, w, wv, do, sm_scale):
-    """The same launches as NSAFunction.forward/backward, stage by stage under event timers."""
-    import torch
-    from flash_nsa.ops.compress_kv import mean_pooling_fwd, construct_block_fwd, construct_block_bwd, mean_pooling_bwd
-    from flash_nsa.ops.act import sigmoid_mul_fwd, sigmoid_mul_bwd
-    from flash_nsa.ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
-    from flash_nsa.ops.topk import slc_topk_indices
-    from flash_nsa.ops.select_attn import slc_attn_fwd, slc_attn_bwd
-    from flash_nsa.ops.sliding_window_attention import swa_fwd, swa_bwd
-    from flash_nsa.ops.combine import combine_fwd, combine_bwd
-    from flash_nsa import _lib
-    from flash_nsa.utils import NSAHelper as H
-    from flash_nsa.modules.megatron_level_nsa import _store_into
-
-    R = timer.run
-    cmp_k = R("pool_k", lambda: mean_pooling_fwd(k))
-    win_v = R("im2col_v", lambda: construct_block_fwd(v))
-    hid_v = R("gemm_cmp_v", lambda: torch.matmul(win_v.flatten(-2, -1), wv.t()))
-    cmp_v = R("sigmoid_mul", lambda: sigmoid_mul_fwd(hid_v))
-    cmp_o, cmp_lse = R("cmp_fwd", lambda: cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale))
-    topk, _ = R("topk", lambda: slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale))
-    slc_o, slc_lse = R("slc_fwd", lambda: slc_attn_fwd(q, k, v, topk, sm_scale=sm_scale))
-    swa_o, swa_lse = R("swa_fwd", lambda: swa_fwd(q, k, v, sm_scale=sm_scale))
-    R("combine_fwd", lambda: combine_fwd(cmp_o, slc_o, swa_o, w))
-
-    dcmp_o, dslc_o, dswa_o, dw, delta = R("combine_bwd", lambda: combine_bwd(cmp_o, slc_o, swa_o, w, do, True))
-    dq = torch.zeros(q.shape, device=q.device, dtype=torch.float32)
-    T, QH, D = q.shape
-    _, KH, VD = v.shape
-
-    def common(kk, vv, lse, lse_st, lse_sh, dlt, dout):
-        return (q.data_ptr(), q.stride(0), q.stride(1), kk.data_ptr(), kk.stride(0), kk.stride(1), vv.data_ptr(),
-                vv.stride(0), vv.stride(1), dout.data_ptr(), dout.stride(0), dout.stride(1), lse.data_ptr(), lse_st,
-                lse_sh, dlt.data_ptr(), dlt.stride(0), dlt.stride(1))
-
-    dk = torch.empty(T, KH, D, device=q.device, dtype=torch.float32)
-    dv = torch.empty(T, KH, VD, device=q.device, dtype=torch.float32)
-    cs = common(k, v, swa_lse, swa_lse.stride(0), swa_lse.stride(1), delta[2], dswa_o)
-    R("swa_dq", lambda: _lib.call("nsa_swa_bwd_dq", *cs, dq.data_ptr(), dq.stride(0), dq.stride(1), 2,
-                                  H.x_cu_seqlens.data_ptr(), H.batch, H.x_maxlen, QH, KH, D, VD, H.window_size,
-                                  sm_scale, _lib.stream_ptr()))
-    R("swa_dkdv", lambda: _lib.call("nsa_swa_bwd_dkdv", *cs, dk.data_ptr(), dk.stride(0), dk.stride(1),
-                                    dv.data_ptr(), dv.stride(0), dv.stride(1), 1, H.x_cu_seqlens.data_ptr(), H.batch,
-                                    H.x_maxlen, QH, KH, D, VD, H.window_size, sm_scale, _lib.stream_ptr()))
-    # inverse index, dk / dv and dq from its dS, for one range of tokens after another
-    R("slc_bwd", lambda: slc_attn_bwd(q, k, v, topk, slc_o, slc_lse, dslc_o, dq=dq, dk=dk, dv=dv, sm_scale=sm_scale,
-                                      delta=delta[1]))
-    cc = common(cmp_k, cmp_v, cmp_lse, cmp_lse.stride(1), cmp_lse.stride(0), delta[0], dcmp_o)
-    dq_out = torch.empty_like(q)  # the last dq kernel adds the fp32 partial sum and stores q's dtype
-    R("cmp_dq", lambda: _lib.call("nsa_cmp_attn_bwd_dq_final", *cc, dq.data_ptr(), dq.stride(0), dq.stride(1),
-                                  dq_out.data_ptr(), dq_out.stride(0), dq_out.stride(1), H.x_cu_seqlens.data_ptr(),
-                                  H.y_cu_seqlens.data_ptr(), H.batch, H.x_maxlen, QH, KH, D, VD, H.kernel_size,
-                                  H.stride, sm_scale, _lib.stream_ptr()))
-    dck = torch.zeros(cmp_k.shape, device=q.device, dtype=torch.float32)
-    dcv = torch.zeros(cmp_v.shape, device=q.device, dtype=torch.float32)
-    R("cmp_dkdv", lambda: _lib.call("nsa_cmp_attn_bwd_dkdv", *cc, dck.data_ptr(), dck.stride(0), dck.stride(1),
-                                    dcv.data_ptr(), dcv.stride(0), dcv.stride(1), H.x_cu_seqlens.data_ptr(),
-                                    H.y_cu_seqlens.data_ptr(), H.batch, H.x_maxlen, H.y_maxlen, QH, KH, D, VD,
-                                    H.kernel_size, H.stride, 0, sm_scale, _lib.stream_ptr()))
-    R("pool_k_bwd", lambda: mean_pooling_bwd(k, dck.to(k.dtype), dk))
-
-    def cmp_v_bwd():
-        dhid = sigmoid_mul_bwd(hid_v, dcv.to(v.dtype), inplace=False)
-        dwin = torch.matmul(dhid, wv).view(*win_v.shape)
-        construct_block_bwd(v, dwin, dv)
-        return torch.matmul(dhid.flatten(0, 1).t(), win_v.flatten(-2, -1).flatten(0, 1))
-
-    R("cmp_v_bwd", cmp_v_bwd)
+            acc[name] = acc.get(name, 0.0) + s.elapsed_time(e) / self.steps
+        acc["rest"] = 2 * acc["step"] - sum(acc.values())
+        del acc["step"]
+        return acc
 
 
 def selection_pattern(name, T, KH, dev, seed=7):
@@ -424,7 +383,7 @@ def main():
     torch.cuda.synchronize()
     ms_per_step = (time.perf_counter() - t0) * 1e3 / args.steps
 
-    # forward-only and per-stage times (HIP events on the launch stream)
+    # forward-only and per-stage times (HIP events; the stages of the whole step on one stream)
     with torch.no_grad():
         core(q, k, v, w, cu)
         torch.cuda.synchronize()
@@ -433,12 +392,12 @@ def main():
             core(q, k, v, w, cu)
         torch.cuda.synchronize()
         fwd_ms = (time.perf_counter() - t0) * 1e3 / args.steps
-        timer = StageTimer()
-        qd, kd, vd, wd = q.detach(), k.detach(), v.detach(), w.detach()
-        staged_step(StageTimer(), qd, kd, vd, wd, core.cmp_v_weight.detach(), do, core.sm_scale)  # warm
-        for _ in range(max(args.steps, 3)):
-            staged_step(timer, qd, kd, vd, wd, core.cmp_v_weight.detach(), do, core.sm_scale)
-        stages = timer.summary()
+
+    StageTimer().step(step)  # warm
+    timer = StageTimer()
+    for _ in range(max(args.steps, 3)):
+        timer.step(step)
+    stages = timer.summary()
 
     fl = stage_flops([T], QH, D, D)
     total_flops = fl["fwd_total"] + fl["bwd_total"]
