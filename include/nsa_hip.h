@@ -340,9 +340,10 @@ int nsa_slc_attn_bwd_dkdv_det(const void* q, int64_t q_st, int64_t q_sh, const v
  * together.  The batch (T rows) is processed in ranges of tokens [tok0, tok1) in ascending order (tok1 = 0: all of it in one;
  * otherwise the range of 128-position groups of a sequence whose first token it holds), so that the scratch stays bounded:
  * nsa_bwd_ds_range_end gives the end of the range that begins at tok0 (T: the last one), in which no branch takes more than
- * 4 GB (stride 0: without the compressed branch, window -1: without the window), or -1 where a range that fills the GPU would:
- * such batches have dq computed apart.  nsa_bwd_ds_next: the same ranges of the compressed branch and the window alone, at least
- * as long as fills the GPU, whatever they take.
+ * 4 GB (stride 0: without the compressed branch, window -1: without the window), or -1 where a range of 16384 / QH tokens would
+ * (sequences past a million tokens; past a window of many thousand keys) or all_below tokens of one sequence would: dq is then
+ * to be computed apart.  nsa_bwd_ds_next: the same ranges of the compressed branch and the window alone, at
+ * least as long as fills the GPU, whatever they take.
  * nsa_bwd_ds_takes: 1 where these shapes, strides and scale have this path.  nsa_*_ds_bytes: scratch of a branch; `ring` is
  * the length of the longest range (0: one range).  The window's scratch holds what the next range needs: the same buffer is
  * passed for all ranges, and a range's dk / dv kernels run after the dq launch of the range before. */

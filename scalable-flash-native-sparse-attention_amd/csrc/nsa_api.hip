@@ -1066,18 +1066,11 @@ int64_t nsa_slc_bwd_before_window_ds_bytes(int T, int B, int x_maxlen, int QH, i
   return ds_layout_far(T, B, x_maxlen, QH / KH, KH, window, all_below, ring).bytes;
 }
 
-// End of the range of tokens that begins at tok0: 4 GB for each branch's dS (stride 0: without the compressed branch, window -1:
-// without the window, all_below 0: without the keys before it), but never fewer tokens than give the dQ kernel 512 workgroups of
-// 256 rows, and no shorter rest; *fit: whether that holds the 4 GB.  Whole step with 2 / 4 / 8 / 40 GB, 64 heads of 128, ms: 64K
-// tokens 52.7 / 52.2 / 51.8 / 52.2, 8 x 6K 19.9 / 19.2 / 19.2 / 19.2.  (As for the selected branch no rule on the number of tokens
-// decides whether dq comes from stored dS: a query's dq is to be the same bits whatever follows it in the batch.  The exceptions
-// are what even the least range does not hold, and batches beside it: sequences past a quarter of a million tokens, and, where
-// top_n * block_size is far beyond the window, of more than so many keys before it.)
-static int ds_least(int QH) { return (131072 / QH + 127) & ~127; }
-static int ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
-                        int all_below, bool* fit) {
-  const int G = QH / KH;
-  const int64_t budget = (int64_t)nsa_tuning_knob("dense_ds_mb", 4096) << 20;
+// End of the range of tokens that begins at tok0: `budget` bytes for each branch's dS (stride 0: without the compressed branch,
+// window -1: without the window, all_below 0: without the keys before it), but never fewer tokens than `least`, and no shorter
+// rest; *fit: whether that holds the budget.
+static int ds_range_end(int tok0, int T, int B, int x_maxlen, int G, int KH, int kernel_size, int stride, int window,
+                        int all_below, int64_t budget, int least, bool* fit) {
   auto fits = [&](int tok1) {
     if (stride > 0 && ds_layout_cmp(T, B, x_maxlen, G, KH, kernel_size, stride, tok0, tok1).bytes > budget) return false;
     if (window < 0) return true;
@@ -1086,7 +1079,6 @@ static int ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, in
   };
   *fit = true;
   if (fits(T)) return T;
-  const int least = ds_least(QH);
   int lo = tok0 + least;
   *fit = lo < T && fits(lo);
   if (lo >= T) return T;
@@ -1101,19 +1093,36 @@ static int ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, in
   const int half = ((T - tok0) / 2 + 127) & ~127;
   return T - tok0 - half >= least ? tok0 + half : lo;
 }
+// 4 GB.  Whole step with 2 / 4 / 8 / 40 GB, 64 heads of 128, ms: 64K tokens 52.7 / 52.2 / 51.8 / 52.2, 8 x 6K 19.9 / 19.2 / 19.2 /
+// 19.2.
+static int64_t ds_budget() { return (int64_t)nsa_tuning_knob("dense_ds_mb", 4096) << 20; }
+// Tokens of a range that give the dQ kernel 512 workgroups of 256 rows, and, where the budget does not hold those, the fewest: an
+// eighth.  Backward of one sequence, 64 / 4 heads of 128, ms, dq recomputed / from stored dS with ranges of the budget at its end
+// (tokens) / with the former whatever they take: 256K 321 / 284 (1.9K) / 282, 512K 1147 / 1001 (0.9K) / 950, 768K 2521 / 2258
+// (0.5K), 1M 4406 / 4257 (256).
+static int ds_least(int QH) { return (131072 / QH + 127) & ~127; }
+static int ds_short(int QH) { return (16384 / QH + 127) & ~127; }
 
 int nsa_bwd_ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
                          int all_below) {
   if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || tok0 < 0 || tok0 >= T) return T;
+  const int G = QH / KH, longest = 1 << 28;
+  const int64_t budget = ds_budget();
+  // What decides whether dq comes from stored dS is not the number of tokens: a query's dq is to be the same bits whatever follows
+  // it in the batch.  So where top_n * block_size is too far beyond the window for one sequence of so many tokens, there is none
+  // for a shorter one either.  (Sequences past a million tokens, for the compressed branch, and past a window of many thousand
+  // keys, which has to be the longest sequence's in a batch of shorter ones, have none.)
+  if (window >= 0 && ds_layout_far(longest, 1, longest, G, KH, window, all_below, 0).bytes > budget) return -1;
   bool fit;
-  const int end = ds_range_end(tok0, T, B, x_maxlen, QH, KH, kernel_size, stride, window, all_below, &fit);
+  int end = ds_range_end(tok0, T, B, x_maxlen, G, KH, kernel_size, stride, window, all_below, budget, ds_least(QH), &fit);
+  if (!fit) end = ds_range_end(tok0, T, B, x_maxlen, G, KH, kernel_size, stride, window, all_below, budget, ds_short(QH), &fit);
   return fit ? end : -1;
 }
 
 int nsa_bwd_ds_next(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window) {
   if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || stride <= 0 || tok0 >= T) return T;
   bool fit;
-  const int end = ds_range_end(tok0, T, B, x_maxlen, QH, KH, kernel_size, stride, window, 0, &fit);
+  const int end = ds_range_end(tok0, T, B, x_maxlen, QH / KH, KH, kernel_size, stride, window, 0, ds_budget(), ds_least(QH), &fit);
   return T - end < ds_least(QH) ? T : end;
 }
 
@@ -1181,7 +1190,8 @@ int nsa_cmp_attn_bwd_dkdv_ds(const void* q, int64_t q_st, int64_t q_sh, const vo
   return nsa_dkdv_reduce_cmp_launch(p, add != 0, B, x_maxlen, y_maxlen, D, VD, (hipStream_t)stream);
 }
 
-// The partial results of a ragged batch are mostly address space: slots are numbered by its longest sequence.
+// Slots are numbered by the longest sequence: a ragged batch takes memory for all of them and writes few, so the limit is wider
+// than that of batches that fill theirs.
 static const int64_t SWA_DS_SLOTS_LIMIT = (int64_t)512 << 20;
 
 // length of the longest share of a sequence

@@ -18,7 +18,10 @@ def takes(q, k, v, do, sm_scale, helper=NSAHelper):
 
 def _st(t, row=0):
     """Address of row `row` of t, strides."""
-    return t.data_ptr() + row * t.stride(0) * t.element_size(), t.stride(0), t.stride(1)
+    at = t.data_ptr()
+    if row:
+        at += row * t.stride(0) * t.element_size()
+    return at, t.stride(0), t.stride(1)
 
 
 class _Part:
@@ -41,17 +44,18 @@ class _Part:
         self.y_cu = helper.y_cu_seqlens[b0:b1 + 1] - self.y0
 
     def plan(self, end_of):
+        end = end_of(0, self.T, self.batch, self.x_maxlen)
+        if end == self.T:
+            self.ranges, self.ring = ((0, 0),), 0
+            return True
         self.ranges, at = [], 0
-        while at < self.T:
-            end = end_of(at, self.T, self.batch, self.x_maxlen)
-            if end < 0:
-                return False
+        while 0 < end:
             self.ranges.append((at, end))
-            at = end
-        if len(self.ranges) == 1:
-            self.ranges = [(0, 0)]
-        self.ring = max(e - s for s, e in self.ranges)
-        return True
+            if end == self.T:
+                self.ring = max(e - s for s, e in self.ranges)
+                return True
+            at, end = end, end_of(end, self.T, self.batch, self.x_maxlen)
+        return False
 
 
 def _cut(cu, b0, b1, end_of):
@@ -87,7 +91,7 @@ class DenseDs:
         parts = [_Part(helper, T=T)]
         self.fits = parts[0].plan(end_of)
         host = getattr(helper, "_host_cu", None)
-        if host is not None and helper.batch > 1 and len(parts[0].ranges) != 1:
+        if host is not None and helper.batch > 1 and not (self.fits and parts[0].ring == 0):
             parts = [_Part(helper, *g) for g in _cut(host, 0, helper.batch, end_of)]
             self.fits = all([p.plan(end_of) for p in parts])
         self.ranges = [(p, *r) for p in parts for r in p.ranges] if self.fits else []
@@ -97,7 +101,7 @@ class DenseDs:
         for p in parts:
             sizes = (p.T, p.batch, p.x_maxlen, QH, self.KH)
             if with_cmp:
-                n_cmp = max(n_cmp, *(_lib.value("nsa_cmp_attn_bwd_ds_bytes", *sizes, *cmp_sizes, *r) for r in p.ranges))
+                n_cmp = max([n_cmp] + [_lib.value("nsa_cmp_attn_bwd_ds_bytes", *sizes, *cmp_sizes, *r) for r in p.ranges])
             if with_swa:
                 n_swa = max(n_swa, _lib.value("nsa_swa_bwd_ds_bytes", *sizes, helper.window_size, p.ring))
             if with_swa and all_below:
@@ -115,14 +119,12 @@ class DenseDs:
 
     def dkdv_cmp(self, r, q, k, v, lse, do, delta, sm_scale, dk=None, dv=None):
         """dk, dv of the compressed rows from the queries of range r, added to those of the ranges before (dk, dv)."""
-        p, *r = r
-        h, VD = self.h, v.size(2)
-
-        def sizes(p):
-            return p.batch, p.x_maxlen, p.y_maxlen, self.QH, self.KH, self.D, VD, h.kernel_size, h.stride
-
+        p, tok0, tok1 = r
+        h = self.h
+        shape = (self.QH, self.KH, self.D, v.size(2), h.kernel_size, h.stride)
         if dk is None:
-            self.cmp_slots = max(_lib.value("nsa_cmp_attn_bwd_dkdv_ds_slot_bytes", *sizes(x), *t) for x, *t in self.ranges)
+            self.cmp_slots = max([_lib.value("nsa_cmp_attn_bwd_dkdv_ds_slot_bytes", x.batch, x.x_maxlen, x.y_maxlen, *shape, *t)
+                                  for x, *t in self.ranges])
             shapes = (k.shape, v.shape)
             if self.cmp_slots <= compress_attn.DKDV_SLOTS_LIMIT:
                 dk, dv = (torch.empty(s, device=q.device, dtype=torch.float32) for s in shapes)
@@ -132,38 +134,38 @@ class DenseDs:
         ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
         _lib.call("nsa_cmp_attn_bwd_dkdv_ds", *_st(q, p.x0), *_st(k, p.y0), *_st(v, p.y0), *_st(do, p.x0),
                   lse.data_ptr() + 4 * p.x0 * lse.stride(1), lse.stride(1), lse.stride(0), *_st(delta, p.x0), *_st(dk, p.y0),
-                  *_st(dv, p.y0), p.x_cu.data_ptr(), p.y_cu.data_ptr(), *sizes(p), sm_scale, p.T, *r, *self.cmp, _lib.ptr(ws), n,
-                  int(r[0] > 0), _lib.stream_ptr())
+                  *_st(dv, p.y0), p.x_cu.data_ptr(), p.y_cu.data_ptr(), p.batch, p.x_maxlen, p.y_maxlen, *shape, sm_scale, p.T,
+                  tok0, tok1, *self.cmp, _lib.ptr(ws), n, int(tok0 > 0), _lib.stream_ptr())
         return dk, dv
 
     def dkdv_swa(self, r, q, k, v, lse, do, delta, sm_scale, dk, dv):
         """dk, dv (bf16 or fp32) of the keys of range r."""
-        p, *r = r
+        p, tok0, tok1 = r
         h, x = self.h, p.x0
         sizes = (p.batch, p.x_maxlen, self.QH, self.KH, self.D, v.size(2), h.window_size)
-        n = _lib.value("nsa_swa_bwd_dkdv_ds_ws_bytes", p.T, *sizes, *r)
+        n = _lib.value("nsa_swa_bwd_dkdv_ds_ws_bytes", p.T, *sizes, tok0, tok1)
         ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
         _lib.call("nsa_swa_bwd_dkdv_ds", *_st(q, x), *_st(k, x), *_st(v, x), *_st(do, x), *_st(lse, x), *_st(delta, x), *_st(dk, x),
-                  *_st(dv, x), int(dk.dtype == torch.float32), p.x_cu.data_ptr(), *sizes, sm_scale, p.T, p.ring, *r, *self.swa,
-                  _lib.ptr(ws), n, _lib.stream_ptr())
+                  *_st(dv, x), int(dk.dtype == torch.float32), p.x_cu.data_ptr(), *sizes, sm_scale, p.T, p.ring, tok0, tok1,
+                  *self.swa, _lib.ptr(ws), n, _lib.stream_ptr())
 
     def dkdv_far(self, r, q, k, v, lse, do, delta, sm_scale, dk, dv):
         """slc_attn_bwd_dkdv_before_window for the keys of range r."""
         if not self.far[1]:
             return
-        p, *r = r
+        p, tok0, tok1 = r
         h, x = self.h, p.x0
         _lib.call("nsa_slc_attn_bwd_dkdv_before_window_ds", *_st(q, x), *_st(k, x), *_st(v, x), *_st(do, x), *_st(lse, x),
                   *_st(delta, x), *_st(dk, x), *_st(dv, x), p.x_cu.data_ptr(), p.batch, p.x_maxlen, self.QH, self.KH, self.D,
-                  v.size(2), h.window_size, self.all_below, sm_scale, p.T, p.ring, *r, *self.far, _lib.stream_ptr())
+                  v.size(2), h.window_size, self.all_below, sm_scale, p.T, p.ring, tok0, tok1, *self.far, _lib.stream_ptr())
 
     def dq(self, r, ck, k, VD, sm_scale, dq, mode, partial=None):
         """dq of the tokens of range r from the compressed rows ck and / or the keys k: mode as nsa_attn_bwd_dq_ds."""
-        p, *r = r
+        p, tok0, tok1 = r
         h = self.h
         none = (None, 0, 0)
         _lib.call("nsa_attn_bwd_dq_ds", *(none if ck is None else _st(ck, p.y0)), *self.cmp,
                   *(none if k is None else _st(k, p.x0)), *self.swa, *self.far, *_st(dq, p.x0), mode,
                   *(none if partial is None else _st(partial, p.x0)), p.x_cu.data_ptr(), p.y_cu.data_ptr(), p.batch, p.x_maxlen,
-                  self.QH, self.KH, self.D, VD, h.kernel_size, h.stride, h.window_size, self.all_below, sm_scale, p.T, p.ring, *r,
+                  self.QH, self.KH, self.D, VD, h.kernel_size, h.stride, h.window_size, self.all_below, sm_scale, p.T, p.ring, tok0, tok1,
                   _lib.stream_ptr())

@@ -355,28 +355,37 @@ def test_grid_of_the_storing_dkdv_covers_every_share_of_a_range():
     ([250000], (64, 4), {}), ([1 << 20], (64, 4), {}), ([1 << 20], (8, 1), {}), ([300000, 500], (32, 2), {}),
 ])
 def test_scratch_of_stored_ds_is_bounded(lens, shape, settings):
-    """No branch's dS takes more than its limit of 4 GB, whatever the settings; where a range that fills the GPU would, there
-    are no ranges.  A lower limit holds as well."""
+    """No branch's dS takes more than its limit of 4 GB, whatever the settings, or there are no ranges; up to a million tokens
+    there are.  A lower limit holds as well."""
     from flash_nsa import NSAHelper, _lib
     from flash_nsa.ops import bwd_ds
+    from flash_nsa.utils import BwdNSAHelper
+
+    def batch_of(lens):
+        NSAHelper.init_cu_seqlens(torch.tensor([0, *lens]).cumsum(0).to(torch.int32))
+        return BwdNSAHelper()
+
     T, (QH, KH) = sum(lens), shape
     q, k = torch.empty(T, QH, 128, device="meta"), torch.empty(T, KH, 128, device="meta")
     NSAHelper.set_hyperparameters(**settings)
-    cu = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
-    NSAHelper.init_cu_seqlens(cu)
+    helper = batch_of(lens)
     fitted = 0
     for mb in (4096, 700, 0):
         _lib.call("nsa_set_tuning", b"dense_ds_mb", mb)
         for with_cmp, with_swa in ((True, True), (True, False), (False, True)):
-            ds = bwd_ds.DenseDs(q, k, with_cmp=with_cmp, with_swa=with_swa,
+            ds = bwd_ds.DenseDs(q, k, helper, with_cmp=with_cmp, with_swa=with_swa,
                                 all_below=NSAHelper.all_below() if with_cmp and with_swa else 0)
             if not ds.fits:
-                assert not ds.ranges
+                assert not ds.ranges and (mb < 4096 or settings.get("block_size") == 128)
                 continue
             fitted += 1
             assert max(n for _, n in (ds.cmp, ds.swa, ds.far)) <= mb << 20
             assert (ds.cmp[1] > 0) == with_cmp and (ds.swa[1] > 0) == with_swa
     assert fitted > 0
+    _lib.call("nsa_reset_tuning")
+    # the same for a short batch: a query's dq is to be the same bits whatever follows it
+    short = bwd_ds.DenseDs(q[:500], k[:500], batch_of([500]), all_below=NSAHelper.all_below())
+    assert short.fits == (settings.get("block_size") != 128)
     NSAHelper.set_hyperparameters()
 
 
