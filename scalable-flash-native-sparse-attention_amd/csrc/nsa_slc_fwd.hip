@@ -17,8 +17,8 @@
 // paged queries 5290 / 5170, 16 heads, 4K tokens 185 / 182.
 // With 128 v channels the V rows of all but long sequences do not pass through LDS at all: an instruction fetches the rows whose
 // scores its lanes hold, so the transposition stays inside a lane (UnitColumns128).  LDS moves 16 KB per unit instead of 32 (a
-// quarter of them transposed reads, the slowest).  This kernel, us, through LDS / so: 64 heads of 128, 8 x 6K tokens 3830 / 3330
-// (25 TB/s of requests), 16 x 2K paged queries behind up to 16K 2941 / 2761, one sequence of 4K tokens, 16 heads 105 / 85; 32 heads of
+// quarter of them transposed reads, the slowest).  This kernel, us, through LDS / so: 64 heads of 128, 8 x 6K tokens 3830 / 3180
+// (26 TB/s of requests), 16 x 2K paged queries behind up to 16K 2941 / 2761, one sequence of 4K tokens, 16 heads 105 / 85; 32 heads of
 // 192, 16K tokens 964 / 869.  Outputs are the same bits.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
@@ -301,10 +301,14 @@ int launch_slc(const NsaSlcParams& p, int B, int max_q_len, hipStream_t stream) 
   // Beyond, memory is, and waves that wait for LDS in turn keep more together: 64K tokens with V in registers everywhere have 11 %
   // more L2 misses.  Calls with V in registers below 0 / 6 / infinitely many MB of K and V per head, us, 64 / 4 heads of 128: one
   // sequence of 8K tokens 1072 / 1012 / 1003, 16K 2489 / 2395 / 2354, 24K 4159 / 4074 / 4136, 32K 6168 / 6060 / 6604, 64K 18988 /
-  // 18979 / 19789; paged, 16 x 2K queries behind 2K 4425 / 4295 / 4264, behind 12K 6625 / 6687 / 6998.  192 channels, at two waves per
-  // SIMD, 0 / 6 / 10 MB / all: 16K tokens 1583 / 1532 / 1490 / 1518, 48K 8407 / 8270 / 8325 / 8388, paged, 8 x 2K queries behind 12K
-  // 1945 / 1947 / 1971 / 1966, behind 16K 2235 / 2235 / 2234 / 2432.  64 channels gain nothing (4K to 8K tokens the same to 0.3 %,
-  // 16K 550 -> 567).
+  // 18979 / 19789; paged, 16 x 2K queries behind 2K 4425 / 4295 / 4264, behind 12K 6625 / 6687 / 6998.  64 channels gain nothing (4K
+  // to 8K tokens the same to 0.3 %, 16K 550 -> 567).
+  // 192 channels, with half of the waves in flight: the line is at 10 MB unpaged.  This launch, us, 32 / 2 heads, 6 / 8 / 10 MB:
+  // 12K tokens 544 / 537 / 537, 16K 785 / 774 / 753, 24K 1328 / 1314 / 1313, 48K 4083 / 4075 / 4099, 3 x 16K 2353 / 2294 / 2250; 10 /
+  // 12 / 16 MB: 16K 757 / 753 / 758, 24K 1288 / 1295 / 1303, 32K 2033 / 2047 / 2084, 48K 4028 / 4029 / 4096.  64 / 4 heads, 6 / 8 / 10:
+  // 16K 1566 / 1543 / 1515, 32K 4026 / 3995 / 3996, 2 x 24K 5381 / 5263 / 5180; 10 / 12 / 16: 24K 2621 / 2648 / 2666, 32K 4004 / 4058 /
+  // 4112, 48K 8200 / 8230 / 8310.  Paged, whole calls, 0 / 6 / 10 MB / all, 8 x 2K queries behind 12K 1945 / 1947 / 1971 / 1966, behind
+  // 16K 2235 / 2235 / 2234 / 2432.
   p2.reg_below = ((D > 128 && !PAGED ? 10 : 6) << 20) / ((D + VD) * 2);
   slc_fwd_kernel<D, VD, PAGED><<<grid, 256, 0, stream>>>(p2);
   return nsa_check_launch("slc_fwd_kernel");

@@ -40,7 +40,7 @@ def cmp_attn_bwd(q, k, v, o, lse, do, dq=None, dkdv_repeat=False, sm_scale=None,
     finalize_dq): a tensor of q's dtype and n; that sum is for the queries at positions below n stored there, for the others
     kept in the buffer.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None); "both" forms dq from the dS that the dk / dv
-    kernel leaves behind where the shapes have that path (bwd_ds).
+    kernel leaves behind where the shapes have that path (bwd_ds: up to 4 GB of scratch).
     dk, dv: fp32 [y_len,KH,*].  Every work item (query chunk of a key tile) stores its partial result into its own slot
     of a scratch buffer and a second launch sums the slots in a fixed order -- bit-identical results across runs.
     Where the slots would take more than DKDV_SLOTS_LIMIT bytes and neither dkdv_repeat nor

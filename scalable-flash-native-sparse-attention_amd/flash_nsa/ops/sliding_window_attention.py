@@ -77,7 +77,7 @@ def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq
     not fill the GPU, partial results added in a fixed order (up to 64 MB of scratch) -- bit-identical across runs.
     parts = "dq" / "dkdv" launches only that kernel (the other results are None), so that a caller can put the
     two on different streams; "both" forms dq from the dS that the dk / dv kernel leaves behind where the shapes have that
-    path (bwd_ds)."""
+    path (bwd_ds: up to 4 GB of scratch for the dS and 512 MB for partial results)."""
     check_thd(do, "do")
     T, QH, D = q.shape
     _, KH, VD = v.shape
