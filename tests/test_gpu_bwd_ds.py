@@ -36,6 +36,11 @@ CASES = [
     (32, 2, 128, 128, [3063, 9859], 200, True, {}),
     # the keys before the window in places taken in turn
     (64, 1, 128, 128, [1100, 1024, 1300, 1111, 1029], 500, True, dict(window_size=100)),
+    # ranges of an eighth of the tokens that fill the GPU
+    (64, 4, 128, 128, [4700], 80, False, {}),
+    (8, 1, 128, 128, [9001], 28, False, {}),
+    (64, 1, 128, 128, [2047, 300, 2500, 5], 80, True, dict(top_n=6)),
+    (64, 4, 192, 128, [130, 4300], 150, True, dict(window_size=300)),
     # a long sequence between many short ones
     (64, 4, 128, 128, [40, 0, 350, 5, 350, 350, 4500, 33, 350, 350, 0, 350, 31], 300, False, {}),
 ]
