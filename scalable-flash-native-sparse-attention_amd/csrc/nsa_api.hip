@@ -1015,7 +1015,7 @@ DsLayout ds_layout_far(int T, int B, int x_maxlen, int G, int KH, int window, in
   const int end = all_below < x_maxlen ? all_below : x_maxlen;
   if ((int64_t)end - 1 - window - 1 < 0) return DsLayout{0, 0, 0, 0, 0};
   const int pitch = (end - 1 - window - 1) / 32 + 1;
-  const int seq_tiles = (end * G + 63) / 64;
+  const int seq_tiles = (int)(((int64_t)end * G + 63) / 64);
   const int64_t tiles = ds_ring_tiles(T, B, G, ring, end);
   if ((int64_t)seq_tiles * B < tiles) return ds_layout((int64_t)seq_tiles * B, seq_tiles, pitch, KH);
   return ds_layout(tiles, 0, pitch, KH);
@@ -1106,12 +1106,12 @@ static int ds_short(int QH) { return (16384 / QH + 127) & ~127; }
 int nsa_bwd_ds_range_end(int tok0, int T, int B, int x_maxlen, int QH, int KH, int kernel_size, int stride, int window,
                          int all_below) {
   if (T <= 0 || B <= 0 || KH <= 0 || QH < KH || tok0 < 0 || tok0 >= T) return T;
-  const int G = QH / KH, longest = 1 << 28;
+  const int G = QH / KH, longest = 1 << 24;
   const int64_t budget = ds_budget();
   // What decides whether dq comes from stored dS is not the number of tokens: a query's dq is to be the same bits whatever follows
   // it in the batch.  So where top_n * block_size is too far beyond the window for one sequence of so many tokens, there is none
-  // for a shorter one either.  (Sequences past a million tokens, for the compressed branch, and past a window of many thousand
-  // keys, which has to be the longest sequence's in a batch of shorter ones, have none.)
+  // for a shorter one either.  (Two exceptions: sequences past a million tokens, and windows of many thousand keys, which act as
+  // the longest sequence's where that is shorter.)
   if (window >= 0 && ds_layout_far(longest, 1, longest, G, KH, window, all_below, 0).bytes > budget) return -1;
   bool fit;
   int end = ds_range_end(tok0, T, B, x_maxlen, G, KH, kernel_size, stride, window, all_below, budget, ds_least(QH), &fit);

@@ -384,6 +384,8 @@ def test_scratch_of_stored_ds_is_bounded(lens, shape, settings):
     assert fitted > 0
     _lib.call("nsa_reset_tuning")
     # the same for a short batch: a query's dq is to be the same bits whatever follows it
+    assert _lib.value("nsa_bwd_ds_range_end", 0, 500, 1, 500, QH, KH, 32, 16, 512, 2 ** 31 - 64) == -1
+    assert _lib.value("nsa_bwd_ds_range_end", 0, 500, 1, 500, QH, KH, 32, 16, 2 ** 31 - 1, 2 ** 31 - 64) == 500
     short = bwd_ds.DenseDs(q[:500], k[:500], batch_of([500]), all_below=NSAHelper.all_below())
     assert short.fits == (settings.get("block_size") != 128)
     NSAHelper.set_hyperparameters()
