@@ -28,18 +28,18 @@ class _Part:
     """Sequences b0 .. b1 - 1 of a batch as a batch of their own: its first token x0 and compressed row y0, lengths, offsets from
     there on, and the ranges of its T tokens (one range: (0, 0)), `ring` tokens the longest of them (one range: 0)."""
 
-    def __init__(self, helper, b0=0, b1=None, T=0):
+    def __init__(self, helper, T, b0=0, b1=None):
         b1 = helper.batch if b1 is None else b1
-        self.batch = b1 - b0
+        self.batch, self.T = b1 - b0, T
         if self.batch == helper.batch:
             self.x0 = self.y0 = 0
-            self.T, self.x_maxlen, self.y_maxlen = T, helper.x_maxlen, helper.y_maxlen
+            self.x_maxlen, self.y_maxlen = helper.x_maxlen, helper.y_maxlen
             self.x_cu, self.y_cu = helper.x_cu_seqlens, helper.y_cu_seqlens
             return
         lens = [e - s for s, e in zip(helper._host_cu, helper._host_cu[1:])]
         y = [max((n - helper.kernel_size) // helper.stride + 1, 0) for n in lens[:b1]]
         self.x0, self.y0 = sum(lens[:b0]), sum(y[:b0])
-        self.T, self.x_maxlen, self.y_maxlen = sum(lens[b0:b1]), max(lens[b0:b1]), max(y[b0:b1])
+        self.x_maxlen, self.y_maxlen = max(lens[b0:b1]), max(y[b0:b1])
         self.x_cu = helper.x_cu_seqlens[b0:b1 + 1] - self.x0
         self.y_cu = helper.y_cu_seqlens[b0:b1 + 1] - self.y0
 
@@ -88,11 +88,11 @@ class DenseDs:
         def end_of(at, T, batch, longest):
             return _lib.value("nsa_bwd_ds_range_end", at, T, batch, longest, QH, self.KH, *branches)
 
-        parts = [_Part(helper, T=T)]
+        parts = [_Part(helper, T)]
         self.fits = parts[0].plan(end_of)
         host = getattr(helper, "_host_cu", None)
         if host is not None and helper.batch > 1 and not (self.fits and parts[0].ring == 0):
-            parts = [_Part(helper, *g) for g in _cut(host, 0, helper.batch, end_of)]
+            parts = [_Part(helper, host[e] - host[b], b, e) for b, e in _cut(host, 0, helper.batch, end_of)]
             self.fits = all([p.plan(end_of) for p in parts])
         self.ranges = [(p, *r) for p in parts for r in p.ranges] if self.fits else []
         if not self.fits:

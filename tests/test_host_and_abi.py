@@ -391,11 +391,12 @@ def test_scratch_of_stored_ds_is_bounded(lens, shape, settings):
     NSAHelper.set_hyperparameters()
 
 
-@pytest.mark.parametrize("lens,most", [
-    ([60000] + [350] * 400, 8), ([350] * 200 + [60000] + [350] * 200, 9), ([16384] + [512] * 96, 3), ([20480] * 2, 2),
-    ([12288] * 10, 4), ([1000] * 100, 2), ([0, 60000, 0, 0, 31, 500, 0], 7), ([65536], 6), ([300] * 20, 1),
+@pytest.mark.parametrize("lens,behind,most", [
+    ([60000] + [350] * 400, 0, 8), ([350] * 200 + [60000] + [350] * 200, 7, 9), ([16384] + [512] * 96, 0, 3), ([20480] * 2, 0, 2),
+    ([12288] * 10, 0, 4), ([1000] * 100, 0, 2), ([0, 60000, 0, 0, 31, 500, 0], 0, 7), ([65536], 0, 6), ([300] * 20, 0, 1),
+    ([1000] * 50, 50000, 1),  # rows of q behind the last sequence
 ])
-def test_parts_of_a_batch_whose_stored_ds_takes_several_ranges(lens, most):
+def test_parts_of_a_batch_whose_stored_ds_takes_several_ranges(lens, behind, most):
     """A batch that one range does not hold is cut between its sequences, so that short ones do not get the width of the longest:
     every token in one part, in order; several ranges in parts of one sequence alone."""
     from flash_nsa import NSAHelper
@@ -404,7 +405,7 @@ def test_parts_of_a_batch_whose_stored_ds_takes_several_ranges(lens, most):
     NSAHelper.set_hyperparameters()
     cu = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
     NSAHelper.init_cu_seqlens(cu)
-    ds = bwd_ds.DenseDs(torch.empty(T, QH, 128, device="meta"), torch.empty(T, KH, 128, device="meta"),
+    ds = bwd_ds.DenseDs(torch.empty(T + behind, QH, 128, device="meta"), torch.empty(T + behind, KH, 128, device="meta"),
                         all_below=NSAHelper.all_below())
     assert ds.fits and len(ds.ranges) <= most
     parts = list(dict.fromkeys(p for p, *_ in ds.ranges))
