@@ -64,8 +64,10 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int l32 = lane & 31;
   const int hl = lane >> 5;
   const int g16 = lane >> 4, i16 = lane & 15;
-  const int b = blockIdx.y;
-  const int kh = blockIdx.z;
+  // (sequences and heads take turns on the XCDs, whose workgroups come round robin)
+  const int seq_head = (blockIdx.x + blockIdx.y) % gridDim.x;
+  const int b = p.last_first ? seq_head / p.KH : blockIdx.y;
+  const int kh = p.last_first ? seq_head % p.KH : blockIdx.z;
   const int G = p.G;
 
   const int x0 = p.x_cu[b];
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int ctx = PAGED ? p.ctx_lens[b] : xl;
   const int qoff = ctx - xl;
   const int rows_total = xl * G;
-  const int r0 = (p.last_first ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * ROWS_WG;
+  const int r0 = (p.last_first ? gridDim.y - 1 - blockIdx.y : blockIdx.x) * ROWS_WG;
   if (r0 >= rows_total) return;
   int nkeys, kbase = 0;
   if (MODE == MODE_CMP) {
@@ -563,11 +565,18 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   if (B <= 0 || max_q_len <= 0) return NSA_OK;
   NsaFwdTileParams p = p0;
   // Queries that select everything see 1 to 24 tiles of keys, the last rows of a short prompt the most: in a launch of few
-  // rounds of workgroups these go first.  Paged, 64 / 4 heads of 128, us, first / last rows first: 3 prompts of 60 to 700 tokens
-  // 73.5 / 72.5, 2 of 300 to 900 75.3 / 70.7, 6 of 60 to 1000 129.8 / 127.1, 12 252.0 / 252.5; one sequence of 4K tokens 159.4 /
-  // 163.9.
-  p.last_first = MODE == MODE_TAIL && max_q_len <= p.all_below &&
-                 (int64_t)cdiv_i(max_q_len * p.G, 128) * B * p.KH <= 16 * nsa_device_cus();
+  // rounds of workgroups the last rows of all sequences and heads go first, so that the longest workgroups start together, on a
+  // CU each, and the short ones fill up.  (Last rows first within each sequence and head: the first rows of the second head met
+  // those of the first on the same CUs while other CUs had one workgroup.)  Whole calls, that / so, us, 64 / 4 heads of 128: 3
+  // prompts of 60 to 700 tokens 79 / 65, 2 of 300 to 900 78 / 68, 6 of 60 to 1000 134 / 125, 16 x 128 to 256 behind up to 256 107 /
+  // 105; forward of 1000 tokens 78 / 69, 1500 160 / 144, 4096 526 / 520; 16 / 2 heads of 64, 20 samples of up to 1100 138 / 124.
+  // Launches of more workgroups take them in the order of their rows, which keeps neighbours' keys in L2 (8 x 6K tokens 18.4 /
+  // 18.7 ms, 16 x 2K paged rows 5.21 / 5.25), short ones from twice as many on: 40 samples of 17 to 1200 218 / 203, 12 prompts
+  // of 60 to 1000 253 / 249.  The compressed branch gains nothing (1500 tokens 205 / 203, 4 x 300 to 1500 156 / 160).
+  const int64_t wgs = (int64_t)cdiv_i(max_q_len * p.G, 128) * B * p.KH;
+  p.last_first = MODE == MODE_TAIL && wgs <= (max_q_len / 2 <= p.all_below ? 32 : 16) * nsa_device_cus();
+  const int tiles = cdiv_i(max_q_len * p.G, 128);
+  const dim3 grid = p.last_first ? dim3(B * p.KH, tiles) : dim3(tiles, B, p.KH);
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there; the window
   // branch, with its short key loops, is level with register staging) and for 192 channels everywhere: two of its unpadded
   // tile buffers fill half of a CU's LDS, two padded ones more than that, which leaves one workgroup on a CU.  32 heads of 192,
@@ -579,11 +588,9 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   const bool async = narrow && (variant == 4 || (variant == 0 && ((MODE == MODE_CMP && pow2) || D == 192)));
   if constexpr (D > 192 || VD > 128) {
     // head dims of 256: the output accumulators alone take 128 registers, one workgroup per CU
-    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 1, false><<<grid, 256, 0, stream>>>(p);
     return nsa_check_launch("fwd_tile_kernel");
   } else if constexpr (MODE == MODE_TAIL) {
-    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     if constexpr (D == 192) {
       if (variant != 1 && narrow) {
         fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, true><<<grid, 256, 0, stream>>>(p);
@@ -592,16 +599,12 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
     }
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, false><<<grid, 256, 0, stream>>>(p);
   } else if (variant == 2) {
-    dim3 grid(cdiv_i(max_q_len * p.G, 256), B, p.KH);
-    fwd_tile_kernel<D, VD, MODE, PAGED, 2, 1, false><<<grid, 256, 0, stream>>>(p);
+    fwd_tile_kernel<D, VD, MODE, PAGED, 2, 1, false><<<dim3(cdiv_i(max_q_len * p.G, 256), B, p.KH), 256, 0, stream>>>(p);
   } else if (variant == 3) {
-    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 1, false><<<grid, 256, 0, stream>>>(p);
   } else if (async) {
-    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, true><<<grid, 256, 0, stream>>>(p);
   } else {
-    dim3 grid(cdiv_i(max_q_len * p.G, 128), B, p.KH);
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, false><<<grid, 256, 0, stream>>>(p);
   }
   return nsa_check_launch("fwd_tile_kernel");

@@ -363,3 +363,24 @@ def test_row_strides_that_a_32_bit_offset_does_not_hold(device, D):
         del wide
     torch.cuda.empty_cache()
     setup_helper(make_cu([64]).to(device))
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens", [
+    (8, 2, 64, 64, [1100, 1, 0, 17, 700, 1040, 513]),
+    (12, 3, 128, 128, [129, 640, 31]),                 # a row tile of 128 holds parts of tokens; odd number of kv heads
+    (16, 1, 192, 128, [300, 33]),
+])
+def test_window_launch_of_few_workgroups_takes_last_rows_first(device, QH, KH, D, VD, lens):
+    """The order of the workgroups changes no bit: sequences among so many others that the launch goes by rows equal the same
+    sequences in a launch that starts with the last rows of all of them, and each alone."""
+    from flash_nsa import NSAConfig, NSACore
+    many = lens + [max(lens)] + [3] * (8192 * 128 // (max(lens) * QH) + 1)  # more than 8192 workgroups, most of them empty
+    q, k, v, w = [t.to(device) for t in make_qkvw(sum(many), QH, KH, D, VD, seed=73)]
+    core = NSACore(NSAConfig(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH))
+    with torch.no_grad():
+        want = core(q, k, v, w, make_cu(many).to(device))
+        n = sum(lens)
+        got = core(q[:n], k[:n], v[:n], w[:n], make_cu(lens).to(device))
+        assert torch.equal(got, want[:n])
+        first = lens[0]
+        assert torch.equal(core(q[:first], k[:first], v[:first], w[:first], make_cu([first]).to(device)), want[:first])
