@@ -2,6 +2,7 @@
 across the three branches and optional recomputation of saved activations
 (mirrors the interface of upstream flash_nsa/modules/megatron_level_nsa.py:46-159, 386-545; the
 context-parallel function of that file is outside this single-GPU build)."""
+import contextlib
 import math
 
 import torch
@@ -26,15 +27,33 @@ from ..ops.sliding_window_attention import (slc_fwd_first_queries, swa_fwd, swa_
 # gain nor lose (64K tokens 55.0 ms either way); the same split of the forward gained nothing.
 # Setting this module attribute to False puts everything back on the caller's stream.
 OVERLAP_STREAMS = True
+# Work that passes between two streams costs the host 70 us of events, waits and first launches, and the GPU as much again, which
+# small batches wait for.  Their second stream is the caller's: those whose tokens x q-heads x longest sequence (at most 2048: the
+# window and the selected blocks end there) x channels (128 on top, for what does not grow with them) stay below this.  Whole
+# steps on two streams / on one, us (this number, 1e9): 64 heads of 128, 1024 tokens 741 / 471 (26), 1300 824 / 583 (42), 1600 839 /
+# 697 (63; mean compression 625 / 602), 2048 811 / 818 (103), 6 x 100 to 600 681 / 464 (21), 12 x 673 / 682 (54), 8 x 100 to 700
+# 789 / 777 (69); 16 heads, 4096 771 / 661 (52), 5000 835 / 788 (63; mean 692 / 736), 6000 844 / 871 (76), 8 x 100 to 1500 809 / 712
+# (68); 32 heads of 192, 1024 744 / 444 (15), 2048 779 / 761 (60), 2500 848 / 892 (73); 16 heads of 64, 5000 804 / 627 (42), 6500 772
+# / 743 (55), 8192 836 / 868 (69), 20 x 200 to 1000 710 / 598 (46), 40 of up to 1200 948 / 1122 (133).
+OVERLAP_FROM = 6e10
 _side_streams = {}
 
 
-def _side_stream(device):
+def _side_stream(main, q, v, helper):
+    """The second stream of this batch's backward beside the caller's, main."""
+    T, QH, D = q.shape
+    if T * QH * min(helper.x_maxlen, 2048) * (D + v.size(-1) + 128) < OVERLAP_FROM:
+        return main
+    device = q.device
     key = device.index if device.index is not None else torch.cuda.current_device()
     s = _side_streams.get(key)
     if s is None:
         s = _side_streams[key] = torch.cuda.Stream(device=device)
     return s
+
+
+def _on(side, main):
+    return torch.cuda.stream(side) if side is not main else contextlib.nullcontext()
 
 
 def weight_grad(inp, grad_out, weight):
@@ -131,14 +150,15 @@ def bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, l
 
     if OVERLAP_STREAMS and len(ds.ranges) == 1:
         # the compressed dk / dv next to the window's, the dense dq next to the selected dk / dv
-        main, side, r = torch.cuda.current_stream(), _side_stream(q.device), ds.ranges[0]
+        main, r = torch.cuda.current_stream(), ds.ranges[0]
+        side = _side_stream(main, q, v, helper)
         side.wait_stream(main)
-        with torch.cuda.stream(side):
+        with _on(side, main):
             dcmp_k, dcmp_v = dkdv_cmp(r)
         dkdv_raw(r)
-        window_done = main.record_event()
-        with torch.cuda.stream(side):
-            side.wait_event(window_done)
+        window_done = main.record_event() if side is not main else None
+        with _on(side, main):
+            wait_for(window_done)
             dense_dq(r)
         dcmp_k.record_stream(main)
         dcmp_v.record_stream(main)
@@ -253,20 +273,20 @@ class NSAFunction(torch.autograd.Function):
         if OVERLAP_STREAMS and stored_ds:
             # the dense dq kernels next to the dk / dv passes whose dS the selected dq waits for, the compressed dk / dv
             # next to the selected dq
-            side = _side_stream(q.device)
+            side = _side_stream(main, q, v, helper)
             side.wait_stream(main)
-            with torch.cuda.stream(side):
+            with _on(side, main):
                 dq = dq_chain()
-                dense_dq = side.record_event()
+                dense_dq = side.record_event() if side is not main else None
                 dcmp_k, dcmp_v = dkdv_cmp()
                 dcmp_k.record_stream(main)
                 dcmp_v.record_stream(main)
             dk, dv = dkdv_raw(dense_dq)
             main.wait_stream(side)
         elif OVERLAP_STREAMS:
-            side = _side_stream(q.device)
+            side = _side_stream(main, q, v, helper)
             side.wait_stream(main)
-            with torch.cuda.stream(side):
+            with _on(side, main):
                 dq = dq_chain()
                 dq.record_stream(main)
             # dk/dv kernels on the caller's stream.  The compressed branch (matrix bound) goes first, next to the selected
