@@ -47,6 +47,32 @@ int nsa_construct_block_bwd(const void* dblock, void* dx, int64_t dx_st, int64_t
 int nsa_glu_fwd(const void* x, void* y, int64_t N, int d, int act, void* stream);
 int nsa_glu_bwd(const void* x, const void* dy, void* dx, int64_t N, int d, int act, void* stream);
 
+/* Learned compression without the windows in memory (flash_nsa/modules/megatron_level_nsa.py:46-86: construct_block, the
+ * product with the weight and the activation).  w [N, kernel*D] with row stride w_st and contiguous columns; hidden [y_len,H,N]
+ * contiguous = windows w^T in bf16; act -1: no activation, N = D; 0 / 1 as nsa_glu_fwd, N = 2D, out [y_len,H,D] = its activation, hidden
+ * may be null. */
+int nsa_compress_linear_fwd(const void* x, int64_t x_st, int64_t x_sh, const void* w, int64_t w_st, void* hidden, void* out,
+                            const int32_t* x_cu, const int32_t* y_cu, int B, int y_maxlen, int H, int D, int kernel_size,
+                            int stride, int N, int act, void* stream);
+/* Its gradient with respect to x, from that of hidden: added to the fp32 dx, or, with dst, dst = bf16(dx + it) for every token
+ * (dx is then only read; null: zeros). */
+int nsa_compress_linear_bwd_dx(const void* dhidden, const void* w, int64_t w_st, void* dx, int64_t dx_st, int64_t dx_sh, void* dst,
+                               int64_t dst_st, int64_t dst_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen,
+                               int H, int D, int kernel_size, int stride, int N, void* stream);
+/* Its gradient with respect to w, summed in a fixed order: dw [N, kernel*D] contiguous, bf16 (stored) or fp32 (added to).
+ * y_len = y_cu[B] > 0. */
+int64_t nsa_compress_linear_bwd_dw_ws_bytes(int64_t y_len, int H, int D, int kernel_size, int N);
+int nsa_compress_linear_bwd_dw(const void* dhidden, const void* x, int64_t x_st, int64_t x_sh, void* dw, int dw_is_f32,
+                               const int32_t* x_cu, const int32_t* y_cu, int B, int64_t y_len, int H, int D, int kernel_size,
+                               int stride, int N, void* ws, int64_t ws_bytes, void* stream);
+
+/* dhidden [rows, N] (bf16) from the fp32 dy [rows, D], which is rounded to bf16 first; act as above (-1: dhidden = bf16(dy)). */
+int nsa_compress_act_bwd(const void* hidden, const void* dy, void* dhidden, int64_t rows, int D, int act, void* stream);
+/* nsa_mean_pool_bwd from the fp32 dy [y_len,H,D] (contiguous, rounded to bf16 first): dst = bf16(dx + it), dx fp32. */
+int nsa_mean_pool_bwd_sum(const void* dy, const void* dx, int64_t dx_st, int64_t dx_sh, void* dst, int64_t dst_st, int64_t dst_sh,
+                          const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int H, int D, int kernel_size, int stride,
+                          void* stream);
+
 /* flash_nsa/ops/combine.py:114-144 combine_fwd */
 int nsa_combine_fwd(const void* a, const void* b, const void* c, int64_t i_st, int64_t i_sh, const void* w,
                     int64_t w_st, int64_t w_sh, void* o, int64_t o_st, int64_t o_sh, int64_t T, int H, int D,

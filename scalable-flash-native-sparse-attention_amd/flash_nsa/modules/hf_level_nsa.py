@@ -5,7 +5,7 @@ import torch
 
 from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
-from ..ops.compress_kv import construct_block, mean_pooling
+from ..ops.compress_kv import compress_linear, construct_block, mean_pooling, takes_weight
 from ..ops.compress_attn import compress_attn
 from ..ops.select_attn import select_attn
 from ..ops.topk import slc_topk_indices
@@ -14,6 +14,11 @@ from ..ops.combine import fused_sigmoid_combine
 from ..ops.sliding_window_attention import swa_varlen_func
 
 _METHODS = ("mean", "sigmoid-mul", "swiglu", "linear")
+
+
+def _hooked(module):
+    return (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
+            "forward" in module.__dict__)
 
 
 class CompressKV(torch.nn.Module):
@@ -34,6 +39,10 @@ class CompressKV(torch.nn.Module):
     def forward(self, x):
         if self.version == "mean":
             return mean_pooling(x)
+        # a plain fc is computed with the windows where they lie; one that has been replaced, wrapped or hooked is called
+        if type(self.fc) is torch.nn.Linear and self.fc.bias is None and not _hooked(self.fc) and \
+                x.dim() == 3 and takes_weight(x, self.fc.weight, self.version):
+            return compress_linear(x, self.fc.weight, self.version)
         windows = construct_block(x)                    # [y_len, H, kernel, D]
         hidden = self.fc(windows.flatten(-2, -1))        # flatten order: (position in window, channel)
         if self.version == "linear":

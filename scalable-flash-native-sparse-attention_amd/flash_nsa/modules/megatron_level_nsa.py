@@ -10,7 +10,8 @@ import torch
 from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
 from ..ops._common import thd_rows
-from ..ops.compress_kv import construct_block_fwd, construct_block_bwd, mean_pooling_fwd, mean_pooling_bwd
+from ..ops.compress_kv import (compress_linear_fwd, compress_linear_bwd, construct_block_fwd, construct_block_bwd, mean_pooling_fwd,
+                               mean_pooling_bwd_sum, takes_weight)
 from ..ops import bwd_ds
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
 from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window,
@@ -66,16 +67,22 @@ def weight_grad(inp, grad_out, weight):
     # bf16 operands, fp32 accumulator added to the fp32 buffer in the GEMM's epilogue: no rounding of dW to bf16
     # (upstream's wgrad GEMM adds its fp32 accumulator tiles the same way, flash_nsa/ops/gemm.py:131-133)
     torch.addmm(main_grad, grad_out.t(), inp, out_dtype=torch.float32, out=main_grad)
+    return _added_to_main_grad(weight, inp)
+
+
+def _added_to_main_grad(weight, like):
     if hasattr(weight, "grad_added_to_main_grad"):
         weight.grad_added_to_main_grad = True
-        return torch.empty(main_grad.shape, dtype=inp.dtype, device=inp.device)
+        return torch.empty(weight.main_grad.shape, dtype=like.dtype, device=like.device)
     return None
 
 
-def compress_kv_fwd(x, weight, version, helper=NSAHelper):
-    """-> (windows or None, pre-activation or None, compressed rows)"""
+def compress_kv_fwd(x, weight, version, helper=NSAHelper, keep=True):
+    """-> (windows or None, pre-activation or None, compressed rows); keep=False: only the rows are asked for"""
     if version == "mean":
         return None, None, mean_pooling_fwd(x, helper=helper)
+    if takes_weight(x, weight, version, helper):
+        return (None, *compress_linear_fwd(x, weight, version, helper, keep))
     windows = construct_block_fwd(x, helper=helper)
     hidden = torch.matmul(windows.flatten(-2, -1), weight.t())
     if version == "linear":
@@ -89,12 +96,19 @@ def compress_kv_fwd(x, weight, version, helper=NSAHelper):
     return windows, hidden, out
 
 
-def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelper, async_dw=False):
-    """Adds the compression gradient into the fp32 buffer dx and returns (dx, dW or a thunk computing it)."""
-    dout = dout.to(x.dtype)
+def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelper):
+    """-> (bf16 sum of the compression gradient and the fp32 buffer dx, which may be overwritten, dW); dout: fp32."""
     if version == "mean":
-        mean_pooling_bwd(x, dout, dx, helper=helper)
-        return dx, None
+        return mean_pooling_bwd_sum(x, dout, dx, helper), None
+    if windows is None:
+        main_grad = getattr(weight, "main_grad", None)
+        if main_grad is not None and (main_grad.dtype != torch.float32 or main_grad.shape != weight.shape or
+                                      main_grad.device != x.device or not main_grad.is_contiguous()):
+            windows = construct_block_fwd(x, helper=helper)
+        else:
+            dx, dw = compress_linear_bwd(x, weight, hidden, dout, dx, version, main_grad, helper)
+            return dx, dw if main_grad is None else _added_to_main_grad(weight, x)
+    dout = dout.to(x.dtype)
     if version == "linear":
         dhidden = dout
     elif version == "sigmoid-mul":
@@ -103,11 +117,7 @@ def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHel
         dhidden = swiglu_bwd(hidden, dout, inplace=False)
     dwindows = torch.matmul(dhidden, weight).view(*windows.shape)
     construct_block_bwd(x, dwindows, dx, helper=helper)
-
-    def dw_fn():
-        return weight_grad(windows.flatten(-2, -1), dhidden, weight)
-
-    return dx, (dw_fn if async_dw else dw_fn())
+    return dx.to(x.dtype), weight_grad(windows.flatten(-2, -1), dhidden, weight)
 
 
 def slc_swa_fwd(q, k, v, topk, sm_scale, helper, cmp_o=None, w=None, store=True):
@@ -181,8 +191,8 @@ class NSAFunction(torch.autograd.Function):
         if sm_scale is None:
             sm_scale = q.size(-1) ** -0.5
         H = NSAHelper
-        win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, H.cmp_k_method)
-        win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method)
+        win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, H.cmp_k_method, keep=for_backward)
+        win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method, keep=for_backward)
         cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
         topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=H.all_below())
         (slc_o, slc_lse), (swa_o, swa_lse), out = slc_swa_fwd(q, k, v, topk, sm_scale, H, cmp_o, combine_weight,
@@ -239,8 +249,8 @@ class NSAFunction(torch.autograd.Function):
             if ds.fits:
                 dq, dk, dv, dcmp_k, dcmp_v = bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa,
                                                          delta, ds_tokens, sm_scale, helper)
-                _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
-                _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+                dk, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+                dv, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
                 return dq, dk, dv, dw, dwk, dwv, None, None
 
         # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
@@ -299,8 +309,8 @@ class NSAFunction(torch.autograd.Function):
             dq = dq_chain()
             dk, dv = dkdv_raw()
             dcmp_k, dcmp_v = dkdv_cmp()
-        _, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
-        _, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+        dk, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+        dv, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
         if OVERLAP_STREAMS and not stored_ds:
             main.wait_stream(side)
         return dq, dk, dv, dw, dwk, dwv, None, None

@@ -5,6 +5,7 @@ import torch
 from .. import _lib
 from ..utils import NSAHelper
 from ._common import check_thd
+from .act import _glu_bwd
 
 
 def mean_pooling_fwd(x, helper=NSAHelper):
@@ -61,6 +62,80 @@ def construct_block_bwd(x, dy, dx=None, helper=NSAHelper):
     return dx
 
 
+_ACT = {"linear": -1, "sigmoid-mul": 0, "swiglu": 1}
+
+
+def takes_weight(x, weight, version, helper=NSAHelper):
+    """Whether the kernels below take this weight (others go through the windows and the library's products)."""
+    D, N = x.size(-1), (1 if version == "linear" else 2) * x.size(-1)
+    return (D % 32 == 0 and x.is_cuda and weight.device == x.device and x.dtype == weight.dtype == torch.bfloat16
+            and weight.shape == (N, helper.kernel_size * D) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
+            and weight.data_ptr() % 16 == 0)
+
+
+def compress_linear_fwd(x, weight, version, helper=NSAHelper, keep=True):
+    """x [T,H,D], weight [N, kernel*D] -> hidden [y_len,H,N], the product of the windows and the weight, and the compressed rows
+    [y_len,H,D], its activation ("linear": itself).  keep=False: nobody asks for hidden."""
+    check_thd(x, "x")
+    H, D = x.shape[1:]
+    N, act = weight.size(0), _ACT[version]
+    hidden = torch.empty(helper.y_len, H, N, device=x.device, dtype=x.dtype) if keep or act < 0 else None
+    out = hidden if act < 0 else torch.empty(helper.y_len, H, D, device=x.device, dtype=x.dtype)
+    _lib.call("nsa_compress_linear_fwd", x.data_ptr(), x.stride(0), x.stride(1), weight.data_ptr(), weight.stride(0),
+              _lib.ptr(hidden), out.data_ptr(), helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), helper.batch,
+              helper.y_maxlen, H, D, helper.kernel_size, helper.stride, N, act, _lib.stream_ptr())
+    return hidden, out
+
+
+def compress_linear_bwd_x(x, weight, dhidden, dx=None, helper=NSAHelper):
+    """The gradient with respect to x, added to the fp32 dx, if given, in bf16."""
+    T, H, D = x.shape
+    dst = torch.empty(T, H, D, device=x.device, dtype=x.dtype)
+    dxs = (None, 0, 0) if dx is None else (dx.data_ptr(), dx.stride(0), dx.stride(1))
+    _lib.call("nsa_compress_linear_bwd_dx", dhidden.data_ptr(), weight.data_ptr(), weight.stride(0), *dxs, dst.data_ptr(),
+              dst.stride(0), dst.stride(1), helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), helper.batch,
+              helper.x_maxlen, H, D, helper.kernel_size, helper.stride, weight.size(0), _lib.stream_ptr())
+    return dst
+
+
+def compress_linear_bwd_weight(x, weight, dhidden, dw=None, helper=NSAHelper):
+    """dW in a new bf16 tensor, or added to the fp32 dw."""
+    H, D = x.shape[1:]
+    N, f32 = weight.size(0), dw is not None
+    if not helper.y_len:
+        return dw if f32 else torch.zeros(weight.shape, device=x.device, dtype=x.dtype)
+    if not f32:
+        dw = torch.empty(weight.shape, device=x.device, dtype=x.dtype)
+    n = _lib.value("nsa_compress_linear_bwd_dw_ws_bytes", helper.y_len, H, D, helper.kernel_size, N)
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    _lib.call("nsa_compress_linear_bwd_dw", dhidden.data_ptr(), x.data_ptr(), x.stride(0), x.stride(1), dw.data_ptr(), int(f32),
+              helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), helper.batch, helper.y_len, H, D,
+              helper.kernel_size, helper.stride, N, ws.data_ptr(), n, _lib.stream_ptr())
+    return dw
+
+
+def compress_linear_bwd(x, weight, hidden, dout, dx, version, dw=None, helper=NSAHelper):
+    """From the fp32 gradient dout of the compressed rows: (the bf16 sum of the fp32 dx and the gradient with respect to x, dw).
+    dw: None for a new bf16 tensor, else an fp32 one that is added to."""
+    H, D = x.shape[1:]
+    assert dout.dtype == dx.dtype == torch.float32 and dout.is_contiguous() and dx.stride(-1) == 1
+    dhidden = torch.empty(helper.y_len, H, weight.size(0), device=x.device, dtype=x.dtype)
+    _lib.call("nsa_compress_act_bwd", hidden.data_ptr(), dout.data_ptr(), dhidden.data_ptr(), helper.y_len * H, D, _ACT[version],
+              _lib.stream_ptr())
+    return (compress_linear_bwd_x(x, weight, dhidden, dx, helper), compress_linear_bwd_weight(x, weight, dhidden, dw, helper))
+
+
+def mean_pooling_bwd_sum(x, dout, dx, helper=NSAHelper):
+    """The bf16 sum of the fp32 dx and the gradient of mean pooling, from the fp32 gradient dout of its rows."""
+    T, H, D = x.shape
+    assert dout.dtype == dx.dtype == torch.float32 and dout.is_contiguous() and dx.stride(-1) == 1
+    dst = torch.empty(T, H, D, device=x.device, dtype=x.dtype)
+    _lib.call("nsa_mean_pool_bwd_sum", dout.data_ptr(), dx.data_ptr(), dx.stride(0), dx.stride(1), dst.data_ptr(), dst.stride(0),
+              dst.stride(1), helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, H, D,
+              helper.kernel_size, helper.stride, _lib.stream_ptr())
+    return dst
+
+
 class _MeanPooling(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
@@ -83,6 +158,29 @@ class _ConstructBlock(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         return construct_block_bwd(ctx.x_meta, dy, helper=ctx.helper)
+
+
+class _CompressLinear(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, version):
+        ctx.helper, ctx.version = NSAHelper.get_bwd_helper(), version
+        needed = any(ctx.needs_input_grad[:2])
+        hidden, out = compress_linear_fwd(x, weight, version, keep=needed)
+        ctx.save_for_backward(x, weight, None if version == "linear" else hidden)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        x, weight, hidden = ctx.saved_tensors
+        dhidden = dout.contiguous() if hidden is None else _glu_bwd(hidden, dout, ctx.version, inplace=False)
+        dx = compress_linear_bwd_x(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[0] else None
+        dw = compress_linear_bwd_weight(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[1] else None
+        return dx, dw, None
+
+
+def compress_linear(x, weight, version):
+    """Windows, product with the weight and activation in one autograd node (weights of takes_weight)."""
+    return _CompressLinear.apply(x, weight, version)
 
 
 def mean_pooling(x):

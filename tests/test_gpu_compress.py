@@ -1,0 +1,172 @@
+"""Learned compression without its windows in memory, against float64 (upstream flash_nsa/modules/megatron_level_nsa.py:46-86)."""
+import pytest
+import torch
+
+from gpu_util import make_cu, make_qkvw, randn_bf16
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -9  # relative rounding error of bf16
+
+
+def rel(got, want):
+    return float((got.double().cpu() - want).norm() / want.norm())
+
+
+def reference(x, w, version, lens, K, S, dout, dx):
+    """hidden, out, dx + gradient and dw in float64; windows in the order (position, channel)."""
+    x, w = x.double().requires_grad_(), w.double().requires_grad_()
+    D, a, rows = x.shape[2], 0, []
+    for n in lens:
+        rows += [x[a + S * i:a + S * i + K].transpose(0, 1).reshape(x.shape[1], -1) for i in range(max((n - K) // S + 1, 0))]
+        a += n
+    hidden = torch.stack(rows) @ w.t()
+    out = hidden
+    if version != "linear":
+        g = hidden[..., :D]
+        out = torch.sigmoid(g) * (g if version == "swiglu" else 1) * hidden[..., D:]
+    out.backward(dout.double())
+    return hidden.detach(), out.detach(), x.grad + dx.double(), w.grad
+
+
+@pytest.mark.parametrize("version", ["linear", "sigmoid-mul", "swiglu"])
+@pytest.mark.parametrize("H,D,K,S,lens", [
+    (4, 128, 32, 16, [700, 31, 32, 0, 47, 1000]),   # sequences without a window, with one, with tokens behind the last
+    (1, 64, 32, 16, [300]),
+    (3, 32, 32, 16, [200, 90, 17]),                 # one block of channels; rows of 128 hold heads of several windows
+    (2, 192, 32, 16, [513, 64]),                    # three pairs of blocks; columns of a chunk not a multiple of 128 * 2
+    (1, 256, 32, 16, [130]),
+    (2, 64, 64, 16, [500, 100]),                    # four windows over a token
+    (2, 128, 16, 16, [100, 15]),                    # windows that do not overlap
+    (5, 64, 16, 4, [77, 33]),
+    (1, 32, 8, 2, [40, 9]),                         # contraction shorter than the waves' parts; chunks of 64 columns
+])
+def test_learned_compression_against_float64(device, version, H, D, K, S, lens):
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops import compress_kv as C
+    T = sum(lens)
+    try:
+        NSAHelper.set_hyperparameters(kernel_size=K, stride=S)
+        NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+        x = randn_bf16(T, 2, H, D, seed=1)[:, 1]    # a strided view
+        N = D if version == "linear" else 2 * D
+        w = (randn_bf16(N, K * D, seed=2).float() * (K * D) ** -0.5).to(torch.bfloat16)
+        dx = randn_bf16(T, H, D, seed=3).float()
+        xd, wd = x.to(device), torch.cat([w, w], 1).to(device)[:, :K * D]
+        assert C.takes_weight(xd, wd, version)
+        hidden, out = C.compress_linear_fwd(xd, wd, version)
+        dout = randn_bf16(*out.shape, seed=4).float() + 1e-3
+        base = torch.full((N, K * D), 0.25, device=device)
+        dst, dw = C.compress_linear_bwd(xd, wd, hidden, dout.to(device), dx.to(device), version)
+        dst2, added = C.compress_linear_bwd(xd, wd, hidden, dout.to(device), dx.to(device), version, base)
+        want = reference(x, w, version, lens, K, S, dout, dx)
+    finally:
+        NSAHelper.set_hyperparameters()
+    assert torch.equal(dst, dst2) and added is base
+    # hidden: one rounding.  Its activation: that of gate and value, the gate's amplified by |g f'(g) / f(g)| <= 1 + |g| < 6, and
+    # its own; the gradients: that of dout, of hidden through the activation's derivative, of dhidden, and their own.
+    assert rel(hidden, want[0]) <= 1.02 * EPS
+    assert rel(out, want[1]) <= (1.02 if version == "linear" else 8) * EPS
+    assert rel(dst, want[2]) <= (3 if version == "linear" else 9) * EPS
+    assert rel(dw, want[3]) <= (3 if version == "linear" else 9) * EPS
+    assert rel(added - 0.25, want[3]) <= (2 if version == "linear" else 8) * EPS
+
+
+@pytest.mark.parametrize("H,D,version,T", [(4, 128, "sigmoid-mul", 26000), (2, 192, "linear", 34000), (1, 32, "swiglu", 600)])
+def test_compressed_rows_do_not_depend_on_the_batch(device, H, D, version, T):
+    """Every form of the forward kernel sums a product in the same order: prefixes of 300 and 9000 tokens give the same bits."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops import compress_kv as C
+    N = D if version == "linear" else 2 * D
+    x, w = randn_bf16(T, H, D, seed=5).to(device), (randn_bf16(N, 32 * D, seed=6) / 64).to(device)
+    NSAHelper.set_hyperparameters()
+    rows = []
+    for n in (T, min(9000, T), 300):
+        NSAHelper.init_cu_seqlens(torch.tensor([0, n], dtype=torch.int32, device=device))
+        rows.append(C.compress_linear_fwd(x[:n], w, version))
+    for got in rows[1:]:
+        for a, b in zip(got, rows[0]):
+            assert torch.equal(a, b[:a.size(0)])
+
+
+@pytest.mark.parametrize("H,D,K,S,lens", [(2, 64, 32, 16, [300, 5, 33]), (3, 128, 16, 4, [50, 0, 16]), (1, 32, 8, 8, [23])])
+def test_mean_pooling_gradient_and_sum_in_one(device, H, D, K, S, lens):
+    """The same bits as the gradient of the rounded rows added to the fp32 buffer, then rounded."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops import compress_kv as C
+    T = sum(lens)
+    try:
+        NSAHelper.set_hyperparameters(kernel_size=K, stride=S)
+        NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+        x = randn_bf16(T, H, D, seed=7).to(device)
+        dout = torch.randn(NSAHelper.y_len, H, D, generator=torch.Generator().manual_seed(8)).to(device)
+        dx = torch.randn(T, H, D, generator=torch.Generator().manual_seed(9)).to(device)
+        got = C.mean_pooling_bwd_sum(x, dout, dx)
+        want = C.mean_pooling_bwd(x, dout.to(torch.bfloat16), dx.clone()).to(torch.bfloat16)
+    finally:
+        NSAHelper.set_hyperparameters()
+    assert torch.equal(got, want)
+
+
+def test_weights_that_the_kernels_do_not_take_go_through_the_windows(device):
+    """A weight whose rows are not 16-byte aligned: windows and library products, the same gradients to rounding."""
+    from flash_nsa import NSAConfig, NSACore
+    lens, D = [200, 77], 64
+    q, k, v, w = [t.to(device) for t in make_qkvw(sum(lens), 8, 1, D, seed=10)]
+    do = randn_bf16(sum(lens), 8, D, seed=11).to(device)
+    cores = []
+    for odd in (False, True):
+        torch.manual_seed(0)
+        core = NSACore(NSAConfig(head_dim=D, num_heads=8, num_kv_heads=1, cmp_k_method="linear", cmp_v_method="swiglu"))
+        core = core.to(device=device, dtype=torch.bfloat16)
+        if odd:
+            for name in ("cmp_k_weight", "cmp_v_weight"):
+                p = getattr(core, name).detach()
+                wide = torch.empty(p.size(0), p.size(1) + 1, device=device, dtype=p.dtype)
+                wide[:, :-1] = p
+                setattr(core, name, torch.nn.Parameter(wide[:, :-1]))
+        ts = [t.clone().requires_grad_() for t in (q, k, v, w)]
+        out = core(*ts, make_cu(lens).to(device))
+        out.backward(do)
+        cores.append([out.detach()] + [t.grad for t in ts] + [core.cmp_k_weight.grad, core.cmp_v_weight.grad])
+    for i, (a, b) in enumerate(zip(*cores)):
+        assert a.dtype == b.dtype and rel(a, b.double().cpu()) < 2e-2, i  # (selections of near-tied blocks aside: all are selected)
+
+
+@pytest.mark.parametrize("version", ["linear", "sigmoid-mul", "swiglu"])
+@pytest.mark.parametrize("H,D,lens", [(2, 64, [300, 0, 31, 77]), (1, 128, [600])])
+def test_module_with_and_without_its_windows(device, version, H, D, lens):
+    """CompressKV computes a plain fc where the windows lie and calls one with a hook on them: the same to rounding, with the same
+    gradient types, also with only one of the two gradients asked for and without any."""
+    from flash_nsa import NSAConfig, NSAHelper
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+    torch.manual_seed(0)
+    mod = CompressKV(NSAConfig(head_dim=D), head_dim=D, version=version).to(device=device, dtype=torch.bfloat16)
+    x = randn_bf16(sum(lens), H, D, seed=12).to(device)
+    do = randn_bf16(NSAHelper.y_len, H, D, seed=13).to(device)
+
+    def run():
+        xs = x.clone().requires_grad_()
+        mod.fc.weight.grad = None
+        out = mod(xs)
+        out.backward(do)
+        return out.detach(), xs.grad, mod.fc.weight.grad
+
+    plain, calls = run(), []
+    hook = mod.fc.register_forward_hook(lambda *a: calls.append(1))
+    through = run()
+    hook.remove()
+    assert calls
+    for a, b in zip(plain, through):
+        assert a.dtype == b.dtype and a.shape == b.shape and rel(a, b.double().cpu()) <= 8 * EPS
+    with torch.no_grad():
+        assert torch.equal(mod(x), plain[0])
+    mod.fc.weight.requires_grad_(False)
+    xs = x.clone().requires_grad_()
+    mod(xs).backward(do)
+    assert torch.equal(xs.grad, plain[1])
+    mod.fc.weight.requires_grad_(True)
+    mod.fc.weight.grad = None
+    mod(x).backward(do)
+    assert torch.equal(mod.fc.weight.grad, plain[2])
