@@ -118,6 +118,15 @@ int nsa_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
                      const void* w, int64_t w_st, int64_t w_sh, void* out, int64_t out_st, int64_t out_sh,
                      int store_branches, const int32_t* x_cu, int B, int x_maxlen, int QH, int KH, int D, int VD,
                      int window, float sm_scale, void* stream);
+/* nsa_cmp_attn_fwd and nsa_swa_fwd_tail in one launch, for batches whose queries all select every block they can see: x_maxlen <=
+ * all_below. */
+int nsa_fwd_short(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh, const void* v,
+                  int64_t v_sr, int64_t v_sh, const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cv, int64_t cv_sr,
+                  int64_t cv_sh, void* cmp_o, int64_t co_st, int64_t co_sh, float* cmp_lse, int64_t cl_st, int64_t cl_sh, void* o,
+                  int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh,
+                  float* slc_lse, int64_t sl_st, int64_t sl_sh, int all_below, const void* w, int64_t w_st, int64_t w_sh, void* out,
+                  int64_t out_st, int64_t out_sh, int store_branches, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen,
+                  int QH, int KH, int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream);
 /* flash_nsa/ops/topk.py:630-775 slc_topk_indices; topk int32 addressed kh*tk_sh + tok*tk_st + slot;
  * imp_out optional fp32 block scores [KH, T, imp_cols] */
 int nsa_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
@@ -452,6 +461,15 @@ int nsa_paged_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void
                            const int32_t* context_lens, const int32_t* block_tables, int table_stride, int page_size,
                            int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale,
                            void* stream);
+/* nsa_paged_cmp_attn_fwd and nsa_paged_swa_fwd_tail (gated sum alone) in one launch, for requests whose contexts are no longer than
+ * all_below; cmp_o, o and slc_o are scratch. */
+int nsa_paged_fwd_short(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                        const void* v_cache, int64_t v_sr, int64_t v_sh, void* cmp_o, int64_t co_st, int64_t co_sh, void* o,
+                        int64_t o_st, int64_t o_sh, void* slc_o, int64_t so_st, int64_t so_sh, int all_below, const void* w,
+                        int64_t w_st, int64_t w_sh, void* out, int64_t out_st, int64_t out_sh, const int32_t* x_cu,
+                        const int32_t* context_lens, const int32_t* block_tables, int table_stride,
+                        const int32_t* cmp_block_tables, int cmp_table_stride, int page_size, int B, int x_maxlen, int QH, int KH,
+                        int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream);
 /* flash_nsa/inference/topk.py:184-298 topk_prefill / :495-623 topk_decode (causality is masked per row here) */
 int nsa_paged_topk_select(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,
                           int64_t k_sh, const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk,

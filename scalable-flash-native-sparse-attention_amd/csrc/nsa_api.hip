@@ -193,6 +193,48 @@ int nsa_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, i
   return nsa_fwd_tile_launch(p, 2, false, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
+// the compressed branch in the same launch
+static void fill_cmp_branch(NsaFwdTileParams& p, const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cv, int64_t cv_sr,
+                            int64_t cv_sh, void* cmp_o, float* cmp_lse, int64_t cl_st, int64_t cl_sh, int kernel_size, int stride) {
+  p.ck = (const bf16_t*)ck; p.ck_sr = ck_sr; p.ck_sh = ck_sh;
+  p.cv = (const bf16_t*)cv; p.cv_sr = cv_sr; p.cv_sh = cv_sh;
+  p.cmp_o_out = (bf16_t*)cmp_o;
+  p.cmp_lse = cmp_lse; p.cl_st = cl_st; p.cl_sh = cl_sh;
+  p.kernel_size = kernel_size; p.stride = stride;
+}
+
+int nsa_fwd_short(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh, const void* v,
+                  int64_t v_sr, int64_t v_sh, const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cv, int64_t cv_sr,
+                  int64_t cv_sh, void* cmp_o, int64_t co_st, int64_t co_sh, float* cmp_lse, int64_t cl_st, int64_t cl_sh, void* o,
+                  int64_t o_st, int64_t o_sh, float* lse, int64_t lse_st, int64_t lse_sh, void* slc_o, int64_t so_st, int64_t so_sh,
+                  float* slc_lse, int64_t sl_st, int64_t sl_sh, int all_below, const void* w, int64_t w_st, int64_t w_sh, void* out,
+                  int64_t out_st, int64_t out_sh, int store_branches, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen,
+                  int QH, int KH, int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream) {
+  int rc = check_heads("fwd_short", QH, KH, D, VD);
+  if (rc) return rc;
+  rc = check_nsa_sizes("fwd_short", kernel_size, stride, 0);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0, NSA_ERR_BAD_ARG, "fwd_short: window %d must be >= 0", window);
+  NSA_REQUIRE(x_maxlen <= all_below, NSA_ERR_BAD_ARG, "fwd_short: %d tokens are more than the %d that select everything", x_maxlen,
+              all_below);
+  NsaFwdTileParams p{};
+  p.q = (const bf16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
+  p.k = (const bf16_t*)k; p.k_sr = k_sr; p.k_sh = k_sh;
+  p.v = (const bf16_t*)v; p.v_sr = v_sr; p.v_sh = v_sh;
+  p.o = (bf16_t*)o; p.o_st = o_st; p.o_sh = o_sh;
+  p.lse = lse; p.lse_st = lse_st; p.lse_sh = lse_sh;
+  p.x_cu = x_cu; p.k_cu = y_cu;
+  p.G = QH / KH; p.KH = KH;
+  p.scale_log2 = sm_scale * NSA_LOG2E;
+  p.window = window;
+  rc = fill_swa_tail(p, "fwd_short", slc_o, so_st, so_sh, slc_lse, sl_st, sl_sh, all_below, cmp_o, co_st, co_sh, w, w_st, w_sh, out,
+                     out_st, out_sh, store_branches);
+  if (rc) return rc;
+  NSA_REQUIRE(cmp_o != nullptr, NSA_ERR_BAD_ARG, "fwd_short: the compressed branch's output is missing");
+  fill_cmp_branch(p, ck, ck_sr, ck_sh, cv, cv_sr, cv_sh, cmp_o, cmp_lse, cl_st, cl_sh, kernel_size, stride);
+  return nsa_fwd_tile_launch(p, 3, false, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
 static int topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const void* ck, int64_t ck_sr, int64_t ck_sh,
                             const float* lse, int64_t lse_st, int64_t lse_sh, int32_t* topk, int64_t tk_sh,
                             int64_t tk_st, float* imp_out, int64_t imp_sh, int64_t imp_st, int imp_cols,
@@ -1421,6 +1463,31 @@ int nsa_paged_swa_fwd_tail(const void* q, int64_t q_st, int64_t q_sh, const void
                      co_sh, w, w_st, w_sh, out, out_st, out_sh, store_branches);
   if (rc) return rc;
   return nsa_fwd_tile_launch(p, 2, true, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
+int nsa_paged_fwd_short(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr, int64_t k_sh,
+                        const void* v_cache, int64_t v_sr, int64_t v_sh, void* cmp_o, int64_t co_st, int64_t co_sh, void* o,
+                        int64_t o_st, int64_t o_sh, void* slc_o, int64_t so_st, int64_t so_sh, int all_below, const void* w,
+                        int64_t w_st, int64_t w_sh, void* out, int64_t out_st, int64_t out_sh, const int32_t* x_cu,
+                        const int32_t* context_lens, const int32_t* block_tables, int table_stride,
+                        const int32_t* cmp_block_tables, int cmp_table_stride, int page_size, int B, int x_maxlen, int QH, int KH,
+                        int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream) {
+  int rc = check_heads("paged_fwd_short", QH, KH, D, VD);
+  if (rc) return rc;
+  rc = check_nsa_sizes("paged_fwd_short", kernel_size, stride, 0);
+  if (rc) return rc;
+  rc = check_page("paged_fwd_short", page_size);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0, NSA_ERR_BAD_ARG, "paged_fwd_short: window %d must be >= 0", window);
+  NsaFwdTileParams p = paged_window_params(q, q_st, q_sh, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, o, o_st, o_sh, nullptr, 0, 0,
+                                           x_cu, context_lens, block_tables, table_stride, page_size, QH, KH, window, sm_scale);
+  rc = fill_swa_tail(p, "paged_fwd_short", slc_o, so_st, so_sh, nullptr, 0, 0, all_below, cmp_o, co_st, co_sh, w, w_st, w_sh, out,
+                     out_st, out_sh, 0);
+  if (rc) return rc;
+  NSA_REQUIRE(cmp_o != nullptr && out != nullptr, NSA_ERR_BAD_ARG, "paged_fwd_short: an output is missing");
+  fill_cmp_branch(p, k_cache, k_sr, k_sh, v_cache, v_sr, v_sh, cmp_o, nullptr, 0, 0, kernel_size, stride);
+  p.c_table = cmp_block_tables; p.c_table_stride = cmp_table_stride;
+  return nsa_fwd_tile_launch(p, 3, true, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
 static int paged_topk_select_impl(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sr,

@@ -28,6 +28,12 @@ struct NsaFwdTileParams {
   const bf16_t* cmp_o; int64_t co_st, co_sh;
   const bf16_t* w; int64_t w_st, w_sh;      // gates [tokens, QH, 3]
   bf16_t* out; int64_t out_st, out_sh;
+  // all branches in one launch: compressed rows (their offsets k_cu, or their block table), where their branch goes
+  const bf16_t* ck; int64_t ck_sr, ck_sh;
+  const bf16_t* cv; int64_t cv_sr, cv_sh;
+  const int32_t* c_table; int c_table_stride;
+  bf16_t* cmp_o_out;                          // cmp_o
+  float* cmp_lse; int64_t cl_st, cl_sh;
   bool last_first;                            // a sequence's last rows first (set by the launcher)
 };
 

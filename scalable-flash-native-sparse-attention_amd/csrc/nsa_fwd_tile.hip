@@ -19,6 +19,7 @@ namespace {
 constexpr int MODE_CMP = 0;
 constexpr int MODE_SWA = 1;
 constexpr int MODE_TAIL = 2;  // MODE_SWA, and what can be finished in the same launch (below)
+constexpr int MODE_ALL = 3;   // MODE_TAIL behind the compressed branch of the same queries (all of them below all_below)
 
 typedef __attribute__((address_space(1))) const void* nsa_gptr_t;
 typedef __attribute__((address_space(3))) void* nsa_lptr_t;
@@ -77,22 +78,29 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int rows_total = xl * G;
   const int r0 = (p.last_first ? gridDim.y - 1 - blockIdx.y : blockIdx.x) * ROWS_WG;
   if (r0 >= rows_total) return;
+  constexpr bool TAIL = MODE == MODE_TAIL || MODE == MODE_ALL;
+  constexpr bool HAS_CMP = MODE == MODE_CMP || MODE == MODE_ALL;
   int nkeys, kbase = 0;
-  if (MODE == MODE_CMP) {
+  if (HAS_CMP) {
     nkeys = ctx >= p.kernel_size ? (ctx - p.kernel_size) / p.stride + 1 : 0;
     if (!PAGED) kbase = p.k_cu[b];
   } else {
     nkeys = ctx;
     if (!PAGED) kbase = x0;
   }
-  const int32_t* table = PAGED ? p.table + (int64_t)b * p.table_stride : nullptr;
+  // where the keys lie: MODE_ALL starts with the compressed rows
+  bool in_cmp = HAS_CMP;
+  const bf16_t *ksrc = MODE == MODE_ALL ? p.ck : p.k, *vsrc = MODE == MODE_ALL ? p.cv : p.v;
+  int64_t k_sr = MODE == MODE_ALL ? p.ck_sr : p.k_sr, v_sr = MODE == MODE_ALL ? p.cv_sr : p.v_sr;
+  int64_t k_sh = MODE == MODE_ALL ? p.ck_sh : p.k_sh, v_sh = MODE == MODE_ALL ? p.cv_sh : p.v_sh;
+  const int32_t* table = !PAGED ? nullptr : MODE == MODE_ALL ? p.c_table + (int64_t)b * p.c_table_stride : p.table + (int64_t)b * p.table_stride;
 
   // ---- per-lane rows ----
   int t_row[RS];
   bool valid[RS];
   int64_t tok[RS];
   int head[RS];
-  int key_hi[RS];  // MODE_CMP: the last key that the row sees
+  int key_hi[RS];  // the last compressed key that the row sees
   bf16x8 qf[RS][D / 16];
 #pragma unroll
   for (int rs = 0; rs < RS; rs++) {
@@ -102,7 +110,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     int n = rr / G;
     int g = rr - n * G;
     t_row[rs] = n + qoff;
-    if (MODE == MODE_CMP) key_hi[rs] = t_row[rs] >= p.kernel_size - 1 ? min((t_row[rs] - p.kernel_size + 1) / p.stride, nkeys - 1) : -1;
+    if (HAS_CMP) key_hi[rs] = t_row[rs] >= p.kernel_size - 1 ? min((t_row[rs] - p.kernel_size + 1) / p.stride, nkeys - 1) : -1;
     tok[rs] = x0 + n;
     head[rs] = kh * G + g;
     const bf16_t* qp = p.q + tok[rs] * p.q_st + (int64_t)head[rs] * p.q_sh + hl * 8;
@@ -119,10 +127,11 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   const int t_hi = min(r0 + ROWS_WG - 1, rows_total - 1) / G + qoff;
 
   int key_begin, key_end;
-  if (MODE == MODE_CMP) {
+  if (HAS_CMP) {
     key_begin = 0;
     key_end = t_hi >= p.kernel_size - 1 ? min((t_hi - p.kernel_size + 1) / p.stride + 1, nkeys) : 0;
-  } else {
+  }
+  if (MODE != MODE_CMP && MODE != MODE_ALL) {
     key_begin = (max(0, t_lo - p.window) / KT) * KT;
     key_end = min(t_hi + 1, nkeys);
   }
@@ -132,15 +141,18 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 
   f32x16 oacc[RS][VD / 32];
   float m_run[RS], l_run[RS];
+  auto reset = [&]() {
 #pragma unroll
-  for (int rs = 0; rs < RS; rs++) {
-    m_run[rs] = NSA_NEG_INF;
-    l_run[rs] = 0.f;
+    for (int rs = 0; rs < RS; rs++) {
+      m_run[rs] = NSA_NEG_INF;
+      l_run[rs] = 0.f;
 #pragma unroll
-    for (int dt = 0; dt < VD / 32; dt++)
+      for (int dt = 0; dt < VD / 32; dt++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) oacc[rs][dt][i] = 0.f;
-  }
+        for (int i = 0; i < 16; i++) oacc[rs][dt][i] = 0.f;
+    }
+  };
+  reset();
   const float sc = p.scale_log2;
 
   // software pipeline: the next tile's global loads are in flight while the current tile is computed.
@@ -161,14 +173,14 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       int pc = tid + j * 256;
       int kr = min(pc / KP, last), dp = pc % KP;
       int64_t row = PAGED ? page_row0 + kr : (int64_t)kbase + kt + kr;
-      kreg[j] = ld_global_b128(p.k + row * p.k_sr + (int64_t)kh * p.k_sh + dp * 8);
+      kreg[j] = ld_global_b128(ksrc + row * k_sr + (int64_t)kh * k_sh + dp * 8);
     }
 #pragma unroll
     for (int j = 0; j < VJ; j++) {
       int pc = tid + j * 256;
       int kr = min(pc / VP, last), dp = pc % VP;
       int64_t row = PAGED ? page_row0 + kr : (int64_t)kbase + kt + kr;
-      vreg[j] = ld_global_b128(p.v + row * p.v_sr + (int64_t)kh * p.v_sh + dp * 8);
+      vreg[j] = ld_global_b128(vsrc + row * v_sr + (int64_t)kh * v_sh + dp * 8);
     }
   };
 
@@ -233,7 +245,7 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
     // ones, 64 more of a wave's 250 vector instructions per tile; short sequences mask two to four of their 2 to 12 tiles.)
     if (mask_hi) {
       asm volatile("");  // keeps it a branch: if-converted, every tile would pay
-      const int bound = (MODE == MODE_CMP ? key_hi[rs] : MODE == MODE_TAIL && t_row[rs] >= t_end ? -0x40000000 : t_row[rs] + khi) -
+      const int bound = (HAS_CMP && in_cmp ? key_hi[rs] : TAIL && t_row[rs] >= t_end ? -0x40000000 : t_row[rs] + khi) -
                         kt - hl * 4;
 #pragma unroll
       for (int nt = 0; nt < 2; nt++)
@@ -317,34 +329,37 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   static_assert(!ASYNC || (KROWS % 16 == 0 && VROWS % 16 == 0 && KJ % KPAT == 0 && VJ % VPAT == 0), "period of the swizzles");
   static_assert(!ASYNC || ((KROWS > VROWS ? KROWS : VROWS) - 1) * async_row_stride(D, VD) * 2 + 512 < (int64_t)1 << 32, "a lane's offset");
   uint32_t goffk[KPAT], goffv[VPAT];
-  if constexpr (ASYNC) {
+  auto set_offsets = [&]() {
+    if constexpr (ASYNC) {
 #pragma unroll
-    for (int j = 0; j < KPAT; j++) {
-      const int pc = tid + j * 256, row = pc / KP;
-      goffk[j] = (uint32_t)((row * p.k_sr + ((pc % KP) ^ swz<KP>(row)) * 8) * 2);
-    }
+      for (int j = 0; j < KPAT; j++) {
+        const int pc = tid + j * 256, row = pc / KP;
+        goffk[j] = (uint32_t)((row * k_sr + ((pc % KP) ^ swz<KP>(row)) * 8) * 2);
+      }
 #pragma unroll
-    for (int j = 0; j < VPAT; j++) {
-      const int pc = tid + j * 256, row = pc / VP;
-      goffv[j] = (uint32_t)((row * p.v_sr + ((pc % VP) ^ swzv<VP>(row)) * 8) * 2);
+      for (int j = 0; j < VPAT; j++) {
+        const int pc = tid + j * 256, row = pc / VP;
+        goffv[j] = (uint32_t)((row * v_sr + ((pc % VP) ^ swzv<VP>(row)) * 8) * 2);
+      }
     }
-  }
+  };
+  set_offsets();
   auto stage_async = [&](int kt, int buf) {
     int64_t row0;
     if (PAGED) row0 = (int64_t)table[kt / p.page_size] * p.page_size + (kt % p.page_size);
     else row0 = (int64_t)kbase + kt;
     const int last = key_end - 1 - kt;  // >= 0; rows past it repeat it (masked)
-    const char* kb = scalar_ptr(p.k + row0 * p.k_sr + (int64_t)kh * p.k_sh);
-    const char* vb = scalar_ptr(p.v + row0 * p.v_sr + (int64_t)kh * p.v_sh);
+    const char* kb = scalar_ptr(ksrc + row0 * k_sr + (int64_t)kh * k_sh);
+    const char* vb = scalar_ptr(vsrc + row0 * v_sr + (int64_t)kh * v_sh);
     if (last >= KT - 1) {  // wave-uniform
 #pragma unroll
       for (int j = 0; j < KJ; j++) {
-        const char* at = kb + (int64_t)(j / KPAT) * KROWS * p.k_sr * 2;
+        const char* at = kb + (int64_t)(j / KPAT) * KROWS * k_sr * 2;
         __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + goffk[j % KPAT]), (nsa_lptr_t)&Ks2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
       }
 #pragma unroll
       for (int j = 0; j < VJ; j++) {
-        const char* at = vb + (int64_t)(j / VPAT) * VROWS * p.v_sr * 2;
+        const char* at = vb + (int64_t)(j / VPAT) * VROWS * v_sr * 2;
         __builtin_amdgcn_global_load_lds((nsa_gptr_t)(at + goffv[j % VPAT]), (nsa_lptr_t)&Vs2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
       }
     } else {
@@ -352,14 +367,14 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
       for (int j = 0; j < KJ; j++) {
         const int pc = tid + j * 256;
         const int row = pc / KP, c = (pc % KP) ^ swz<KP>(row);
-        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(kb + ((int64_t)min(row, last) * p.k_sr + c * 8) * 2),
+        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(kb + ((int64_t)min(row, last) * k_sr + c * 8) * 2),
                                          (nsa_lptr_t)&Ks2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
       }
 #pragma unroll
       for (int j = 0; j < VJ; j++) {
         const int pc = tid + j * 256;
         const int row = pc / VP, c = (pc % VP) ^ swzv<VP>(row);
-        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(vb + ((int64_t)min(row, last) * p.v_sr + c * 8) * 2),
+        __builtin_amdgcn_global_load_lds((nsa_gptr_t)(vb + ((int64_t)min(row, last) * v_sr + c * 8) * 2),
                                          (nsa_lptr_t)&Vs2[buf][(j * 256 + wave * 64) * 8], 16, 0, 0);
       }
     }
@@ -390,12 +405,12 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
 
       // wave-uniform visibility classification of this tile
       bool any_vis, mask_hi, mask_lo = false;
-      if (MODE == MODE_CMP) {
+      if (HAS_CMP && in_cmp) {
         any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
         mask_hi = tw_lo < p.stride * (kt + KT - 1) + p.kernel_size - 1 || kt + KT > nkeys;
       } else {
         any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
-        mask_hi = kt + KT - 1 > tw_lo + khi || (MODE == MODE_TAIL && tw_hi >= t_end);
+        mask_hi = kt + KT - 1 > tw_lo + khi || (TAIL && tw_hi >= t_end);
         mask_lo = kt < tw_hi + klo;
       }
       if (!any_vis) continue;
@@ -456,7 +471,27 @@ __global__ __launch_bounds__(256, MINB) void fwd_tile_kernel(NsaFwdTileParams p)
   constexpr int ALL = 0x7fffffff;
   run_keys();
   __syncthreads();  // the tile buffers are free
-  if constexpr (MODE != MODE_TAIL) {
+  if constexpr (MODE == MODE_ALL) {
+    // Sequences whose queries all select everything have few compressed keys (63 at 1024 tokens: one tile), and nothing waits for
+    // their log-sum-exps: the branch needs no launch of its own, and the same queries are read once.  Calls in two launches / in
+    // one, us, 64 / 4 heads of 128: 3 prompts of 60 to 700 tokens 64.5 / 61, 2 of 300 to 900 69 / 65, 6 of 60 to 1000 125 / 119, 12
+    // 252 / 237; forward of 1000 tokens 68 / 66, 16 / 1 heads, 3 of 100 to 400 65 / 47; 16 / 2 heads of 64, 40 of up to 1000 117 / 98,
+    // 8 prompts 62 / 50.
+    emit(p.cmp_o_out, p.co_st, p.co_sh, p.cmp_lse, p.cl_st, p.cl_sh, ALL);
+    __syncthreads();
+    reset();
+    in_cmp = false;
+    ksrc = p.k; vsrc = p.v; k_sr = p.k_sr; v_sr = p.v_sr; k_sh = p.k_sh; v_sh = p.v_sh;
+    if (PAGED) table = p.table + (int64_t)b * p.table_stride;
+    else kbase = x0;
+    nkeys = ctx;
+    set_offsets();
+    key_begin = (max(0, t_lo - p.window) / KT) * KT;
+    key_end = min(t_hi + 1, nkeys);
+    run_keys();
+    __syncthreads();
+  }
+  if constexpr (!TAIL) {
     emit(p.o, p.o_st, p.o_sh, p.lse, p.lse_st, p.lse_sh, ALL);
   } else {
     static_assert(RS == 1, "");
@@ -574,7 +609,7 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   // 18.7 ms, 16 x 2K paged rows 5.21 / 5.25), short ones from twice as many on: 40 samples of 17 to 1200 218 / 203, 12 prompts
   // of 60 to 1000 253 / 249.  The compressed branch gains nothing (1500 tokens 205 / 203, 4 x 300 to 1500 156 / 160).
   const int64_t wgs = (int64_t)cdiv_i(max_q_len * p.G, 128) * B * p.KH;
-  p.last_first = MODE == MODE_TAIL && wgs <= (max_q_len / 2 <= p.all_below ? 32 : 16) * nsa_device_cus();
+  p.last_first = MODE >= MODE_TAIL && wgs <= (max_q_len / 2 <= p.all_below ? 32 : 16) * nsa_device_cus();
   const int tiles = cdiv_i(max_q_len * p.G, 128);
   const dim3 grid = p.last_first ? dim3(B * p.KH, tiles) : dim3(tiles, B, p.KH);
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there; the window
@@ -584,13 +619,14 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   // queries behind up to 8K 1352 / 1118.  1..4 force one variant for experiments.
   const int variant = nsa_tuning_knob("fwd_variant", 0);
   constexpr bool pow2 = (D == 64 || D == 128) && (VD == 64 || VD == 128);
-  const bool narrow = p.k_sr >= 0 && p.v_sr >= 0 && p.k_sr <= async_row_stride(D, VD) && p.v_sr <= async_row_stride(D, VD);
+  auto fits = [](int64_t stride) { return stride >= 0 && stride <= async_row_stride(D, VD); };
+  const bool narrow = fits(p.k_sr) && fits(p.v_sr) && (MODE != MODE_ALL || (fits(p.ck_sr) && fits(p.cv_sr)));
   const bool async = narrow && (variant == 4 || (variant == 0 && ((MODE == MODE_CMP && pow2) || D == 192)));
   if constexpr (D > 192 || VD > 128) {
     // head dims of 256: the output accumulators alone take 128 registers, one workgroup per CU
     fwd_tile_kernel<D, VD, MODE, PAGED, 1, 1, false><<<grid, 256, 0, stream>>>(p);
     return nsa_check_launch("fwd_tile_kernel");
-  } else if constexpr (MODE == MODE_TAIL) {
+  } else if constexpr (MODE >= MODE_TAIL) {
     if constexpr (D == 192) {
       if (variant != 1 && narrow) {
         fwd_tile_kernel<D, VD, MODE, PAGED, 1, 2, true><<<grid, 256, 0, stream>>>(p);
@@ -628,6 +664,10 @@ int nsa_fwd_tile_launch(const NsaFwdTileParams& p, int mode, bool paged, int B, 
   if (mode == MODE_CMP) {
     return paged ? dispatch_fwd_tile<MODE_CMP, true>(p, B, max_q_len, D, VD, stream)
                  : dispatch_fwd_tile<MODE_CMP, false>(p, B, max_q_len, D, VD, stream);
+  }
+  if (mode == MODE_ALL) {
+    return paged ? dispatch_fwd_tile<MODE_ALL, true>(p, B, max_q_len, D, VD, stream)
+                 : dispatch_fwd_tile<MODE_ALL, false>(p, B, max_q_len, D, VD, stream);
   }
   if (mode == MODE_TAIL) {
     return paged ? dispatch_fwd_tile<MODE_TAIL, true>(p, B, max_q_len, D, VD, stream)

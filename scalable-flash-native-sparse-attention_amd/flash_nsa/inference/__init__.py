@@ -6,7 +6,7 @@ never synchronise with the host, so the decode step can be captured in a HIP gra
 from ..ops._common import check_bf16
 from .stages import (mean_pooling_prefill, kv_mean_pooling_decode, cmp_attn_prefill, cmp_attn_decode, topk_prefill,
                      topk_decode, slc_attn_prefill, fused_slc_swa_attn_decode, swa_prefill, combine_prefill,
-                     swa_combine_prefill, combine_decode, mean_pooling_decode, slc_attn_decode,
+                     swa_combine_prefill, short_prefill, combine_decode, mean_pooling_decode, slc_attn_decode,
                      fused_decode_supported, decode_cmp_topk,
                      decode_slc_swa_combine, decode_cmp_split, decode_one_launch, decode_one_launch_fits,
                      store_kvcache, store_kvcache_and_pool_prefill, decode_split, decode_split_fits,
@@ -40,6 +40,9 @@ def nsa_prefill(q, k, v, w, x_cu_seqlens, y_cu_seqlens, x_maxlen, y_maxlen, cont
                              kernel_size=kernel_size, stride=stride)
     # queries with at most top_n blocks in sight select them all; no context is longer than its row of the page table
     full = dict(all_below=top_n * block_size, max_context=block_tables.size(1) * k.size(1))
+    if 0 < full["max_context"] <= full["all_below"]:
+        return short_prefill(q, k, v, w, x_cu_seqlens, x_maxlen, block_tables, cmp_block_tables, context_lens, full["all_below"],
+                             kernel_size=kernel_size, stride=stride, window_size=window_size, sm_scale=sm_scale)
     cmp_o, lse = cmp_attn_prefill(q, k, v, x_cu_seqlens, x_maxlen, block_tables=cmp_block_tables,
                                   context_lens=context_lens, kernel_size=kernel_size, stride=stride,
                                   sm_scale=sm_scale)

@@ -227,6 +227,30 @@ def swa_combine_prefill(q, k, v, cmp_o, slc_o, w, x_cu_seqlens, x_maxlen, block_
     return out
 
 
+def short_prefill(q, k, v, w, x_cu_seqlens, x_maxlen, block_tables, cmp_block_tables, context_lens, all_below, kernel_size=32,
+                  stride=16, window_size=512, sm_scale=None):
+    """cmp_attn_prefill and swa_combine_prefill in one launch -> o [t,QH,VD], for contexts of at most all_below tokens: their
+    queries select every block they can see."""
+    check_bf16(q), check_bf16(w)
+    page, KH, D, ksr, ksh = _pool_args(k)
+    _, _, VD, vsr, vsh = _pool_args(v)
+    t, QH, _ = q.shape
+    B = x_cu_seqlens.numel() - 1
+    sm_scale = q.size(-1) ** -0.5 if sm_scale is None else sm_scale
+    assert w.shape == (t, QH, 3)
+    out = torch.empty(t, QH, VD, device=q.device, dtype=q.dtype)
+    scratch = torch.empty(3, t, QH, VD, device=q.device, dtype=q.dtype)
+    rows = (out.stride(0), out.stride(1))
+    size = scratch.stride(0) * 2
+    at = scratch.data_ptr()
+    _lib.call("nsa_paged_fwd_short", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), ksr, ksh, v.data_ptr(), vsr, vsh, at,
+              *rows, at + size, *rows, at + 2 * size, *rows, all_below, w.data_ptr(), w.stride(0), w.stride(1), out.data_ptr(), *rows,
+              _i32(x_cu_seqlens).data_ptr(), _i32(context_lens).data_ptr(), _i32(block_tables).data_ptr(), block_tables.stride(0),
+              _i32(cmp_block_tables).data_ptr(), cmp_block_tables.stride(0), page, B, int(x_maxlen), QH, KH, D, VD, kernel_size,
+              stride, window_size, sm_scale, _lib.stream_ptr())
+    return out
+
+
 def slc_attn_decode(q, k, v, topk, block_tables, context_lens, num_splits=0, block_size=64, top_n=16,
                     sm_scale=None):
     B = q.size(0)

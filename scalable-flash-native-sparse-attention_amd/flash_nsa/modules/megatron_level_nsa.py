@@ -19,7 +19,7 @@ from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_bef
 from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
 from ..ops.combine import combine_bwd_gates
-from ..ops.sliding_window_attention import (slc_fwd_first_queries, swa_fwd, swa_fwd_tail, swa_bwd,
+from ..ops.sliding_window_attention import (short_fwd, slc_fwd_first_queries, swa_fwd, swa_fwd_tail, swa_bwd,
                                             swa_bwd_dq_tail)
 
 
@@ -193,10 +193,15 @@ class NSAFunction(torch.autograd.Function):
         H = NSAHelper
         win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, H.cmp_k_method, keep=for_backward)
         win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method, keep=for_backward)
-        cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
-        topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=H.all_below())
-        (slc_o, slc_lse), (swa_o, swa_lse), out = slc_swa_fwd(q, k, v, topk, sm_scale, H, cmp_o, combine_weight,
-                                                              store=for_backward)
+        if 0 < H.x_maxlen <= H.all_below():  # nothing to choose from: no block is selected
+            topk = torch.empty(k.size(1), q.size(0), H.top_n, device=q.device, dtype=torch.int32)
+            (cmp_o, cmp_lse), (slc_o, slc_lse), (swa_o, swa_lse), out = short_fwd(q, k, v, cmp_k, cmp_v, combine_weight, H.all_below(),
+                                                                                 for_backward, sm_scale, H)
+        else:
+            cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale)
+            topk, _ = slc_topk_indices(q, cmp_k, cmp_lse, sm_scale=sm_scale, all_below=H.all_below())
+            (slc_o, slc_lse), (swa_o, swa_lse), out = slc_swa_fwd(q, k, v, topk, sm_scale, H, cmp_o, combine_weight,
+                                                                  store=for_backward)
         if not for_backward:
             return out
 

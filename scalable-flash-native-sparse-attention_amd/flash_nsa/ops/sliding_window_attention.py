@@ -47,6 +47,32 @@ def swa_fwd_tail(q, k, v, slc_o, slc_lse, all_below, cmp_o=None, w=None, store=T
     return o, lse, out
 
 
+def short_fwd(q, k, v, cmp_k, cmp_v, w, all_below, store=True, sm_scale=None, helper=NSAHelper):
+    """cmp_attn_fwd and swa_fwd_tail in one launch, for batches of sequences of at most all_below tokens (their queries select every
+    block they can see) -> (cmp_o, cmp_lse), (slc_o, slc_lse), (swa_o, swa_lse), out; with store=False only out is defined."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (cmp_k, "k"), (cmp_v, "v")):
+        check_thd(t, n)
+    check_bf16(w)
+    T, QH, D = q.shape
+    _, KH, VD = v.shape
+    assert cmp_k.shape == (helper.y_len, KH, D) and cmp_v.shape == (helper.y_len, KH, VD) and QH % KH == 0
+    assert w.shape == (T, QH, 3)
+    new = lambda *shape: torch.empty(*shape, T, QH, VD, device=q.device, dtype=q.dtype)
+    out = new()
+    cmp_o, slc_o, swa_o = (new(), new(), new()) if store else new(3).unbind()
+    cmp_lse = slc_lse = swa_lse = None
+    if store:
+        cmp_lse = torch.empty(QH, T, device=q.device, dtype=torch.float32)
+        slc_lse, swa_lse = (torch.empty(T, QH, device=q.device, dtype=torch.float32) for _ in range(2))
+    st = lambda t: (None, 0, 0) if t is None else (t.data_ptr(), t.stride(0), t.stride(1))
+    lse_c = (None, 0, 0) if cmp_lse is None else (cmp_lse.data_ptr(), cmp_lse.stride(1), cmp_lse.stride(0))
+    _lib.call("nsa_fwd_short", *st(q), *st(k), *st(v), *st(cmp_k), *st(cmp_v), *st(cmp_o), *lse_c, *st(swa_o), *st(swa_lse), *st(slc_o),
+              *st(slc_lse), all_below, *st(w), *st(out), int(store), helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(),
+              helper.batch, helper.x_maxlen, QH, KH, D, VD, helper.kernel_size, helper.stride, helper.window_size,
+              default_scale(q, sm_scale), _lib.stream_ptr())
+    return (cmp_o, cmp_lse), (slc_o, slc_lse), (swa_o, swa_lse), out
+
+
 def slc_fwd_first_queries(q, k, v, slc_o, slc_lse, all_below, sm_scale=None, helper=NSAHelper):
     """What swa_fwd_tail does for the selected branch alone: slc_o / slc_lse of the queries at positions below all_below."""
     T, QH, D = q.shape

@@ -384,3 +384,37 @@ def test_window_launch_of_few_workgroups_takes_last_rows_first(device, QH, KH, D
         assert torch.equal(got, want[:n])
         first = lens[0]
         assert torch.equal(core(q[:first], k[:first], v[:first], w[:first], make_cu([first]).to(device)), want[:first])
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens,kw", [
+    (8, 2, 64, 64, [1, 31, 32, 700, 0, 1024], {}),                       # no compressed key, one, 63 in one tile
+    (12, 3, 128, 128, [513, 640, 33], {}),
+    (4, 1, 192, 128, [300, 47], dict(window_size=100)),                  # direct-to-LDS tiles, sources of other strides
+    (3, 1, 32, 32, [200], dict(top_n=8, window_size=64)),
+    (2, 1, 256, 256, [150], {}),
+    (8, 1, 64, 64, [500], dict(kernel_size=16, stride=2, window_size=40)),  # several tiles of compressed keys
+])
+def test_short_batches_in_one_launch_equal_two(device, QH, KH, D, VD, lens, kw):
+    """Sequences whose queries all select everything: the compressed branch, the window, the selected branch and the gated sum of one
+    launch are the bits of two, with and without what the backward asks for."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.compress_attn import cmp_attn_fwd
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.sliding_window_attention import short_fwd, swa_fwd_tail
+    T = sum(lens)
+    try:
+        setup_helper(make_cu(lens).to(device), **kw)
+        q, k, v, w = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=74)]
+        kk = torch.cat([k, k], 1)[:, :KH]  # the keys' strides are not those of the compressed rows
+        ck, cv, below = mean_pooling_fwd(k), mean_pooling_fwd(v), NSAHelper.all_below()
+        cmp_o, cmp_lse = cmp_attn_fwd(q, ck, cv)
+        slc_o, slc_lse = torch.empty_like(cmp_o), torch.empty(T, QH, device=device)
+        swa_o, swa_lse, out = swa_fwd_tail(q, kk, v, slc_o, slc_lse, below, cmp_o, w)
+        one = short_fwd(q, kk, v, ck, cv, w, below)
+        bare = short_fwd(q, kk, v, ck, cv, w, below, store=False)[3]
+    finally:
+        NSAHelper.set_hyperparameters()
+    want = ((cmp_o, cmp_lse), (slc_o, slc_lse), (swa_o, swa_lse))
+    for got, ref in zip(one[:3], want):
+        assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+    assert torch.equal(one[3], out) and torch.equal(bare, out)

@@ -937,3 +937,25 @@ def test_one_launch_decode_with_four_waves(device, QH, KH, D, VD, cap):
         assert int((~same).sum()) <= 1, "selections differ"   # one fp32 near-tie at the cut is excused
     bad = (runs[4][0].float() - ref.float()).abs() > 2 ** -7 + 2 ** -7 * ref.float().abs()
     assert int(bad.flatten(1).any(1).sum()) <= 1              # the request of that tie
+
+
+@pytest.mark.parametrize("QH,KH,D,page,cached,new", [
+    (16, 2, 64, 64, [0, 130, 0, 900], [700, 17, 1, 124]),    # whole prompts, chunks behind prefixes, the longest context that fits
+    (6, 2, 128, 128, [37, 0], [300, 5]),                     # groups of 3 q-heads
+    (64, 4, 128, 256, [0, 0, 200], [498, 345, 56]),
+])
+def test_prefill_of_short_contexts_in_one_launch_equals_two(device, QH, KH, D, page, cached, new):
+    """Contexts of at most top_n * block_size tokens: every branch and the gated sum in one launch are the bits of the compressed
+    branch's launch and the window's."""
+    from flash_nsa.inference import stages as S
+    ctx = [c + n for c, n in zip(cached, new)]
+    case = build_pool(ctx, KH, D, D, page=page, seed=9)
+    prepool(case, ctx)
+    d = to_dev(case, device)
+    xcu, t = make_cu(new).to(device), sum(new)
+    q, w = randn_bf16(t, QH, D, seed=10).to(device), randn_bf16(t, QH, 3, seed=11).to(device)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32).to(device)
+    got = S.short_prefill(q, d["k"], d["v"], w, xcu, max(new), d["bt"], d["cbt"], ctx_t, 1024)
+    cmp_o, _ = S.cmp_attn_prefill(q, d["k"], d["v"], xcu, max(new), d["cbt"], ctx_t)
+    want = S.swa_combine_prefill(q, d["k"], d["v"], cmp_o, torch.empty_like(cmp_o), w, xcu, max(new), d["bt"], ctx_t, all_below=1024)
+    assert torch.equal(got, want)
