@@ -237,6 +237,18 @@ int nsa_swa_bwd_dq(const void* q, int64_t q_st, int64_t q_sh, const void* k, int
                    const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,
                    int64_t delta_sh, void* dq, int64_t dq_st, int64_t dq_sh, int dq_mode, const int32_t* x_cu,
                    int B, int x_maxlen, int QH, int KH, int D, int VD, int window, float sm_scale, void* stream);
+/* dq of the compressed branch, the window and, for the queries at positions below all_below, the keys before it, in one: those
+ * queries' dq goes to dq in bf16, that of the others to the fp32 dq_partial (may be null if x_maxlen <= all_below).  The gradients,
+ * log-sum-exps and deltas of window, selected and compressed branch as nsa_swa_bwd_dq_tail and nsa_cmp_attn_bwd_dq take them. */
+int nsa_bwd_dq_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh, const void* v, int64_t v_sr,
+                     int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh,
+                     const float* delta, int64_t delta_st, int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh,
+                     const float* slc_lse, int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                     int all_below, const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cv, int64_t cv_sr, int64_t cv_sh,
+                     const void* cmp_dO, int64_t cdo_st, int64_t cdo_sh, const float* cmp_lse, int64_t cl_st, int64_t cl_sh,
+                     const float* cmp_delta, int64_t cd_st, int64_t cd_sh, void* dq, int64_t dq_st, int64_t dq_sh, float* dq_partial,
+                     int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH,
+                     int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream);
 /* nsa_swa_bwd_dq with dq_mode 2 (add into fp32) for gradients from nsa_combine_bwd_gates: the queries at positions below
  * all_below also take the selected branch's keys before their window, and their dq is stored instead of added */
 int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,

@@ -642,6 +642,41 @@ static int swa_bwd_dq_tail_impl(int dq_mode, const void* q, int64_t q_st, int64_
   return nsa_bwd_dq_tile_launch(p, 2, B, x_maxlen, D, VD, (hipStream_t)stream);
 }
 
+int nsa_bwd_dq_dense(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh, const void* v, int64_t v_sr,
+                     int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh, const float* lse, int64_t lse_st, int64_t lse_sh,
+                     const float* delta, int64_t delta_st, int64_t delta_sh, const void* slc_dO, int64_t sdo_st, int64_t sdo_sh,
+                     const float* slc_lse, int64_t sl_st, int64_t sl_sh, const float* slc_delta, int64_t sd_st, int64_t sd_sh,
+                     int all_below, const void* ck, int64_t ck_sr, int64_t ck_sh, const void* cv, int64_t cv_sr, int64_t cv_sh,
+                     const void* cmp_dO, int64_t cdo_st, int64_t cdo_sh, const float* cmp_lse, int64_t cl_st, int64_t cl_sh,
+                     const float* cmp_delta, int64_t cd_st, int64_t cd_sh, void* dq, int64_t dq_st, int64_t dq_sh, float* dq_partial,
+                     int64_t dqp_st, int64_t dqp_sh, const int32_t* x_cu, const int32_t* y_cu, int B, int x_maxlen, int QH, int KH,
+                     int D, int VD, int kernel_size, int stride, int window, float sm_scale, void* stream) {
+  int rc = check_heads("bwd_dq_dense", QH, KH, D, VD);
+  if (rc) return rc;
+  rc = check_nsa_sizes("bwd_dq_dense", kernel_size, stride, 0);
+  if (rc) return rc;
+  NSA_REQUIRE(window >= 0 && all_below >= 0, NSA_ERR_BAD_ARG, "bwd_dq_dense: window %d and all_below %d must be >= 0", window,
+              all_below);
+  NSA_REQUIRE(dq != nullptr && (dq_partial != nullptr || x_maxlen <= all_below), NSA_ERR_BAD_ARG, "bwd_dq_dense: null dq buffers");
+  BwdCommon c{q, q_st, q_sh, k, k_sr, k_sh, v, v_sr, v_sh, dO, do_st, do_sh, lse, lse_st, lse_sh, delta, delta_st,
+              delta_sh};
+  NsaBwdTileParams p = make_bwd(c, QH, KH, sm_scale);
+  p.dq = dq; p.dq_st = dq_st; p.dq_sh = dq_sh;
+  p.dq_partial = dq_partial; p.dqp_st = dqp_st; p.dqp_sh = dqp_sh;
+  p.x_cu = x_cu; p.k_cu = x_cu; p.c_cu = y_cu;
+  p.kernel_size = kernel_size; p.stride = stride; p.window = window;
+  p.all_below = all_below;
+  p.dO2 = (const bf16_t*)slc_dO; p.do2_st = sdo_st; p.do2_sh = sdo_sh;
+  p.lse2 = slc_lse; p.lse2_st = sl_st; p.lse2_sh = sl_sh;
+  p.delta2 = slc_delta; p.delta2_st = sd_st; p.delta2_sh = sd_sh;
+  p.ck = (const bf16_t*)ck; p.ck_sr = ck_sr; p.ck_sh = ck_sh;
+  p.cv = (const bf16_t*)cv; p.cv_sr = cv_sr; p.cv_sh = cv_sh;
+  p.dO3 = (const bf16_t*)cmp_dO; p.do3_st = cdo_st; p.do3_sh = cdo_sh;
+  p.lse3 = cmp_lse; p.lse3_st = cl_st; p.lse3_sh = cl_sh;
+  p.delta3 = cmp_delta; p.delta3_st = cd_st; p.delta3_sh = cd_sh;
+  return nsa_bwd_dq_tile_launch(p, 3, B, x_maxlen, D, VD, (hipStream_t)stream);
+}
+
 int nsa_swa_bwd_dq_tail(const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sr, int64_t k_sh,
                         const void* v, int64_t v_sr, int64_t v_sh, const void* dO, int64_t do_st, int64_t do_sh,
                         const float* lse, int64_t lse_st, int64_t lse_sh, const float* delta, int64_t delta_st,

@@ -131,6 +131,14 @@ struct NsaBwdTileParams {
   const bf16_t* dO2; int64_t do2_st, do2_sh;
   const float* lse2; int64_t lse2_st, lse2_sh;
   const float* delta2; int64_t delta2_st, delta2_sh;
+  // dq of the dense branches in one: the compressed rows, their offsets and dO3 / lse3 / delta3; below all_below dq goes to dq, in
+  // bf16, else to dq_partial
+  const bf16_t* ck; int64_t ck_sr, ck_sh;
+  const bf16_t* cv; int64_t cv_sr, cv_sh;
+  const int32_t* c_cu;
+  const bf16_t* dO3; int64_t do3_st, do3_sh;
+  const float* lse3; int64_t lse3_st, lse3_sh;
+  const float* delta3; int64_t delta3_st, delta3_sh;
   int q_chunk_tokens;          // compressed / window dkdv: query tokens per grid.x chunk
   int grid_chunks;             // window dkdv with dkv_mode 3 / 4: query chunks per key tile in grid.x
 };

@@ -11,6 +11,7 @@ namespace {
 constexpr int MODE_CMP = 0;
 constexpr int MODE_SWA = 1;
 constexpr int MODE_TAIL = 2;  // MODE_SWA; queries below all_below also take the keys before their window (selected branch)
+constexpr int MODE_ALL = 3;   // MODE_TAIL and the compressed branch: what is left for the selected branch alone
 
 template <int D, int VD, int MODE, int MINB, bool DO_LDS>
 __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams p) {
@@ -39,6 +40,10 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
   const int rows_total = xl * G;
   const int r0 = blockIdx.x * ROWS_WG;
   if (r0 >= rows_total) return;
+  constexpr bool TAIL = MODE == MODE_TAIL || MODE == MODE_ALL;
+  bool in_cmp = MODE == MODE_CMP;
+  const bf16_t *ksrc = p.k, *vsrc = p.v;
+  int64_t k_sr = p.k_sr, k_sh = p.k_sh, v_sr = p.v_sr, v_sh = p.v_sh;
   int nkeys, kbase;
   if (MODE == MODE_CMP) {
     kbase = p.k_cu[b];
@@ -111,13 +116,13 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
     for (int j = 0; j < KJ; j++) {
       int pc = tid + j * 256;
       int kr = min(pc / KP, last), dp = pc % KP;
-      kreg[j] = ld_global_b128(p.k + ((int64_t)kbase + kt + kr) * p.k_sr + (int64_t)kh * p.k_sh + dp * 8);
+      kreg[j] = ld_global_b128(ksrc + ((int64_t)kbase + kt + kr) * k_sr + (int64_t)kh * k_sh + dp * 8);
     }
 #pragma unroll
     for (int j = 0; j < VJ; j++) {
       int pc = tid + j * 256;
       int kr = min(pc / VP, last), dp = pc % VP;
-      vreg[j] = ld_global_b128(p.v + ((int64_t)kbase + kt + kr) * p.v_sr + (int64_t)kh * p.v_sh + dp * 8);
+      vreg[j] = ld_global_b128(vsrc + ((int64_t)kbase + kt + kr) * v_sr + (int64_t)kh * v_sh + dp * 8);
     }
   };
   // window: keys t + klo .. t + khi; before the window: keys .. t + khi, of queries at positions below t_end
@@ -141,12 +146,12 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
     if (kt + KT < key_end) gload(kt + KT);
     if (!wave_active) continue;
     bool any_vis, mask_hi, mask_lo = false;
-    if (MODE == MODE_CMP) {
+    if (MODE == MODE_CMP || (MODE == MODE_ALL && in_cmp)) {
       any_vis = tw_hi >= p.stride * kt + p.kernel_size - 1;
       mask_hi = tw_lo < p.stride * (kt + KT - 1) + p.kernel_size - 1 || kt + KT > nkeys;
     } else {
       any_vis = (kt <= tw_hi + khi) && (kt + KT - 1 >= tw_lo + klo);
-      mask_hi = kt + KT - 1 > tw_lo + khi || (MODE == MODE_TAIL && tw_hi >= t_end);
+      mask_hi = kt + KT - 1 > tw_lo + khi || (TAIL && tw_hi >= t_end);
       mask_lo = kt < tw_hi + klo;
     }
     if (!any_vis) continue;
@@ -216,22 +221,27 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
   }
 
   };
+  // the rows' incoming gradient, log-sum-exp and delta of another branch
+  auto take = [&](const bf16_t* g, int64_t g_st, int64_t g_sh, const float* l, int64_t l_st, int64_t l_sh, const float* d,
+                  int64_t d_st, int64_t d_sh) {
+    const bf16_t* dp = g + tok * g_st + (int64_t)head * g_sh + hl * 8;
+#pragma unroll
+    for (int kc = 0; kc < VD / 16; kc++) {
+      bf16x8 t8 = ld_global_b128(dp + kc * 16);
+      if (DO_LDS) *reinterpret_cast<bf16x8*>(&dOs[(wave * 32 + l32) * VLD + hl * 8 + kc * 16]) = t8;
+      else dof[kc] = t8;
+    }
+    lse = l[tok * l_st + (int64_t)head * l_sh];
+    delta = d[tok * d_st + (int64_t)head * d_sh];
+  };
   run_keys();
-  if constexpr (MODE == MODE_TAIL) {
+  if constexpr (TAIL) {
     // The selected branch of these queries inside the window has been folded into the window's incoming gradient; what
     // is left are the keys before the window.  40 samples of up to 1.2K tokens, 16 heads of 64: the selected dq kernel
     // 401 -> 51 us, this one 98 -> 110 us; 8 x 6K tokens, 64 heads of 128: 6829 -> 6080 and 1914 -> 1924 us.
     const int far_end = min(t_hi, p.all_below - 1) - p.window;  // keys before some query's window
     if (far_end > 0 && t_lo < p.all_below) {                    // workgroup-uniform
-      const bf16_t* dp = p.dO2 + tok * p.do2_st + (int64_t)head * p.do2_sh + hl * 8;
-#pragma unroll
-      for (int kc = 0; kc < VD / 16; kc++) {
-        bf16x8 t8 = ld_global_b128(dp + kc * 16);
-        if (DO_LDS) *reinterpret_cast<bf16x8*>(&dOs[(wave * 32 + l32) * VLD + hl * 8 + kc * 16]) = t8;
-        else dof[kc] = t8;
-      }
-      lse = p.lse2[tok * p.lse2_st + (int64_t)head * p.lse2_sh];
-      delta = p.delta2[tok * p.delta2_st + (int64_t)head * p.delta2_sh];
+      take(p.dO2, p.do2_st, p.do2_sh, p.lse2, p.lse2_st, p.lse2_sh, p.delta2, p.delta2_st, p.delta2_sh);
       key_begin = 0;
       key_end = far_end;
       klo = -0x40000000;
@@ -239,6 +249,23 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       t_end = p.all_below;
       key_lo = 0;
       key_hi = t < t_end ? t + khi : -1;
+      run_keys();
+    }
+  }
+  if constexpr (MODE == MODE_ALL) {
+    // Into the same accumulators, instead of a launch that reads the queries and the fp32 sum again.  dq, 16 / 2 heads of 64, two
+    // launches / one, us: 40 samples of up to 1.2K tokens 335 / 258, 80 of up to 600 224 / 153, 4K 55 / 41, 16K 262 / 233, 48K 1682 /
+    // 1259; whole steps 48K 5517 / 5365.
+    const int kc0 = p.c_cu[b];
+    nkeys = p.c_cu[b + 1] - kc0;
+    key_begin = 0;
+    key_end = t_hi >= p.kernel_size - 1 ? min((t_hi - p.kernel_size + 1) / p.stride + 1, nkeys) : 0;
+    if (key_end > 0) {  // workgroup-uniform
+      in_cmp = true;
+      ksrc = p.ck; vsrc = p.cv; k_sr = p.ck_sr; k_sh = p.ck_sh; v_sr = p.cv_sr; v_sh = p.cv_sh;
+      kbase = kc0;
+      take(p.dO3, p.do3_st, p.do3_sh, p.lse3, p.lse3_st, p.lse3_sh, p.delta3, p.delta3_st, p.delta3_sh);
+      key_hi = t >= p.kernel_size - 1 ? min((t - p.kernel_size + 1) / p.stride, nkeys - 1) : -1;
       run_keys();
     }
   }
@@ -253,7 +280,10 @@ __global__ __launch_bounds__(256, MINB) void bwd_dq_tile_kernel(NsaBwdTileParams
       int d = dt * 32 + i4 * 8 + hl * 4;
       f32x4 val = {dqacc[dt][i4 * 4 + 0] * osc, dqacc[dt][i4 * 4 + 1] * osc, dqacc[dt][i4 * 4 + 2] * osc,
                    dqacc[dt][i4 * 4 + 3] * osc};
-      if (p.dq_mode == 0) {
+      if (MODE == MODE_ALL) {
+        if (t < p.all_below) *reinterpret_cast<bf16x4*>((bf16_t*)p.dq + off + d) = pack4(val[0], val[1], val[2], val[3]);
+        else *reinterpret_cast<f32x4*>(p.dq_partial + tok * p.dqp_st + (int64_t)head * p.dqp_sh + d) = val;
+      } else if (p.dq_mode == 0) {
         *reinterpret_cast<bf16x4*>((bf16_t*)p.dq + off + d) = pack4(val[0], val[1], val[2], val[3]);
       } else if (p.dq_mode >= 3) {
         float* part = p.dq_partial + tok * p.dqp_st + (int64_t)head * p.dqp_sh + d;
@@ -297,6 +327,7 @@ int dispatch(const NsaBwdTileParams& p, int B, int max_q_len, int D, int VD, hip
 
 int nsa_bwd_dq_tile_launch(const NsaBwdTileParams& p, int mode, int B, int max_q_len, int D, int VD,
                            hipStream_t stream) {
+  if (mode == MODE_ALL) return dispatch<MODE_ALL>(p, B, max_q_len, D, VD, stream);
   if (mode == MODE_TAIL) return dispatch<MODE_TAIL>(p, B, max_q_len, D, VD, stream);
   return mode == MODE_CMP ? dispatch<MODE_CMP>(p, B, max_q_len, D, VD, stream)
                           : dispatch<MODE_SWA>(p, B, max_q_len, D, VD, stream);

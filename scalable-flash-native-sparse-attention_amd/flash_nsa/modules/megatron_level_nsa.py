@@ -20,7 +20,7 @@ from ..ops.topk import slc_topk_indices
 from ..ops.act import swiglu_fwd, swiglu_bwd, sigmoid_mul_fwd, sigmoid_mul_bwd
 from ..ops.combine import combine_bwd_gates
 from ..ops.sliding_window_attention import (short_fwd, slc_fwd_first_queries, swa_fwd, swa_fwd_tail, swa_bwd,
-                                            swa_bwd_dq_tail)
+                                            swa_bwd_dq_tail, dense_bwd_dq)
 
 
 # The backward runs on two streams, the dense dq kernels next to the dk/dv passes: batches that do not fill the GPU gain
@@ -259,19 +259,23 @@ class NSAFunction(torch.autograd.Function):
                 return dq, dk, dv, dw, dwk, dwv, None, None
 
         # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
-        # branches' and writes q's dtype (the compressed branch does for the queries that the gather leaves out).  Else it
-        # stores first, the window branch (matrix bound, with bandwidth to spare for the read-modify-write) adds, or stores
-        # where the selected branch left rows out, and the compressed branch adds and writes q's dtype.
-        dq32 = torch.empty(q.shape, device=q.device, dtype=torch.float32)
-        dq_last = torch.empty_like(q) if stored_ds else None
+        # branches', which one launch forms, and writes q's dtype (that launch does for the queries that the gather leaves out, and
+        # for short batches there are no others).  Else it stores first, the window branch (matrix bound, with bandwidth to spare
+        # for the read-modify-write) adds, or stores where the selected branch left rows out, and the compressed branch adds and
+        # writes q's dtype.
+        short = helper.x_maxlen <= all_below
+        dq32 = None if short else torch.empty(q.shape, device=q.device, dtype=torch.float32)
+        dq_last = torch.empty_like(q) if stored_ds or short else None
 
         def dq_chain():
-            if not stored_ds:
-                slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, _store_into(dq32), delta=delta[1], parts="dq",
-                             t_begin=all_below, **kw)
-            swa_bwd_dq_tail(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, dq32, store=stored_ds, **kw)
+            if dq_last is not None:
+                return dense_bwd_dq(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, cmp_k, cmp_v, cmp_lse, dcmp_o,
+                                    delta[0], dq_last, dq32, **kw)
+            slc_attn_bwd(q, k, v, topk, slc_o, lse_slc, do, _store_into(dq32), delta=delta[1], parts="dq",
+                         t_begin=all_below, **kw)
+            swa_bwd_dq_tail(q, k, v, lse_swa, do, delta[2], lse_slc, do, delta[1], all_below, dq32, **kw)
             return cmp_attn_bwd(q, cmp_k, cmp_v, cmp_o, cmp_lse, dcmp_o, dq32, delta=delta[0], finalize_dq=True,
-                                parts="dq", finalize_below=(dq_last, all_below) if stored_ds else None, **kw)[0]
+                                parts="dq", **kw)[0]
 
         def dkdv_raw(dq_after=None):
             # the window branch writes every element of dk / dv, the selected branch then adds to them

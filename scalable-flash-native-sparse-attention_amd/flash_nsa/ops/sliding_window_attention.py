@@ -97,6 +97,20 @@ def swa_bwd_dq_tail(q, k, v, lse, do, delta, slc_lse, slc_do, slc_delta, all_bel
               KH, D, VD, helper.window_size, default_scale(q, sm_scale), _lib.stream_ptr())
 
 
+def dense_bwd_dq(q, k, v, lse, do, delta, slc_lse, slc_do, slc_delta, all_below, cmp_k, cmp_v, cmp_lse, cmp_do, cmp_delta, dq, dq32=None,
+                 sm_scale=None, helper=NSAHelper):
+    """dq of the compressed branch and of swa_bwd_dq_tail's in one launch: the queries at positions below all_below into dq (q's dtype),
+    the others into the fp32 dq32 (None: there are none)."""
+    T, QH, D = q.shape
+    _, KH, VD = v.shape
+    st = lambda t: (None, 0, 0) if t is None else (t.data_ptr(), t.stride(0), t.stride(1))
+    _lib.call("nsa_bwd_dq_dense", *st(q), *st(k), *st(v), *st(do), *st(lse), *st(delta), *st(slc_do), *st(slc_lse), *st(slc_delta),
+              all_below, *st(cmp_k), *st(cmp_v), *st(cmp_do), cmp_lse.data_ptr(), cmp_lse.stride(1), cmp_lse.stride(0), *st(cmp_delta),
+              *st(dq), *st(dq32), helper.x_cu_seqlens.data_ptr(), helper.y_cu_seqlens.data_ptr(), helper.batch, helper.x_maxlen, QH, KH,
+              D, VD, helper.kernel_size, helper.stride, helper.window_size, default_scale(q, sm_scale), _lib.stream_ptr())
+    return dq
+
+
 def swa_bwd(q, k, v, o, lse, do, sm_scale=None, helper=NSAHelper, delta=None, dq=None, dkv_fp32=False, parts="both"):
     """Backward of the window branch.  Returns (dq, dk, dv); dq is a fresh bf16 tensor or the caller's fp32
     buffer (added into); dk/dv are fresh (bf16, or fp32 when dkv_fp32): one writer per element, or, for batches that do

@@ -206,3 +206,51 @@ def test_paged_selected_attention_rotates_blocks_in_long_chunks_only(device, KH,
     # P and o are rounded to bf16 once each in either: 4 * 2^-9 of the largest value
     assert (o.float() - ref.float()).abs().max() <= 2 ** -7 * v.float().abs().max()
     assert (lse - ref_lse).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,lens,kw", [
+    (16, 2, 64, 64, [1200, 31, 0, 33, 700], {}),
+    (8, 2, 64, 64, [1024, 1, 129], {}),                                    # nobody is at or above all_below
+    (6, 2, 32, 32, [300, 17], dict(top_n=4, window_size=50)),              # groups of 3; keys before the window
+    (12, 3, 128, 128, [90, 400], dict(top_n=2, num_init_blocks=1, num_local_blocks=1, window_size=200)),
+    (4, 1, 192, 128, [500], dict(top_n=4)),
+    (2, 1, 256, 256, [260], dict(top_n=2, window_size=64)),
+    (8, 1, 64, 64, [300], dict(kernel_size=16, stride=2, top_n=3)),        # several tiles of compressed keys
+])
+def test_dense_dq_in_one_launch_equals_two(device, QH, KH, D, VD, lens, kw):
+    """Window, keys before it and compressed branch in one launch against the window's launch and the compressed branch's that adds
+    to it: the same products summed in fp32 in another order, so the fp32 rows to 1e-5 and the bf16 ones to a rounding."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.compress_attn import cmp_attn_bwd, cmp_attn_fwd
+    from flash_nsa.ops.compress_kv import mean_pooling_fwd
+    from flash_nsa.ops.sliding_window_attention import dense_bwd_dq, swa_bwd_dq_tail, swa_fwd
+    T = sum(lens)
+    try:
+        NSAHelper.set_hyperparameters(**kw)
+        NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+        below, short = NSAHelper.all_below(), max(lens) <= NSAHelper.all_below()
+        q, k, v, _ = [t.to(device) for t in make_qkvw(T, QH, KH, D, VD, seed=120)]
+        ck, cv = mean_pooling_fwd(k), mean_pooling_fwd(v)
+        _, cmp_lse = cmp_attn_fwd(q, ck, cv)
+        _, lse = swa_fwd(q, k, v)
+        do, cmp_do = [randn_bf16(T, QH, VD, seed=s).to(device) for s in (125, 126)]
+        delta = torch.randn(3, T, QH, generator=torch.Generator().manual_seed(127)).to(device)
+        slc_lse = lse + 1
+        nan = lambda dtype: torch.full((T, QH, D), float("nan"), device=device, dtype=dtype)
+        want32, want = nan(torch.float32), nan(torch.bfloat16)
+        swa_bwd_dq_tail(q, k, v, lse, do, delta[2], slc_lse, do, delta[1], below, want32, store=True)
+        cmp_attn_bwd(q, ck, cv, None, cmp_lse, cmp_do, want32, delta=delta[0], finalize_dq=True, parts="dq",
+                     finalize_below=(want, below))
+        got32, got = None if short else nan(torch.float32), nan(torch.bfloat16)
+        dense_bwd_dq(q, k, v, lse, do, delta[2], slc_lse, do, delta[1], below, ck, cv, cmp_lse, cmp_do, delta[0], got, got32)
+    finally:
+        NSAHelper.set_hyperparameters()
+    low = torch.cat([torch.arange(n) < below for n in lens]).to(device)
+    a, b = got[low].float(), want[low].float()
+    # (a step between neighbours of bf16 is up to 2^-7 of the value; sums that cancel: fp32 of the row's largest value)
+    over = (a - b).abs() - 2.0 ** -7 * b.abs() - 1e-5 * b.abs().amax(-1, keepdim=True)
+    assert float(over.max()) <= 0, (float(over.max()), float((a != b).float().mean()))
+    if not short:
+        a, b = got32[~low], want32[~low]
+        assert float((a - b).norm() / b.norm()) < 1e-5, float((a - b).norm() / b.norm())
+        assert bool(got[~low].isnan().all()) and bool(got32[low].isnan().all())  # written by nobody
