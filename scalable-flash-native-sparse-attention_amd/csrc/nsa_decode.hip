@@ -578,13 +578,13 @@ NSA_DEVICE int select_blocks_lds(float* imp, int t, int nb_cap, const NsaDecodeP
   return result;
 }
 
-// cand_v / cand_i: 64 floats + 64 ints of LDS private to the selecting wave
-template <int UNROLL>
+// cand_v / cand_i: 64 floats (16-byte aligned) + 64 ints of LDS private to the selecting wave
+template <bool SHORT_CODE>
 NSA_DEVICE int select_blocks_wave(float* imp, int t, int nb_cap, const NsaDecodeParams& p, int lane, float* cand_v,
                                   int* cand_i) {
-  if (nb_cap <= 512) return select_blocks_short_list<UNROLL, 8>(imp, t, nb_cap, p, lane, cand_v, cand_i);
-  if (nb_cap <= 1024) return select_blocks_short_list<UNROLL, 16>(imp, t, nb_cap, p, lane, cand_v, cand_i);
-  if (nb_cap <= 2048) return select_blocks_short_list<UNROLL, 32>(imp, t, nb_cap, p, lane, cand_v, cand_i);
+  if (nb_cap <= 512) return select_blocks_short_list<SHORT_CODE, 8>(imp, t, nb_cap, p, lane, cand_v, cand_i);
+  if (nb_cap <= 1024) return select_blocks_short_list<SHORT_CODE, 16>(imp, t, nb_cap, p, lane, cand_v, cand_i);
+  if (nb_cap <= 2048) return select_blocks_short_list<SHORT_CODE, 32>(imp, t, nb_cap, p, lane, cand_v, cand_i);
   return select_blocks_lds(imp, t, nb_cap, p, lane);
 }
 
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_cmp_topk_kernel(NsaDeco
   __syncthreads();
   if (wave != 0) return;
   // the waves' partial statistics are consumed: their space is the selector's candidate list
-  const int result = select_blocks_wave<64>(imp, t, p.nb_cap, p, lane, part_m, reinterpret_cast<int*>(part_l));
+  const int result = select_blocks_wave<false>(imp, t, p.nb_cap, p, lane, part_m, reinterpret_cast<int*>(part_l));
   if (lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + (int64_t)b * p.tk_st + lane] = result;
 }
 
@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void decode_slc_swa_kernel(NsaDecod
   uf.init(p.q + (int64_t)b * p.q_st + (int64_t)head * p.q_sh, p.scale_log2, lane, Vs_all + wave * SLOT);
   const int w_first = select_here ? 1 : 0;
   if (wave < w_first) {
-    const int result = select_blocks_wave<64>(imp, t, nb, p, lane, cand_v, cand_i);
+    const int result = select_blocks_wave<false>(imp, t, nb, p, lane, cand_v, cand_i);
     blk_s[lane] = lane < nvalid ? max(result, 0) : 0;
     if (p.topk && part == 0 && lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + (int64_t)b * p.tk_st + lane] = result;
   } else {
@@ -1497,7 +1497,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_fused_kernel(NsaDecodeParam
   const int nvalid = t >= 0 ? min(p.top_n, t / Bs + 1) : 0;
   uf.reset();
   if (wave == 0) {
-    const int result = select_blocks_wave<8>(imp, t, p.nb_cap, p, lane, cand_v, cand_i);
+    const int result = select_blocks_wave<true>(imp, t, p.nb_cap, p, lane, cand_v, cand_i);
     blk_s[lane] = lane < nvalid ? max(result, 0) : 0;
     if (p.topk && lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + (int64_t)b * p.tk_st + lane] = result;
   } else {

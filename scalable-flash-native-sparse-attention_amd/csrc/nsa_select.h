@@ -91,20 +91,73 @@ NSA_DEVICE float wave_fmax_uniform(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 63));
 }
 
-// The same selection as select_blocks_regs over a short list instead of the NV registers of every lane: the R-th largest
-// of the 64 lane maxima is a lower bound of the R-th largest score (R = number of scored slots), so only the scores at or
+// A theta that at least `rounds` lanes' m reach, -1 where fewer hold a score (scores are not negative): their bits order as
+// integers do.  Halved between the wave's maximum and 2^-16 of it (or 0, if too few reach that) until at most SLACK lanes more
+// than `rounds` reach theta: every lower bound of the rounds-th largest score selects the same, only the list gets longer.
+template <bool SHORT_CODE>
+NSA_DEVICE float lane_bound(float m, int rounds) {
+  if constexpr (SHORT_CODE) {  // the largest such m: every lane compares its own with all others
+    int above = 0;
+#pragma unroll 8
+    for (int j = 0; j < 64; j++)
+      above += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j)) > m;
+    return fmaxf(-wave_fmax_uniform(above < rounds ? -m : -__builtin_inff()), -1.f);
+  }
+  constexpr int SLACK = 3;
+  const int key = __builtin_bit_cast(int, m);
+  auto reach = [&](int at) { return (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key >= at)); };
+  const int top = max(__builtin_bit_cast(int, wave_fmax_uniform(m)), 0);
+  int lo = max(top - (16 << 23), 0), n = reach(lo);
+  if (n < rounds) {
+    lo = 0;
+    n = reach(0);
+    if (n < rounds) return -1.f;
+  }
+  int width = top - lo;  // (the maximum itself: fewer than `rounds` above it)
+  while (n > rounds + SLACK && width > 0) {
+    const int half = (width + 1) >> 1, at = reach(lo + half);
+    if (at >= rounds) {
+      lo += half;
+      width -= half;
+      n = at;
+    } else {
+      width = half - 1;
+    }
+  }
+  return __builtin_bit_cast(float, lo);
+}
+
+// Makes the loads of all N values precede the first use of one (else the compiler puts each behind the condition under which it is
+// used, and one round trip after another is waited for)
+template <int N>
+NSA_DEVICE void load_together(float (&v)[N]) {
+  static_assert(N == 2 || N % 4 == 0, "");
+  if constexpr (N == 2) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]));
+  } else if constexpr (N == 4) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; k += 8)
+      asm volatile("" : "+v"(v[k]), "+v"(v[k + 1]), "+v"(v[k + 2]), "+v"(v[k + 3]), "+v"(v[k + 4]), "+v"(v[k + 5]), "+v"(v[k + 6]),
+                        "+v"(v[k + 7]));
+  }
+}
+
+// The same selection as select_blocks_regs over a short list instead of the NV registers of every lane: a lower bound of the R-th
+// largest of the 64 lane maxima is one of the R-th largest score (R = number of scored slots), so only the scores at or
 // above it can be selected; they are compacted (ballot + prefix count) into a wave-private list of at most 64 entries in LDS
-// (cand_v / cand_i), one per lane, in ascending order of the block.  The picks and their order are those of
+// (cand_v, 16-byte aligned, / cand_i), one per lane, in ascending order of the block.  The picks and their order are those of
 // select_blocks_regs (descending score, lowest index on ties); rows with more than 64 scores at the bound (many equal values)
 // take that function.
-// Bound and places come from counting: every lane compares its value with all others, broadcast one by one, which are
-// independent instructions.  (Repeated wave-wide maxima are a dependent chain of about 200 ns per round, twice R of them: one
-// request of 32K tokens, 512 blocks, the selection 5.5 -> 2.7 us; 16 of 128K, 2048 blocks, 8.0 -> 5.1; in the one-launch decode
-// kernel, beside the window, 24 requests of 1K to 4K, 16 / 2 heads of 64, 28.9 -> 26.7 us, 64 / 4 heads of 128, 33.8 -> 33.3.)
-// UNROLL: of the bound's loop.  64 where nothing runs beside the selection (with 8 one request of 32K tokens 35.5 -> 35.7 us);
-// 8 in the one-launch kernel, where more code costs batches that wait for memory and not for this (64 requests of 4K to 32K
-// tokens 73.8 us with maxima, 73.8 with 8, 74.2 with 64; 64 of up to 2K 46.1, 46.4, 46.6).
-template <int UNROLL, int NV, class P>
+// Places come from counting: every entry is compared with all others, which are independent instructions.  (Repeated wave-wide
+// maxima are a dependent chain of about 200 ns per round, twice R of them: one request of 32K tokens, 512 blocks, the selection
+// 5.5 -> 2.7 us; 16 of 128K, 2048 blocks, 8.0 -> 5.1.)
+// SHORT_CODE: bound and places with one broadcast per lane and entry, and scores loaded as they are used: for the one-launch decode
+// kernel, where more code costs batches that wait for memory and not for this (512 requests of 4K tokens 327.8 us; 330.8 with the
+// other form, which gains the split kernel's 16 of 128K 1 %, 8 of 2K to 8K with 16 / 2 heads of 64 25.6 -> 24.8 us, and a wave per
+// row of the training and prefill path 460 -> 175 vector instructions).
+template <bool SHORT_CODE, int NV, class P>
 NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, const P& p, int lane, float* cand_v,
                                         int* cand_i) {
   const int nk = t >= 0 ? t / p.block_size : -1;
@@ -122,47 +175,68 @@ NSA_DEVICE int select_blocks_short_list(const float* imp, int t, int nb_cap, con
   float v[NV];
   float m = -3.f;
 #pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = !SHORT_CODE || lane + 64 * k <= jmax ? imp[min(lane + 64 * k, jmax)] : -3.f;
+  if constexpr (!SHORT_CODE) load_together(v);
+#pragma unroll
   for (int k = 0; k < NV; k++) {
     const int j = lane + 64 * k;
-    float x = j <= jmax ? imp[min(j, nb_cap - 1)] : -3.f;
-    if (j <= jmax && (j < p.num_init || j > nk - p.num_local)) x = -1.f;  // forced blocks: behind every real score
-    v[k] = x;
+    float x = j < p.num_init || j > nk - p.num_local ? -1.f : v[k];  // forced blocks: behind every real score
+    v[k] = x = j <= jmax ? x : -3.f;
     m = fmaxf(m, x);
   }
-  // bound: the smallest lane maximum that fewer than `rounds` exceed; -1 where fewer lanes than rounds hold a candidate
-  int above = 0;
-#pragma unroll UNROLL
-  for (int j = 0; j < 64; j++)
-    above += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j)) > m;
-  const float theta = fmaxf(-wave_fmax_uniform(above < rounds ? -m : -__builtin_inff()), -1.f);
+  const float theta = lane_bound<SHORT_CODE>(m, rounds);
+  if (!SHORT_CODE) cand_v[lane] = -3.f;  // (behind the last entry)
   // compaction of the scores >= theta, register by register (ascending block number within a register)
   int base = 0;
 #pragma unroll
   for (int k = 0; k < NV; k++) {
-    const bool q = v[k] >= theta;
-    const uint64_t mask = __builtin_amdgcn_ballot_w64(q);
-    const int pos = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-    if (q && pos < 64) { cand_v[pos] = v[k]; cand_i[pos] = lane + 64 * k; }
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(v[k] >= theta);
+    const int pos = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, (uint32_t)base));
+    if (v[k] >= theta && pos < 64) { cand_v[pos] = v[k]; cand_i[pos] = lane + 64 * k; }
     base += __builtin_popcountll(mask);
   }
-  if (base > 64) return select_blocks_regs<NV>(imp, t, nb_cap, p, lane);  // wave-uniform
+  if (base > 64) return select_blocks_regs<(NV < 8 ? 8 : NV)>(imp, t, nb_cap, p, lane);  // wave-uniform
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float cv = lane < base ? cand_v[lane] : -3.f;
-  const int ci = lane < base ? cand_i[lane] : 0;
+  const float cv = !SHORT_CODE || lane < base ? cand_v[lane] : -3.f;
+  const int ci = !SHORT_CODE || lane < base ? cand_i[lane] : 0;
   int place = 0;  // scores ahead of this lane's: greater ones, and equal ones of lower blocks
-#pragma unroll 4
-  for (int j = 0; j < base; j++) {
-    const float other = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cv), j));
-    place += other > cv || (other == cv && j < lane);
+  auto store = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane < base && place < rounds) cand_i[place] = ci;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  bool equal = SHORT_CODE || base > 32;
+  if (!equal) {
+    // the two halves of the wave compare the same 32 entries with 16 each, read as they lie instead of broadcast lane by lane
+    const float mine = cand_v[lane & 31];
+    const f32x4* others = reinterpret_cast<const f32x4*>(cand_v + (lane >> 5) * 16);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f32x4 o = others[i];
+#pragma unroll
+      for (int e = 0; e < 4; e++) place += o[e] > mine;
+    }
+    const auto both = __builtin_amdgcn_permlane32_swap((uint32_t)place, (uint32_t)place, false, false);
+    place = (int)(both[0] + both[1]);
+    store();
+    // equal scores have taken the same place: only one of them finds itself there
+    const bool lost = lane < base && place < rounds && cand_i[min(place, 63)] != ci;
+    equal = __builtin_amdgcn_ballot_w64(lost) != 0;
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  if (lane < base && place < rounds) cand_i[place] = ci;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (equal) {
+    place = 0;
+#pragma unroll 4
+    for (int j = 0; j < base; j++) {
+      const float other = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cv), j));
+      place += other > cv || (other == cv && j < lane);
+    }
+    store();
+  }
   if (lane >= forced && lane < nsel) result = lane - forced < base ? cand_i[lane - forced] : 0x7fffffff;
   return result;
 }

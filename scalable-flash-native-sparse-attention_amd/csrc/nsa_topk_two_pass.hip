@@ -10,7 +10,11 @@
 //                      are folded into the scores of the selection blocks the tile completes (overlap weights
 //                      area/stride, ascending key order) and stored.  128 registers: four waves per SIMD.
 //   topk_pick_kernel   one wave per (kv head, token): the visible scores of the row in registers, forced initial and
-//                      local blocks first, then repeated arg-max (lowest index on ties).
+//                      local blocks first, then the largest scores (lowest index on ties).  Bound by the instructions per
+//                      row and by waits for its scores, not by their bytes: all loads of a row in flight, as many registers
+//                      as its blocks need, sequence and bounds in one round trip; us with 8 registers per row loaded one by
+//                      one and 460 vector instructions / now, 175: 16 chunks of 2K at 0 to 16K 144 / 111, 16K of 2 kv heads
+//                      36 / 24.  (Several rows per wave, 8 waves per group: no faster.)
 //
 // The one-launch kernel of nsa_topk.hip keeps the scores of its tokens in LDS, which holds it at two waves per SIMD;
 // it remains the path for shapes this one does not take (more than 16 q-heads per kv head, selection blocks that are
@@ -275,41 +279,48 @@ struct PickParams {
   int block_size, top_n, num_init, num_local, ignore_index, t_begin;
 };
 
+// MAXNV: selection blocks that any row can hold, by 64
+template <int MAXNV>
 __global__ __launch_bounds__(256) void topk_pick_kernel(PickParams p) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t r = (int64_t)blockIdx.x * 4 + wave;
-  if (r >= (int64_t)p.KH * p.ntok) return;
-  const int kh = (int)(r / p.ntok);
-  const int tr = (int)(r - (int64_t)kh * p.ntok);
-  const int64_t tok = (int64_t)p.tok_lo + tr;
-  // sequence of the token: its number of sequence ends at or before the token, counted 64 at a time
-  int b = 0;
-  for (int i0 = 0; i0 < p.B; i0 += 64) {
-    const bool before = i0 + lane < p.B && p.x_cu[i0 + lane + 1] <= tok;
-    b += (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
+  const int kh = blockIdx.y;
+  const int tr = blockIdx.x * 4 + wave;
+  if (tr >= p.ntok) return;
+  const int tok = p.tok_lo + tr;
+  // sequence of the token: its number of sequence ends at or before the token, counted 64 at a time; with it its bounds
+  int n = 64, t_of = 0;
+  for (int i0 = 0; i0 < p.B && n == 64; i0 += 64) {
+    const int i = min(i0 + lane, p.B - 1);
+    const int begin = p.x_cu[i], end = p.x_cu[i + 1];
+    t_of = (p.ctx_lens != nullptr ? p.ctx_lens[i] : end - begin) - end;
+    n = (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(end <= tok));
   }
-  if (b >= p.B) return;  // past the last sequence
-  const int x_end = p.x_cu[b + 1];
-  const int t = __builtin_amdgcn_readfirstlane((p.ctx_lens != nullptr ? p.ctx_lens[b] : x_end - p.x_cu[b]) - x_end +
-                                               (int)tok);
+  if (n == 64) return;  // past the last sequence
+  const int t = __builtin_amdgcn_readlane(t_of, n) + tok;
   if (t < p.t_begin) return;
-  const float* imp = p.imp + r * p.row_stride;
+  const float* imp = p.imp + ((int64_t)kh * p.ntok + tr) * p.row_stride;
   const int nk = t / p.block_size;
   const int jmax = min(nk, p.nb_max - 1);
   if (p.imp_out != nullptr) {
-    float* dst = p.imp_out + (int64_t)kh * p.imp_sh + tok * p.imp_st;
+    float* dst = p.imp_out + (int64_t)kh * p.imp_sh + (int64_t)tok * p.imp_st;
     for (int j = lane; j < p.imp_cols; j += 64) dst[j] = j <= jmax ? imp[j] : 0.f;
   }
   // candidates per lane sized by the row's own number of visible blocks (wave-uniform)
   const int cap = min(p.nb_max, p.row_stride);
-  __shared__ float cand_v[4][64];
+  __shared__ __attribute__((aligned(16))) float cand_v[4][64];
   __shared__ int cand_i[4][64];
   int result;
-  if (jmax < 512) result = select_blocks_short_list<64, 8>(imp, t, min(cap, 512), p, lane, cand_v[wave], cand_i[wave]);
-  else if (jmax < 1024) result = select_blocks_short_list<64, 16>(imp, t, min(cap, 1024), p, lane, cand_v[wave], cand_i[wave]);
-  else result = select_blocks_short_list<64, 32>(imp, t, min(cap, 2048), p, lane, cand_v[wave], cand_i[wave]);
-  if (lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + tok * p.tk_st + lane] = result;
+  auto select = [&](auto nv) {
+    constexpr int NV = decltype(nv)::value < MAXNV ? decltype(nv)::value : MAXNV;
+    result = select_blocks_short_list<false, NV>(imp, t, min(cap, NV * 64), p, lane, cand_v[wave], cand_i[wave]);
+  };
+  if (jmax < 128) select(std::integral_constant<int, 2>{});
+  else if (jmax < 256) select(std::integral_constant<int, 4>{});
+  else if (MAXNV <= 8 || jmax < 512) select(std::integral_constant<int, 8>{});
+  else if (MAXNV <= 16 || jmax < 1024) select(std::integral_constant<int, 16>{});
+  else select(std::integral_constant<int, 32>{});
+  if (lane < p.top_n) p.topk[(int64_t)kh * p.tk_sh + (int64_t)tok * p.tk_st + lane] = result;
 }
 
 template <int D, int GP, bool PAGED>
@@ -375,8 +386,10 @@ int nsa_topk_two_pass_launch(const NsaTopkParams& p, bool paged, int B, int max_
     pp.ntok = ntok; pp.tok_lo = (int)lo; pp.row_stride = rs; pp.nb_max = p.nb_max; pp.KH = p.KH;
     pp.block_size = p.block_size; pp.top_n = p.top_n; pp.num_init = p.num_init; pp.num_local = p.num_local;
     pp.ignore_index = p.ignore_index;
-    const int64_t rows = (int64_t)p.KH * ntok;
-    topk_pick_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, stream>>>(pp);
+    const dim3 groups((unsigned)((ntok + 3) / 4), p.KH);
+    if (p.nb_max <= 512) topk_pick_kernel<8><<<groups, 256, 0, stream>>>(pp);
+    else if (p.nb_max <= 1024) topk_pick_kernel<16><<<groups, 256, 0, stream>>>(pp);
+    else topk_pick_kernel<32><<<groups, 256, 0, stream>>>(pp);
     rc = nsa_check_launch("topk_pick_kernel");
     if (rc) return rc;
   }

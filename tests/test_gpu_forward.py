@@ -418,3 +418,47 @@ def test_short_batches_in_one_launch_equal_two(device, QH, KH, D, VD, lens, kw):
     for got, ref in zip(one[:3], want):
         assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
     assert torch.equal(one[3], out) and torch.equal(bare, out)
+
+
+@pytest.mark.parametrize("lens,kind,kw", [
+    ([66100], "random", {}),                                    # every list length, registers per lane changing on the way
+    ([9000], "random", dict(top_n=48)),                         # more picks than half a wave holds
+    ([8200, 17000], "pairs", {}),                               # equal scores in pairs
+    ([8200], "few", {}),                                        # seven different scores
+    ([5000], "zero", {}), ([5000], "large", {}),
+    ([70] * 100 + [0, 2100, 1, 0], "random", dict(top_n=8)),    # sequences counted in two steps
+])
+def test_block_selection_is_that_of_its_scores(device, lens, kind, kw):
+    """Picks of the two-launch selector against a stable descending sort of the scores that it returns: exact."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.topk import slc_topk_indices
+    T, QH, KH, D = sum(lens), 4, 2, 64
+    g = torch.Generator().manual_seed(31)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).to(device)
+    try:
+        NSAHelper.set_hyperparameters(**kw)
+        NSAHelper.init_cu_seqlens(cu)
+        h = NSAHelper
+        Y = int(h.y_cu_seqlens[-1])
+        q = torch.randn(T, QH, D, generator=g).bfloat16().to(device)
+        rows = torch.randn(Y, KH, D, generator=g).bfloat16().to(device)
+        period = dict(pairs=Y // 2 // 4 * 4, few=28).get(kind, Y)  # (4 compressed rows per selection block)
+        ck = rows[torch.arange(Y, device=device) % period].contiguous()
+        lse = torch.full((QH, T), dict(zero=1e4, large=-60.0).get(kind, 4.0), device=device)
+        topk, probs = slc_topk_indices(q, ck, lse, return_slc_prob=True)
+        top_n, init, local, bs = h.top_n, h.num_init_blocks, h.num_local_blocks, h.block_size
+        ignore = -(-max(lens) // bs)
+        t = torch.cat([torch.arange(n) for n in lens]).to(device)
+        for r0 in range(0, T, 16384):
+            nk = t[r0:r0 + 16384, None] // bs
+            p, got = probs[:, r0:r0 + 16384], topk[:, r0:r0 + 16384]
+            j = torch.arange(p.size(-1), device=device)
+            free = (j >= init) & (j <= nk - local)
+            order = torch.where(free, p, -1.0).sort(dim=-1, descending=True, stable=True).indices
+            slot = torch.arange(top_n, device=device)
+            want = order[..., (slot - init - local).clamp(min=0)]
+            want = torch.where(slot < init, slot, torch.where(slot < init + local, nk - (slot - init), want))
+            want = torch.where(slot <= nk, want, ignore)
+            assert torch.equal(got, want.int()), (got != want).nonzero()[:4]
+    finally:
+        NSAHelper.set_hyperparameters()
