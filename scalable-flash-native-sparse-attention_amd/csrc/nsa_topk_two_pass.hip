@@ -14,7 +14,8 @@
 //                      row and by waits for its scores, not by their bytes: all loads of a row in flight, as many registers
 //                      as its blocks need, sequence and bounds in one round trip; us with 8 registers per row loaded one by
 //                      one and 460 vector instructions / now, 175: 16 chunks of 2K at 0 to 16K 144 / 111, 16K of 2 kv heads
-//                      36 / 24.  (Several rows per wave, 8 waves per group: no faster.)
+//                      36 / 24, 8 x 4K to 8K of 4 kv heads 163 / 103, 64K 388 / 231.  (Several rows per wave, 8 waves per
+//                      group: no faster.)
 //
 // The one-launch kernel of nsa_topk.hip keeps the scores of its tokens in LDS, which holds it at two waves per SIMD;
 // it remains the path for shapes this one does not take (more than 16 q-heads per kv head, selection blocks that are
