@@ -5,7 +5,10 @@
 // All three are bound by round trips to memory and LDS, not by bytes, and stand on the critical path in front of the
 // selected dK/dV kernel.  us for count + scan + fill, with one search per entry, a scan and a fill that wait for every
 // element -> as below: one sequence of 4K tokens, 1 kv head 79 -> 24, 40 of up to 1.2K, 2 kv heads 101 -> 31, 8 x 6K,
-// 4 kv heads 149 -> 58, 64K 171 -> 82.
+// 4 kv heads 149 -> 58, 64K 171 -> 82.  Four threads per token, and sequences found at one look, fill alone: 40 of up to 1.2K
+// 14 -> 8, 4K 14 to 29 -> 10, 16K 19 -> 12 (a chunk's workgroup is often alone on its CU: one wave per SIMD before).  Reading 32
+// chunk counts at a time in the scan takes 109 registers a thread, and the launch then waits for the kernels beside it: 8 x 6K
+// 34 -> 217.
 // Upstream: flash_nsa/ops/topk.py:782-945 (get_bind_from_find, dense scatter + per-row sort).
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
@@ -26,18 +29,26 @@ __device__ __forceinline__ int find_seq(const int32_t* x_cu, int B, int tok) {
   return lo;
 }
 
-// One thread per query token: where its sequence's blocks begin, how many there are and how many slots of its selection
+// The same for a token that is the same in all lanes: up to 64 sequences in one round trip to memory
+__device__ __forceinline__ int find_seq_uniform(const int32_t* x_cu, int B, int tok) {
+  if (B > 64) return find_seq(x_cu, B, tok);
+  const int lane = lane_id();
+  const bool from = x_cu[min(lane, B - 1)] <= tok && lane > 0 && lane < B;
+  return (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(from));
+}
+
+// A query token of the sequences b0 .. b1: where its sequence's blocks begin, how many there are and how many slots of its selection
 // count.  (One search per token; one per entry was most of the counting kernel.)
 struct TokenRow {
   const int32_t* slots;
   int n, kb, nb, nvalid;
 };
 __device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
-                                              const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok, int t1, int kh,
-                                              int block_size, int t_begin) {
+                                              const int32_t* x_cu, const int32_t* kblk_cu, int b0, int b1, int tok, int t1,
+                                              int kh, int block_size, int t_begin) {
   TokenRow r{topk, 0, 0, 0, 0};
   if (tok >= t1) return r;
-  const int b = find_seq(x_cu, B, tok);
+  const int b = b0 + find_seq(x_cu + b0, b1 - b0 + 1, tok);
   if (tok >= x_cu[b + 1]) return r;  // behind the last sequence
   r.slots = topk + (int64_t)kh * tk_sh + (int64_t)tok * tk_st;
   r.n = tok - x_cu[b];
@@ -46,12 +57,12 @@ __device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh
   r.nvalid = r.n >= t_begin ? min(top_n, r.n / block_size + 1) : 0;
   return r;
 }
-// fn(global block, slot) for every block that the token selected; the ids are fetched ROW at a time, so that they share one
-// round trip to memory
-constexpr int ROW = 16;
+// fn(global block, slot) for the blocks that the token selected, slots ROW part .. ROW part + ROW - 1 of every ROW * PARTS: PARTS
+// threads share a token; the ids are fetched ROW at a time, so that they share one round trip to memory
+constexpr int PARTS = 4, ROW = 4, NT = 256 * PARTS;
 template <class Fn>
-__device__ __forceinline__ void for_each_block(const TokenRow& r, Fn fn) {
-  for (int s0 = 0; s0 < r.nvalid; s0 += ROW) {
+__device__ __forceinline__ void for_each_block(const TokenRow& r, int part, Fn fn) {
+  for (int s0 = part * ROW; s0 < r.nvalid; s0 += ROW * PARTS) {
     int j[ROW];
 #pragma unroll
     for (int s = 0; s < ROW; s++) j[s] = s0 + s < r.nvalid ? r.slots[s0 + s] : -1;
@@ -61,25 +72,28 @@ __device__ __forceinline__ void for_each_block(const TokenRow& r, Fn fn) {
   }
 }
 
-// grid (nchunks, KH), 256 threads, dynamic LDS nblk ints
-__global__ __launch_bounds__(256) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+// grid (nchunks, KH), dynamic LDS nblk ints
+__global__ __launch_bounds__(NT) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
                                                         const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
                                                         int T, int nblk, int block_size, int t_begin,
                                                         int32_t* chunk_cnt) {
   extern __shared__ int hist[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
-  for (int i = threadIdx.x; i < nblk; i += 256) hist[i] = 0;
+  const int part = threadIdx.x >> 8;
+  for (int i = threadIdx.x; i < nblk; i += NT) hist[i] = 0;
   __syncthreads();
   const int CT = counting_chunk(T);
   const int t0 = tok0 + chunk * CT;
   const int t1 = min(tok0 + T, t0 + CT);
+  const int b0 = find_seq_uniform(x_cu, B, t0), b1 = find_seq_uniform(x_cu, B, t1 - 1);
   for (int tb = t0; tb < t1; tb += 256) {
-    const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + threadIdx.x, t1, kh, block_size, t_begin);
-    for_each_block(r, [&](int jb, int) { atomicAdd(&hist[jb], 1); });
+    const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, b0, b1, tb + (threadIdx.x & 255), t1, kh, block_size,
+                                 t_begin);
+    for_each_block(r, part, [&](int jb, int) { atomicAdd(&hist[jb], 1); });
   }
   __syncthreads();
   int32_t* dst = chunk_cnt + ((int64_t)kh * gridDim.x + chunk) * nblk;
-  for (int i = threadIdx.x; i < nblk; i += 256) dst[i] = hist[i];
+  for (int i = threadIdx.x; i < nblk; i += NT) dst[i] = hist[i];
 }
 
 // grid (KH), 1024 threads: chunk counts -> chunk bases (in place), list offsets, work-item offsets
@@ -139,13 +153,13 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
   }
 }
 
-// grid (nchunks, KH), 256 threads: in-order fill.  The position of a token in a block's list is the number of earlier
+// grid (nchunks, KH): in-order fill.  The position of a token in a block's list is the number of earlier
 // tokens that selected the block.  256 tokens at a time set their bit in the block's 256-bit mask, so the count is that
 // of the bits below the token's own and no token waits for another (a wave that walked the tokens one by one took as
 // long as 256 dependent LDS updates, whatever the size of the batch).  LDS holds the masks of FILL_BLOCKS blocks; more
 // blocks than that are taken in several rounds.
 constexpr int FILL_BLOCKS = 1024, FILL_WORDS = 256 / 32;
-__global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+__global__ __launch_bounds__(NT) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
                                                        const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
                                                        int T, int nblk, int block_size, int t_begin,
                                                        const int32_t* chunk_base, const int32_t* csr_off,
@@ -153,7 +167,7 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int6
   __shared__ int cursor[FILL_BLOCKS];
   __shared__ __attribute__((aligned(16))) uint32_t mask[FILL_BLOCKS * FILL_WORDS];
   const int chunk = blockIdx.x, kh = blockIdx.y;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, part = tid >> 8, row = tid & 255;
   const int CT = counting_chunk(T);
   const int t0 = tok0 + chunk * CT;
   const int t1 = min(tok0 + T, t0 + CT);
@@ -161,23 +175,24 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int6
   const int32_t* base = chunk_base + ((int64_t)kh * gridDim.x + chunk) * nblk;
   const int32_t* off = csr_off + (int64_t)kh * (nblk + 1);
   // the blocks of this chunk's sequences
-  const int b0 = find_seq(x_cu, B, t0), b1 = find_seq(x_cu, B, t1 - 1);
+  const int b0 = find_seq_uniform(x_cu, B, t0), b1 = find_seq_uniform(x_cu, B, t1 - 1);
   const int blk_lo = kblk_cu[b0];
   const int blk_hi = kblk_cu[b1 + 1];
-  const int word = tid >> 5;
-  const uint32_t bit = 1u << (tid & 31);
+  const int word = row >> 5;
+  const uint32_t bit = 1u << (row & 31);
   for (int r0 = blk_lo; r0 < blk_hi; r0 += FILL_BLOCKS) {
     const int nr = min(FILL_BLOCKS, blk_hi - r0);
-    for (int i = tid; i < nr; i += 256) cursor[i] = base[r0 + i] + off[r0 + i];
+    for (int i = tid; i < nr; i += NT) cursor[i] = base[r0 + i] + off[r0 + i];
     for (int tb = t0; tb < t1; tb += 256) {
-      for (int i = tid; i < nr * FILL_WORDS; i += 256) mask[i] = 0;
+      for (int i = tid; i < nr * FILL_WORDS; i += NT) mask[i] = 0;
       __syncthreads();
-      const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tb + tid, t1, kh, block_size, t_begin);
-      for_each_block(r, [&](int jb, int) {
+      const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, b0, b1, tb + row, t1, kh, block_size,
+                                   t_begin);
+      for_each_block(r, part, [&](int jb, int) {
         if ((unsigned)(jb - r0) < (unsigned)nr) atomicOr(&mask[(jb - r0) * FILL_WORDS + word], bit);
       });
       __syncthreads();
-      for_each_block(r, [&](int jb, int slot) {
+      for_each_block(r, part, [&](int jb, int slot) {
         if ((unsigned)(jb - r0) >= (unsigned)nr) return;
         const uint32_t* m = &mask[(jb - r0) * FILL_WORDS];
         int pos = cursor[jb - r0];
@@ -188,7 +203,7 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* topk, int6
       });
       __syncthreads();
       if (tb + 256 < t1) {
-        for (int i = tid; i < nr; i += 256) {
+        for (int i = tid; i < nr; i += NT) {
           int add = 0;
 #pragma unroll
           for (int w = 0; w < FILL_WORDS; w++) add += __popc(mask[i * FILL_WORDS + w]);
@@ -246,7 +261,7 @@ int nsa_build_inverse_index_slots(const int32_t* topk, int64_t tk_sh, int64_t tk
   int nchunks = (T + CT - 1) / CT;
   size_t lds = (size_t)nblk_total * sizeof(int);
   dim3 grid(nchunks, KH);
-  csr_count_kernel<<<grid, 256, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
+  csr_count_kernel<<<grid, NT, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
                                           t_begin, workspace);
   int rc = nsa_check_launch("csr_count_kernel");
   if (rc) return rc;
@@ -254,7 +269,7 @@ int nsa_build_inverse_index_slots(const int32_t* topk, int64_t tk_sh, int64_t tk
                                       item_off);
   rc = nsa_check_launch("csr_scan_kernel");
   if (rc) return rc;
-  csr_fill_kernel<<<grid, 256, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
+  csr_fill_kernel<<<grid, NT, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
                                         t_begin, workspace, csr_off, csr_tok, csr_slot);
   return nsa_check_launch("csr_fill_kernel");
 }
