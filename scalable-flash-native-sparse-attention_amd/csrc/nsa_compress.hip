@@ -367,7 +367,17 @@ __global__ void compress_dw_reduce_kernel(const float* slots, int parts, int64_t
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n4) return;
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < parts; k++) sum += *reinterpret_cast<const f32x4*>(slots + (k * n4 + i) * 4);
+  // READ parts in flight: one by one they are a chain of round trips to memory (two launches of 40 samples of up to 1.2K tokens 18.4 -> 11.5 us)
+  constexpr int READ = 8;
+  int k = 0;
+  for (; k + READ <= parts; k += READ) {
+    f32x4 v[READ];
+#pragma unroll
+    for (int u = 0; u < READ; u++) v[u] = *reinterpret_cast<const f32x4*>(slots + ((k + u) * n4 + i) * 4);
+#pragma unroll
+    for (int u = 0; u < READ; u++) sum += v[u];
+  }
+  for (; k < parts; k++) sum += *reinterpret_cast<const f32x4*>(slots + (k * n4 + i) * 4);
   if (dw != nullptr) *reinterpret_cast<bf16x4*>(dw + i * 4) = pack4(sum[0], sum[1], sum[2], sum[3]);
   else *reinterpret_cast<f32x4*>(dw32 + i * 4) += sum;
 }
