@@ -15,17 +15,19 @@ NSA_DEVICE void acc8(float* a, bf16x8 v) {
 #pragma unroll
   for (int e = 0; e < 8; e++) a[e] += (float)v[e];
 }
-// Sum of K rows in row order, fetched eight at a time: one by one they are K round trips to memory, which is what bounds
-// the pooling of all but the longest batches (K and V, us, one by one -> so: 4K tokens, 1 kv head 28 -> 14; 16K tokens, 2
-// kv heads 33 -> 17; chunks of 16 x 2K tokens behind prefixes 67 -> 33; three short prompts with the cache write 15 -> 8.5).
+// Sum of K rows in row order, fetched 16 at a time: one by one they are K round trips to memory, which is what bounds
+// the pooling of all but the longest batches (K and V, us, one by one / 8 / 16 / 32: 4K tokens, 1 kv head 28 / 13.2 / 11.0 / 13.8;
+// 16K tokens, 2 kv heads 33 / 17.5 / 17.0 / 19.5; chunks of 16 x 2K tokens behind prefixes 67 / 32.6 / 31.7 / 48.6; three short
+// prompts with the cache write 15 / 8.1 / 7.9 / 21.2; 64K tokens, 4 kv heads - / 52 / 46 / 60).
 template <class RowPtr>
 NSA_DEVICE void sum_rows(float* a, int K, RowPtr ptr) {
-  for (int r = 0; r < K; r += 8) {
-    bf16x8 x[8];
+  constexpr int READ = 16;
+  for (int r = 0; r < K; r += READ) {
+    bf16x8 x[READ];
 #pragma unroll
-    for (int u = 0; u < 8; u++) x[u] = ld_global_b128(ptr(min(r + u, K - 1)));
+    for (int u = 0; u < READ; u++) x[u] = ld_global_b128(ptr(min(r + u, K - 1)));
 #pragma unroll
-    for (int u = 0; u < 8; u++)
+    for (int u = 0; u < READ; u++)
       if (r + u < K) acc8(a, x[u]);
   }
 }
