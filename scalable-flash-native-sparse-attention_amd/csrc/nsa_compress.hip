@@ -484,8 +484,8 @@ int nsa_compress_linear_fwd(const void* x, int64_t x_st, int64_t x_sh, const voi
                             int stride, int N, int act, void* stream) {
   const int rc = check("compress_linear_fwd", H, D, kernel_size, stride, N, act);
   if (rc != NSA_OK) return rc;
+  if (B <= 0 || y_maxlen <= 0) return NSA_OK;  // (no compressed row: the outputs are empty and may be null)
   NSA_REQUIRE(act < 0 ? hidden != nullptr : out != nullptr, NSA_ERR_BAD_ARG, "compress_linear_fwd: no output given");
-  if (B <= 0 || y_maxlen <= 0) return NSA_OK;
   CompressParams p = {};
   p.x = (const bf16_t*)x; p.x_st = x_st; p.x_sh = x_sh; p.w = (const bf16_t*)w; p.w_st = w_st;
   p.hidden = (bf16_t*)hidden; p.out = (bf16_t*)out; p.x_cu = x_cu; p.y_cu = y_cu;

@@ -170,3 +170,29 @@ def test_module_with_and_without_its_windows(device, version, H, D, lens):
     mod.fc.weight.grad = None
     mod(x).backward(do)
     assert torch.equal(mod.fc.weight.grad, plain[2])
+
+
+@pytest.mark.parametrize("methods", [("linear", "swiglu"), ("sigmoid-mul", "linear")])
+@pytest.mark.parametrize("lens", [[20, 5, 0, 31], [1]])
+def test_batches_without_a_window(device, methods, lens):
+    """Every sequence is shorter than a window: no compressed row, so learned compression is mean pooling bit for bit and the weights'
+    gradients are zero, in the fused and the staged core."""
+    from flash_nsa import HFNSACore, NSAConfig, NSACore
+    T, D = sum(lens), 64
+    ins = [t.to(device) for t in make_qkvw(T, 8, 2, D, seed=14)]
+    do, cu = randn_bf16(T, 8, D, seed=15).to(device), make_cu(lens).to(device)
+    for Core in (NSACore, HFNSACore):
+        runs = []
+        for k_method, v_method in (methods, ("mean", "mean")):
+            core = Core(NSAConfig(head_dim=D, num_heads=8, num_kv_heads=2, cmp_k_method=k_method, cmp_v_method=v_method))
+            core = core.to(device=device, dtype=torch.bfloat16)
+            ts = [t.clone().requires_grad_() for t in ins]
+            out = core(*ts, cu)
+            out.backward(do)
+            with torch.no_grad():
+                assert torch.equal(core(*ins, cu), out)
+            runs.append([out.detach()] + [t.grad for t in ts])
+            for p in core.parameters():
+                assert p.grad.dtype == p.dtype and int(p.grad.count_nonzero()) == 0
+        for a, b in zip(*runs):
+            assert torch.equal(a, b)

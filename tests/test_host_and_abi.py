@@ -37,6 +37,15 @@ def test_entry_points_reject_bad_arguments_without_a_gpu():
                   None, None, 1, 64, 1, 1, 16, 1, 128, 128, 64, 4, 0, 8, 0.1, 1 << 20, 1 << 30, None)
 
 
+@pytest.mark.parametrize("N,act", [(64, -1), (128, 0), (128, 1)])
+def test_learned_compression_of_no_windows_has_nothing_to_do(N, act):
+    """Sequences that are all shorter than a window: the compressed rows are empty tensors, whose addresses are null."""
+    from flash_nsa import _lib
+    _lib.call("nsa_compress_linear_fwd", None, 64, 64, None, 2048, None, None, None, None, 2, 0, 1, 64, 32, 16, N, act, None)
+    with pytest.raises(RuntimeError, match="no output"):
+        _lib.call("nsa_compress_linear_fwd", None, 64, 64, None, 2048, None, None, None, None, 2, 1, 1, 64, 32, 16, N, act, None)
+
+
 def test_nsa_helper_metadata():
     from flash_nsa import NSAHelper
     NSAHelper.set_hyperparameters()
