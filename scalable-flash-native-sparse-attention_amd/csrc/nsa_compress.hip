@@ -486,6 +486,7 @@ int nsa_compress_linear_fwd(const void* x, int64_t x_st, int64_t x_sh, const voi
   if (rc != NSA_OK) return rc;
   if (B <= 0 || y_maxlen <= 0) return NSA_OK;  // (no compressed row: the outputs are empty and may be null)
   NSA_REQUIRE(act < 0 ? hidden != nullptr : out != nullptr, NSA_ERR_BAD_ARG, "compress_linear_fwd: no output given");
+  NSA_REQUIRE(x != nullptr && w != nullptr, NSA_ERR_BAD_ARG, "compress_linear_fwd: x or the weight is null");
   CompressParams p = {};
   p.x = (const bf16_t*)x; p.x_st = x_st; p.x_sh = x_sh; p.w = (const bf16_t*)w; p.w_st = w_st;
   p.hidden = (bf16_t*)hidden; p.out = (bf16_t*)out; p.x_cu = x_cu; p.y_cu = y_cu;
@@ -503,6 +504,9 @@ int nsa_compress_linear_bwd_dx(const void* dhidden, const void* w, int64_t w_st,
   if (rc != NSA_OK) return rc;
   NSA_REQUIRE(dx != nullptr || dst != nullptr, NSA_ERR_BAD_ARG, "compress_linear_bwd_dx: no output given");
   if (B <= 0 || x_maxlen <= 0) return NSA_OK;
+  // (the gradient of no compressed row is not read and may be null)
+  NSA_REQUIRE(w != nullptr && (dhidden != nullptr || x_maxlen < kernel_size), NSA_ERR_BAD_ARG,
+              "compress_linear_bwd_dx: the weight or the gradient is null");
   CompressParams p = {};
   p.hidden = (bf16_t*)dhidden; p.w = (const bf16_t*)w; p.w_st = w_st;
   p.dx = (float*)dx; p.dx_st = dx_st; p.dx_sh = dx_sh; p.dst = (bf16_t*)dst; p.dst_st = dst_st; p.dst_sh = dst_sh;
@@ -522,6 +526,8 @@ int nsa_compress_linear_bwd_dw(const void* dhidden, const void* x, int64_t x_st,
   const int rc = check("compress_linear_bwd_dw", H, D, kernel_size, stride, N, N == D ? -1 : 0);
   if (rc != NSA_OK) return rc;
   NSA_REQUIRE(B > 0 && y_len > 0, NSA_ERR_BAD_ARG, "compress_linear_bwd_dw: no compressed rows");
+  NSA_REQUIRE(dhidden != nullptr && x != nullptr && dw != nullptr && ws != nullptr, NSA_ERR_BAD_ARG,
+              "compress_linear_bwd_dw: an operand or the workspace is null");
   NSA_REQUIRE(ws_bytes >= nsa_compress_linear_bwd_dw_ws_bytes(y_len, H, D, kernel_size, N), NSA_ERR_WORKSPACE,
               "compress_linear_bwd_dw: workspace of %lld bytes is too small", (long long)ws_bytes);
   CompressParams p = {};
@@ -544,6 +550,7 @@ int nsa_compress_linear_bwd_dw(const void* dhidden, const void* x, int64_t x_st,
 int nsa_compress_act_bwd(const void* hidden, const void* dy, void* dhidden, int64_t rows, int D, int act, void* stream) {
   NSA_REQUIRE(D % 8 == 0 && D > 0 && act >= -1 && act <= 1, NSA_ERR_BAD_ARG, "compress_act_bwd: head dim %d, act %d", D, act);
   if (rows <= 0) return NSA_OK;
+  NSA_REQUIRE(dy != nullptr && dhidden != nullptr && (act < 0 || hidden != nullptr), NSA_ERR_BAD_ARG, "compress_act_bwd: an operand is null");
   const int64_t n8 = rows * (D / 8);
   const unsigned g = (unsigned)((n8 + 255) / 256);
   hipStream_t s = (hipStream_t)stream;
@@ -558,6 +565,8 @@ int nsa_mean_pool_bwd_sum(const void* dy, const void* dx, int64_t dx_st, int64_t
                           void* stream) {
   NSA_REQUIRE(D % 8 == 0 && D > 0, NSA_ERR_BAD_ARG, "mean_pool_bwd_sum: head dim %d must be a multiple of 8", D);
   if (B <= 0 || x_maxlen <= 0) return NSA_OK;
+  NSA_REQUIRE(dx != nullptr && dst != nullptr && (dy != nullptr || x_maxlen < kernel_size), NSA_ERR_BAD_ARG,
+              "mean_pool_bwd_sum: an operand is null");
   const dim3 grid((unsigned)(((int64_t)x_maxlen * H * (D / 8) + 255) / 256), B);
   mean_pool_bwd_sum_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const float*)dy, (const float*)dx, dx_st, dx_sh, (bf16_t*)dst,
                                                                   dst_st, dst_sh, x_cu, y_cu, H, D, kernel_size, stride);

@@ -66,11 +66,12 @@ _ACT = {"linear": -1, "sigmoid-mul": 0, "swiglu": 1}
 
 
 def takes_weight(x, weight, version, helper=NSAHelper):
-    """Whether the kernels below take this weight (others go through the windows and the library's products)."""
+    """Whether the kernels below take this weight (others go through the windows and the library's products).  Subclasses that wrap
+    other tensors (quantised, distributed) have the shape and the type of a weight, but no memory of their own."""
     D, N = x.size(-1), (1 if version == "linear" else 2) * x.size(-1)
-    return (D % 32 == 0 and x.is_cuda and weight.device == x.device and x.dtype == weight.dtype == torch.bfloat16
-            and weight.shape == (N, helper.kernel_size * D) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
-            and weight.data_ptr() % 16 == 0)
+    return (type(weight) in (torch.nn.Parameter, torch.Tensor) and D % 32 == 0 and x.is_cuda and weight.device == x.device
+            and x.dtype == weight.dtype == torch.bfloat16 and weight.shape == (N, helper.kernel_size * D) and weight.stride(1) == 1
+            and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0 and weight.data_ptr() != 0)
 
 
 def compress_linear_fwd(x, weight, version, helper=NSAHelper, keep=True):

@@ -58,3 +58,19 @@ def bar_violations(dev, ref, atol=ATOL, rtol=RTOL, row_scale=False):
     if row_scale and ref.numel():
         mag = torch.maximum(mag, ref.pow(2).mean(-1, keepdim=True).sqrt())
     return int((err > atol + rtol * mag).sum()), ref.numel(), float(err.max()) if ref.numel() else 0.0
+
+
+class Wrapper(torch.Tensor):
+    """A tensor whose values lie in another one, as quantised and distributed weights are made."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, strides=inner.stride(), dtype=inner.dtype, device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        out = func(*[a.inner if isinstance(a, cls) else a for a in args], **(kwargs or {}))
+        return cls(out) if func is torch.ops.aten.detach.default else out

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from gpu_util import make_cu, make_qkvw, randn_bf16
+from gpu_util import Wrapper, make_cu, make_qkvw, randn_bf16
 
 pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -9  # relative rounding error of bf16
@@ -196,3 +196,22 @@ def test_batches_without_a_window(device, methods, lens):
                 assert p.grad.dtype == p.dtype and int(p.grad.count_nonzero()) == 0
         for a, b in zip(*runs):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("version", ["linear", "swiglu"])
+def test_weights_that_wrap_another_tensor_go_through_the_library(device, version):
+    """They have no memory of their own to hand to a kernel; their products are those of the tensor inside, to rounding."""
+    from flash_nsa import NSAConfig, NSAHelper
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    from flash_nsa.modules.megatron_level_nsa import compress_kv_fwd
+    lens, D = [200, 77], 64
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+    torch.manual_seed(0)
+    mod = CompressKV(NSAConfig(head_dim=D), head_dim=D, version=version).to(device=device, dtype=torch.bfloat16)
+    x = randn_bf16(sum(lens), 2, D, seed=16).to(device)
+    with torch.no_grad():
+        plain = mod(x)
+        mod.fc.weight = torch.nn.Parameter(Wrapper(mod.fc.weight.detach()), requires_grad=False)
+        for got in (mod(x), compress_kv_fwd(x, mod.fc.weight, version)[2]):
+            assert rel(got, plain.double().cpu()) <= 8 * EPS

@@ -46,6 +46,42 @@ def test_learned_compression_of_no_windows_has_nothing_to_do(N, act):
         _lib.call("nsa_compress_linear_fwd", None, 64, 64, None, 2048, None, None, None, None, 2, 1, 1, 64, 32, 16, N, act, None)
 
 
+def test_learned_compression_takes_only_weights_with_memory_of_their_own():
+    """A weight that wraps another tensor looks like one that the kernels take, but has no address: it stays with the library."""
+    from types import SimpleNamespace
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops.compress_kv import takes_weight
+    from gpu_util import Wrapper
+    NSAHelper.set_hyperparameters()
+    x = SimpleNamespace(size=lambda i: 64, is_cuda=True, device=torch.device("cpu"), dtype=torch.bfloat16)
+    w = torch.randn(64, 32 * 64).bfloat16()
+    wrapped = Wrapper(w)
+    assert wrapped.dtype == w.dtype and wrapped.shape == w.shape and wrapped.stride() == w.stride()
+    assert takes_weight(x, w, "linear") and takes_weight(x, torch.nn.Parameter(w), "linear")
+    assert not takes_weight(x, wrapped, "linear") and not takes_weight(x, torch.nn.Parameter(wrapped), "linear")
+
+
+def test_learned_compression_refuses_null_operands():
+    """The entry points of learned compression name a missing operand instead of launching on it."""
+    from flash_nsa import _lib
+    some, sizes = 1 << 20, (1, 8, 1, 64, 32, 16)  # never dereferenced: every call below is refused
+    for x, w in ((None, some), (some, None)):
+        with pytest.raises(RuntimeError, match="null"):
+            _lib.call("nsa_compress_linear_fwd", x, 64, 64, w, 2048, some, some, some, some, *sizes, 64, -1, None)
+    for dhidden, w, n in ((None, some, 40), (some, None, 40), (None, None, 20)):
+        with pytest.raises(RuntimeError, match="null"):
+            _lib.call("nsa_compress_linear_bwd_dx", dhidden, w, 2048, None, 0, 0, some, 64, 64, some, some, 1, n, 1, 64, 32, 16, 64, None)
+    for dhidden, x, dw, ws in ((None, *(some,) * 3), (some, None, some, some), (some, some, None, some), (*(some,) * 3, None)):
+        with pytest.raises(RuntimeError, match="null"):
+            _lib.call("nsa_compress_linear_bwd_dw", dhidden, x, 64, 64, dw, 0, some, some, *sizes, 64, ws, 1 << 30, None)
+    for hidden, dy, dhidden in ((None, some, some), (some, None, some), (some, some, None)):
+        with pytest.raises(RuntimeError, match="null"):
+            _lib.call("nsa_compress_act_bwd", hidden, dy, dhidden, 8, 64, 0, None)
+    for dy, dx, dst in ((None, some, some), (some, None, some), (some, some, None)):
+        with pytest.raises(RuntimeError, match="null"):
+            _lib.call("nsa_mean_pool_bwd_sum", dy, dx, 64, 64, dst, 64, 64, some, some, 1, 40, 1, 64, 32, 16, None)
+
+
 def test_nsa_helper_metadata():
     from flash_nsa import NSAHelper
     NSAHelper.set_hyperparameters()
