@@ -17,8 +17,12 @@ _METHODS = ("mean", "sigmoid-mul", "swiglu", "linear")
 
 
 def _hooked(module):
-    return (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
-            "forward" in module.__dict__)
+    """Whether something waits for a call of this module: its own hooks, those registered for all modules (profilers and FLOP counters
+    work with them), or another forward."""
+    m = torch.nn.modules.module
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
+                m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks or
+                "forward" in module.__dict__)
 
 
 class CompressKV(torch.nn.Module):

@@ -215,3 +215,22 @@ def test_weights_that_wrap_another_tensor_go_through_the_library(device, version
         mod.fc.weight = torch.nn.Parameter(Wrapper(mod.fc.weight.detach()), requires_grad=False)
         for got in (mod(x), compress_kv_fwd(x, mod.fc.weight, version)[2]):
             assert rel(got, plain.double().cpu()) <= 8 * EPS
+
+
+def test_hooks_on_all_modules_see_the_linear_layer(device):
+    """A hook registered for every module (as FLOP counters do) fires for CompressKV's fc, forward and backward."""
+    from flash_nsa import NSAConfig, NSAHelper
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu([100]).to(device))
+    mod = CompressKV(NSAConfig(head_dim=64), head_dim=64, version="linear").to(device=device, dtype=torch.bfloat16)
+    x, seen = randn_bf16(100, 1, 64, seed=17).to(device).requires_grad_(), []
+    m = torch.nn.modules.module
+    handles = [m.register_module_forward_hook(lambda mod, *a: seen.append(("forward", mod))),
+               m.register_module_full_backward_hook(lambda mod, *a: seen.append(("backward", mod)))]
+    try:
+        mod(x).float().sum().backward()
+    finally:
+        for h in handles:
+            h.remove()
+    assert ("forward", mod.fc) in seen and ("backward", mod.fc) in seen

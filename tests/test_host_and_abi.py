@@ -82,6 +82,21 @@ def test_learned_compression_refuses_null_operands():
             _lib.call("nsa_mean_pool_bwd_sum", dy, dx, 64, 64, dst, 64, 64, some, some, 1, 40, 1, 64, 32, 16, None)
 
 
+@pytest.mark.parametrize("kind", ["forward_hook", "forward_pre_hook", "full_backward_hook", "full_backward_pre_hook"])
+def test_hooks_of_a_linear_layer_are_seen(kind):
+    """Hooks on the layer and hooks on all modules: learned compression calls a layer that anything waits for."""
+    from flash_nsa.modules.hf_level_nsa import _hooked
+    fc, fn = torch.nn.Linear(4, 4), lambda *a: None
+    assert not _hooked(fc)
+    for register in (getattr(fc, "register_" + kind), getattr(torch.nn.modules.module, "register_module_" + kind)):
+        handle = register(fn)
+        try:
+            assert _hooked(fc)
+        finally:
+            handle.remove()
+        assert not _hooked(fc)
+
+
 def test_nsa_helper_metadata():
     from flash_nsa import NSAHelper
     NSAHelper.set_hyperparameters()
