@@ -25,6 +25,11 @@ def _hooked(module):
                 "forward" in module.__dict__)
 
 
+def _autocast_elsewhere(device):
+    """Whether a layer called here would give its result in another type than bf16."""
+    return torch.is_autocast_enabled(device.type) and torch.get_autocast_dtype(device.type) != torch.bfloat16
+
+
 class CompressKV(torch.nn.Module):
     """Compresses [T,H,D] into one row per window of kernel_size tokens every stride tokens.
     mean: average; linear: fc over the flattened window; sigmoid-mul / swiglu: gated fc (2*D outputs)."""
@@ -45,7 +50,7 @@ class CompressKV(torch.nn.Module):
             return mean_pooling(x)
         # a plain fc is computed with the windows where they lie; one that has been replaced, wrapped or hooked is called
         if type(self.fc) is torch.nn.Linear and self.fc.bias is None and not _hooked(self.fc) and \
-                x.dim() == 3 and takes_weight(x, self.fc.weight, self.version):
+                not _autocast_elsewhere(x.device) and x.dim() == 3 and takes_weight(x, self.fc.weight, self.version):
             return compress_linear(x, self.fc.weight, self.version)
         windows = construct_block(x)                    # [y_len, H, kernel, D]
         hidden = self.fc(windows.flatten(-2, -1))        # flatten order: (position in window, channel)

@@ -234,3 +234,17 @@ def test_hooks_on_all_modules_see_the_linear_layer(device):
         for h in handles:
             h.remove()
     assert ("forward", mod.fc) in seen and ("backward", mod.fc) in seen
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_autocast_decides_the_type_of_linear_compression(device, dtype):
+    """CompressKV("linear") under autocast returns what its layer returns there."""
+    from flash_nsa import NSAConfig, NSAHelper, construct_block
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu([100]).to(device))
+    mod = CompressKV(NSAConfig(head_dim=64), head_dim=64, version="linear").to(device=device, dtype=torch.bfloat16)
+    x = randn_bf16(100, 1, 64, seed=18).to(device)
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        got, want = mod(x), mod.fc(construct_block(x).flatten(-2, -1))
+    assert got.dtype == want.dtype == dtype and rel(got, want.double().cpu()) <= 2 * EPS
