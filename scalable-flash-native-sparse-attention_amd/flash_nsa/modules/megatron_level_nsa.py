@@ -11,7 +11,7 @@ from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
 from ..ops._common import thd_rows
 from ..ops.compress_kv import (compress_linear_fwd, compress_linear_bwd, construct_block_fwd, construct_block_bwd, mean_pooling_fwd,
-                               mean_pooling_bwd_sum, takes_weight)
+                               mean_pooling_bwd, mean_pooling_bwd_sum, takes_weight)
 from ..ops import bwd_ds
 from ..ops.compress_attn import cmp_attn_fwd, cmp_attn_bwd
 from ..ops.select_attn import (slc_attn_fwd, slc_attn_bwd, slc_attn_bwd_dkdv_before_window,
@@ -77,8 +77,8 @@ def _added_to_main_grad(weight, like):
     return None
 
 
-def compress_kv_fwd(x, weight, version, helper=NSAHelper, keep=True):
-    """-> (windows or None, pre-activation or None, compressed rows); keep=False: only the rows are asked for"""
+def _compress_fwd(x, weight, version, helper=NSAHelper, keep=True):
+    """compress_kv_fwd without the windows where the kernels do not need them; keep=False: only the rows are asked for"""
     if version == "mean":
         return None, None, mean_pooling_fwd(x, helper=helper)
     if takes_weight(x, weight, version, helper):
@@ -96,8 +96,17 @@ def compress_kv_fwd(x, weight, version, helper=NSAHelper, keep=True):
     return windows, hidden, out
 
 
-def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelper):
-    """-> (bf16 sum of the compression gradient and the fp32 buffer dx, which may be overwritten, dW); dout: fp32."""
+def compress_kv_fwd(x, weight, version, helper=NSAHelper):
+    """-> (windows or None, pre-activation or None, compressed rows)"""
+    windows, hidden, out = _compress_fwd(x, weight, version, helper)
+    if windows is None and hidden is not None:
+        windows = construct_block_fwd(x, helper=helper)
+    return windows, hidden, out
+
+
+def _compress_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelper):
+    """For what _compress_fwd returned -> (bf16 sum of the compression gradient and the fp32 buffer dx, which may be overwritten, dW);
+    dout: fp32."""
     if version == "mean":
         return mean_pooling_bwd_sum(x, dout, dx, helper), None
     if windows is None:
@@ -108,7 +117,16 @@ def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHel
         else:
             dx, dw = compress_linear_bwd(x, weight, hidden, dout, dx, version, main_grad, helper)
             return dx, dw if main_grad is None else _added_to_main_grad(weight, x)
+    dx, dw = compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper)
+    return dx.to(x.dtype), dw
+
+
+def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelper, async_dw=False):
+    """Adds the compression gradient into the fp32 buffer dx and returns (dx, dW or a thunk computing it)."""
     dout = dout.to(x.dtype)
+    if version == "mean":
+        mean_pooling_bwd(x, dout, dx, helper=helper)
+        return dx, None
     if version == "linear":
         dhidden = dout
     elif version == "sigmoid-mul":
@@ -117,7 +135,11 @@ def compress_kv_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHel
         dhidden = swiglu_bwd(hidden, dout, inplace=False)
     dwindows = torch.matmul(dhidden, weight).view(*windows.shape)
     construct_block_bwd(x, dwindows, dx, helper=helper)
-    return dx.to(x.dtype), weight_grad(windows.flatten(-2, -1), dhidden, weight)
+
+    def dw_fn():
+        return weight_grad(windows.flatten(-2, -1), dhidden, weight)
+
+    return dx, (dw_fn if async_dw else dw_fn())
 
 
 def slc_swa_fwd(q, k, v, topk, sm_scale, helper, cmp_o=None, w=None, store=True):
@@ -191,8 +213,8 @@ class NSAFunction(torch.autograd.Function):
         if sm_scale is None:
             sm_scale = q.size(-1) ** -0.5
         H = NSAHelper
-        win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, H.cmp_k_method, keep=for_backward)
-        win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, H.cmp_v_method, keep=for_backward)
+        win_k, hid_k, cmp_k = _compress_fwd(k, cmp_k_weight, H.cmp_k_method, keep=for_backward)
+        win_v, hid_v, cmp_v = _compress_fwd(v, cmp_v_weight, H.cmp_v_method, keep=for_backward)
         if 0 < H.x_maxlen <= H.all_below():  # nothing to choose from: no block is selected
             topk = torch.empty(k.size(1), q.size(0), H.top_n, device=q.device, dtype=torch.int32)
             (cmp_o, cmp_lse), (slc_o, slc_lse), (swa_o, swa_lse), out = short_fwd(q, k, v, cmp_k, cmp_v, combine_weight, H.all_below(),
@@ -226,8 +248,8 @@ class NSAFunction(torch.autograd.Function):
         do = thd_rows(do)
 
         if cmp_k is None:
-            win_k, hid_k, cmp_k = compress_kv_fwd(k, cmp_k_weight, k_method, helper)
-            win_v, hid_v, cmp_v = compress_kv_fwd(v, cmp_v_weight, v_method, helper)
+            win_k, hid_k, cmp_k = _compress_fwd(k, cmp_k_weight, k_method, helper)
+            win_v, hid_v, cmp_v = _compress_fwd(v, cmp_v_weight, v_method, helper)
         if cmp_o is None:
             cmp_o, cmp_lse = cmp_attn_fwd(q, cmp_k, cmp_v, sm_scale=sm_scale, helper=helper)
         if slc_o is None and swa_o is None:
@@ -254,8 +276,8 @@ class NSAFunction(torch.autograd.Function):
             if ds.fits:
                 dq, dk, dv, dcmp_k, dcmp_v = bwd_from_ds(ds, q, k, v, topk, cmp_k, cmp_v, do, dcmp_o, cmp_lse, lse_slc, lse_swa,
                                                          delta, ds_tokens, sm_scale, helper)
-                dk, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
-                dv, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+                dk, dwk = _compress_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+                dv, dwv = _compress_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
                 return dq, dk, dv, dw, dwk, dwv, None, None
 
         # Where the selected branch's dk / dv pass can leave its dS behind, the selected dq comes last: it adds the other
@@ -318,8 +340,8 @@ class NSAFunction(torch.autograd.Function):
             dq = dq_chain()
             dk, dv = dkdv_raw()
             dcmp_k, dcmp_v = dkdv_cmp()
-        dk, dwk = compress_kv_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
-        dv, dwv = compress_kv_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
+        dk, dwk = _compress_bwd(k, cmp_k_weight, win_k, hid_k, dcmp_k, dk, k_method, helper)
+        dv, dwv = _compress_bwd(v, cmp_v_weight, win_v, hid_v, dcmp_v, dv, v_method, helper)
         if OVERLAP_STREAMS and not stored_ds:
             main.wait_stream(side)
         return dq, dk, dv, dw, dwk, dwv, None, None

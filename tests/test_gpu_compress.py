@@ -248,3 +248,39 @@ def test_autocast_decides_the_type_of_linear_compression(device, dtype):
     with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
         got, want = mod(x), mod.fc(construct_block(x).flatten(-2, -1))
     assert got.dtype == want.dtype == dtype and rel(got, want.double().cpu()) <= 2 * EPS
+
+
+@pytest.mark.parametrize("dout_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("version", ["mean", "linear", "sigmoid-mul", "swiglu"])
+def test_compress_kv_functions_keep_their_contract(device, version, dout_dtype):
+    """compress_kv_fwd returns the windows, compress_kv_bwd adds into the caller's fp32 buffer and returns it with dW, or with a function
+    that computes it, from gradients of either type."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.modules.megatron_level_nsa import compress_kv_bwd, compress_kv_fwd
+    from flash_nsa.ops import compress_kv as C
+    lens, H, D = [200, 20, 90], 2, 64
+    T, N = sum(lens), D if version == "linear" else 2 * D
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+    x = randn_bf16(T, H, D, seed=19)
+    w = None if version == "mean" else (randn_bf16(N, 32 * D, seed=20).float() * (32 * D) ** -0.5).to(torch.bfloat16)
+    xd, wd = x.to(device), w if w is None else w.to(device)
+    windows, hidden, out = compress_kv_fwd(xd, wd, version)
+    dout = randn_bf16(*out.shape, seed=21).to(device, dout_dtype)
+    runs = []
+    for kw in ({}, {"async_dw": True}):
+        dx = torch.ones(T, H, D, device=device)
+        got, dw = compress_kv_bwd(xd, wd, windows, hidden, dout, dx, version, NSAHelper, **kw)
+        assert got is dx
+        runs.append((dx, dw() if callable(dw) else dw))
+        assert callable(dw) == (version != "mean" and bool(kw))
+    assert torch.equal(runs[0][0], runs[1][0])
+    if version == "mean":
+        assert windows is None and hidden is None and runs[0][1] is None
+        assert torch.equal(dx, C.mean_pooling_bwd(xd, dout.to(torch.bfloat16), torch.ones_like(dx)))
+        return
+    assert torch.equal(windows, C.construct_block_fwd(xd)) and torch.equal(runs[0][1], runs[1][1])
+    want = reference(x, w, version, lens, 32, 16, dout.cpu(), torch.ones(T, H, D))
+    # as in test_learned_compression_against_float64; dx also has the rounding of the windows' gradient
+    for a, b, n in ((hidden, want[0], 1.02), (out, want[1], 8), (dx, want[2], 10), (runs[0][1], want[3], 9)):
+        assert rel(a, b) <= n * EPS
