@@ -70,6 +70,14 @@ def weight_grad(inp, grad_out, weight):
     return _added_to_main_grad(weight, inp)
 
 
+def _kernels_add_to(main_grad, weight):
+    """Whether the kernels add dW to this buffer: they read and write four fp32 values at a time, and a view into the flat buffer of an
+    optimizer may begin anywhere."""
+    return (type(main_grad) in (torch.Tensor, torch.nn.Parameter) and main_grad.dtype == torch.float32 and
+            main_grad.shape == weight.shape and main_grad.device == weight.device and main_grad.is_contiguous() and
+            main_grad.data_ptr() % 16 == 0 and main_grad.data_ptr() != 0)
+
+
 def _added_to_main_grad(weight, like):
     if hasattr(weight, "grad_added_to_main_grad"):
         weight.grad_added_to_main_grad = True
@@ -111,8 +119,7 @@ def _compress_bwd(x, weight, windows, hidden, dout, dx, version, helper=NSAHelpe
         return mean_pooling_bwd_sum(x, dout, dx, helper), None
     if windows is None:
         main_grad = getattr(weight, "main_grad", None)
-        if main_grad is not None and (main_grad.dtype != torch.float32 or main_grad.shape != weight.shape or
-                                      main_grad.device != x.device or not main_grad.is_contiguous()):
+        if main_grad is not None and not _kernels_add_to(main_grad, weight):
             windows = construct_block_fwd(x, helper=helper)
         else:
             dx, dw = compress_linear_bwd(x, weight, hidden, dout, dx, version, main_grad, helper)

@@ -61,6 +61,21 @@ def test_learned_compression_takes_only_weights_with_memory_of_their_own():
     assert not takes_weight(x, wrapped, "linear") and not takes_weight(x, torch.nn.Parameter(wrapped), "linear")
 
 
+def test_weight_gradients_are_added_to_aligned_buffers_by_the_kernels():
+    """Other places of a main_grad are left to the library's product, which takes any."""
+    from flash_nsa.modules.megatron_level_nsa import _kernels_add_to
+    from gpu_util import Wrapper
+    w = torch.empty(8, 64, dtype=torch.bfloat16)
+    flat = torch.zeros(2 * w.numel() + 64)
+    at = -flat.data_ptr() // 4 % 4  # the first 16-byte boundary
+    view = lambda offset: flat[at + offset:at + offset + w.numel()].view(w.shape)
+    assert _kernels_add_to(view(0), w) and _kernels_add_to(view(4), w)
+    assert not any(_kernels_add_to(view(n), w) for n in (1, 2, 3))
+    wide = torch.zeros(8, 128)
+    for other in (wide[:, :64], view(0).t(), view(0).bfloat16(), view(0).view(-1), Wrapper(view(0))):
+        assert not _kernels_add_to(other, w)
+
+
 def test_learned_compression_refuses_null_operands():
     """The entry points of learned compression name a missing operand instead of launching on it."""
     from flash_nsa import _lib
