@@ -4,7 +4,7 @@ import torch
 
 from .. import _lib
 from ..utils import NSAHelper
-from ._common import check_thd
+from ._common import check_thd, thd_rows
 from .act import _glu_bwd
 
 
@@ -173,7 +173,8 @@ class _CompressLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         x, weight, hidden = ctx.saved_tensors
-        dhidden = dout.contiguous() if hidden is None else _glu_bwd(hidden, dout, ctx.version, inplace=False)
+        # (the products read whole 16 bytes; a contiguous gradient may still be a view that begins between them)
+        dhidden = thd_rows(dout.contiguous()) if hidden is None else _glu_bwd(hidden, dout, ctx.version, inplace=False)
         dx = compress_linear_bwd_x(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[0] else None
         dw = compress_linear_bwd_weight(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[1] else None
         return dx, dw, None

@@ -284,3 +284,26 @@ def test_compress_kv_functions_keep_their_contract(device, version, dout_dtype):
     # as in test_learned_compression_against_float64; dx also has the rounding of the windows' gradient
     for a, b, n in ((hidden, want[0], 1.02), (out, want[1], 8), (dx, want[2], 10), (runs[0][1], want[3], 9)):
         assert rel(a, b) <= n * EPS
+
+
+def test_gradients_that_begin_between_16_bytes(device, monkeypatch):
+    """A gradient of the linear method that is contiguous at an odd offset: the kernels get an aligned copy, the results are those of
+    an aligned gradient bit for bit."""
+    from flash_nsa import NSAHelper
+    from flash_nsa.ops import compress_kv as C
+    lens, H, D = [150, 60], 2, 64
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+    x, w = randn_bf16(sum(lens), H, D, seed=22).to(device), (randn_bf16(D, 32 * D, seed=23) / 32).to(device)
+    do = randn_bf16(NSAHelper.y_len, H, D, seed=24).to(device)
+    flat = torch.empty(do.numel() + 1, device=device, dtype=do.dtype)
+    flat[1:] = do.flatten()
+    seen, product = [], C.compress_linear_bwd_x
+    monkeypatch.setattr(C, "compress_linear_bwd_x", lambda x, w, g, *a, **kw: seen.append(g.data_ptr() % 16) or product(x, w, g, *a, **kw))
+    grads = []
+    for g in (do, flat[1:].view(do.shape)):
+        xs, ws = x.clone().requires_grad_(), w.clone().requires_grad_()
+        C.compress_linear(xs, ws, "linear").backward(g)
+        grads.append((xs.grad, ws.grad))
+    assert seen == [0, 0]
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
