@@ -151,14 +151,14 @@ class _MeanPooling(torch.autograd.Function):
 
 class _ConstructBlock(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x):
-        ctx.helper = NSAHelper.get_bwd_helper()
+    def forward(ctx, x, helper):
+        ctx.helper = NSAHelper.get_bwd_helper() if helper is None else helper
         ctx.x_meta = x
-        return construct_block_fwd(x)
+        return construct_block_fwd(x, ctx.helper)
 
     @staticmethod
     def backward(ctx, dy):
-        return construct_block_bwd(ctx.x_meta, dy, helper=ctx.helper)
+        return construct_block_bwd(ctx.x_meta, dy, helper=ctx.helper), None
 
 
 class _CompressLinear(torch.autograd.Function):
@@ -176,7 +176,12 @@ class _CompressLinear(torch.autograd.Function):
         # (the products read whole 16 bytes; a contiguous gradient may still be a view that begins between them)
         dhidden = thd_rows(dout.contiguous()) if hidden is None else _glu_bwd(hidden, dout, ctx.version, inplace=False)
         dx = compress_linear_bwd_x(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[0] else None
-        dw = compress_linear_bwd_weight(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[1] else None
+        if not ctx.needs_input_grad[1]:
+            dw = None
+        elif torch.is_grad_enabled():  # create_graph: dW is differentiated again, as a product of the gradient and the windows
+            dw = torch.matmul(dhidden.flatten(0, 1).t(), _ConstructBlock.apply(x, ctx.helper).flatten(0, 1).flatten(1))
+        else:
+            dw = compress_linear_bwd_weight(x, weight, dhidden, helper=ctx.helper)
         return dx, dw, None
 
 
@@ -190,4 +195,4 @@ def mean_pooling(x):
 
 
 def construct_block(x):
-    return _ConstructBlock.apply(x)
+    return _ConstructBlock.apply(x, None)

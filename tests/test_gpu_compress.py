@@ -307,3 +307,33 @@ def test_gradients_that_begin_between_16_bytes(device, monkeypatch):
         grads.append((xs.grad, ws.grad))
     assert seen == [0, 0]
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("version", ["linear", "swiglu"])
+def test_weight_gradients_can_be_differentiated_again(device, version):
+    """create_graph=True through CompressKV: a penalty on dW has the gradients that it has where the layer is called."""
+    from flash_nsa import NSAConfig, NSAHelper
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    lens, H, D = [200, 20, 90], 2, 64
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu(lens).to(device))
+    torch.manual_seed(0)
+    mod = CompressKV(NSAConfig(head_dim=D), head_dim=D, version=version).to(device=device, dtype=torch.bfloat16)
+    x, do = randn_bf16(sum(lens), H, D, seed=25).to(device), randn_bf16(NSAHelper.y_len, H, D, seed=26).to(device)
+
+    def penalty():
+        xs, ds, mod.fc.weight.grad = x.clone().requires_grad_(), do.clone().requires_grad_(), None
+        dw, = torch.autograd.grad((mod(xs) * ds).sum(), mod.fc.weight, create_graph=True)
+        assert dw.requires_grad
+        dw.float().pow(2).sum().backward()
+        return [dw.detach(), xs.grad] + ([ds.grad] if version == "linear" else [])  # (nothing goes through the gate's gradient twice)
+
+    plain = penalty()
+    hook = mod.fc.register_forward_hook(lambda *a: None)
+    called = penalty()
+    hook.remove()
+    # "linear": products of the same operands, dW rounded once on either side; its gradients have dW's rounding, that of a product and
+    # their own on either side.  The gate: the 8 of test_module_with_and_without_its_windows in dW, and twice that and 4 behind it.
+    for i, (a, b) in enumerate(zip(plain, called)):
+        bound = {"linear": (2, 6), "swiglu": (8, 20)}[version][i > 0]
+        assert rel(a, b.double().cpu()) <= bound * EPS
