@@ -2,6 +2,7 @@
 (mirrors the interface of upstream flash_nsa/modules/hf_level_nsa.py:17-158)."""
 
 import torch
+from torch.autograd import forward_ad
 
 from ..config import NSAConfig, check_supported
 from ..utils import NSAHelper
@@ -30,6 +31,11 @@ def _autocast_elsewhere(device):
     return torch.is_autocast_enabled(device.type) and torch.get_autocast_dtype(device.type) != torch.bfloat16
 
 
+def _has_tangent(t):
+    """Whether forward-mode differentiation is under way for this tensor (products carry a tangent on, the kernels do not)."""
+    return forward_ad.unpack_dual(t).tangent is not None
+
+
 class CompressKV(torch.nn.Module):
     """Compresses [T,H,D] into one row per window of kernel_size tokens every stride tokens.
     mean: average; linear: fc over the flattened window; sigmoid-mul / swiglu: gated fc (2*D outputs)."""
@@ -50,7 +56,8 @@ class CompressKV(torch.nn.Module):
             return mean_pooling(x)
         # a plain fc is computed with the windows where they lie; one that has been replaced, wrapped or hooked is called
         if type(self.fc) is torch.nn.Linear and self.fc.bias is None and not _hooked(self.fc) and \
-                not _autocast_elsewhere(x.device) and x.dim() == 3 and takes_weight(x, self.fc.weight, self.version):
+                not _autocast_elsewhere(x.device) and x.dim() == 3 and takes_weight(x, self.fc.weight, self.version) and \
+                not _has_tangent(self.fc.weight):
             return compress_linear(x, self.fc.weight, self.version)
         windows = construct_block(x)                    # [y_len, H, kernel, D]
         hidden = self.fc(windows.flatten(-2, -1))        # flatten order: (position in window, channel)

@@ -337,3 +337,22 @@ def test_weight_gradients_can_be_differentiated_again(device, version):
     for i, (a, b) in enumerate(zip(plain, called)):
         bound = {"linear": (2, 6), "swiglu": (8, 20)}[version][i > 0]
         assert rel(a, b.double().cpu()) <= bound * EPS
+
+
+def test_a_tangent_of_the_weight_goes_through_the_linear_layer(device):
+    """Forward-mode differentiation of CompressKV("linear") with respect to its weight: the product of the windows and the tangent."""
+    from flash_nsa import NSAConfig, NSAHelper, construct_block
+    from flash_nsa.modules.hf_level_nsa import CompressKV
+    from torch.autograd import forward_ad
+    NSAHelper.set_hyperparameters()
+    NSAHelper.init_cu_seqlens(make_cu([100, 40]).to(device))
+    mod = CompressKV(NSAConfig(head_dim=64), head_dim=64, version="linear").to(device=device, dtype=torch.bfloat16)
+    x, dw = randn_bf16(140, 1, 64, seed=27).to(device), randn_bf16(64, 32 * 64, seed=28).to(device)
+    plain = mod(x).detach()
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(mod.fc.weight.detach(), dw)
+        out, tangent = forward_ad.unpack_dual(torch.func.functional_call(mod, {"fc.weight": dual}, (x,)))
+        assert torch.equal(mod(x), plain)  # (a weight without a tangent beside it)
+    windows = construct_block(x).flatten(-2, -1).double().cpu()
+    assert rel(tangent, windows @ dw.double().cpu().t()) <= 1.02 * EPS
+    assert rel(out, plain.double().cpu()) <= 2 * EPS

@@ -112,6 +112,18 @@ def test_hooks_of_a_linear_layer_are_seen(kind):
         assert not _hooked(fc)
 
 
+def test_tangents_of_a_weight_are_seen():
+    """Inside forward-mode differentiation, the tensors that carry a tangent and no others."""
+    from flash_nsa.modules.hf_level_nsa import _has_tangent
+    from torch.autograd import forward_ad
+    w = torch.nn.Parameter(torch.randn(4, 4))
+    assert not _has_tangent(w)
+    with forward_ad.dual_level():
+        assert not _has_tangent(w)
+        assert _has_tangent(forward_ad.make_dual(w.detach(), torch.ones(4, 4)))
+    assert not _has_tangent(w)
+
+
 def test_nsa_helper_metadata():
     from flash_nsa import NSAHelper
     NSAHelper.set_hyperparameters()
