@@ -74,6 +74,13 @@ def takes_weight(x, weight, version, helper=NSAHelper):
             and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0 and weight.data_ptr() != 0)
 
 
+def weight_rows(weight):
+    """weight, or a copy of it where its layout is not one that takes_weight accepts."""
+    if weight.stride(1) == 1 and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0:
+        return weight
+    return weight.clone(memory_format=torch.contiguous_format)
+
+
 def compress_linear_fwd(x, weight, version, helper=NSAHelper, keep=True):
     """x [T,H,D], weight [N, kernel*D] -> hidden [y_len,H,N], the product of the windows and the weight, and the compressed rows
     [y_len,H,D], its activation ("linear": itself).  keep=False: nobody asks for hidden."""
@@ -119,6 +126,7 @@ def compress_linear_bwd(x, weight, hidden, dout, dx, version, dw=None, helper=NS
     """From the fp32 gradient dout of the compressed rows: (the bf16 sum of the fp32 dx and the gradient with respect to x, dw).
     dw: None for a new bf16 tensor, else an fp32 one that is added to."""
     H, D = x.shape[1:]
+    weight, hidden = weight_rows(weight), thd_rows(hidden.contiguous())  # (saved-tensor hooks may give them back in any layout)
     assert dout.dtype == dx.dtype == torch.float32 and dout.is_contiguous() and dx.stride(-1) == 1
     dhidden = torch.empty(helper.y_len, H, weight.size(0), device=x.device, dtype=x.dtype)
     _lib.call("nsa_compress_act_bwd", hidden.data_ptr(), dout.data_ptr(), dhidden.data_ptr(), helper.y_len * H, D, _ACT[version],
@@ -173,7 +181,9 @@ class _CompressLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         x, weight, hidden = ctx.saved_tensors
-        # (the products read whole 16 bytes; a contiguous gradient may still be a view that begins between them)
+        # (the products read whole 16 bytes; a contiguous gradient may still be a view that begins between them, and so may what
+        # saved-tensor hooks give back)
+        x, weight = thd_rows(x), weight_rows(weight)
         dhidden = thd_rows(dout.contiguous()) if hidden is None else _glu_bwd(hidden, dout, ctx.version, inplace=False)
         dx = compress_linear_bwd_x(x, weight, dhidden, helper=ctx.helper) if ctx.needs_input_grad[0] else None
         if not ctx.needs_input_grad[1]:

@@ -356,3 +356,41 @@ def test_a_tangent_of_the_weight_goes_through_the_linear_layer(device):
     windows = construct_block(x).flatten(-2, -1).double().cpu()
     assert rel(tangent, windows @ dw.double().cpu().t()) <= 1.02 * EPS
     assert rel(out, plain.double().cpu()) <= 2 * EPS
+
+
+@pytest.mark.parametrize("core_name", ["NSACore", "HFNSACore"])
+@pytest.mark.parametrize("k_method,v_method", [("linear", "swiglu"), ("sigmoid-mul", "linear")])
+def test_saved_tensors_that_come_back_in_another_layout(device, core_name, k_method, v_method):
+    """Saved-tensor hooks that keep weights at odd offsets and pre-activations in another order of their axes: the same gradients."""
+    import flash_nsa
+    lens, D, moved = [200, 77], 64, []
+    T = sum(lens)
+    core = getattr(flash_nsa, core_name)(flash_nsa.NSAConfig(head_dim=D, num_heads=8, num_kv_heads=2, cmp_k_method=k_method,
+                                                             cmp_v_method=v_method)).to(device=device, dtype=torch.bfloat16)
+    ins = [t.to(device) for t in make_qkvw(T, 8, 2, D, seed=29)]
+    do, cu = randn_bf16(T, 8, D, seed=30).to(device), make_cu(lens).to(device)
+
+    def pack(t):
+        if t.dtype == torch.bfloat16 and t.dim() == 2:
+            flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
+            flat[1:] = t.detach().flatten()
+            t = flat[1:].view(t.shape)
+        elif t.dtype == torch.bfloat16 and t.size(-1) == 2 * D:
+            t = t.detach().transpose(0, 1).contiguous().transpose(0, 1)
+        else:
+            return t
+        moved.append(t)
+        return t
+
+    def grads():
+        core.zero_grad()
+        ts = [t.clone().requires_grad_() for t in ins]
+        core(*ts, cu).backward(do)
+        return [t.grad for t in ts] + [p.grad for p in core.parameters()]
+
+    plain = grads()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        hooked = grads()
+    assert len(moved) == 3 and sum(t.data_ptr() % 16 != 0 for t in moved) == 2 and sum(not t.is_contiguous() for t in moved) == 1
+    for a, b in zip(hooked, plain):  # (dk, dv and what follows from them: sums of fp32 atomics)
+        assert a.dtype == b.dtype and rel(a, b.double().cpu()) <= EPS

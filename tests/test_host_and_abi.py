@@ -61,6 +61,20 @@ def test_learned_compression_takes_only_weights_with_memory_of_their_own():
     assert not takes_weight(x, wrapped, "linear") and not takes_weight(x, torch.nn.Parameter(wrapped), "linear")
 
 
+def test_weights_of_any_layout_are_copied_for_the_kernels():
+    """What saved-tensor hooks give back may begin anywhere and lie in any order: the kernels get whole, aligned rows."""
+    from flash_nsa.ops.compress_kv import weight_rows
+    flat = torch.randn(8 * 64 + 16).bfloat16()
+    at = -flat.data_ptr() // 2 % 8  # the first 16-byte boundary
+    view = lambda offset: flat[at + offset:at + offset + 512].view(8, 64)
+    wide = torch.randn(8, 72).bfloat16()
+    for same in (view(0), view(8), wide[:, :64]):
+        assert weight_rows(same) is same
+    for other in (view(1), view(4), view(0).view(64, 8).t(), torch.randn(8, 65).bfloat16()[:, :64]):
+        got = weight_rows(other)
+        assert torch.equal(got, other) and got.is_contiguous() and got.data_ptr() % 16 == 0
+
+
 def test_weight_gradients_are_added_to_aligned_buffers_by_the_kernels():
     """Other places of a main_grad are left to the library's product, which takes any."""
     from flash_nsa.modules.megatron_level_nsa import _kernels_add_to
