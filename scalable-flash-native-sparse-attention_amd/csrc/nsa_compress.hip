@@ -460,18 +460,20 @@ void launch_fwd(const CompressParams& p, int y_maxlen, hipStream_t s) {
   compress_linear_kernel<GB, GLU, RS, AHEAD><<<dim3((unsigned)((rows + 32 * RS - 1) / (32 * RS)), p.B, p.D / 32 / GB), 512, 0, s>>>(p);
 }
 // All forms sum a product in the same order, so a row's bits do not depend on the batch it is in.  Few rows: 32 by 32 channels per
-// workgroup, so that as much of the GPU as there is reads the weight; more of both where that gives every CU a workgroup, which read
-// the weight and the windows less often.  This launch, us, 32 rows by 32 channels / 64 by 32 / 64 by 64 (windows + library product):
-// gated, 128 channels, 1 head, 1200 tokens (12 workgroups of the first form) 11.8 / 16.3 / 25.0 (15.9); 4 heads, 8K (256) 20.7 / 20.0 /
-// 27.0 (22.2), 16K (512) 35.5 / 28.9 / 30.8 (31.0), 8 x 6K (1500) 94.6 / 74.6 / 66.2 (76.0), 64K (2048) 136 / 106 / 76.7 (106); 192 channels,
-// 2 heads, 12K (282) 46.0 / 29.7 / 41.7 (31.0); 64 channels, 2 heads, 40 x 600 (240) 10.6 / 13.0 / 17.7 (18.4).  Linear: 8K 12.2 /
-// 14.0 / 16.0 (18.8), 16K 23.2 / 20.9 / 18.0 (32.6), 64K 92.8 / 85.6 / 51.8 (81.6).
+// workgroup, so that as much of the GPU as there is reads the weight; more of both where that still gives the GPU one round of
+// workgroups, of which the larger forms fit a CU once (their stages take 82 to 140 KB of LDS): 64 by 32 up to half as many workgroups
+// as CUs, 64 by 64 beyond, which reads the weight and the windows least often.  This launch without the hidden rows, us, 32 rows by 32
+// channels / 64 by 32 / 64 by 64 (windows + library product), by rows (workgroups of the first form): gated, 128 channels: 2000 (252)
+// 18.5 / 18.7 / 25.8 (40), 3000 (376) 30.6 / 24.2 / 30.0 (40), 4100 (516) 44.0 / 40.3 / 30.9 (50), 6000 (752) 47.4 / 54.3 / 35.6 (54), 24000
+// 172 / 148 / 111 (146); 64 channels: 6000 (376) 17.1 / 13.9 / 17.5, 8200 (514) 22.6 / 24.5 / 19.9 (40), 12000 (750) 25.8 / 27.9 / 21.0; linear:
+// 128 channels 3000 21.3 / 18.3 / 18.7 (33), 6000 32.6 / 43.5 / 24.8 (41); 192: 2000 (378) 31.6 / 21.1 / 23.7 (35), 3000 (564) 47.4 / 51.4 /
+// 30.6 (51); 256: 2000 (504) 50.9 / 29.5 / 31.6 (40), 3000 (752) 71.0 / 71.8 / 39.3 (50).
 template <bool GLU>
 void dispatch_fwd(const CompressParams& p, int y_maxlen, hipStream_t s) {
   const int64_t blocks = p.D / 32, wgs = ((int64_t)y_maxlen * p.H + 31) / 32 * p.B * blocks;
   const int cus = nsa_device_cus();
   if (wgs <= cus) launch_fwd<1, GLU, 1, 2>(p, y_maxlen, s);
-  else if (wgs <= 3 * cus || blocks % 2 != 0) launch_fwd<1, GLU, 2, 2>(p, y_maxlen, s);
+  else if (wgs <= 2 * cus || blocks % 2 != 0) launch_fwd<1, GLU, 2, 2>(p, y_maxlen, s);
   else launch_fwd<2, GLU, 2, 1>(p, y_maxlen, s);
 }
 
