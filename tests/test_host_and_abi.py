@@ -61,6 +61,21 @@ def test_learned_compression_takes_only_weights_with_memory_of_their_own():
     assert not takes_weight(x, wrapped, "linear") and not takes_weight(x, torch.nn.Parameter(wrapped), "linear")
 
 
+@pytest.mark.parametrize("D,version,heads,tokens,taken", [
+    (256, "swiglu", 1, 40016, True), (256, "swiglu", 1, 40032, False),           # 2500 and 2501 rows
+    (256, "linear", 4, 160016, True), (256, "linear", 4, 160032, False),         # 40000 and 40004
+    (192, "sigmoid-mul", 4, 160016, False), (192, "linear", 4, 160032, False),
+    (128, "swiglu", 4, 1 << 20, True), (64, "linear", 8, 1 << 20, True)])
+def test_long_products_with_wide_weights_stay_with_the_library(D, version, heads, tokens, taken):
+    """The line lies at a number of rows that depends on the weight's size."""
+    from types import SimpleNamespace
+    from flash_nsa.ops.compress_kv import takes_weight
+    helper = SimpleNamespace(kernel_size=32, y_len=(tokens - 32) // 16 + 1)
+    x = SimpleNamespace(size=lambda i: (tokens, heads, D)[i], is_cuda=True, device=torch.device("cpu"), dtype=torch.bfloat16)
+    w = torch.empty(D if version == "linear" else 2 * D, 32 * D, dtype=torch.bfloat16)
+    assert takes_weight(x, w, version, helper) == taken
+
+
 def test_weights_of_any_layout_are_copied_for_the_kernels():
     """What saved-tensor hooks give back may begin anywhere and lie in any order: the kernels get whole, aligned rows."""
     from flash_nsa.ops.compress_kv import weight_rows
