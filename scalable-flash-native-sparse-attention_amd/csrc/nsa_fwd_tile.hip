@@ -604,12 +604,21 @@ int launch_fwd_tile(const NsaFwdTileParams& p0, int B, int max_q_len, hipStream_
   // CU each, and the short ones fill up.  (Last rows first within each sequence and head: the first rows of the second head met
   // those of the first on the same CUs while other CUs had one workgroup.)  Whole calls, that / so, us, 64 / 4 heads of 128: 3
   // prompts of 60 to 700 tokens 79 / 65, 2 of 300 to 900 78 / 68, 6 of 60 to 1000 134 / 125, 16 x 128 to 256 behind up to 256 107 /
-  // 105; forward of 1000 tokens 78 / 69, 1500 160 / 144, 4096 526 / 520; 16 / 2 heads of 64, 20 samples of up to 1100 138 / 124.
-  // Launches of more workgroups take them in the order of their rows, which keeps neighbours' keys in L2 (8 x 6K tokens 18.4 /
-  // 18.7 ms, 16 x 2K paged rows 5.21 / 5.25), short ones from twice as many on: 40 samples of 17 to 1200 218 / 203, 12 prompts
-  // of 60 to 1000 253 / 249.  The compressed branch gains nothing (1500 tokens 205 / 203, 4 x 300 to 1500 156 / 160).
+  // 105.  Forwards, rows in their order / so, us, by workgroups per CU: sequences of at most all_below (1024) tokens, 64 / 4 heads of
+  // 128: 1000 tokens (2.0) 65 / 57, 8 x 600 (9.4) 148 / 145; 32 / 8 heads: 20 x 1000 (20.0) 524 / 419; 16 / 2 of 64: 20 x 1000 (9.8)
+  // 122 / 112, 60 x 1000 (29.5) 324 / 322; 16 / 4 of 256: 20 x 1000 (10.0) 929 / 642; of up to twice as many: 64 / 4 of 128: 1500 (2.9)
+  // 151 / 139, 2000 (3.9) 209 / 201; 16 / 1: 4 x 2000 (3.9) 208 / 200, 16 x 1100 (8.6) 246 / 235; 16 / 2 of 64: 24 x 100 to 1940 (22.9) 297 /
+  // 287, 40 x 17 to 1187 (23.4) 176 / 164.  Not so, there in one round, which has no order to speak of: 16 / 1 of 128: 1500 (0.7) 97 /
+  // 99, 2000 (1.0) 100 / 103; not longer sequences, whose longest rows are the first: 3000 (1.5) 119 / 125, 6000 (2.9) 213 / 220, 4 x
+  // 1500 to 3000 (5.9) 256 / 261, 32 / 2 of 192: 3000 (2.9) 217 / 228 (64 / 4 heads of 128 alone gain 1 %); not launches of more
+  // workgroups, where neighbours' keys stay in L2 with rows in their order: 64 / 4 of 128: 16 x 1100 (34.5) 844 / 866, 20 x 1000 (39.1)
+  // 756 / 781, paged 8 x 500 to 2000 (31.3) 703 / 715, with 192 and 256 channels, of whose rows L2 holds fewer, from half as many on: 32 / 2
+  // of 192: 8 x 600 (4.7) 100 / 90, 4 x 2000 (7.8) 425 / 418, 16 x 1100 (17.2) 517 / 533, 20 x 1000 (19.5) 442 / 460; 16 / 4 of 256: 24 x
+  // 100 to 2000 (23.6) 4376 / 4428.  The compressed branch gains nothing (1500 tokens 205 / 203, 4 x 300 to 1500 156 / 160).
   const int64_t wgs = (int64_t)cdiv_i(max_q_len * p.G, 128) * B * p.KH;
-  p.last_first = MODE >= MODE_TAIL && wgs <= (max_q_len / 2 <= p.all_below ? 32 : 16) * nsa_device_cus();
+  const int cus = nsa_device_cus();
+  const bool all = max_q_len <= p.all_below;
+  p.last_first = MODE >= MODE_TAIL && max_q_len / 2 <= p.all_below && wgs <= (D >= 192 ? 16 : all ? 32 : 24) * cus && (all || wgs > cus);
   const int tiles = cdiv_i(max_q_len * p.G, 128);
   const dim3 grid = p.last_first ? dim3(B * p.KH, tiles) : dim3(tiles, B, p.KH);
   // 0 (default): direct-to-LDS staging for the compressed branch with power-of-two head dims (4.5 % faster there; the window

@@ -462,3 +462,18 @@ def test_block_selection_is_that_of_its_scores(device, lens, kind, kw):
             assert torch.equal(got, want.int()), (got != want).nonzero()[:4]
     finally:
         NSAHelper.set_hyperparameters()
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,n,counts", [(16, 1, 64, 64, 1500, (1, 3, 60)), (16, 2, 128, 128, 1000, (1, 20, 40)),
+                                                 (16, 1, 192, 128, 1100, (1, 8, 40)), (8, 2, 256, 256, 700, (1, 5, 50))])
+def test_a_sequence_does_not_depend_on_the_batch_around_it(device, QH, KH, D, VD, n, counts):
+    """Forwards whose launches take the rows in their order and those that start the last rows first (by sequence length and number of
+    workgroups): every copy of a sequence has the same bits."""
+    from flash_nsa import NSAConfig, NSACore
+    core = NSACore(NSAConfig(qk_head_dim=D, v_head_dim=VD, num_heads=QH, num_kv_heads=KH))
+    ins, want = [t.to(device) for t in make_qkvw(n, QH, KH, D, VD, seed=70)], None
+    for count in counts:
+        with torch.no_grad():
+            out = core(*(t.repeat(count, 1, 1) for t in ins), make_cu([n] * count).to(device)).view(count, n, QH, VD)
+        want = out[0].clone() if want is None else want
+        assert bool((out == want).all())
