@@ -660,7 +660,9 @@ int dispatch_fwd_tile(const NsaFwdTileParams& p, int B, int max_q_len, int D, in
   if (D == 128 && VD == 128) return launch_fwd_tile<128, 128, MODE, PAGED>(p, B, max_q_len, stream);
   if (D == 64 && VD == 64) return launch_fwd_tile<64, 64, MODE, PAGED>(p, B, max_q_len, stream);
   if (D == 192 && VD == 128) return launch_fwd_tile<192, 128, MODE, PAGED>(p, B, max_q_len, stream);
-  if (D == 256 && VD == 256) return launch_fwd_tile<256, 256, MODE, PAGED>(p, B, max_q_len, stream);
+  if constexpr (MODE != MODE_ALL) {
+    if (D == 256 && VD == 256) return launch_fwd_tile<256, 256, MODE, PAGED>(p, B, max_q_len, stream);
+  }
   if (D == 32 && VD == 32) return launch_fwd_tile<32, 32, MODE, PAGED>(p, B, max_q_len, stream);
   nsa_set_error("attention forward: unsupported head dims D=%d VD=%d (built: 128/128, 64/64, 192/128, 256/256, 32/32)", D, VD);
   return NSA_ERR_UNSUPPORTED;
@@ -673,6 +675,18 @@ int nsa_fwd_tile_launch(const NsaFwdTileParams& p, int mode, bool paged, int B, 
   if (mode == MODE_CMP) {
     return paged ? dispatch_fwd_tile<MODE_CMP, true>(p, B, max_q_len, D, VD, stream)
                  : dispatch_fwd_tile<MODE_CMP, false>(p, B, max_q_len, D, VD, stream);
+  }
+  if (mode == MODE_ALL && D == 256) {
+    // The branches' pointers do not fit beside 256 channels' accumulators: in one launch 96 to 116 bytes a lane are spilled.  16 / 4 heads,
+    // one launch / two, us: 1000 tokens 102 / 96, paged 32 x 1 to 32 behind up to 600 80 / 75, 64 x 100 to 1000 1095 / 1075.
+    NsaFwdTileParams c = p;
+    c.k = p.ck; c.k_sr = p.ck_sr; c.k_sh = p.ck_sh;
+    c.v = p.cv; c.v_sr = p.cv_sr; c.v_sh = p.cv_sh;
+    c.table = p.c_table; c.table_stride = p.c_table_stride;
+    c.o = p.cmp_o_out; c.o_st = p.co_st; c.o_sh = p.co_sh;
+    c.lse = p.cmp_lse; c.lse_st = p.cl_st; c.lse_sh = p.cl_sh;
+    const int rc = nsa_fwd_tile_launch(c, MODE_CMP, paged, B, max_q_len, D, VD, stream);
+    return rc != NSA_OK ? rc : nsa_fwd_tile_launch(p, MODE_TAIL, paged, B, max_q_len, D, VD, stream);
   }
   if (mode == MODE_ALL) {
     return paged ? dispatch_fwd_tile<MODE_ALL, true>(p, B, max_q_len, D, VD, stream)
