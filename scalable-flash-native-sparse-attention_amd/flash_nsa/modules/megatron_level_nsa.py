@@ -28,22 +28,44 @@ from ..ops.sliding_window_attention import (short_fwd, slc_fwd_first_queries, sw
 # gain nor lose (64K tokens 55.0 ms either way); the same split of the forward gained nothing.
 # Setting this module attribute to False puts everything back on the caller's stream.
 OVERLAP_STREAMS = True
-# Work that passes between two streams costs the host 70 us of events, waits and first launches, and the GPU as much again, which
-# small batches wait for.  Their second stream is the caller's: those whose tokens x q-heads x longest sequence (at most 2048: the
-# window and the selected blocks end there) x channels (128 on top, for what does not grow with them) stay below this.  Whole
-# steps on two streams / on one, us (this number, 1e9): 64 heads of 128, 1024 tokens 741 / 471 (26), 1300 824 / 583 (42), 1600 839 /
-# 697 (63; mean compression 625 / 602), 2048 811 / 818 (103), 6 x 100 to 600 681 / 464 (21), 12 x 673 / 682 (54), 8 x 100 to 700
-# 789 / 777 (69); 16 heads, 4096 771 / 661 (52), 5000 835 / 788 (63; mean 692 / 736), 6000 844 / 871 (76), 8 x 100 to 1500 809 / 712
-# (68); 32 heads of 192, 1024 744 / 444 (15), 2048 779 / 761 (60), 2500 848 / 892 (73); 16 heads of 64, 5000 804 / 627 (42), 6500 772
-# / 743 (55), 8192 836 / 868 (69), 20 x 200 to 1000 710 / 598 (46), 40 of up to 1200 948 / 1122 (133).
-OVERLAP_FROM = 6e10
+# A second stream costs a small step 60 to 100 us of events, waits and first launches, of the host and of the GPU.  The second stream of
+# small batches is therefore the caller's: of those whose tokens x q-heads x longest sequence (at most 2048: the window and the selected
+# blocks end there) x channels (128 on top, for what does not grow with them) stay below this.  Whole steps on two streams / on one, us
+# (this number, 1e9): 64 / 4 heads of 128, 1024 tokens 448 / 352 (26), 1500 586 / 538 (55), 2000 689 / 728 (98), 8 x 700 848 / 853 (96); 16
+# / 1, 3000 571 / 472 (38), 4096 575 / 530 (52), 4 x 1500 498 to 580 / 541 (55), 6000 721 / 773 (75); 32 / 2 of 192, 1500 568 / 514 (32), 2000 618
+# / 671 (57), 12 x 400 531 / 508 (28); 16 / 2 of 64, 4096 511 / 431 (34), 6000 541 / 566 (50), 9000 779 / 836 (75); 8 / 1 of 128, 6000 677 /
+# 570 (38), 9000 766 / 798 (57).
+# Shapes without a dk / dv pass that stores dS have longer kernels, and a lower line.  More than 128 channels, a fifth: 16 / 4 heads of
+# 256, 4 x 500 429 / 422 (10), 12 x 400 787 / 828 (20); 20 / 4 of 192, 1024 403 / 341 (9.4), 12 x 400 412 / 423 (17), 1500 570 / 610 (20).
+# Batches that select everything, two fifths: 24 / 8 of 128, 4 x 500 285 / 221 (9.2), 8 x 700 546 / 586 (36); 16 / 16 of 64, 8 x 700 395 /
+# 331 (16); 32 / 8, 12 x 400 441 / 439 (24).  Others, counted in whole groups of 16 q-heads, of which the kernels of the selected blocks
+# are made, 1.78 times: 12 / 4 of 128 (64 heads), 2000 596 / 558 (98), 3000 777 / 827 (151), 6000 1519 / 1629 (302); 8 / 8 of 32 (128
+# heads), 2000 528 / 445 (98), 3000 654 / 679 (151), 6000 1216 / 1257 (302); 12 / 2 of 64, 4096 549 / 508 (69), 6000 626 / 675 (101).
+# Ordered sums, two ninths whatever the shape: 16 / 1 of 128, 12 x 400 383 / 334 (12), 1500 664 / 724 (14), 4096 857 / 915 (52); 8 / 1,
+# 2000 527 / 526 (12), 3000 545 / 591 (19); 32 / 2 of 192, 1024 570 / 578 (15).
+OVERLAP_FROM = 5.6e10
 _side_streams = {}
+
+
+def _gains_from_overlap(q, v, helper):
+    T, QH, D = q.shape
+    KH, VD = v.shape[1:]
+    heads, line = QH, OVERLAP_FROM
+    if getattr(helper, "deterministic", False):
+        line /= 4.5
+    elif QH // KH not in (8, 16, 32, 64) or (D, VD) not in ((64, 64), (128, 128), (192, 128)):
+        if max(D, VD) > 128:
+            line /= 5
+        elif helper.x_maxlen <= helper.all_below():
+            line *= 0.4
+        else:
+            heads, line = KH * 16 * -(-QH // KH // 16), line * 1.78
+    return T * heads * min(helper.x_maxlen, 2048) * (D + VD + 128) >= line
 
 
 def _side_stream(main, q, v, helper):
     """The second stream of this batch's backward beside the caller's, main."""
-    T, QH, D = q.shape
-    if T * QH * min(helper.x_maxlen, 2048) * (D + v.size(-1) + 128) < OVERLAP_FROM:
+    if not _gains_from_overlap(q, v, helper):
         return main
     device = q.device
     key = device.index if device.index is not None else torch.cuda.current_device()

@@ -76,6 +76,25 @@ def test_long_products_with_wide_weights_stay_with_the_library(D, version, heads
     assert takes_weight(x, w, version, helper) == taken
 
 
+@pytest.mark.parametrize("shape,tokens,longest,deterministic,two", [
+    ((16, 1, 128, 128), 4096, 4096, False, False), ((16, 1, 128, 128), 6000, 6000, False, True),      # dS is stored
+    ((32, 2, 192, 128), 2000, 2000, False, True), ((64, 4, 128, 128), 1024, 1024, False, False),
+    ((16, 1, 128, 128), 1500, 1500, True, True), ((16, 1, 128, 128), 4800, 400, True, False),         # ordered sums
+    ((12, 4, 128, 128), 2000, 2000, False, False), ((12, 4, 128, 128), 3000, 3000, False, True),      # groups of other sizes
+    ((8, 8, 32, 32), 2000, 2000, False, False), ((8, 8, 32, 32), 3000, 3000, False, True),
+    ((12, 4, 128, 128), 5600, 700, False, False), ((24, 8, 128, 128), 5600, 700, False, True),        # every block selected
+    ((16, 4, 256, 256), 1000, 1000, False, False), ((16, 4, 256, 256), 4800, 400, False, True),       # wide channels
+    ((16, 1, 128, 128), 0, 0, False, False)])
+def test_batches_that_gain_from_a_second_stream(shape, tokens, longest, deterministic, two):
+    """The fused backward forks for these batches and not for those, by the kernels that their shapes have."""
+    from types import SimpleNamespace
+    from flash_nsa.modules.megatron_level_nsa import _gains_from_overlap
+    QH, KH, D, VD = shape
+    q, v = torch.empty(tokens, QH, D, device="meta"), torch.empty(tokens, KH, VD, device="meta")
+    helper = SimpleNamespace(x_maxlen=longest, all_below=lambda: 1024, deterministic=deterministic)
+    assert _gains_from_overlap(q, v, helper) == two
+
+
 def test_weights_of_any_layout_are_copied_for_the_kernels():
     """What saved-tensor hooks give back may begin anywhere and lie in any order: the kernels get whole, aligned rows."""
     from flash_nsa.ops.compress_kv import weight_rows
