@@ -6,7 +6,8 @@
 // selected dK/dV kernel.  us for count + scan + fill, with one search per entry, a scan and a fill that wait for every
 // element -> as below: one sequence of 4K tokens, 1 kv head 79 -> 24, 40 of up to 1.2K, 2 kv heads 101 -> 31, 8 x 6K,
 // 4 kv heads 149 -> 58, 64K 171 -> 82.  Four threads per token, and sequences found at one look, fill alone: 40 of up to 1.2K
-// 14 -> 8, 4K 14 to 29 -> 10, 16K 19 -> 12 (a chunk's workgroup is often alone on its CU: one wave per SIMD before).  Reading 32
+// 14 -> 8, 4K 14 to 29 -> 10, 16K 19 -> 12 (a chunk's workgroup is often alone on its CU: one wave per SIMD before); 64 sequences a look also
+// where there are more (two binary searches before): 1000 sequences of 60, 4 kv heads, 61 -> 55, 8 kv heads 84 -> 72.  Reading 32
 // chunk counts at a time in the scan takes 109 registers a thread, and the launch then waits for the kernels beside it: 8 x 6K
 // 34 -> 217.
 // Upstream: flash_nsa/ops/topk.py:782-945 (get_bind_from_find, dense scatter + per-row sort).
@@ -29,12 +30,18 @@ __device__ __forceinline__ int find_seq(const int32_t* x_cu, int B, int tok) {
   return lo;
 }
 
-// The same for a token that is the same in all lanes: up to 64 sequences in one round trip to memory
+// The same for a token that is the same in all lanes: 64 sequences, or parts of their list, at a look
 __device__ __forceinline__ int find_seq_uniform(const int32_t* x_cu, int B, int tok) {
-  if (B > 64) return find_seq(x_cu, B, tok);
   const int lane = lane_id();
-  const bool from = x_cu[min(lane, B - 1)] <= tok && lane > 0 && lane < B;
-  return (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(from));
+  int lo = 0;
+  for (int n = B; n > 1;) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const bool from = x_cu[lo + min(i, n - 1)] <= tok && lane > 0 && i < n;
+    const int k = (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(from));
+    lo += k * step;
+    n = min(step, n - k * step);
+  }
+  return lo;
 }
 
 // A query token of the sequences b0 .. b1: where its sequence's blocks begin, how many there are and how many slots of its selection
@@ -57,12 +64,12 @@ __device__ __forceinline__ TokenRow token_row(const int32_t* topk, int64_t tk_sh
   r.nvalid = r.n >= t_begin ? min(top_n, r.n / block_size + 1) : 0;
   return r;
 }
-// fn(global block, slot) for the blocks that the token selected, slots ROW part .. ROW part + ROW - 1 of every ROW * PARTS: PARTS
-// threads share a token; the ids are fetched ROW at a time, so that they share one round trip to memory
-constexpr int PARTS = 4, ROW = 4, NT = 256 * PARTS;
-template <class Fn>
+// fn(global block, slot) for the blocks that the token selected, slots ROW part .. ROW part + ROW - 1 of every 16: PARTS threads share
+// a token; the ids are fetched ROW at a time, so that they share one round trip to memory
+template <int PARTS, class Fn>
 __device__ __forceinline__ void for_each_block(const TokenRow& r, int part, Fn fn) {
-  for (int s0 = part * ROW; s0 < r.nvalid; s0 += ROW * PARTS) {
+  constexpr int ROW = 16 / PARTS;
+  for (int s0 = part * ROW; s0 < r.nvalid; s0 += 16) {
     int j[ROW];
 #pragma unroll
     for (int s = 0; s < ROW; s++) j[s] = s0 + s < r.nvalid ? r.slots[s0 + s] : -1;
@@ -73,10 +80,12 @@ __device__ __forceinline__ void for_each_block(const TokenRow& r, int part, Fn f
 }
 
 // grid (nchunks, KH), dynamic LDS nblk ints
-__global__ __launch_bounds__(NT) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+template <int PARTS>
+__global__ __launch_bounds__(256 * PARTS) void csr_count_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
                                                         const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
                                                         int T, int nblk, int block_size, int t_begin,
                                                         int32_t* chunk_cnt) {
+  constexpr int NT = 256 * PARTS;
   extern __shared__ int hist[];
   const int chunk = blockIdx.x, kh = blockIdx.y;
   const int part = threadIdx.x >> 8;
@@ -89,7 +98,7 @@ __global__ __launch_bounds__(NT) void csr_count_kernel(const int32_t* topk, int6
   for (int tb = t0; tb < t1; tb += 256) {
     const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, b0, b1, tb + (threadIdx.x & 255), t1, kh, block_size,
                                  t_begin);
-    for_each_block(r, part, [&](int jb, int) { atomicAdd(&hist[jb], 1); });
+    for_each_block<PARTS>(r, part, [&](int jb, int) { atomicAdd(&hist[jb], 1); });
   }
   __syncthreads();
   int32_t* dst = chunk_cnt + ((int64_t)kh * gridDim.x + chunk) * nblk;
@@ -159,11 +168,13 @@ __global__ __launch_bounds__(1024) void csr_scan_kernel(int32_t* chunk_cnt, int 
 // long as 256 dependent LDS updates, whatever the size of the batch).  LDS holds the masks of FILL_BLOCKS blocks; more
 // blocks than that are taken in several rounds.
 constexpr int FILL_BLOCKS = 1024, FILL_WORDS = 256 / 32;
-__global__ __launch_bounds__(NT) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
+template <int PARTS>
+__global__ __launch_bounds__(256 * PARTS) void csr_fill_kernel(const int32_t* topk, int64_t tk_sh, int64_t tk_st, int top_n,
                                                        const int32_t* x_cu, const int32_t* kblk_cu, int B, int tok0,
                                                        int T, int nblk, int block_size, int t_begin,
                                                        const int32_t* chunk_base, const int32_t* csr_off,
                                                        int32_t* csr_tok, uint8_t* csr_slot) {
+  constexpr int NT = 256 * PARTS;
   __shared__ int cursor[FILL_BLOCKS];
   __shared__ __attribute__((aligned(16))) uint32_t mask[FILL_BLOCKS * FILL_WORDS];
   const int chunk = blockIdx.x, kh = blockIdx.y;
@@ -188,11 +199,11 @@ __global__ __launch_bounds__(NT) void csr_fill_kernel(const int32_t* topk, int64
       __syncthreads();
       const TokenRow r = token_row(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, b0, b1, tb + row, t1, kh, block_size,
                                    t_begin);
-      for_each_block(r, part, [&](int jb, int) {
+      for_each_block<PARTS>(r, part, [&](int jb, int) {
         if ((unsigned)(jb - r0) < (unsigned)nr) atomicOr(&mask[(jb - r0) * FILL_WORDS + word], bit);
       });
       __syncthreads();
-      for_each_block(r, part, [&](int jb, int slot) {
+      for_each_block<PARTS>(r, part, [&](int jb, int slot) {
         if ((unsigned)(jb - r0) >= (unsigned)nr) return;
         const uint32_t* m = &mask[(jb - r0) * FILL_WORDS];
         int pos = cursor[jb - r0];
@@ -261,16 +272,30 @@ int nsa_build_inverse_index_slots(const int32_t* topk, int64_t tk_sh, int64_t tk
   int nchunks = (T + CT - 1) / CT;
   size_t lds = (size_t)nblk_total * sizeof(int);
   dim3 grid(nchunks, KH);
-  csr_count_kernel<<<grid, NT, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
-                                          t_begin, workspace);
+  // Four threads per token: workgroups of 1024, of which a CU holds two, so more than that pay only where a token has many slots to look at
+  // (blocks per sequence on average; 16 slots are one thread's read).  One thread / four, us, count + scan + fill, by workgroups: 16K tokens
+  // of 1 kv head (64) 27 / 22, 40 x 1200 of 2 (376) 43 / 39, 64K of 2 (512) 61 / 56, 200 x 300 of 2 (470) 45.3 / 45.7; of 4: 8 x 6K, top_n 16
+  // (752) 56.2 / 55.8, 8 37 / 42, 32 147 / 138, 64 153 / 145, 200 x 300 (940) 51 / 57, 40 x 3000 (1876) 278 / 279, top_n 32 847 / 828; of 8: 200
+  // x 300 (1880) 60 / 75.  (64K of 1, top_n 64, 256 workgroups: 91 / 97.)
+  const int seq_blocks = nblk_total / B;
+  const bool few = (int64_t)nchunks * KH <= 2 * nsa_device_cus() || (top_n < seq_blocks ? top_n : seq_blocks) > 16;
+  auto count = [&](auto kernel, int threads) {
+    kernel<<<grid, threads, lds, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size, t_begin, workspace);
+  };
+  if (few) count(csr_count_kernel<4>, 1024);
+  else count(csr_count_kernel<1>, 256);
   int rc = nsa_check_launch("csr_count_kernel");
   if (rc) return rc;
   csr_scan_kernel<<<KH, 1024, 0, s>>>(workspace, nchunks, nblk_total, (int64_t)T * top_n, chunk_tokens, csr_off,
                                       item_off);
   rc = nsa_check_launch("csr_scan_kernel");
   if (rc) return rc;
-  csr_fill_kernel<<<grid, NT, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size,
-                                        t_begin, workspace, csr_off, csr_tok, csr_slot);
+  auto fill = [&](auto kernel, int threads) {
+    kernel<<<grid, threads, 0, s>>>(topk, tk_sh, tk_st, top_n, x_cu, kblk_cu, B, tok0, T, nblk_total, block_size, t_begin, workspace, csr_off,
+                                    csr_tok, csr_slot);
+  };
+  if (few) fill(csr_fill_kernel<4>, 1024);
+  else fill(csr_fill_kernel<1>, 256);
   return nsa_check_launch("csr_fill_kernel");
 }
 
