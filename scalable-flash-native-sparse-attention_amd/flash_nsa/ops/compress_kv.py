@@ -72,20 +72,23 @@ def takes_weight(x, weight, version, helper=NSAHelper):
     return (type(weight) in (torch.nn.Parameter, torch.Tensor) and D % 32 == 0 and x.is_cuda and weight.device == x.device
             and x.dtype == weight.dtype == torch.bfloat16 and weight.shape == (N, helper.kernel_size * D) and weight.stride(1) == 1
             and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0 and weight.data_ptr() != 0
-            and not (weight.numel() > MIB and _long(helper.y_len * x.size(1), weight.numel())))
+            and not (weight.numel() > MIB and _faster_by_products(helper.y_len * x.size(1), weight.numel(), D)))
 
 
 MIB = 1 << 20
 
 
-def _long(rows, weight):
+def _faster_by_products(rows, weight, D):
     """Whether the library's products of so many rows are faster than the kernels'.  These read a weight of more than 4 MB (2 M numbers)
     from behind an XCD's L2 again for every tile of rows, and the sums of dW's parts grow with it.  Forward and backward, us, kernels /
-    windows and library, by rows: 256 channels, gated: 2000 141 / 142 (the kernels in fewer launches), 3000 222 / 181, 8200 585 / 481,
-    65500 4175 / 2977; 192, gated: 3000 162 / 146, 6000 263 / 255, 16400 656 / 690, 65500 2440 / 2253 (the forward alone: 6000 91 / 70, 16400
-    187 / 175).  Weights of more than 2 MB: 192, linear: 32800 962 / 1073, 48000 1405 / 1466, 65500 1948 / 1861, 262000 7996 / 6842; 256,
-    linear: 32800 1251 / 1410, 48000 1823 / 1862 (forward 595 / 481), 131000 4990 / 4676.  Smaller ones: 128, gated: 2000 68 / 110, 65500
-    1146 / 1428, 262000 4632 / 5125."""
+    windows and library, by rows: 256 channels, gated: 250 85 / 55, 1000 109 / 96, 3000 222 / 181, 8200 585 / 481, 65500 4175 / 2977; linear:
+    250 60 / 44, 500 64 / 60, 1000 72 / 82, 32800 1251 / 1410, 48000 1823 / 1862 (forward 595 / 481), 131000 4990 / 4676 (short batches save 80 us
+    of the host with the kernels, and attention of 256 channels waits for it up to 100 rows: staged steps of 16 / 4 heads, 300 tokens, 68
+    rows, 630 / 840, 700 tokens, 172 rows, 968 / 935).  192, gated: 2000 104 / 119, 3000 162 / 146, 6000 263 / 255, 16400 656 / 690, 65500 2440 /
+    2253 (the forward alone: 6000 91 / 70, 16400 187 / 175); linear: 32800 962 / 1073, 48000 1405 / 1466, 65500 1948 / 1861, 262000 7996 / 6842.
+    Smaller weights: 128, gated: 2000 68 / 110, 65500 1146 / 1428, 262000 4632 / 5125."""
+    if D > 192:
+        return rows > 100 and (weight > 2 * MIB or not 700 < rows <= 40000)
     return rows > (2500 if weight > 2 * MIB else 40000)
 
 

@@ -62,7 +62,9 @@ def test_learned_compression_takes_only_weights_with_memory_of_their_own():
 
 
 @pytest.mark.parametrize("D,version,heads,tokens,taken", [
-    (256, "swiglu", 1, 40016, True), (256, "swiglu", 1, 40032, False),           # 2500 and 2501 rows
+    (256, "swiglu", 1, 1616, True), (256, "swiglu", 1, 1632, False),             # 100 and 101 rows
+    (256, "linear", 4, 416, True), (256, "linear", 1, 1632, False), (256, "linear", 1, 11216, False), (256, "linear", 1, 11232, True),
+    (192, "swiglu", 1, 40016, True), (192, "swiglu", 1, 40032, False),           # 2500 and 2501
     (256, "linear", 4, 160016, True), (256, "linear", 4, 160032, False),         # 40000 and 40004
     (192, "sigmoid-mul", 4, 160016, False), (192, "linear", 4, 160032, False),
     (128, "swiglu", 4, 1 << 20, True), (64, "linear", 8, 1 << 20, True)])
