@@ -4,8 +4,10 @@
 // rows of D channels every `stride` rows, is read where it lies in x: element j * D + d of it is x[stride * i + j][d].
 // A row of these products is a (compressed row, kv head) pair, row-major in that order.
 //
-// What bounds them is the L2 traffic of the weight (forward, dx) or of the windows (dW) at long batches, and at short ones the
-// launches: a library product costs the host 33 us, and the windows took two more launches and two passes over them.
+// What bounds them at long batches is round trips to L2: every tile reads the weight (forward, dx) or the windows (dW) again, and the waves
+// wait 30 % (forward), 58 % (dx) and 69 % (dW) of their cycles, with the matrix cores busy 18, 17 and 10 % and LDS 38, 34 and 18 % (64K
+// tokens, 4 heads of 128, gated).  At short batches it is the launches: a library product costs the host 33 us, and the windows took two more
+// launches and two passes over them.
 #include "nsa_common.h"
 #include "nsa_api_internal.h"
 #include "../../include/nsa_hip.h"
@@ -273,8 +275,8 @@ __global__ __launch_bounds__(256, 2) void compress_linear_dx_kernel(CompressPara
   }
 }
 
-// dW, 64K tokens, 4 heads of 128, N 256: 131 us, bound by the transposed reads of LDS (library product 152); 40 samples of up to 1.2K,
-// 2 heads of 64, both weights 35 + 18 for the sums (72: 32 workgroups).
+// dW, 64K tokens, 4 heads of 128, N 256: 131 us, of which the waves wait 69 % for the next step's rows (library product 152); 40 samples of
+// up to 1.2K, 2 heads of 64, both weights 35 + 12 for the sums (72: 32 workgroups).
 // dW = (gradient of hidden)^T windows, cut along the contraction into gridDim.z parts whose sums go to slots.  A workgroup: NT * 32
 // rows of dW by 128 columns, both tiles (their rows are the contraction index) in LDS, read transposed.
 // grid (N / 32 / NT, ceil(kernel * D / 128), parts)
