@@ -37,10 +37,11 @@ OVERLAP_STREAMS = True
 # 570 (38), 9000 766 / 798 (57).
 # Shapes without a dk / dv pass that stores dS have longer kernels, and a lower line.  More than 128 channels, a fifth: 16 / 4 heads of
 # 256, 4 x 500 429 / 422 (10), 12 x 400 787 / 828 (20); 20 / 4 of 192, 1024 403 / 341 (9.4), 12 x 400 412 / 423 (17), 1500 570 / 610 (20).
-# Batches that select everything, two fifths: 24 / 8 of 128, 4 x 500 285 / 221 (9.2), 8 x 700 546 / 586 (36); 16 / 16 of 64, 8 x 700 395 /
-# 331 (16); 32 / 8, 12 x 400 441 / 439 (24).  Others, counted in whole groups of 16 q-heads, of which the kernels of the selected blocks
-# are made, 1.78 times: 12 / 4 of 128 (64 heads), 2000 596 / 558 (98), 3000 777 / 827 (151), 6000 1519 / 1629 (302); 8 / 8 of 32 (128
-# heads), 2000 528 / 445 (98), 3000 654 / 679 (151), 6000 1216 / 1257 (302); 12 / 2 of 64, 4096 549 / 508 (69), 6000 626 / 675 (101).
+# Batches that select everything, two fifths above 64 channels: 24 / 8 of 128, 4 x 500 285 / 221 (9.2), 8 x 700 546 / 586 (36); 32 / 8, 12
+# x 400 441 / 439 (24); the whole up to 64: 16 / 16 of 64, 8 x 700 395 / 331 (16); 8 / 8 of 32, 4 x 3000 with top_n 64 382 to 397 / 286 to
+# 331 (38). Others, counted in whole groups of 16 q-heads, of which the kernels of the selected blocks are made, 1.78 times: 12 / 4 of 128
+# (64 heads), 2000 596 / 558 (98), 3000 777 / 827 (151), 6000 1519 / 1629 (302); 8 / 8 of 32 (128 heads), 2000 528 / 445 (98), 3000 654 /
+# 679 (151), 6000 1216 / 1257 (302); 12 / 2 of 64, 4096 549 / 508 (69), 6000 626 / 675 (101).
 # Ordered sums, two ninths whatever the shape: 16 / 1 of 128, 12 x 400 383 / 334 (12), 1500 664 / 724 (14), 4096 857 / 915 (52); 8 / 1,
 # 2000 527 / 526 (12), 3000 545 / 591 (19); 32 / 2 of 192, 1024 570 / 578 (15).
 OVERLAP_FROM = 5.6e10
@@ -57,7 +58,7 @@ def _gains_from_overlap(q, v, helper):
         if max(D, VD) > 128:
             line /= 5
         elif helper.x_maxlen <= helper.all_below():
-            line *= 0.4
+            line *= 0.4 if max(D, VD) > 64 else 1
         else:
             heads, line = KH * 16 * -(-QH // KH // 16), line * 1.78
     return T * heads * min(helper.x_maxlen, 2048) * (D + VD + 128) >= line

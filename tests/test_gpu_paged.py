@@ -959,3 +959,26 @@ def test_prefill_of_short_contexts_in_one_launch_equals_two(device, QH, KH, D, p
     cmp_o, _ = S.cmp_attn_prefill(q, d["k"], d["v"], xcu, max(new), d["cbt"], ctx_t)
     want = S.swa_combine_prefill(q, d["k"], d["v"], cmp_o, torch.empty_like(cmp_o), w, xcu, max(new), d["bt"], ctx_t, all_below=1024)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("QH,KH,D,VD,all_below", [(16, 1, 128, 128, 2560), (6, 2, 64, 64, 3072), (8, 2, 192, 128, 1024), (4, 1, 256, 256, 2560)])
+def test_short_prefill_of_a_request_does_not_depend_on_the_others(device, QH, KH, D, VD, all_below):
+    """All orders in which a launch takes its rows (by the longest context that selects everything): each request has the bits that it has
+    alone."""
+    from flash_nsa.inference import stages as S
+    cached, new = ([0, 130, 1500, 1, 0], [2560, 700, 33, 129, 1]) if all_below > 1024 else ([0, 130, 900, 1, 0], [1024, 700, 33, 129, 1])
+    ctx = [c + n for c, n in zip(cached, new)]
+    case = build_pool(ctx, KH, D, VD, page=64, seed=12)
+    prepool(case, ctx)
+    d = to_dev(case, device)
+    t = sum(new)
+    q, w = randn_bf16(t, QH, D, seed=13).to(device), randn_bf16(t, QH, 3, seed=14).to(device)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32).to(device)
+    got = S.short_prefill(q, d["k"], d["v"], w, make_cu(new).to(device), max(new), d["bt"], d["cbt"], ctx_t, all_below)
+    assert bool(torch.isfinite(got).all())
+    at = 0
+    for b, n in enumerate(new):
+        alone = S.short_prefill(q[at:at + n], d["k"], d["v"], w[at:at + n], make_cu([n]).to(device), n, d["bt"][b:b + 1], d["cbt"][b:b + 1],
+                                ctx_t[b:b + 1], all_below)
+        assert torch.equal(got[at:at + n], alone), b
+        at += n

@@ -85,6 +85,7 @@ def test_long_products_with_wide_weights_stay_with_the_library(D, version, heads
     ((12, 4, 128, 128), 2000, 2000, False, False), ((12, 4, 128, 128), 3000, 3000, False, True),      # groups of other sizes
     ((8, 8, 32, 32), 2000, 2000, False, False), ((8, 8, 32, 32), 3000, 3000, False, True),
     ((12, 4, 128, 128), 5600, 700, False, False), ((24, 8, 128, 128), 5600, 700, False, True),        # every block selected
+    ((16, 16, 64, 64), 5600, 700, False, False), ((16, 16, 64, 64), 24000, 1000, False, True),
     ((16, 4, 256, 256), 1000, 1000, False, False), ((16, 4, 256, 256), 4800, 400, False, True),       # wide channels
     ((16, 1, 128, 128), 0, 0, False, False)])
 def test_batches_that_gain_from_a_second_stream(shape, tokens, longest, deterministic, two):
