@@ -38,7 +38,8 @@ def _has_tangent(t):
 
 class CompressKV(torch.nn.Module):
     """Compresses [T,H,D] into one row per window of kernel_size tokens every stride tokens.
-    mean: average; linear: fc over the flattened window; sigmoid-mul / swiglu: gated fc (2*D outputs)."""
+    mean: average; linear: fc over the flattened window; sigmoid-mul / swiglu: gated fc (2*D outputs).
+    A fc's gradient reads x again: x is not to be changed in place before the backward (autograd refuses it)."""
 
     def __init__(self, config: NSAConfig, head_dim=128, version=None):
         super().__init__()
